@@ -15,6 +15,8 @@ from __future__ import annotations
 import ctypes as C
 import weakref
 import os
+import struct
+from array import array
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Sequence
 
@@ -53,7 +55,7 @@ EXPORTED_SYMBOLS = [
     "sr_batch_append_tokens", "sr_batch_append_tokens_masks", "sr_batch_upload_mask_ids", "sr_mask_register",
     "sr_mask_release", "sr_mask_and", "sr_pack_allow_mask_launch",
     "sr_sample_launch", "sr_resample_rows_launch", "sr_sample_batch", "sr_argmax_rows_launch", "sr_argmax_rows_launch_noalloc",
-    "sr_argmax_rows",
+    "sr_argmax_rows", "sr_argmax_rows_both",
     "sr_build_distribution_launch", "sr_sample_with_distribution_launch", "sr_sample_from_probs_launch",
     "sr_resample_residual_launch", "sr_spec_verify_launch", "sr_mtp_verify_launch", "sr_pack_allow_mask",
     "sr_build_distribution", "sr_sample_with_distribution", "sr_sample_from_probs", "sr_resample_residual",
@@ -139,9 +141,9 @@ def load_library():
         L = C.CDLL(_LIB_PATH)
     except OSError as e:  # pragma: no cover - depends on the host
         raise NativeLibraryError(f"cannot load {_LIB_PATH}: {e}") from e
-    vp, i32, i64, u32p, i32p, f32p, f64p = (C.c_void_p, C.c_int32, C.c_int64, C.POINTER(C.c_uint32),
-                                             C.POINTER(C.c_int32), C.POINTER(C.c_float), C.POINTER(C.c_double))
-    rpp = C.POINTER(RowParams)
+    # (arrays go in as addresses: a typed ctypes pointer made from a numpy array is a reference cycle, and a call per token
+    # that leaves a few of those behind pays for the collector's passes over the whole process)
+    vp, i32, i64 = C.c_void_p, C.c_int32, C.c_int64
     L.sr_create.argtypes = [C.c_int, C.POINTER(vp)]
     L.sr_destroy.argtypes = [vp]
     L.sr_destroy.restype = None
@@ -155,36 +157,37 @@ def load_library():
     L.sr_batch_create.argtypes = [vp, C.POINTER(vp)]
     L.sr_batch_destroy.argtypes = [vp]
     L.sr_batch_destroy.restype = None
-    L.sr_batch_upload.argtypes = [vp, i32, i32, rpp, i32p, i32p, i32p, f32p, i32p, u32p, i64,
-                                  C.POINTER(C.c_uint8), f64p, i32]
-    L.sr_batch_set_uniforms.argtypes = [vp, f64p]
-    L.sr_batch_append_tokens.argtypes = [vp, i32p, f64p]
-    L.sr_batch_append_tokens_masks.argtypes = [vp, i32p, f64p, i32p]
-    L.sr_batch_upload_mask_ids.argtypes = [vp, i32, i32, rpp, i32p, i32p, i32p, f32p, i32p, i32p, f64p, i32]
-    L.sr_mask_register.argtypes = [vp, vp, C.c_int, i32, i32p]
+    L.sr_batch_upload.argtypes = [vp, i32, i32, vp, vp, vp, vp, vp, vp, vp, i64,
+                                  vp, vp, i32]
+    L.sr_batch_set_uniforms.argtypes = [vp, vp]
+    L.sr_batch_append_tokens.argtypes = [vp, vp, vp]
+    L.sr_batch_append_tokens_masks.argtypes = [vp, vp, vp, vp]
+    L.sr_batch_upload_mask_ids.argtypes = [vp, i32, i32, vp, vp, vp, vp, vp, vp, vp, vp, i32]
+    L.sr_mask_register.argtypes = [vp, vp, C.c_int, i32, vp]
     L.sr_mask_release.argtypes = [vp, i32]
-    L.sr_mask_and.argtypes = [vp, i32p, i32, i32p]
+    L.sr_mask_and.argtypes = [vp, vp, i32, vp]
     L.sr_pack_allow_mask_launch.argtypes = [vp, vp, C.c_int, i32, i32, i64, vp, i64]
     L.sr_sample_launch.argtypes = [vp, vp, vp, C.c_int, i64, vp, vp]
-    L.sr_resample_rows_launch.argtypes = [vp, vp, vp, C.c_int, i64, i32p, i32, vp, vp]
-    L.sr_sample_batch.argtypes = [vp, vp, C.c_int, C.c_int, i32, i32, i64, rpp, i32p, i32p, i32p, f32p, i32p,
-                                  u32p, i64, C.POINTER(C.c_uint8), f64p, i32p, u32p]
+    L.sr_resample_rows_launch.argtypes = [vp, vp, vp, C.c_int, i64, vp, i32, vp, vp]
+    L.sr_sample_batch.argtypes = [vp, vp, C.c_int, C.c_int, i32, i32, i64, vp, vp, vp, vp, vp, vp,
+                                  vp, i64, vp, vp, vp, vp]
     L.sr_argmax_rows_launch.argtypes = [vp, vp, C.c_int, i32, i32, i64, vp, vp]
     L.sr_argmax_rows_launch_noalloc.argtypes = [vp, vp, C.c_int, i32, i32, i64, vp, vp]
-    L.sr_argmax_rows.argtypes = [vp, vp, C.c_int, C.c_int, i32, i32, i64, i32p, f32p]
+    L.sr_argmax_rows.argtypes = [vp, vp, C.c_int, C.c_int, i32, i32, i64, vp, vp]
+    L.sr_argmax_rows_both.argtypes = [vp, vp, C.c_int, i32, i32, i64, vp, vp, vp, vp]
     L.sr_build_distribution_launch.argtypes = [vp, vp, vp, C.c_int, i64, vp, i64, i32]
     L.sr_sample_with_distribution_launch.argtypes = [vp, vp, vp, C.c_int, i64, vp, i64, i32, vp]
-    L.sr_sample_from_probs_launch.argtypes = [vp, vp, i32, i32, i64, f64p, vp]
-    L.sr_resample_residual_launch.argtypes = [vp, vp, i32, i64, vp, i32, i64, i32, f64p, vp]
+    L.sr_sample_from_probs_launch.argtypes = [vp, vp, i32, i32, i64, vp, vp]
+    L.sr_resample_residual_launch.argtypes = [vp, vp, i32, i64, vp, i32, i64, i32, vp, vp]
     L.sr_spec_verify_launch.argtypes = [vp, vp, vp, vp, vp, i32, vp, vp]
     L.sr_mtp_verify_launch.argtypes = [vp, vp, i32, i32, i64, vp, C.c_float, vp, vp, vp]
-    L.sr_pack_allow_mask.argtypes = [f32p, i32, u32p]
+    L.sr_pack_allow_mask.argtypes = [vp, i32, vp]
     _lib = L
     return L
 
 
-def _ptr(a: Optional[np.ndarray], ctype):
-    return None if a is None else a.ctypes.data_as(C.POINTER(ctype))
+def _ptr(a: Optional[np.ndarray]):
+    return None if a is None else a.ctypes.data
 
 
 def pack_allow_mask(allowed: np.ndarray) -> np.ndarray:
@@ -200,6 +203,49 @@ def pack_allow_mask(allowed: np.ndarray) -> np.ndarray:
     return words[0] if one else words
 
 
+_ROW = struct.Struct("=fifffifffI")  # sr_row_params
+
+
+def _i32(values: List[int]) -> np.ndarray:
+    try:
+        return np.frombuffer(array("i", values), dtype=np.int32)  # (three times as fast as np.array over a list of ints)
+    except (TypeError, OverflowError):
+        return np.array(values, dtype=np.int32)
+
+
+def _pack_params(params: Sequence[SamplingParams], histories: Optional[Sequence[Optional[Sequence[int]]]] = None):
+    """The arrays of sr_batch_upload that come from the rows' parameters: sr_row_params, histories (in place of the rows'
+    PreviousTokens when given), logit bias.  A history that no penalty of its row looks at stays behind."""
+    row_bytes = []
+    hist: List[int] = []
+    hoff = [0]
+    bids: List[int] = []
+    bvals: List[float] = []
+    boff = [0]
+    for i, p in enumerate(params):
+        bias = p.LogitBias
+        try:
+            row_bytes.append(_ROW.pack(p.Temperature, p.TopK, p.TopP, p.MinP, p.RepetitionPenalty, p.RepeatLastN, p.PresencePenalty,
+                                       p.FrequencyPenalty, p.SpecDraftPMin, (SR_ROW_HAS_LOGIT_BIAS if bias else 0)
+                                       | (SR_ROW_DRAFT_FROM_LOOKUP if p.SpecDraftFromLookup else 0)))
+        except (struct.error, OverflowError):  # (values that ctypes narrows)
+            row_bytes.append(bytes(p.to_row()))
+        if p.RepetitionPenalty != 1.0 or p.PresencePenalty != 0.0 or p.FrequencyPenalty != 0.0:
+            h = p.PreviousTokens if histories is None else histories[i]
+            if h is not None:
+                hist.extend(h)
+        hoff.append(len(hist))
+        if bias:
+            bids.extend(int(k) for k in bias.keys())
+            bvals.extend(float(v) for v in bias.values())
+        boff.append(len(bids))
+    return (b"".join(row_bytes) if row_bytes else bytes(_ROW.size), _i32(hist) if hist else None,
+            _i32(hoff), _i32(bids) if bids else None, np.array(bvals, dtype=np.float32) if bids else None, _i32(boff) if bids else None)
+
+
+assert _ROW.size == C.sizeof(RowParams)
+
+
 class _Batch:
     def __init__(self, ctx: "SamplerContext"):
         self.ctx = ctx
@@ -210,31 +256,12 @@ class _Batch:
         self.vocab = 0
 
     def upload(self, params: Sequence[SamplingParams], vocab: int, uniforms=None, allow_mask=None,
-               mask_active=None, uniforms_per_row: Optional[int] = None, mask_ids=None):
+               mask_active=None, uniforms_per_row: Optional[int] = None, mask_ids=None, histories=None):
         """mask_ids: per row the id of a registered allow-mask (SamplerContext.register_mask), -1 for none, instead
-        of allow_mask / mask_active."""
+        of allow_mask / mask_active.  histories: per row the previous tokens (None for none), in place of the rows'
+        PreviousTokens."""
         rows = len(params)
-        arr = (RowParams * max(rows, 1))()
-        hist: List[int] = []
-        hoff = [0]
-        bids: List[int] = []
-        bvals: List[float] = []
-        boff = [0]
-        for i, p in enumerate(params):
-            arr[i] = p.to_row()
-            if p.PreviousTokens is not None:
-                hist.extend(int(t) for t in p.PreviousTokens)
-            hoff.append(len(hist))
-            if p.LogitBias:
-                for k_, v_ in p.LogitBias.items():
-                    bids.append(int(k_))
-                    bvals.append(float(v_))
-            boff.append(len(bids))
-        h_ids = np.asarray(hist, dtype=np.int32) if hist else None
-        h_off = np.asarray(hoff, dtype=np.int32)
-        b_ids = np.asarray(bids, dtype=np.int32) if bids else None
-        b_vals = np.asarray(bvals, dtype=np.float32) if bids else None
-        b_off = np.asarray(boff, dtype=np.int32) if bids else None
+        arr, h_ids, h_off, b_ids, b_vals, b_off = _pack_params(params, histories)
         m = None
         stride = 0
         act = None
@@ -256,8 +283,8 @@ class _Batch:
             ids = np.ascontiguousarray(np.asarray(mask_ids, dtype=np.int32))
             assert ids.shape == (rows,)
             self.ctx._check(self.ctx.L.sr_batch_upload_mask_ids(
-                self.h, rows, vocab, arr, _ptr(h_ids, C.c_int32), _ptr(h_off, C.c_int32), _ptr(b_ids, C.c_int32),
-                _ptr(b_vals, C.c_float), _ptr(b_off, C.c_int32), _ptr(ids, C.c_int32), _ptr(u, C.c_double), upr))
+                self.h, rows, vocab, arr, _ptr(h_ids), _ptr(h_off), _ptr(b_ids),
+                _ptr(b_vals), _ptr(b_off), _ptr(ids), _ptr(u), upr))
             return self
         return self.reupload()
 
@@ -266,32 +293,32 @@ class _Batch:
         gathering its parameters."""
         rows, vocab, arr, h_ids, h_off, b_ids, b_vals, b_off, m, stride, act, u, upr = self._packed
         self.ctx._check(self.ctx.L.sr_batch_upload(
-            self.h, rows, vocab, arr, _ptr(h_ids, C.c_int32), _ptr(h_off, C.c_int32),
-            _ptr(b_ids, C.c_int32), _ptr(b_vals, C.c_float), _ptr(b_off, C.c_int32),
-            _ptr(m, C.c_uint32), stride, _ptr(act, C.c_uint8), _ptr(u, C.c_double), upr))
+            self.h, rows, vocab, arr, _ptr(h_ids), _ptr(h_off),
+            _ptr(b_ids), _ptr(b_vals), _ptr(b_off),
+            _ptr(m), stride, _ptr(act), _ptr(u), upr))
         return self
 
     def append_tokens(self, tokens, uniforms=None, mask_ids=None):
         """sr_batch_append_tokens: one more token per row (negative = none) at the end of the histories of the last
         upload(), and optionally the uniforms of the next step.  mask_ids (batches uploaded with mask ids): the
         registered allow-mask of every row for the next step (sr_batch_append_tokens_masks)."""
-        t = np.ascontiguousarray(np.asarray(tokens, dtype=np.int32))
+        t = np.ascontiguousarray(tokens, dtype=np.int32)
         assert t.shape == (self.rows,)
         u = None
         if uniforms is not None:
-            u = np.ascontiguousarray(np.asarray(uniforms, dtype=np.float64))
+            u = np.ascontiguousarray(uniforms, dtype=np.float64)
         if mask_ids is not None:
-            ids = np.ascontiguousarray(np.asarray(mask_ids, dtype=np.int32))
+            ids = np.ascontiguousarray(mask_ids, dtype=np.int32)
             assert ids.shape == (self.rows,)
-            self.ctx._check(self.ctx.L.sr_batch_append_tokens_masks(self.h, _ptr(t, C.c_int32), _ptr(u, C.c_double),
-                                                                    _ptr(ids, C.c_int32)))
+            self.ctx._check(self.ctx.L.sr_batch_append_tokens_masks(self.h, _ptr(t), _ptr(u),
+                                                                    _ptr(ids)))
             return self
-        self.ctx._check(self.ctx.L.sr_batch_append_tokens(self.h, _ptr(t, C.c_int32), _ptr(u, C.c_double)))
+        self.ctx._check(self.ctx.L.sr_batch_append_tokens(self.h, _ptr(t), _ptr(u)))
         return self
 
     def set_uniforms(self, uniforms):
-        u = np.ascontiguousarray(np.asarray(uniforms, dtype=np.float64))
-        self.ctx._check(self.ctx.L.sr_batch_set_uniforms(self.h, _ptr(u, C.c_double)))
+        u = np.ascontiguousarray(uniforms, dtype=np.float64)
+        self.ctx._check(self.ctx.L.sr_batch_set_uniforms(self.h, _ptr(u)))
 
     def close(self):
         if self.h:
@@ -359,7 +386,7 @@ class SamplerContext:
         if isinstance(words, np.ndarray):
             w = np.ascontiguousarray(words, dtype=np.uint32)
             assert w.size >= (vocab + 31) // 32
-            self._check(self.L.sr_mask_register(self.h, w.ctypes.data_as(C.c_void_p), 0, vocab, C.byref(out)))
+            self._check(self.L.sr_mask_register(self.h, _ptr(w), 0, vocab, C.byref(out)))
         else:
             assert words.is_cuda and words.numel() >= (vocab + 31) // 32
             self._check(self.L.sr_mask_register(self.h, C.c_void_p(words.data_ptr()), 1, vocab, C.byref(out)))
@@ -370,7 +397,7 @@ class SamplerContext:
         left to intersect or the intersection allows no token (the row then goes unmasked)."""
         ids = np.ascontiguousarray(np.asarray(mask_ids, dtype=np.int32))
         out = C.c_int32(-1)
-        self._check(self.L.sr_mask_and(self.h, _ptr(ids, C.c_int32), int(ids.size), C.byref(out)))
+        self._check(self.L.sr_mask_and(self.h, _ptr(ids), int(ids.size), C.byref(out)))
         return int(out.value)
 
     def release_mask(self, mask_id: int) -> None:
@@ -417,54 +444,61 @@ class SamplerContext:
         """Async: logits [rows, vocab] CUDA tensor (row stride in elements), outputs CUDA int32."""
         assert logits.is_cuda and out_tokens.is_cuda
         self._check(self.L.sr_sample_launch(
-            self.h, batch.h, C.c_void_p(logits.data_ptr()), self._dtype_of(logits), self._row_stride(logits),
-            C.c_void_p(out_tokens.data_ptr()), C.c_void_p(out_flags.data_ptr() if out_flags is not None else 0)))
+            self.h, batch.h, logits.data_ptr(), self._dtype_of(logits), self._row_stride(logits),
+            out_tokens.data_ptr(), None if out_flags is None else out_flags.data_ptr()))
 
     def resample_rows_launch(self, batch: _Batch, logits, rows, out_tokens, out_flags=None):
         """Async: SampleTopK by device-wide sorts for the given rows of the batch (those a launch flagged
         SR_OUT_ROW_UNSUPPORTED); same tensors as sample_launch."""
         r = np.ascontiguousarray(rows, dtype=np.int32)
         self._check(self.L.sr_resample_rows_launch(
-            self.h, batch.h, C.c_void_p(logits.data_ptr()), self._dtype_of(logits), self._row_stride(logits),
-            r.ctypes.data_as(C.POINTER(C.c_int32)), int(r.size),
-            C.c_void_p(out_tokens.data_ptr()), C.c_void_p(out_flags.data_ptr() if out_flags is not None else 0)))
+            self.h, batch.h, logits.data_ptr(), self._dtype_of(logits), self._row_stride(logits),
+            _ptr(r), int(r.size),
+            out_tokens.data_ptr(), None if out_flags is None else out_flags.data_ptr()))
 
     def sample_batch(self, logits, params: Sequence[SamplingParams], uniforms, allow_mask=None, mask_active=None,
                      return_flags: bool = False):
         """Sampler.Sample for every row (preceded by the row's mask). logits: CUDA tensor [rows, vocab].
         Returns numpy int32 tokens (and flags)."""
-        import torch
-
         rows, vocab = logits.shape
-        batch = self.new_batch().upload(params, vocab, uniforms, allow_mask, mask_active)
-        toks = torch.empty(rows, dtype=torch.int32, device=logits.device)
-        flags = torch.zeros(rows, dtype=torch.int32, device=logits.device)
-        self.sample_launch(batch, logits, toks, flags)
-        self.synchronize()
-        torch.cuda.synchronize()
-        redo = np.nonzero(flags.cpu().numpy().view(np.uint32) & np.uint32(SR_OUT_ROW_UNSUPPORTED))[0]
-        if redo.size:  # rows that overflowed the selection kernel's row tail: as sr_sample_batch does
-            self.resample_rows_launch(batch, logits, redo, toks, flags)
-            self.synchronize()
-            torch.cuda.synchronize()
-        batch.close()
-        t = toks.cpu().numpy()
-        return (t, flags.cpu().numpy().view(np.uint32)) if return_flags else t
+        if len(params) > rows:
+            raise ValueError(f"{len(params)} parameter sets for {rows} rows")
+        toks = np.zeros(rows, dtype=np.int32)
+        flags = np.zeros(rows, dtype=np.uint32)
+        arr, h_ids, h_off, b_ids, b_vals, b_off = _pack_params(params)
+        m = act = u = None
+        if allow_mask is not None:
+            m = np.ascontiguousarray(np.asarray(allow_mask, dtype=np.uint32))
+            assert m.ndim == 2 and m.shape[0] == len(params)
+            if mask_active is not None:
+                act = np.ascontiguousarray(np.asarray(mask_active, dtype=np.uint8))
+        if uniforms is not None and len(params) > 0:
+            u = np.ascontiguousarray(np.asarray(uniforms, dtype=np.float64).reshape(len(params), -1)[:, 0])
+        self._check(self.L.sr_sample_batch(
+            self.h, logits.data_ptr(), self._dtype_of(logits), 1, len(params), vocab, self._row_stride(logits) if rows > 0 else vocab,
+            arr, _ptr(h_ids), _ptr(h_off), _ptr(b_ids), _ptr(b_vals), _ptr(b_off), _ptr(m), 0 if m is None else m.shape[1],
+            _ptr(act), _ptr(u), _ptr(toks), _ptr(flags)))
+        return (toks, flags) if return_flags else toks
 
     def argmax_rows(self, logits, out=None, noalloc=False):
         """(int Token, float Logit)[] per row -- BatchForwardMultiArgmax's result shape.  out=(idx, val) device
         tensors to write into; noalloc=True goes through the entry point that allocates no device memory."""
-        import torch
-
         rows, vocab = logits.shape
-        idx, val = out if out is not None else (torch.empty(rows, dtype=torch.int32, device=logits.device),
-                                                torch.empty(rows, dtype=torch.float32, device=logits.device))
-        fn = self.L.sr_argmax_rows_launch_noalloc if noalloc else self.L.sr_argmax_rows_launch
-        self._check(fn(
-            self.h, C.c_void_p(logits.data_ptr()), self._dtype_of(logits), rows, vocab,
-            self._row_stride(logits) if rows > 0 and vocab > 0 else vocab, C.c_void_p(idx.data_ptr()), C.c_void_p(val.data_ptr())))
-        self.synchronize()
-        return idx.cpu().numpy(), val.cpu().numpy()
+        stride = self._row_stride(logits) if rows > 0 and vocab > 0 else vocab
+        if noalloc:
+            import torch
+
+            idx, val = out if out is not None else (torch.empty(rows, dtype=torch.int32, device=logits.device),
+                                                    torch.empty(rows, dtype=torch.float32, device=logits.device))
+            self._check(self.L.sr_argmax_rows_launch_noalloc(self.h, logits.data_ptr(), self._dtype_of(logits), rows, vocab, stride,
+                                                             idx.data_ptr(), val.data_ptr()))
+            self.synchronize()
+            return idx.cpu().numpy(), val.cpu().numpy()
+        host_idx, host_val = np.empty(rows, dtype=np.int32), np.empty(rows, dtype=np.float32)
+        self._check(self.L.sr_argmax_rows_both(
+            self.h, logits.data_ptr(), self._dtype_of(logits), rows, vocab, stride, None if out is None else out[0].data_ptr(),
+            None if out is None else out[1].data_ptr(), _ptr(host_idx), _ptr(host_val)))
+        return host_idx, host_val
 
     def build_distribution(self, logits, params: Sequence[SamplingParams], probs_len: Optional[int] = None,
                            allow_mask=None, mask_active=None):
@@ -476,7 +510,7 @@ class SamplerContext:
         out = torch.zeros((rows, n), dtype=torch.float32, device=logits.device)
         try:
             self._check(self.L.sr_build_distribution_launch(
-                self.h, batch.h, C.c_void_p(logits.data_ptr()), self._dtype_of(logits), self._row_stride(logits),
+                self.h, batch.h, logits.data_ptr(), self._dtype_of(logits), self._row_stride(logits),
                 C.c_void_p(out.data_ptr()), self._row_stride(out), n))
             self.synchronize()
         finally:
@@ -492,7 +526,7 @@ class SamplerContext:
         toks = torch.empty(rows, dtype=torch.int32, device=logits.device)
         try:
             self._check(self.L.sr_sample_with_distribution_launch(
-                self.h, batch.h, C.c_void_p(logits.data_ptr()), self._dtype_of(logits), self._row_stride(logits),
+                self.h, batch.h, logits.data_ptr(), self._dtype_of(logits), self._row_stride(logits),
                 C.c_void_p(out.data_ptr()), self._row_stride(out), vocab, C.c_void_p(toks.data_ptr())))
             self.synchronize()
         finally:
@@ -504,8 +538,8 @@ class SamplerContext:
         every row stay on the device (out_probs [rows, vocab] fp32, out_tokens [rows] int32, CUDA tensors)."""
         vocab = logits.shape[-1]
         self._check(self.L.sr_sample_with_distribution_launch(
-            self.h, batch.h, C.c_void_p(logits.data_ptr()), self._dtype_of(logits), self._row_stride(logits),
-            C.c_void_p(out_probs.data_ptr()), self._row_stride(out_probs), vocab, C.c_void_p(out_tokens.data_ptr())))
+            self.h, batch.h, logits.data_ptr(), self._dtype_of(logits), self._row_stride(logits),
+            C.c_void_p(out_probs.data_ptr()), self._row_stride(out_probs), vocab, out_tokens.data_ptr()))
 
     def spec_verify_launch(self, batch: _Batch, target_logits, draft_probs, draft_tokens, out_accepted, out_tokens):
         """Async: sr_spec_verify_launch over device tensors (target [rows, L+1, V], q [rows, L, V], tokens [rows, L])."""
@@ -514,7 +548,7 @@ class SamplerContext:
             self.h, batch.h, C.c_void_p(target_logits.data_ptr()),
             C.c_void_p(None if draft_probs is None else draft_probs.data_ptr()),
             C.c_void_p(draft_tokens.data_ptr()), L, C.c_void_p(out_accepted.data_ptr()),
-            C.c_void_p(out_tokens.data_ptr())))
+            out_tokens.data_ptr()))
 
     def sample_from_probs(self, probs, uniforms):
         import torch
@@ -523,7 +557,7 @@ class SamplerContext:
         u = None if uniforms is None else np.ascontiguousarray(np.asarray(uniforms, dtype=np.float64))
         toks = torch.empty(rows, dtype=torch.int32, device=probs.device)
         self._check(self.L.sr_sample_from_probs_launch(
-            self.h, C.c_void_p(probs.data_ptr()), rows, vocab, self._row_stride(probs), _ptr(u, C.c_double),
+            self.h, C.c_void_p(probs.data_ptr()), rows, vocab, self._row_stride(probs), _ptr(u),
             C.c_void_p(toks.data_ptr())))
         self.synchronize()
         return toks.cpu().numpy()
@@ -536,7 +570,7 @@ class SamplerContext:
         toks = torch.empty(rows, dtype=torch.int32, device=p.device)
         self._check(self.L.sr_resample_residual_launch(
             self.h, C.c_void_p(p.data_ptr()), p.shape[1], self._row_stride(p), C.c_void_p(q.data_ptr()), q.shape[1],
-            self._row_stride(q), rows, _ptr(u, C.c_double), C.c_void_p(toks.data_ptr())))
+            self._row_stride(q), rows, _ptr(u), C.c_void_p(toks.data_ptr())))
         self.synchronize()
         return toks.cpu().numpy()
 
@@ -568,7 +602,7 @@ class SamplerContext:
         ok = torch.empty(rows, dtype=torch.int32, device=logits.device)
         pr = torch.empty(rows, dtype=torch.float32, device=logits.device)
         self._check(self.L.sr_mtp_verify_launch(
-            self.h, C.c_void_p(logits.data_ptr()), rows, vocab, self._row_stride(logits),
+            self.h, logits.data_ptr(), rows, vocab, self._row_stride(logits),
             C.c_void_p(draft_tokens.data_ptr()), p_min, C.c_void_p(am.data_ptr()), C.c_void_p(ok.data_ptr()),
             C.c_void_p(pr.data_ptr())))
         self.synchronize()

@@ -14,6 +14,8 @@
 const uint32_t* sr_batch_mask_ptr(const sr_batch* b) { return b->mask_ids ? b->ctx->mask_pool.as<uint32_t>() : b->d_mask.as<uint32_t>(); }
 int64_t sr_batch_mask_stride(const sr_batch* b) { return b->mask_ids ? (int64_t)b->ctx->pool_words : b->mask_stride; }
 
+const double* sr_batch_uniforms(const sr_batch* b) { return b->uni_now ? b->uni_now : b->d_uniforms.as<double>(); }
+
 int sr_batch_masks_valid(sr_ctx* ctx, const sr_batch* b, const char* who)
 {
     if (!b->mask_ids) return SR_OK;
@@ -62,16 +64,12 @@ void topk_geometry(int vocab, int dtype, int n_rows, int cu_count, int* chunks, 
 // called before anything that reads the destinations is enqueued.
 hipError_t batch_flush(sr_batch* b, hipStream_t st)
 {
-    if (b->segs.empty()) return hipSuccess;
-    const SrCopySeg* table = (const SrCopySeg*)b->stage.put(b->segs.data(), b->segs.size() * sizeof(SrCopySeg));
     hipError_t e = hipSuccess;
-    if (table) {
-        e = sr_launch_scatter(table, (int)b->segs.size(), st);
-    } else {  // no room for the list (the pinned memory grows for the next upload): one copy per piece
-        for (const SrCopySeg& s : b->segs) {
-            e = hipMemcpyAsync(s.dst, s.src, (size_t)s.bytes, hipMemcpyHostToDevice, st);
-            if (e != hipSuccess) break;
-        }
+    for (size_t i = 0; i < b->segs.size() && e == hipSuccess; i += SR_COPY_SEGS) {
+        SrCopyTable t{};
+        t.n = (int32_t)std::min(b->segs.size() - i, (size_t)SR_COPY_SEGS);
+        std::copy_n(b->segs.begin() + (ptrdiff_t)i, t.n, t.seg);
+        e = sr_launch_scatter(t, st);
     }
     b->segs.clear();
     return e;
@@ -101,11 +99,11 @@ hipError_t batch_copy(sr_batch* b, bool staged, void* dst, const void* src, size
 // (Re)builds the scan masks of a batch for logits of the given vector width and alignment.  Rows without an
 // allow-mask and without excluded history ids share one mask row when every row starts at the same offset
 // inside its first vector.
-int prepare_scan(sr_batch* b, int epv, unsigned long long base_addr, long long stride_bytes, bool staged = false)
+int prepare_scan(sr_batch* b, int epv, unsigned long long base_addr, long long stride_bytes)
 {
     sr_ctx* ctx = b->ctx;
     hipStream_t st = ctx->stream;
-    const int base_mod = (int)(base_addr & 15ull), stride_mod = (int)(stride_bytes & 15ll);
+    const int base_mod = (int)(base_addr & 15ull), stride_mod = b->rows <= 1 ? 0 : (int)(stride_bytes & 15ll);
     if (b->scan_epv == epv && b->scan_base_mod == base_mod && b->scan_stride_mod == stride_mod) return SR_OK;
     const bool can_share = stride_mod == 0 || b->rows <= 1;
     b->h_scan.clear();
@@ -251,7 +249,7 @@ int prepare_scan(sr_batch* b, int epv, unsigned long long base_addr, long long s
         b->n_items = total_items;
         b->own_rows = affine;
         SR_HIP(ctx, b->d_sched.reserve(sched.size() * sizeof(int32_t), st));
-        SR_HIP(ctx, batch_copy(b, staged, b->d_sched.p, sched.data(), sched.size() * sizeof(int32_t), st));
+        SR_HIP(ctx, batch_copy(b, true, b->d_sched.p, sched.data(), sched.size() * sizeof(int32_t), st));
     }
     b->scan_stride = (int64_t)chunks * SR_TK_THREADS * SR_TK_MASK_WORDS;
     b->scan_chunks = chunks;
@@ -260,18 +258,64 @@ int prepare_scan(sr_batch* b, int epv, unsigned long long base_addr, long long s
     b->scan_stride_bytes = stride_bytes;
     if (rows_changed) {
         b->spec_positions = 0;
-        SR_HIP(ctx, batch_copy(b, staged, b->d_rows.p, b->h_rows.data(), b->h_rows.size() * sizeof(SrRow), st));
+        SR_HIP(ctx, batch_copy(b, true, b->d_rows.p, b->h_rows.data(), b->h_rows.size() * sizeof(SrRow), st));
     }
     SR_HIP(ctx, b->d_scan_desc.reserve(b->h_scan.size() * sizeof(SrScanDesc), st));
-    SR_HIP(ctx, batch_copy(b, staged, b->d_scan_desc.p, b->h_scan.data(), b->h_scan.size() * sizeof(SrScanDesc), st));
+    SR_HIP(ctx, batch_copy(b, true, b->d_scan_desc.p, b->h_scan.data(), b->h_scan.size() * sizeof(SrScanDesc), st));
     SR_HIP(ctx, b->d_scan_mask.reserve(b->h_scan.size() * (size_t)b->scan_stride * sizeof(uint32_t), st));
+    const SrScanDesc* descs = b->d_scan_desc.as<SrScanDesc>();
+    const SrRow* rows = b->d_rows.as<SrRow>();
+    const SrEdit* edits = b->d_edits.as<SrEdit>();
+    SrCopyTable together{};
+    const SrCopyTable* pieces = nullptr;
+    if (!b->segs.empty() && b->segs.size() <= SR_COPY_SEGS) {
+        // A small upload: the workgroups that build the scan masks read the descriptors and the edits where the host packed
+        // them, and further workgroups of the same launch put the pieces in their places -- a launch and the gap behind it
+        // (6 us of a call for one row) less.  Every chunk's workgroup reads its row's edits over the bus, so this pays while
+        // they are few.
+        const SrCopySeg *sd = nullptr, *sr = nullptr, *se = nullptr;
+        size_t bytes = 0;
+        for (const SrCopySeg& s : b->segs) {
+            if (s.dst == b->d_scan_desc.p) sd = &s;
+            if (s.dst == b->d_rows.p) sr = &s;
+            if (s.dst == b->d_edits.p) se = &s;
+            bytes += (size_t)s.bytes;
+        }
+        if (sd && sr && (se || b->h_edits.empty()) && bytes * (size_t)chunks <= 65536) {
+            descs = (const SrScanDesc*)sd->src;
+            rows = (const SrRow*)sr->src;
+            if (se) edits = (const SrEdit*)se->src;
+            together.n = (int32_t)b->segs.size();
+            std::copy(b->segs.begin(), b->segs.end(), together.seg);
+            pieces = &together;
+            b->segs.clear();
+        }
+    }
     SR_HIP(ctx, batch_flush(b, st));
-    SR_HIP(ctx, sr_launch_build_scan_mask(b->d_scan_desc.as<SrScanDesc>(), nullptr, (int)b->h_scan.size(), b->d_rows.as<SrRow>(),
-                                          b->d_edits.as<SrEdit>(), sr_batch_mask_ptr(b), sr_batch_mask_stride(b),
-                                          b->d_scan_mask.as<uint32_t>(), b->scan_stride, b->vocab, epv, chunks, chunk_vecs,
-                                          base_addr, stride_bytes, st));
-    // the host vectors are read by the async copies above
-    if (!staged) SR_HIP(ctx, hipStreamSynchronize(st));
+    SR_HIP(ctx, sr_launch_build_scan_mask(descs, nullptr, (int)b->h_scan.size(), rows, edits, sr_batch_mask_ptr(b),
+                                          sr_batch_mask_stride(b), b->d_scan_mask.as<uint32_t>(), b->scan_stride, b->vocab, epv,
+                                          chunks, chunk_vecs, base_addr, stride_bytes, pieces, st));
+    return SR_OK;
+}
+
+// The scan masks of a batch for the logits of a launch: those the upload made, when it guessed their layout, or made again
+// (through the batch's pinned memory, like an upload).
+int scan_for_launch(sr_batch* b, int epv, unsigned long long base_addr, long long stride_bytes)
+{
+    sr_ctx* ctx = b->ctx;
+    ctx->last_epv = epv;
+    ctx->last_base_mod = (unsigned)(base_addr & 15ull);
+    ctx->last_stride_mod = (unsigned)(stride_bytes & 15ll);
+    if (b->scan_epv == epv && b->scan_base_mod == (int)ctx->last_base_mod &&
+        b->scan_stride_mod == (b->rows <= 1 ? 0 : (int)ctx->last_stride_mod))
+        return SR_OK;
+    SR_HIP(ctx, b->stage.begin(ctx->pinned));
+    b->segs.clear();
+    b->upload_must_wait = false;
+    const int rc = prepare_scan(b, epv, base_addr, stride_bytes);
+    if (rc != SR_OK) return rc;
+    if (b->upload_must_wait) SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    SR_HIP(ctx, b->stage.end(ctx->stream));
     return SR_OK;
 }
 
@@ -316,12 +360,14 @@ void sr_destroy(sr_ctx* ctx)
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->tmp_batch) sr_batch_destroy(ctx->tmp_batch);
     DeviceBuf* bufs[] = {&ctx->cand, &ctx->gmax, &ctx->gmax2, &ctx->gpos, &ctx->gbound, &ctx->row_done, &ctx->argmax_best, &ctx->argmax_done, &ctx->mask_pool, &ctx->mask_any,
-                         &ctx->work, &ctx->edit_tab, &ctx->host_logits, &ctx->stage_probs, &ctx->out_tokens, &ctx->out_flags, &ctx->out_val,
+                         &ctx->work, &ctx->edit_tab, &ctx->host_logits, &ctx->stage_probs, &ctx->out_tokens,
                          &ctx->full_state, &ctx->sort_k0, &ctx->sort_v0,
                          &ctx->sort_v1, &ctx->ident, &ctx->redo_list, &ctx->spec_probs, &ctx->spec_resid, &ctx->spec_reject,
                          &ctx->seg_part, &ctx->seg_func, &ctx->full_row_sync, &ctx->full_seg_func, &ctx->full_seg_ms, &ctx->full_watch, &ctx->full_watch_cnt, &ctx->full_seg_keys};
     for (DeviceBuf* b : bufs) b->release();
-    ctx->uni_ring.release();
+    ctx->uni_ring.release(ctx->pinned);
+    ctx->pinned.release();
+    ctx->results.release();
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
     delete ctx;
 }
@@ -383,19 +429,21 @@ void sr_batch_destroy(sr_batch* b)
     DeviceBuf* bufs[] = {&b->d_rows, &b->d_edits, &b->d_sel_list, &b->d_full_list, &b->d_wide_list, &b->d_scan_desc,
                          &b->d_mask, &b->d_scan_mask, &b->d_uniforms, &b->d_sched, &b->spec_rows};
     for (DeviceBuf* d : bufs) d->release();
-    b->stage.release();
-    b->patch_ring.release();
+    b->stage.release(b->ctx->pinned);
+    b->patch_ring.release(b->ctx->pinned);
+    b->uni_ring.release(b->ctx->pinned);
     delete b;
 }
 
 // sr_batch_upload.  retain: keep what sr_batch_append_tokens needs of the inputs; keep_uniforms: the uniforms on the
-// device stay as they are (uniforms is not read).
+// device stay as they are (uniforms is not read); waited_for: the caller waits for a launch behind the upload before the batch
+// is touched again, so no event marks the end of the upload's reads of pinned memory.
 static int batch_upload_impl(sr_batch* b, int32_t rows, int32_t vocab, const sr_row_params* params,
                              const int32_t* hist_ids, const int32_t* hist_offsets,
                              const int32_t* bias_ids, const float* bias_vals, const int32_t* bias_offsets,
                              const uint32_t* allow_mask, int64_t mask_stride_words, const uint8_t* mask_active,
                              const double* uniforms, int32_t uniforms_per_row, bool retain, bool keep_uniforms,
-                             const int32_t* mask_ids = nullptr)
+                             const int32_t* mask_ids = nullptr, bool waited_for = false)
 {
     if (!b || !b->ctx) return SR_ERR_NULL_ARGUMENT;
     sr_ctx* ctx = b->ctx;
@@ -422,7 +470,11 @@ static int batch_upload_impl(sr_batch* b, int32_t rows, int32_t vocab, const sr_
     }
     SR_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    SR_HIP(ctx, b->stage.begin());  // (waits for the copies of this batch's previous upload)
+    // (waits for the copies of this batch's previous upload; the estimate: descriptors, lists and programs, an edit per
+    // history id and logit bias with the room behind it)
+    const size_t n_edits_most = (size_t)(hist_offsets ? std::max(0, hist_offsets[rows] - hist_offsets[0]) : 0) +
+                                (size_t)(bias_offsets ? std::max(0, bias_offsets[rows] - bias_offsets[0]) : 0);
+    SR_HIP(ctx, b->stage.begin(ctx->pinned, b->stage.cap > 0 ? 0 : 4096 + (size_t)rows * 1024 + n_edits_most * 40));
     b->segs.clear();
     b->upload_must_wait = false;
 
@@ -660,12 +712,12 @@ static int batch_upload_impl(sr_batch* b, int32_t rows, int32_t vocab, const sr_
         SR_HIP(ctx, b->d_mask.reserve(bytes, st));
         SR_HIP(ctx, batch_copy(b, false, b->d_mask.p, allow_mask, bytes, st));
     }
+    if (!keep_uniforms) b->uni_now = nullptr;
     if (uniforms_per_row > 0 && !keep_uniforms)
         SR_HIP(ctx, up(b->d_uniforms, uniforms, (size_t)rows * (size_t)uniforms_per_row * sizeof(double)));
-    // scan masks for the layout of the last launch (16-byte aligned rows); a launch with another layout rebuilds
+    // scan masks for the layout of the last launch; a launch with another layout rebuilds them
     if (!b->h_sel_list.empty()) {
-        const int epv = ctx->last_epv;
-        int rc = prepare_scan(b, epv, 0ull, 0ll, true);
+        int rc = prepare_scan(b, ctx->last_epv, ctx->last_base_mod, ctx->last_stride_mod);
         if (rc != SR_OK) return rc;
     }
     // Everything small went through the batch's pinned memory: the copies and the scan-mask kernel run on while
@@ -673,7 +725,7 @@ static int batch_upload_impl(sr_batch* b, int32_t rows, int32_t vocab, const sr_
     // directly (the caller's allow-mask; anything the pinned memory had no room for yet) must be waited for.
     SR_HIP(ctx, batch_flush(b, st));
     if (b->upload_must_wait) SR_HIP(ctx, hipStreamSynchronize(st));
-    SR_HIP(ctx, b->stage.end(st));
+    if (!waited_for) SR_HIP(ctx, b->stage.end(st));
     return SR_OK;
 }
 
@@ -685,6 +737,20 @@ int sr_batch_upload(sr_batch* b, int32_t rows, int32_t vocab, const sr_row_param
 {
     return batch_upload_impl(b, rows, vocab, params, hist_ids, hist_offsets, bias_ids, bias_vals, bias_offsets, allow_mask,
                              mask_stride_words, mask_active, uniforms, uniforms_per_row, true, false);
+}
+
+// The uniforms of the next step: copied into pinned memory of the batch, where the sampling kernels read them (each row's
+// workgroup asks for its own long before the draw needs it): no copy command, which waited for the stream -- 17 us of
+// a step of 256 rows --, and no kernel that puts them into device memory.
+static int uniforms_in_place(sr_batch* b, const double* uniforms)
+{
+    sr_ctx* ctx = b->ctx;
+    const size_t bytes = (size_t)b->rows * (size_t)b->upr * sizeof(double);
+    SR_HIP(ctx, b->uni_ring.begin(ctx->pinned, bytes + 256, ctx->stream, 0, ctx->stream_epoch, true));
+    const void* at = b->uni_ring.put(uniforms, bytes);
+    if (!at) return sr_fail(ctx, SR_ERR_OUT_OF_MEMORY, "no pinned memory for the uniforms");
+    b->uni_now = (const double*)at;
+    return SR_OK;
 }
 
 // The batch as sr_batch_upload would build it for the histories as they are now (rows the in-place update does not
@@ -792,9 +858,9 @@ static int append_impl(sr_batch* b, const int32_t* tokens, const double* uniform
         const sr_row_params& p = b->keep_params[(size_t)r];
         const std::vector<int32_t>& hist = b->keep_hist[(size_t)r];
         const int32_t n_new = (int32_t)hist.size(), n_old = n_new - 1;
-        if (!has_history_penalty(p)) {  // the history is never looked at
+        if (!has_history_penalty(p)) {  // the history is never looked at, nor is its length
             d.n_prev = n_new;
-            rp.push_back(SrRowPatch{r, d.n_prev, d.edit_cnt, d.mask_row, d.sel, d.edit_off});
+            if (mask_changed) rp.push_back(SrRowPatch{r, d.n_prev, d.edit_cnt, d.mask_row, d.sel, d.edit_off});
             continue;
         }
         if (n_old == 0 || d.edit_cnt == 0 || d.path == SR_PATH_TOPK_WIDE) {
@@ -906,34 +972,33 @@ static int append_impl(sr_batch* b, const int32_t* tokens, const double* uniform
     // One kernel applies everything, reading the lists straight from the batch's pinned memory: no copy calls.
     SR_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    const size_t n_uni = (uniforms && b->upr > 0) ? (size_t)rows * (size_t)b->upr : 0;
     const size_t need = rp.size() * sizeof(SrRowPatch) + ep.size() * sizeof(SrEditPatch) + mc.size() * sizeof(SrMaskClear) +
-                        n_uni * sizeof(double) + scan_again.size() * sizeof(int32_t) + 5 * 256;
+                        scan_again.size() * sizeof(int32_t) + 4 * 256;
     // (a ring that is made now is made for the largest call to come as well: every row of the batch out of room at once,
     // all edits sent again -- rows that were uploaded together run out of room together)
     b->host_ahead = true;  // (until everything below has been enqueued)
-    SR_HIP(ctx, b->patch_ring.begin(need, st, b->h_edits.size() * sizeof(SrEditPatch) + (size_t)rows * 64 + n_uni * sizeof(double) + 65536,
+    SR_HIP(ctx, b->patch_ring.begin(ctx->pinned, need, st, b->h_edits.size() * sizeof(SrEditPatch) + (size_t)rows * 64 + 65536,
                                     ctx->stream_epoch));
     const SrRowPatch* rp_d = (const SrRowPatch*)b->patch_ring.put(rp.data(), rp.size() * sizeof(SrRowPatch));
     const SrEditPatch* ep_d = (const SrEditPatch*)b->patch_ring.put(ep.data(), ep.size() * sizeof(SrEditPatch));
     const SrMaskClear* mc_d = (const SrMaskClear*)b->patch_ring.put(mc.data(), mc.size() * sizeof(SrMaskClear));
-    const double* un_d = (const double*)b->patch_ring.put(uniforms, n_uni * sizeof(double));
     const int32_t* sa_d = (const int32_t*)b->patch_ring.put(scan_again.data(), scan_again.size() * sizeof(int32_t));
-    if (!rp_d || !ep_d || !mc_d || !un_d || !sa_d) return sr_fail(ctx, SR_ERR_OUT_OF_MEMORY, "sr_batch_append_tokens: no pinned memory");
+    if (!rp_d || !ep_d || !mc_d || !sa_d) return sr_fail(ctx, SR_ERR_OUT_OF_MEMORY, "sr_batch_append_tokens: no pinned memory");
     // scan masks that are not built yet are built from the patched edits when they are needed
     const bool masks = b->scan_epv != 0 && b->d_scan_mask.p != nullptr;
     b->spec_positions = 0;
     SR_HIP(ctx, sr_launch_apply_patches(b->d_rows.as<SrRow>(), rp_d, (int)rp.size(), b->d_edits.as<SrEdit>(), ep_d,
                                         (int)ep.size(), mc_d, masks ? (int)mc.size() : 0, b->d_scan_mask.as<uint32_t>(),
                                         b->scan_stride, masks ? b->scan_epv : 4, masks ? b->scan_chunk_vecs : 64,
-                                        b->scan_base_addr, b->scan_stride_bytes, b->d_uniforms.as<double>(), un_d,
-                                        (int)n_uni, st));
+                                        b->scan_base_addr, b->scan_stride_bytes, st));
+    if (uniforms && b->upr > 0)
+        if (int rc = uniforms_in_place(b, uniforms)) return rc;
     // rows whose allow-mask changed: their scan-mask rows are built again, from the new mask and the patched history
     if (masks && !scan_again.empty())
         SR_HIP(ctx, sr_launch_build_scan_mask(b->d_scan_desc.as<SrScanDesc>(), sa_d, (int)scan_again.size(), b->d_rows.as<SrRow>(),
                                               b->d_edits.as<SrEdit>(), sr_batch_mask_ptr(b), sr_batch_mask_stride(b),
                                               b->d_scan_mask.as<uint32_t>(), b->scan_stride, b->vocab, b->scan_epv,
-                                              b->scan_chunks, b->scan_chunk_vecs, b->scan_base_addr, b->scan_stride_bytes, st));
+                                              b->scan_chunks, b->scan_chunk_vecs, b->scan_base_addr, b->scan_stride_bytes, nullptr, st));
     b->host_ahead = false;
     return SR_OK;
 }
@@ -1096,10 +1161,7 @@ int sr_batch_set_uniforms(sr_batch* b, const double* uniforms)
     if (!uniforms) return sr_fail(ctx, SR_ERR_NULL_ARGUMENT, "sr_batch_set_uniforms: uniforms is null");
     if (b->upr <= 0 || b->rows <= 0) return SR_OK;
     SR_HIP(ctx, hipSetDevice(ctx->device));
-    SR_HIP(ctx, hipMemcpyAsync(b->d_uniforms.p, uniforms, (size_t)b->rows * b->upr * sizeof(double),
-                               hipMemcpyHostToDevice, ctx->stream));
-    SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return SR_OK;
+    return uniforms_in_place(b, uniforms);
 }
 
 int sr_sample_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int dtype, int64_t row_stride_elems,
@@ -1128,9 +1190,8 @@ int sr_sample_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int
         a.dtype = dtype;
         a.n_rows = n_sel;
         const int epv = dtype == SR_DTYPE_BF16 ? 8 : 4;
-        ctx->last_epv = epv;
-        int rc = prepare_scan(const_cast<sr_batch*>(b), epv, (unsigned long long)(uintptr_t)logits_dev,
-                              (long long)row_stride_elems * (dtype == SR_DTYPE_BF16 ? 2 : 4));
+        int rc = scan_for_launch(const_cast<sr_batch*>(b), epv, (unsigned long long)(uintptr_t)logits_dev,
+                                 (long long)row_stride_elems * (dtype == SR_DTYPE_BF16 ? 2 : 4));
         if (rc != SR_OK) return rc;
         topk_geometry(b->vocab, dtype, n_sel, ctx->cu_count, &a.chunks, &a.chunk_vecs);
         if (a.chunks > SR_TK_MAX_CHUNKS)
@@ -1171,7 +1232,7 @@ int sr_sample_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int
         a.done_cap = (uint32_t)ctx->done_cap;
         a.parity = (uint32_t)(ctx->launch_no++ & 1u);
         a.spin_limit = ctx->spin_limit;
-        a.uniforms = b->d_uniforms.as<double>();
+        a.uniforms = sr_batch_uniforms(b);
         a.uniforms_per_row = b->upr;
         a.out_tokens = out_tokens_dev;
         a.out_flags = out_flags_dev;
@@ -1243,38 +1304,43 @@ int sr_sample_batch(sr_ctx* ctx, const void* logits, int dtype, int logits_on_de
         int rc = sr_batch_create(ctx, &ctx->tmp_batch);
         if (rc != SR_OK) return rc;
     }
-    int rc = sr_batch_upload(ctx->tmp_batch, rows, vocab, params, hist_ids, hist_offsets, bias_ids, bias_vals,
-                             bias_offsets, allow_mask, mask_stride_words, mask_active, uniforms, uniforms ? 1 : 0);
-    if (rc != SR_OK) return rc;
+    // (the layout of this call's logits is known before the upload: the scan masks are made for it)
+    ctx->last_epv = dtype == SR_DTYPE_BF16 ? 8 : 4;
+    ctx->last_base_mod = logits_on_device ? (unsigned)((uintptr_t)logits & 15u) : 0u;
+    ctx->last_stride_mod = (unsigned)((row_stride_elems * (dtype == SR_DTYPE_BF16 ? 2 : 4)) & 15);
+    int rc = batch_upload_impl(ctx->tmp_batch, rows, vocab, params, hist_ids, hist_offsets, bias_ids, bias_vals, bias_offsets, allow_mask,
+                               mask_stride_words, mask_active, uniforms, uniforms ? 1 : 0, false, false, nullptr, true);
     const void* dev = nullptr;
-    rc = stage_logits(ctx, logits, dtype, logits_on_device, rows, vocab, row_stride_elems, &dev);
-    if (rc != SR_OK) return rc;
-    SR_HIP(ctx, ctx->out_tokens.reserve((size_t)rows * sizeof(int32_t), ctx->stream));
-    SR_HIP(ctx, ctx->out_flags.reserve((size_t)rows * sizeof(uint32_t), ctx->stream));
-    rc = sr_sample_launch(ctx, ctx->tmp_batch, dev, dtype, row_stride_elems, ctx->out_tokens.as<int32_t>(),
-                          ctx->out_flags.as<uint32_t>());
-    if (rc != SR_OK) return rc;
-    SR_HIP(ctx, hipMemcpyAsync(out_tokens, ctx->out_tokens.p, (size_t)rows * sizeof(int32_t), hipMemcpyDeviceToHost,
-                               ctx->stream));
-    std::vector<uint32_t> flags((size_t)rows);
-    SR_HIP(ctx, hipMemcpyAsync(flags.data(), ctx->out_flags.p, (size_t)rows * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                               ctx->stream));
-    SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (rc == SR_OK) rc = stage_logits(ctx, logits, dtype, logits_on_device, rows, vocab, row_stride_elems, &dev);
+    // the kernels write tokens and flags straight into pinned memory
+    const size_t n = (size_t)rows;
+    if (rc == SR_OK) {
+        hipError_t e = ctx->results.reserve(2 * n);
+        if (e != hipSuccess) rc = sr_fail_hip(ctx, e, "pinned memory for the results");
+    }
+    if (rc == SR_OK) {
+        ctx->results.arm(0, n, SR_NO_TOKEN);
+        ctx->results.arm(n, n, SR_NO_FLAGS);
+        rc = sr_sample_launch(ctx, ctx->tmp_batch, dev, dtype, row_stride_elems, (int32_t*)ctx->results.p, ctx->results.p + n);
+    }
+    if (rc != SR_OK) {
+        (void)hipStreamSynchronize(ctx->stream);  // (what was enqueued reads the batch's pinned memory)
+        return rc;
+    }
+    SR_HIP(ctx, ctx->results.wait(0, n, SR_NO_TOKEN, ctx->stream));
+    SR_HIP(ctx, ctx->results.wait(n, n, SR_NO_FLAGS, ctx->stream));
     // rows that overflowed the selection kernel's row tail (thousands of equal logits at the cut) take the sort path
     std::vector<int32_t> redo;
     for (int32_t r = 0; r < rows; r++)
-        if (flags[(size_t)r] & SR_KFLAG_UNSUPPORTED) redo.push_back(r);
+        if (ctx->results.p[n + (size_t)r] & SR_KFLAG_UNSUPPORTED) redo.push_back(r);
     if (!redo.empty()) {
         rc = sr_resample_rows_launch(ctx, ctx->tmp_batch, dev, dtype, row_stride_elems, redo.data(), (int32_t)redo.size(),
-                                     ctx->out_tokens.as<int32_t>(), ctx->out_flags.as<uint32_t>());
+                                     (int32_t*)ctx->results.p, ctx->results.p + n);
         if (rc != SR_OK) return rc;
-        SR_HIP(ctx, hipMemcpyAsync(out_tokens, ctx->out_tokens.p, (size_t)rows * sizeof(int32_t), hipMemcpyDeviceToHost,
-                                   ctx->stream));
-        SR_HIP(ctx, hipMemcpyAsync(flags.data(), ctx->out_flags.p, (size_t)rows * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                                   ctx->stream));
         SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
     }
-    if (out_flags) memcpy(out_flags, flags.data(), (size_t)rows * sizeof(uint32_t));
+    memcpy(out_tokens, ctx->results.p, n * sizeof(int32_t));
+    if (out_flags) memcpy(out_flags, ctx->results.p + n, n * sizeof(uint32_t));
     return SR_OK;
 }
 
@@ -1304,20 +1370,17 @@ static SrArgmaxArgs argmax_args(sr_ctx* ctx, const void* logits_dev, int dtype, 
     return a;
 }
 
-int sr_argmax_rows_launch(sr_ctx* ctx, const void* logits_dev, int dtype, int32_t rows, int32_t vocab,
-                          int64_t row_stride_elems, int32_t* out_idx_dev, float* out_val_dev)
+// (arguments checked, the device current; host: pinned memory that gets the results as well, or null)
+static int argmax_enqueue(sr_ctx* ctx, const void* logits_dev, int dtype, int32_t rows, int32_t vocab, int64_t row_stride_elems,
+                          int32_t* out_idx_dev, float* out_val_dev, unsigned long long* host)
 {
-    if (!ctx) return SR_ERR_NULL_ARGUMENT;
-    if (rows == 0) return SR_OK;
-    int rc = argmax_check(ctx, logits_dev, dtype, rows, vocab, row_stride_elems, out_idx_dev);
-    if (rc != SR_OK) return rc;
-    SR_HIP(ctx, hipSetDevice(ctx->device));
     // slots and counters: zero when allocated, and every launch leaves them zero again
     SR_HIP(ctx, ctx->argmax_best.reserve((size_t)rows * sizeof(unsigned long long), ctx->stream, true));
     SR_HIP(ctx, ctx->argmax_done.reserve((size_t)rows * sizeof(uint32_t), ctx->stream, true));
     SrArgmaxArgs a = argmax_args(ctx, logits_dev, dtype, rows, vocab, row_stride_elems, out_idx_dev, out_val_dev);
     a.best = ctx->argmax_best.as<unsigned long long>();
     a.done = ctx->argmax_done.as<uint32_t>();
+    a.host = host;
     // (a launch that failed may have left slots and counters that are not zero: every later call would be wrong, silently)
     if (ctx->argmax_scratch_dirty) {
         SR_HIP(ctx, hipMemsetAsync(ctx->argmax_best.p, 0, ctx->argmax_best.cap, ctx->stream));
@@ -1327,6 +1390,42 @@ int sr_argmax_rows_launch(sr_ctx* ctx, const void* logits_dev, int dtype, int32_
     const hipError_t e = sr_launch_argmax_rows(a, false, ctx->stream);
     if (e != hipSuccess) ctx->argmax_scratch_dirty = true;
     SR_HIP(ctx, e);
+    return SR_OK;
+}
+
+int sr_argmax_rows_launch(sr_ctx* ctx, const void* logits_dev, int dtype, int32_t rows, int32_t vocab,
+                          int64_t row_stride_elems, int32_t* out_idx_dev, float* out_val_dev)
+{
+    if (!ctx) return SR_ERR_NULL_ARGUMENT;
+    if (rows == 0) return SR_OK;
+    int rc = argmax_check(ctx, logits_dev, dtype, rows, vocab, row_stride_elems, out_idx_dev);
+    if (rc != SR_OK) return rc;
+    SR_HIP(ctx, hipSetDevice(ctx->device));
+    return argmax_enqueue(ctx, logits_dev, dtype, rows, vocab, row_stride_elems, out_idx_dev, out_val_dev, nullptr);
+}
+
+int sr_argmax_rows_both(sr_ctx* ctx, const void* logits_dev, int dtype, int32_t rows, int32_t vocab, int64_t row_stride_elems,
+                        int32_t* out_idx_dev, float* out_val_dev, int32_t* out_idx, float* out_val)
+{
+    if (!ctx) return SR_ERR_NULL_ARGUMENT;
+    if (rows == 0) return SR_OK;
+    int rc = argmax_check(ctx, logits_dev, dtype, rows, vocab, row_stride_elems, out_idx);
+    if (rc != SR_OK) return rc;
+    SR_HIP(ctx, hipSetDevice(ctx->device));
+    HostResults& res = ctx->results;
+    const size_t n = (size_t)rows;
+    SR_HIP(ctx, res.reserve(2 * n));
+    res.arm(0, n, SR_NO_TOKEN, 2);
+    rc = argmax_enqueue(ctx, logits_dev, dtype, rows, vocab, row_stride_elems, out_idx_dev, out_val_dev, (unsigned long long*)res.p);
+    if (rc != SR_OK) {
+        (void)hipStreamSynchronize(ctx->stream);
+        return rc;
+    }
+    SR_HIP(ctx, res.wait(0, n, SR_NO_TOKEN, ctx->stream, 2));
+    for (size_t r = 0; r < n; r++) {
+        out_idx[r] = (int32_t)res.p[2 * r];
+        if (out_val) memcpy(&out_val[r], &res.p[2 * r + 1], sizeof(float));
+    }
     return SR_OK;
 }
 
@@ -1369,16 +1468,9 @@ int sr_argmax_rows(sr_ctx* ctx, const void* logits, int dtype, int logits_on_dev
         int rc = stage_logits(ctx, logits, dtype, logits_on_device, rows, vocab, row_stride_elems, &dev);
         if (rc != SR_OK) return rc;
     }
-    SR_HIP(ctx, ctx->out_tokens.reserve((size_t)rows * sizeof(int32_t), ctx->stream));
-    SR_HIP(ctx, ctx->out_val.reserve((size_t)rows * sizeof(float), ctx->stream));
-    int rc = sr_argmax_rows_launch(ctx, dev, dtype, rows, vocab, row_stride_elems, ctx->out_tokens.as<int32_t>(),
-                                   ctx->out_val.as<float>());
-    if (rc != SR_OK) return rc;
-    SR_HIP(ctx, hipMemcpyAsync(out_idx, ctx->out_tokens.p, (size_t)rows * sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-    if (out_val)
-        SR_HIP(ctx, hipMemcpyAsync(out_val, ctx->out_val.p, (size_t)rows * sizeof(float), hipMemcpyDeviceToHost, ctx->stream));
-    SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return SR_OK;
+    const int rc = sr_argmax_rows_both(ctx, dev, dtype, rows, vocab, row_stride_elems, nullptr, nullptr, out_idx, out_val);
+    if (rc != SR_OK) (void)hipStreamSynchronize(ctx->stream);  // (the copy of host logits may still be reading the caller's memory)
+    return rc;
 }
 
 int sr_pack_allow_mask(const float* masked_logits, int32_t vocab, uint32_t* out_words)

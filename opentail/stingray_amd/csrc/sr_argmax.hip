@@ -128,8 +128,12 @@ template <int ES, bool kVec> __global__ __launch_bounds__(kThreads) void k_argma
         __hip_atomic_store(&a.done[row], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     const int idx = best ? (int)(0xffffffffu - (uint32_t)(best & 0xffffffffull)) : 0;  // empty row -> 0
-    a.out_idx[row] = idx;
-    if (a.out_val) a.out_val[row] = a.vocab > 0 ? load_elem<ES>(rowp, idx) : 0.0f;  // the original bits, not a decode
+    const float val = a.vocab > 0 ? load_elem<ES>(rowp, idx) : 0.0f;  // the original bits, not a decode
+    if (a.host)  // one store, seen by the host as a whole
+        __hip_atomic_store(&a.host[row], ((unsigned long long)sr_f2u(val) << 32) | (unsigned long long)(uint32_t)idx, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+    if (a.out_idx) a.out_idx[row] = idx;
+    if (a.out_val) a.out_val[row] = val;
 }
 
 #ifdef SR_TEST_HOOKS

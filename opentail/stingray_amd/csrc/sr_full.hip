@@ -40,6 +40,7 @@ struct FullSmem {
     float ckpt[kCkpt];  // running sum behind every tile of a row's exact sum (SeqMarks)
     float segst[SR_SEG_MAX];  // running sum behind every segment of a prepared row (seg_walk)
     uint32_t segbc[4];
+    double u;  // the row's uniform (k_full_row)
     unsigned long long sortbuf[kSmall];
     float sprob[kSmall];
     uint32_t tags[kSmall];
@@ -1842,7 +1843,7 @@ __device__ __forceinline__ void finish_from_ordered_list(const SrFullArgs& a, fl
         const float inv = scale ? __fdiv_rn(1.0f, sum) : 1.0f;
         if (a.mode != 0 && scale) row_pass<true>(p, n, [&](float x, int) -> float { return __fmul_rn(x, inv); });
         if (a.mode != 1 && tid == 0) {
-            const float r = __double2float_rn(a.uniforms[(size_t)row * a.uniforms_per_row]);
+            const float r = __double2float_rn(sm.u);
             int token = n - 1;
             if (!(r > 0.0f)) {
                 token = 0;  // the running sum starts at p[0] >= 0: index 0 reaches a target of zero whatever it holds
@@ -1895,7 +1896,7 @@ __device__ __forceinline__ void finish_from_ordered_list(const SrFullArgs& a, fl
     const float inv = scale ? __fdiv_rn(1.0f, sum) : 1.0f;
     if (a.mode != 0 && scale) row_pass<true>(p, n, [&](float x, int) -> float { return __fmul_rn(x, inv); });
     if (a.mode == 1) return;
-    const float r = __double2float_rn(a.uniforms[(size_t)row * a.uniforms_per_row]);
+    const float r = __double2float_rn(sm.u);
     int token = n - 1;
     bool done = false;  // (what wave 0 knows)
     if (!(r > 0.0f)) {
@@ -2453,7 +2454,7 @@ __device__ __forceinline__ int nucleus_from_histogram(const SrFullArgs& a, float
         __syncthreads();
         normalize_row(w, n, sm);
         if (a.mode != 1) {
-            const int token = draw_from_row(w, n, a.uniforms[(size_t)row * a.uniforms_per_row], sm);
+            const int token = draw_from_row(w, n, sm.u, sm);
             if (tid == 0 && a.out_tokens) a.out_tokens[row] = token;
         }
         return kNucleusDone;
@@ -2605,6 +2606,9 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
         return;
     }
 
+    // The uniform may lie in host memory, a trip over the bus: one thread asks for it now and hands it on when the sum is there.
+    double u_row = 0.0;
+    if (tid == kT - 1 && a.mode != 1) u_row = a.uniforms[(size_t)row * a.uniforms_per_row];
     {
         FPROF(a, slot, 0);
         // Softmax (Sampler.cs:448-472): the maximum and e = expf(x - max) were computed by the kernels before
@@ -2622,6 +2626,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
             const float uni = n > 0 ? __fdiv_rn(1.0f, (float)n) : 0.0f;
             row_pass<true>(p, n, [&](float, int) -> float { return uni; });
             flags |= SR_KFLAG_DEGENERATE;
+            if (tid == kT - 1) sm.u = u_row;
             __syncthreads();
         } else {
             if (row_edits_on_the_fly(rd, a) && !a.seg_func) {
@@ -2702,6 +2707,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
             } else {
                 sum = seq_sum_row<false>(p, n, 0.0f, 0.0f, &dummy, sm);
             }
+            if (tid == kT - 1) sm.u = u_row;
             __syncthreads();
             const int n_watched = watch_min_p ? (int)sm.bc[4] : -1;
             const bool from_watch = n_watched >= 0 && n_watched <= kSmall;  // (else the row is read again, as before)
@@ -3077,7 +3083,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     FPROF(a, slot, 8);
     int token = -1;
     if (a.mode != 1) {
-        token = draw_from_row(p, n, a.uniforms[(size_t)row * a.uniforms_per_row], sm);
+        token = draw_from_row(p, n, sm.u, sm);
         if (tid == 0 && a.out_tokens) a.out_tokens[row] = token;
     }
     FPROF(a, slot, 9);

@@ -122,7 +122,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             }
         }
     }
-    a.uniforms = b->d_uniforms.as<double>();
+    a.uniforms = sr_batch_uniforms(b);
     a.uniforms_per_row = b->upr;
     a.out_tokens = out_tokens_dev;
     a.out_flags = out_flags_dev;
@@ -166,7 +166,7 @@ int identity_list(sr_ctx* ctx, int rows, const int32_t** out)
 int upload_uniforms(sr_ctx* ctx, const double* uniforms, int rows, const double** dev)
 {
     const size_t bytes = (size_t)rows * sizeof(double);
-    SR_HIP(ctx, ctx->uni_ring.begin(bytes + 256, ctx->stream, 0, ctx->stream_epoch));
+    SR_HIP(ctx, ctx->uni_ring.begin(ctx->pinned, bytes + 256, ctx->stream, 0, ctx->stream_epoch));
     const void* at = ctx->uni_ring.put(uniforms, bytes);
     if (!at) return sr_fail(ctx, SR_ERR_OUT_OF_MEMORY, "no pinned memory for the uniforms");
     *dev = (const double*)at;
@@ -217,7 +217,7 @@ int sr_wide_rows_launch(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev,
     a.sort_vals_in = ctx->sort_v0.as<int32_t>();
     a.wide_ids = ctx->sort_v1.as<int32_t>();
     a.sort_stride = stride;
-    a.uniforms = b->d_uniforms.as<double>();
+    a.uniforms = sr_batch_uniforms(b);
     a.uniforms_per_row = b->upr;
     a.out_tokens = out_tokens_dev;
     a.out_flags = out_flags_dev;
@@ -492,7 +492,7 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     a.target_logits = target_logits_dev;
     a.draft_probs = draft_probs_dev;
     a.draft_tokens = draft_tokens_dev;
-    a.uniforms = b->d_uniforms.as<double>();
+    a.uniforms = sr_batch_uniforms(b);
     a.uniforms_per_row = b->upr;
     a.out_accepted = out_accepted_dev;
     a.out_tokens = out_tokens_dev;

@@ -43,6 +43,43 @@ struct DeviceBuf {
     template <typename T> T* as() const { return (T*)p; }
 };
 
+// Pinned host memory takes tens of microseconds to allocate and to free: a batch that is destroyed leaves its blocks to its
+// context (a few of them, the rest is freed), and the next batch starts with those.  The context's calls never overlap
+// and a batch waits for the stream before it gives its memory back.
+struct PinnedPool {
+    struct Block { char* p; size_t cap; };
+    std::vector<Block> free_blocks;
+    static constexpr size_t kMostBlocks = 16, kMostBytes = (size_t)1 << 20;  // ... of at most a megabyte each
+    // a block of at least `bytes`; *cap = what it holds
+    hipError_t take(size_t bytes, char** p, size_t* cap)
+    {
+        size_t best = free_blocks.size();
+        for (size_t i = 0; i < free_blocks.size(); i++)
+            if (free_blocks[i].cap >= bytes && (best == free_blocks.size() || free_blocks[i].cap < free_blocks[best].cap)) best = i;
+        if (best < free_blocks.size()) {
+            *p = free_blocks[best].p;
+            *cap = free_blocks[best].cap;
+            free_blocks.erase(free_blocks.begin() + (ptrdiff_t)best);
+            return hipSuccess;
+        }
+        hipError_t e = hipHostMalloc((void**)p, bytes, hipHostMallocDefault);
+        if (e != hipSuccess) { *p = nullptr; *cap = 0; return e; }
+        *cap = bytes;
+        return hipSuccess;
+    }
+    void give(char* p, size_t cap)
+    {
+        if (!p) return;
+        if (cap <= kMostBytes && free_blocks.size() < kMostBlocks) free_blocks.push_back(Block{p, cap});
+        else (void)hipHostFree(p);
+    }
+    void release()
+    {
+        for (Block& b : free_blocks) (void)hipHostFree(b.p);
+        free_blocks.clear();
+    }
+};
+
 // Pinned host memory that a batch packs its small uploads into, so that the copies to the device are truly
 // asynchronous and the upload need not wait for them.  An event marks the end of the copies of one upload; the next
 // upload waits for it before it overwrites the memory.
@@ -51,22 +88,22 @@ struct HostStage {
     size_t cap = 0, used = 0, wanted = 0;
     hipEvent_t ev = nullptr;
     bool busy = false;
-    hipError_t begin()
+    // `expect`: about what the upload will pack (an upload that does not fit sends pieces unpacked and waits)
+    hipError_t begin(PinnedPool& pool, size_t expect = 0)
     {
+        wanted = std::max(wanted, expect);
         if (busy) {
             hipError_t e = hipEventSynchronize(ev);
             if (e != hipSuccess) return e;
             busy = false;
         }
         if (wanted > cap) {
-            if (p) (void)hipHostFree(p);
+            pool.give(p, cap);
             p = nullptr;
             cap = 0;
-            // roomy (a decode loop's edit lists grow; an upload that does not fit sends pieces unpacked and waits)
-            const size_t want = 4 * wanted + 65536;
-            hipError_t e = hipHostMalloc((void**)&p, want, hipHostMallocDefault);
-            if (e != hipSuccess) { p = nullptr; return e; }
-            cap = want;
+            // (roomy: a decode loop's edit lists grow)
+            hipError_t e = pool.take(4 * wanted + 65536, &p, &cap);
+            if (e != hipSuccess) return e;
         }
         used = wanted = 0;
         return hipSuccess;
@@ -92,9 +129,9 @@ struct HostStage {
         if (e == hipSuccess) busy = true;
         return e;
     }
-    void release()
+    void release(PinnedPool& pool)
     {
-        if (p) (void)hipHostFree(p);
+        pool.give(p, cap);
         if (ev) (void)hipEventDestroy(ev);
         p = nullptr;
         ev = nullptr;
@@ -110,7 +147,7 @@ struct HostStage {
 // waits for the one recorded when the other half was left, many steps ago.
 struct HostRing {
     char* p = nullptr;
-    size_t half = 0, used = 0;
+    size_t cap = 0, half = 0, used = 0;
     int cur = 0;
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool pending[2] = {false, false};
@@ -120,28 +157,33 @@ struct HostRing {
     // room for `need` bytes in the present half (its pieces are handed out by put)
     // (want_half: what a half should hold when the ring has to be made or made again anyway)
     // (owner_epoch: the context counts its changes of stream, and waits for the stream it leaves at every one of them)
-    hipError_t begin(size_t need, hipStream_t st, size_t want_half = 0, uint32_t owner_epoch = 0)
+    // (keep_newest: the newest piece may be read by launches that are still to come -- on the new stream as well --, so
+    // a change of streams does not start the half over)
+    hipError_t begin(PinnedPool& pool, size_t need, hipStream_t st, size_t want_half = 0, uint32_t owner_epoch = 0, bool keep_newest = false)
     {
         hipError_t e = hipSuccess;
         if (dirty && st != last) {  // the caller changed streams: nothing orders the old stream's readers before new events
             // When the context itself made the change it has waited for the old stream already -- which the caller may
             // have destroyed since: it is not touched again.
             if (owner_epoch == epoch && (e = hipStreamSynchronize(last)) != hipSuccess) return e;
-            pending[0] = pending[1] = dirty = false;
-            used = 0;
+            pending[0] = pending[1] = false;
+            if (!keep_newest) {
+                dirty = false;
+                used = 0;
+            }
         }
         epoch = owner_epoch;
         last = st;
         if (need > half) {  // grow: nothing may still be reading the old memory
             if (dirty && (e = hipStreamSynchronize(st)) != hipSuccess) return e;
-            if (p) (void)hipHostFree(p);
+            pool.give(p, cap);
             p = nullptr;
-            half = used = 0;
+            cap = half = used = 0;
             pending[0] = pending[1] = dirty = false;
             // (room for many calls of the usual size; a call that needs much -- every row of a batch moving its edits at
             // once -- gets room for two of its kind: pinned memory is slow to allocate)
             const size_t want = std::max(want_half, (need <= 65536 ? 16 * need : 2 * need) + 65536);
-            if ((e = hipHostMalloc((void**)&p, 2 * want, hipHostMallocDefault)) != hipSuccess) { p = nullptr; return e; }
+            if ((e = pool.take(2 * want, &p, &cap)) != hipSuccess) return e;
             half = want;
             cur = 0;
         }
@@ -170,17 +212,58 @@ struct HostRing {
         dirty = true;
         return dst;
     }
-    void release()  // (the owner has waited for the stream)
+    void release(PinnedPool& pool)  // (the owner has waited for the stream)
     {
-        if (p) (void)hipHostFree(p);
+        pool.give(p, cap);
         for (int h = 0; h < 2; h++)
             if (ev[h]) (void)hipEventDestroy(ev[h]);
         p = nullptr;
         ev[0] = ev[1] = nullptr;
-        half = used = 0;
+        cap = half = used = 0;
         pending[0] = pending[1] = dirty = false;
     }
 };
+
+// Where the kernels of a call with host results leave them: pinned host memory, one 32-bit word per result.  The caller
+// puts a value there that no kernel writes and looks until it is gone, which takes a microsecond or two from the store;
+// a wait for the stream and a copy command per array took 14 us each.
+struct HostResults {
+    uint32_t* p = nullptr;
+    size_t cap = 0;
+    hipError_t reserve(size_t words)  // (nothing is in flight between calls: every call waits for its results)
+    {
+        if (words <= cap) return hipSuccess;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        cap = 0;
+        const size_t want = std::max(words, (size_t)2048);
+        hipError_t e = hipHostMalloc((void**)&p, want * sizeof(uint32_t), hipHostMallocCoherent | hipHostMallocMapped);
+        if (e != hipSuccess) { p = nullptr; return e; }
+        cap = want;
+        return hipSuccess;
+    }
+    void arm(size_t first, size_t n, uint32_t none, size_t step = 1) { for (size_t i = 0; i < n; i++) p[first + i * step] = none; }
+    // until none of the words is `none` any more; a stream that takes long (the forward pass in front) is waited for
+    hipError_t wait(size_t first, size_t n, uint32_t none, hipStream_t st, size_t step = 1) const
+    {
+        constexpr int kSpins = 20000;  // about a millisecond
+        size_t i = 0;
+        for (int spin = 0; spin < kSpins; spin++) {
+            while (i < n && __atomic_load_n(p + first + i * step, __ATOMIC_ACQUIRE) != none) i++;
+            if (i == n) return hipSuccess;
+            __builtin_ia32_pause();
+        }
+        return hipStreamSynchronize(st);
+    }
+    void release()
+    {
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        cap = 0;
+    }
+};
+#define SR_NO_TOKEN 0x80000000u  // ... for a token or an index (both -1 and above)
+#define SR_NO_FLAGS 0x7fffffffu  // ... for a row's flags (no row carries them all)
 
 struct sr_ctx {
     int device = 0;
@@ -199,7 +282,7 @@ struct sr_ctx {
     uint32_t full_seq = 0;   // number of the last launch of that path (SrFullState::maxkey)
     DeviceBuf host_logits;   // staging for host-resident logits
     DeviceBuf stage_probs;   // staging for host-resident distributions
-    DeviceBuf out_tokens, out_flags, out_val;
+    DeviceBuf out_tokens;
     HostRing uni_ring;       // uniforms of the calls that take them as host arrays and enqueue a kernel (read in place)
     DeviceBuf sort_k0, sort_v0, sort_v1;  // sort segments of rows: top-p survivors, wide top-k rows (and their token ids)
     DeviceBuf ident;         // identity row list
@@ -213,8 +296,12 @@ struct sr_ctx {
     DeviceBuf full_row_sync;
     DeviceBuf full_seg_func, full_seg_ms, full_watch, full_watch_cnt, full_seg_keys;  // ... of the full-vocabulary path's denominators
     sr_batch* tmp_batch = nullptr;
+    PinnedPool pinned;
+    HostResults results;
     unsigned long long* prof = nullptr;  // test hook: phase timestamps of the selection kernel
-    int last_epv = 4;                    // vector width of the last launch: what an upload builds scan masks for
+    // vector width and alignment of the last launch's logits: what an upload builds scan masks for
+    int last_epv = 4;
+    unsigned last_base_mod = 0, last_stride_mod = 0;
     // Registered allow-masks (sr_mask_register): one device array of `pool_cap` slots of `pool_words` words each, the
     // id of a mask is its slot.  One vocabulary size per context at a time.
     DeviceBuf mask_pool;
@@ -263,7 +350,12 @@ struct sr_batch {
     unsigned mask_pool_gen = 0;          // ... the pool's generation at that time
     int32_t max_sel = 0;
     HostStage stage;
-    HostRing patch_ring;  // the lists of sr_batch_append_tokens          // pinned copies of what an upload sends to the device
+    HostRing patch_ring;  // the lists of sr_batch_append_tokens
+    // The uniforms of steps after the upload (sr_batch_set_uniforms, sr_batch_append_tokens): pieces of pinned memory that
+    // the sampling kernels read in place, or null while d_uniforms holds the present ones.  A piece is written over only
+    // by newer ones, behind an event of the launches that read it.
+    HostRing uni_ring;
+    const double* uni_now = nullptr;
     std::vector<SrCopySeg> segs;  // ... the pieces that are packed and not yet sent
     bool upload_must_wait = false;  // some copy of the running upload reads pageable memory directly
     // geometry the scan masks were built with (sr_batch_append_tokens clears single bits in place)
@@ -310,6 +402,8 @@ int sr_batch_masks_valid(sr_ctx* ctx, const sr_batch* b, const char* who);
 // where a batch's allow-masks lie: its own upload, or the context's registered masks (sr_api.cpp)
 const uint32_t* sr_batch_mask_ptr(const sr_batch* b);
 int64_t sr_batch_mask_stride(const sr_batch* b);
+// ... and its uniforms
+const double* sr_batch_uniforms(const sr_batch* b);
 
 // Full-vocabulary rows of a batch (sr_full_host.cpp).  mode: 0 = sample, 1 = build distribution,
 // 2 = build distribution and sample from it.

@@ -79,7 +79,7 @@ hipError_t sr_launch_topk(const SrTopkArgs& a, int n_rows, hipStream_t stream);
 // Builds scan row i for descs[i]; base_addr / stride_bytes are those of the logits the mask is used with
 // (they decide where a row starts inside its first 16-byte vector), epv = 4 (fp32) or 8 (bf16).
 // all pieces of an upload in one launch: segs (itself in pinned host memory) lists n pieces
-hipError_t sr_launch_scatter(const SrCopySeg* segs, int n, hipStream_t stream);
+hipError_t sr_launch_scatter(const SrCopyTable& t, hipStream_t stream);
 // scan_ids: the n_scan scan rows to build (NULL: rows 0 .. n_scan - 1)
 hipError_t sr_launch_pack_allow_mask(const void* logits, int dtype, int rows, int vocab, int64_t row_stride, uint32_t* out,
                                      int64_t out_stride, hipStream_t stream);
@@ -88,19 +88,19 @@ hipError_t sr_launch_pack_allow_mask(const void* logits, int dtype, int rows, in
 #define SR_MASK_AND_MAX 8
 hipError_t sr_launch_mask_and(uint32_t* pool, int64_t pool_words, const int32_t* ids_host, int n, int dst, int vocab, uint32_t* any,
                               hipStream_t stream);
+// pieces: when not null, the pieces of an upload are put in their places by further workgroups of the same launch (descs, rows
+// and edits are then where the host packed them)
 hipError_t sr_launch_build_scan_mask(const SrScanDesc* descs, const int32_t* scan_ids, int n_scan, const SrRow* rows, const SrEdit* edits,
                                      const uint32_t* mask, int64_t mask_stride, uint32_t* scan_mask, int64_t scan_stride,
                                      int vocab, int epv, int chunks, int chunk_vecs, unsigned long long base_addr,
-                                     long long stride_bytes, hipStream_t stream);
+                                     long long stride_bytes, const SrCopyTable* pieces, hipStream_t stream);
 
 // What one appended token per row changes (sr_batch_append_tokens): history length and edit count of n_rowp rows,
-// n_edits whole edits, n_clears keep-bits of scan masks built with the given geometry, n_uni uniforms.  The lists
-// may lie in pinned host memory.
+// n_edits whole edits, n_clears keep-bits of scan masks built with the given geometry.  The lists may lie in pinned host memory.
 hipError_t sr_launch_apply_patches(SrRow* rows, const SrRowPatch* rp, int n_rowp, SrEdit* edits, const SrEditPatch* ep,
                                    int n_edits, const SrMaskClear* mc, int n_clears, uint32_t* scan_mask,
                                    int64_t scan_stride, int epv, int chunk_vecs, unsigned long long base_addr,
-                                   long long stride_bytes, double* uni_dst, const double* uni_src, int n_uni,
-                                   hipStream_t stream);
+                                   long long stride_bytes, hipStream_t stream);
 
 struct SrArgmaxArgs {
     const void* logits;
@@ -115,8 +115,9 @@ struct SrArgmaxArgs {
     // the launch and zero again after it
     unsigned long long* best;
     uint32_t* done;
-    int32_t* out_idx;
+    int32_t* out_idx;         // may be null
     float* out_val;           // may be null
+    unsigned long long* host; // pinned host memory, or null: value bits << 32 | index of every row
 };
 // fills chunks, chunk_len and vec from the other fields
 void sr_argmax_plan(SrArgmaxArgs& a, int cu_count);

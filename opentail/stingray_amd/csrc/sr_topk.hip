@@ -2189,14 +2189,39 @@ __global__ __launch_bounds__(kThreads, (kKept || kRoomy) ? 2 : 4) void k_topk_ro
 // lies inside the row, its allow-mask (if any) admits it and, for rows whose tail fetches the history logits by
 // id, it is not a history id.  One workgroup per (scan row, chunk): the words are built in LDS, the history ids
 // that fall into the chunk are cleared there, then the words are written out.
+// The pieces of a batch upload lie where the host packed them (pinned host memory, over the bus) and are written where
+// they belong by one launch (a copy command per piece cost the stream about 20 us whatever its size).  Sources and
+// destinations are 16-byte aligned.  `block` of `blocks` workgroups of kBlock threads on a piece; the list of pieces
+// comes in the kernel's arguments, so that a piece is one trip over the bus.
+template <int kBlock>
+__device__ __forceinline__ void copy_piece(const SrCopySeg& s, int block, int blocks)
+{
+    const unsigned long long n16 = s.bytes / 16;
+    const uint4* src = (const uint4*)s.src;
+    uint4* dst = (uint4*)s.dst;
+    for (unsigned long long i = (unsigned long long)block * kBlock + threadIdx.x; i < n16; i += (unsigned long long)blocks * kBlock)
+        dst[i] = src[i];
+    if (block == 0) {
+        const unsigned long long done = n16 * 16;
+        if (done + threadIdx.x < s.bytes) ((char*)s.dst)[done + threadIdx.x] = ((const char*)s.src)[done + threadIdx.x];
+    }
+}
+
+// With pieces.n > 0 the workgroups behind the scan_blocks first ones put the pieces of an upload in their places, one
+// workgroup to a piece (small uploads: see prepare_scan).
 __global__ __launch_bounds__(kThreads) void k_build_scan_mask(const SrScanDesc* descs, const int32_t* scan_ids,
                                                               const SrRow* rows, const SrEdit* edits,
                                                               const uint32_t* mask, int64_t mask_stride, uint32_t* scan_mask,
                                                               int64_t scan_stride, int vocab, int epv, int es, int chunks,
                                                               int chunk_vecs, int vecs_per_thread,
-                                                              unsigned long long base_addr, long long stride_bytes)
+                                                              unsigned long long base_addr, long long stride_bytes,
+                                                              int scan_blocks, SrCopyTable pieces)
 {
     __shared__ uint32_t words[kThreads * SR_TK_MASK_WORDS];
+    if ((int)blockIdx.x >= scan_blocks) {
+        copy_piece<kThreads>(pieces.seg[(int)blockIdx.x - scan_blocks], 0, 1);
+        return;
+    }
     const int nth = blockIdx.x / chunks, c = blockIdx.x - nth * chunks;
     const int srow = scan_ids ? scan_ids[nth] : nth;  // a list of scan rows to build again, or all of them
     const int t = threadIdx.x;
@@ -2248,23 +2273,20 @@ __global__ __launch_bounds__(kThreads) void k_build_scan_mask(const SrScanDesc* 
 
 // Applies what one appended token per row changes: history length and edit count of rows, whole edits at given
 // positions of the edit array, single keep-bits of scan-mask rows cleared for ids that entered a history (same
-// element -> bit mapping as above), and the uniforms of the next step.  The lists are read where the host wrote
-// them (pinned host memory).
+// element -> bit mapping as above).  The lists are read where the host wrote them (pinned host memory).
 __global__ __launch_bounds__(256) void k_apply_patches(SrRow* rows, const SrRowPatch* rp, int n_rowp, SrEdit* edits,
                                                        const SrEditPatch* ep, int n_edits, const SrMaskClear* mc,
                                                        int n_clears, uint32_t* scan_mask, int64_t scan_stride, int epv,
                                                        int es, int chunk_vecs, unsigned long long base_addr,
-                                                       long long stride_bytes, double* uni_dst, const double* uni_src,
-                                                       int n_uni)
+                                                       long long stride_bytes)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    // The lists lie in pinned host memory: every read is a trip over the bus.  All four are read first, without
+    // The lists lie in pinned host memory: every read is a trip over the bus.  All three are read first, without
     // conditions (a thread past a list's end reads the list's last entry, or whatever stands at the head of an empty
     // list's 256 bytes), so that the trips run side by side; then the changes are applied.
     const SrRowPatch r = rp[min(i, max(n_rowp, 1) - 1)];
     const SrEditPatch e = ep[min(i, max(n_edits, 1) - 1)];
     const SrMaskClear m = mc[min(i, max(n_clears, 1) - 1)];
-    const double u = uni_src[min(i, max(n_uni, 1) - 1)];
     if (i < n_rowp) {
         rows[r.row].n_prev = r.n_prev;
         rows[r.row].edit_cnt = r.edit_cnt;
@@ -2283,25 +2305,10 @@ __global__ __launch_bounds__(256) void k_apply_patches(SrRow* rows, const SrRowP
         atomicAnd(&scan_mask[(size_t)m.scan_row * scan_stride + ((size_t)c * kThreads + tt) * SR_TK_MASK_WORDS + (b >> 5)],
                   ~(1u << (b & 31)));
     }
-    if (i < n_uni) uni_dst[i] = u;
 }
 
-// The pieces of a batch upload, read where the host packed them (pinned host memory, over the bus) and written
-// where they belong: one launch instead of one copy command per piece (each of which costs the stream about 20 us
-// whatever its size).  Sources and destinations are 16-byte aligned.
-__global__ __launch_bounds__(256) void k_scatter(const SrCopySeg* segs)
-{
-    const SrCopySeg s = segs[blockIdx.y];
-    const unsigned long long n16 = s.bytes / 16;
-    const uint4* src = (const uint4*)s.src;
-    uint4* dst = (uint4*)s.dst;
-    for (unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x; i < n16; i += (unsigned long long)gridDim.x * 256)
-        dst[i] = src[i];
-    if (blockIdx.x == 0) {
-        const unsigned long long done = n16 * 16;
-        if (done + threadIdx.x < s.bytes) ((char*)s.dst)[done + threadIdx.x] = ((const char*)s.src)[done + threadIdx.x];
-    }
-}
+// All pieces of an upload.
+__global__ __launch_bounds__(256) void k_scatter(SrCopyTable t) { copy_piece<256>(t.seg[blockIdx.y], (int)blockIdx.x, (int)gridDim.x); }
 
 // Packed allow-bits of rows that hold -inf where a token is not allowed (ITokenConstraint.Filter's output,
 // ITokenConstraint.cs:31-42): bit (i & 31) of word (i >> 5) = the row's element i is not -inf.  One wave per 64
@@ -2350,10 +2357,10 @@ __global__ __launch_bounds__(256) void k_mask_and(uint32_t* pool, int64_t pool_w
 }
 }  // namespace
 
-hipError_t sr_launch_scatter(const SrCopySeg* segs, int n, hipStream_t stream)
+hipError_t sr_launch_scatter(const SrCopyTable& t, hipStream_t stream)
 {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scatter, dim3(24, (unsigned)n), dim3(256), 0, stream, segs);
+    if (t.n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_scatter, dim3(24, (unsigned)t.n), dim3(256), 0, stream, t);
     return hipGetLastError();
 }
 
@@ -2381,14 +2388,13 @@ hipError_t sr_launch_mask_and(uint32_t* pool, int64_t pool_words, const int32_t*
 hipError_t sr_launch_apply_patches(SrRow* rows, const SrRowPatch* rp, int n_rowp, SrEdit* edits, const SrEditPatch* ep,
                                    int n_edits, const SrMaskClear* mc, int n_clears, uint32_t* scan_mask,
                                    int64_t scan_stride, int epv, int chunk_vecs, unsigned long long base_addr,
-                                   long long stride_bytes, double* uni_dst, const double* uni_src, int n_uni,
-                                   hipStream_t stream)
+                                   long long stride_bytes, hipStream_t stream)
 {
-    const int n = std::max(std::max(n_rowp, n_edits), std::max(n_clears, n_uni));
+    const int n = std::max(std::max(n_rowp, n_edits), n_clears);
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_apply_patches, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, rows, rp, n_rowp, edits, ep,
                        n_edits, mc, n_clears, scan_mask, scan_stride, epv, epv == 8 ? 2 : 4, chunk_vecs, base_addr,
-                       stride_bytes, uni_dst, uni_src, n_uni);
+                       stride_bytes);
     return hipGetLastError();
 }
 
@@ -2422,11 +2428,12 @@ hipError_t sr_launch_topk(const SrTopkArgs& a, int n_rows, hipStream_t stream)
 hipError_t sr_launch_build_scan_mask(const SrScanDesc* descs, const int32_t* scan_ids, int n_scan, const SrRow* rows, const SrEdit* edits,
                                      const uint32_t* mask, int64_t mask_stride, uint32_t* scan_mask, int64_t scan_stride,
                                      int vocab, int epv, int chunks, int chunk_vecs, unsigned long long base_addr,
-                                     long long stride_bytes, hipStream_t stream)
+                                     long long stride_bytes, const SrCopyTable* pieces, hipStream_t stream)
 {
     if (n_scan <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_build_scan_mask, dim3((unsigned)(n_scan * chunks)), dim3(kThreads), 0, stream, descs, scan_ids, rows, edits,
+    const SrCopyTable t = pieces ? *pieces : SrCopyTable{};
+    hipLaunchKernelGGL(k_build_scan_mask, dim3((unsigned)(n_scan * chunks + t.n)), dim3(kThreads), 0, stream, descs, scan_ids, rows, edits,
                        mask, mask_stride, scan_mask, scan_stride, vocab, epv, epv == 8 ? 2 : 4, chunks, chunk_vecs,
-                       epv == 8 ? SR_TK_VEC_BF16 : SR_TK_VEC, base_addr, stride_bytes);
+                       epv == 8 ? SR_TK_VEC_BF16 : SR_TK_VEC, base_addr, stride_bytes, n_scan * chunks, t);
     return hipGetLastError();
 }

@@ -58,6 +58,13 @@ struct SrCopySeg {
     void* dst;
     unsigned long long bytes;
 };
+// ... and all of them, in a kernel's arguments
+#define SR_COPY_SEGS 12
+struct SrCopyTable {
+    int32_t n;
+    int32_t pad;
+    SrCopySeg seg[SR_COPY_SEGS];
+};
 struct SrRowPatch {
     int32_t row;
     int32_t n_prev;

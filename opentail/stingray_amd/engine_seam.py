@@ -117,17 +117,11 @@ class RocmBatchSampler:
         prev = inputs.PreviousTokens
         if (same_rows_as_last_step and self._history_valid and rows == self._rows and vocab == self._vocab
                 and prev is not None and len(prev) == rows):
-            self._batch.append_tokens(np.asarray(prev, dtype=np.int32), np.asarray(inputs.Uniforms, dtype=np.float64),
-                                      mask_ids=np.asarray(inputs.MaskIds, dtype=np.int32))
+            self._batch.append_tokens(prev, inputs.Uniforms, mask_ids=inputs.MaskIds)
             self.appends += 1
         else:
-            params = []
-            for p, h in zip(inputs.Params, inputs.Histories):
-                q = SamplingParams(**{k: getattr(p, k) for k in p.__dataclass_fields__})
-                q.PreviousTokens = list(h) if h else None     # `sp with { PreviousTokens = seq.RecentTokens }` (:640-642)
-                params.append(q)
-            self._batch.upload(params, vocab, np.asarray(inputs.Uniforms, dtype=np.float64),
-                               mask_ids=np.asarray(inputs.MaskIds, dtype=np.int32))
+            # `sp with { PreviousTokens = seq.RecentTokens }` (:640-642)
+            self._batch.upload(inputs.Params, vocab, inputs.Uniforms, mask_ids=inputs.MaskIds, histories=inputs.Histories)
             self._rows, self._vocab = rows, vocab
             self.uploads += 1
         self.ctx.sample_launch(self._batch, logits_dev, tokens_dev, flags_dev)

@@ -75,6 +75,9 @@ internal static unsafe partial class StingraySamplerInterop
     [LibraryImport(Lib, EntryPoint = "sr_argmax_rows_launch")]
     internal static partial int ArgmaxRowsLaunch(nint ctx, nint logitsDev, int dtype, int rows, int vocab,
         long rowStrideElems, nint outIdxDev, nint outValDev);
+    [LibraryImport(Lib, EntryPoint = "sr_argmax_rows_both")]
+    internal static partial int ArgmaxRowsBoth(nint ctx, nint logitsDev, int dtype, int rows, int vocab,
+        long rowStrideElems, nint outIdxDev, nint outValDev, int* outIdx, float* outVal);
     [LibraryImport(Lib, EntryPoint = "sr_mask_register")]
     internal static partial int MaskRegister(nint ctx, uint* words, int wordsOnDevice, int vocab, out int maskId);
     [LibraryImport(Lib, EntryPoint = "sr_mask_release")]
