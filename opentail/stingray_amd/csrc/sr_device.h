@@ -117,6 +117,24 @@ __device__ __forceinline__ void sr_drain_stores() { __builtin_amdgcn_s_waitcnt(0
 // whatever a loop has prefetched for its next turn.
 __device__ __forceinline__ void sr_barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
+// Sixteen bytes from (to) an address that is a multiple of an element's size only: one instruction like the aligned form --
+// the memory system splits what crosses a line --, so rows at odd addresses need no loads of single elements.
+template <int kAlign> struct __attribute__((packed, aligned(kAlign))) SrPacked16 { uint32_t x, y, z, w; };
+template <int kAlign> __device__ __forceinline__ uint4 sr_load16(const void* p)
+{
+    const SrPacked16<kAlign> v = *(const SrPacked16<kAlign>*)p;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+__device__ __forceinline__ float4 sr_load_f4(const float* p)
+{
+    const uint4 v = sr_load16<4>(p);
+    return make_float4(sr_u2f(v.x), sr_u2f(v.y), sr_u2f(v.z), sr_u2f(v.w));
+}
+__device__ __forceinline__ void sr_store_f4(float* p, float x, float y, float z, float w)
+{
+    *(SrPacked16<4>*)p = SrPacked16<4>{sr_f2u(x), sr_f2u(y), sr_f2u(z), sr_f2u(w)};
+}
+
 // ---- wave / block primitives --------------------------------------------------------------------
 __device__ __forceinline__ int sr_lane() { return (int)(threadIdx.x & (SR_WAVE - 1)); }
 __device__ __forceinline__ int sr_wave_id() { return (int)(threadIdx.x >> 6); }

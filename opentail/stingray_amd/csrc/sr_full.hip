@@ -1275,7 +1275,7 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
 #pragma unroll
             for (int k = 0; k < K; k++) {
                 const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * E;
-                raw[k] = *(const uint4*)(src.rowp + (size_t)i0 * ES);
+                raw[k] = sr_load16<ES>(src.rowp + (size_t)i0 * ES);
                 keep[k] = 0xffffffffu;
                 if (src.mrow) keep[k] = src.mrow[i0 >> 5] >> (i0 & 31);
             }
@@ -1304,7 +1304,7 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
             for (int k = 0; k < K; k++)
 #pragma unroll
                 for (int q4 = 0; q4 < E / 4; q4++)
-                    rw[k * (E / 4) + q4] = *(const float4*)(src.w + seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * E + 4 * q4);
+                    rw[k * (E / 4) + q4] = sr_load_f4(src.w + seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * E + 4 * q4);
 #pragma unroll
             for (int v = 0; v < K * E / 4; v++) {
                 x[4 * v] = rw[v].x; x[4 * v + 1] = rw[v].y; x[4 * v + 2] = rw[v].z; x[4 * v + 3] = rw[v].w;
@@ -1326,7 +1326,7 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
 #pragma unroll
             for (int q4 = 0; q4 < E; q4 += 4) {
                 if (whole) {
-                    const float4 v = *(const float4*)(src.w + i0 + q4);
+                    const float4 v = sr_load_f4(src.w + i0 + q4);
                     xv[q4] = v.x; xv[q4 + 1] = v.y; xv[q4 + 2] = v.z; xv[q4 + 3] = v.w;
                 } else {
 #pragma unroll
@@ -1338,7 +1338,7 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
         uint32_t keep = (1u << E) - 1u;
         if (src.mrow) keep = src.mrow[i0 >> 5] >> (i0 & 31);
         if (whole) {
-            const uint4 v = *(const uint4*)(src.rowp + (size_t)i0 * ES);
+            const uint4 v = sr_load16<ES>(src.rowp + (size_t)i0 * ES);
             if (ES == 4) {
                 xv[0] = sr_u2f(v.x); xv[1] = sr_u2f(v.y); xv[2] = sr_u2f(v.z); xv[3] = sr_u2f(v.w);
             } else {
@@ -1448,7 +1448,7 @@ __device__ __forceinline__ void seg_pass2(const SrFullArgs& a, const SegPass2& c
         if (i0 + E <= n) {
 #pragma unroll
             for (int q = 0; q < E; q += 4)
-                *(float4*)(c.w + i0 + q) = make_float4(e[k * E + q], e[k * E + q + 1], e[k * E + q + 2], e[k * E + q + 3]);
+                sr_store_f4(c.w + i0 + q, e[k * E + q], e[k * E + q + 1], e[k * E + q + 2], e[k * E + q + 3]);
         } else {
 #pragma unroll
             for (int q = 0; q < E; q++)

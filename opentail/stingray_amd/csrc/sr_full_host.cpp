@@ -43,16 +43,11 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     a.lazy_scale = lazy_scale ? 1 : 0;
     // Which of the rows that come here keep an adjusted copy, and which have their edits applied where they are read
     // (the rows of the batch that take this path: every row in modes 1 / 2).
-    // Long rows that start on 16-byte boundaries, logits and work rows alike: the softmax denominators are prepared by
+    // Long rows: the softmax denominators are prepared by
     // the pass over the whole device (k_full_softmax_seg) and the rows' workgroups only walk the records.  That pass also
     // applies the edits of the rows without an adjusted copy itself: they need no table and no kernel in front.
     const int nseg = (vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
-    const bool seg_mode = [&] {
-        const int es = dtype == SR_DTYPE_BF16 ? 2 : 4;
-        const bool aligned = (((uintptr_t)logits_dev) & 15u) == 0u && ((row_stride * es) & 15) == 0 &&
-                             (((uintptr_t)a.work) & 15u) == 0u && ((a.work_stride * 4) & 15) == 0;
-        return vocab >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX && aligned;
-    }();
+    const bool seg_mode = vocab >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX;
     a.edits_in_pass = seg_mode ? 1 : 0;
     bool any_table = false, any_copy = false, any_edits = false;
     int n_sampled = 0, n_seen = 0;
