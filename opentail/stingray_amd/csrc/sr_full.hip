@@ -355,77 +355,78 @@ struct SegRec {
 };
 __device__ __forceinline__ void seg_load_rec(const SeqSegFunc* funcs, int seg, int nseg, SegRec& r)
 {
-    const uint4 z = make_uint4(0u, 0u, 0u, 0u);
-    r.f = r.g = r.x0 = r.x1 = r.x2 = r.x3 = z;
-    if (seg < nseg) {
-        const uint4* q = (const uint4*)(funcs + seg);
-        r.f = q[0]; r.g = q[1]; r.x0 = q[2]; r.x1 = q[3]; r.x2 = q[4]; r.x3 = q[5];
-    }
+    const uint4* q = (const uint4*)(funcs + min(seg, nseg - 1));
+    r.f = q[0]; r.g = q[1]; r.x0 = q[2]; r.x1 = q[3]; r.x2 = q[4]; r.x3 = q[5];
+    if (seg >= nseg) r.f.w = SR_SEG_ZERO;
 }
 
-// The exact running sum over terms[0, n) from s0, by the 64 lanes of ONE wave.  With kSearch it stops at the first term at
-// which the running sum reaches `target`: *found = its index and the returned value is the running sum at that term.
-// With `states` (not with kSearch) the running sum behind segment g is left at states[g].
-template <bool kSearch>
-__device__ __forceinline__ float seg_walk(const float* terms, int n, const SeqSegFunc* funcs, float s0, float target, int* found,
-                                          float* states)
+// The exact running sum over the terms of nseg segments from s0, by the 64 lanes of ONE wave.  With kSearch it stops at the
+// first term at which the running sum reaches `target`: *found = its index and the returned value is the running sum at that
+// term.  With `states` (not with kSearch) the running sum behind segment g is left at states[g].
+// load(segment, x) gives the lane's 16 terms of a segment, wherever the terms come from.
+//
+// 64 segments at a time, a lane each, the next 64 loading meanwhile.  The segments that are one function with the same
+// increment for both parities -- nearly all -- are summed up once (inclusive sums T over the lanes); from then on a run of
+// them that was made for the binade the sum is in costs two lane reads and an integer addition, and only the segment that ends
+// the run is looked at by itself: one in which the sum changes binade, one with an increment per parity, one whose
+// prediction missed.  (A scan of the 64 functions after every such segment -- fifteen or so in a row whose sum starts at zero --
+// was most of the 8 us that a walk over 149 segments took.)
+template <bool kSearch, typename Load>
+__device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSegFunc* funcs, float s0, float target, int* found,
+                                               float* states)
 {
     const int lane = sr_lane();
-    const int nseg = seg_count(n);
-    const bool aligned = ((uintptr_t)terms & 15u) == 0u;
-    float s = s0;
+    uint32_t sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(s0));  // the running sum's bits, the same in every lane
     *found = -1;
     SegRec next;
     seg_load_rec(funcs, lane, nseg, next);
     for (int base = 0; base < nseg; base += SR_WAVE) {
-        const int seg = base + lane;
-        const bool have = seg < nseg;
         const SegRec r = next;
-        seg_load_rec(funcs, seg + SR_WAVE, nseg, next);  // (the records of the next 64 segments come in meanwhile)
+        seg_load_rec(funcs, base + SR_WAVE + lane, nseg, next);  // (the records of the next 64 segments come in meanwhile)
+        const int cnt = min(SR_WAVE, nseg - base);
         const uint32_t kind = r.f.w & 0xffu;
-        int lstart = 0;  // the segments of the lanes below are settled
+        const bool zero = kind == SR_SEG_ZERO, simple = kind == SR_SEG_PLAIN && r.f.x == r.f.y && r.f.x < (1u << 24);
+        const unsigned long long zeros = __ballot(zero), simples = __ballot(simple);
+        const uint32_t T = (uint32_t)sr_wave_incl_scan_i32(simple ? (int)r.f.x : 0);
+        int pos = 0;  // the segments below are settled
         for (;;) {
-            uint32_t n_in;
+            uint32_t n;
             int eb;
-            sr_split(s, &n_in, &eb);
-            SrInc m;
-            m.a0 = 0u; m.a1 = 0u;
-            if (have && lane >= lstart) {
-                if (kind == SR_SEG_PLAIN && (int)r.f.z == eb) { m.a0 = r.f.x; m.a1 = r.f.y; }
-                else { m.a0 = SR_SEQ_SAT; m.a1 = SR_SEQ_SAT; }  // made for another binade, or not one function
+            sr_split(sr_u2f(sb), &n, &eb);
+            // the run of segments from pos on that the binade's integer additions take
+            const unsigned long long take = zeros | (simples & __ballot((int)r.f.z == eb));
+            const unsigned long long stop = ~take & (~0ull << pos);
+            int end = stop ? (int)__ffsll((long long)stop) - 1 : SR_WAVE;
+            end = min(end, cnt);
+            const uint32_t t0 = pos > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)T, pos - 1) : 0u;
+            if (end > pos) {
+                const uint32_t mine = n + (T - t0);  // (the running sum behind this lane's segment, for the lanes of the run)
+                bool ev = mine >= (1u << 24);
+                if (kSearch) ev = ev || sr_join(mine, eb) >= target;
+                // (a run may leave its binade, or reach the target, on its way: up to there)
+                const unsigned long long over = __ballot(ev && lane >= pos && lane < end);
+                if (over) end = (int)__ffsll((long long)over) - 1;
+                if (!kSearch && states && lane >= pos && lane < end) states[base + lane] = sr_join(mine, eb);
+                if (end > pos) {
+                    n += (uint32_t)__builtin_amdgcn_readlane((int)T, end - 1) - t0;
+                    sb = sr_f2u(sr_join(n, eb));
+                }
             }
-            const SrInc sc = sr_scan_inc<false>(m);
-            SrInc ex;
-            ex.a0 = __shfl_up(sc.a0, 1);
-            ex.a1 = __shfl_up(sc.a1, 1);
-            if (lane == 0) { ex.a0 = 0u; ex.a1 = 0u; }
-            const bool odd = (n_in & 1u) != 0u;
-            const uint32_t before = sr_sat_add(n_in, odd ? ex.a1 : ex.a0);
-            const uint32_t after = sr_sat_add(n_in, odd ? sc.a1 : sc.a0);
-            bool ev = after >= (1u << 24);
-            if (kSearch) ev = ev || sr_join(after, eb) >= target;
-            const unsigned long long evl = __ballot(ev && have && lane >= lstart);
-            const int fl = evl ? (int)__ffsll((long long)evl) - 1 : SR_WAVE;
-            if (!kSearch && states && have && lane >= lstart && lane < fl) states[seg] = sr_join(after, eb);
-            if (!evl) {
-                const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)(odd ? sc.a1 : sc.a0), SR_WAVE - 1);
-                s = sr_join(n_in + tot, eb);
-                break;
-            }
-            // The first segment that the plain functions do not settle.  Its lane tries what its record offers, from
-            // the exact sum in front of the segment; every step is checked, and a record that does not fit that sum
-            // (or a search that would end inside the segment) leaves the segment to be added from its terms.
-            const float s_before = sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(sr_join(before, eb)), fl));
+            if (end >= cnt) break;
+            // The segment that ends the run, from the exact sum in front of it.  Every step is checked, and a record that does
+            // not fit that sum (or a search that would end inside the segment) leaves the segment to be added from its terms.
             float s_try = 0.0f;
             bool ok = false;
-            if (lane == fl) {
-                if (kind == SR_SEG_EXACT && sr_f2u(s_before) == 0u) {
+            if (lane == end) {
+                if (kind == SR_SEG_EXACT) {
                     s_try = sr_u2f(r.g.w);
-                    ok = true;
-                } else if (kind == SR_SEG_SPLIT && (int)r.f.z == eb) {
-                    const uint32_t n1 = sr_sat_add(before, (before & 1u) ? r.f.y : r.f.x);
-                    if (n1 < (1u << 24)) {
-                        float acc = sr_join(n1, eb);
+                    ok = sb == 0u;
+                } else if (kind != SR_SEG_ZERO && (int)r.f.z == eb) {
+                    const uint32_t n1 = sr_sat_add(n, (n & 1u) ? r.f.y : r.f.x);
+                    float acc = sr_join(n1, eb);
+                    ok = n1 < (1u << 24);
+                    s_try = acc;
+                    if (kind == SR_SEG_SPLIT) {
                         const uint32_t xs[16] = {r.x0.x, r.x0.y, r.x0.z, r.x0.w, r.x1.x, r.x1.y, r.x1.z, r.x1.w,
                                                  r.x2.x, r.x2.y, r.x2.z, r.x2.w, r.x3.x, r.x3.y, r.x3.z, r.x3.w};
 #pragma unroll
@@ -433,36 +434,44 @@ __device__ __forceinline__ float seg_walk(const float* terms, int n, const SeqSe
                         uint32_t n2;
                         int eb2;
                         sr_split(acc, &n2, &eb2);
-                        if (eb2 == (int)r.g.z) {
-                            const uint32_t n3 = sr_sat_add(n2, (n2 & 1u) ? r.g.y : r.g.x);
-                            if (n3 < (1u << 24)) {
-                                s_try = sr_join(n3, eb2);
-                                ok = true;
-                            }
-                        }
+                        const uint32_t n3 = sr_sat_add(n2, (n2 & 1u) ? r.g.y : r.g.x);
+                        ok = ok && eb2 == (int)r.g.z && n3 < (1u << 24);
+                        s_try = sr_join(n3, eb2);
                     }
                 }
-                if (kSearch && ok && s_try >= target) ok = false;  // the answer lies inside: from the terms
+                if (kSearch && s_try >= target) ok = false;  // the answer lies inside: from the terms
             }
-            ok = __builtin_amdgcn_readlane((int)ok, fl) != 0;
-            if (ok) {
-                s = sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(s_try), fl));
+            if (__builtin_amdgcn_readlane((int)ok, end) != 0) {
+                sb = (uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(s_try), end);
             } else {
                 float x[SR_SEQ_RUN];
-                seq_load_run(terms, aligned, (base + fl) * SR_SEG_TERMS + lane * SR_SEQ_RUN, n, x);
+                load(base + end, x);
                 int at;
-                s = sr_seq_wave<SR_SEQ_RUN, kSearch>(x, s_before, target, &at);
+                const float s = sr_seq_wave<SR_SEQ_RUN, kSearch>(x, sr_u2f(sb), target, &at);
                 if (kSearch && at >= 0) {
-                    *found = (base + fl) * SR_SEG_TERMS + at;
+                    *found = (base + end) * SR_SEG_TERMS + at;
                     return s;
                 }
+                sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(s));
             }
-            if (!kSearch && states && lane == 0) states[base + fl] = s;
-            lstart = fl + 1;
-            if (lstart >= SR_WAVE) break;
+            if (!kSearch && states && lane == 0) states[base + end] = sr_u2f(sb);
+            pos = end + 1;
+            if (pos >= cnt) break;
         }
     }
-    return s;
+    return sr_u2f(sb);
+}
+
+// ... over terms[0, n) in memory
+template <bool kSearch>
+__device__ __forceinline__ float seg_walk(const float* terms, int n, const SeqSegFunc* funcs, float s0, float target, int* found,
+                                          float* states)
+{
+    const bool aligned = ((uintptr_t)terms & 15u) == 0u;
+    const int lane = sr_lane();
+    return seg_walk_from<kSearch>([&](int seg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
+        seq_load_run(terms, aligned, seg * SR_SEG_TERMS + lane * SR_SEQ_RUN, n, x);
+    }, seg_count(n), funcs, s0, target, found, states);
 }
 
 // The record of one segment (SeqSegFunc) from its terms x (lane l holds the terms 16 l ... 16 l + 15 of the segment) and
@@ -473,6 +482,16 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
                                                 float seg_sum = -1.0f)
 {
     const int lane = sr_lane();
+    {
+        // a segment without a term (masked, or cut) changes no sum whatever its binade
+        float any = x[0];
+#pragma unroll
+        for (int j = 1; j < SR_SEQ_RUN; j++) any = sr_max_f32(any, x[j]);
+        if (__ballot(any > 0.0f) == 0ull) {
+            if (lane == 0) ((uint4*)out)[0] = make_uint4(0u, 0u, 0u, SR_SEG_ZERO);
+            return;
+        }
+    }
     if (seg > 0 && seg_sum >= 0.0f) {
         const float lo = __double2float_rn(before), hi = lo + seg_sum;
         uint32_t nn;
@@ -1034,11 +1053,23 @@ __device__ __forceinline__ void hist_count(uint32_t* hcnt, uint32_t* bad, float 
     }
 }
 
-// which rows take which way: asked by the passes over the whole device and by the row's workgroup alike
-__device__ __forceinline__ bool row_watch_min_p(const SrRow& rd, const SrFullArgs& a)
+// Which rows take which way: asked by the passes over the whole device and by the row's workgroup alike.
+// A sampled row that only min-p and top-p cut: the pass over the whole device lists what can be in its nucleus, and the
+// row's workgroup finds the cut in that list.  (Not where a verifier reads e in place.)
+__device__ __forceinline__ bool row_is_listed(const SrRow& rd, const SrFullArgs& a)
 {
-    return rd.min_p > 0.0f && !(rd.top_k > 0 && rd.top_k < a.vocab) && a.mode == 0 && a.vocab >= 8;
+    return !a.lazy_scale && a.seg_func != nullptr && rd.temperature > 0.0f && sr_row_cut(rd) && !(rd.top_k > 0 && rd.top_k < a.vocab);
 }
+// A sampled row that nothing cuts.
+__device__ __forceinline__ bool row_is_plain(const SrRow& rd, const SrFullArgs& a)
+{
+    return a.seg_func != nullptr && rd.temperature > 0.0f && !sr_row_cut(rd) && !(rd.top_k > 0 && rd.top_k < a.vocab);
+}
+// Where e = expf(x - max) of a row lies: in the work row, or, where distributions are handed out, in scratch memory of its own.
+// (One place for all rows of a launch: with a choice per row the compiler, clang 22, took the stride of one buffer and the
+// base of the other.)
+__device__ __forceinline__ float* row_e(const SrFullArgs& a, int slot) { return a.e_rows + (size_t)slot * (size_t)a.e_stride; }
+// the walk by slabs over the row itself, for a row in scratch memory that only top-p cuts and whose list was too long
 __device__ __forceinline__ bool row_fast_nucleus(const SrRow& rd, const SrFullArgs& a)
 {
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
@@ -1240,7 +1271,7 @@ template <int ES>
 __device__ __forceinline__ SegSource<ES> seg_source(const SrRow& rd, const SrFullArgs& a, int slot, int row)
 {
     SegSource<ES> src;
-    src.w = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;
+    src.w = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;  // (the adjusted copy, where the row keeps one)
     src.rowp = nullptr;
     src.mrow = nullptr;
     src.scale = false;
@@ -1403,135 +1434,69 @@ __device__ __forceinline__ void seg_apply_edits(const SrFullArgs& a, const SrRow
     }
 }
 
-// Both passes are one launch (k_full_softmax_seg): a wave keeps its segments in registers in between, so the logits
-// are read once.  The workgroups of a row meet between the passes: each leaves its segments' maxima and approximate
-// sums, counts itself in (SR_ROW_SYNC_STRIDE), and waits until the row's count is full.  Workgroups start in the order
-// of their numbers, a row's side by side, so those that a waiting workgroup waits for are running or next to start;
-// the wait is bounded all the same.  A workgroup whose wait runs out marks its segments (SR_SEG_LATE) and leaves;
-// whichever workgroup of the row is the last to get behind the meeting point -- the row's maxima are all in then --
-// finds the marks and finishes those segments, whose inputs nobody has touched.  What a segment gets is the same
-// whichever way it is finished.
-struct SegPass2 {
-    const uint64_t* tab;   // the expf table in shared memory
-    float4* turn;          // the wave's SR_WAVE * 5 vectors of shared memory
-    float* w;
-    uint16_t* keys;
-    bool watch;
-    float e_low, m;
-    int slot, n;
-};
-// e = expf(x - m) of one segment (x as seg_load_logits left it): written to the work row, its 16-bit keys and the
-// entries a min-p cut watches where the row asks for them, and the segment's record
-template <int ES>
-__device__ __forceinline__ void seg_pass2(const SrFullArgs& a, const SegPass2& c, int seg, int lane, const float (&x)[SR_SEQ_RUN],
-                                          float before, float own_sum)
+// Everything is one launch (k_full_softmax_seg): a wave keeps its segments in registers, so the logits are read once.  The
+// workgroups of a row meet twice: each folds its largest logit into the row's and counts itself in; when the count is
+// full it computes e = expf(x - max), leaves its segments' sums (and, for rows that top-p cuts, its share of the row's
+// mass by size of e), meets again, and makes the segments' records from the sums in front of them.  Workgroups start in
+// the order of their numbers, a row's side by side, so those that a waiting workgroup waits for are running or next to
+// start; the waits are bounded all the same: a workgroup whose wait runs out marks the row (SrFullState::late), counts itself
+// in everywhere and leaves, and the row's own workgroup does the whole row by itself from the logits (row_alone).
+//
+// What bounds it: the vector units (the double-precision expf is 30 instructions an element).  The first pass used to
+// take a fast exponential of every element, for approximate sums relative to the segment's own maximum, to save the second
+// meeting; the sums come from e itself now, which costs a meeting of 2 - 3 us and a quarter fewer instructions.
+
+// a segment's largest value as an ordered key; 0xffffffff = it holds a NaN (which propagates: TensorPrimitives.Max)
+__device__ __forceinline__ uint32_t seg_max_key(const float (&x)[SR_SEQ_RUN])
 {
-    constexpr int E = 16 / ES, K = SR_SEG_TERMS / (SR_WAVE * E);
-    const int n = c.n;
-    float e[SR_SEQ_RUN];
-    // (a whole segment without a test per element: the 16 chains of a lane then run interleaved)
-    if ((seg + 1) * SR_SEG_TERMS <= n) {
+    float m = x[0];
+    bool nan = x[0] != x[0];
 #pragma unroll
-        for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = sr_expf_tab(__fsub_rn(x[j], c.m), c.tab);
-    } else {
-#pragma unroll
-        for (int k = 0; k < K; k++)
-#pragma unroll
-            for (int q = 0; q < E; q++) {
-                const int i = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * E + q;
-                e[k * E + q] = i < n ? sr_expf_tab(__fsub_rn(x[k * E + q], c.m), c.tab) : 0.0f;
-            }
+    for (int j = 1; j < SR_SEQ_RUN; j++) {
+        m = sr_max_f32(m, x[j]);
+        nan = nan || x[j] != x[j];
     }
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * E;
-        if (i0 + E <= n) {
-#pragma unroll
-            for (int q = 0; q < E; q += 4)
-                sr_store_f4(c.w + i0 + q, e[k * E + q], e[k * E + q + 1], e[k * E + q + 2], e[k * E + q + 3]);
-        } else {
-#pragma unroll
-            for (int q = 0; q < E; q++)
-                if (i0 + q < n) c.w[i0 + q] = e[k * E + q];
-        }
-        if (c.keys) {
-            uint32_t kk[E];
-#pragma unroll
-            for (int q = 0; q < E; q++) kk[q] = e[k * E + q] > 0.0f ? max(sr_f2u(e[k * E + q]) >> 16, 1u) : 0u;
-            if (i0 + E <= n) {
-#pragma unroll
-                for (int q = 0; q < E; q += 4)
-                    *(uint2*)(c.keys + i0 + q) = make_uint2(kk[q] | (kk[q + 1] << 16), kk[q + 2] | (kk[q + 3] << 16));
-            } else {
-#pragma unroll
-                for (int q = 0; q < E; q++)
-                    if (i0 + q < n) c.keys[i0 + q] = (uint16_t)kk[q];
-            }
-        }
-        if (c.watch) {
-#pragma unroll
-            for (int q = 0; q < E; q++)
-                if (e[k * E + q] >= c.e_low && i0 + q < n) {
-                    const uint32_t pos = atomicAdd(&a.watch_cnt[c.slot], 1u);
-                    if (pos < (uint32_t)kSmall)
-                        a.watch[(size_t)c.slot * kSmall + pos] = ((unsigned long long)sr_f2u(e[k * E + q]) << 32) |
-                                                                 (unsigned long long)(0xffffffffu - (uint32_t)(i0 + q));
-                }
-        }
-    }
-    // through shared memory into the order of the sum: lane l gets the terms 16 l ... 16 l + 15 of the segment (only
-    // this wave touches its part: the wave's own order of shared-memory operations is all it needs)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-#pragma unroll
-    for (int k = 0; k < K; k++)
-#pragma unroll
-        for (int q = 0; q < E; q += 4) {
-            const int i = (k * SR_WAVE + lane) * E + q;  // the element's place in the segment
-            c.turn[(i >> 4) * 5 + ((i & 15) >> 2)] = make_float4(e[k * E + q], e[k * E + q + 1], e[k * E + q + 2], e[k * E + q + 3]);
-        }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float t[SR_SEQ_RUN];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        const float4 v = c.turn[lane * 5 + k];
-        t[4 * k] = v.x; t[4 * k + 1] = v.y; t[4 * k + 2] = v.z; t[4 * k + 3] = v.w;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    seg_make_record(t, seg, (double)before, a.seg_func + (size_t)c.slot * a.seg_stride + seg, own_sum);
+    return nan ? 0xffffffffu : sr_okey(m);
 }
-// a segment's own maximum (as an ordered key; 0xffffffff = it holds a NaN) and the sum of exp(x - that maximum)
-__device__ __forceinline__ unsigned long long seg_pass1(const float (&x)[SR_SEQ_RUN])
+// The mass of a row's e by size: kMassBuckets buckets, eight to a doubling, bucket 0 just below 1, the last one everything
+// small.  From the sums over all of the row: the smallest value (as bits) whose bucket still has to be listed for the
+// listed entries to hold `share` of the row's mass and a little more.
+constexpr int kMassBuckets = 256;
+__device__ __forceinline__ uint32_t mass_bucket(float e)  // (e in [0, 1])
 {
-    uint32_t k = 0u;
-#pragma unroll
-    for (int j = 0; j < 16; j++) {
-        const uint32_t kv = (x[j] != x[j]) ? 0xffffffffu : sr_okey(x[j]);  // NaN propagates (TensorPrimitives.Max)
-        k = kv > k ? kv : k;
-    }
-    k = sr_wave_max_u32(k);
-    float sum = 0.0f;
-    if (k != 0xffffffffu && k > 0x007fffffu) {
-        const float m = sr_okey_inv(k);
-#pragma unroll
-        for (int j = 0; j < 16; j++) sum += __expf(x[j] - m);
-    }
-    sum = sr_wave_sum_f32(sum);
-    return ((unsigned long long)sr_f2u(sum) << 32) | (unsigned long long)k;
+    return min((0x3f800000u - sr_f2u(e)) >> 20, (uint32_t)(kMassBuckets - 1));
 }
-// what a segment's (maximum, sum) adds to the row's approximate sum when the row's maximum is m
-__device__ __forceinline__ float seg_share(unsigned long long ms, float m)
+__device__ __forceinline__ uint32_t mass_list_from(const float* mass, float share)
 {
-    const uint32_t k = (uint32_t)ms;
-    const float sum = sr_u2f((uint32_t)(ms >> 32));
-    return (sum > 0.0f && k != 0xffffffffu) ? sum * __expf(sr_okey_inv(k) - m) : 0.0f;
+    static_assert(kMassBuckets == 4 * SR_WAVE, "four buckets per lane");
+    const int lane = sr_lane();
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = sr_load_agent(mass + 4 * lane + q);
+    const float own = (v[0] + v[1]) + (v[2] + v[3]);
+    const float incl = sr_wave_incl_sum_f32(own);
+    const float total = sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(incl), SR_WAVE - 1));
+    const float target = share * total * 1.0005f;
+    float c = incl - own;
+    int d = kMassBuckets;
+#pragma unroll
+    for (int q = 3; q >= 0; q--) {
+        float upto = c;
+#pragma unroll
+        for (int k = 0; k <= q; k++) upto += v[k];
+        if (upto >= target) d = 4 * lane + q;
+    }
+    d = sr_wave_min_i32(d);
+    if (d >= kMassBuckets - 1) return 1u;  // everything above zero
+    return 0x3f800000u - ((uint32_t)(d + 1) << 20) + 1u;
 }
+
 template <int ES, int kW, int kS>
 __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_seg(SrFullArgs a)
 {
     constexpr int kThreads = kW * SR_WAVE;
+    constexpr int E = 16 / ES, K = SR_SEG_TERMS / (SR_WAVE * E);
+    static_assert(kW == SR_HALF_BLOCK_SEGS, "a workgroup's segments are whole half blocks");
     const int slot = blockIdx.y, lane = sr_lane(), wave = sr_wave_id();
     const int row = a.row_list[slot];
     const SrRow rd = a.rows[row];
@@ -1539,10 +1504,12 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
     __shared__ uint64_t tab[32];  // the expf table: a lookup per element from global memory is a long dependent load
     // a wave's segment on its way from the order of the loads to 16 terms a lane: a lane's 16 terms lie together, 16
     // bytes apart from the next lane's, so that neither the stores nor the loads of 16 bytes a lane collide on a bank
-    __shared__ float4 turn[kW][SR_WAVE * 5];
-    __shared__ float share[SR_SEG_MAX];  // every segment's part of the row's approximate sum
+    __shared__ float4 turn_all[kW][SR_WAVE * 5];
+    __shared__ float share[SR_SEG_MAX];   // every segment's part of the row's sum
+    __shared__ float mass[kMassBuckets];  // this workgroup's part of the row's mass by size of e
+    __shared__ float chains[kS][SR_SEQ_CHAINS];
     __shared__ uint32_t wkey[kW];
-    __shared__ uint32_t bc[2];           // 0: the row's count came in   1: what k_full_edits made the row's maximum
+    __shared__ uint32_t bc[2];            // 0: the row's count came in   1: the row's maximum
     // the row's edits that fall into this workgroup's segments (id << 32 | place in the row's edit list), and how many
     // there are (more than the list holds: the waves go through the row's whole edit list instead)
     constexpr int kHitCap = 256;
@@ -1551,26 +1518,22 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
     const int n = a.vocab, nseg = seg_count(n);
     SrFullState* st = a.state + slot;
     unsigned long long* sync = a.row_sync + (size_t)slot * SR_ROW_SYNC_STRIDE;
-    unsigned long long* ms = (unsigned long long*)(a.seg_ms + (size_t)slot * a.seg_stride);
     const unsigned long long stamp = (unsigned long long)a.seq << 32;
     SeqSegFunc* recs = a.seg_func + (size_t)slot * a.seg_stride;
+    float* sums = a.seg_sum + (size_t)slot * a.seg_stride;
     if (threadIdx.x < 32) tab[threadIdx.x] = sr_exp2f_tab[threadIdx.x];
     const SegSource<ES> src = seg_source<ES>(rd, a, slot, row);
-    SegPass2 c;
-    c.tab = tab;
-    c.turn = turn[wave];
-    c.w = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;
-    // (a row that only top-p cuts needs the histogram of its e by their upper 16 bits: counting it here, one atomic per
-    // element, took longer than it saved, so the pass leaves those 16 bits of every e beside the row, and the row's
-    // workgroup counts them -- half the bytes of the row -- while one of its waves walks the sum)
-    c.keys = (row_fast_nucleus(rd, a) && a.seg_keys) ? a.seg_keys + (size_t)slot * (size_t)a.seg_key_stride : nullptr;
-    c.watch = row_watch_min_p(rd, a);
-    c.e_low = __fmul_rn(rd.min_p, 0.999999f);
-    c.slot = slot;
-    c.n = n;
-    c.m = 0.0f;
+    float* const w = row_e(a, slot);
+    const bool plain = row_is_plain(rd, a), listed = row_is_listed(rd, a);
+    const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
+    // (a min-p cut that leaves a few hundred entries at most needs no second bound)
+    const bool by_mass = listed && use_top_p && rd.min_p < 0.01f;
+    // (the row's sum is at least 1: n entries below this make up less than half of what top-p leaves out)
+    const float mass_min = (1.0f - rd.top_p) * 0.5f / (float)n;
+    if (by_mass)
+        for (int i = threadIdx.x; i < kMassBuckets; i += kThreads) mass[i] = 0.0f;
+    if (plain && threadIdx.x < kS * SR_SEQ_CHAINS) (&chains[0][0])[threadIdx.x] = 0.0f;
 
-    // the first pass: the segment's maximum and approximate sum, written through for the row's other workgroups
     // A row that keeps no adjusted copy although bias or penalties touch some of its ids: the workgroup looks through
     // the row's edit list for the ids of its own segments, and its waves put the adjusted values in place of what they load
     // (the ids are asked for in front of the logits and looked at behind them: the loads overlap)
@@ -1588,25 +1551,12 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
             ids[j] = e < rd.edit_cnt ? ed[e].id : -1;
         }
     }
-    auto apply_edits = [&](int seg, float (&x)[SR_SEQ_RUN], bool from_hits) {
-        if (from_hits && n_hits <= (uint32_t)kHitCap)
-            seg_apply_edits<ES>(a, rd, src, seg, lane, (int)n_hits, [&](int i, int& id, int& e) {
-                const unsigned long long h = hits[i];
-                id = (int)(h >> 32);
-                e = (int)(uint32_t)h;
-            }, x);
-        else
-            seg_apply_edits<ES>(a, rd, src, seg, lane, rd.edit_cnt, [&](int i, int& id, int& e) {
-                id = ed[i].id;
-                e = i;
-            }, x);
-    };
     // (a wave takes kS segments, the workgroup's waves side by side: every one of its loads is out before the first is used)
     const int seg0 = (int)blockIdx.x * (kW * kS) + wave;
-    float xs[kS][SR_SEQ_RUN];
+    float t[kS][SR_SEQ_RUN];
 #pragma unroll
     for (int s = 0; s < kS; s++)
-        if (seg0 + s * kW < nseg) seg_load_logits<ES>(src, seg0 + s * kW, lane, n, xs[s]);
+        if (seg0 + s * kW < nseg) seg_load_logits<ES>(src, seg0 + s * kW, lane, n, t[s]);
     if (edits) {
         const int lo = (int)blockIdx.x * (kW * kS) * SR_SEG_TERMS, hi = lo + kW * kS * SR_SEG_TERMS;
 #pragma unroll
@@ -1618,130 +1568,191 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
             }
         }
         sr_barrier_lds();
+        const bool from_hits = n_hits <= (uint32_t)kHitCap;
 #pragma unroll
         for (int s = 0; s < kS; s++)
-            if (seg0 + s * kW < nseg) apply_edits(seg0 + s * kW, xs[s], true);
+            if (seg0 + s * kW < nseg)
+                seg_apply_edits<ES>(a, rd, src, seg0 + s * kW, lane, from_hits ? (int)n_hits : rd.edit_cnt, [&](int i, int& id, int& e) {
+                    if (from_hits) {
+                        const unsigned long long h = hits[i];
+                        id = (int)(h >> 32);
+                        e = (int)(uint32_t)h;
+                    } else {
+                        id = ed[i].id;
+                        e = i;
+                    }
+                }, t[s]);
     }
+    uint32_t k = 0u;
 #pragma unroll
     for (int s = 0; s < kS; s++)
-        if (seg0 + s * kW < nseg) {
-            const unsigned long long v = seg_pass1(xs[s]);
-            if (lane == 0) sr_store_agent(&ms[seg0 + s * kW], v);
-        }
-    sr_drain_stores();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __hip_atomic_fetch_max(sync, stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_fetch_add(sync, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long edited = sr_load_agent(&st->maxkey);  // (final: k_full_edits ran before)
-        uint32_t ok = 0u;
-        for (uint32_t it = 0; it < a.row_wait_limit; it++) {
-            const unsigned long long v = sr_load_agent(sync);
-            if ((uint32_t)(v >> 32) == a.seq && (uint32_t)(v & 0xffffu) == gridDim.x) { ok = 1u; break; }
-            __builtin_amdgcn_s_sleep(8);
-        }
-        bc[0] = ok;
-        bc[1] = full_maxkey_of(a, edited);
-    }
-    __syncthreads();
-    const bool met = bc[0] != 0u;
-    if (!met) {
-        // the wait ran out: the segments are left, marked, to the last of the row's workgroups
-#pragma unroll
-        for (int s = 0; s < kS; s++)
-            if (seg0 + s * kW < nseg && lane == 0) {
-                sr_store_agent(&recs[seg0 + s * kW].kind, SR_SEG_LATE);
-                sr_store_agent(&recs[seg0 + s * kW].a0, a.seq);
-            }
-        sr_drain_stores();
-        __syncthreads();
+        if (seg0 + s * kW < nseg) k = max(k, seg_max_key(t[s]));
+    k = sr_wave_max_u32(k);
+    if (lane == 0) wkey[wave] = k;
+    // The meeting point: `ready` goes in (behind everything the workgroup has written through or added), and the workgroup
+    // waits until the row's workgroups are all in.  part = 0, 1: the first, the second meeting.
+    auto met = [&](int part) -> bool {
         if (threadIdx.x == 0) {
-            sr_store_agent(&st->late, a.seq);
-            sr_drain_stores();
+            __hip_atomic_fetch_add(sync, 1ull << (16 * part), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            uint32_t ok = 0u;
+            for (uint32_t it = 0; it < a.row_wait_limit; it++) {
+                const unsigned long long v = sr_load_agent(sync);
+                if ((uint32_t)(v >> 32) == a.seq && ((uint32_t)(v >> (16 * part)) & 0xffffu) == gridDim.x) { ok = 1u; break; }
+                __builtin_amdgcn_s_sleep(2);
+            }
+            if (ok == 0u) {
+                // the wait ran out: the row is left to its own workgroup, and nobody waits for this one
+                sr_store_agent(&st->late, a.seq);
+                if (part == 0) __hip_atomic_fetch_add(sync, 1ull << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else if (part == 0) {
+                bc[1] = full_maxkey_of(a, sr_load_agent(&st->maxkey));
+            }
+            bc[0] = ok;
         }
-    }
-    // (the count as this workgroup found it is looked at behind the second pass: nothing waits for it here)
-    unsigned long long behind = 0ull;
-    if (threadIdx.x == 0) behind = __hip_atomic_fetch_add(sync, 1ull << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-
-    uint32_t mk = 0u;
-    if (met) {
-        // the row's maximum and the segments' shares of the approximate sum (single precision does: a prediction that
-        // misses costs time only)
-        constexpr int kPer = (SR_SEG_MAX + kThreads - 1) / kThreads;
-        unsigned long long mv[kPer];
-        uint32_t kk = 0u;
-#pragma unroll
-        for (int j = 0; j < kPer; j++) {
-            const int g = (int)threadIdx.x + kThreads * j;
-            mv[j] = g < nseg ? sr_load_agent(&ms[g]) : 0ull;
-            kk = max(kk, (uint32_t)mv[j]);
-        }
-        kk = sr_wave_max_u32(kk);
-        if (lane == 0) wkey[wave] = kk;
         __syncthreads();
-        mk = bc[1];
+        return bc[0] != 0u;
+    };
+    sr_barrier_lds();
+    if (threadIdx.x == 0) {
+        k = wkey[0];
 #pragma unroll
-        for (int j = 0; j < kW; j++) mk = max(mk, wkey[j]);
-        if (blockIdx.x == 0 && threadIdx.x == 0 && mk != 0u) atomicMax(&st->maxkey, full_maxkey(a, mk));  // for the row's kernel
-        if (mk != 0xffffffffu && mk > 0x007fffffu) {  // (else a NaN, or nothing above -inf: the row kernel makes it uniform)
-            c.m = sr_okey_inv(mk);
+        for (int j = 1; j < kW; j++) k = max(k, wkey[j]);
+        // (each atomic's returned value is waited for before the next is issued: whoever finds the count full finds the
+        // maximum complete)
+        const unsigned long long s0 = __hip_atomic_fetch_max(sync, stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long s1 = __hip_atomic_fetch_max(&st->maxkey, full_maxkey(a, k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" : : "v"(s0), "v"(s1) : "memory");
+    }
+    if (!met(0)) return;
+    const uint32_t mk = bc[1];
+    if (mk == 0xffffffffu || mk <= 0x007fffffu) return;  // a NaN, or nothing above -inf: the row's workgroup makes it uniform
+    const float m = sr_okey_inv(mk);
+
+    // e of the wave's segments: written to the row, counted by size, and turned into the order of the sum
+    float own[kS];
+    float4* const turn = turn_all[wave];
 #pragma unroll
-            for (int j = 0; j < kPer; j++) {
-                const int g = (int)threadIdx.x + kThreads * j;
-                if (g < nseg) share[g] = seg_share(mv[j], c.m);
-            }
-            __syncthreads();
+    for (int s = 0; s < kS; s++) {
+        own[s] = 0.0f;
+        const int seg = seg0 + s * kW;
+        if (seg >= nseg) continue;
+        float e[SR_SEQ_RUN];
+        // (a whole segment without a test per element: the 16 chains of a lane then run interleaved)
+        if ((seg + 1) * SR_SEG_TERMS <= n) {
 #pragma unroll
-            for (int s = 0; s < kS; s++) {
-                const int seg = seg0 + s * kW;
-                if (seg < nseg) {
-                    float before = 0.0f;
-                    for (int g = lane; g < seg; g += SR_WAVE) before += share[g];
-                    before = sr_wave_sum_f32(before);
-                    seg_pass2<ES>(a, c, seg, lane, xs[s], before, share[seg]);
-                }
+            for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = sr_expf_tab(__fsub_rn(t[s][j], m), tab);
+        } else {
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = seg_elem<ES>(seg, lane, j) < n ? sr_expf_tab(__fsub_rn(t[s][j], m), tab) : 0.0f;
+        }
+#pragma unroll
+        for (int k2 = 0; k2 < K; k2++) {
+            const int i0 = seg * SR_SEG_TERMS + (k2 * SR_WAVE + lane) * E;
+            if (i0 + E <= n) {
+#pragma unroll
+                for (int q = 0; q < E; q += 4) sr_store_f4(w + i0 + q, e[k2 * E + q], e[k2 * E + q + 1], e[k2 * E + q + 2], e[k2 * E + q + 3]);
+            } else {
+#pragma unroll
+                for (int q = 0; q < E; q++)
+                    if (i0 + q < n) w[i0 + q] = e[k2 * E + q];
             }
         }
-    }
-    if (wave != 0) return;
-
-    // The last of the row's workgroups to get behind the meeting point finishes what others left: one wave, segment by
-    // segment.  (Every workgroup's first pass is complete by then, and the marks were written before their workgroup
-    // counted itself.)
-    const uint32_t was = __shfl((uint32_t)(behind >> 16) & 0xffffu, 0);
-    if (was != gridDim.x - 1u) return;
-    if (sr_load_agent(&st->late) != a.seq) return;
-    if (!met) {
-        uint32_t kk = bc[1];
-        for (int g = lane; g < nseg; g += SR_WAVE) kk = max(kk, (uint32_t)sr_load_agent(&ms[g]));
-        mk = sr_wave_max_u32(kk);
-    }
-    // (the row's first workgroup, which leaves the maximum for the row's kernel, may be one of those that left)
-    if (lane == 0 && mk != 0u) atomicMax(&st->maxkey, full_maxkey(a, mk));
-    if (mk == 0xffffffffu || mk <= 0x007fffffu) return;
-    if (!met) {
-        c.m = sr_okey_inv(mk);
-        for (int g = lane; g < nseg; g += SR_WAVE) share[g] = seg_share(sr_load_agent(&ms[g]), c.m);
+        if (by_mass) {
+            // (entries so small that all of them together cannot reach into the nucleus are summed in registers, as the last
+            // bucket -- most of a sharp row: shared-memory atomics queue)
+            float small = 0.0f;
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) {
+                const uint32_t d = mass_bucket(e[j]);
+                if (e[j] >= mass_min && d < (uint32_t)(kMassBuckets - 1)) unsafeAtomicAdd(&mass[d], e[j]);
+                else small += e[j];
+            }
+            small = sr_wave_sum_f32(small);
+            if (lane == 0) unsafeAtomicAdd(&mass[kMassBuckets - 1], small);
+        }
+        float sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < SR_SEQ_RUN; j++) sum += e[j];
+        own[s] = sr_wave_sum_f32(sum);
+        // through shared memory into the order of the sum: lane l gets the terms 16 l ... 16 l + 15 of the segment (only
+        // this wave touches its part: the wave's own order of shared-memory operations is all it needs)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+#pragma unroll
+        for (int k2 = 0; k2 < K; k2++)
+#pragma unroll
+            for (int q = 0; q < E; q += 4) {
+                const int i = (k2 * SR_WAVE + lane) * E + q;  // the element's place in the segment
+                turn[(i >> 4) * 5 + ((i & 15) >> 2)] = make_float4(e[k2 * E + q], e[k2 * E + q + 1], e[k2 * E + q + 2], e[k2 * E + q + 3]);
+            }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    for (int g = 0; g < nseg; g++) {
-        uint32_t kind = 0u, whose = 0u;
-        if (lane == 0) {
-            kind = sr_load_agent(&recs[g].kind);
-            whose = sr_load_agent(&recs[g].a0);
+#pragma unroll
+        for (int k2 = 0; k2 < 4; k2++) {
+            const float4 v = turn[lane * 5 + k2];
+            t[s][4 * k2] = v.x; t[s][4 * k2 + 1] = v.y; t[s][4 * k2 + 2] = v.z; t[s][4 * k2 + 3] = v.w;
         }
-        kind = __shfl(kind, 0);
-        whose = __shfl(whose, 0);
-        if (kind != SR_SEG_LATE || whose != a.seq) continue;
-        seg_load_logits<ES>(src, g, lane, n, xs[0]);
-        if (edits) apply_edits(g, xs[0], false);  // (the list in shared memory is of this workgroup's own segments)
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (plain) {
+            // the segment's part of the eight lane accumulators of the final Normalize
+#pragma unroll
+            for (int g = 0; g < SR_SEQ_CHAINS; g++) {
+                const float c = sr_wave_sum_f32(t[s][g] + t[s][g + 8]);
+                if (lane == 0) unsafeAtomicAdd(&chains[s][g], c);
+            }
+        }
+        if (lane == 0) sr_store_agent(&sums[seg], own[s]);
+    }
+    sr_barrier_lds();
+    if (by_mass)
+        for (int i = threadIdx.x; i < kMassBuckets; i += kThreads)
+            if (mass[i] > 0.0f) unsafeAtomicAdd(a.mass + (size_t)slot * kMassBuckets + i, mass[i]);
+    if (plain && threadIdx.x < kS * SR_SEQ_CHAINS) {
+        const int hb = (int)blockIdx.x * kS + (int)threadIdx.x / SR_SEQ_CHAINS;
+        if (hb < a.chain_stride / SR_SEQ_CHAINS)
+            a.chain_sum[(size_t)slot * a.chain_stride + (size_t)hb * SR_SEQ_CHAINS + (threadIdx.x & (SR_SEQ_CHAINS - 1))] = (&chains[0][0])[threadIdx.x];
+    }
+    sr_drain_stores();
+    __syncthreads();
+    if (!met(1)) return;
+    for (int g = threadIdx.x; g < nseg; g += kThreads) share[g] = sr_load_agent(&sums[g]);
+    // what the list of a row that is cut holds: everything that can survive its min-p, or enough of the largest for top-p
+    uint32_t from = 0xffffffffu;
+    if (listed) {
+        from = by_mass ? mass_list_from(a.mass + (size_t)slot * kMassBuckets, rd.top_p) : 1u;
+        if (rd.min_p > 0.0f) from = max(from, sr_f2u(fmaxf(__fmul_rn(rd.min_p, 0.999999f), 0.0f)));
+        from = max(from, 1u);
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->list_from = from;
+    }
+    sr_barrier_lds();
+#pragma unroll
+    for (int s = 0; s < kS; s++) {
+        const int seg = seg0 + s * kW;
+        if (seg >= nseg) continue;
         float before = 0.0f;
-        for (int h = lane; h < g; h += SR_WAVE) before += share[h];
+        for (int g = lane; g < seg; g += SR_WAVE) before += share[g];
         before = sr_wave_sum_f32(before);
-        seg_pass2<ES>(a, c, g, lane, xs[0], before, share[g]);
+        seg_make_record(t[s], seg, (double)before, recs + seg, own[s]);
+        if (listed) {
+            // the segment's entries of the list, in the order of their indices, at the segment's own place in the row's lists
+            uint32_t bits = 0u;
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) bits |= sr_f2u(t[s][j]) >= from ? 1u << j : 0u;
+            const int mine = __popc(bits);
+            const int incl = sr_wave_incl_scan_i32(mine);
+            if (lane == SR_WAVE - 1) a.seg_cnt[(size_t)slot * a.seg_stride + seg] = (uint32_t)incl;
+            size_t at = (size_t)slot * (size_t)a.sort_stride + (size_t)seg * SR_SEG_TERMS + (size_t)(incl - mine);
+            if (__ballot(bits != 0u) != 0ull) {
+#pragma unroll
+                for (int j = 0; j < SR_SEQ_RUN; j++)
+                    if ((bits >> j) & 1u) {
+                        a.sort_keys_in[at] = sr_f2u(t[s][j]);
+                        a.sort_vals_in[at] = seg * SR_SEG_TERMS + lane * SR_SEQ_RUN + j;
+                        at++;
+                    }
+            }
+        }
     }
 }
 
@@ -2565,6 +2576,402 @@ __device__ __forceinline__ void sort_survivors_in_place(uint32_t* keys, int32_t*
     }
 }
 
+// ---- the cut of a row whose candidates the pass over the whole device has listed ----------------------------------------
+// a.sort_keys_in / a.sort_vals_in hold, per segment, the entries e >= SrFullState::list_from in the order of their indices,
+// a.seg_cnt how many.  Their values are sorted in shared memory, the min-p threshold and the exact running sum of
+// top-p name the cut, and a nucleus of up to `finish_most` members is normalised and drawn from here; a larger one, and every
+// row whose distribution is handed out, is left to the whole device (k_chain_records ... k_prepared_token): its members
+// are known by the value at the cut and, among equal ones, by the last index.
+// (One workgroup used to count the row's e into a histogram, read the row once per 8,192 entries of its nucleus to list
+// them, and once more to list the members: 113 us a launch of 16 constrained rows of 151,936, of which the listing reads
+// -- 600 KB each at what one compute unit takes in -- were two thirds.)
+enum ListWay : int { kListDone = 0, kListDeferred = 1, kListGeneral = 2 };
+__device__ __forceinline__ int list_place(int i) { return i + (i >> 4); }  // (runs of 16 start in different banks)
+__device__ __forceinline__ int list_cap(bool big) { return big ? SR_LIST_CAP_BIG : SR_LIST_CAP_SMALL; }
+
+__device__ __forceinline__ uint32_t* list_values(uint32_t* more, FullSmem& sm) { return more ? more : (uint32_t*)sm.sortbuf; }
+
+// the row's members are left to the whole device: the factors and the cut, and what k_chain_records and k_prepared_draw
+// need to know of the sums in front of their blocks
+__device__ __forceinline__ void row_deferred(const SrFullArgs& a, SrFullState* st, float inv, float ycut, int idx_last)
+{
+    if (threadIdx.x == 0) {
+        st->mul1 = inv;
+        st->mul2 = 1.0f;
+        st->ycut = ycut;
+        st->idx_last = idx_last;
+        st->deferred = a.seq;
+    }
+}
+
+__device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& rd, SrFullState* st, float* p, int n, int slot, int row,
+                                             bool do_scale, float inv, int N, FullSmem& sm, uint32_t* more)
+{
+    constexpr int kPer = SR_LIST_CAP_BIG / kT;  // entries of a thread
+    const int tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
+    const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f, use_min_p = rd.min_p > 0.0f;
+    const int nseg = seg_count(n);
+    const uint32_t from = st->list_from;
+    const float mp = do_scale ? __fmul_rn(1.0f, inv) : 1.0f;  // the largest probability: the largest e is expf(0) = 1
+    const float thr = use_min_p ? __fmul_rn(rd.min_p, mp) : 0.0f;
+    const int G = more ? SR_LIST_GROUPS_BIG : SR_LIST_GROUPS_SMALL;
+    uint32_t* const grp = list_values(more, sm);
+    uint32_t* const cnt = more ? (uint32_t*)sm.sortbuf : grp + list_place(SR_LIST_CAP_SMALL);
+    uint32_t* const gmin = cnt + G;
+    uint32_t* const gmax = cnt + 2 * G;
+    int* const off = (int*)sm.segst;  // [nseg] where a segment's entries start
+    static_assert(3 * SR_LIST_GROUPS_BIG * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags) &&
+                  (3 * SR_LIST_GROUPS_SMALL + SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16) * 4 <=
+                      sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags), "the tables fit the three arrays");
+    // (behind the barrier that follows the gathering)
+    const int i0 = tid * kPer;
+    const int mine = max(0, min(kPer, N - i0));
+    uint32_t ev[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; r++) ev[r] = r < mine ? grp[list_place(i0 + r)] : 0u;
+    auto prob = [&](uint32_t ebits) -> float { return do_scale ? __fmul_rn(sr_u2f(ebits), inv) : sr_u2f(ebits); };
+
+    // sorted by value: groups of equal width in the bit patterns, counted, placed, and every value ranked inside its group
+    // (groups of one value need no ranks: the equal logits of a coarse grid)
+    for (int i = tid; i < G; i += kT) { cnt[i] = 0u; gmin[i] = 0xffffffffu; gmax[i] = 0u; }
+    if (tid == 0) sm.bc[12] = 0u;
+    __syncthreads();
+    const uint32_t span = 0x3f800000u - min(from, 0x3f800000u);
+    int gshift = 0;
+    while ((span >> gshift) >= (uint32_t)G) gshift++;
+    auto group_of = [&](uint32_t v) -> uint32_t { return min((0x3f800000u - v) >> gshift, (uint32_t)(G - 1)); };
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+        if (r < mine) {
+            const uint32_t g = group_of(ev[r]);
+            atomicAdd(&cnt[g], 1u);
+            atomicMin(&gmin[g], ev[r]);
+            atomicMax(&gmax[g], ev[r]);
+        }
+    __syncthreads();
+    {
+        const int per = G / kT;  // 4 or 2
+        uint32_t c4[SR_LIST_GROUPS_BIG / kT];
+        int own = 0;
+#pragma unroll
+        for (int q = 0; q < SR_LIST_GROUPS_BIG / kT; q++) {
+            c4[q] = q < per ? cnt[tid * per + q] : 0u;
+            own += (int)c4[q];
+            if (c4[q] > 128u && gmin[tid * per + q] != gmax[tid * per + q]) sm.bc[12] = 1u;
+        }
+        int tot;
+        int at = blk_excl_scan(own, &tot, sm);
+#pragma unroll
+        for (int q = 0; q < SR_LIST_GROUPS_BIG / kT; q++)
+            if (q < per) { cnt[tid * per + q] = (uint32_t)at; at += (int)c4[q]; }
+    }
+    __syncthreads();
+    if (sm.bc[12] != 0u) return kListGeneral;
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+        if (r < mine) grp[list_place((int)atomicAdd(&cnt[group_of(ev[r])], 1u))] = ev[r];
+    __syncthreads();  // cnt[g] is now where group g ends
+    {
+        uint32_t v[kPer];
+        int rank[kPer];
+#pragma unroll
+        for (int r = 0; r < kPer; r++) {
+            v[r] = 0u;
+            rank[r] = 0;
+            if (r < mine) {
+                const int i = i0 + r;
+                v[r] = grp[list_place(i)];
+                const uint32_t g = group_of(v[r]);
+                rank[r] = i;
+                if (gmin[g] != gmax[g]) {
+                    const int b = g > 0u ? (int)cnt[g - 1u] : 0, e = (int)cnt[g];
+                    int k = b;
+                    for (int j = b; j < e; j++) {
+                        const uint32_t o = grp[list_place(j)];
+                        k += (o > v[r] || (o == v[r] && j < i)) ? 1 : 0;
+                    }
+                    rank[r] = k;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if (r < mine) grp[list_place(rank[r])] = v[r];
+    }
+    // the survivors of min-p (the largest ones)
+    int ns = N;
+    if (use_min_p) {
+        int c = 0;
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if (r < mine) {
+                const float y = prob(ev[r]);
+                SR_AMB_IF(sr_near(y, thr));  // an entry on the threshold
+                c += y >= thr ? 1 : 0;
+            }
+        ns = blk_sum_i(c, sm);
+    }
+    __syncthreads();
+    if (ns <= 0) return kListGeneral;
+    FPROF(a, slot, 11);
+    int found = -1;
+    if (use_top_p) {
+        if (ns <= SR_WAVE) {
+            // a handful of survivors: one thread adds them the way the scalar loop does
+            if (tid == 0) {
+                float s = 0.0f;
+                int f = -1;
+                for (int i = 0; i < ns && f < 0; i++) {
+                    s = __fadd_rn(s, prob(grp[list_place(i)]));
+                    if (s >= rd.top_p) f = i;
+                }
+                sm.segbc[1] = (uint32_t)f;
+                sm.segbc[2] = sr_f2u(s);
+            }
+            __syncthreads();
+            found = (int)sm.segbc[1];
+        } else {
+            const float run = seq_sum<true>([&](int i) -> float { return prob(grp[list_place(i)]); }, ns, 0.0f, rd.top_p, &found, sm);
+            if (tid == 0) sm.segbc[2] = sr_f2u(run);
+            __syncthreads();
+        }
+        // the list ended before the sum was there, and the row goes on behind it
+        if (found < 0 && from > 1u && !(use_min_p && sr_f2u(__fmul_rn(rd.min_p, 0.999999f)) >= from)) return kListGeneral;
+        if (tid == 0) {
+            const float run = sr_u2f(sm.segbc[2]);
+            if (found >= 0) {
+                const float y = prob(grp[list_place(found)]);
+                SR_AMB_IF(sr_stop_near(run, y, rd.top_p) || (found + 1 < ns && prob(grp[list_place(found + 1)]) == y));
+            } else {
+                SR_AMB_IF(sr_near(run, rd.top_p));
+            }
+        }
+    }
+    const int cutoff = found >= 0 ? found + 1 : ns;
+    const float ycut = prob(grp[list_place(cutoff - 1)]);
+    // Members: everything above the value at the cut, and of the entries equal to it the first ones by index.
+    int gt = 0, eq = 0;
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+        if (r < mine) {
+            const float y = prob(ev[r]);
+            gt += y > ycut ? 1 : 0;
+            eq += y == ycut ? 1 : 0;
+        }
+    int tot_eq;
+    const int eq0 = blk_excl_scan(eq, &tot_eq, sm);
+    const int keep_eq = cutoff - blk_sum_i(gt, sm);
+    uint32_t members = 0u;
+    int last_here = -1;
+    {
+        int k = eq0;
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if (r < mine) {
+                const float y = prob(ev[r]);
+                const bool tie = y == ycut;
+                if (y > ycut || (tie && k < keep_eq)) members |= 1u << r;
+                if (tie && k == keep_eq - 1) last_here = r;
+                k += tie ? 1 : 0;
+            }
+    }
+    const int m = cutoff;
+    const bool finish = a.mode == 0 && m <= a.finish_most;
+    if (!finish && !a.prepared) return kListGeneral;
+    // The members by their places in the list: a bit each, and how many stand in front of every sixteen.  The waves then go
+    // through the segments once more and know the index and the rank of every member they meet.
+    uint16_t* const bits = more ? (uint16_t*)more : (uint16_t*)sm.tags;
+    int* const in_front = (int*)(bits + kT);
+    static_assert(kT * (2 + 4) <= sizeof(FullSmem::tags), "the members' bits fit");
+    if (tid == 0) sm.bc[9] = 0u;
+    {
+        int tot;
+        const int at = blk_excl_scan(__popc(members), &tot, sm);  // (its barriers: the sorted values have been read)
+        bits[tid] = (uint16_t)members;
+        in_front[tid] = at;
+        if (last_here >= 0) sm.bc[10] = (uint32_t)(i0 + last_here);
+    }
+    float* const ssum = (float*)sm.sortbuf;
+    float* const csum = ssum + SR_SEG_MAX;
+    static_assert((SR_SEG_MAX + SR_SEG_MAX / SR_HALF_BLOCK_SEGS * SR_SEQ_CHAINS) * 4 <= sizeof(FullSmem::sortbuf), "the sums fit");
+    if (!finish)
+        for (int i = tid; i < a.chain_stride; i += kT) csum[i] = 0.0f;
+    __syncthreads();
+    FPROF(a, slot, 12);
+    const uint32_t* gk = a.sort_keys_in + (size_t)slot * (size_t)a.sort_stride;
+    const int32_t* gi = a.sort_vals_in + (size_t)slot * (size_t)a.sort_stride;
+    const int last_place = (int)sm.bc[10], nv8 = (n / 8) * 8;
+    for (int s0 = wave; s0 < nseg; s0 += 4 * kW) {
+        uint32_t v[4];
+        int id[4], at[4], len[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int sg = s0 + q * kW;
+            at[q] = sg < nseg ? off[sg] : 0;
+            len[q] = sg < nseg ? (sg + 1 < nseg ? off[sg + 1] : N) - at[q] : 0;
+            v[q] = lane < len[q] ? gk[(size_t)sg * SR_SEG_TERMS + lane] : 0u;
+            id[q] = lane < len[q] ? gi[(size_t)sg * SR_SEG_TERMS + lane] : 0;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int sg = s0 + q * kW;
+            float own = 0.0f;
+            for (int i = lane; i < len[q]; i += SR_WAVE) {
+                const int place = at[q] + i;
+                const uint32_t ebits = i < SR_WAVE ? v[q] : gk[(size_t)sg * SR_SEG_TERMS + i];
+                const int idx = i < SR_WAVE ? id[q] : gi[(size_t)sg * SR_SEG_TERMS + i];
+                if (place == last_place) sm.bc[9] = (uint32_t)idx;
+                const uint32_t b = bits[place >> 4];
+                if (!((b >> (place & 15)) & 1u)) continue;
+                if (finish) {
+                    const int rank = in_front[place >> 4] + __popc(b & ((1u << (place & 15)) - 1u));
+                    sm.sortbuf[rank] = ((unsigned long long)(0xffffffffu - (uint32_t)idx) << 32) | (unsigned long long)sr_f2u(prob(ebits));
+                } else {
+                    own += sr_u2f(ebits);
+                    if (idx < nv8) unsafeAtomicAdd(&csum[idx / (SR_HALF_BLOCK_SEGS * SR_SEG_TERMS) * SR_SEQ_CHAINS + (idx & (SR_SEQ_CHAINS - 1))], sr_u2f(ebits));
+                }
+            }
+            if (!finish && sg < nseg) {
+                own = sr_wave_sum_f32(own);
+                if (lane == 0) ssum[sg] = own;
+            }
+        }
+    }
+    __syncthreads();
+    if (finish) {
+        finish_from_ordered_list(a, p, n, m, row, sm, NoFill(), m <= kSmall ? kSmall : 2 * kSmall);
+        return kListDone;
+    }
+    // left to the whole device: the members' part of every segment and of every half block of the eight accumulators
+    for (int i = tid; i < nseg; i += kT) a.seg_sum[(size_t)slot * a.seg_stride + i] = ssum[i];
+    for (int i = tid; i < a.chain_stride; i += kT) a.chain_sum[(size_t)slot * a.chain_stride + i] = csum[i];
+    row_deferred(a, st, inv, ycut, (int)sm.bc[9]);
+    return kListDeferred;
+}
+
+// ... of a list of at most 64 entries, a sharp row's: by one wave, an entry a lane.  sm.hist[0, N) holds the values of e, sm.hist[64,
+// 64 + N) the indices, in the order of the indices.  (The general way's block-wide steps took 14 us for 20 entries.)
+__device__ __forceinline__ int cut_from_short_list(const SrFullArgs& a, const SrRow& rd, SrFullState* st, float* p, int n, int slot, int row,
+                                                   bool do_scale, float inv, int N, FullSmem& sm)
+{
+    const int tid = threadIdx.x, lane = sr_lane();
+    const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f, use_min_p = rd.min_p > 0.0f;
+    const int nseg = seg_count(n);
+    const uint32_t from = st->list_from;
+    float* const ssum = (float*)sm.sortbuf + 2 * SR_WAVE;  // (behind the members of the list)
+    float* const csum = ssum + SR_SEG_MAX;
+    if (a.mode != 0) {
+        for (int i = tid; i < nseg; i += kT) ssum[i] = 0.0f;
+        for (int i = tid; i < a.chain_stride; i += kT) csum[i] = 0.0f;
+        __syncthreads();
+    }
+    if (sr_wave_id() == 0) {
+        const float mp = do_scale ? __fmul_rn(1.0f, inv) : 1.0f;  // the largest probability: the largest e is expf(0) = 1
+        const float thr = use_min_p ? __fmul_rn(rd.min_p, mp) : 0.0f;
+        const float e = lane < N ? sr_u2f(sm.hist[lane]) : 0.0f;
+        const int idx = lane < N ? (int)sm.hist[SR_WAVE + lane] : 0;
+        const float y = do_scale ? __fmul_rn(e, inv) : e;
+        bool amb = lane < N && use_min_p && sr_near(y, thr);
+        const bool in = lane < N && !(use_min_p && y < thr);
+        const int ns = __popcll(__ballot(in));
+        // place in the order of the values, equal ones by index
+        const float key = in ? y : -1.0f;
+        int rank = 0;
+        for (int j = 0; j < N; j++) {
+            const float o = sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(key), j));
+            rank += (o > key || (o == key && j < lane)) ? 1 : 0;
+        }
+        if (in) sm.sprob[rank] = y;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const float sorted = lane < ns ? sm.sprob[lane] : 0.0f;
+        auto at = [&](int i) -> float { return sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(sorted), i)); };
+        int found = -1;
+        if (use_top_p) {
+            float run = 0.0f;
+            for (int i = 0; i < ns && found < 0; i++) {
+                run = __fadd_rn(run, at(i));
+                if (run >= rd.top_p) found = i;
+            }
+            if (found >= 0) {
+                amb = amb || sr_stop_near(run, at(found), rd.top_p) || (found + 1 < ns && at(found + 1) == at(found));
+            } else if (from > 1u && !(use_min_p && sr_f2u(__fmul_rn(rd.min_p, 0.999999f)) >= from)) {
+                found = -2;  // the list ended before the sum was there, and the row goes on behind it
+            } else {
+                amb = amb || sr_near(run, rd.top_p);
+            }
+        }
+        const int cutoff = found >= 0 ? found + 1 : ns;
+        const bool member = in && rank < cutoff;
+        const unsigned long long ms = __ballot(member);
+        if (__ballot(amb) != 0ull && found != -2 && lane == 0) sm.bc[SR_AMB_WORD] = 1u;
+        if (member) {
+            sm.sortbuf[__popcll(ms & ((1ull << lane) - 1ull))] = ((unsigned long long)(0xffffffffu - (uint32_t)idx) << 32) | (unsigned long long)sr_f2u(y);
+            if (rank == cutoff - 1) { sm.bc[9] = (uint32_t)idx; sm.bc[10] = sr_f2u(y); }
+            if (a.mode != 0) {
+                unsafeAtomicAdd(&ssum[idx / SR_SEG_TERMS], e);
+                if (idx < (n / 8) * 8) unsafeAtomicAdd(&csum[idx / (SR_HALF_BLOCK_SEGS * SR_SEG_TERMS) * SR_SEQ_CHAINS + (idx & (SR_SEQ_CHAINS - 1))], e);
+            }
+        }
+        if (lane == 0) sm.segbc[1] = (uint32_t)(found == -2 ? 0 : cutoff);
+    }
+    __syncthreads();
+    const int m = (int)sm.segbc[1];
+    if (m <= 0) return kListGeneral;
+    if (a.mode == 0) {
+        finish_from_ordered_list(a, p, n, m, row, sm);
+        return kListDone;
+    }
+    for (int i = tid; i < nseg; i += kT) a.seg_sum[(size_t)slot * a.seg_stride + i] = ssum[i];
+    for (int i = tid; i < a.chain_stride; i += kT) a.chain_sum[(size_t)slot * a.chain_stride + i] = csum[i];
+    row_deferred(a, st, inv, sr_u2f(sm.bc[10]), (int)sm.bc[9]);
+    return kListDeferred;
+}
+
+// A row whose workgroups did not meet (SrFullState::late): everything by this workgroup alone, from the logits -- the adjusted
+// row and its maximum as an ordered key (0xffffffff: it holds a NaN), then e in place.  Slow; no launch is known to need it.
+__device__ __forceinline__ float row_alone_logit(const SrFullArgs& a, const char* rowp, const uint32_t* mrow, int i)
+{
+    const float x = a.dtype == 1 ? load_logit<2>(rowp, i) : load_logit<4>(rowp, i);
+    return (mrow && !((mrow[i >> 5] >> (i & 31)) & 1u)) ? SR_NEG_INF : x;
+}
+__device__ __forceinline__ uint32_t row_alone(const SrFullArgs& a, const SrRow& rd, float* p, int n, int row, FullSmem& sm)
+{
+    const int tid = threadIdx.x;
+    const char* rowp = (const char*)a.logits + (size_t)row * (size_t)a.row_stride * (a.dtype == 1 ? 2 : 4);
+    const uint32_t* mrow = (rd.mask_row >= 0) ? a.mask + (size_t)rd.mask_row * a.mask_stride : nullptr;
+    const bool scale = rd.temperature != 1.0f, pen = (rd.flags & SR_ROWFLAG_HAS_PENALTY) != 0u;
+    const float inv_temp = scale ? __fdiv_rn(1.0f, rd.temperature) : 1.0f;
+    for (int i = tid; i < n; i += kT) {
+        const float x = row_alone_logit(a, rowp, mrow, i);
+        p[i] = scale ? __fmul_rn(x, inv_temp) : x;
+    }
+    sr_drain_stores();
+    __syncthreads();
+    const SrEdit* ed = a.edits + rd.edit_off;
+    for (int e = tid; e < rd.edit_cnt; e += kT) {
+        const float x = edited_logit(row_alone_logit(a, rowp, mrow, ed[e].id), ed[e], rd, true, pen);
+        p[ed[e].id] = scale ? __fmul_rn(x, inv_temp) : x;
+    }
+    sr_drain_stores();
+    __syncthreads();
+    uint32_t k = 0u;
+    row_pass<false>(p, n, [&](float x, int) -> float {
+        k = max(k, x != x ? 0xffffffffu : sr_okey(x));
+        return x;
+    });
+    k = (uint32_t)(blk_max_u64((unsigned long long)k, sm));
+    if (k != 0xffffffffu && k > 0x007fffffu) {
+        const float m = sr_okey_inv(k);
+        row_pass<true>(p, n, [&](float x, int) -> float { return sr_expf(__fsub_rn(x, m)); });
+        sr_drain_stores();
+        __syncthreads();
+    }
+    return k;
+}
+
 // ---- stage 3: softmax, top-k, min-p, top-p on the work row --------------------------------------------
 // One workgroup per row, one launch: the row is cut, normalised and drawn from here.  A nucleus that the walk by
 // slabs cannot close has its survivors compacted into the row's sort segment and sorted there by this workgroup.
@@ -2582,15 +2989,11 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
     if (tid == 0) {
         sm.bc[SR_AMB_WORD] = 0u;  // (every path that can set it passes a barrier first)
-        // What the launch after this one expects of the row's scalars: the factors of a row that is not left to its
-        // reader are 1, and the list of entries to watch is empty (the expf pass only appends to it).  No kernel of the
-        // pipeline before this one runs for every row of every launch.
+        // what the reader of a row that is not left to it expects: factors of 1
         st->mul1 = st->mul2 = 1.0f;
-        if (a.watch_cnt) {
-            sm.segbc[3] = a.watch_cnt[slot];
-            a.watch_cnt[slot] = 0u;
-        }
     }
+    // (the next launch of the pass over the whole device finds the row's mass by size at zero)
+    if (a.seg_func && tid < kMassBuckets) a.mass[(size_t)slot * kMassBuckets + tid] = 0.0f;
 
     if (greedy) {
         // Greedy / GreedyWithHistoryPenalties on the adjusted row; distributions become one-hot
@@ -2612,7 +3015,11 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     {
         FPROF(a, slot, 0);
         // Softmax (Sampler.cs:448-472): the maximum and e = expf(x - max) were computed by the kernels before
-        const uint32_t mk = full_maxkey_of(a, st->maxkey);
+        const bool alone = a.seg_func != nullptr && st->late == a.seq;
+        const bool walked = a.seg_func != nullptr && !alone;
+        const bool has_list = walked && row_is_listed(rd, a), plain = walked && row_is_plain(rd, a);
+        float* const e_row = walked ? row_e(a, slot) : p;
+        const uint32_t mk = alone ? row_alone(a, rd, p, n, row, sm) : full_maxkey_of(a, st->maxkey);
         const bool any_nan = mk == 0xffffffffu;
         const float m = mk == 0u ? SR_NEG_INF : sr_okey_inv(mk);
         FPROF(a, slot, 1);
@@ -2638,82 +3045,74 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                 sr_drain_stores();  // (this compute unit has not read these lines before: the loads below find them in L2)
                 __syncthreads();
             }
+            extern __shared__ uint32_t more_lds[];  // when a.big_slabs, else nothing
+            uint32_t* const more = a.big_slabs ? more_lds : nullptr;
             int dummy;
-            // A row that min-p cuts, with no top-k stage before the cut and no distribution to hand out, is not read a
-            // second time for the cut: a survivor has fl(e * inv) >= fl(min_p * inv), so e >= min_p * (1 - 2^-22), and
-            // the few entries that large are listed while the sum passes over them; the exact test follows below.
-            const bool watch_min_p = row_watch_min_p(rd, a);
-            const float e_low = __fmul_rn(rd.min_p, 0.999999f);
-            if (watch_min_p) {
-                if (tid == 0) sm.bc[4] = 0u;
-                __syncthreads();
-            }
-            // A row that only top-p cuts and that is only sampled from: see nucleus_from_histogram
-            const bool fast_nucleus = row_fast_nucleus(rd, a);
-            const bool walked = a.seg_func != nullptr && (!fast_nucleus || a.seg_keys != nullptr);
-            if (fast_nucleus) {
-                uint32_t* hcnt = (uint32_t*)sm.sortbuf;
-                for (int i = tid; i < kHistPos; i += kT) hcnt[i] = 0u;
-                if (tid == 0) sm.bc[5] = 0u;
-                __syncthreads();
-            }
             float sum;
+            int n_list = 0;
             if (walked) {
-                // the whole device has prepared the sum (k_full_softmax_seg): one wave walks the segments' records, and the
-                // entries that can survive the min-p cut were listed by the same pass
+                // the whole device has prepared the sum (k_full_softmax_seg): one wave walks the segments' records while the
+                // others fetch the row's list, if it has one
+                if (has_list) {
+                    const int nseg = seg_count(n);
+                    const int c = tid < nseg ? (int)a.seg_cnt[(size_t)slot * a.seg_stride + tid] : 0;
+                    static_assert(SR_SEG_MAX <= kT, "a thread per segment");
+                    const int o = blk_excl_scan(c, &n_list, sm);
+                    if (tid < nseg) ((int*)sm.segst)[tid] = o;
+                    static_assert(kCkpt >= SR_WAVE, "a word per entry of a short list");
+                    if (n_list <= SR_WAVE)  // where every entry of a short list lies
+                        for (int k = 0; k < c; k++) ((int*)sm.ckpt)[o + k] = tid * SR_SEG_TERMS + k;
+                }
                 __syncthreads();
                 if (sr_wave_id() == 0) {
-                    const float s = seg_walk<false>(p, n, a.seg_func + (size_t)slot * a.seg_stride, 0.0f, 0.0f, &dummy, nullptr);
+                    const float s = seg_walk<false>(e_row, n, a.seg_func + (size_t)slot * a.seg_stride, 0.0f, 0.0f, &dummy, nullptr);
                     if (sr_lane() == 0) sm.segbc[0] = sr_f2u(s);
-                } else if (fast_nucleus) {
-                    // the histogram of e from the 16 bits per entry that the expf pass left
-                    uint32_t* hcnt = (uint32_t*)sm.sortbuf;
-                    const uint16_t* keys = a.seg_keys + (size_t)slot * (size_t)a.seg_key_stride;
-                    auto count = [&](uint32_t key) {
-                        if (key != 0u) {
-                            if (key <= kHistTopKey) atomicAdd(&hcnt[min(kHistTopKey - key, (uint32_t)(kHistPos - 1))], 1u);
-                            else sm.bc[5] = 1u;  // (no e exceeds 1; if one does, the general way takes the row)
-                        }
-                    };
-                    const int n8 = n / 8;  // (the rows of keys start on 16-byte boundaries)
-                    for (int v0 = tid - SR_WAVE; v0 < n8; v0 += 2 * (kT - SR_WAVE)) {
-                        const int v1 = v0 + (kT - SR_WAVE);
-                        const uint4 ka = ((const uint4*)keys)[v0];
-                        const uint4 kb = v1 < n8 ? ((const uint4*)keys)[v1] : make_uint4(0u, 0u, 0u, 0u);
-                        const uint32_t ww[8] = {ka.x, ka.y, ka.z, ka.w, kb.x, kb.y, kb.z, kb.w};
-#pragma unroll
-                        for (int q = 0; q < 8; q++) { count(ww[q] & 0xffffu); count(ww[q] >> 16); }
+                } else if (has_list && n_list <= SR_WAVE) {
+                    const int l = tid - SR_WAVE;
+                    if (l < n_list) {
+                        const size_t at = (size_t)slot * (size_t)a.sort_stride + (size_t)((const int*)sm.ckpt)[l];
+                        sm.hist[l] = a.sort_keys_in[at];
+                        sm.hist[SR_WAVE + l] = (uint32_t)a.sort_vals_in[at];
                     }
-                    for (int i = n8 * 8 + tid - SR_WAVE; i < n; i += kT - SR_WAVE) count(keys[i]);
-                } else if (watch_min_p) {
-                    const uint32_t cw = sm.segbc[3];
-                    const unsigned long long* wl = a.watch + (size_t)slot * kSmall;
-                    for (int i = tid - SR_WAVE; i < (int)min(cw, (uint32_t)kSmall); i += kT - SR_WAVE) sm.sortbuf[i] = wl[i];
-                    if (tid == SR_WAVE) sm.bc[4] = cw;
+                } else if (has_list && n_list <= list_cap(more != nullptr)) {
+                    uint32_t* const grp = list_values(more, sm);
+                    const int nseg = seg_count(n), lane = sr_lane();
+                    const int* off = (const int*)sm.segst;
+                    const uint32_t* gk = a.sort_keys_in + (size_t)slot * (size_t)a.sort_stride;
+                    // (four segments' first entries on their way at a time)
+                    for (int s0 = sr_wave_id() - 1; s0 < nseg; s0 += 4 * (kW - 1)) {
+                        uint32_t v[4];
+                        int at[4], len[4];
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            const int sg = s0 + q * (kW - 1);
+                            at[q] = sg < nseg ? off[sg] : 0;
+                            len[q] = sg < nseg ? (sg + 1 < nseg ? off[sg + 1] : n_list) - at[q] : 0;
+                            v[q] = lane < len[q] ? gk[(size_t)sg * SR_SEG_TERMS + lane] : 0u;
+                        }
+#pragma unroll
+                        for (int q = 0; q < 4; q++) {
+                            const int sg = s0 + q * (kW - 1);
+                            if (lane < len[q]) grp[list_place(at[q] + lane)] = v[q];
+                            for (int i = lane + SR_WAVE; i < len[q]; i += SR_WAVE) grp[list_place(at[q] + i)] = gk[(size_t)sg * SR_SEG_TERMS + i];
+                        }
+                    }
                 }
                 __syncthreads();
                 sum = sr_u2f(sm.segbc[0]);
-            } else if (fast_nucleus) {
-                uint32_t* hcnt = (uint32_t*)sm.sortbuf;
-                sum = seq_sum_row<false>(p, n, 0.0f, 0.0f, &dummy, sm, 1.0f, 1.0f, [&](float x, int) { hist_count(hcnt, &sm.bc[5], x); });
-            } else if (watch_min_p) {
-                sum = seq_sum_row<false>(p, n, 0.0f, 0.0f, &dummy, sm, 1.0f, 1.0f, [&](float x, int i) {
-                    if (x >= e_low) {
-                        const uint32_t pos = atomicAdd(&sm.bc[4], 1u);
-                        if (pos < (uint32_t)kSmall)
-                            sm.sortbuf[pos] = ((unsigned long long)sr_f2u(x) << 32) | (unsigned long long)(0xffffffffu - (uint32_t)i);
-                    }
-                });
             } else {
                 sum = seq_sum_row<false>(p, n, 0.0f, 0.0f, &dummy, sm);
             }
             if (tid == kT - 1) sm.u = u_row;
             __syncthreads();
-            const int n_watched = watch_min_p ? (int)sm.bc[4] : -1;
-            const bool from_watch = n_watched >= 0 && n_watched <= kSmall;  // (else the row is read again, as before)
             FPROF(a, slot, 2);
             const bool do_scale = sum > 0.0f && sum != 1.0f;
             const float inv = do_scale ? __fdiv_rn(1.0f, sum) : 1.0f;
+            if (plain && a.prepared) {
+                row_deferred(a, st, inv, -1.0f, 0);
+                if (tid == 0) st->flags = flags;
+                return;
+            }
             if (a.lazy_scale && a.mode == 1 && !(rd.top_k > 0 && rd.top_k < n) && !(rd.min_p > 0.0f) && !use_top_p) {
                 // No filter touches the row: its final entries are fmul(fmul(e, inv), inv2) with inv2 from the final
                 // Normalize (Sampler.cs:91-92) over the scaled values.  The reader applies the two factors; the row
@@ -2729,10 +3128,40 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                 }
                 return;
             }
-            extern __shared__ uint32_t more_lds[];  // 16 kSmall bytes when a.big_slabs, else nothing
-            const int way = fast_nucleus ? nucleus_from_histogram(a, rd.top_p, p, n, slot, row, do_scale, inv, sm,
-                                                                  a.big_slabs ? more_lds : nullptr)
-                                         : kNucleusGeneral;
+            if (has_list) {
+                int way = kListGeneral;
+                if (n_list > 0 && n_list <= SR_WAVE)
+                    way = cut_from_short_list(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm);
+                else if (n_list > 0 && n_list <= list_cap(more != nullptr))
+                    way = cut_from_list(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm, more);
+                if (way != kListGeneral) {
+                    FPROF(a, slot, 9);
+                    __syncthreads();
+                    if (tid == 0) {
+                        const uint32_t f = flags | (sm.bc[SR_AMB_WORD] ? SR_KFLAG_AMBIGUOUS : 0u);
+                        st->flags = f;
+                        if (way == kListDone && a.out_flags) a.out_flags[row] = f;
+                    }
+                    return;
+                }
+            }
+            if (e_row != p) {
+                // (a row whose list was too long goes on here: its probabilities take shape in the caller's row)
+                for (int i = tid; i < n; i += kT) p[i] = e_row[i];
+                sr_drain_stores();
+                __syncthreads();
+            }
+            const bool fast_nucleus = row_fast_nucleus(rd, a);
+            if (fast_nucleus) {
+                uint32_t* hcnt = (uint32_t*)sm.sortbuf;
+                __syncthreads();
+                for (int i = tid; i < kHistPos; i += kT) hcnt[i] = 0u;
+                if (tid == 0) sm.bc[5] = 0u;
+                __syncthreads();
+                row_pass<false>(p, n, [&](float x, int) -> float { hist_count(hcnt, &sm.bc[5], x); return x; });
+                __syncthreads();
+            }
+            const int way = fast_nucleus ? nucleus_from_histogram(a, rd.top_p, p, n, slot, row, do_scale, inv, sm, more) : kNucleusGeneral;
             no_slabs = way == kNucleusGeneralNoSlabs;
             if (way == kNucleusDone) {
                 FPROF(a, slot, 9);
@@ -2775,20 +3204,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                     return y;
                 };
                 const bool read_only = list_now && a.mode == 0 && n >= 8;
-                if (from_watch) {
-                    // the entries listed during the sum, put to the exact test; the survivors are listed again
-                    static_assert(kSmall % kT == 0, "whole candidates per thread");
-                    unsigned long long cand[kSmall / kT];
-#pragma unroll
-                    for (int r = 0; r < kSmall / kT; r++) cand[r] = (r * kT + tid < n_watched) ? sm.sortbuf[r * kT + tid] : 0ull;
-                    __syncthreads();
-                    if (tid == 0) sm.bc[4] = 0u;
-                    __syncthreads();
-#pragma unroll
-                    for (int r = 0; r < kSmall / kT; r++)
-                        if (r * kT + tid < n_watched)
-                            (void)body(sr_u2f((uint32_t)(cand[r] >> 32)), (int)(0xffffffffu - (uint32_t)cand[r]));
-                } else if (read_only) {
+                if (read_only) {
                     row_pass<false>(p, n, body);
                 } else {
                     row_pass<true>(p, n, body);
@@ -3089,6 +3505,192 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     FPROF(a, slot, 9);
     __syncthreads();
     if (tid == 0 && a.out_flags) a.out_flags[row] = st->flags | (sm.bc[SR_AMB_WORD] ? SR_KFLAG_AMBIGUOUS : 0u);
+}
+
+// ---- rows left to the whole device: final Normalize and draw (Sampler.cs:91-92, :553-576) --------------------------------
+// The members' probabilities y = fl(e inv) are known by the cut (all of them, in a row that nothing cuts).  Three launches
+// instead of one workgroup per row, which took 48 us to pass over 262,144 entries once and such a row passed three times:
+//   k_chain_records   the increment functions of the eight lane accumulators of TensorPrimitives.Sum, a block of 8,192
+//                     entries (1,024 terms of each) to a workgroup, a chain to a wave
+//   k_prepared_draw   every workgroup walks the eight chains (a wave each; the same work in all of them costs less than one
+//                     more launch), then its waves take a segment each: z = fl(y / sum), written where the distribution is
+//                     handed out, and the segment's record for the running sum of the draw
+//   k_prepared_token  one wave per row walks the records to the draw's target
+// 16 rows of 262,144 with top-p or without a filter: 128 -> 31 us behind the pass over the logits.
+struct PreparedRow {
+    const float* e;
+    float inv, ycut;
+    int idx_last, n;
+    __device__ __forceinline__ float cut(float ev, int i) const  // y, or 0 outside the nucleus
+    {
+        const float y = __fmul_rn(ev, inv);
+        return (y > ycut || (y == ycut && i <= idx_last)) ? y : 0.0f;
+    }
+};
+__device__ __forceinline__ PreparedRow prepared_row(const SrFullArgs& a, const SrFullState* st, int slot)
+{
+    PreparedRow r;
+    r.e = row_e(a, slot);
+    r.inv = st->mul1;
+    r.ycut = st->ycut;
+    r.idx_last = st->idx_last;
+    r.n = a.vocab;
+    return r;
+}
+constexpr int kPrepT = 512;
+static_assert(kPrepT / SR_WAVE == SR_SEQ_CHAINS, "a wave per chain");
+__global__ __launch_bounds__(kPrepT) void k_chain_records(SrFullArgs a)
+{
+    __shared__ float buf[8192];
+    const int slot = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
+    const SrFullState* st = a.state + slot;
+    if (st->deferred != a.seq) return;
+    const PreparedRow r = prepared_row(a, st, slot);
+    const int body = (r.n / 8) * 8;
+    float4 v[4];
+#pragma unroll
+    for (int h = 0; h < 4; h++) {  // (the rows of e start on 16-byte boundaries)
+        const int x0 = blk * 8192 + 4 * (tid + h * kPrepT);
+        v[h] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (x0 + 4 <= body) v[h] = *(const float4*)(r.e + x0);  // (body is a multiple of 8)
+    }
+    const float* cs = a.chain_sum + (size_t)slot * a.chain_stride;
+    float before = 0.0f;
+    for (int hb = lane; hb < 2 * blk; hb += SR_WAVE) before += cs[hb * SR_SEQ_CHAINS + wave];
+    before = sr_wave_sum_f32(before) * r.inv;
+    const int hb1 = a.chain_stride / SR_SEQ_CHAINS;
+    float own = cs[2 * blk * SR_SEQ_CHAINS + wave];
+    if (2 * blk + 1 < hb1) own += cs[(2 * blk + 1) * SR_SEQ_CHAINS + wave];
+    // chain by chain in shared memory: the place of term 16 l + j of chain g is g 1024 + 64 j + (l + 2 j) mod 64, so that
+    // the lanes of a wave read a term from 64 consecutive places and a piece's stores fall two to a bank
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+        const int t2 = tid + h * kPrepT, x0 = blk * 8192 + 4 * t2;
+        const int vec = t2 >> 1, j = vec & 15, l = vec >> 4;
+        float* at = buf + (4 * (t2 & 1)) * 1024 + 64 * j + ((l + 2 * j) & 63);
+        at[0] = r.cut(v[h].x, x0); at[1024] = r.cut(v[h].y, x0 + 1); at[2048] = r.cut(v[h].z, x0 + 2); at[3072] = r.cut(v[h].w, x0 + 3);
+    }
+    __syncthreads();
+    float x[SR_SEQ_RUN];
+#pragma unroll
+    for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = buf[wave * 1024 + 64 * j + ((lane + 2 * j) & 63)];
+    seg_make_record(x, blk, (double)before, a.chain_func + ((size_t)slot * SR_SEQ_CHAINS + wave) * a.chain_blocks + blk, own * r.inv);
+}
+
+__global__ __launch_bounds__(kPrepT) void k_prepared_draw(SrFullArgs a)
+{
+    __shared__ float4 turn_all[SR_SEQ_CHAINS][SR_WAVE * 5];
+    __shared__ float lane_sum[SR_SEQ_CHAINS];
+    const int slot = blockIdx.y, lane = sr_lane(), wave = sr_wave_id();
+    SrFullState* st = a.state + slot;
+    if (st->deferred != a.seq) return;
+    const int row = a.row_list[slot];
+    const PreparedRow r = prepared_row(a, st, slot);
+    const int n = r.n, nv = n / 8, rem = n - nv * 8, nblk = (nv + SR_SEG_TERMS - 1) / SR_SEG_TERMS, nseg = seg_count(n);
+    const int seg = (int)blockIdx.x * SR_SEQ_CHAINS + wave;
+    const bool have = seg < nseg && !a.lazy_scale;
+    // the wave's segment is asked for in front of the walk
+    float4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
+        v[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (have && i0 < n) {
+            if (i0 + 4 <= n) {
+                v[k] = *(const float4*)(r.e + i0);
+            } else {
+                v[k].x = r.e[i0];
+                if (i0 + 1 < n) v[k].y = r.e[i0 + 1];
+                if (i0 + 2 < n) v[k].z = r.e[i0 + 2];
+            }
+        }
+    }
+    float before = 0.0f;
+    if (have && a.mode != 1) {
+        const float* sums = a.seg_sum + (size_t)slot * a.seg_stride;
+        for (int g = lane; g < seg; g += SR_WAVE) before += sums[g];
+        before = sr_wave_sum_f32(before);
+    }
+    {
+        int dummy;
+        float s = seg_walk_from<false>([&](int blk, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) {
+                const int t = blk * SR_SEG_TERMS + lane * SR_SEQ_RUN + j, i = t * 8 + wave;
+                x[j] = t < nv ? r.cut(r.e[i], i) : 0.0f;
+            }
+        }, nblk, a.chain_func + ((size_t)slot * SR_SEQ_CHAINS + wave) * a.chain_blocks, 0.0f, 0.0f, &dummy, nullptr);
+        if (rem > 0 && wave >= 8 - rem) s = __fadd_rn(s, r.cut(r.e[n - 8 + wave], n - 8 + wave));  // the overlapped last vector
+        if (lane == 0) lane_sum[wave] = s;
+    }
+    __syncthreads();
+    const float l0 = lane_sum[0], l1 = lane_sum[1], l2 = lane_sum[2], l3 = lane_sum[3], l4 = lane_sum[4], l5 = lane_sum[5],
+                l6 = lane_sum[6], l7 = lane_sum[7];
+    const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
+    const float inv2 = (sum > 0.0f && sum != 1.0f) ? __fdiv_rn(1.0f, sum) : 1.0f;
+    if (blockIdx.x == 0 && threadIdx.x == 0) st->mul2 = inv2;
+    if (!have) return;
+    float* const p = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
+        v[k].x = __fmul_rn(r.cut(v[k].x, i0), inv2); v[k].y = __fmul_rn(r.cut(v[k].y, i0 + 1), inv2);
+        v[k].z = __fmul_rn(r.cut(v[k].z, i0 + 2), inv2); v[k].w = __fmul_rn(r.cut(v[k].w, i0 + 3), inv2);
+        if (a.mode != 0) {
+            if (i0 + 4 <= n) {
+                sr_store_f4(p + i0, v[k].x, v[k].y, v[k].z, v[k].w);
+            } else if (i0 < n) {
+                p[i0] = v[k].x;
+                if (i0 + 1 < n) p[i0 + 1] = v[k].y;
+                if (i0 + 2 < n) p[i0 + 2] = v[k].z;
+            }
+        }
+    }
+    if (a.mode == 1) return;
+    float4* const turn = turn_all[wave];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i = (k * SR_WAVE + lane) * 4;
+        turn[(i >> 4) * 5 + ((i & 15) >> 2)] = v[k];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float t[SR_SEQ_RUN];
+    float own = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float4 q = turn[lane * 5 + k];
+        t[4 * k] = q.x; t[4 * k + 1] = q.y; t[4 * k + 2] = q.z; t[4 * k + 3] = q.w;
+        own += (q.x + q.y) + (q.z + q.w);
+    }
+    own = sr_wave_sum_f32(own);
+    // (the records of the denominator have been walked: theirs take their place)
+    seg_make_record(t, seg, (double)(before * r.inv * inv2), a.seg_func + (size_t)slot * a.seg_stride + seg, own);
+}
+
+__global__ __launch_bounds__(SR_WAVE) void k_prepared_token(SrFullArgs a)
+{
+    const int slot = blockIdx.x, lane = sr_lane();
+    const SrFullState* st = a.state + slot;
+    if (st->deferred != a.seq) return;
+    const int row = a.row_list[slot];
+    const float u = __double2float_rn(a.uniforms[(size_t)row * a.uniforms_per_row]);
+    const PreparedRow r = prepared_row(a, st, slot);
+    const float inv2 = st->mul2;
+    const int n = r.n;
+    auto term = [&](int i) -> float { return i < n ? __fmul_rn(r.cut(r.e[i], i), inv2) : 0.0f; };
+    int found;
+    const float at = seg_walk_from<true>([&](int seg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
+        const int i0 = seg * SR_SEG_TERMS + lane * SR_SEQ_RUN;
+#pragma unroll
+        for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = term(i0 + j);
+    }, seg_count(n), a.seg_func + (size_t)slot * a.seg_stride, 0.0f, u, &found, nullptr);
+    if (lane == 0) {
+        const bool amb = found >= 0 ? sr_stop_near(at, term(found), u) : sr_near(at, u);
+        if (a.out_tokens) a.out_tokens[row] = found >= 0 ? found : n - 1;
+        if (a.out_flags) a.out_flags[row] = st->flags | (amb ? SR_KFLAG_AMBIGUOUS : 0u);
+    }
 }
 
 // ---- SampleTopK (Sampler.cs:216-357) for rows wider than the selection kernel takes -----------------------
@@ -3444,7 +4046,7 @@ __global__ __launch_bounds__(SR_WAVE) void k_spec_walk(SrSpecArgs a)
     if (true_spec) {
         // (every draft accepted, and a bonus token to draw: position L, whose scaled row k_spec_residual writes out)
         if (a.seg_func && rd.temperature > 0.0f) reject = L;
-        const float* pr = a.p_all + (size_t)row * (L + 1) * n;
+        const float* pr = a.p_all + (size_t)row * (L + 1) * (size_t)a.p_stride;
         const double* u = a.uniforms + (size_t)row * a.uniforms_per_row;
         for (int i0 = 0; i0 < L; i0 += SR_WAVE) {
             const int i = i0 + lane;
@@ -3454,7 +4056,7 @@ __global__ __launch_bounds__(SR_WAVE) void k_spec_walk(SrSpecArgs a)
                 bad = (uint32_t)tok >= (uint32_t)n;
                 if (!bad) {
                     const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
-                    const float px = __fmul_rn(__fmul_rn(pr[(size_t)i * n + tok], sl->mul1), sl->mul2);
+                    const float px = __fmul_rn(__fmul_rn(pr[(size_t)i * (size_t)a.p_stride + tok], sl->mul1), sl->mul2);
                     const float qx = a.draft_probs[((size_t)row * L + i) * n + tok];
                     const float acc = qx > 0.0f ? fminf(1.0f, __fdiv_rn(px, qx)) : (px > 0.0f ? 1.0f : 0.0f);
                     stop = !(u[i] < (double)acc);  // (every position before it was accepted and drew one uniform)
@@ -3482,7 +4084,7 @@ __global__ __launch_bounds__(256) void k_spec_residual(SrSpecArgs a)
     if (i < 0) return;
     const int n = a.vocab, L = a.n_draft, lane = sr_lane();
     const bool bonus = i == L;
-    const float* pd = a.p_all + ((size_t)row * (L + 1) + i) * n;
+    const float* pd = a.p_all + ((size_t)row * (L + 1) + i) * (size_t)a.p_stride;
     const float* qd = bonus ? pd : a.draft_probs + ((size_t)row * L + i) * n;
     const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
     const float m1 = sl->mul1, m2 = sl->mul2;
@@ -3549,7 +4151,7 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
     const int row = blockIdx.x;
     const SrRow rd = a.rows[row];
     const int n = a.vocab, L = a.n_draft;
-    const float* pr = a.p_all + (size_t)row * (L + 1) * n;
+    const float* pr = a.p_all + (size_t)row * (L + 1) * (size_t)a.p_stride;
     const float* lg = a.target_logits + (size_t)row * (L + 1) * n;
     const double* u = a.uniforms + (size_t)row * a.uniforms_per_row;
     int* out = a.out_tokens + (size_t)row * (L + 1);
@@ -3569,7 +4171,7 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
             const int tok = a.draft_tokens[(size_t)row * L + i];
             const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
             const bool in_range = (uint32_t)tok < (uint32_t)n;  // an id outside the vocabulary is never dereferenced
-            sm.sprob[i] = in_range ? __fmul_rn(__fmul_rn(pr[(size_t)i * n + tok], sl->mul1), sl->mul2) : 0.0f;
+            sm.sprob[i] = in_range ? __fmul_rn(__fmul_rn(pr[(size_t)i * (size_t)a.p_stride + tok], sl->mul1), sl->mul2) : 0.0f;
             sm.sprob[kStage + i] = (true_spec && in_range) ? a.draft_probs[((size_t)row * L + i) * n + tok] : 0.0f;
             sm.sprob[2 * kStage + i] = __int_as_float(tok);
         }
@@ -3578,7 +4180,7 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
         __syncthreads();
     }
     for (int i = 0; i < L; i++) {
-        const float* pd = pr + (size_t)i * n;
+        const float* pd = pr + (size_t)i * (size_t)a.p_stride;
         const float* qd = a.draft_probs + ((size_t)row * L + i) * n;
         const int tok = staged ? __float_as_int(sm.sprob[2 * kStage + i]) : a.draft_tokens[(size_t)row * L + i];
         const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
@@ -3615,7 +4217,7 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
     }
     if (correction < 0 && !bad_id) {
         // every draft accepted: bonus token from the last position (greedy rows: its argmax, no draw)
-        const float* pd = pr + (size_t)L * n;
+        const float* pd = pr + (size_t)L * (size_t)a.p_stride;
         const SrFullState* sl = a.state + (size_t)row * (L + 1) + L;
         if (rd.temperature <= 0.0f) correction = row_argmax(pd, n, sm);
         else if (a.seg_func && a.reject[row] == L)  // the scaled row and its segments' functions are there
@@ -3780,9 +4382,9 @@ hipError_t sr_launch_wide_tail(const SrFullArgs& a, int n_rows, hipStream_t st)
 hipError_t sr_launch_full_row(const SrFullArgs& a, int n_rows, hipStream_t st)
 {
     if (n_rows <= 0) return hipSuccess;
-    // (rows that only top-p cuts walk their nucleus in slabs of twice the size when the launch gives the room: see
-    // nucleus_from_histogram)
-    const unsigned more = a.big_slabs ? 16u * (unsigned)kSmall : 0u;
+    // (longer lists of candidates, slabs of twice the size: see cut_from_list and nucleus_from_histogram)
+    static_assert((SR_LIST_CAP_BIG + SR_LIST_CAP_BIG / 16) * 4 >= 16 * kSmall, "room for the slabs as well");
+    const unsigned more = a.big_slabs ? (unsigned)((SR_LIST_CAP_BIG + SR_LIST_CAP_BIG / 16) * 4) : 0u;
     if (more) {
         static bool allowed[64] = {};  // (once per device)
         int dev = 0;
@@ -3795,6 +4397,13 @@ hipError_t sr_launch_full_row(const SrFullArgs& a, int n_rows, hipStream_t st)
         }
     }
     hipLaunchKernelGGL(k_full_row, dim3(n_rows), dim3(kT), more, st, a);
+    if (a.prepared) {
+        const int nseg = (a.vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
+        hipLaunchKernelGGL(k_chain_records, dim3((unsigned)a.chain_blocks, n_rows), dim3(kPrepT), 0, st, a);
+        hipLaunchKernelGGL(k_prepared_draw, dim3(a.lazy_scale ? 1u : (unsigned)((nseg + SR_SEQ_CHAINS - 1) / SR_SEQ_CHAINS), n_rows),
+                           dim3(kPrepT), 0, st, a);
+        if (a.mode != 1) hipLaunchKernelGGL(k_prepared_token, dim3(n_rows), dim3(SR_WAVE), 0, st, a);
+    }
     return hipGetLastError();
 }
 hipError_t sr_launch_draw_rows(const float* probs, int64_t stride, int n, int rows, const double* u, int* out,

@@ -49,7 +49,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     const int nseg = (vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
     const bool seg_mode = vocab >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX;
     a.edits_in_pass = seg_mode ? 1 : 0;
-    bool any_table = false, any_copy = false, any_edits = false;
+    bool any_table = false, any_copy = false, any_edits = false, any_list = false, prepared = false;
     int n_sampled = 0, n_seen = 0;
     for (const SrRow& r : (host_rows ? *host_rows : b->h_rows)) {
         if (mode == 0 && r.path != SR_PATH_FULL) continue;
@@ -59,6 +59,13 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
         n_seen++;
         any_edits = any_edits || (r.edit_cnt > 0 && !(on_the_fly && seg_mode));
         any_copy = any_copy || !(r.temperature > 0.0f && (r.edit_cnt <= 0 || on_the_fly));
+        if (seg_mode && r.temperature > 0.0f && !(r.top_k > 0 && r.top_k < vocab)) {
+            any_list = any_list || sr_row_cut(r);
+            // Rows that the row kernel may leave to the whole device: those that nothing cuts, that only top-p cuts (a few
+            // members or tens of thousands), and all of them where distributions are handed out.  A min-p of some size
+            // leaves a few hundred entries at most, and three launches that find nothing to do cost 6 us.
+            prepared = prepared || !sr_row_cut(r) || mode != 0 || !(r.min_p >= 0.002f);
+        }
     }
     a.any_copy = any_copy ? 1 : 0;
     a.any_edits = any_edits ? 1 : 0;
@@ -75,7 +82,6 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     a.state = ctx->full_state.as<SrFullState>();
     if (++ctx->full_seq == 0u) {  // the numbers have gone round: nothing of an earlier launch may look like this one's
         SR_HIP(ctx, hipMemsetAsync(ctx->full_state.p, 0, ctx->full_state.cap, st));
-        if (ctx->full_seg_func.p) SR_HIP(ctx, hipMemsetAsync(ctx->full_seg_func.p, 0, ctx->full_seg_func.cap, st));
         if (ctx->full_row_sync.p) SR_HIP(ctx, hipMemsetAsync(ctx->full_row_sync.p, 0, ctx->full_row_sync.cap, st));
         ctx->full_seq = 1u;
     }
@@ -85,7 +91,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     const int64_t seg_stride = (vocab + 3) & ~3;
     if ((int64_t)n_rows * seg_stride >= (int64_t)1 << 31)
         return sr_fail(ctx, SR_ERR_UNSUPPORTED, "full-vocabulary path: rows x vocab exceeds 2^31 entries");
-    if (any_top_p) {
+    if (any_top_p || any_list) {
         // a row's segment: scratch of its top-p stage (histogram sums, the members of a long nucleus, and the survivors
         // of a row that the walk by slabs cannot close, sorted there by the row's workgroup)
         const size_t items = (size_t)n_rows * seg_stride;
@@ -99,21 +105,35 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     a.sort_stride = seg_stride;
     {
         if (seg_mode) {
-            SR_HIP(ctx, ctx->full_seg_func.reserve((size_t)n_rows * (size_t)nseg * sizeof(SeqSegFunc), st, true));
-            SR_HIP(ctx, ctx->full_seg_ms.reserve((size_t)n_rows * (size_t)nseg * sizeof(float2), st));
-            SR_HIP(ctx, ctx->full_watch.reserve((size_t)n_rows * SR_FULL_SMALL_CAP * sizeof(unsigned long long), st));
-            SR_HIP(ctx, ctx->full_watch_cnt.reserve((size_t)n_rows * sizeof(uint32_t), st, true));
+            const size_t segs = (size_t)n_rows * (size_t)nseg;
+            const int half_blocks = (nseg + SR_HALF_BLOCK_SEGS - 1) / SR_HALF_BLOCK_SEGS;
+            SR_HIP(ctx, ctx->full_seg_func.reserve(segs * sizeof(SeqSegFunc), st));
+            SR_HIP(ctx, ctx->full_seg_sum.reserve(segs * sizeof(float), st));
+            SR_HIP(ctx, ctx->full_seg_cnt.reserve(segs * sizeof(uint32_t), st));
+            SR_HIP(ctx, ctx->full_mass.reserve((size_t)n_rows * 256 * sizeof(float), st, true));
             SR_HIP(ctx, ctx->full_row_sync.reserve((size_t)n_rows * SR_ROW_SYNC_STRIDE * sizeof(unsigned long long), st, true));
             a.row_sync = ctx->full_row_sync.as<unsigned long long>();
             a.seg_func = (SeqSegFunc*)ctx->full_seg_func.p;
-            a.seg_ms = (float2*)ctx->full_seg_ms.p;
+            a.seg_sum = ctx->full_seg_sum.as<float>();
+            a.seg_cnt = ctx->full_seg_cnt.as<uint32_t>();
+            a.mass = ctx->full_mass.as<float>();
             a.seg_stride = nseg;
-            a.watch = ctx->full_watch.as<unsigned long long>();
-            a.watch_cnt = ctx->full_watch_cnt.as<uint32_t>();
-            if (any_top_p && mode == 0) {
-                a.seg_key_stride = ((int64_t)vocab + 7) & ~(int64_t)7;
-                SR_HIP(ctx, ctx->full_seg_keys.reserve((size_t)n_rows * (size_t)a.seg_key_stride * sizeof(uint16_t), st));
-                a.seg_keys = ctx->full_seg_keys.as<uint16_t>();
+            a.chain_stride = half_blocks * 8;
+            a.chain_blocks = (half_blocks + 1) / 2;
+            SR_HIP(ctx, ctx->full_chain_sum.reserve((size_t)n_rows * (size_t)a.chain_stride * sizeof(float), st));
+            SR_HIP(ctx, ctx->full_chain_func.reserve((size_t)n_rows * 8 * (size_t)a.chain_blocks * sizeof(SeqSegFunc), st));
+            a.chain_sum = ctx->full_chain_sum.as<float>();
+            a.chain_func = (SeqSegFunc*)ctx->full_chain_func.p;
+            a.prepared = prepared ? 1 : 0;
+            a.finish_most = prepared ? 1024 : 8192;  // (up to 1,024 members cost the row's workgroup less than the launches behind it)
+            // e = expf(x - max): in the work rows of tokens-only launches and of the verifier (whose reader applies the factors);
+            // apart from the caller's rows where the probabilities take shape there
+            a.e_rows = a.work;
+            a.e_stride = a.work_stride;
+            if (mode != 0 && !lazy_scale) {
+                a.e_stride = seg_stride;
+                SR_HIP(ctx, ctx->work.reserve((size_t)n_rows * (size_t)a.e_stride * sizeof(float), st));
+                a.e_rows = ctx->work.as<float>();
             }
         }
     }
@@ -121,9 +141,9 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     a.uniforms_per_row = b->upr;
     a.out_tokens = out_tokens_dev;
     a.out_flags = out_flags_dev;
-    // With a compute unit per row the row kernel's workgroups can have more shared memory each: rows that only top-p
-    // cuts then walk their nucleus in slabs of twice the size.  (With more rows, two workgroups share a compute unit.)
-    a.big_slabs = (mode == 0 && any_top_p && n_rows <= ctx->cu_count) ? 1 : 0;
+    // With a compute unit per row the row kernel's workgroups can have more shared memory each: longer lists of candidates
+    // and slabs of twice the size.  (With more rows, two workgroups share a compute unit.)
+    a.big_slabs = ((any_top_p || any_list) && n_rows <= ctx->cu_count) ? 1 : 0;
 
     SR_HIP(ctx, sr_launch_full_prep(a, n_rows, st));
     SR_HIP(ctx, sr_launch_full_row(a, n_rows, st));  // (every row is finished by this one launch)
@@ -461,7 +481,8 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
         SR_HIP(ctx, sr_launch_expand_rows(b->d_rows.as<SrRow>(), b->spec_rows.as<SrRow>(), rows, P, st));
         b->spec_positions = P;
     }
-    SR_HIP(ctx, ctx->spec_probs.reserve((size_t)rows * P * V * sizeof(float), st));
+    const int64_t p_stride = ((int64_t)V + 3) & ~(int64_t)3;  // (rows of e start on 16-byte boundaries)
+    SR_HIP(ctx, ctx->spec_probs.reserve((size_t)rows * P * (size_t)p_stride * sizeof(float), st));
     sr_batch tmp;  // a view: expanded rows, the original edits
     tmp.ctx = ctx;
     tmp.rows = rows * P;
@@ -473,7 +494,7 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     const int32_t* list = nullptr;
     int rc = identity_list(ctx, rows * P, &list);
     if (rc == SR_OK)
-        rc = run_full(ctx, &tmp, list, rows * P, any_top_p, target_logits_dev, SR_DTYPE_F32, V, 1, ctx->spec_probs.as<float>(), V,
+        rc = run_full(ctx, &tmp, list, rows * P, any_top_p, target_logits_dev, SR_DTYPE_F32, V, 1, ctx->spec_probs.as<float>(), p_stride,
                       nullptr, nullptr, true, &b->h_rows);  // (the verifier applies the normalising factors of unfiltered rows itself)
     tmp.d_rows.p = nullptr;  // borrowed
     tmp.d_edits.p = nullptr;
@@ -483,6 +504,7 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     a.vocab = V;
     a.n_draft = n_draft;
     a.p_all = ctx->spec_probs.as<float>();
+    a.p_stride = p_stride;
     a.state = ctx->full_state.as<SrFullState>();
     a.target_logits = target_logits_dev;
     a.draft_probs = draft_probs_dev;

@@ -294,7 +294,7 @@ struct sr_ctx {
     DeviceBuf spec_resid, spec_reject;  // ... the residual row of every row's first rejected position, that position
     DeviceBuf seg_part, seg_func;       // approximate sums and increment functions of the segments of prepared rows
     DeviceBuf full_row_sync;
-    DeviceBuf full_seg_func, full_seg_ms, full_watch, full_watch_cnt, full_seg_keys;  // ... of the full-vocabulary path's denominators
+    DeviceBuf full_seg_func, full_seg_sum, full_seg_cnt, full_mass, full_chain_sum, full_chain_func;  // ... of the full-vocabulary path's denominators
     sr_batch* tmp_batch = nullptr;
     PinnedPool pinned;
     HostResults results;

@@ -30,6 +30,9 @@ static inline __host__ __device__ bool sr_row_edits_on_the_fly(const SrRow& rd, 
     return rd.temperature > 0.0f && rd.edit_cnt > 0 && rd.edit_cnt <= SR_FULL_EDIT_VALUES;
 }
 
+// min-p or top-p cuts the row
+static inline __host__ __device__ bool sr_row_cut(const SrRow& rd) { return rd.min_p > 0.0f || (rd.top_p < 1.0f && rd.top_p > 0.0f); }
+
 #define SR_TK_MAX_XCD 16
 struct SrTopkArgs {
     const void* logits;
@@ -137,13 +140,17 @@ struct SrFullState {
     uint32_t flags;
     int32_t n_survivors;  // entries with probability > 0 when top-p starts
     float mul1, mul2;     // the row's entries are to be multiplied by these two, in this order (1 unless lazy_scale)
-    uint32_t late;        // the number of the last launch in which a workgroup of the row stopped waiting at the meeting point
-    int32_t pad;
+    uint32_t late;        // the number of the last launch in which a workgroup of the row stopped waiting at a meeting point
+    uint32_t deferred;    // the number of the last launch that left the row's normalisation and draw to the whole device
+    float ycut;           // ... whose members are the probabilities above ycut, and of those equal to it the ones up to idx_last
+    int32_t idx_last;
+    uint32_t list_from;   // the row's list of candidates holds its e from this value on (as bits)
+    int32_t pad[5];
 };
-static_assert(sizeof(SrFullState) == 32, "the 8-byte word, aligned, in front");
+static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // SrFullArgs::row_sync, a word per row (rows 256 bytes apart: every workgroup of a row adds to its word and polls it):
-// launch number << 32 | workgroups of k_full_softmax_seg behind the row's meeting point << 16 | workgroups counted in.
-// The number is put in by an atomic maximum before the first count of a launch, so nothing clears the words.
+// launch number << 32 | workgroups of k_full_softmax_seg at the second meeting point << 16 | at the first.  The number is
+// put in by an atomic maximum before the first count of a launch, so nothing clears the words.
 #define SR_ROW_SYNC_STRIDE 32
 
 struct SeqSegFunc;
@@ -179,13 +186,18 @@ struct SrFullArgs {
     // The softmax denominators prepared by the whole device (k_full_softmax_seg, seg_walk); seg_func is
     // null when the launch is not laid out for it (short or unaligned rows) and the rows are added by their workgroups.
     SeqSegFunc* seg_func;          // [slot][seg_stride]
-    float2* seg_ms;                // [slot][seg_stride], 8 bytes each: a segment's maximum m (as an ordered key) and the
-                                   // sum of exp(x - m) over it, approximately
     int32_t seg_stride;
-    unsigned long long* watch;     // [slot][SR_FULL_SMALL_CAP]: the entries that can survive a row's min-p cut (value << 32 | ~index)
-    uint32_t* watch_cnt;           // [slot]
-    uint16_t* seg_keys;            // [slot][seg_key_stride]: the upper 16 bits of every e of a row that only top-p cuts (0: e = 0)
-    int64_t seg_key_stride;
+    float* seg_sum;                // [slot][seg_stride] about the sum of every segment's e (of its members, in a row that is cut)
+    float* chain_sum;              // [slot][chain_stride] ... of every half block's share of each of the eight lane accumulators
+    int32_t chain_stride;
+    int32_t chain_blocks;
+    SeqSegFunc* chain_func;        // [slot][8][chain_blocks]
+    float* mass;                   // [slot][256] the row's mass by size of e; zero between launches
+    uint32_t* seg_cnt;             // [slot][seg_stride] entries of every segment in the row's list (sort_keys_in, sort_vals_in)
+    float* e_rows;                 // [slot][e_stride] expf(x - max) of the rows; starts on 16 bytes
+    int64_t e_stride;
+    int32_t prepared;              // the launches behind k_full_row follow: it may leave rows to the whole device
+    int32_t finish_most;           // members up to which k_full_row normalises and draws by itself
     uint32_t seq;                  // the launch's number (never 0): see SrFullState::maxkey
     int32_t n_sampled;             // rows of the launch with a temperature above 0 (greedy rows leave the passes at once)
     int32_t any_edits;             // some row of the launch has edits for k_full_edits (else it is not launched)
@@ -193,7 +205,7 @@ struct SrFullArgs {
                                    // need no table either (k_full_softmax_seg applies their edits where it loads the row)
     unsigned long long* row_sync;  // [slot * SR_ROW_SYNC_STRIDE]
     uint32_t row_wait_limit;       // polls of a row's count before a workgroup of k_full_softmax_seg stops waiting for it
-    int32_t big_slabs;             // k_full_row gets 64 KB of shared memory more: slabs of 8,192 entries for rows that only top-p cuts
+    int32_t big_slabs;             // k_full_row gets 68 KB of shared memory more: lists of 16,384 candidates, slabs of 8,192 entries
 };
 hipError_t sr_launch_full_prep(const SrFullArgs& a, int n_rows, hipStream_t st);
 hipError_t sr_launch_full_row(const SrFullArgs& a, int n_rows, hipStream_t st);
@@ -217,7 +229,7 @@ hipError_t sr_launch_residual_rows(const float* p, int64_t ps, const float* q, i
 #define SR_SEG_PLAIN 0u
 #define SR_SEG_EXACT 1u
 #define SR_SEG_SPLIT 2u
-#define SR_SEG_LATE 3u   // no record yet: left by a workgroup that stopped waiting, with the launch's number in a0
+#define SR_SEG_ZERO 3u   // no term above zero: no sum changes
 struct SeqSegFunc {  // 96 bytes
     uint32_t a0, a1;
     int32_t eb;
@@ -231,7 +243,8 @@ struct SrSpecArgs {
     const SrRow* rows;
     int32_t vocab;
     int32_t n_draft;
-    const float* p_all;          // [rows][n_draft + 1][vocab] filtered target distributions, to be multiplied by ...
+    const float* p_all;          // [rows][n_draft + 1][p_stride] filtered target distributions, to be multiplied by ...
+    int64_t p_stride;
     const SrFullState* state;    // ... mul1 and mul2 of [rows][n_draft + 1]
     const float* target_logits;  // [rows][n_draft + 1][vocab]
     const float* draft_probs;    // [rows][n_draft][vocab]

@@ -102,4 +102,10 @@ struct SrMaskClear {
 #define SR_FULL_SMALL_CAP 4096
 #define SR_SEG_TERMS 1024                  // terms per segment of a sum that the whole device prepares (64 lanes x 16)
 #define SR_SEG_MIN_VOCAB 4096              // shorter rows are not worth the preparation
+#define SR_HALF_BLOCK_SEGS 4               // segments of a half block of the final Normalize's eight accumulators (4,096 entries)
+// candidates of a row that k_full_row sorts, and the groups it sorts them by: with a compute unit to itself, and without
+#define SR_LIST_CAP_BIG 16384
+#define SR_LIST_CAP_SMALL 4096
+#define SR_LIST_GROUPS_BIG 4096
+#define SR_LIST_GROUPS_SMALL 2048
 #define SR_SEG_MAX 1024                    // most segments of such a row: longer rows are added the plain way
