@@ -808,6 +808,29 @@ template <int kMask> __device__ __forceinline__ uint32_t lane_xor_u32(uint32_t v
     const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
     return (sr_lane() & 32) ? r[0] : r[1];
 }
+// The wave's sums of eight values per lane: lane l returns that of c[l & 7].  (Three exchanges halve what a lane holds, three
+// more add up the groups of eight lanes: ten additions where eight sums by themselves take 48.)
+__device__ __forceinline__ float wave_sum_8(const float (&c)[8])
+{
+    const int lane = sr_lane();
+    float h[4], q[2];
+    const bool b4 = (lane & 4) != 0, b2 = (lane & 2) != 0, b1 = (lane & 1) != 0;
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+        const float keep = b4 ? c[g + 4] : c[g], send = b4 ? c[g] : c[g + 4];
+        h[g] = keep + sr_u2f(lane_xor_u32<4>(sr_f2u(send)));
+    }
+#pragma unroll
+    for (int g = 0; g < 2; g++) {
+        const float keep = b2 ? h[g + 2] : h[g], send = b2 ? h[g] : h[g + 2];
+        q[g] = keep + sr_u2f(lane_xor_u32<2>(sr_f2u(send)));
+    }
+    float v = (b1 ? q[1] : q[0]) + sr_u2f(lane_xor_u32<1>(sr_f2u(b1 ? q[0] : q[1])));
+    v += sr_u2f(lane_xor_u32<8>(sr_f2u(v)));
+    v += sr_u2f(lane_xor_u32<16>(sr_f2u(v)));
+    v += sr_u2f(lane_xor_u32<32>(sr_f2u(v)));
+    return v;
+}
 template <int kMask> __device__ __forceinline__ unsigned long long lane_xor_key(unsigned long long v)
 {
     return ((unsigned long long)lane_xor_u32<kMask>((uint32_t)(v >> 32)) << 32) | (unsigned long long)lane_xor_u32<kMask>((uint32_t)v);
@@ -1058,7 +1081,7 @@ __device__ __forceinline__ void hist_count(uint32_t* hcnt, uint32_t* bad, float 
 // row's workgroup finds the cut in that list.  (Not where a verifier reads e in place.)
 __device__ __forceinline__ bool row_is_listed(const SrRow& rd, const SrFullArgs& a)
 {
-    return !a.lazy_scale && a.seg_func != nullptr && rd.temperature > 0.0f && sr_row_cut(rd) && !(rd.top_k > 0 && rd.top_k < a.vocab);
+    return !a.lazy_scale && (a.mode == 0 || a.prepared) && a.seg_func != nullptr && rd.temperature > 0.0f && sr_row_cut(rd) && !(rd.top_k > 0 && rd.top_k < a.vocab);
 }
 // A sampled row that nothing cuts.
 __device__ __forceinline__ bool row_is_plain(const SrRow& rd, const SrFullArgs& a)
@@ -1446,16 +1469,16 @@ __device__ __forceinline__ void seg_apply_edits(const SrFullArgs& a, const SrRow
 // take a fast exponential of every element, for approximate sums relative to the segment's own maximum, to save the second
 // meeting; the sums come from e itself now, which costs a meeting of 2 - 3 us and a quarter fewer instructions.
 
+constexpr uint32_t kKeyInf = 0xff800000u;  // +inf as an ordered key; above it: a NaN
 // a segment's largest value as an ordered key; 0xffffffff = it holds a NaN (which propagates: TensorPrimitives.Max)
 __device__ __forceinline__ uint32_t seg_max_key(const float (&x)[SR_SEQ_RUN])
 {
     float m = x[0];
-    bool nan = x[0] != x[0];
+    bool nan = false;
 #pragma unroll
-    for (int j = 1; j < SR_SEQ_RUN; j++) {
-        m = sr_max_f32(m, x[j]);
-        nan = nan || x[j] != x[j];
-    }
+    for (int j = 1; j < SR_SEQ_RUN; j++) m = sr_max_f32(m, x[j]);
+#pragma unroll
+    for (int j = 0; j < SR_SEQ_RUN; j += 2) nan = nan || __builtin_isunordered(x[j], x[j + 1]);
     return nan ? 0xffffffffu : sr_okey(m);
 }
 // The mass of a row's e by size: kMassBuckets buckets, eight to a doubling, bucket 0 just below 1, the last one everything
@@ -1491,8 +1514,16 @@ __device__ __forceinline__ uint32_t mass_list_from(const float* mass, float shar
     return 0x3f800000u - ((uint32_t)(d + 1) << 20) + 1u;
 }
 
+// The smallest e that can be a survivor of the row's min-p or so near its threshold that the row counts as ambiguous: the
+// probabilities fl(e inv) and the threshold fl(min_p inv) are three roundings apart at most -- where they are normal
+// numbers (inv is 1 / 2^20 at least); a smaller min_p bounds nothing.
+__device__ __forceinline__ uint32_t min_p_list_from(const SrRow& rd)
+{
+    return rd.min_p >= 1e-30f ? sr_f2u(__fmul_rn(rd.min_p, 1.0f - 2.0f * SR_AMBIG_REL - 1e-6f)) : 0u;
+}
+
 template <int ES, int kW, int kS>
-__global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_seg(SrFullArgs a)
+__global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_seg(SrFullArgs a)
 {
     constexpr int kThreads = kW * SR_WAVE;
     constexpr int E = 16 / ES, K = SR_SEG_TERMS / (SR_WAVE * E);
@@ -1505,7 +1536,8 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
     // a wave's segment on its way from the order of the loads to 16 terms a lane: a lane's 16 terms lie together, 16
     // bytes apart from the next lane's, so that neither the stores nor the loads of 16 bytes a lane collide on a bank
     __shared__ float4 turn_all[kW][SR_WAVE * 5];
-    __shared__ float share[SR_SEG_MAX];   // every segment's part of the row's sum
+    float* const share = (float*)&turn_all[0][0];  // every segment's part of the row's sum (behind the second meeting)
+    static_assert(SR_SEG_MAX * sizeof(float) <= sizeof(turn_all), "in the same place");
     __shared__ float mass[kMassBuckets];  // this workgroup's part of the row's mass by size of e
     __shared__ float chains[kS][SR_SEQ_CHAINS];
     __shared__ uint32_t wkey[kW];
@@ -1524,10 +1556,11 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
     if (threadIdx.x < 32) tab[threadIdx.x] = sr_exp2f_tab[threadIdx.x];
     const SegSource<ES> src = seg_source<ES>(rd, a, slot, row);
     float* const w = row_e(a, slot);
-    const bool plain = row_is_plain(rd, a), listed = row_is_listed(rd, a);
+    const bool plain = a.prepared && row_is_plain(rd, a), listed = row_is_listed(rd, a);
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
-    // (a min-p cut that leaves a few hundred entries at most needs no second bound)
-    const bool by_mass = listed && use_top_p && rd.min_p < 0.01f;
+    // (a row that min-p cuts as well lists everything down to its threshold: entries on it count for SR_OUT_AMBIGUOUS wherever
+    // top-p ends)
+    const bool by_mass = listed && use_top_p && !(rd.min_p > 0.0f);
     // (the row's sum is at least 1: n entries below this make up less than half of what top-p leaves out)
     const float mass_min = (1.0f - rd.top_p) * 0.5f / (float)n;
     if (by_mass)
@@ -1625,7 +1658,9 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
     }
     if (!met(0)) return;
     const uint32_t mk = bc[1];
-    if (mk == 0xffffffffu || mk <= 0x007fffffu) return;  // a NaN, or nothing above -inf: the row's workgroup makes it uniform
+    // A NaN, or nothing above -inf: the row's workgroup makes it uniform.  A maximum of +inf, beside which e is no number where it
+    // stands: the row's workgroup takes the row alone, so that every x - max below is at most 0, or -inf.
+    if (mk >= kKeyInf || mk <= 0x007fffffu) return;
     const float m = sr_okey_inv(mk);
 
     // e of the wave's segments: written to the row, counted by size, and turned into the order of the sum
@@ -1640,10 +1675,10 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
         // (a whole segment without a test per element: the 16 chains of a lane then run interleaved)
         if ((seg + 1) * SR_SEG_TERMS <= n) {
 #pragma unroll
-            for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = sr_expf_tab(__fsub_rn(t[s][j], m), tab);
+            for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = sr_expf_neg(__fsub_rn(t[s][j], m), tab);
         } else {
 #pragma unroll
-            for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = seg_elem<ES>(seg, lane, j) < n ? sr_expf_tab(__fsub_rn(t[s][j], m), tab) : 0.0f;
+            for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = seg_elem<ES>(seg, lane, j) < n ? sr_expf_neg(__fsub_rn(t[s][j], m), tab) : 0.0f;
         }
 #pragma unroll
         for (int k2 = 0; k2 < K; k2++) {
@@ -1696,11 +1731,11 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
         __builtin_amdgcn_wave_barrier();
         if (plain) {
             // the segment's part of the eight lane accumulators of the final Normalize
+            float c[SR_SEQ_CHAINS];
 #pragma unroll
-            for (int g = 0; g < SR_SEQ_CHAINS; g++) {
-                const float c = sr_wave_sum_f32(t[s][g] + t[s][g + 8]);
-                if (lane == 0) unsafeAtomicAdd(&chains[s][g], c);
-            }
+            for (int g = 0; g < SR_SEQ_CHAINS; g++) c[g] = t[s][g] + t[s][g + 8];
+            const float mine = wave_sum_8(c);
+            if (lane < SR_SEQ_CHAINS) unsafeAtomicAdd(&chains[s][lane], mine);
         }
         if (lane == 0) sr_store_agent(&sums[seg], own[s]);
     }
@@ -1721,7 +1756,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 2 ? 5 : 3) void k_full_softmax_
     uint32_t from = 0xffffffffu;
     if (listed) {
         from = by_mass ? mass_list_from(a.mass + (size_t)slot * kMassBuckets, rd.top_p) : 1u;
-        if (rd.min_p > 0.0f) from = max(from, sr_f2u(fmaxf(__fmul_rn(rd.min_p, 0.999999f), 0.0f)));
+        from = max(from, min_p_list_from(rd));
         from = max(from, 1u);
         if (blockIdx.x == 0 && threadIdx.x == 0) st->list_from = from;
     }
@@ -2737,7 +2772,9 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
             __syncthreads();
         }
         // the list ended before the sum was there, and the row goes on behind it
-        if (found < 0 && from > 1u && !(use_min_p && sr_f2u(__fmul_rn(rd.min_p, 0.999999f)) >= from)) return kListGeneral;
+        if (found < 0 && from > 1u && min_p_list_from(rd) < from) return kListGeneral;
+        // ... or an entry behind the list's end shares the probability at the cut
+        if (found >= 0 && from > 1u && prob(from - 1u) >= prob(grp[list_place(found)])) return kListGeneral;
         if (tid == 0) {
             const float run = sr_u2f(sm.segbc[2]);
             if (found >= 0) {
@@ -2895,10 +2932,13 @@ __device__ __forceinline__ int cut_from_short_list(const SrFullArgs& a, const Sr
                 run = __fadd_rn(run, at(i));
                 if (run >= rd.top_p) found = i;
             }
-            if (found >= 0) {
+            const float behind = from > 1u ? __fmul_rn(sr_u2f(from - 1u), do_scale ? inv : 1.0f) : -1.0f;
+            if (found >= 0 ? behind >= at(found) : from > 1u && min_p_list_from(rd) < from) {
+                // the list ended before the sum was there, and the row goes on behind it -- or an entry behind the list's
+                // end shares the probability at the cut
+                found = -2;
+            } else if (found >= 0) {
                 amb = amb || sr_stop_near(run, at(found), rd.top_p) || (found + 1 < ns && at(found + 1) == at(found));
-            } else if (from > 1u && !(use_min_p && sr_f2u(__fmul_rn(rd.min_p, 0.999999f)) >= from)) {
-                found = -2;  // the list ended before the sum was there, and the row goes on behind it
             } else {
                 amb = amb || sr_near(run, rd.top_p);
             }
@@ -3015,7 +3055,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     {
         FPROF(a, slot, 0);
         // Softmax (Sampler.cs:448-472): the maximum and e = expf(x - max) were computed by the kernels before
-        const bool alone = a.seg_func != nullptr && st->late == a.seq;
+        const bool alone = a.seg_func != nullptr && (st->late == a.seq || full_maxkey_of(a, st->maxkey) == kKeyInf);
         const bool walked = a.seg_func != nullptr && !alone;
         const bool has_list = walked && row_is_listed(rd, a), plain = walked && row_is_plain(rd, a);
         float* const e_row = walked ? row_e(a, slot) : p;
@@ -3516,7 +3556,8 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
 //                     more launch), then its waves take a segment each: z = fl(y / sum), written where the distribution is
 //                     handed out, and the segment's record for the running sum of the draw
 //   k_prepared_token  one wave per row walks the records to the draw's target
-// 16 rows of 262,144 with top-p or without a filter: 128 -> 31 us behind the pass over the logits.
+// Distributions and tokens of 16 rows of 262,144 with top-p or without a filter: 150 -> 85 us a call; tokens of 32 ragged bf16
+// rows of 100,003: 98 -> 76.
 struct PreparedRow {
     const float* e;
     float inv, ycut;
@@ -4333,16 +4374,21 @@ hipError_t sr_launch_full_prep(const SrFullArgs& a, int n_rows, hipStream_t st)
     }
     if (a.seg_func) {
         const int nseg = (a.vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
-        // a wave takes one segment, or two where the launch's sampled rows have more segments than the device holds waves
-        // of the one-segment kind at a time: the waves of a row's workgroups wait for each other between the passes
-        const bool two = (long long)a.n_sampled * nseg > 3072;
-        const int per_group = 4 * (two ? 2 : 1);
+        // A wave takes one segment, or two where the launch's sampled rows have more segments than half of the device's waves:
+        // the workgroups of a row wait for each other between the passes, and fewer of them wait less (16 rows of 262,144
+        // fp32: 33 -> 26 us, 64 of 151,936: 55 -> 36).  Below, one and two measure the same, and one starts sooner (a row
+        // of 151,936, whole step: 56.6 against 58.9 us).  Four for the verifier's large launches, whose waves keep nothing
+        // else in registers (144 rows of 262,144: 98 -> 92 us; 36 rows: 119.6 -> 121.6 a call).
+        const long long segs = (long long)a.n_sampled * nseg;
+        const bool four = a.lazy_scale && a.dtype != 1 && segs > 12288, two = segs > 3072;
+        const int per_group = 4 * (four ? 4 : two ? 2 : 1);
         dim3 fgrid((unsigned)((nseg + per_group - 1) / per_group), n_rows);
         if (a.dtype == 1) {
             if (two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2>), fgrid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 1>), fgrid, dim3(256), 0, st, a);
         } else {
-            if (two) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 2>), fgrid, dim3(256), 0, st, a);
+            if (four) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 4>), fgrid, dim3(256), 0, st, a);
+            else if (two) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 2>), fgrid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 1>), fgrid, dim3(256), 0, st, a);
         }
     } else if (a.dtype == 1) {

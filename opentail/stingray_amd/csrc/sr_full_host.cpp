@@ -67,6 +67,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             prepared = prepared || !sr_row_cut(r) || mode != 0 || !(r.min_p >= 0.002f);
         }
     }
+    prepared = prepared && (long long)n_rows * nseg <= (lazy_scale ? SR_PREPARED_SEGS_VERIFY : mode != 0 ? SR_PREPARED_SEGS_DISTRIBUTIONS : SR_PREPARED_SEGS);
     a.any_copy = any_copy ? 1 : 0;
     a.any_edits = any_edits ? 1 : 0;
     a.n_sampled = (int)((long long)n_sampled * n_rows / std::max(1, n_seen));  // (a verifier's launch has every row several times)
@@ -130,7 +131,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             // apart from the caller's rows where the probabilities take shape there
             a.e_rows = a.work;
             a.e_stride = a.work_stride;
-            if (mode != 0 && !lazy_scale) {
+            if (mode != 0 && !lazy_scale && prepared) {
                 a.e_stride = seg_stride;
                 SR_HIP(ctx, ctx->work.reserve((size_t)n_rows * (size_t)a.e_stride * sizeof(float), st));
                 a.e_rows = ctx->work.as<float>();

@@ -103,6 +103,14 @@ struct SrMaskClear {
 #define SR_SEG_TERMS 1024                  // terms per segment of a sum that the whole device prepares (64 lanes x 16)
 #define SR_SEG_MIN_VOCAB 4096              // shorter rows are not worth the preparation
 #define SR_HALF_BLOCK_SEGS 4               // segments of a half block of the final Normalize's eight accumulators (4,096 entries)
+// Segments of all of a launch's rows up to which it leaves its long rows to the whole device.  The row's own workgroup costs about
+// the same for one row and for 256; the launches behind it cost 25 us and what the rows hold together: tokens of 192
+// rows of 151,936 (28,608 segments) 182 -> 159 us, distributions of 64 rows 132 -> 109 and of 128 rows (19,072) 161 -> 164;
+// the verifier, where the workgroup passes over its row once and not three times: 24 rows of 262,144 (6,144) 108 -> 103, 36
+// rows 118.5 -> 119.6.
+#define SR_PREPARED_SEGS 32768
+#define SR_PREPARED_SEGS_DISTRIBUTIONS 16384
+#define SR_PREPARED_SEGS_VERIFY 8192
 // candidates of a row that k_full_row sorts, and the groups it sorts them by: with a compute unit to itself, and without
 #define SR_LIST_CAP_BIG 16384
 #define SR_LIST_CAP_SMALL 4096

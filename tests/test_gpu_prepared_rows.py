@@ -1,0 +1,74 @@
+"""Rows of the full-vocabulary path whose cut comes from a list of candidates and whose normalisation and draw are left to
+the whole device: the sizes at which segments, half blocks and blocks end, coarse logits (runs of equal probabilities across
+the cut), lists that are empty, short, longer than they may be, and launches with too many rows for that way."""
+import numpy as np
+import pytest
+import torch
+
+from opentail.stingray_amd import SamplerContext, SamplingParams
+from oracle import binding as orc
+from tests.helpers import oracle_tokens, to_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = SamplerContext(0)
+    yield c
+    c.close()
+
+
+PARAMS = [SamplingParams(), SamplingParams(Temperature=0.7, TopP=0.9), SamplingParams(Temperature=1.3, TopP=0.999),
+          SamplingParams(TopP=1e-6), SamplingParams(Temperature=0.8, MinP=1e-4), SamplingParams(MinP=1e-3, TopP=0.95),
+          SamplingParams(Temperature=2.0, TopP=0.5), SamplingParams(MinP=1e-34, TopP=0.9),
+          SamplingParams(Temperature=0.9, TopP=0.97, FrequencyPenalty=0.3, PreviousTokens=[5, 4000, 5, 17])]
+
+
+def _check(ctx, logits, dev, params, rng):
+    for r, u in enumerate([rng.random(len(params)), np.zeros(len(params)), np.full(len(params), 1.0 - 2.0 ** -53)]):
+        got = ctx.sample_batch(dev, params, u)
+        assert np.array_equal(got, oracle_tokens(logits, params, u)), (logits.shape, r)
+    tokens, probs = ctx.sample_with_distribution(dev, params, u)
+    probs = probs.cpu().numpy()
+    assert np.array_equal(tokens, got), logits.shape
+    for r, p in enumerate(params):
+        want = orc.build_filtered_distribution(logits[r], to_oracle(p))
+        assert np.array_equal(probs[r].view(np.uint32), want.view(np.uint32)), (logits.shape, r)
+
+
+@pytest.mark.parametrize("vocab", [4096, 4097, 5119, 8191, 8200, 16385, 65_537, 151_936])
+@pytest.mark.parametrize("kind", ["f32", "bf16", "coarse"])
+def test_rows_prepared_by_the_whole_device(ctx, vocab, kind):
+    rng = np.random.default_rng(vocab)
+    x = torch.from_numpy(rng.normal(0, 1.5, (len(PARAMS), vocab)).astype(np.float32))
+    if kind == "bf16":
+        x = x.to(torch.bfloat16)
+    elif kind == "coarse":
+        x = torch.round(x * 2) / 2
+    _check(ctx, x.float().numpy(), x.cuda(), PARAMS, rng)
+
+
+def test_rows_with_a_sharp_head_and_rows_with_equal_logits(ctx):
+    rng = np.random.default_rng(3)
+    logits = rng.normal(0, 1.5, (len(PARAMS), 20_011)).astype(np.float32)
+    logits[:, 4_321] = 40.0                        # lists of a single entry
+    _check(ctx, logits, torch.from_numpy(logits).cuda(), PARAMS, rng)
+    logits[:] = 0.25                               # every entry in the first bucket
+    _check(ctx, logits, torch.from_numpy(logits).cuda(), PARAMS, rng)
+    logits[:, 9:] = float("-inf")
+    _check(ctx, logits, torch.from_numpy(logits).cuda(), PARAMS, rng)
+
+
+def test_launches_of_more_rows_than_the_whole_device_takes(ctx):
+    rng = np.random.default_rng(4)
+    base = rng.normal(0, 1.5, (len(PARAMS), 66_000)).astype(np.float32)
+    rows = 520                                     # 65 segments each: beyond the limits of tokens and distributions
+    params = [PARAMS[i % len(PARAMS)] for i in range(rows)]
+    u = np.repeat(rng.random(rows // len(PARAMS) + 1), len(PARAMS))[:rows]
+    dev = torch.from_numpy(base).cuda()[torch.arange(rows, device="cuda") % len(PARAMS)].contiguous()
+    got = ctx.sample_batch(dev, params, u)
+    want = oracle_tokens(base[np.arange(18) % len(PARAMS)], params[:18], u[:18])
+    assert np.array_equal(got[:18], want)
+    few = ctx.sample_batch(dev[:90], params[:90], u[:90])
+    assert np.array_equal(got[:90], few)
