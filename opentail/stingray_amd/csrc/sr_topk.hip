@@ -2209,6 +2209,7 @@ __device__ __forceinline__ void copy_piece(const SrCopySeg& s, int block, int bl
 
 // With pieces.n > 0 the workgroups behind the scan_blocks first ones put the pieces of an upload in their places, one
 // workgroup to a piece (small uploads: see prepare_scan).
+constexpr int kMaskAhead = 10;
 __global__ __launch_bounds__(kThreads) void k_build_scan_mask(const SrScanDesc* descs, const int32_t* scan_ids,
                                                               const SrRow* rows, const SrEdit* edits,
                                                               const uint32_t* mask, int64_t mask_stride, uint32_t* scan_mask,
@@ -2235,21 +2236,35 @@ __global__ __launch_bounds__(kThreads) void k_build_scan_mask(const SrScanDesc* 
     uint32_t w[SR_TK_MASK_WORDS];
 #pragma unroll
     for (int k = 0; k < SR_TK_MASK_WORDS; k++) w[k] = 0u;
-    for (int j = 0; j < vecs_per_thread; j++) {
-        const int fl = j * kThreads + t;
-        if (fl >= nv) break;
-        const long long e0 = (long long)(f0 + fl) * epv - mis;  // row element under q = 0
-        uint32_t bits = 0u;
-        if (!src && e0 >= 0 && e0 + epv <= vocab) {
-            bits = (1u << epv) - 1u;
-        } else {
-            for (int q = 0; q < epv; q++) {
-                const long long e = e0 + q;
-                if (e >= 0 && e < vocab && (!src || mask_bit(src, (int)e))) bits |= 1u << q;
+    // Bound by latency: the words of ten vectors are asked for before the first is looked at, two words to a vector -- a row
+    // that starts off 16 bytes has vectors across words --, both inside the row's mask.  (A word per bit, a vector
+    // behind the other: 16 fp32 rows of 151,936 took 21.6 us.)
+    const uint32_t all = (1u << epv) - 1u;
+    const int last_word = (vocab - 1) >> 5;
+    for (int j0 = 0; j0 < vecs_per_thread; j0 += kMaskAhead) {
+        uint32_t lo[kMaskAhead], hi[kMaskAhead];
+#pragma unroll
+        for (int k = 0; k < kMaskAhead; k++) {
+            const long long e0 = (long long)(f0 + (j0 + k) * kThreads + t) * epv - mis;  // row element under q = 0
+            const int first = max(0, min(last_word, (int)(e0 >> 5)));
+            lo[k] = hi[k] = 0xffffffffu;
+            if (src) {
+                lo[k] = src[first];
+                hi[k] = src[max(0, min(last_word, (int)((e0 >> 5) + 1)))];
             }
         }
-        const int b = j * epv;
-        w[b >> 5] |= bits << (b & 31);
+#pragma unroll
+        for (int k = 0; k < kMaskAhead; k++) {
+            const int j = j0 + k, fl = j * kThreads + t;
+            if (j >= vecs_per_thread || fl >= nv) break;
+            const int e0 = (f0 + fl) * epv - mis;
+            // (a first vector that starts in front of the row has its elements in the row's first word, which hi is)
+            uint32_t bits = (uint32_t)((((unsigned long long)hi[k] << 32) | (unsigned long long)lo[k]) >> (e0 & 31)) & all;
+            if (e0 < 0) bits &= all << -e0;
+            if (e0 + epv > vocab) bits &= e0 < vocab ? (1u << (vocab - e0)) - 1u : 0u;
+            const int b = j * epv;
+            w[b >> 5] |= bits << (b & 31);
+        }
     }
 #pragma unroll
     for (int k = 0; k < SR_TK_MASK_WORDS; k++) words[t * SR_TK_MASK_WORDS + k] = w[k];
