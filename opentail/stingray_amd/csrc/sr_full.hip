@@ -492,7 +492,8 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
             return;
         }
     }
-    if (seg > 0 && seg_sum >= 0.0f) {
+    const bool first = seg == 0 || before == 0.0;  // nothing in front
+    if (!first && seg_sum >= 0.0f) {
         const float lo = __double2float_rn(before), hi = lo + seg_sum;
         uint32_t nn;
         int eb_lo, eb_hi;
@@ -524,8 +525,8 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
     f.a0 = f.a1 = f.b0 = f.b1 = SR_SEQ_SAT;
     f.eb = eb_first; f.eb2 = eb_last; f.kind = SR_SEG_PLAIN; f.end_bits = 0u;
     int cross = -1;
-    if (seg == 0) {
-        // the row's first segment starts from +0 exactly: its end, once and for all
+    if (first) {
+        // the row's first segment (that has a term) starts from +0 exactly: its end, once and for all
         int dummy;
         const float end = sr_seq_wave<SR_SEQ_RUN, false>(x, 0.0f, 0.0f, &dummy);
         f.kind = SR_SEG_EXACT;
@@ -2642,33 +2643,37 @@ __device__ __forceinline__ void row_deferred(const SrFullArgs& a, SrFullState* s
 __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& rd, SrFullState* st, float* p, int n, int slot, int row,
                                              bool do_scale, float inv, int N, FullSmem& sm, uint32_t* more)
 {
-    constexpr int kPer = SR_LIST_CAP_BIG / kT;  // entries of a thread
+    constexpr int kPer = SR_LIST_CAP_BIG / kT;  // most entries of a thread
     const int tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f, use_min_p = rd.min_p > 0.0f;
     const int nseg = seg_count(n);
     const uint32_t from = st->list_from;
     const float mp = do_scale ? __fmul_rn(1.0f, inv) : 1.0f;  // the largest probability: the largest e is expf(0) = 1
     const float thr = use_min_p ? __fmul_rn(rd.min_p, mp) : 0.0f;
-    const int G = more ? SR_LIST_GROUPS_BIG : SR_LIST_GROUPS_SMALL;
     uint32_t* const grp = list_values(more, sm);
     uint32_t* const cnt = more ? (uint32_t*)sm.sortbuf : grp + list_place(SR_LIST_CAP_SMALL);
-    uint32_t* const gmin = cnt + G;
-    uint32_t* const gmax = cnt + 2 * G;
     int* const off = (int*)sm.segst;  // [nseg] where a segment's entries start
-    static_assert(3 * SR_LIST_GROUPS_BIG * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags) &&
-                  (3 * SR_LIST_GROUPS_SMALL + SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16) * 4 <=
+    static_assert(SR_LIST_GROUPS_BIG * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags) &&
+                  (SR_LIST_GROUPS_SMALL + SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16) * 4 <=
                       sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags), "the tables fit the three arrays");
     // (behind the barrier that follows the gathering)
-    const int i0 = tid * kPer;
-    const int mine = max(0, min(kPer, N - i0));
+    // A thread takes 2^sh consecutive entries, as few as the list's length allows (always 16: a list of 1,000 kept one wave
+    // busy, 12 us).
+    int sh = 0;
+    while ((kT << sh) < N) sh++;
+    const int per = 1 << sh;
+    const int G = min(more ? SR_LIST_GROUPS_BIG : SR_LIST_GROUPS_SMALL, kT << (sh + 1));  // groups: two to an entry, where there is room
+    const int i0 = tid << sh;
+    const int mine = max(0, min(per, N - i0));
     uint32_t ev[kPer];
 #pragma unroll
     for (int r = 0; r < kPer; r++) ev[r] = r < mine ? grp[list_place(i0 + r)] : 0u;
     auto prob = [&](uint32_t ebits) -> float { return do_scale ? __fmul_rn(sr_u2f(ebits), inv) : sr_u2f(ebits); };
 
-    // sorted by value: groups of equal width in the bit patterns, counted, placed, and every value ranked inside its group
-    // (groups of one value need no ranks: the equal logits of a coarse grid)
-    for (int i = tid; i < G; i += kT) { cnt[i] = 0u; gmin[i] = 0xffffffffu; gmax[i] = 0u; }
+    // Sorted by value: groups of equal width in the bit patterns, counted, placed, and every value ranked inside its group -- a group of one value (the equal logits of a coarse grid) needs no ranks and is
+    // told by its neighbours.  (4,096 groups with their extremes counted along: 12 - 20 us for 14,000 entries, most of it the
+    // longest group of every wave looked through 16 times.)
+    for (int i = tid; i < G; i += kT) cnt[i] = 0u;
     if (tid == 0) sm.bc[12] = 0u;
     __syncthreads();
     const uint32_t span = 0x3f800000u - min(from, 0x3f800000u);
@@ -2677,51 +2682,54 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     auto group_of = [&](uint32_t v) -> uint32_t { return min((0x3f800000u - v) >> gshift, (uint32_t)(G - 1)); };
 #pragma unroll
     for (int r = 0; r < kPer; r++)
-        if (r < mine) {
-            const uint32_t g = group_of(ev[r]);
-            atomicAdd(&cnt[g], 1u);
-            atomicMin(&gmin[g], ev[r]);
-            atomicMax(&gmax[g], ev[r]);
-        }
+        if (r < mine) atomicAdd(&cnt[group_of(ev[r])], 1u);
     __syncthreads();
     {
-        const int per = G / kT;  // 4 or 2
-        uint32_t c4[SR_LIST_GROUPS_BIG / kT];
-        int own = 0;
-#pragma unroll
-        for (int q = 0; q < SR_LIST_GROUPS_BIG / kT; q++) {
-            c4[q] = q < per ? cnt[tid * per + q] : 0u;
-            own += (int)c4[q];
-            if (c4[q] > 128u && gmin[tid * per + q] != gmax[tid * per + q]) sm.bc[12] = 1u;
+        // a wave's share of the groups, 64 at a time: the sums inside the wave, then what stands in front of it
+        const int g0 = wave * (G / kW);
+        int in_wave = 0;
+        for (int g = g0; g < g0 + G / kW; g += SR_WAVE) {
+            const int c = (int)cnt[g + lane];
+            const int incl = sr_wave_incl_scan_i32(c);
+            cnt[g + lane] = (uint32_t)(in_wave + incl - c);
+            in_wave += __builtin_amdgcn_readlane(incl, SR_WAVE - 1);
         }
-        int tot;
-        int at = blk_excl_scan(own, &tot, sm);
+        if (lane == 0) sm.redi[wave] = in_wave;
+        __syncthreads();
+        int before = 0;
 #pragma unroll
-        for (int q = 0; q < SR_LIST_GROUPS_BIG / kT; q++)
-            if (q < per) { cnt[tid * per + q] = (uint32_t)at; at += (int)c4[q]; }
+        for (int w = 0; w < kW; w++) before += w < wave ? sm.redi[w] : 0;
+        for (int g = g0; g < g0 + G / kW; g += SR_WAVE) cnt[g + lane] += (uint32_t)before;
     }
     __syncthreads();
-    if (sm.bc[12] != 0u) return kListGeneral;
 #pragma unroll
     for (int r = 0; r < kPer; r++)
         if (r < mine) grp[list_place((int)atomicAdd(&cnt[group_of(ev[r])], 1u))] = ev[r];
     __syncthreads();  // cnt[g] is now where group g ends
     {
+        constexpr uint32_t kMixed = 0x80000000u;  // (of cnt: the group holds more than one value)
         uint32_t v[kPer];
+        uint32_t last = (mine > 0 && i0 > 0) ? grp[list_place(i0 - 1)] : 0u;
+#pragma unroll
+        for (int r = 0; r < kPer; r++) v[r] = r < mine ? grp[list_place(i0 + r)] : 0u;
+#pragma unroll
+        for (int r = 0; r < kPer; r++) {
+            if (r < mine && v[r] != last && i0 + r > 0 && group_of(v[r]) == group_of(last)) atomicOr(&cnt[group_of(v[r])], kMixed);
+            last = v[r];
+        }
+        __syncthreads();
         int rank[kPer];
 #pragma unroll
         for (int r = 0; r < kPer; r++) {
-            v[r] = 0u;
-            rank[r] = 0;
+            rank[r] = i0 + r;
             if (r < mine) {
                 const int i = i0 + r;
-                v[r] = grp[list_place(i)];
-                const uint32_t g = group_of(v[r]);
-                rank[r] = i;
-                if (gmin[g] != gmax[g]) {
-                    const int b = g > 0u ? (int)cnt[g - 1u] : 0, e = (int)cnt[g];
+                const uint32_t g = group_of(v[r]), ce = cnt[g];
+                if (ce & kMixed) {
+                    const int b = g > 0u ? (int)(cnt[g - 1u] & ~kMixed) : 0, e = (int)(ce & ~kMixed);
+                    if (e - b > 128) sm.bc[12] = 1u;
                     int k = b;
-                    for (int j = b; j < e; j++) {
+                    for (int j = b; j < min(e, b + 128); j++) {
                         const uint32_t o = grp[list_place(j)];
                         k += (o > v[r] || (o == v[r] && j < i)) ? 1 : 0;
                     }
@@ -2730,6 +2738,7 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
             }
         }
         __syncthreads();
+        if (sm.bc[12] != 0u) return kListGeneral;
 #pragma unroll
         for (int r = 0; r < kPer; r++)
             if (r < mine) grp[list_place(rank[r])] = v[r];
@@ -2763,6 +2772,26 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
                 }
                 sm.segbc[1] = (uint32_t)f;
                 sm.segbc[2] = sr_f2u(s);
+            }
+            __syncthreads();
+            found = (int)sm.segbc[1];
+        } else if (ns <= 2 * SR_SEG_TERMS) {
+            // up to two thousand: one wave, without the block-wide steps
+            if (wave == 0) {
+                float s = 0.0f;
+                int f = -1;
+                for (int b0 = 0; b0 < ns && f < 0; b0 += SR_SEG_TERMS) {
+                    float x[SR_SEQ_RUN];
+#pragma unroll
+                    for (int j = 0; j < SR_SEQ_RUN; j++) {
+                        const int i = b0 + lane * SR_SEQ_RUN + j;
+                        x[j] = i < ns ? prob(grp[list_place(i)]) : 0.0f;
+                    }
+                    int at;
+                    s = sr_seq_wave<SR_SEQ_RUN, true>(x, s, rd.top_p, &at);
+                    if (at >= 0) f = b0 + at;
+                }
+                if (lane == 0) { sm.segbc[1] = (uint32_t)f; sm.segbc[2] = sr_f2u(s); }
             }
             __syncthreads();
             found = (int)sm.segbc[1];
@@ -2816,7 +2845,7 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     const int m = cutoff;
     const bool finish = a.mode == 0 && m <= a.finish_most;
     if (!finish && !a.prepared) return kListGeneral;
-    // The members by their places in the list: a bit each, and how many stand in front of every sixteen.  The waves then go
+    // The members by their places in the list: a bit each, and how many stand in front of every thread's.  The waves then go
     // through the segments once more and know the index and the rank of every member they meet.
     uint16_t* const bits = more ? (uint16_t*)more : (uint16_t*)sm.tags;
     int* const in_front = (int*)(bits + kT);
@@ -2840,15 +2869,18 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     const int32_t* gi = a.sort_vals_in + (size_t)slot * (size_t)a.sort_stride;
     const int last_place = (int)sm.bc[10], nv8 = (n / 8) * 8;
     for (int s0 = wave; s0 < nseg; s0 += 4 * kW) {
-        uint32_t v[4];
-        int id[4], at[4], len[4];
+        uint32_t v[4], v2[4];
+        int id[4], id2[4], at[4], len[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < 4; q++) {  // (the first 128 entries of four segments on their way at a time)
             const int sg = s0 + q * kW;
+            const size_t from_seg = (size_t)sg * SR_SEG_TERMS + lane;
             at[q] = sg < nseg ? off[sg] : 0;
             len[q] = sg < nseg ? (sg + 1 < nseg ? off[sg + 1] : N) - at[q] : 0;
-            v[q] = lane < len[q] ? gk[(size_t)sg * SR_SEG_TERMS + lane] : 0u;
-            id[q] = lane < len[q] ? gi[(size_t)sg * SR_SEG_TERMS + lane] : 0;
+            v[q] = lane < len[q] ? gk[from_seg] : 0u;
+            id[q] = lane < len[q] ? gi[from_seg] : 0;
+            v2[q] = lane + SR_WAVE < len[q] ? gk[from_seg + SR_WAVE] : 0u;
+            id2[q] = lane + SR_WAVE < len[q] ? gi[from_seg + SR_WAVE] : 0;
         }
 #pragma unroll
         for (int q = 0; q < 4; q++) {
@@ -2856,13 +2888,14 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
             float own = 0.0f;
             for (int i = lane; i < len[q]; i += SR_WAVE) {
                 const int place = at[q] + i;
-                const uint32_t ebits = i < SR_WAVE ? v[q] : gk[(size_t)sg * SR_SEG_TERMS + i];
-                const int idx = i < SR_WAVE ? id[q] : gi[(size_t)sg * SR_SEG_TERMS + i];
+                const uint32_t ebits = i < SR_WAVE ? v[q] : i < 2 * SR_WAVE ? v2[q] : gk[(size_t)sg * SR_SEG_TERMS + i];
+                const int idx = i < SR_WAVE ? id[q] : i < 2 * SR_WAVE ? id2[q] : gi[(size_t)sg * SR_SEG_TERMS + i];
                 if (place == last_place) sm.bc[9] = (uint32_t)idx;
-                const uint32_t b = bits[place >> 4];
-                if (!((b >> (place & 15)) & 1u)) continue;
+                const uint32_t b = bits[place >> sh];
+                const int in_run = place & (per - 1);
+                if (!((b >> in_run) & 1u)) continue;
                 if (finish) {
-                    const int rank = in_front[place >> 4] + __popc(b & ((1u << (place & 15)) - 1u));
+                    const int rank = in_front[place >> sh] + __popc(b & ((1u << in_run) - 1u));
                     sm.sortbuf[rank] = ((unsigned long long)(0xffffffffu - (uint32_t)idx) << 32) | (unsigned long long)sr_f2u(prob(ebits));
                 } else {
                     own += sr_u2f(ebits);

@@ -114,6 +114,6 @@ struct SrMaskClear {
 // candidates of a row that k_full_row sorts, and the groups it sorts them by: with a compute unit to itself, and without
 #define SR_LIST_CAP_BIG 16384
 #define SR_LIST_CAP_SMALL 4096
-#define SR_LIST_GROUPS_BIG 4096
-#define SR_LIST_GROUPS_SMALL 2048
+#define SR_LIST_GROUPS_BIG 16384
+#define SR_LIST_GROUPS_SMALL 8192
 #define SR_SEG_MAX 1024                    // most segments of such a row: longer rows are added the plain way
