@@ -3688,11 +3688,12 @@ __global__ __launch_bounds__(kPrepT) void k_prepared_draw(SrFullArgs a)
     {
         int dummy;
         float s = seg_walk_from<false>([&](int blk, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
+            // (no condition stands between the loads: with one each they wait for each other)
+            const int t0 = blk * SR_SEG_TERMS + lane * SR_SEQ_RUN;
 #pragma unroll
-            for (int j = 0; j < SR_SEQ_RUN; j++) {
-                const int t = blk * SR_SEG_TERMS + lane * SR_SEQ_RUN + j, i = t * 8 + wave;
-                x[j] = t < nv ? r.cut(r.e[i], i) : 0.0f;
-            }
+            for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = r.e[min(t0 + j, nv - 1) * 8 + wave];
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = t0 + j < nv ? r.cut(x[j], (t0 + j) * 8 + wave) : 0.0f;
         }, nblk, a.chain_func + ((size_t)slot * SR_SEQ_CHAINS + wave) * a.chain_blocks, 0.0f, 0.0f, &dummy, nullptr);
         if (rem > 0 && wave >= 8 - rem) s = __fadd_rn(s, r.cut(r.e[n - 8 + wave], n - 8 + wave));  // the overlapped last vector
         if (lane == 0) lane_sum[wave] = s;
@@ -3757,8 +3758,9 @@ __global__ __launch_bounds__(SR_WAVE) void k_prepared_token(SrFullArgs a)
     int found;
     const float at = seg_walk_from<true>([&](int seg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
         const int i0 = seg * SR_SEG_TERMS + lane * SR_SEQ_RUN;
+        seq_load_run(r.e, true, i0, n, x);  // (the rows of e start on 16-byte boundaries; zeros past the end stay zeros)
 #pragma unroll
-        for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = term(i0 + j);
+        for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = __fmul_rn(r.cut(x[j], i0 + j), inv2);
     }, seg_count(n), a.seg_func + (size_t)slot * a.seg_stride, 0.0f, u, &found, nullptr);
     if (lane == 0) {
         const bool amb = found >= 0 ? sr_stop_near(at, term(found), u) : sr_near(at, u);
