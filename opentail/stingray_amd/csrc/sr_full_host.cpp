@@ -67,7 +67,9 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             prepared = prepared || !sr_row_cut(r) || mode != 0 || !(r.min_p >= 0.002f);
         }
     }
-    prepared = prepared && (long long)n_rows * nseg <= (lazy_scale ? SR_PREPARED_SEGS_VERIFY : mode != 0 ? SR_PREPARED_SEGS_DISTRIBUTIONS : SR_PREPARED_SEGS);
+    const bool odd_rows = mode != 0 && (probs_stride & 3) != 0;
+    prepared = prepared && nseg >= (lazy_scale ? SR_PREPARED_MIN_SEGS_VERIFY : odd_rows ? SR_PREPARED_MIN_SEGS_ODD : SR_PREPARED_MIN_SEGS) &&
+               (long long)n_rows * nseg <= (lazy_scale ? SR_PREPARED_SEGS_VERIFY : mode != 0 ? SR_PREPARED_SEGS_DISTRIBUTIONS : SR_PREPARED_SEGS);
     a.any_copy = any_copy ? 1 : 0;
     a.any_edits = any_edits ? 1 : 0;
     a.n_sampled = (int)((long long)n_sampled * n_rows / std::max(1, n_seen));  // (a verifier's launch has every row several times)

@@ -108,6 +108,12 @@ struct SrMaskClear {
 // rows of 151,936 (28,608 segments) 182 -> 159 us, distributions of 64 rows 132 -> 109 and of 128 rows (19,072) 161 -> 164;
 // the verifier, where the workgroup passes over its row once and not three times: 24 rows of 262,144 (6,144) 108 -> 103, 36
 // rows 118.5 -> 119.6.
+// (And down to how many segments of a row: those launches cost the same for a short row, which its workgroup passes over in less.
+// Tokens, 16 rows of 16,384: 58.1 against 51.8 us, of 32,768 both 58, of 49,152: 58 against 67; the verifier, 20 rows of
+// 65,536: 69 against 65 us, of 131,072: 80 against 79, 2 rows of 262,144: 70 against 84.)
+#define SR_PREPARED_MIN_SEGS 32
+#define SR_PREPARED_MIN_SEGS_VERIFY 128
+#define SR_PREPARED_MIN_SEGS_ODD 16  // distributions at odd addresses, 16 rows of 24,001: 57 against 78 us
 #define SR_PREPARED_SEGS 32768
 #define SR_PREPARED_SEGS_DISTRIBUTIONS 16384
 #define SR_PREPARED_SEGS_VERIFY 8192

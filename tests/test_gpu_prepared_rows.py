@@ -37,7 +37,7 @@ def _check(ctx, logits, dev, params, rng):
         assert np.array_equal(probs[r].view(np.uint32), want.view(np.uint32)), (logits.shape, r)
 
 
-@pytest.mark.parametrize("vocab", [4096, 4097, 5119, 8191, 8200, 16385, 65_537, 151_936])
+@pytest.mark.parametrize("vocab", [4096, 4097, 8191, 16385, 31_745, 32_768, 33_791, 36_865, 40_967, 65_537, 151_936])
 @pytest.mark.parametrize("kind", ["f32", "bf16", "coarse"])
 def test_rows_prepared_by_the_whole_device(ctx, vocab, kind):
     rng = np.random.default_rng(vocab)
