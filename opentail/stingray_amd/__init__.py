@@ -460,6 +460,7 @@ class SamplerContext:
                      return_flags: bool = False):
         """Sampler.Sample for every row (preceded by the row's mask). logits: CUDA tensor [rows, vocab].
         Returns numpy int32 tokens (and flags)."""
+        assert logits.is_cuda  # (the address goes to a kernel)
         rows, vocab = logits.shape
         if len(params) > rows:
             raise ValueError(f"{len(params)} parameter sets for {rows} rows")
