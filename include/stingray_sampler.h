@@ -236,8 +236,9 @@ SR_API int sr_argmax_rows_launch(sr_ctx* ctx, const void* logits_dev, int dtype,
 SR_API int sr_argmax_rows_launch_noalloc(sr_ctx* ctx, const void* logits_dev, int dtype, int32_t rows,
                                          int32_t vocab, int64_t row_stride_elems,
                                          int32_t* out_idx_dev, float* out_val_dev);
-/* The same with the results in HOST arrays as well: the call returns when they are there (out_val may be NULL), and the
- * device arrays (either may be NULL) are written by the same launch. */
+/* The same with the results in HOST arrays as well: the call returns when they are there (out_val may be NULL).  The same
+ * launch has written the device arrays (either may be NULL) by then: they can be read on any stream, or freed, at once.  The
+ * kernel itself may end a little later; it neither reads the logits nor writes an array of the caller's any more. */
 SR_API int sr_argmax_rows_both(sr_ctx* ctx, const void* logits_dev, int dtype, int32_t rows, int32_t vocab,
                                int64_t row_stride_elems, int32_t* out_idx_dev, float* out_val_dev,
                                int32_t* out_idx, float* out_val);

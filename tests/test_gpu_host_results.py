@@ -34,6 +34,37 @@ def test_argmax_host_and_device_results_agree(ctx, rows, vocab):
         assert np.array_equal(out[0].cpu().numpy(), want) and np.array_equal(out[1].cpu().numpy(), v0)
 
 
+@pytest.mark.parametrize("own_stream", [False, True])
+@pytest.mark.parametrize("rows,vocab", [(1, 40_000), (33, 151_936), (257, 2048), (1500, 513)])
+def test_argmax_device_results_are_there_for_other_streams(rows, vocab, own_stream):
+    """The device arrays are read on a stream that is not ordered behind the context's, and given away at once: what the
+    allocator hands out next keeps what is put there."""
+    import torch
+
+    torch.cuda.synchronize()
+    c = SamplerContext(0, use_torch_stream=not own_stream)
+    rng = np.random.default_rng(rows)
+    m = rng.normal(0, 2, (4, rows, vocab)).astype(np.float32)
+    dev = [torch.from_numpy(x).cuda() for x in m]
+    want = m.argmax(axis=2)
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for i in range(24):
+        k = i % 4
+        with torch.cuda.stream(other):
+            out = (torch.full((rows,), -3, dtype=torch.int32, device="cuda"), torch.full((rows,), 9.0, device="cuda"))
+            other.synchronize()
+            idx, val = c.argmax_rows(dev[k], out=out)
+            got = (out[0].clone(), out[1].clone())
+            del out
+            new = [torch.full((rows,), 77, dtype=torch.int32, device="cuda") for _ in range(2)]
+        other.synchronize()
+        assert np.array_equal(idx, want[k]) and np.array_equal(val, m[k][np.arange(rows), want[k]])
+        assert np.array_equal(got[0].cpu().numpy(), idx) and np.array_equal(got[1].cpu().numpy(), val), i
+        assert all(bool((t == 77).all()) for t in new), i
+    c.close()
+
+
 @pytest.mark.parametrize("topk", [0, 40])
 def test_uniforms_of_launches_in_flight_are_not_overwritten(ctx, topk):
     """400 steps of new uniforms without a wait (the ring of a batch of 40 rows goes round several times), the context on
