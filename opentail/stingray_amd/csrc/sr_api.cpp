@@ -746,6 +746,9 @@ static int uniforms_in_place(sr_batch* b, const double* uniforms)
 {
     sr_ctx* ctx = b->ctx;
     const size_t bytes = (size_t)b->rows * (size_t)b->upr * sizeof(double);
+    // (a ring that grows gives its old block away before it has the new one: from here to the end of the call the uniforms of
+    // the upload count, also when the call fails)
+    b->uni_now = nullptr;
     SR_HIP(ctx, b->uni_ring.begin(ctx->pinned, bytes + 256, ctx->stream, 0, ctx->stream_epoch, true));
     const void* at = b->uni_ring.put(uniforms, bytes);
     if (!at) return sr_fail(ctx, SR_ERR_OUT_OF_MEMORY, "no pinned memory for the uniforms");
