@@ -151,6 +151,8 @@ SR_API void sr_batch_destroy(sr_batch* batch);
  * Every host array may be reused when the call returns.  The copies to the device run on the context's stream
  * and are not waited for (except for an allow-mask): launches that follow on the same stream see the batch
  * complete; sr_set_stream synchronises the stream it leaves.
+ * A call whose arguments are refused leaves the batch as it was.  One that fails later (no memory) leaves a batch that every
+ * call but an upload refuses with SR_ERR_INVALID_ARGUMENT.
  */
 SR_API int sr_batch_upload(sr_batch* batch, int32_t rows, int32_t vocab,
                            const sr_row_params* params,

@@ -16,6 +16,12 @@ int64_t sr_batch_mask_stride(const sr_batch* b) { return b->mask_ids ? (int64_t)
 
 const double* sr_batch_uniforms(const sr_batch* b) { return b->uni_now ? b->uni_now : b->d_uniforms.as<double>(); }
 
+int sr_batch_complete(sr_ctx* ctx, const sr_batch* b, const char* who)
+{
+    if (!b->incomplete) return SR_OK;
+    return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, std::string(who) + ": the batch's last upload failed; upload it again");
+}
+
 int sr_batch_masks_valid(sr_ctx* ctx, const sr_batch* b, const char* who)
 {
     if (!b->mask_ids) return SR_OK;
@@ -478,6 +484,7 @@ static int batch_upload_impl(sr_batch* b, int32_t rows, int32_t vocab, const sr_
     b->segs.clear();
     b->upload_must_wait = false;
 
+    b->incomplete = true;  // (until the end of this function)
     b->rows = rows;
     b->vocab = vocab;
     b->upr = uniforms_per_row;
@@ -726,6 +733,7 @@ static int batch_upload_impl(sr_batch* b, int32_t rows, int32_t vocab, const sr_
     SR_HIP(ctx, batch_flush(b, st));
     if (b->upload_must_wait) SR_HIP(ctx, hipStreamSynchronize(st));
     if (!waited_for) SR_HIP(ctx, b->stage.end(st));
+    b->incomplete = false;
     return SR_OK;
 }
 
@@ -785,6 +793,9 @@ static int append_impl(sr_batch* b, const int32_t* tokens, const double* uniform
         return sr_fail(ctx, SR_ERR_UNSUPPORTED, "sr_batch_append_tokens: the batch was not uploaded, or was uploaded with "
                                                 "allow-masks of its own (register the masks and upload their ids, or "
                                                 "upload it again with the new masks)");
+    // (a rebuild of an earlier append that failed is made good below, from the inputs that were kept)
+    if (!b->host_ahead)
+        if (int rc = sr_batch_complete(ctx, b, "sr_batch_append_tokens")) return rc;
     if (new_mask_ids && !b->mask_ids)
         return sr_fail(ctx, SR_ERR_UNSUPPORTED, "sr_batch_append_tokens_masks: the batch was not uploaded with mask ids");
     const int32_t rows = b->rows, vocab = b->vocab;
@@ -1163,6 +1174,7 @@ int sr_batch_set_uniforms(sr_batch* b, const double* uniforms)
     sr_ctx* ctx = b->ctx;
     if (!uniforms) return sr_fail(ctx, SR_ERR_NULL_ARGUMENT, "sr_batch_set_uniforms: uniforms is null");
     if (b->upr <= 0 || b->rows <= 0) return SR_OK;
+    if (int rc = sr_batch_complete(ctx, b, "sr_batch_set_uniforms")) return rc;
     SR_HIP(ctx, hipSetDevice(ctx->device));
     return uniforms_in_place(b, uniforms);
 }
@@ -1177,6 +1189,7 @@ int sr_sample_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int
         return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, "sr_sample_launch: unknown dtype");
     if (row_stride_elems < b->vocab) return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, "sr_sample_launch: row stride < vocab");
     if (b->vocab <= 0) return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, "sr_sample_launch: empty vocabulary");
+    if (int rc = sr_batch_complete(ctx, b, "sr_sample_launch")) return rc;
     if (int rc = sr_batch_masks_valid(ctx, b, "sr_sample_launch")) return rc;
     for (const SrRow& r : b->h_rows)
         if (r.path != SR_PATH_GREEDY && r.path != SR_PATH_GREEDY_PEN && b->upr < 1)
@@ -1263,6 +1276,7 @@ int sr_resample_rows_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_d
         return sr_fail(ctx, SR_ERR_NULL_ARGUMENT, "sr_resample_rows_launch: null argument");
     if (n_rows < 0 || (dtype != SR_DTYPE_F32 && dtype != SR_DTYPE_BF16) || row_stride_elems < b->vocab)
         return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, "sr_resample_rows_launch: bad shape or dtype");
+    if (int rc = sr_batch_complete(ctx, b, "sr_resample_rows_launch")) return rc;
     for (int32_t i = 0; i < n_rows; i++) {
         const int32_t r = rows_host[i];
         if (r < 0 || r >= b->rows) return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, "sr_resample_rows_launch: row out of range");

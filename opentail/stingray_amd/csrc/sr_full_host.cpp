@@ -161,6 +161,7 @@ int check_batch_call(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int
     if (dtype != SR_DTYPE_F32 && dtype != SR_DTYPE_BF16) return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, std::string(who) + ": unknown dtype");
     if (b->vocab <= 0) return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, std::string(who) + ": empty vocabulary");
     if (row_stride < b->vocab) return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, std::string(who) + ": row stride < vocab");
+    if (int rc = sr_batch_complete(ctx, b, who)) return rc;
     return sr_batch_masks_valid(ctx, b, who);
 }
 
@@ -456,6 +457,7 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     if (!ctx || !b) return SR_ERR_NULL_ARGUMENT;
     if (b->rows == 0) return SR_OK;
     if (n_draft < 0) return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, "sr_spec_verify_launch: negative draft length");
+    if (int rc = sr_batch_complete(ctx, b, "sr_spec_verify_launch")) return rc;
     if (!target_logits_dev || !out_accepted_dev || !out_tokens_dev || (n_draft > 0 && !draft_tokens_dev))
         return sr_fail(ctx, SR_ERR_NULL_ARGUMENT, "sr_spec_verify_launch: null tensor");
     if (n_draft > 0 && !draft_probs_dev) {

@@ -365,6 +365,7 @@ struct sr_batch {
     // What sr_batch_append_tokens needs of the last upload: the inputs of a batch without allow-masks (kept flat as
     // they came; the histories are split per row by the first append) and the room each row's edit range has.
     bool can_append = false, hist_split = false;
+    bool incomplete = false;  // the last upload failed after it had begun to change the batch: nothing is launched until one succeeds
     bool host_ahead = false;  // an append call failed after it had changed the host's copies: the next one rebuilds the batch
     int32_t append_rebuilds = 0;  // calls of sr_batch_append_tokens that rebuilt the batch (test hook)
     int32_t append_moves = 0;     // ... rows that were moved to the end of the edit array instead
@@ -396,6 +397,9 @@ inline int sr_fail_hip(sr_ctx* ctx, hipError_t e, const char* what)
         if (_e != hipSuccess) return sr_fail_hip((ctx), _e, #call);   \
     } while (0)
 
+// SR_OK, or SR_ERR_INVALID_ARGUMENT when the batch's last upload failed half way (its descriptors, lists and uniforms on the
+// device belong to different uploads, or are not there): to be called before every launch that reads a batch
+int sr_batch_complete(sr_ctx* ctx, const sr_batch* b, const char* who);
 // SR_OK, or SR_ERR_INVALID_ARGUMENT when the batch names a registered mask that was released (or whose pool was
 // started again for another vocabulary) after the batch took the id: to be called before every launch that reads masks
 int sr_batch_masks_valid(sr_ctx* ctx, const sr_batch* b, const char* who);

@@ -41,28 +41,39 @@ def _launch(ctx, batch, addr=4096, dtype=sa.SR_DTYPE_F32, stride=None):
 
 
 @pytest.mark.parametrize("topk", [0, 40])
-def test_uniforms_are_never_read_from_memory_that_was_given_away(ctx, topk):
-    """A batch that could not be uploaded with more rows, and then has no pinned memory for that many uniforms."""
+def test_a_batch_whose_upload_failed_is_refused_until_one_succeeds(ctx, topk):
+    """A batch that could not be uploaded with more rows names device memory of an older, smaller one: no call launches it or
+    gives it uniforms (whose old place may have been given away), and it works again once it has been uploaded."""
     rows, vocab = 5_000, 1_000
     p = [SamplingParams(Temperature=0.8, TopK=topk)]
     u = np.random.default_rng(1).random(20 * rows)
+    uniforms = lambda: np.ctypeslib.as_array((C.c_double * rows).from_address(ctx.L.cpu_uniforms()))
     b = ctx.new_batch().upload(p * rows, vocab, u[:rows])
     _launch(ctx, b)
     assert ctx.L.cpu_live(ctx.L.cpu_uniforms()) >= 8 * rows
     b.set_uniforms(u[:rows])
     _launch(ctx, b)
-    assert np.array_equal(np.ctypeslib.as_array((C.c_double * rows).from_address(ctx.L.cpu_uniforms())), u[:rows])
+    assert np.array_equal(uniforms(), u[:rows])
     ctx.L.cpu_fail(1, 1)
     with pytest.raises(RuntimeError):
         ctx._check(ctx.L.sr_batch_upload(b.h, 20 * rows, vocab, b._packed[2] * 20, *[None] * 6, 0, None, u.ctypes.data, 1))
-    with pytest.raises(RuntimeError):
+    launches = ctx.L.cpu_launches()
+    with pytest.raises(ValueError, match="upload"):
         b.set_uniforms(u)
+    with pytest.raises(ValueError, match="upload"):
+        b.append_tokens(np.full(rows, -1), None)
     ctx.L.cpu_fail(0, 0)
-    _launch(ctx, b)
-    assert ctx.L.cpu_live(ctx.L.cpu_uniforms()) > 0
-    # a batch that fails once goes on working
+    with pytest.raises(ValueError, match="upload"):
+        _launch(ctx, b)
+    out = np.zeros(64, dtype=np.float32).ctypes.data
+    for call in (lambda: ctx.L.sr_build_distribution_launch(ctx.h, b.h, 4096, 0, vocab, out, vocab, vocab),
+                 lambda: ctx.L.sr_sample_with_distribution_launch(ctx.h, b.h, 4096, 0, vocab, out, vocab, vocab, 64),
+                 lambda: ctx.L.sr_spec_verify_launch(ctx.h, b.h, 4096, None, None, 0, 64, 64),
+                 lambda: ctx.L.sr_resample_rows_launch(ctx.h, b.h, 4096, 0, vocab, np.zeros(1, np.int32).ctypes.data, 1, 64, None)):
+        assert call() == sa.SR_ERR_INVALID_ARGUMENT
+    assert ctx.L.cpu_launches() == launches
     b.upload(p * rows, vocab, u[:rows])
     b.set_uniforms(u[rows:2 * rows])
     _launch(ctx, b)
-    assert np.array_equal(np.ctypeslib.as_array((C.c_double * rows).from_address(ctx.L.cpu_uniforms())), u[rows:2 * rows])
+    assert np.array_equal(uniforms(), u[rows:2 * rows])
     b.close()
