@@ -319,7 +319,12 @@ int scan_for_launch(sr_batch* b, int epv, unsigned long long base_addr, long lon
     b->segs.clear();
     b->upload_must_wait = false;
     const int rc = prepare_scan(b, epv, base_addr, stride_bytes);
-    if (rc != SR_OK) return rc;
+    if (rc != SR_OK) {
+        // what the device holds is of neither layout: masks and descriptors are sent again by the next launch
+        b->scan_epv = 0;
+        for (int32_t r : b->h_sel_list) b->h_rows[(size_t)r].scan_row = -1;
+        return rc;
+    }
     if (b->upload_must_wait) SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
     SR_HIP(ctx, b->stage.end(ctx->stream));
     return SR_OK;

@@ -13,6 +13,7 @@ int fail_device = 0, fail_pinned = 0;
 struct Seen {
     int64_t scan_builds, stream_waits, launches;
     const double* uniforms;
+    const SrRow* rows;
 } seen;
 
 hipError_t take(void** p, size_t n, int fail)
@@ -37,6 +38,7 @@ int64_t cpu_scan_builds() { return seen.scan_builds; }
 int64_t cpu_stream_waits() { return seen.stream_waits; }
 int64_t cpu_launches() { return seen.launches; }
 const double* cpu_uniforms() { return seen.uniforms; }
+int cpu_scan_row(int row) { return seen.rows[row].scan_row; }
 // bytes of live memory from p on (0: p is in none)
 int64_t cpu_live(const void* p)
 {
@@ -83,7 +85,7 @@ hipError_t sr_launch_build_scan_mask(const SrScanDesc*, const int32_t*, int, con
     seen.scan_builds++;
     return pieces ? put(*pieces) : launched();
 }
-hipError_t sr_launch_topk(const SrTopkArgs& a, int, hipStream_t) { seen.uniforms = a.uniforms; return launched(); }
+hipError_t sr_launch_topk(const SrTopkArgs& a, int, hipStream_t) { seen.uniforms = a.uniforms; seen.rows = a.rows; return launched(); }
 hipError_t sr_launch_full_prep(const SrFullArgs& a, int, hipStream_t) { seen.uniforms = a.uniforms; return launched(); }
 hipError_t sr_launch_full_row(const SrFullArgs&, int, hipStream_t) { return launched(); }
 hipError_t sr_launch_pack_allow_mask(const void*, int, int, int, int64_t, uint32_t*, int64_t, hipStream_t) { return launched(); }

@@ -77,3 +77,19 @@ def test_a_batch_whose_upload_failed_is_refused_until_one_succeeds(ctx, topk):
     _launch(ctx, b)
     assert np.array_equal(uniforms(), u[rows:2 * rows])
     b.close()
+
+
+def test_scan_masks_that_could_not_be_made_are_made_by_the_next_launch(ctx):
+    vocab = 1_000
+    b = ctx.new_batch().upload([SamplingParams(Temperature=0.8, TopK=40)] * 8, vocab, np.full(8, 0.5))
+    _launch(ctx, b)
+    made = ctx.L.cpu_scan_builds()
+    ctx.L.cpu_fail(1, 1)
+    with pytest.raises(RuntimeError):  # rows at eight different offsets: eight mask rows instead of one
+        _launch(ctx, b, stride=vocab + 1)
+    ctx.L.cpu_fail(0, 0)
+    assert ctx.L.cpu_scan_builds() == made
+    _launch(ctx, b, stride=vocab + 1)
+    assert ctx.L.cpu_scan_builds() == made + 1
+    assert [ctx.L.cpu_scan_row(r) for r in range(8)] == list(range(8))  # the descriptors that the kernel reads
+    b.close()
