@@ -309,11 +309,11 @@ int prepare_scan(sr_batch* b, int epv, unsigned long long base_addr, long long s
 int scan_for_launch(sr_batch* b, int epv, unsigned long long base_addr, long long stride_bytes)
 {
     sr_ctx* ctx = b->ctx;
-    ctx->last_epv = epv;
-    ctx->last_base_mod = (unsigned)(base_addr & 15ull);
-    ctx->last_stride_mod = (unsigned)(stride_bytes & 15ll);
-    if (b->scan_epv == epv && b->scan_base_mod == (int)ctx->last_base_mod &&
-        b->scan_stride_mod == (b->rows <= 1 ? 0 : (int)ctx->last_stride_mod))
+    b->layout = ScanLayout{epv, (unsigned)(base_addr & 15ull), (unsigned)(stride_bytes & 15ll)};
+    b->layout_known = true;
+    ctx->last_layout = b->layout;
+    if (b->scan_epv == epv && b->scan_base_mod == (int)b->layout.base_mod &&
+        b->scan_stride_mod == (b->rows <= 1 ? 0 : (int)b->layout.stride_mod))
         return SR_OK;
     SR_HIP(ctx, b->stage.begin(ctx->pinned));
     b->segs.clear();
@@ -727,9 +727,11 @@ static int batch_upload_impl(sr_batch* b, int32_t rows, int32_t vocab, const sr_
     if (!keep_uniforms) b->uni_now = nullptr;
     if (uniforms_per_row > 0 && !keep_uniforms)
         SR_HIP(ctx, up(b->d_uniforms, uniforms, (size_t)rows * (size_t)uniforms_per_row * sizeof(double)));
-    // scan masks for the layout of the last launch; a launch with another layout rebuilds them
+    // scan masks for the layout of the batch's last launch (of the context's, before it has had one); a launch with another
+    // layout builds them again
     if (!b->h_sel_list.empty()) {
-        int rc = prepare_scan(b, ctx->last_epv, ctx->last_base_mod, ctx->last_stride_mod);
+        const ScanLayout& guess = b->layout_known ? b->layout : ctx->last_layout;
+        int rc = prepare_scan(b, guess.epv, guess.base_mod, guess.stride_mod);
         if (rc != SR_OK) return rc;
     }
     // Everything small went through the batch's pinned memory: the copies and the scan-mask kernel run on while
@@ -1327,9 +1329,9 @@ int sr_sample_batch(sr_ctx* ctx, const void* logits, int dtype, int logits_on_de
         if (rc != SR_OK) return rc;
     }
     // (the layout of this call's logits is known before the upload: the scan masks are made for it)
-    ctx->last_epv = dtype == SR_DTYPE_BF16 ? 8 : 4;
-    ctx->last_base_mod = logits_on_device ? (unsigned)((uintptr_t)logits & 15u) : 0u;
-    ctx->last_stride_mod = (unsigned)((row_stride_elems * (dtype == SR_DTYPE_BF16 ? 2 : 4)) & 15);
+    ctx->tmp_batch->layout = ScanLayout{dtype == SR_DTYPE_BF16 ? 8 : 4, logits_on_device ? (unsigned)((uintptr_t)logits & 15u) : 0u,
+                                        (unsigned)((row_stride_elems * (dtype == SR_DTYPE_BF16 ? 2 : 4)) & 15)};
+    ctx->tmp_batch->layout_known = true;
     int rc = batch_upload_impl(ctx->tmp_batch, rows, vocab, params, hist_ids, hist_offsets, bias_ids, bias_vals, bias_offsets, allow_mask,
                                mask_stride_words, mask_active, uniforms, uniforms ? 1 : 0, false, false, nullptr, true);
     const void* dev = nullptr;

@@ -265,6 +265,13 @@ struct HostResults {
 #define SR_NO_TOKEN 0x80000000u  // ... for a token or an index (both -1 and above)
 #define SR_NO_FLAGS 0x7fffffffu  // ... for a row's flags (no row carries them all)
 
+// What scan masks depend on of the logits that they are used with: elements of a 16-byte vector, base address and row
+// stride (bytes) modulo 16.
+struct ScanLayout {
+    int epv = 4;
+    unsigned base_mod = 0, stride_mod = 0;
+};
+
 struct sr_ctx {
     int device = 0;
     hipStream_t own_stream = nullptr;
@@ -299,9 +306,7 @@ struct sr_ctx {
     PinnedPool pinned;
     HostResults results;
     unsigned long long* prof = nullptr;  // test hook: phase timestamps of the selection kernel
-    // vector width and alignment of the last launch's logits: what an upload builds scan masks for
-    int last_epv = 4;
-    unsigned last_base_mod = 0, last_stride_mod = 0;
+    ScanLayout last_layout;  // of the last launch's logits: what the first upload of a batch builds scan masks for
     // Registered allow-masks (sr_mask_register): one device array of `pool_cap` slots of `pool_words` words each, the
     // id of a mask is its slot.  One vocabulary size per context at a time.
     DeviceBuf mask_pool;
@@ -343,6 +348,10 @@ struct sr_batch {
     // what the scan masks were built for: elements per 16-byte vector, the logits base address modulo 16 and
     // the row stride in bytes modulo 16 (rows share a mask row only when all start at the same offset)
     int32_t scan_epv = 0, scan_base_mod = -1, scan_stride_mod = -1;
+    // of the logits that the batch was last launched with, the guess for the next upload's (a batch mostly meets the same
+    // tensor again; the context's other batches may meet others)
+    bool layout_known = false;
+    ScanLayout layout;
     bool has_mask = false;
     bool mask_ids = false;               // the rows' allow-masks are registered masks of the context (mask_row = id)
     std::vector<int32_t> keep_mask_ids;  // ... per row, -1 none

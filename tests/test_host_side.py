@@ -93,3 +93,19 @@ def test_scan_masks_that_could_not_be_made_are_made_by_the_next_launch(ctx):
     assert ctx.L.cpu_scan_builds() == made + 1
     assert [ctx.L.cpu_scan_row(r) for r in range(8)] == list(range(8))  # the descriptors that the kernel reads
     b.close()
+
+
+def test_an_upload_makes_scan_masks_for_the_logits_of_its_own_batch(ctx):
+    """Two batches take turns on one context, one with aligned fp32 logits, one with bf16 rows at odd addresses: after each has
+    been launched once, no launch builds masks again or waits."""
+    p = [SamplingParams(Temperature=0.8, TopK=40)] * 4
+    a, b = ctx.new_batch(), ctx.new_batch()
+    for step in range(4):
+        for batch, vocab, addr, dtype in ((a, 1_000, 4096, sa.SR_DTYPE_F32), (b, 1_001, 4098, sa.SR_DTYPE_BF16)):
+            batch.upload(p, vocab, np.full(4, 0.5))
+            made, waits = ctx.L.cpu_scan_builds(), ctx.L.cpu_stream_waits()
+            _launch(ctx, batch, addr, dtype)
+            if step:
+                assert (ctx.L.cpu_scan_builds(), ctx.L.cpu_stream_waits()) == (made, waits)
+    a.close()
+    b.close()
