@@ -72,3 +72,16 @@ def test_launches_of_more_rows_than_the_whole_device_takes(ctx):
     assert np.array_equal(got[:18], want)
     few = ctx.sample_batch(dev[:90], params[:90], u[:90])
     assert np.array_equal(got[:90], few)
+
+
+@pytest.mark.parametrize("vocab", [8_191, 40_003])
+@pytest.mark.parametrize("spread", [0.0, 0.02, 6.0, 60.0])
+def test_rows_whose_mass_lies_anywhere_between_one_size_and_many(ctx, vocab, spread):
+    """What a row's workgroups add up by size decides how much of the row is listed: mass in one bucket (to its full count of a
+    workgroup, 8,192 equal entries), around a boundary of two, over every doubling that there is, in zeros and denormals."""
+    rng = np.random.default_rng(int(10 * spread))
+    logits = (-spread * rng.random((len(PARAMS), vocab))).astype(np.float32)
+    logits[:, vocab // 2] = 0.0
+    if spread == 60.0:
+        logits[:, ::3] -= 60.0                     # e down to 1e-52: denormals, zeros
+    _check(ctx, logits, torch.from_numpy(logits).cuda(), PARAMS, rng)
