@@ -1084,6 +1084,8 @@ __device__ __forceinline__ bool row_is_listed(const SrRow& rd, const SrFullArgs&
 {
     return !a.lazy_scale && (a.mode == 0 || a.prepared) && a.seg_func != nullptr && rd.temperature > 0.0f && sr_row_cut(rd) && !(rd.top_k > 0 && rd.top_k < a.vocab);
 }
+// the longest list that its workgroup takes
+__device__ __forceinline__ int list_cap(bool big) { return big ? SR_LIST_CAP_BIG : SR_LIST_CAP_SMALL; }
 // A sampled row that nothing cuts.
 __device__ __forceinline__ bool row_is_plain(const SrRow& rd, const SrFullArgs& a)
 {
@@ -1484,7 +1486,8 @@ __device__ __forceinline__ uint32_t seg_max_key(const float (&x)[SR_SEQ_RUN])
 }
 // The mass of a row's e by size: kMassBuckets buckets, eight to a doubling, bucket 0 just below 1, the last one everything
 // small.  From the sums over all of the row: the smallest value (as bits) whose bucket still has to be listed for the
-// listed entries to hold `share` of the row's mass and a little more.
+// listed entries to hold `share` of the row's mass and a little more; *least = that many entries the list has at least (a
+// bucket's mass over its largest value; the values of a bucket differ by an eighth at most).
 constexpr int kMassBuckets = 256;
 // A workgroup adds up its share in whole numbers: an entry e in (0, 1], x = 0x3f800000 - its bits, is 2^24 - x mod 2^23 units of
 // 2^(-24 - k) where k = x >> 23 counts the doublings down from 1, the same for all of a bucket; the upper 17 bits of that, added
@@ -1497,13 +1500,10 @@ __device__ __forceinline__ float mass_of_units(uint32_t units, int bucket)
 {
     return (float)units * sr_u2f((uint32_t)(127 - 24 + kMassDrop - (bucket >> 3)) << 23);
 }
-__device__ __forceinline__ uint32_t mass_list_from(const float* mass, float share)
+__device__ __forceinline__ uint32_t mass_list_from(const float (&v)[4], float share, float* least)
 {
     static_assert(kMassBuckets == 4 * SR_WAVE, "four buckets per lane");
     const int lane = sr_lane();
-    float v[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) v[q] = sr_load_agent(mass + 4 * lane + q);
     const float own = (v[0] + v[1]) + (v[2] + v[3]);
     const float incl = sr_wave_incl_sum_f32(own);
     const float total = sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(incl), SR_WAVE - 1));
@@ -1518,6 +1518,11 @@ __device__ __forceinline__ uint32_t mass_list_from(const float* mass, float shar
         if (upto >= target) d = 4 * lane + q;
     }
     d = sr_wave_min_i32(d);
+    float c_least = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; q++)  // (the last bucket's entries are of any size below the others')
+        if (4 * lane + q <= min(d, kMassBuckets - 2)) c_least += v[q] * __builtin_amdgcn_rcpf(sr_u2f(0x3f800000u - ((uint32_t)(4 * lane + q) << 20)));
+    *least = 0.99f * sr_wave_sum_f32(c_least);  // (sums and reciprocals are rounded)
     if (d >= kMassBuckets - 1) return 1u;  // everything above zero
     return 0x3f800000u - ((uint32_t)(d + 1) << 20) + 1u;
 }
@@ -1570,9 +1575,11 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_
     // (a row that min-p cuts as well lists everything down to its threshold: entries on it count for SR_OUT_AMBIGUOUS wherever
     // top-p ends)
     const bool by_mass = listed && use_top_p && !(rd.min_p > 0.0f);
+    const bool by_count = listed && !by_mass && a.mode != 0;
+    const uint32_t min_p_from = max(min_p_list_from(rd), 1u);
     // (the row's sum is at least 1: n entries below this make up less than half of what top-p leaves out)
     const float mass_min = (1.0f - rd.top_p) * 0.5f / (float)n;
-    if (by_mass) {
+    if (by_mass || by_count) {
         for (int i = threadIdx.x; i < kMassBuckets; i += kThreads) mass[i] = 0u;
         if (threadIdx.x == 0) mass_rest = 0.0f;
     }
@@ -1715,6 +1722,12 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_
             }
             small = sr_wave_sum_f32(small);
             if (lane == 0) unsafeAtomicAdd(&mass_rest, small);
+        } else if (by_count) {
+            // how many entries the list will have
+            int c = 0;
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) c += __popcll(__ballot(sr_f2u(e[j]) >= min_p_from));
+            if (lane == 0 && c > 0) atomicAdd(&mass[0], (uint32_t)c);
         }
         float sum = 0.0f;
 #pragma unroll
@@ -1751,11 +1764,14 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_
         if (lane == 0) sr_store_agent(&sums[seg], own[s]);
     }
     sr_barrier_lds();
-    if (by_mass)
+    if (by_mass) {
         for (int i = threadIdx.x; i < kMassBuckets; i += kThreads) {
             const float v = i < kMassBuckets - 1 ? mass_of_units(mass[i], i) : mass_rest;
             if (v > 0.0f) unsafeAtomicAdd(a.mass + (size_t)slot * kMassBuckets + i, v);
         }
+    } else if (by_count && threadIdx.x == 0 && mass[0] > 0u) {
+        unsafeAtomicAdd(a.mass + (size_t)slot * kMassBuckets, (float)mass[0]);  // (a whole number below 2^24)
+    }
     if (plain && threadIdx.x < kS * SR_SEQ_CHAINS) {
         const int hb = (int)blockIdx.x * kS + (int)threadIdx.x / SR_SEQ_CHAINS;
         if (hb < a.chain_stride / SR_SEQ_CHAINS)
@@ -1764,14 +1780,35 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_
     sr_drain_stores();
     __syncthreads();
     if (!met(1)) return;
+    // (the row's mass by size, four buckets a lane, or the length of its list, on its way beside the segments' sums)
+    float row_mass[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const float* const mass_at = a.mass + (size_t)slot * kMassBuckets;
+    if (by_mass) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) row_mass[q] = sr_load_agent(mass_at + 4 * lane + q);
+    } else if (by_count) {
+        row_mass[0] = sr_load_agent(mass_at);
+    }
     for (int g = threadIdx.x; g < nseg; g += kThreads) share[g] = sr_load_agent(&sums[g]);
     // what the list of a row that is cut holds: everything that can survive its min-p, or enough of the largest for top-p
     uint32_t from = 0xffffffffu;
+    bool too_long = false;
     if (listed) {
-        from = by_mass ? mass_list_from(a.mass + (size_t)slot * kMassBuckets, rd.top_p) : 1u;
-        from = max(from, min_p_list_from(rd));
-        from = max(from, 1u);
-        if (blockIdx.x == 0 && threadIdx.x == 0) st->list_from = from;
+        // A list that is longer than the row's workgroup takes is not made: a flat row's held most of the row, eight bytes an
+        // entry, for nothing.  Where a distribution is handed out the row goes on from e in the caller's row, and that is put
+        // there from here.  Every workgroup of the row comes to the same answer from the same sums.  (Distributions of 16
+        // flat rows of 151,936 that min-p cuts: 196 us with the list and a copy of the row by its one workgroup, this 138; the
+        // pass over 64 rows of tokens at temperature 2, before its sums were whole numbers, 114 -> 81.  Counting costs 0.8 us of
+        // 35 where min-p cuts; tokens alone gain by it only in flat rows, 16 of them 159 -> 136 us, and go without.)
+        float least;
+        if (by_mass) {
+            from = mass_list_from(row_mass, rd.top_p, &least);
+        } else {
+            from = min_p_from;
+            least = row_mass[0];
+        }
+        too_long = least > (float)list_cap(a.big_slabs != 0);
+        if (blockIdx.x == 0 && threadIdx.x == 0) st->list_from = too_long ? 0u : from;
     }
     sr_barrier_lds();
 #pragma unroll
@@ -1782,7 +1819,22 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_
         for (int g = lane; g < seg; g += SR_WAVE) before += share[g];
         before = sr_wave_sum_f32(before);
         seg_make_record(t[s], seg, (double)before, recs + seg, own[s]);
-        if (listed) {
+        if (too_long) {
+            if (a.mode != 0) {
+                float* const p = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;
+                const int i0 = seg * SR_SEG_TERMS + lane * SR_SEQ_RUN;
+#pragma unroll
+                for (int j = 0; j < SR_SEQ_RUN; j += 4) {
+                    if (i0 + j + 4 <= n) {
+                        sr_store_f4(p + i0 + j, t[s][j], t[s][j + 1], t[s][j + 2], t[s][j + 3]);
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < 4; q++)
+                            if (i0 + j + q < n) p[i0 + j + q] = t[s][j + q];
+                    }
+                }
+            }
+        } else if (listed) {
             // the segment's entries of the list, in the order of their indices, at the segment's own place in the row's lists
             uint32_t bits = 0u;
 #pragma unroll
@@ -2635,7 +2687,6 @@ __device__ __forceinline__ void sort_survivors_in_place(uint32_t* keys, int32_t*
 // -- 600 KB each at what one compute unit takes in -- were two thirds.)
 enum ListWay : int { kListDone = 0, kListDeferred = 1, kListGeneral = 2 };
 __device__ __forceinline__ int list_place(int i) { return i + (i >> 4); }  // (runs of 16 start in different banks)
-__device__ __forceinline__ int list_cap(bool big) { return big ? SR_LIST_CAP_BIG : SR_LIST_CAP_SMALL; }
 
 __device__ __forceinline__ uint32_t* list_values(uint32_t* more, FullSmem& sm) { return more ? more : (uint32_t*)sm.sortbuf; }
 
@@ -3102,7 +3153,8 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
         // Softmax (Sampler.cs:448-472): the maximum and e = expf(x - max) were computed by the kernels before
         const bool alone = a.seg_func != nullptr && (st->late == a.seq || full_maxkey_of(a, st->maxkey) == kKeyInf);
         const bool walked = a.seg_func != nullptr && !alone;
-        const bool has_list = walked && row_is_listed(rd, a), plain = walked && row_is_plain(rd, a);
+        // (a list that would have been too long was not made)
+        const bool has_list = walked && row_is_listed(rd, a) && st->list_from != 0u, plain = walked && row_is_plain(rd, a);
         float* const e_row = walked ? row_e(a, slot) : p;
         const uint32_t mk = alone ? row_alone(a, rd, p, n, row, sm) : full_maxkey_of(a, st->maxkey);
         const bool any_nan = mk == 0xffffffffu;
@@ -3230,8 +3282,8 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                     return;
                 }
             }
-            if (e_row != p) {
-                // (a row whose list was too long goes on here: its probabilities take shape in the caller's row)
+            if (e_row != p && !(row_is_listed(rd, a) && st->list_from == 0u)) {
+                // (a row that goes on here has its probabilities take shape in the caller's row; one without a list has e there)
                 for (int i = tid; i < n; i += kT) p[i] = e_row[i];
                 sr_drain_stores();
                 __syncthreads();

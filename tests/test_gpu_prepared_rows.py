@@ -85,3 +85,32 @@ def test_rows_whose_mass_lies_anywhere_between_one_size_and_many(ctx, vocab, spr
     if spread == 60.0:
         logits[:, ::3] -= 60.0                     # e down to 1e-52: denormals, zeros
     _check(ctx, logits, torch.from_numpy(logits).cuda(), PARAMS, rng)
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("rows,candidates", [(9, 16_383), (9, 16_384), (9, 16_385), (9, 18_700), (9, 40_003), (300, 4_096), (300, 4_097), (300, 4_800)])
+def test_lists_around_the_longest_that_a_row_takes(ctx, rows, candidates, dtype):
+    """`candidates` entries near the maximum, the rest far below: lists that just fit, that do not but cannot be told from the
+    sums by size, and that are not made; rows at odd addresses, with a compute unit each and without."""
+    vocab = 40_003
+    rng = np.random.default_rng(candidates)
+    base = rng.normal(-30.0, 0.5, (9, vocab)).astype(np.float32)
+    for r in range(9):
+        at = rng.permutation(vocab)[:candidates]
+        base[r, at] = 3.0 + 0.25 * rng.random(candidates).astype(np.float32) * (r % 3)
+    x = torch.from_numpy(base).to(torch.bfloat16 if dtype == "bf16" else torch.float32)
+    base = x.float().numpy()
+    some = [SamplingParams(TopP=0.9999), SamplingParams(MinP=0.3), SamplingParams(MinP=0.3, TopP=0.9), SamplingParams(TopP=0.6),
+            SamplingParams(MinP=0.02, TopP=0.999), SamplingParams(MinP=0.9), SamplingParams(TopP=0.9999, FrequencyPenalty=0.1, PreviousTokens=[1, 2, 2]),
+            SamplingParams(MinP=0.3, TopP=0.2), SamplingParams(Temperature=2.0, TopP=0.9)]
+    params, u = [some[i % 9] for i in range(rows)], np.repeat(rng.random(rows // 9 + 1), 9)[:rows]
+    dev = x.cuda()[torch.arange(rows, device="cuda") % 9].contiguous()
+    few = rows if rows < 20 else 18
+    logits = base[np.arange(few) % 9]
+    got = ctx.sample_batch(dev, params, u)
+    assert np.array_equal(got[:few], oracle_tokens(logits, params[:few], u[:few]))
+    tokens, probs = ctx.sample_with_distribution(dev, params, u)
+    assert np.array_equal(tokens, got)
+    for r in range(9):
+        want = orc.build_filtered_distribution(logits[r], to_oracle(params[r]))
+        assert np.array_equal(probs[r].cpu().numpy().view(np.uint32), want.view(np.uint32)), r
