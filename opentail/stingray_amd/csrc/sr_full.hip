@@ -1570,7 +1570,8 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_
     if (threadIdx.x < 32) tab[threadIdx.x] = sr_exp2f_tab[threadIdx.x];
     const SegSource<ES> src = seg_source<ES>(rd, a, slot, row);
     float* const w = row_e(a, slot);
-    const bool plain = a.prepared && row_is_plain(rd, a), listed = row_is_listed(rd, a);
+    // (four segments a wave: the verifier's launches, which list nothing)
+    const bool plain = a.prepared && row_is_plain(rd, a), listed = kS != 4 && row_is_listed(rd, a);
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
     // (a row that min-p cuts as well lists everything down to its threshold: entries on it count for SR_OUT_AMBIGUOUS wherever
     // top-p ends)
@@ -1820,19 +1821,12 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_
         before = sr_wave_sum_f32(before);
         seg_make_record(t[s], seg, (double)before, recs + seg, own[s]);
         if (too_long) {
-            if (a.mode != 0) {
+            if (a.mode != 0) {  // (what is left of the row's last four, k_full_row copies)
                 float* const p = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;
                 const int i0 = seg * SR_SEG_TERMS + lane * SR_SEQ_RUN;
 #pragma unroll
-                for (int j = 0; j < SR_SEQ_RUN; j += 4) {
-                    if (i0 + j + 4 <= n) {
-                        sr_store_f4(p + i0 + j, t[s][j], t[s][j + 1], t[s][j + 2], t[s][j + 3]);
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < 4; q++)
-                            if (i0 + j + q < n) p[i0 + j + q] = t[s][j + q];
-                    }
-                }
+                for (int j = 0; j < SR_SEQ_RUN; j += 4)
+                    if (i0 + j + 4 <= n) sr_store_f4(p + i0 + j, t[s][j], t[s][j + 1], t[s][j + 2], t[s][j + 3]);
             }
         } else if (listed) {
             // the segment's entries of the list, in the order of their indices, at the segment's own place in the row's lists
@@ -3282,9 +3276,10 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                     return;
                 }
             }
-            if (e_row != p && !(row_is_listed(rd, a) && st->list_from == 0u)) {
-                // (a row that goes on here has its probabilities take shape in the caller's row; one without a list has e there)
-                for (int i = tid; i < n; i += kT) p[i] = e_row[i];
+            if (e_row != p) {
+                // (a row that goes on here has its probabilities take shape in the caller's row; one whose list was not made has
+                // all but the last of e there)
+                for (int i = tid + (row_is_listed(rd, a) && st->list_from == 0u ? n & ~3 : 0); i < n; i += kT) p[i] = e_row[i];
                 sr_drain_stores();
                 __syncthreads();
             }

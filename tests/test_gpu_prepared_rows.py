@@ -114,3 +114,22 @@ def test_lists_around_the_longest_that_a_row_takes(ctx, rows, candidates, dtype)
     for r in range(9):
         want = orc.build_filtered_distribution(logits[r], to_oracle(params[r]))
         assert np.array_equal(probs[r].cpu().numpy().view(np.uint32), want.view(np.uint32)), r
+
+
+@pytest.mark.parametrize("vocab", [8, 900, 4_095, 1_048_577])
+def test_rows_that_their_own_workgroup_adds(ctx, vocab):
+    """Too short or too long for the whole device, cut by min-p: nothing but the maximum left, a few entries, as many as the
+    survivors' list holds and more, a threshold too small to bound anything."""
+    rng = np.random.default_rng(vocab)
+    some = [SamplingParams(MinP=0.3), SamplingParams(MinP=0.05, TopP=0.9), SamplingParams(Temperature=2.0, MinP=0.002), SamplingParams(MinP=1e-33),
+            SamplingParams(MinP=1.0), SamplingParams(Temperature=0.5, MinP=0.01, PresencePenalty=0.5, PreviousTokens=[3, 3, 5])]
+    some = some[:3] if vocab > 1_000_000 else some
+    logits = rng.normal(0, 1.5, (len(some), vocab)).astype(np.float32)
+    _check(ctx, logits, torch.from_numpy(logits).cuda(), some, rng)
+    at = rng.permutation(vocab)
+    for close in (vocab, 4_097, 4_096):            # equal entries at the top: as many as the list holds, one more, all
+        logits[:] = -9.0
+        logits[:, at[:close]] = 1.0
+        _check(ctx, logits, torch.from_numpy(logits).cuda(), some, rng)
+        if close >= vocab and vocab < 4_096:
+            break
