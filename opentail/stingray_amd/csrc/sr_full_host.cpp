@@ -49,7 +49,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     const int nseg = (vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
     const bool seg_mode = vocab >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX;
     a.edits_in_pass = seg_mode ? 1 : 0;
-    bool any_table = false, any_copy = false, any_edits = false, any_list = false, prepared = false;
+    bool any_table = false, any_copy = false, any_edits = false, any_list = false, prepared = false, any_min_p = false;
     int n_sampled = 0, n_seen = 0;
     for (const SrRow& r : (host_rows ? *host_rows : b->h_rows)) {
         if (mode == 0 && r.path != SR_PATH_FULL) continue;
@@ -61,15 +61,22 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
         any_copy = any_copy || !(r.temperature > 0.0f && (r.edit_cnt <= 0 || on_the_fly));
         if (seg_mode && r.temperature > 0.0f && !(r.top_k > 0 && r.top_k < vocab)) {
             any_list = any_list || sr_row_cut(r);
-            // Rows that the row kernel may leave to the whole device: those that nothing cuts, that only top-p cuts (a few
-            // members or tens of thousands), and all of them where distributions are handed out.  A min-p of some size
-            // leaves a few hundred entries at most, and three launches that find nothing to do cost 6 us.
-            prepared = prepared || !sr_row_cut(r) || mode != 0 || !(r.min_p >= 0.002f);
+            // Rows that the row kernel may leave to the whole device: those that nothing cuts and, but for the verifier, whose
+            // reader takes e where it is, those that only top-p cuts (a few members or tens of thousands).  What a min-p of some
+            // size leaves is mostly little, and nobody knows before the launch: tokens of 64 rows of 151,936 with 300 entries left
+            // take 72 us, 78 where three launches follow that find nothing to do; with 2,000 77 against 128, since up to 8,192
+            // the row's workgroup then finishes by itself; with 8,300 to 16,384 184 against 147, and with more the launches find
+            // nothing again.  Distributions: SR_PREPARED_MIN_SEGS_MIN_P, whatever the min-p.
+            const bool by_min_p = mode != 0 ? r.min_p > 0.0f : r.min_p >= 0.002f;
+            prepared = prepared || (lazy_scale ? !sr_row_cut(r) : !by_min_p);
+            any_min_p = any_min_p || by_min_p;
         }
     }
     const bool odd_rows = mode != 0 && (probs_stride & 3) != 0;
     prepared = prepared && nseg >= (lazy_scale ? SR_PREPARED_MIN_SEGS_VERIFY : odd_rows ? SR_PREPARED_MIN_SEGS_ODD : SR_PREPARED_MIN_SEGS) &&
                (long long)n_rows * nseg <= (lazy_scale ? SR_PREPARED_SEGS_VERIFY : mode != 0 ? SR_PREPARED_SEGS_DISTRIBUTIONS : SR_PREPARED_SEGS);
+    if (mode != 0 && !lazy_scale && any_min_p)
+        prepared = prepared || (nseg >= SR_PREPARED_MIN_SEGS_MIN_P && (long long)n_rows * nseg <= SR_PREPARED_SEGS_MIN_P);
     a.any_copy = any_copy ? 1 : 0;
     a.any_edits = any_edits ? 1 : 0;
     a.n_sampled = (int)((long long)n_sampled * n_rows / std::max(1, n_seen));  // (a verifier's launch has every row several times)

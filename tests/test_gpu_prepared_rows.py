@@ -133,3 +133,27 @@ def test_rows_that_their_own_workgroup_adds(ctx, vocab):
         _check(ctx, logits, torch.from_numpy(logits).cuda(), some, rng)
         if close >= vocab and vocab < 4_096:
             break
+
+
+@pytest.mark.parametrize("vocab", [16_385, 40_000, 131_073])
+@pytest.mark.parametrize("rows", [1, 17, 40])
+def test_launches_that_min_p_alone_cuts(ctx, vocab, rows):
+    """On both sides of the lines between the whole device and the row's workgroup: distributions of few long rows, of more and of
+    shorter ones, with a handful, hundreds and most of the entries left."""
+    rng = np.random.default_rng(vocab + rows)
+    some = [SamplingParams(MinP=0.05), SamplingParams(Temperature=2.0, MinP=0.002, TopP=0.9), SamplingParams(Temperature=30.0, MinP=0.6)]
+    base = rng.normal(0, 1.5, (3, vocab)).astype(np.float32)
+    base[0, :20] += 12.0 * np.arange(1, 21, dtype=np.float32) ** -1.1
+    params, u = [some[i % 3] for i in range(rows)], rng.random(rows)
+    x = torch.from_numpy(base).cuda()[torch.arange(rows, device="cuda") % 3].contiguous()
+    tokens, probs = ctx.sample_with_distribution(x, params, u)
+    few = min(rows, 6)
+    logits = base[np.arange(few) % 3]
+    want = oracle_tokens(logits, params[:few], u[:few])
+    assert np.array_equal(tokens[:few], want)
+    assert np.array_equal(ctx.sample_batch(x, params, u), tokens)
+    for r in range(rows):
+        assert torch.equal(probs[r], probs[r % 3])
+    for r in range(min(rows, 3)):
+        want = orc.build_filtered_distribution(logits[r], to_oracle(params[r]))
+        assert np.array_equal(probs[r].cpu().numpy().view(np.uint32), want.view(np.uint32)), r
