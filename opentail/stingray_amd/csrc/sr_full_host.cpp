@@ -72,8 +72,12 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             any_min_p = any_min_p || by_min_p;
         }
     }
-    const bool odd_rows = mode != 0 && (probs_stride & 3) != 0;
-    prepared = prepared && nseg >= (lazy_scale ? SR_PREPARED_MIN_SEGS_VERIFY : odd_rows ? SR_PREPARED_MIN_SEGS_ODD : SR_PREPARED_MIN_SEGS) &&
+    // (distributions at odd addresses, where the row's workgroup passes over its row an entry at a time: at every length.  1, 16 and
+    // 64 rows cut by top-p, of 4,099: 59, 67, 70 us against 95, 106, 109; of 12,289: 71, 81, 82 against 115, 120, 122; of 24,001:
+    // 83, 91, 97 against 141, 174, 176; that nothing cuts, of 4,099: 41, 45, 50 against 50, 53, 56; only sharp rows of some lengths lose, 16 of 12,289 at top-p
+    // 0.9 and temperature 0.4 59 against 50, of 4,097 49 against 88)
+    const bool odd_rows = mode != 0 && !lazy_scale && (probs_stride & 3) != 0;
+    prepared = prepared && (odd_rows || nseg >= (lazy_scale ? SR_PREPARED_MIN_SEGS_VERIFY : SR_PREPARED_MIN_SEGS)) &&
                (long long)n_rows * nseg <= (lazy_scale ? SR_PREPARED_SEGS_VERIFY : mode != 0 ? SR_PREPARED_SEGS_DISTRIBUTIONS : SR_PREPARED_SEGS);
     if (mode != 0 && !lazy_scale && any_min_p)
         prepared = prepared || (nseg >= SR_PREPARED_MIN_SEGS_MIN_P && (long long)n_rows * nseg <= SR_PREPARED_SEGS_MIN_P);

@@ -113,7 +113,6 @@ struct SrMaskClear {
 // 65,536: 69 against 65 us, of 131,072: 80 against 79, 2 rows of 262,144: 70 against 84.)
 #define SR_PREPARED_MIN_SEGS 32
 #define SR_PREPARED_MIN_SEGS_VERIFY 128
-#define SR_PREPARED_MIN_SEGS_ODD 16  // distributions at odd addresses, 16 rows of 24,001: 57 against 78 us
 // Distributions of rows that min-p cuts, where no other row asks for those launches: worth it for few long rows.  20,
 // 200, 2,000, 8,000 and 15,000 entries left, 16 rows of 262,144: 71, 98, 106, 120, 143 us against 88, 99, 118, 181, 184 without;
 // of 131,072: 59, 79, 83, 101, 126 against 56, 68, 85, 112, 113; one row: 47, 63, 68, 87, 104 against 51, 60, 78, 102, 103; 64 rows
