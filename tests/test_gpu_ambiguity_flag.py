@@ -104,3 +104,78 @@ def test_a_random_batch_flags_few_rows(ctx):
     w2 = synthetic.config2()
     got, flags = ctx.sample_batch(_cuda(w2.logits), w2.params, w2.uniforms, return_flags=True)
     assert int(((flags & SR_OUT_AMBIGUOUS) != 0).sum()) <= 1
+
+
+# ---- rows that the whole device prepares (4,096 entries and more; normalised and drawn by it from 32,768 on) ---------------
+
+LONG = {"short_list": SamplingParams(Temperature=0.35, TopP=0.9),  # a nucleus of a handful: one wave cuts and draws
+        "list": SamplingParams(Temperature=0.8, TopP=0.5),          # hundreds: the row's workgroup
+        "long_nucleus": SamplingParams(TopP=0.9),                   # thousands: the whole device
+        "min_p": SamplingParams(Temperature=0.9, MinP=0.02),
+        "min_p_top_p": SamplingParams(Temperature=0.9, MinP=0.1, TopP=0.9),
+        "plain": SamplingParams(Temperature=1.2)}
+# (how many members each has, which is what decides the way that the row takes)
+LONG_MEMBERS = {"short_list": (4, 30), "list": (100, 1_000), "long_nucleus": (1_100, 16_000), "min_p": (100, 1_000),
+                "min_p_top_p": (65, 1_000), "plain": (33_000, 33_000)}
+
+
+def _long_row(rng):
+    row = rng.normal(0, 1.5, 33_000).astype(np.float32)
+    row[rng.integers(0, len(row), 12)] += np.linspace(6, 2, 12).astype(np.float32)
+    return row
+
+
+@pytest.mark.parametrize("kind", list(LONG))
+def test_draws_of_long_rows_on_and_off_a_boundary(ctx, kind):
+    rng = np.random.default_rng(list(LONG).index(kind) + 20)
+    row, p = _long_row(rng), LONG[kind]
+    lo, hi = LONG_MEMBERS[kind]
+    assert lo <= int((orc.build_filtered_distribution(row, to_oracle(p)) > 0).sum()) <= hi
+    on, mid = _boundaries(row, p, 8, rng)
+    assert len(on) >= 6 and len(mid) >= 6
+    us = np.array(on + mid)
+    logits = np.tile(row, (len(us), 1))
+    got, flags = ctx.sample_batch(_cuda(logits), [p] * len(us), us, return_flags=True)
+    assert np.array_equal(got, oracle_tokens(logits, [p] * len(us), us))
+    amb = (flags & SR_OUT_AMBIGUOUS) != 0
+    assert amb[: len(on)].all(), (kind, np.nonzero(~amb[: len(on)])[0])
+    assert not amb[len(on):].any(), (kind, np.nonzero(amb[len(on):])[0])
+
+
+def test_cuts_of_long_rows_on_and_off_a_boundary(ctx):
+    """top-p set to the running sum behind the k-th probability and min-p to the ratio of the k-th to the first: the cut is flagged
+    wherever it is made, and not when it lies between two far apart."""
+    rng = np.random.default_rng(31)
+    row = _long_row(rng)
+    e = np.exp(row - row.max())
+    y = np.sort(e * np.float32(1.0 / np.cumsum(e, dtype=np.float32)[-1]))[::-1]
+    run = np.cumsum(y, dtype=np.float32)
+    params, want = [], []
+    for k in (1, 9, 40, 300, 900, 1_500, 7_000):
+        params += [SamplingParams(TopP=float(run[k])), SamplingParams(MinP=float(y[k] / y[0])), SamplingParams(MinP=1e-4, TopP=float(run[k]))]
+        want += [True, True, True]
+    for k in (1, 3, 6):                                # halfway between sums, between probabilities
+        params += [SamplingParams(TopP=float(run[k] + y[k + 1] / 2)), SamplingParams(MinP=float((y[k] + y[k + 1]) / 2 / y[0]))]
+        want += [False, False]
+    u = np.full(len(params), 0.0)                      # (the first member: far from any boundary of the draw)
+    first = int(np.argmax(row))
+    row[[0, first]] = row[[first, 0]]                  # ... the row's largest entry, so that u = 0.2 of it draws it
+    u[:] = 0.2 * float(y[0])
+    logits = np.tile(row, (len(params), 1))
+    got, flags = ctx.sample_batch(_cuda(logits), params, u, return_flags=True)
+    assert np.array_equal(got, oracle_tokens(logits, params, u))
+    amb = (flags & SR_OUT_AMBIGUOUS) != 0
+    assert np.array_equal(amb, np.array(want)), [(i, params[i]) for i in np.nonzero(amb != np.array(want))[0]]
+
+
+@pytest.mark.parametrize("run_length", [30, 500, 6_000])
+def test_cuts_of_long_rows_inside_a_run_of_equal_probabilities_are_flagged(ctx, run_length):
+    rng = np.random.default_rng(run_length)
+    row = rng.normal(-12.0, 0.5, 33_000).astype(np.float32)
+    row[rng.permutation(len(row))[:run_length]] = 2.0
+    params = [SamplingParams(TopP=0.5), SamplingParams(MinP=0.5, TopP=0.5), SamplingParams(MinP=0.5)]  # (min-p keeps the whole run)
+    logits = np.tile(row, (3, 1))
+    u = np.full(3, 0.3)
+    got, flags = ctx.sample_batch(_cuda(logits), params, u, return_flags=True)
+    assert np.array_equal(got, oracle_tokens(logits, params, u))
+    assert ((flags & SR_OUT_AMBIGUOUS) != 0).tolist()[:2] == [True, True]

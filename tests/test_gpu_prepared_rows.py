@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from opentail.stingray_amd import SamplerContext, SamplingParams
+from opentail.stingray_amd import SamplerContext, SamplingParams, pack_allow_mask
 from oracle import binding as orc
 from tests.helpers import oracle_tokens, to_oracle
 
@@ -157,3 +157,42 @@ def test_launches_that_min_p_alone_cuts(ctx, vocab, rows):
     for r in range(min(rows, 3)):
         want = orc.build_filtered_distribution(logits[r], to_oracle(params[r]))
         assert np.array_equal(probs[r].cpu().numpy().view(np.uint32), want.view(np.uint32)), r
+
+
+def test_masked_biased_and_penalised_rows(ctx):
+    """Allow-masks from three tokens to nearly all, logit bias (on ids that are masked, outside the vocabulary, enough to change the
+    maximum) and long histories, on every way that a prepared row takes; distributions built alone as well."""
+    rng = np.random.default_rng(8)
+    vocab = 50_021
+    some = [SamplingParams(), SamplingParams(TopP=0.9), SamplingParams(Temperature=1.5, TopP=0.98), SamplingParams(MinP=0.02),
+            SamplingParams(Temperature=0.7, MinP=0.001, TopP=0.95)]
+    rows = 3 * len(some)
+    logits = rng.normal(0, 1.5, (rows, vocab)).astype(np.float32)
+    allowed = np.ones((rows, vocab), dtype=bool)
+    params = []
+    for r in range(rows):
+        p = some[r % len(some)]
+        if r < 5:
+            allowed[r] = rng.random(vocab) < (0.5, 0.01, 0.9, 0.3, 0.05)[r]
+            allowed[r, [3, 4_000, vocab - 1]] = True
+        elif r < 10:
+            ids = [int(i) for i in rng.integers(0, vocab, 40)] + [0, vocab - 1]
+            p = SamplingParams(Temperature=p.Temperature, TopP=p.TopP, MinP=p.MinP, LogitBias={**{i: float(b) for i, b in zip(ids, rng.normal(0, 4, len(ids)))}, 7: 9.5, vocab + 3: 50.0})
+        else:
+            p = SamplingParams(Temperature=p.Temperature, TopP=p.TopP, MinP=p.MinP, RepetitionPenalty=1.3, FrequencyPenalty=0.2,
+                               RepeatLastN=300, PreviousTokens=[int(i) for i in rng.integers(0, vocab, 700)])
+        params.append(p)
+    allowed[12, ::2] = False                       # a mask beside penalties
+    allowed[6, 7] = False                          # ... and in front of a bias
+    mask = pack_allow_mask(allowed)
+    u = rng.random(rows)
+    got = ctx.sample_batch(torch.from_numpy(logits).cuda(), params, u, mask)
+    assert np.array_equal(got, oracle_tokens(logits, params, u, mask))
+    masked = np.where(allowed, logits, -np.inf).astype(np.float32)
+    with_masks = ctx.build_distribution(torch.from_numpy(logits).cuda(), params, allow_mask=mask).cpu().numpy()
+    tokens, drawn_from = ctx.sample_with_distribution(torch.from_numpy(masked).cuda(), params, u)
+    for r, p in enumerate(params):
+        want = orc.build_filtered_distribution(masked[r], to_oracle(p))
+        assert np.array_equal(with_masks[r].view(np.uint32), want.view(np.uint32)), r
+        assert np.array_equal(drawn_from[r].cpu().numpy().view(np.uint32), want.view(np.uint32)), r
+    assert np.array_equal(tokens, got)
