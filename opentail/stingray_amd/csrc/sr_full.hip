@@ -1091,9 +1091,8 @@ __device__ __forceinline__ bool row_is_plain(const SrRow& rd, const SrFullArgs& 
 {
     return a.seg_func != nullptr && rd.temperature > 0.0f && !sr_row_cut(rd) && !(rd.top_k > 0 && rd.top_k < a.vocab);
 }
-// Where e = expf(x - max) of a row lies: in the work row, or, where distributions are handed out, in scratch memory of its own.
-// (One place for all rows of a launch: with a choice per row the compiler, clang 22, took the stride of one buffer and the
-// base of the other.)
+// Where e = expf(x - max) of a row lies: in the work row, or, where distributions are handed out and the launches behind k_full_row
+// follow, in scratch memory of its own (one place for all rows of a launch, which the host names).
 __device__ __forceinline__ float* row_e(const SrFullArgs& a, int slot) { return a.e_rows + (size_t)slot * (size_t)a.e_stride; }
 // the walk by slabs over the row itself, for a row in scratch memory that only top-p cuts and whose list was too long
 __device__ __forceinline__ bool row_fast_nucleus(const SrRow& rd, const SrFullArgs& a)
@@ -1277,14 +1276,12 @@ __global__ __launch_bounds__(256) void k_full_exp(SrFullArgs a)
     }
 }
 
-// ---- the same two passes, laid out for a denominator that the whole device prepares -------------------------
-// (launches whose rows are long and start on 16-byte boundaries: a.seg_func is set.)  A wave takes whole segments of
-// SR_SEG_TERMS elements, every lane 16 consecutive ones, so that the second pass can leave, beside e = expf(x - max), the
-// record of the segment's exact sum (SeqSegFunc) for the row's workgroup to walk (seg_walk).  The binade that a
-// record is made for comes from approximate sums: the first pass leaves every segment's own maximum m and the sum
-// of exp(x - m) over it, and the second, which knows the row's maximum M, adds up S exp(m - M) over the segments in
-// front.  The ids that the row's edits touch take their adjusted values from the work row, where k_full_edits left
-// them: e is final when the second pass has written it.
+// ---- the same in one pass, laid out for a denominator that the whole device prepares ---------------------------
+// (launches of rows of SR_SEG_MIN_VOCAB to SR_SEG_MAX x SR_SEG_TERMS entries, at any address: a.seg_func is set.)  A wave takes whole
+// segments of SR_SEG_TERMS elements, in the end every lane 16 consecutive ones, and leaves beside e = expf(x - max) the
+// record of the segment's exact sum (SeqSegFunc) for the row's workgroup to walk (seg_walk).  The binade that a record is
+// made for comes from the segments' approximate sums of e.  The ids that a row's edits touch take their adjusted values as the
+// pass loads them (seg_apply_edits), or from the row's adjusted copy, where it keeps one: e is final when the pass has written it.
 template <int ES>
 struct SegSource {
     const char* rowp;      // the row's logits, or null: the adjusted copy in w
@@ -2164,7 +2161,7 @@ __device__ __forceinline__ int list_stretch(const float* p, int w0, int w1, bool
 
 // ---- the nucleus of a row that only top-p cuts, without a pass that writes the row ---------------------------------
 // The row holds e = expf(x - max); its probabilities are y = fl(e * inv) (y = e when the sum is 1), which rise with e.
-// While the exact sum passed over the row, the caller counted the e by their upper 16 bits in hcnt (LDS, kHistPos
+// The caller has counted the e by their upper 16 bits in hcnt (LDS, kHistPos
 // positions: position d holds the keys 0x3f80 - d, position 0 is e = 1, the last position everything below).  From the
 // counts: the longest run of positions from the top that holds at most kSmall entries (a slab), the first one shortened
 // to where a lower bound of its probability mass (count x the position's smallest value) passes top_p with a margin.

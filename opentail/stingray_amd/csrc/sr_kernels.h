@@ -144,7 +144,7 @@ struct SrFullState {
     uint32_t deferred;    // the number of the last launch that left the row's normalisation and draw to the whole device
     float ycut;           // ... whose members are the probabilities above ycut, and of those equal to it the ones up to idx_last
     int32_t idx_last;
-    uint32_t list_from;   // the row's list of candidates holds its e from this value on (as bits)
+    uint32_t list_from;   // the row's list of candidates holds its e from this value on (as bits); 0: it would have been too long
     int32_t pad[5];
 };
 static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
@@ -184,7 +184,7 @@ struct SrFullArgs {
     uint32_t* out_flags;       // [row], may be null
     unsigned long long* prof;  // optional phase timestamps of slot 0 [32] (test hook), normally null
     // The softmax denominators prepared by the whole device (k_full_softmax_seg, seg_walk); seg_func is
-    // null when the launch is not laid out for it (short or unaligned rows) and the rows are added by their workgroups.
+    // null where the rows are added by their workgroups (fewer entries than SR_SEG_MIN_VOCAB, or more than SR_SEG_MAX segments).
     SeqSegFunc* seg_func;          // [slot][seg_stride]
     int32_t seg_stride;
     float* seg_sum;                // [slot][seg_stride] about the sum of every segment's e (of its members, in a row that is cut)
@@ -192,7 +192,7 @@ struct SrFullArgs {
     int32_t chain_stride;
     int32_t chain_blocks;
     SeqSegFunc* chain_func;        // [slot][8][chain_blocks]
-    float* mass;                   // [slot][256] the row's mass by size of e; zero between launches
+    float* mass;                   // [slot][256] the row's mass by size of e, or (the first) the length of its list; zero between launches
     uint32_t* seg_cnt;             // [slot][seg_stride] entries of every segment in the row's list (sort_keys_in, sort_vals_in)
     float* e_rows;                 // [slot][e_stride] expf(x - max) of the rows; starts on 16 bytes
     int64_t e_stride;
