@@ -80,7 +80,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     prepared = prepared && (odd_rows || nseg >= (lazy_scale ? SR_PREPARED_MIN_SEGS_VERIFY : SR_PREPARED_MIN_SEGS)) &&
                (long long)n_rows * nseg <= (lazy_scale ? SR_PREPARED_SEGS_VERIFY : mode != 0 ? SR_PREPARED_SEGS_DISTRIBUTIONS : SR_PREPARED_SEGS);
     if (mode != 0 && !lazy_scale && any_min_p)
-        prepared = prepared || (nseg >= SR_PREPARED_MIN_SEGS_MIN_P && (long long)n_rows * nseg <= SR_PREPARED_SEGS_MIN_P);
+        prepared = prepared || (nseg >= (odd_rows ? SR_PREPARED_MIN_SEGS_MIN_P_ODD : SR_PREPARED_MIN_SEGS_MIN_P) && (long long)n_rows * nseg <= SR_PREPARED_SEGS_MIN_P);
     a.any_copy = any_copy ? 1 : 0;
     a.any_edits = any_edits ? 1 : 0;
     a.n_sampled = (int)((long long)n_sampled * n_rows / std::max(1, n_seen));  // (a verifier's launch has every row several times)

@@ -117,7 +117,10 @@ struct SrMaskClear {
 // 200, 2,000, 8,000 and 15,000 entries left, 16 rows of 262,144: 71, 98, 106, 120, 143 us against 88, 99, 118, 181, 184 without;
 // of 131,072: 59, 79, 83, 101, 126 against 56, 68, 85, 112, 113; one row: 47, 63, 68, 87, 104 against 51, 60, 78, 102, 103; 64 rows
 // of 151,936: 96, 125, 131, 145, 165 against 78, 90, 109, 145, 145; 16 rows of 32,768: 52, 68, 70, 90, 112 against 33, 48, 61, 62, 63.
+// At odd addresses, 16 rows of 65,537: 54, 72, 76, 93, 116 against 45, 56, 72, 129, 129; of 100,003: 58, 77, 80, 100, 121 against 51,
+// 62, 80, 163, 163; 64 rows of 100,003: 84, 109, 107, 123, 149 against 62, 76, 91, 176, 174.
 #define SR_PREPARED_MIN_SEGS_MIN_P 128
+#define SR_PREPARED_MIN_SEGS_MIN_P_ODD 96
 #define SR_PREPARED_SEGS_MIN_P 4096
 #define SR_PREPARED_SEGS 32768
 #define SR_PREPARED_SEGS_DISTRIBUTIONS 16384

@@ -135,7 +135,7 @@ def test_rows_that_their_own_workgroup_adds(ctx, vocab):
             break
 
 
-@pytest.mark.parametrize("vocab", [16_385, 40_000, 131_073])
+@pytest.mark.parametrize("vocab", [16_385, 40_000, 98_305, 131_072])
 @pytest.mark.parametrize("rows", [1, 17, 40])
 def test_launches_that_min_p_alone_cuts(ctx, vocab, rows):
     """On both sides of the lines between the whole device and the row's workgroup: distributions of few long rows, of more and of
