@@ -706,7 +706,7 @@ __device__ __forceinline__ float tp_sum_row(const float* p, int n, float mul, bo
 #pragma unroll
             for (int j = 0; j < 16; j++) x[j] = b[64 * j + ((lane + 2 * j) & 63)];
             int dummy;
-            sc = sr_seq_wave<16, false>(x, sc, 0.0f, &dummy);
+            sc = sr_seq_wave<16, false, true>(x, sc, 0.0f, &dummy);
         }
     };
     // (behind the last round the loop fetches that round again, to no effect: the compiler can wait for "all but the

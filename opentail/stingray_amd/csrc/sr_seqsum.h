@@ -290,56 +290,95 @@ __device__ __forceinline__ void sr_seq_tile(const float (&x)[SR_SEQ_RUN], float*
 }
 
 // ---- one wave by itself --------------------------------------------------------------------------------
-// The running sum s of the wave's 64 x N terms (lane order = term order, N consecutive terms per lane), crossing after
-// crossing, with no barrier and no shared memory: what a short list needs (a row tail's few hundred probabilities).
+// The running sum s of the wave's 64 x N terms (lane order = term order, N consecutive terms per lane), with no barrier
+// and no shared memory: what a short list (a row tail's few hundred probabilities), or one segment of a long sum, needs.
 // When kSearch, stops at the first term at which the running sum reaches `target`: *found = its index (lane * N + j,
 // else -1) and the returned value is the running sum AT that term.  Terms past the end must be 0.  All 64 lanes call.
-template <int N, bool kSearch>
+//
+// What bounds it is the chain of binades that the sum goes through.  An approximate prefix sum tells every lane the binade
+// its run will start in, so one pass gives all lanes their increments, each in its own binade, and one scan sums them up;
+// a stretch of lanes in the binade that the exact sum is in then costs two lane reads and an integer addition, and only the lane
+// that ends it -- its run crosses into the next binade, depends on the parity, or was predicted wrong -- is added term by
+// term.  (All lanes in the binade of the sum, and the rest again behind every crossing: 0.4 us for each of a dozen, where a
+// crossing takes 0.1 us now.)  Behind the fourth prediction that missed -- small terms that are rounded away beside a sum just short of
+// a power of two -- the rest takes the sum's own binade, which holds up to the next crossing.
+template <int N, bool kSearch, bool kGrown = false>
 __device__ __forceinline__ float sr_seq_wave(const float (&x)[N], float s, float target, int* found)
 {
+    constexpr int kMisses = 4;
     const int lane = sr_lane();
-    int lstart = 0;  // lanes below are settled
-    *found = -1;
-    for (;;) {
-        uint32_t n_w;
-        int eb_w;
-        sr_split(s, &n_w, &eb_w);
-        SrInc m;
-        m.a0 = 0u; m.a1 = 0u;
-        if (lane >= lstart) m = sr_run_inc(x, eb_w);
-        const SrInc sc = sr_scan_inc<false>(m);
-        SrInc ex;
-        ex.a0 = __shfl_up(sc.a0, 1);
-        ex.a1 = __shfl_up(sc.a1, 1);
-        if (lane == 0) { ex.a0 = 0u; ex.a1 = 0u; }
-        const bool odd = (n_w & 1u) != 0u;
-        // exact integer state before / after this lane's run, valid while below 2^24
-        const uint32_t before = sr_sat_add(n_w, odd ? ex.a1 : ex.a0);
-        const uint32_t after = sr_sat_add(n_w, odd ? sc.a1 : sc.a0);
-        bool ev = after >= (1u << 24);
-        if (kSearch) ev = ev || sr_join(after, eb_w) >= target;
-        const unsigned long long evl = __ballot(ev && lane >= lstart);
-        if (!evl) {  // the rest of the wave stays in the binade and below the target
-            const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)(odd ? sc.a1 : sc.a0), SR_WAVE - 1);
-            return sr_join(n_w + tot, eb_w);
-        }
-        const int fl = (int)__ffsll((long long)evl) - 1;
-        // the first such lane's run, replayed with real float adds from its exact input (every lane replays its own)
-        float acc = sr_join(before, eb_w), hit = 0.0f;
-        int wj = -1;
+    uint32_t sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(s));  // the running sum's bits, the same in every lane
+    uint32_t nn;
+    int eb_mine;
+    if (kGrown) {
+        sr_split(sr_u2f(sb), &nn, &eb_mine);
+    } else {
+        float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int j = 0; j < N; j++) {
-            acc = __fadd_rn(acc, x[j]);
-            if (kSearch && wj < 0 && acc >= target) { wj = j; hit = acc; }
+        for (int j = 0; j < N; j++) part[j & 3] += x[j];
+        const float own = (part[0] + part[1]) + (part[2] + part[3]);
+        sr_split(sr_u2f(sb) + (sr_wave_incl_sum_f32(own) - own), &nn, &eb_mine);
+    }
+    *found = -1;
+    int pos = 0, misses = 0;  // the lanes below pos are settled
+    for (;;) {
+        const SrInc m = sr_run_inc(x, eb_mine);
+        const bool simple = m.a0 == m.a1 && m.a0 < (1u << 24);
+        const unsigned long long simples = __ballot(simple);
+        if (kGrown && !kSearch && pos == 0 && simples == ~0ull) {
+            uint32_t n;
+            int eb;
+            sr_split(sr_u2f(sb), &n, &eb);
+            n += (uint32_t)sr_wave_sum_i32((int)m.a0);
+            if (n < (1u << 24)) return sr_join(n, eb);
         }
-        wj = __builtin_amdgcn_readlane(wj, fl);
-        if (kSearch && wj >= 0) {
-            *found = fl * N + wj;
-            return sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(hit), fl));
+        const uint32_t T = (uint32_t)sr_wave_incl_scan_i32(simple ? (int)m.a0 : 0);
+        for (;;) {
+            uint32_t n;
+            int eb;
+            sr_split(sr_u2f(sb), &n, &eb);
+            const unsigned long long here = __ballot(eb_mine == eb);
+            const unsigned long long stop = ~(simples & here) & (~0ull << pos);
+            int end = stop ? (int)__ffsll((long long)stop) - 1 : SR_WAVE;
+            if (end > pos) {
+                const uint32_t t0 = pos > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)T, pos - 1) : 0u;
+                const uint32_t mine = n + (T - t0);  // the exact sum behind this lane's run, for the lanes of the stretch
+                bool ev = mine >= (1u << 24);
+                if (kSearch) ev = ev || sr_join(mine, eb) >= target;
+                const unsigned long long over = __ballot(ev && lane >= pos && lane < end);
+                if (over) end = (int)__ffsll((long long)over) - 1;
+                if (end > pos) sb = sr_f2u(sr_join(n + (uint32_t)__builtin_amdgcn_readlane((int)T, end - 1) - t0, eb));
+            }
+            if (end >= SR_WAVE) return sr_u2f(sb);
+            // the lane that ends the stretch, with real float adds from the exact sum (every lane replays its own run)
+            float acc = sr_u2f(sb);
+#pragma unroll
+            for (int j = 0; j < N; j++) acc = __fadd_rn(acc, x[j]);
+            const uint32_t behind = (uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(acc), end);
+            if (kSearch && sr_u2f(behind) >= target) {
+                float hit = 0.0f;
+                int wj = -1;
+                acc = sr_u2f(sb);
+#pragma unroll
+                for (int j = 0; j < N; j++) {
+                    acc = __fadd_rn(acc, x[j]);
+                    if (wj < 0 && acc >= target) { wj = j; hit = acc; }
+                }
+                *found = end * N + __builtin_amdgcn_readlane(wj, end);
+                return sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(hit), end));
+            }
+            sb = behind;
+            pos = end + 1;
+            if (pos >= SR_WAVE) return sr_u2f(sb);
+            if (kGrown) {
+                int eb_behind;
+                sr_split(sr_u2f(sb), &nn, &eb_behind);
+                if (eb_behind != eb) break;
+            } else if (((here >> end) & 1ull) == 0ull && ++misses >= kMisses) {
+                break;
+            }
         }
-        s = sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(acc), fl));
-        lstart = fl + 1;
-        if (lstart >= SR_WAVE) return s;
+        sr_split(sr_u2f(sb), &nn, &eb_mine);
     }
 }
 

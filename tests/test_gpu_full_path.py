@@ -118,6 +118,37 @@ def test_sums_prepared_by_the_whole_device_do_not_depend_on_the_predictions(ctx)
                             assert gs[1].tobytes() == at.tobytes(), (len(x), skew, frac, gs[1], at)
 
 
+@pytest.mark.parametrize("kind", ["just below a power of two", "a binade with every term", "half way", "sparse", "below the normal range", "ordinary"])
+@pytest.mark.parametrize("n", [1, 16, 17, 1023, 1024, 1500])
+def test_one_waves_running_sum_where_predicted_binades_miss(ctx, kind, n):
+    """The lanes of a wave take the binade that an approximate prefix sum names: terms that are rounded away beside a sum just
+    short of a power of two make that wrong for every lane, terms that double the sum make every lane cross binades, and terms of
+    half an ulp make every increment depend on the parity."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    x = {"just below a power of two": lambda: np.concatenate([[1.0 - 2.0 ** -24], np.full(n, 2.0 ** -26)])[:n],
+         "a binade with every term": lambda: 2.0 ** (np.arange(n) % 120 - 60.0),
+         "half way": lambda: np.concatenate([[1.0 + 2.0 ** -23], np.tile([2.0 ** -24, 3 * 2.0 ** -24], n)])[:n],
+         "sparse": lambda: np.where(rng.random(n) < 0.01, rng.random(n), 0.0),
+         "below the normal range": lambda: rng.random(n) * 1e-41,
+         "ordinary": lambda: np.exp(rng.normal(0.0, 2.5, n) - 9.0)}[kind]().astype(np.float32)
+    buf = _cuda(x)
+    s = torch.zeros(2, dtype=torch.float32, device="cuda")
+    idx = torch.zeros(2, dtype=torch.int32, device="cuda")
+    want, _ = orc.seq_sum(x)
+    for skew in (1.0, 0.0):
+        for frac in (float("nan"), 0.0, 0.3, 0.9999, 1.5):
+            tgt = np.float32(frac * float(want)) if frac == frac else np.float32("nan")
+            ctx._check(hooks_lib().sr_selftest_segsum(ctx.h, C.c_void_p(buf.data_ptr()), n, skew, float(tgt), C.c_void_p(s.data_ptr()),
+                                                      C.c_void_p(idx.data_ptr())))
+            ctx.synchronize()
+            gs, gi = s.cpu().numpy(), idx.cpu().numpy()
+            assert gs[0].tobytes() == want.tobytes(), (skew, frac, gs[0], want)
+            if frac == frac:
+                assert gi[0] == gi[1] == orc.seq_sum(x, 0.0, float(tgt))[1], (skew, frac, gi)
+
+
 def _check_rows(ctx, logits, params, uniforms, allow_mask=None, mask_active=None):
     got, flags = ctx.sample_batch(_cuda(logits), params, uniforms, allow_mask, mask_active, return_flags=True)
     want = oracle_tokens(logits, params, uniforms, allow_mask, mask_active)
