@@ -353,10 +353,22 @@ static_assert(SR_SEG_TERMS == SR_WAVE * SR_SEQ_RUN && sizeof(SeqSegFunc) == 96, 
 struct SegRec {
     uint4 f, g, x0, x1, x2, x3;
 };
+// (kAgent: the records were written by other workgroups of the same launch)
+template <bool kAgent>
 __device__ __forceinline__ void seg_load_rec(const SeqSegFunc* funcs, int seg, int nseg, SegRec& r)
 {
-    const uint4* q = (const uint4*)(funcs + min(seg, nseg - 1));
-    r.f = q[0]; r.g = q[1]; r.x0 = q[2]; r.x1 = q[3]; r.x2 = q[4]; r.x3 = q[5];
+    const SeqSegFunc* f = funcs + min(seg, nseg - 1);
+    if (kAgent) {
+        const unsigned long long* q = (const unsigned long long*)f;
+        unsigned long long v[12];
+#pragma unroll
+        for (int i = 0; i < 12; i++) v[i] = sr_load_agent(q + i);
+        auto word = [&](int i) -> uint4 { return make_uint4((uint32_t)v[2 * i], (uint32_t)(v[2 * i] >> 32), (uint32_t)v[2 * i + 1], (uint32_t)(v[2 * i + 1] >> 32)); };
+        r.f = word(0); r.g = word(1); r.x0 = word(2); r.x1 = word(3); r.x2 = word(4); r.x3 = word(5);
+    } else {
+        const uint4* q = (const uint4*)f;
+        r.f = q[0]; r.g = q[1]; r.x0 = q[2]; r.x1 = q[3]; r.x2 = q[4]; r.x3 = q[5];
+    }
     if (seg >= nseg) r.f.w = SR_SEG_ZERO;
 }
 
@@ -366,12 +378,14 @@ __device__ __forceinline__ void seg_load_rec(const SeqSegFunc* funcs, int seg, i
 // load(segment, x) gives the lane's 16 terms of a segment, wherever the terms come from.
 //
 // 64 segments at a time, a lane each, the next 64 loading meanwhile.  The segments that are one function with the same
-// increment for both parities -- nearly all -- are summed up once (inclusive sums T over the lanes); from then on a run of
-// them that was made for the binade the sum is in costs two lane reads and an integer addition, and only the segment that ends
-// the run is looked at by itself: one in which the sum changes binade, one with an increment per parity, one whose
-// prediction missed.  (A scan of the 64 functions after every such segment -- fifteen or so in a row whose sum starts at zero --
-// was most of the 8 us that a walk over 149 segments took.)
-template <bool kSearch, typename Load>
+// increment for both parities -- nearly all -- are summed up once (inclusive sums T over the lanes).  The others are known
+// beforehand and taken one by one: the exact sum in front of one is a lane read and an addition, its record gives the sum
+// behind it; a record that does not fit that sum leaves the segment to be added from its terms.  Only then is it looked at
+// whether every segment lay in the binade its record was made for; the first that did not is added from its terms, and what
+// follows is done again.  A segment taken by itself costs some 50 instructions of the one wave, 0.1 us, a sum that
+// starts at zero has about a dozen; looking for the end of every run of segments as it went, the walk took 0.45 us for each:
+// 98 segments of a row of 100,003 entries 5.3 us, and a search over as many 7.5.
+template <bool kSearch, bool kAgent = false, typename Load>
 __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSegFunc* funcs, float s0, float target, int* found,
                                                float* states)
 {
@@ -379,85 +393,104 @@ __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSeg
     uint32_t sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(s0));  // the running sum's bits, the same in every lane
     *found = -1;
     SegRec next;
-    seg_load_rec(funcs, lane, nseg, next);
+    seg_load_rec<kAgent>(funcs, lane, nseg, next);
     for (int base = 0; base < nseg; base += SR_WAVE) {
         const SegRec r = next;
-        seg_load_rec(funcs, base + SR_WAVE + lane, nseg, next);  // (the records of the next 64 segments come in meanwhile)
-        const int cnt = min(SR_WAVE, nseg - base);
+        if (base + SR_WAVE < nseg) seg_load_rec<kAgent>(funcs, base + SR_WAVE + lane, nseg, next);  // (the next 64 segments' come in meanwhile)
         const uint32_t kind = r.f.w & 0xffu;
-        const bool zero = kind == SR_SEG_ZERO, simple = kind == SR_SEG_PLAIN && r.f.x == r.f.y && r.f.x < (1u << 24);
-        const unsigned long long zeros = __ballot(zero), simples = __ballot(simple);
+        const bool simple = kind == SR_SEG_PLAIN && r.f.x == r.f.y && r.f.x < (1u << 24), split = kind == SR_SEG_SPLIT;
+        const unsigned long long stops = ~__ballot(simple || kind == SR_SEG_ZERO);
         const uint32_t T = (uint32_t)sr_wave_incl_scan_i32(simple ? (int)r.f.x : 0);
-        int pos = 0;  // the segments below are settled
-        for (;;) {
-            uint32_t n;
-            int eb;
-            sr_split(sr_u2f(sb), &n, &eb);
-            // the run of segments from pos on that the binade's integer additions take
-            const unsigned long long take = zeros | (simples & __ballot((int)r.f.z == eb));
-            const unsigned long long stop = ~take & (~0ull << pos);
-            int end = stop ? (int)__ffsll((long long)stop) - 1 : SR_WAVE;
-            end = min(end, cnt);
-            const uint32_t t0 = pos > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)T, pos - 1) : 0u;
-            if (end > pos) {
-                const uint32_t mine = n + (T - t0);  // (the running sum behind this lane's segment, for the lanes of the run)
-                bool ev = mine >= (1u << 24);
-                if (kSearch) ev = ev || sr_join(mine, eb) >= target;
-                // (a run may leave its binade, or reach the target, on its way: up to there)
-                const unsigned long long over = __ballot(ev && lane >= pos && lane < end);
-                if (over) end = (int)__ffsll((long long)over) - 1;
-                if (!kSearch && states && lane >= pos && lane < end) states[base + lane] = sr_join(mine, eb);
-                if (end > pos) {
-                    n += (uint32_t)__builtin_amdgcn_readlane((int)T, end - 1) - t0;
-                    sb = sr_f2u(sr_join(n, eb));
-                }
-            }
-            if (end >= cnt) break;
-            // The segment that ends the run, from the exact sum in front of it.  Every step is checked, and a record that does
-            // not fit that sum (or a search that would end inside the segment) leaves the segment to be added from its terms.
-            float s_try = 0.0f;
-            bool ok = false;
-            if (lane == end) {
-                if (kind == SR_SEG_EXACT) {
-                    s_try = sr_u2f(r.g.w);
-                    ok = sb == 0u;
-                } else if (kind != SR_SEG_ZERO && (int)r.f.z == eb) {
-                    const uint32_t n1 = sr_sat_add(n, (n & 1u) ? r.f.y : r.f.x);
-                    float acc = sr_join(n1, eb);
-                    ok = n1 < (1u << 24);
-                    s_try = acc;
-                    if (kind == SR_SEG_SPLIT) {
-                        const uint32_t xs[16] = {r.x0.x, r.x0.y, r.x0.z, r.x0.w, r.x1.x, r.x1.y, r.x1.z, r.x1.w,
-                                                 r.x2.x, r.x2.y, r.x2.z, r.x2.w, r.x3.x, r.x3.y, r.x3.z, r.x3.w};
+        uint32_t eb = sr_state_eb(sb), off = sr_state_n(sb, eb);
+        uint32_t pre = off, ebv = eb;  // behind a lane's segment the sum is pre + T in the binade ebv
+        // One form for both kinds of records, no branch per segment: a plain one has sixteen zeros for the terms of its crossing and a
+        // second function that adds nothing.  [lo2, lo2 + size2): the bits of the second function's binade.
+        const uint32_t eb1 = kind == SR_SEG_PLAIN || split ? (uint32_t)r.f.z : 0xffffu, odd1 = r.f.y - r.f.x;
+        const uint32_t inc2 = split ? r.g.x : 0u, odd2 = split ? r.g.y - r.g.x : 0u, eb2 = split ? (uint32_t)r.g.z : eb1;
+        const uint32_t lo2 = eb2 > 1u ? eb2 << 23 : 0u, size2 = eb2 > 1u ? 1u << 23 : 1u << 24;
+        const uint32_t words[16] = {r.x0.x, r.x0.y, r.x0.z, r.x0.w, r.x1.x, r.x1.y, r.x1.z, r.x1.w,
+                                    r.x2.x, r.x2.y, r.x2.z, r.x2.w, r.x3.x, r.x3.y, r.x3.z, r.x3.w};
+        float xs[16];
 #pragma unroll
-                        for (int j = 0; j < 16; j++) acc = __fadd_rn(acc, sr_u2f(xs[j]));
-                        uint32_t n2;
-                        int eb2;
-                        sr_split(acc, &n2, &eb2);
-                        const uint32_t n3 = sr_sat_add(n2, (n2 & 1u) ? r.g.y : r.g.x);
-                        ok = ok && eb2 == (int)r.g.z && n3 < (1u << 24);
-                        s_try = sr_join(n3, eb2);
-                    }
+        for (int j = 0; j < 16; j++) xs[j] = split ? sr_u2f(words[j]) : 0.0f;
+        auto terms = [&](int t, uint32_t before) __attribute__((always_inline)) -> uint32_t {
+            float x[SR_SEQ_RUN];
+            load(base + t, x);
+            int at;
+            return (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(sr_seq_wave<SR_SEQ_RUN, false>(x, sr_u2f(before), 0.0f, &at)));
+        };
+        unsigned long long todo = stops;
+        int pos = 0;     // the segments below were where they were planned
+        int again = -1;  // a segment to be added from its terms, everything in front of which is exact
+        if (sb == 0u) {
+            // the first segment that has a term, where its record carries the sum behind it
+            const unsigned long long exacts = __ballot(kind == SR_SEG_EXACT);
+            if (exacts != 0ull && (stops & (0ull - stops)) == (exacts & (0ull - exacts))) {
+                const int t = (int)__ffsll((long long)stops) - 1;
+                const uint32_t Tt = (uint32_t)__builtin_amdgcn_readlane((int)T, t);
+                if (Tt == 0u) {
+                    const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)r.g.w, t);
+                    eb = sr_state_eb(to);
+                    off = sr_state_n(to, eb);
+                    if (lane >= t) { pre = off; ebv = eb; }
+                    todo &= todo - 1ull;
                 }
-                if (kSearch && s_try >= target) ok = false;  // the answer lies inside: from the terms
             }
-            if (__builtin_amdgcn_readlane((int)ok, end) != 0) {
-                sb = (uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(s_try), end);
-            } else {
-                float x[SR_SEQ_RUN];
-                load(base + end, x);
-                int at;
-                const float s = sr_seq_wave<SR_SEQ_RUN, kSearch>(x, sr_u2f(sb), target, &at);
-                if (kSearch && at >= 0) {
-                    *found = (base + end) * SR_SEG_TERMS + at;
-                    return s;
-                }
-                sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(s));
-            }
-            if (!kSearch && states && lane == 0) states[base + end] = sr_u2f(sb);
-            pos = end + 1;
-            if (pos >= cnt) break;
         }
+        for (;;) {
+            while (todo != 0ull || again >= 0) {
+                const int t = again >= 0 ? again : (int)__ffsll((long long)todo) - 1;
+                const uint32_t Tt = (uint32_t)__builtin_amdgcn_readlane((int)T, t);
+                uint32_t to, before;
+                bool fits = false;
+                if (again >= 0) {
+                    before = t > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)sr_state_bits(pre + T, ebv), t - 1) : sb;
+                    to = 0u;
+                    again = -1;
+                } else {
+                    todo &= todo - 1ull;
+                    const uint32_t n = off + Tt;
+                    if (n >= (1u << 24)) break;  // (a segment in front of this one left its binade unforeseen)
+                    before = sr_state_bits(n, eb);
+                    const uint32_t b1 = before + (r.f.x + (odd1 & (0u - (n & 1u))));
+                    float acc = sr_u2f(b1);
+#pragma unroll
+                    for (int j = 0; j < 16; j++) acc = __fadd_rn(acc, xs[j]);
+                    const uint32_t b2 = sr_f2u(acc), b3 = b2 + (inc2 + (odd2 & (0u - (b2 & 1u))));
+                    // (one comparison each: the record is for the binade the sum is in, the first function ends in it, the second one
+                    // starts and ends in its own)
+                    const unsigned long long ok = __ballot(eb1 == eb) & __ballot(b1 < sr_state_bits(1u << 24, eb)) & __ballot(b2 >= lo2) & __ballot(b3 - lo2 < size2);
+                    fits = ((ok >> t) & 1ull) != 0ull;
+                    to = (uint32_t)__builtin_amdgcn_readlane((int)b3, t);
+                }
+                if (!fits) to = terms(t, before);
+                eb = sr_state_eb(to);
+                off = sr_state_n(to, eb) - Tt;
+                if (lane >= t) { pre = off; ebv = eb; }
+            }
+            const unsigned long long bad = __ballot(simple && lane >= pos && (eb1 != ebv || pre + T >= (1u << 24)));
+            if (bad == 0ull) break;
+            // (everything in front of this segment is exact)
+            again = (int)__ffsll((long long)bad) - 1;
+            pos = again + 1;
+            todo = pos < SR_WAVE ? stops & (~0ull << pos) : 0ull;
+        }
+        const uint32_t ends = sr_state_bits(pre + T, ebv);
+        if (!kSearch && states && base + lane < nseg) states[base + lane] = sr_u2f(ends);
+        if (kSearch) {
+            const unsigned long long reach = __ballot(sr_u2f(ends) >= target && base + lane < nseg);
+            if (reach != 0ull) {
+                const int t = (int)__ffsll((long long)reach) - 1;
+                const uint32_t before = t > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)ends, t - 1) : sb;
+                float x[SR_SEQ_RUN];
+                load(base + t, x);
+                int at;
+                const float s = sr_seq_wave<SR_SEQ_RUN, true>(x, sr_u2f(before), target, &at);
+                *found = (base + t) * SR_SEG_TERMS + at;
+                return s;
+            }
+        }
+        sb = (uint32_t)__builtin_amdgcn_readlane((int)ends, SR_WAVE - 1);
     }
     return sr_u2f(sb);
 }
@@ -478,17 +511,23 @@ __device__ __forceinline__ float seg_walk(const float* terms, int n, const SeqSe
 // the approximate sum `before` of everything in front of the segment.  One wave.
 // With `seg_sum` (>= 0: the approximate sum of the segment's own terms, known beforehand) a segment whose start and
 // end lie well inside one binade gets its one function without a look at where inside it the sum would change binade.
+// (kAgent: the record will be read by other workgroups of the same launch)
+template <bool kAgent = false>
 __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], int seg, double before, SeqSegFunc* out,
                                                 float seg_sum = -1.0f)
 {
     const int lane = sr_lane();
+    auto put = [&](int i, uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3) {
+        if (kAgent) sr_store_agent_f4((float4*)out + i, sr_u2f(v0), sr_u2f(v1), sr_u2f(v2), sr_u2f(v3));
+        else ((uint4*)out)[i] = make_uint4(v0, v1, v2, v3);
+    };
     {
         // a segment without a term (masked, or cut) changes no sum whatever its binade
         float any = x[0];
 #pragma unroll
         for (int j = 1; j < SR_SEQ_RUN; j++) any = sr_max_f32(any, x[j]);
         if (__ballot(any > 0.0f) == 0ull) {
-            if (lane == 0) ((uint4*)out)[0] = make_uint4(0u, 0u, 0u, SR_SEG_ZERO);
+            if (lane == 0) put(0, 0u, 0u, 0u, SR_SEG_ZERO);
             return;
         }
     }
@@ -502,9 +541,8 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
         if (eb_lo == eb_hi) {  // (wave-uniform: both are the same in every lane)
             const SrInc sc = sr_scan_inc<false>(sr_run_inc(x, eb_lo));
             if (lane == SR_WAVE - 1) {
-                uint4* q = (uint4*)out;
-                q[0] = make_uint4(sc.a0, sc.a1, (uint32_t)eb_lo, SR_SEG_PLAIN);
-                q[1] = make_uint4(SR_SEQ_SAT, SR_SEQ_SAT, (uint32_t)eb_lo, 0u);
+                put(0, sc.a0, sc.a1, (uint32_t)eb_lo, SR_SEG_PLAIN);
+                put(1, SR_SEQ_SAT, SR_SEQ_SAT, (uint32_t)eb_lo, 0u);
             }
             return;
         }
@@ -557,13 +595,12 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
         }
     }
     if (lane == 0) {
-        uint4* q = (uint4*)out;
-        q[0] = make_uint4(f.a0, f.a1, (uint32_t)f.eb, f.kind);
-        q[1] = make_uint4(f.b0, f.b1, (uint32_t)f.eb2, f.end_bits);
+        put(0, f.a0, f.a1, (uint32_t)f.eb, f.kind);
+        put(1, f.b0, f.b1, (uint32_t)f.eb2, f.end_bits);
     }
     if (lane == cross) {
 #pragma unroll
-        for (int j = 0; j < 16; j++) out->x[j] = x[j];
+        for (int j = 0; j < 16; j += 4) put(2 + j / 4, sr_f2u(x[j]), sr_f2u(x[j + 1]), sr_f2u(x[j + 2]), sr_f2u(x[j + 3]));
     }
 }
 
@@ -652,7 +689,7 @@ __device__ __forceinline__ float tp_sum(Term term, int n, FullSmem& sm)
 // The same sum over a long row in memory (times mul when do_mul), one wave per lane accumulator.  The row comes in
 // through LDS 8,192 entries at a time -- every thread brings two 16-byte pieces, two rounds ahead of the round that is
 // added --, laid out chain by chain, and the wave of a chain adds its 1,024 terms of the round with the wave's own
-// exact scan (sr_seq_wave): no block-wide step but one barrier per round, so a round costs what its 32 KB take to
+// exact scan (sr_seq_wave_grown): no block-wide step but one barrier per round, so a round costs what its 32 KB take to
 // arrive.  The place of term v = 16 l + j of chain g is g * 1024 + 64 j + (l + 2 j) mod 64: the 64 lanes of a wave
 // read a term from 64 consecutive places, and the stores of a piece's four entries fall two to a bank.
 __device__ __forceinline__ float tp_sum_row(const float* p, int n, float mul, bool do_mul, FullSmem& sm)
@@ -706,7 +743,7 @@ __device__ __forceinline__ float tp_sum_row(const float* p, int n, float mul, bo
 #pragma unroll
             for (int j = 0; j < 16; j++) x[j] = b[64 * j + ((lane + 2 * j) & 63)];
             int dummy;
-            sc = sr_seq_wave<16, false, true>(x, sc, 0.0f, &dummy);
+            sc = sr_seq_wave_grown<16, false>(x, sc, 0.0f, &dummy);
         }
     };
     // (behind the last round the loop fetches that round again, to no effect: the compiler can wait for "all but the

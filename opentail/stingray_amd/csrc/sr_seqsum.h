@@ -290,95 +290,165 @@ __device__ __forceinline__ void sr_seq_tile(const float (&x)[SR_SEQ_RUN], float*
 }
 
 // ---- one wave by itself --------------------------------------------------------------------------------
+// the sum's state by its bits (uniform): the integer n and the binade's exponent field, as sr_split and sr_join have them
+__device__ __forceinline__ uint32_t sr_state_eb(uint32_t bits) { return max(bits >> 23, 1u); }
+__device__ __forceinline__ uint32_t sr_state_n(uint32_t bits, uint32_t eb) { return bits - ((eb - 1u) << 23); }
+__device__ __forceinline__ uint32_t sr_state_bits(uint32_t n, uint32_t eb) { return n + ((eb - 1u) << 23); }
+
 // The running sum s of the wave's 64 x N terms (lane order = term order, N consecutive terms per lane), with no barrier
 // and no shared memory: what a short list (a row tail's few hundred probabilities), or one segment of a long sum, needs.
 // When kSearch, stops at the first term at which the running sum reaches `target`: *found = its index (lane * N + j,
 // else -1) and the returned value is the running sum AT that term.  Terms past the end must be 0.  All 64 lanes call.
 //
-// What bounds it is the chain of binades that the sum goes through.  An approximate prefix sum tells every lane the binade
-// its run will start in, so one pass gives all lanes their increments, each in its own binade, and one scan sums them up;
-// a stretch of lanes in the binade that the exact sum is in then costs two lane reads and an integer addition, and only the lane
-// that ends it -- its run crosses into the next binade, depends on the parity, or was predicted wrong -- is added term by
-// term.  (All lanes in the binade of the sum, and the rest again behind every crossing: 0.4 us for each of a dozen, where a
-// crossing takes 0.1 us now.)  Behind the fourth prediction that missed -- small terms that are rounded away beside a sum just short of
-// a power of two -- the rest takes the sum's own binade, which holds up to the next crossing.
-template <int N, bool kSearch, bool kGrown = false>
+// What bounds it is the chain of binades that the sum goes through, instruction by instruction of one wave (5 clocks each).
+// An approximate prefix sum tells every lane the binade its run starts in and whether it leaves it, so one pass gives the lanes
+// that stay their increments, each in its own binade, and one scan sums them up.  The others -- and those whose increment
+// depends on the parity -- are known beforehand and taken one by one: the exact sum in front of one is a lane read and an
+// addition, its run is added term by term.  Only then is it looked at whether every lane was in the binade it was planned
+// for; the first that was not is added term by term from the exact sum in front of it, and what follows is done again.  Behind the
+// fourth of those -- small terms that are rounded away beside a sum just short of a power of two -- the rest is planned in
+// the sum's own binade, which holds up to the next crossing.  (The rest scanned again behind every crossing, with all lanes in the
+// binade of the sum: 0.3 - 0.4 us for each of a dozen; 0.07 now.)
+template <int N, bool kSearch>
 __device__ __forceinline__ float sr_seq_wave(const float (&x)[N], float s, float target, int* found)
 {
     constexpr int kMisses = 4;
     const int lane = sr_lane();
-    uint32_t sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(s));  // the running sum's bits, the same in every lane
-    uint32_t nn;
-    int eb_mine;
-    if (kGrown) {
-        sr_split(sr_u2f(sb), &nn, &eb_mine);
-    } else {
+    const uint32_t s0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(s));  // the sum's bits, the same in every lane
+    uint32_t eb = sr_state_eb(s0), n = sr_state_n(s0, eb);
+    uint32_t eb_mine = eb;  // the binade this lane's run is planned in ...
+    bool cross = false;     // ... and expected to leave
+    {
         float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int j = 0; j < N; j++) part[j & 3] += x[j];
         const float own = (part[0] + part[1]) + (part[2] + part[3]);
-        sr_split(sr_u2f(sb) + (sr_wave_incl_sum_f32(own) - own), &nn, &eb_mine);
+        const float incl = sr_wave_incl_sum_f32(own);
+        eb_mine = sr_state_eb(sr_f2u(sr_u2f(s0) + (incl - own)));
+        cross = sr_state_eb(sr_f2u(sr_u2f(s0) + incl)) != eb_mine;
     }
     *found = -1;
-    int pos = 0, misses = 0;  // the lanes below pos are settled
+    uint32_t ends = 0u;  // the sum's bits behind this lane's run
+    int from = 0, misses = 0;
     for (;;) {
-        const SrInc m = sr_run_inc(x, eb_mine);
-        const bool simple = m.a0 == m.a1 && m.a0 < (1u << 24);
-        const unsigned long long simples = __ballot(simple);
-        if (kGrown && !kSearch && pos == 0 && simples == ~0ull) {
-            uint32_t n;
-            int eb;
-            sr_split(sr_u2f(sb), &n, &eb);
-            n += (uint32_t)sr_wave_sum_i32((int)m.a0);
-            if (n < (1u << 24)) return sr_join(n, eb);
-        }
+        // the lanes [from, 64) are planned, and n, eb is the exact sum in front of them
+        const SrInc m = sr_run_inc(x, (int)eb_mine);
+        const bool simple = !cross && m.a0 == m.a1 && m.a0 < (1u << 24);
+        const unsigned long long stops = ~__ballot(simple);
         const uint32_t T = (uint32_t)sr_wave_incl_scan_i32(simple ? (int)m.a0 : 0);
+        uint32_t off = n - (from > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)T, from - 1) : 0u);
+        uint32_t pre = off, ebv = eb;  // behind a lane's run the sum is pre + T in the binade ebv
+        unsigned long long todo = stops & (~0ull << from);
+        int pos = from;                // the lanes below were where they were planned
+        bool again = false;
         for (;;) {
-            uint32_t n;
-            int eb;
-            sr_split(sr_u2f(sb), &n, &eb);
-            const unsigned long long here = __ballot(eb_mine == eb);
-            const unsigned long long stop = ~(simples & here) & (~0ull << pos);
-            int end = stop ? (int)__ffsll((long long)stop) - 1 : SR_WAVE;
-            if (end > pos) {
-                const uint32_t t0 = pos > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)T, pos - 1) : 0u;
-                const uint32_t mine = n + (T - t0);  // the exact sum behind this lane's run, for the lanes of the stretch
-                bool ev = mine >= (1u << 24);
-                if (kSearch) ev = ev || sr_join(mine, eb) >= target;
-                const unsigned long long over = __ballot(ev && lane >= pos && lane < end);
-                if (over) end = (int)__ffsll((long long)over) - 1;
-                if (end > pos) sb = sr_f2u(sr_join(n + (uint32_t)__builtin_amdgcn_readlane((int)T, end - 1) - t0, eb));
+            while (todo != 0ull) {
+                const int t = (int)__ffsll((long long)todo) - 1;
+                todo &= todo - 1ull;
+                const uint32_t Tt = (uint32_t)__builtin_amdgcn_readlane((int)T, t);
+                if (off + Tt >= (1u << 24)) break;  // (a lane in front of this one left its binade unforeseen)
+                float acc = sr_u2f(sr_state_bits(off + Tt, eb));
+#pragma unroll
+                for (int j = 0; j < N; j++) acc = __fadd_rn(acc, x[j]);
+                const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(acc), t);
+                eb = sr_state_eb(to);
+                off = sr_state_n(to, eb) - Tt;
+                if (lane >= t) { pre = off; ebv = eb; }
             }
-            if (end >= SR_WAVE) return sr_u2f(sb);
-            // the lane that ends the stretch, with real float adds from the exact sum (every lane replays its own run)
-            float acc = sr_u2f(sb);
+            const unsigned long long bad = __ballot(simple && lane >= pos && (eb_mine != ebv || pre + T >= (1u << 24)));
+            ends = lane >= from ? sr_state_bits(pre + T, ebv) : ends;
+            if (bad == 0ull) break;
+            const int f = (int)__ffsll((long long)bad) - 1;
+            float acc = sr_u2f(f > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)ends, f - 1) : s0);
 #pragma unroll
             for (int j = 0; j < N; j++) acc = __fadd_rn(acc, x[j]);
-            const uint32_t behind = (uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(acc), end);
-            if (kSearch && sr_u2f(behind) >= target) {
-                float hit = 0.0f;
-                int wj = -1;
-                acc = sr_u2f(sb);
-#pragma unroll
-                for (int j = 0; j < N; j++) {
-                    acc = __fadd_rn(acc, x[j]);
-                    if (wj < 0 && acc >= target) { wj = j; hit = acc; }
-                }
-                *found = end * N + __builtin_amdgcn_readlane(wj, end);
-                return sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(hit), end));
-            }
-            sb = behind;
-            pos = end + 1;
-            if (pos >= SR_WAVE) return sr_u2f(sb);
-            if (kGrown) {
-                int eb_behind;
-                sr_split(sr_u2f(sb), &nn, &eb_behind);
-                if (eb_behind != eb) break;
-            } else if (((here >> end) & 1ull) == 0ull && ++misses >= kMisses) {
+            const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(acc), f);
+            eb = sr_state_eb(to);
+            n = sr_state_n(to, eb);
+            ends = lane == f ? to : ends;
+            pos = f + 1;
+            if (pos >= SR_WAVE) break;
+            if (++misses >= kMisses) {
+                again = true;
                 break;
             }
+            off = n - (uint32_t)__builtin_amdgcn_readlane((int)T, f);
+            if (lane >= f) { pre = off; ebv = eb; }
+            todo = stops & (~0ull << pos);
         }
-        sr_split(sr_u2f(sb), &nn, &eb_mine);
+        if (!again) break;
+        from = pos;
+        eb_mine = eb;
+        cross = false;
+    }
+    if (kSearch) {
+        const unsigned long long reach = __ballot(sr_u2f(ends) >= target);
+        if (reach != 0ull) {
+            const int t = (int)__ffsll((long long)reach) - 1;
+            float acc = sr_u2f(t > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)ends, t - 1) : s0), hit = 0.0f;
+            int wj = -1;
+#pragma unroll
+            for (int j = 0; j < N; j++) {
+                acc = __fadd_rn(acc, x[j]);
+                if (wj < 0 && acc >= target) { wj = j; hit = acc; }
+            }
+            *found = t * N + __builtin_amdgcn_readlane(wj, t);
+            return sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(hit), t));
+        }
+    }
+    return sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)ends, SR_WAVE - 1));
+}
+
+// ... of a sum that is no longer small and so mostly stays in its binade: all lanes take that binade, increments that depend on the
+// parity are composed by the scan, and the lanes behind a crossing are scanned again.  (The row tails of the selection kernel:
+// 40.4 us at 256 rows of 151,936 where the one above takes 40.6; the final Normalize of a long row by its own workgroup,
+// eight chains of 32 rounds: 48 us against 54.)
+template <int N, bool kSearch>
+__device__ __forceinline__ float sr_seq_wave_grown(const float (&x)[N], float s, float target, int* found)
+{
+    const int lane = sr_lane();
+    int lstart = 0;  // lanes below are settled
+    *found = -1;
+    for (;;) {
+        uint32_t n_w;
+        int eb_w;
+        sr_split(s, &n_w, &eb_w);
+        SrInc m;
+        m.a0 = 0u; m.a1 = 0u;
+        if (lane >= lstart) m = sr_run_inc(x, eb_w);
+        const SrInc sc = sr_scan_inc<false>(m);
+        SrInc ex;
+        ex.a0 = __shfl_up(sc.a0, 1);
+        ex.a1 = __shfl_up(sc.a1, 1);
+        if (lane == 0) { ex.a0 = 0u; ex.a1 = 0u; }
+        const bool odd = (n_w & 1u) != 0u;
+        // exact integer state before / after this lane's run, valid while below 2^24
+        const uint32_t before = sr_sat_add(n_w, odd ? ex.a1 : ex.a0);
+        const uint32_t after = sr_sat_add(n_w, odd ? sc.a1 : sc.a0);
+        bool ev = after >= (1u << 24);
+        if (kSearch) ev = ev || sr_join(after, eb_w) >= target;
+        const unsigned long long evl = __ballot(ev && lane >= lstart);
+        if (!evl) {  // the rest of the wave stays in the binade and below the target
+            const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)(odd ? sc.a1 : sc.a0), SR_WAVE - 1);
+            return sr_join(n_w + tot, eb_w);
+        }
+        const int fl = (int)__ffsll((long long)evl) - 1;
+        // the first such lane's run, replayed with real float adds from its exact input (every lane replays its own)
+        float acc = sr_join(before, eb_w), hit = 0.0f;
+        int wj = -1;
+#pragma unroll
+        for (int j = 0; j < N; j++) {
+            acc = __fadd_rn(acc, x[j]);
+            if (kSearch && wj < 0 && acc >= target) { wj = j; hit = acc; }
+        }
+        wj = __builtin_amdgcn_readlane(wj, fl);
+        if (kSearch && wj >= 0) {
+            *found = fl * N + wj;
+            return sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(hit), fl));
+        }
+        s = sr_u2f((uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(acc), fl));
+        lstart = fl + 1;
+        if (lstart >= SR_WAVE) return s;
     }
 }
 

@@ -1212,7 +1212,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
                 float x[kRun];
                 load_run(base, n_sum, x);
                 int unused;
-                sum = sr_seq_wave<kRun, false, true>(x, sum, 0.0f, &unused);
+                sum = sr_seq_wave_grown<kRun, false>(x, sum, 0.0f, &unused);
             }
             if (sr_lane() == 0) sm.bcast[5] = sr_f2u(sum);
         }
@@ -1292,7 +1292,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
                 float x[kRun];
                 load_run(base, limit_all, x);
                 int f;
-                cum = sr_seq_wave<kRun, true, true>(x, cum, target, &f);
+                cum = sr_seq_wave_grown<kRun, true>(x, cum, target, &f);
                 if (f >= 0) { *val = cum; return base + f; }
             }
             *val = cum;
