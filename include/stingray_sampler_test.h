@@ -45,7 +45,9 @@ SR_API int sr_debug_set_spin_limit(sr_ctx* ctx, uint32_t polls);
 /* How often a workgroup of the full-vocabulary path's pass over long rows polls its row's count (every workgroup of the
  * row leaves its segments' maxima and counts itself in) before it stops waiting, marks its segments and leaves them to
  * the last of the row's workgroups (default 2^15, tens of milliseconds).  0 makes every workgroup leave its segments;
- * 1 or 2 make some of them do so: the results must not change. */
+ * 1 or 2 make some of them do so: the results must not change.  The same limit holds for the launch that normalises and
+ * draws from rows that are left to the whole device (the row's last workgroup then does the whole row); with the highest bit
+ * set it holds for that launch alone. */
 SR_API int sr_debug_set_row_wait_limit(sr_ctx* ctx, uint32_t polls);
 
 /* Profiling builds (-DSR_PROFILE) only, SR_ERR_UNSUPPORTED otherwise: phase timestamps (wall_clock64, 100 MHz) of

@@ -1531,7 +1531,8 @@ int sr_debug_set_spin_limit(sr_ctx* ctx, uint32_t polls)
 int sr_debug_set_row_wait_limit(sr_ctx* ctx, uint32_t polls)
 {
     if (!ctx) return SR_ERR_NULL_ARGUMENT;
-    ctx->row_wait_limit = polls;
+    ctx->behind_wait_limit = polls & 0x7fffffffu;
+    if (!(polls & 0x80000000u)) ctx->row_wait_limit = polls;
     return SR_OK;
 }
 

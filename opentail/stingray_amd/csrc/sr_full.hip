@@ -2708,7 +2708,7 @@ __device__ __forceinline__ void sort_survivors_in_place(uint32_t* keys, int32_t*
 // a.sort_keys_in / a.sort_vals_in hold, per segment, the entries e >= SrFullState::list_from in the order of their indices,
 // a.seg_cnt how many.  Their values are sorted in shared memory, the min-p threshold and the exact running sum of
 // top-p name the cut, and a nucleus of up to `finish_most` members is normalised and drawn from here; a larger one, and every
-// row whose distribution is handed out, is left to the whole device (k_chain_records ... k_prepared_token): its members
+// row whose distribution is handed out, is left to the whole device (k_prepared_row): its members
 // are known by the value at the cut and, among equal ones, by the last index.
 // (One workgroup used to count the row's e into a histogram, read the row once per 8,192 entries of its nucleus to list
 // them, and once more to list the members: 113 us a launch of 16 constrained rows of 151,936, of which the listing reads
@@ -2718,16 +2718,18 @@ __device__ __forceinline__ int list_place(int i) { return i + (i >> 4); }  // (r
 
 __device__ __forceinline__ uint32_t* list_values(uint32_t* more, FullSmem& sm) { return more ? more : (uint32_t*)sm.sortbuf; }
 
-// the row's members are left to the whole device: the factors and the cut, and what k_chain_records and k_prepared_draw
-// need to know of the sums in front of their blocks
-__device__ __forceinline__ void row_deferred(const SrFullArgs& a, SrFullState* st, float inv, float ycut, int idx_last)
+// the row's members are left to the whole device: the factors and the cut, and what k_prepared_row
+// needs to know of the sums in front of its blocks
+__device__ __forceinline__ void row_deferred(const SrFullArgs& a, SrFullState* st, float inv, float ycut, int idx_last, const FullSmem& sm)
 {
     if (threadIdx.x == 0) {
         st->mul1 = inv;
         st->mul2 = 1.0f;
         st->ycut = ycut;
         st->idx_last = idx_last;
+        st->u = __double2float_rn(sm.u);  // (the uniform may lie in host memory: fetched once, by k_full_row)
         st->deferred = a.seq;
+        a.row_sync[(size_t)(st - a.state) * SR_ROW_SYNC_STRIDE + 1] = (unsigned long long)a.seq << 32;  // nobody has counted in
     }
 }
 
@@ -3007,7 +3009,7 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     // left to the whole device: the members' part of every segment and of every half block of the eight accumulators
     for (int i = tid; i < nseg; i += kT) a.seg_sum[(size_t)slot * a.seg_stride + i] = ssum[i];
     for (int i = tid; i < a.chain_stride; i += kT) a.chain_sum[(size_t)slot * a.chain_stride + i] = csum[i];
-    row_deferred(a, st, inv, ycut, (int)sm.bc[9]);
+    row_deferred(a, st, inv, ycut, (int)sm.bc[9], sm);
     return kListDeferred;
 }
 
@@ -3090,7 +3092,7 @@ __device__ __forceinline__ int cut_from_short_list(const SrFullArgs& a, const Sr
     }
     for (int i = tid; i < nseg; i += kT) a.seg_sum[(size_t)slot * a.seg_stride + i] = ssum[i];
     for (int i = tid; i < a.chain_stride; i += kT) a.chain_sum[(size_t)slot * a.chain_stride + i] = csum[i];
-    row_deferred(a, st, inv, sr_u2f(sm.bc[10]), (int)sm.bc[9]);
+    row_deferred(a, st, inv, sr_u2f(sm.bc[10]), (int)sm.bc[9], sm);
     return kListDeferred;
 }
 
@@ -3274,7 +3276,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
             const bool do_scale = sum > 0.0f && sum != 1.0f;
             const float inv = do_scale ? __fdiv_rn(1.0f, sum) : 1.0f;
             if (plain && a.prepared) {
-                row_deferred(a, st, inv, -1.0f, 0);
+                row_deferred(a, st, inv, -1.0f, 0, sm);
                 if (tid == 0) st->flags = flags;
                 return;
             }
@@ -3674,16 +3676,18 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
 }
 
 // ---- rows left to the whole device: final Normalize and draw (Sampler.cs:91-92, :553-576) --------------------------------
-// The members' probabilities y = fl(e inv) are known by the cut (all of them, in a row that nothing cuts).  Three launches
-// instead of one workgroup per row, which took 48 us to pass over 262,144 entries once and such a row passed three times:
-//   k_chain_records   the increment functions of the eight lane accumulators of TensorPrimitives.Sum, a block of 8,192
-//                     entries (1,024 terms of each) to a workgroup, a chain to a wave
-//   k_prepared_draw   every workgroup walks the eight chains (a wave each; the same work in all of them costs less than one
-//                     more launch), then its waves take a segment each: z = fl(y / sum), written where the distribution is
-//                     handed out, and the segment's record for the running sum of the draw
-//   k_prepared_token  one wave per row walks the records to the draw's target
-// Distributions and tokens of 16 rows of 262,144 with top-p or without a filter: 150 -> 81 us a call; tokens of 32 ragged bf16
-// rows of 100,003: 98 -> 70.
+// The members' probabilities y = fl(e inv) are known by the cut (all of them, in a row that nothing cuts).  One launch
+// (k_prepared_row), a workgroup per block of 8,192 entries, which it reads once:
+//   its waves, one per lane accumulator of TensorPrimitives.Sum, make the records of their 1,024 terms of the block;
+//   when the row's workgroups are all there, every one of them walks the eight accumulators (the same work in all of them
+//   costs less than a second meeting), and its waves take a segment each: z = fl(y / sum), written where the distribution is
+//   handed out, and the segment's record for the running sum of the draw;
+//   whoever comes last walks those records to the draw's target.
+// What bounds it: the serial chain (data, records, meeting, walk of the accumulators, records, walk of the draw), about a
+// third of it trips to memory.  32 ragged bf16 rows of 100,003: 23 us, 16 rows of 262,144 fp32: 33; as three launches --
+// each 4 us before its first byte, and the row read twice -- the same steps took 27 and 38.
+// The wait is bounded: a workgroup whose wait runs out marks the row (SrFullState::late_behind), counts itself in as if it had done
+// its block, and whoever comes last does all blocks of the row from the records of the accumulators, which are all there.
 struct PreparedRow {
     const float* e;
     float inv, ycut;
@@ -3691,7 +3695,7 @@ struct PreparedRow {
     __device__ __forceinline__ float cut(float ev, int i) const  // y, or 0 outside the nucleus
     {
         const float y = __fmul_rn(ev, inv);
-        return (y > ycut || (y == ycut && i <= idx_last)) ? y : 0.0f;
+        return (y > ycut) | ((y == ycut) & (i <= idx_last)) ? y : 0.0f;  // (no branch per entry)
     }
 };
 __device__ __forceinline__ PreparedRow prepared_row(const SrFullArgs& a, const SrFullState* st, int slot)
@@ -3705,112 +3709,39 @@ __device__ __forceinline__ PreparedRow prepared_row(const SrFullArgs& a, const S
     return r;
 }
 constexpr int kPrepT = 512;
-static_assert(kPrepT / SR_WAVE == SR_SEQ_CHAINS, "a wave per chain");
-__global__ __launch_bounds__(kPrepT) void k_chain_records(SrFullArgs a)
+static_assert(kPrepT / SR_WAVE == SR_SEQ_CHAINS, "a wave per chain, and one per segment");
+constexpr int kPrepBlock = SR_SEQ_CHAINS * SR_SEG_TERMS;
+// y of the wave's segment of block blk, as it is loaded: lane l the pieces l, 64 + l, ... of four entries
+__device__ __forceinline__ void prepared_load(const PreparedRow& r, int blk, int wave, int lane, float4 (&v)[4])
 {
-    __shared__ float buf[8192];
-    const int slot = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
-    const SrFullState* st = a.state + slot;
-    if (st->deferred != a.seq) return;
-    const PreparedRow r = prepared_row(a, st, slot);
-    const int body = (r.n / 8) * 8;
-    float4 v[4];
-#pragma unroll
-    for (int h = 0; h < 4; h++) {  // (the rows of e start on 16-byte boundaries)
-        const int x0 = blk * 8192 + 4 * (tid + h * kPrepT);
-        v[h] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (x0 + 4 <= body) v[h] = *(const float4*)(r.e + x0);  // (body is a multiple of 8)
-    }
-    const float* cs = a.chain_sum + (size_t)slot * a.chain_stride;
-    float before = 0.0f;
-    for (int hb = lane; hb < 2 * blk; hb += SR_WAVE) before += cs[hb * SR_SEQ_CHAINS + wave];
-    before = sr_wave_sum_f32(before) * r.inv;
-    const int hb1 = a.chain_stride / SR_SEQ_CHAINS;
-    float own = cs[2 * blk * SR_SEQ_CHAINS + wave];
-    if (2 * blk + 1 < hb1) own += cs[(2 * blk + 1) * SR_SEQ_CHAINS + wave];
-    // chain by chain in shared memory: the place of term 16 l + j of chain g is g 1024 + 64 j + (l + 2 j) mod 64, so that
-    // the lanes of a wave read a term from 64 consecutive places and a piece's stores fall two to a bank
-#pragma unroll
-    for (int h = 0; h < 4; h++) {
-        const int t2 = tid + h * kPrepT, x0 = blk * 8192 + 4 * t2;
-        const int vec = t2 >> 1, j = vec & 15, l = vec >> 4;
-        float* at = buf + (4 * (t2 & 1)) * 1024 + 64 * j + ((l + 2 * j) & 63);
-        at[0] = r.cut(v[h].x, x0); at[1024] = r.cut(v[h].y, x0 + 1); at[2048] = r.cut(v[h].z, x0 + 2); at[3072] = r.cut(v[h].w, x0 + 3);
-    }
-    __syncthreads();
-    float x[SR_SEQ_RUN];
-#pragma unroll
-    for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = buf[wave * 1024 + 64 * j + ((lane + 2 * j) & 63)];
-    seg_make_record(x, blk, (double)before, a.chain_func + ((size_t)slot * SR_SEQ_CHAINS + wave) * a.chain_blocks + blk, own * r.inv);
-}
-
-__global__ __launch_bounds__(kPrepT) void k_prepared_draw(SrFullArgs a)
-{
-    __shared__ float4 turn_all[SR_SEQ_CHAINS][SR_WAVE * 5];
-    __shared__ float lane_sum[SR_SEQ_CHAINS];
-    const int slot = blockIdx.y, lane = sr_lane(), wave = sr_wave_id();
-    SrFullState* st = a.state + slot;
-    if (st->deferred != a.seq) return;
-    const int row = a.row_list[slot];
-    const PreparedRow r = prepared_row(a, st, slot);
-    const int n = r.n, nv = n / 8, rem = n - nv * 8, nblk = (nv + SR_SEG_TERMS - 1) / SR_SEG_TERMS, nseg = seg_count(n);
-    const int seg = (int)blockIdx.x * SR_SEQ_CHAINS + wave;
-    const bool have = seg < nseg && !a.lazy_scale;
-    // the wave's segment is asked for in front of the walk
-    float4 v[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
-        const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
+        const int i0 = blk * kPrepBlock + wave * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
         v[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (have && i0 < n) {
-            if (i0 + 4 <= n) {
-                v[k] = *(const float4*)(r.e + i0);
-            } else {
-                v[k].x = r.e[i0];
-                if (i0 + 1 < n) v[k].y = r.e[i0 + 1];
-                if (i0 + 2 < n) v[k].z = r.e[i0 + 2];
-            }
+        if (i0 + 4 <= r.n) {
+            v[k] = *(const float4*)(r.e + i0);  // (the rows of e start on 16-byte boundaries)
+        } else if (i0 < r.n) {
+            v[k].x = r.e[i0];
+            if (i0 + 1 < r.n) v[k].y = r.e[i0 + 1];
+            if (i0 + 2 < r.n) v[k].z = r.e[i0 + 2];
         }
     }
-    float before = 0.0f;
-    if (have && a.mode != 1) {
-        const float* sums = a.seg_sum + (size_t)slot * a.seg_stride;
-        for (int g = lane; g < seg; g += SR_WAVE) before += sums[g];
-        before = sr_wave_sum_f32(before);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int i0 = blk * kPrepBlock + wave * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
+        v[k].x = r.cut(v[k].x, i0); v[k].y = r.cut(v[k].y, i0 + 1); v[k].z = r.cut(v[k].z, i0 + 2); v[k].w = r.cut(v[k].w, i0 + 3);
     }
-    {
-        int dummy;
-        float s = seg_walk_from<false>([&](int blk, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
-            // (no condition stands between the loads: with one each they wait for each other; a whole block by offsets from one
-            // address, 16 rows of 262,144: 21.9 -> 17.9 us a launch)
-            const int t0 = blk * SR_SEG_TERMS + lane * SR_SEQ_RUN;
-            const float* const e0 = r.e + (size_t)t0 * 8 + wave;
-            if ((blk + 1) * SR_SEG_TERMS <= nv) {
-#pragma unroll
-                for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = e0[j * 8];
-            } else {
-#pragma unroll
-                for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = r.e[min(t0 + j, nv - 1) * 8 + wave];
-            }
-#pragma unroll
-            for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = t0 + j < nv ? r.cut(x[j], (t0 + j) * 8 + wave) : 0.0f;
-        }, nblk, a.chain_func + ((size_t)slot * SR_SEQ_CHAINS + wave) * a.chain_blocks, 0.0f, 0.0f, &dummy, nullptr);
-        if (rem > 0 && wave >= 8 - rem) s = __fadd_rn(s, r.cut(r.e[n - 8 + wave], n - 8 + wave));  // the overlapped last vector
-        if (lane == 0) lane_sum[wave] = s;
-    }
-    __syncthreads();
-    const float l0 = lane_sum[0], l1 = lane_sum[1], l2 = lane_sum[2], l3 = lane_sum[3], l4 = lane_sum[4], l5 = lane_sum[5],
-                l6 = lane_sum[6], l7 = lane_sum[7];
-    const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
-    const float inv2 = (sum > 0.0f && sum != 1.0f) ? __fdiv_rn(1.0f, sum) : 1.0f;
-    if (blockIdx.x == 0 && threadIdx.x == 0) st->mul2 = inv2;
-    if (!have) return;
+}
+// z of the wave's segment: to the caller's row where the distribution is handed out, and the segment's record for the draw
+__device__ __forceinline__ void prepared_segment(const SrFullArgs& a, const PreparedRow& r, int slot, int row, int seg, int lane, float4 (&v)[4],
+                                                 float before, float inv2, float4* turn)
+{
+    const int n = r.n;
     float* const p = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
-        v[k].x = __fmul_rn(r.cut(v[k].x, i0), inv2); v[k].y = __fmul_rn(r.cut(v[k].y, i0 + 1), inv2);
-        v[k].z = __fmul_rn(r.cut(v[k].z, i0 + 2), inv2); v[k].w = __fmul_rn(r.cut(v[k].w, i0 + 3), inv2);
+        v[k].x = __fmul_rn(v[k].x, inv2); v[k].y = __fmul_rn(v[k].y, inv2); v[k].z = __fmul_rn(v[k].z, inv2); v[k].w = __fmul_rn(v[k].w, inv2);
         if (a.mode != 0) {
             if (i0 + 4 <= n) {
                 sr_store_f4(p + i0, v[k].x, v[k].y, v[k].z, v[k].w);
@@ -3822,7 +3753,8 @@ __global__ __launch_bounds__(kPrepT) void k_prepared_draw(SrFullArgs a)
         }
     }
     if (a.mode == 1) return;
-    float4* const turn = turn_all[wave];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int i = (k * SR_WAVE + lane) * 4;
@@ -3841,29 +3773,139 @@ __global__ __launch_bounds__(kPrepT) void k_prepared_draw(SrFullArgs a)
     }
     own = sr_wave_sum_f32(own);
     // (the records of the denominator have been walked: theirs take their place)
-    seg_make_record(t, seg, (double)(before * r.inv * inv2), a.seg_func + (size_t)slot * a.seg_stride + seg, own);
+    seg_make_record<true>(t, seg, (double)(before * r.inv * inv2), a.seg_func + (size_t)slot * a.seg_stride + seg, own);
 }
-
-__global__ __launch_bounds__(SR_WAVE) void k_prepared_token(SrFullArgs a)
+__global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
 {
-    const int slot = blockIdx.x, lane = sr_lane();
-    const SrFullState* st = a.state + slot;
+    __shared__ float4 room[SR_SEQ_CHAINS * SR_WAVE * 5];  // the block chain by chain, then every wave's segment on its way to 16 terms a lane
+    __shared__ float lane_sum[SR_SEQ_CHAINS];
+    __shared__ uint32_t bc;
+    const int slot = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
+    SrFullState* st = a.state + slot;
     if (st->deferred != a.seq) return;
     const int row = a.row_list[slot];
-    const float u = __double2float_rn(a.uniforms[(size_t)row * a.uniforms_per_row]);
     const PreparedRow r = prepared_row(a, st, slot);
-    const float inv2 = st->mul2;
-    const int n = r.n;
-    auto term = [&](int i) -> float { return i < n ? __fmul_rn(r.cut(r.e[i], i), inv2) : 0.0f; };
+    const int n = r.n, nv = n / 8, rem = n - nv * 8, body = nv * 8, nblk = (nv + SR_SEG_TERMS - 1) / SR_SEG_TERMS, nseg = seg_count(n);
+    unsigned long long* const sync = a.row_sync + (size_t)slot * SR_ROW_SYNC_STRIDE + 1;
+    const float* const sums = a.seg_sum + (size_t)slot * a.seg_stride;
+    SeqSegFunc* const chain = a.chain_func + ((size_t)slot * SR_SEQ_CHAINS + wave) * a.chain_blocks;
+    const int seg = blk * SR_SEQ_CHAINS + wave;
+    float4 v[4];
+    prepared_load(r, blk, wave, lane, v);
+    // about what stands in front of the block's terms of the wave's chain, and of the wave's segment
+    const float* const cs = a.chain_sum + (size_t)slot * a.chain_stride;
+    float before = 0.0f, before_seg = 0.0f, own = 0.0f;
+    const int hb1 = a.chain_stride / SR_SEQ_CHAINS;
+    for (int hb = lane; hb < 2 * blk; hb += SR_WAVE) before += cs[hb * SR_SEQ_CHAINS + wave];
+    if (2 * blk < hb1) own = cs[2 * blk * SR_SEQ_CHAINS + wave];
+    if (2 * blk + 1 < hb1) own += cs[(2 * blk + 1) * SR_SEQ_CHAINS + wave];
+    if (!a.lazy_scale && a.mode != 1 && seg < nseg)
+        for (int g = lane; g < seg; g += SR_WAVE) before_seg += sums[g];
+    if (blk < nblk) {
+        before = sr_wave_sum_f32(before) * r.inv;
+        // chain by chain in shared memory: the place of term 16 l + j of chain g is g 1024 + 64 j + (l + 2 j) mod 64, so that
+        // the lanes of a wave read a term from 64 consecutive places and a piece's stores fall two to a bank
+        float* const buf = (float*)room;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int t4 = wave * (SR_SEG_TERMS / 4) + k * SR_WAVE + lane;  // the piece's number within the block
+            const int vec = t4 >> 1, j = vec & 15, l = vec >> 4;
+            const bool in = blk * kPrepBlock + 4 * t4 < body;  // (body is a multiple of 8)
+            float* at = buf + (4 * (t4 & 1)) * 1024 + 64 * j + ((l + 2 * j) & 63);
+            at[0] = in ? v[k].x : 0.0f; at[1024] = in ? v[k].y : 0.0f; at[2048] = in ? v[k].z : 0.0f; at[3072] = in ? v[k].w : 0.0f;
+        }
+        __syncthreads();
+        float x[SR_SEQ_RUN];
+#pragma unroll
+        for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = buf[wave * 1024 + 64 * j + ((lane + 2 * j) & 63)];
+        seg_make_record<true>(x, blk, (double)before, chain + blk, own * r.inv);
+    }
+    sr_drain_stores();
+    __syncthreads();  // (the workgroup's records are out, and nobody reads the block any more)
+    if (tid == 0) {
+        const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint32_t ok = ((uint32_t)was & 0xffffu) + 1u == gridDim.x ? 1u : 0u;
+        if (!a.lazy_scale) {
+            for (uint32_t it = 0; ok == 0u && it < a.behind_wait_limit; it++) {
+                ok = ((uint32_t)sr_load_agent(sync) & 0xffffu) == gridDim.x ? 1u : 0u;
+                if (ok == 0u) __builtin_amdgcn_s_sleep(1);
+            }
+            if (ok == 0u) sr_store_agent(&st->late_behind, a.seq);
+        }
+        bc = ok;
+    }
+    __syncthreads();
+    bool here = bc != 0u;
+    if (a.lazy_scale && !here) return;  // (the last one has all there is to do)
+    // the eight accumulators, a wave each: the sum of the members, and 1 over it
+    auto normaliser = [&]() __attribute__((always_inline)) -> float {
+        int dummy;
+        float s = seg_walk_from<false, true>([&](int b, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
+            // (no condition stands between the loads: with one each they wait for each other; a whole block by offsets from one
+            // address)
+            const int t0 = b * SR_SEG_TERMS + lane * SR_SEQ_RUN;
+            const float* const e0 = r.e + (size_t)t0 * 8 + wave;
+            if ((b + 1) * SR_SEG_TERMS <= nv) {
+#pragma unroll
+                for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = e0[j * 8];
+            } else {
+#pragma unroll
+                for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = r.e[min(t0 + j, nv - 1) * 8 + wave];
+            }
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = t0 + j < nv ? r.cut(x[j], (t0 + j) * 8 + wave) : 0.0f;
+        }, nblk, chain, 0.0f, 0.0f, &dummy, nullptr);
+        if (rem > 0 && wave >= 8 - rem) s = __fadd_rn(s, r.cut(r.e[n - 8 + wave], n - 8 + wave));  // the overlapped last vector
+        if (lane == 0) lane_sum[wave] = s;
+        __syncthreads();
+        const float l0 = lane_sum[0], l1 = lane_sum[1], l2 = lane_sum[2], l3 = lane_sum[3], l4 = lane_sum[4], l5 = lane_sum[5],
+                    l6 = lane_sum[6], l7 = lane_sum[7];
+        const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
+        return (sum > 0.0f && sum != 1.0f) ? __fdiv_rn(1.0f, sum) : 1.0f;
+    };
+    float inv2 = 1.0f;
+    if (here) {
+        inv2 = normaliser();
+        if (a.lazy_scale) {
+            if (tid == 0) st->mul2 = inv2;
+            return;
+        }
+        if (seg < nseg) prepared_segment(a, r, slot, row, seg, lane, v, sr_wave_sum_f32(before_seg), inv2, room + wave * SR_WAVE * 5);
+    }
+    sr_drain_stores();
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        bc = ((uint32_t)(was >> 16) & 0xffffu) + 1u == gridDim.x ? (sr_load_agent(&st->late_behind) == a.seq ? 2u : 1u) : 0u;
+    }
+    __syncthreads();
+    if (bc == 0u) return;
+    if (bc == 2u) {
+        // some workgroup stopped waiting: all of the row again, from the accumulators' records
+        inv2 = normaliser();
+        for (int b = 0; b < (int)gridDim.x; b++) {
+            const int sg = b * SR_SEQ_CHAINS + wave;
+            if (sg >= nseg) break;
+            prepared_load(r, b, wave, lane, v);
+            float front = 0.0f;
+            for (int g = lane; g < sg; g += SR_WAVE) front += sums[g];
+            prepared_segment(a, r, slot, row, sg, lane, v, sr_wave_sum_f32(front), inv2, room + wave * SR_WAVE * 5);
+        }
+        sr_drain_stores();
+        __syncthreads();
+    }
+    if (tid == 0) st->mul2 = inv2;
+    if (a.mode == 1 || wave != 0) return;
+    const float u = st->u;
     int found;
-    const float at = seg_walk_from<true>([&](int seg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
-        const int i0 = seg * SR_SEG_TERMS + lane * SR_SEQ_RUN;
-        seq_load_run(r.e, true, i0, n, x);  // (the rows of e start on 16-byte boundaries; zeros past the end stay zeros)
+    const float at = seg_walk_from<true, true>([&](int sg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
+        const int i0 = sg * SR_SEG_TERMS + lane * SR_SEQ_RUN;
+        seq_load_run(r.e, true, i0, n, x);  // (zeros past the end stay zeros)
 #pragma unroll
         for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = __fmul_rn(r.cut(x[j], i0 + j), inv2);
-    }, seg_count(n), a.seg_func + (size_t)slot * a.seg_stride, 0.0f, u, &found, nullptr);
+    }, nseg, a.seg_func + (size_t)slot * a.seg_stride, 0.0f, u, &found, nullptr);
     if (lane == 0) {
-        const bool amb = found >= 0 ? sr_stop_near(at, term(found), u) : sr_near(at, u);
+        const bool amb = found >= 0 ? sr_stop_near(at, __fmul_rn(r.cut(r.e[found], found), inv2), u) : sr_near(at, u);
         if (a.out_tokens) a.out_tokens[row] = found >= 0 ? found : n - 1;
         if (a.out_flags) a.out_flags[row] = st->flags | (amb ? SR_KFLAG_AMBIGUOUS : 0u);
     }
@@ -4580,10 +4622,7 @@ hipError_t sr_launch_full_row(const SrFullArgs& a, int n_rows, hipStream_t st)
     hipLaunchKernelGGL(k_full_row, dim3(n_rows), dim3(kT), more, st, a);
     if (a.prepared) {
         const int nseg = (a.vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
-        hipLaunchKernelGGL(k_chain_records, dim3((unsigned)a.chain_blocks, n_rows), dim3(kPrepT), 0, st, a);
-        hipLaunchKernelGGL(k_prepared_draw, dim3(a.lazy_scale ? 1u : (unsigned)((nseg + SR_SEQ_CHAINS - 1) / SR_SEQ_CHAINS), n_rows),
-                           dim3(kPrepT), 0, st, a);
-        if (a.mode != 1) hipLaunchKernelGGL(k_prepared_token, dim3(n_rows), dim3(SR_WAVE), 0, st, a);
+        hipLaunchKernelGGL(k_prepared_row, dim3((unsigned)((nseg + SR_SEQ_CHAINS - 1) / SR_SEQ_CHAINS), n_rows), dim3(kPrepT), 0, st, a);
     }
     return hipGetLastError();
 }

@@ -101,6 +101,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     }
     a.seq = ctx->full_seq;
     a.row_wait_limit = ctx->row_wait_limit;
+    a.behind_wait_limit = ctx->behind_wait_limit;
     // sort segments are laid out with the work stride of mode 0; in modes 1/2 use a private stride
     const int64_t seg_stride = (vocab + 3) & ~3;
     if ((int64_t)n_rows * seg_stride >= (int64_t)1 << 31)

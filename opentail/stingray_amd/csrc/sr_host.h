@@ -323,6 +323,7 @@ struct sr_ctx {
     unsigned launch_no = 0;
     uint32_t spin_limit = 1u << 22;
     uint32_t row_wait_limit = 1u << 15;  // SrFullArgs::row_wait_limit (a poll is a round trip to device memory: tens of ms)
+    uint32_t behind_wait_limit = 1u << 15;  // SrFullArgs::behind_wait_limit
 };
 
 struct sr_batch {

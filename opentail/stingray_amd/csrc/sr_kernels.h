@@ -145,12 +145,15 @@ struct SrFullState {
     float ycut;           // ... whose members are the probabilities above ycut, and of those equal to it the ones up to idx_last
     int32_t idx_last;
     uint32_t list_from;   // the row's list of candidates holds its e from this value on (as bits); 0: it would have been too long
-    int32_t pad[5];
+    uint32_t late_behind; // the number of the last launch in which a workgroup of k_prepared_row stopped waiting for the row's others
+    float u;              // the uniform of the draw, of a row left to the whole device
+    int32_t pad[3];
 };
 static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // SrFullArgs::row_sync, a word per row (rows 256 bytes apart: every workgroup of a row adds to its word and polls it):
 // launch number << 32 | workgroups of k_full_softmax_seg at the second meeting point << 16 | at the first.  The number is
-// put in by an atomic maximum before the first count of a launch, so nothing clears the words.
+// put in by an atomic maximum before the first count of a launch, so nothing clears the words.  The word behind it counts the
+// workgroups of k_prepared_row the same way; k_full_row, which leaves the row to them, starts it.
 #define SR_ROW_SYNC_STRIDE 32
 
 struct SeqSegFunc;
@@ -205,6 +208,7 @@ struct SrFullArgs {
                                    // need no table either (k_full_softmax_seg applies their edits where it loads the row)
     unsigned long long* row_sync;  // [slot * SR_ROW_SYNC_STRIDE]
     uint32_t row_wait_limit;       // polls of a row's count before a workgroup of k_full_softmax_seg stops waiting for it
+    uint32_t behind_wait_limit;    // ... of k_prepared_row
     int32_t big_slabs;             // k_full_row gets 68 KB of shared memory more: lists of 16,384 candidates, slabs of 8,192 entries
 };
 hipError_t sr_launch_full_prep(const SrFullArgs& a, int n_rows, hipStream_t st);

@@ -795,6 +795,33 @@ def test_workgroups_that_stop_waiting_for_their_row_leave_their_segments_to_the_
         ctx._check(H.sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
 
 
+@pytest.mark.parametrize("vocab", [40_968, 49_153, 65_543])  # whole pieces of eight; one entry in a block of its own; seven left over
+def test_workgroups_that_stop_waiting_leave_a_prepared_row_to_the_last_one(ctx, vocab):
+    """Rows that are normalised and drawn by the whole device in one launch: its workgroups wait for each other once, and where
+    the wait runs out (from the first poll on, or behind a few) the last workgroup of the row does all of it.  Rows
+    that nothing cuts, rows that top-p cuts to thousands of members, a sharp row; tokens and distributions."""
+    rng = np.random.default_rng(vocab)
+    params = [SamplingParams(), SamplingParams(Temperature=1.2, TopP=0.95), SamplingParams(Temperature=0.9, TopP=0.5),
+              SamplingParams(Temperature=1.3, TopP=0.9, RepetitionPenalty=1.2, PreviousTokens=rng.integers(0, vocab, 60).tolist())]
+    logits = rng.normal(0, 2.0, (len(params), vocab)).astype(np.float32)
+    logits[2, 7] += 14.0
+    H = hooks_lib()
+    try:
+        for polls in (0, 1, 3, 1 << 15):
+            ctx._check(H.sr_debug_set_row_wait_limit(ctx.h, 0x80000000 | polls))
+            for _ in range(2):
+                _check_rows(ctx, logits, params, rng.random(len(params)))
+            _check_distribution(ctx, logits, params)
+            u = rng.random(len(params))
+            toks, probs = ctx.sample_with_distribution(_cuda(logits), params, u)
+            probs = probs.cpu().numpy()
+            for r, p in enumerate(params):
+                t, d = orc.sample_with_distribution(logits[r], to_oracle(p), orc.Rng(replay=[u[r]]))
+                assert toks[r] == t and np.array_equal(probs[r].view(np.uint32), np.asarray(d, dtype=np.float32).view(np.uint32)), (polls, r)
+    finally:
+        ctx._check(H.sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
+
+
 def test_edits_crowded_into_a_few_segments_of_a_long_row(ctx):
     """The pass over long rows applies the edits of a sampled row where it loads the row: a workgroup lists the edits
     that fall into its segments (room for 256) and goes through the row's whole edit list when there are more.  Rows
