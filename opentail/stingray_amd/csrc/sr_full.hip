@@ -385,15 +385,17 @@ __device__ __forceinline__ void seg_load_rec(const SeqSegFunc* funcs, int seg, i
 // follows is done again.  A segment taken by itself costs some 50 instructions of the one wave, 0.1 us, a sum that
 // starts at zero has about a dozen; looking for the end of every run of segments as it went, the walk took 0.45 us for each:
 // 98 segments of a row of 100,003 entries 5.3 us, and a search over as many 7.5.
+// first64: the first 64 records, where the caller has asked for them already.
 template <bool kSearch, bool kAgent = false, typename Load>
 __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSegFunc* funcs, float s0, float target, int* found,
-                                               float* states)
+                                               float* states, const SegRec* first64 = nullptr)
 {
     const int lane = sr_lane();
     uint32_t sb = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(s0));  // the running sum's bits, the same in every lane
     *found = -1;
     SegRec next;
-    seg_load_rec<kAgent>(funcs, lane, nseg, next);
+    if (first64) next = *first64;
+    else seg_load_rec<kAgent>(funcs, lane, nseg, next);
     for (int base = 0; base < nseg; base += SR_WAVE) {
         const SegRec r = next;
         if (base + SR_WAVE < nseg) seg_load_rec<kAgent>(funcs, base + SR_WAVE + lane, nseg, next);  // (the next 64 segments' come in meanwhile)
@@ -498,13 +500,13 @@ __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSeg
 // ... over terms[0, n) in memory
 template <bool kSearch>
 __device__ __forceinline__ float seg_walk(const float* terms, int n, const SeqSegFunc* funcs, float s0, float target, int* found,
-                                          float* states)
+                                          float* states, const SegRec* first64 = nullptr)
 {
     const bool aligned = ((uintptr_t)terms & 15u) == 0u;
     const int lane = sr_lane();
     return seg_walk_from<kSearch>([&](int seg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
         seq_load_run(terms, aligned, seg * SR_SEG_TERMS + lane * SR_SEQ_RUN, n, x);
-    }, seg_count(n), funcs, s0, target, found, states);
+    }, seg_count(n), funcs, s0, target, found, states, first64);
 }
 
 // The record of one segment (SeqSegFunc) from its terms x (lane l holds the terms 16 l ... 16 l + 15 of the segment) and
@@ -3152,11 +3154,30 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     __shared__ FullSmem sm;
     const int tid = threadIdx.x;
     const int slot = blockIdx.x;
+    const int n = a.vocab;
+    SrFullState* st = a.state + slot;
+    // What does not hang on the row's descriptor is asked for beside it: the row's state, the first records of its sum (by the
+    // wave that will walk them) and how many entries its segments have listed (by the others).
+    const uint32_t st_late = st->late, st_list_from = st->list_from;
+    const unsigned long long st_maxkey = st->maxkey;
+    SegRec first64 = {};
+    constexpr int kCntAhead = 4;
+    int cnt_ahead[kCntAhead] = {};
+    if (a.seg_func) {
+        const int nseg = seg_count(n);
+        if (sr_wave_id() == 0) {
+            seg_load_rec<false>(a.seg_func + (size_t)slot * a.seg_stride, sr_lane(), nseg, first64);
+        } else {
+#pragma unroll
+            for (int q = 0; q < kCntAhead; q++) {
+                const int g = q * SR_WAVE + sr_lane();
+                cnt_ahead[q] = g < nseg ? (int)a.seg_cnt[(size_t)slot * a.seg_stride + g] : 0;
+            }
+        }
+    }
     const int row = a.row_list[slot];
     const SrRow rd = a.rows[row];
-    const int n = a.vocab;
     float* p = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;
-    SrFullState* st = a.state + slot;
     const bool greedy = rd.temperature <= 0.0f;
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
     if (tid == 0) {
@@ -3187,12 +3208,12 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     {
         FPROF(a, slot, 0);
         // Softmax (Sampler.cs:448-472): the maximum and e = expf(x - max) were computed by the kernels before
-        const bool alone = a.seg_func != nullptr && (st->late == a.seq || full_maxkey_of(a, st->maxkey) == kKeyInf);
+        const bool alone = a.seg_func != nullptr && (st_late == a.seq || full_maxkey_of(a, st_maxkey) == kKeyInf);
         const bool walked = a.seg_func != nullptr && !alone;
         // (a list that would have been too long was not made)
-        const bool has_list = walked && row_is_listed(rd, a) && st->list_from != 0u, plain = walked && row_is_plain(rd, a);
+        const bool has_list = walked && row_is_listed(rd, a) && st_list_from != 0u, plain = walked && row_is_plain(rd, a);
         float* const e_row = walked ? row_e(a, slot) : p;
-        const uint32_t mk = alone ? row_alone(a, rd, p, n, row, sm) : full_maxkey_of(a, st->maxkey);
+        const uint32_t mk = alone ? row_alone(a, rd, p, n, row, sm) : full_maxkey_of(a, st_maxkey);
         const bool any_nan = mk == 0xffffffffu;
         const float m = mk == 0u ? SR_NEG_INF : sr_okey_inv(mk);
         FPROF(a, slot, 1);
@@ -3226,53 +3247,64 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
             if (walked) {
                 // the whole device has prepared the sum (k_full_softmax_seg): one wave walks the segments' records while the
                 // others fetch the row's list, if it has one
-                if (has_list) {
-                    const int nseg = seg_count(n);
-                    const int c = tid < nseg ? (int)a.seg_cnt[(size_t)slot * a.seg_stride + tid] : 0;
-                    static_assert(SR_SEG_MAX <= kT, "a thread per segment");
-                    const int o = blk_excl_scan(c, &n_list, sm);
-                    if (tid < nseg) ((int*)sm.segst)[tid] = o;
-                    static_assert(kCkpt >= SR_WAVE, "a word per entry of a short list");
-                    if (n_list <= SR_WAVE)  // where every entry of a short list lies
-                        for (int k = 0; k < c; k++) ((int*)sm.ckpt)[o + k] = tid * SR_SEG_TERMS + k;
-                }
-                __syncthreads();
                 if (sr_wave_id() == 0) {
-                    const float s = seg_walk<false>(e_row, n, a.seg_func + (size_t)slot * a.seg_stride, 0.0f, 0.0f, &dummy, nullptr);
+                    const float s = seg_walk<false>(e_row, n, a.seg_func + (size_t)slot * a.seg_stride, 0.0f, 0.0f, &dummy, nullptr, &first64);
                     if (sr_lane() == 0) sm.segbc[0] = sr_f2u(s);
-                } else if (has_list && n_list <= SR_WAVE) {
-                    const int l = tid - SR_WAVE;
-                    if (l < n_list) {
-                        const size_t at = (size_t)slot * (size_t)a.sort_stride + (size_t)((const int*)sm.ckpt)[l];
-                        sm.hist[l] = a.sort_keys_in[at];
-                        sm.hist[SR_WAVE + l] = (uint32_t)a.sort_vals_in[at];
-                    }
-                } else if (has_list && n_list <= list_cap(more != nullptr)) {
-                    uint32_t* const grp = list_values(more, sm);
+                } else if (has_list) {
+                    // where the segments' entries start: every wave adds up the counts for itself and writes all of them, the
+                    // same values (a scan by the workgroup, in front of the walk, was two barriers)
                     const int nseg = seg_count(n), lane = sr_lane();
-                    const int* off = (const int*)sm.segst;
-                    const uint32_t* gk = a.sort_keys_in + (size_t)slot * (size_t)a.sort_stride;
-                    // (four segments' first entries on their way at a time)
-                    for (int s0 = sr_wave_id() - 1; s0 < nseg; s0 += 4 * (kW - 1)) {
-                        uint32_t v[4];
-                        int at[4], len[4];
+                    int* const off = (int*)sm.segst;
+                    static_assert(kCkpt >= SR_WAVE, "a word per entry of a short list");
+                    auto count = [&](int g0, int c) __attribute__((always_inline)) {
+                        const int incl = sr_wave_incl_scan_i32(c), o = n_list + incl - c, g = g0 + lane;
+                        if (g < nseg) off[g] = o;
+                        if (sr_wave_id() == 1)  // where every entry of a short list lies
+                            for (int k = 0; k < c && o + k < SR_WAVE; k++) ((int*)sm.ckpt)[o + k] = g * SR_SEG_TERMS + k;
+                        n_list += __builtin_amdgcn_readlane(incl, SR_WAVE - 1);
+                    };
 #pragma unroll
-                        for (int q = 0; q < 4; q++) {
-                            const int sg = s0 + q * (kW - 1);
-                            at[q] = sg < nseg ? off[sg] : 0;
-                            len[q] = sg < nseg ? (sg + 1 < nseg ? off[sg + 1] : n_list) - at[q] : 0;
-                            v[q] = lane < len[q] ? gk[(size_t)sg * SR_SEG_TERMS + lane] : 0u;
+                    for (int q = 0; q < kCntAhead; q++)
+                        if (q * SR_WAVE < nseg) count(q * SR_WAVE, cnt_ahead[q]);
+                    for (int g0 = kCntAhead * SR_WAVE; g0 < nseg; g0 += SR_WAVE)
+                        count(g0, g0 + lane < nseg ? (int)a.seg_cnt[(size_t)slot * a.seg_stride + g0 + lane] : 0);
+                    if (tid == SR_WAVE) sm.segbc[3] = (uint32_t)n_list;
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    if (n_list <= SR_WAVE) {
+                        const int l = tid - SR_WAVE;
+                        if (l < n_list) {
+                            const size_t at = (size_t)slot * (size_t)a.sort_stride + (size_t)((const int*)sm.ckpt)[l];
+                            sm.hist[l] = a.sort_keys_in[at];
+                            sm.hist[SR_WAVE + l] = (uint32_t)a.sort_vals_in[at];
                         }
+                    } else if (n_list <= list_cap(more != nullptr)) {
+                        uint32_t* const grp = list_values(more, sm);
+                        const uint32_t* gk = a.sort_keys_in + (size_t)slot * (size_t)a.sort_stride;
+                        // (four segments' first entries on their way at a time)
+                        for (int s0 = sr_wave_id() - 1; s0 < nseg; s0 += 4 * (kW - 1)) {
+                            uint32_t v[4];
+                            int at[4], len[4];
 #pragma unroll
-                        for (int q = 0; q < 4; q++) {
-                            const int sg = s0 + q * (kW - 1);
-                            if (lane < len[q]) grp[list_place(at[q] + lane)] = v[q];
-                            for (int i = lane + SR_WAVE; i < len[q]; i += SR_WAVE) grp[list_place(at[q] + i)] = gk[(size_t)sg * SR_SEG_TERMS + i];
+                            for (int q = 0; q < 4; q++) {
+                                const int sg = s0 + q * (kW - 1);
+                                at[q] = sg < nseg ? off[sg] : 0;
+                                len[q] = sg < nseg ? (sg + 1 < nseg ? off[sg + 1] : n_list) - at[q] : 0;
+                                v[q] = lane < len[q] ? gk[(size_t)sg * SR_SEG_TERMS + lane] : 0u;
+                            }
+#pragma unroll
+                            for (int q = 0; q < 4; q++) {
+                                const int sg = s0 + q * (kW - 1);
+                                if (lane < len[q]) grp[list_place(at[q] + lane)] = v[q];
+                                for (int i = lane + SR_WAVE; i < len[q]; i += SR_WAVE) grp[list_place(at[q] + i)] = gk[(size_t)sg * SR_SEG_TERMS + i];
+                            }
                         }
                     }
                 }
                 __syncthreads();
                 sum = sr_u2f(sm.segbc[0]);
+                if (has_list) n_list = (int)sm.segbc[3];
             } else {
                 sum = seq_sum_row<false>(p, n, 0.0f, 0.0f, &dummy, sm);
             }
@@ -3321,7 +3353,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
             if (e_row != p) {
                 // (a row that goes on here has its probabilities take shape in the caller's row; one whose list was not made has
                 // all but the last of e there)
-                for (int i = tid + (row_is_listed(rd, a) && st->list_from == 0u ? n & ~3 : 0); i < n; i += kT) p[i] = e_row[i];
+                for (int i = tid + (row_is_listed(rd, a) && st_list_from == 0u ? n & ~3 : 0); i < n; i += kT) p[i] = e_row[i];
                 sr_drain_stores();
                 __syncthreads();
             }
