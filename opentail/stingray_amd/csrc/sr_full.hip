@@ -608,21 +608,18 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
 
 // The search that follows a sum over the same terms: the first term at which the running sum reaches `target`, from
 // the states the sum left (one wave; -1 when the sum stays below the target).
-__device__ __forceinline__ int seg_search_states(const float* terms, int n, const float* states, float target, float* at_sum)
+template <typename Load>
+__device__ __forceinline__ int seg_search_states(Load load, int nseg, const float* states, float target, float* at_sum)
 {
-    const int lane = sr_lane();
-    const int nseg = seg_count(n);
-    const bool aligned = ((uintptr_t)terms & 15u) == 0u;
     int first = nseg;
-    for (int g = lane; g < nseg; g += SR_WAVE)
+    for (int g = sr_lane(); g < nseg; g += SR_WAVE)
         if (states[g] >= target) { first = g; break; }
     first = sr_wave_min_i32(first);
     if (first >= nseg) return -1;
-    const float s_before = first > 0 ? states[first - 1] : 0.0f;
     float x[SR_SEQ_RUN];
-    seq_load_run(terms, aligned, first * SR_SEG_TERMS + lane * SR_SEQ_RUN, n, x);
+    load(first, x);
     int at;
-    *at_sum = sr_seq_wave<SR_SEQ_RUN, true>(x, s_before, target, &at);
+    *at_sum = sr_seq_wave<SR_SEQ_RUN, true>(x, first > 0 ? states[first - 1] : 0.0f, target, &at);
     return at >= 0 ? first * SR_SEG_TERMS + at : -1;
 }
 
@@ -4216,67 +4213,6 @@ __device__ __forceinline__ int resample_residual_stored(const float* res, const 
     return found >= 0 ? found : edge(false);  // (rounding: the sum of the search fell short of the target)
 }
 
-// ... with the increment functions of the stored row's segments at hand (k_seq_funcs): one wave walks them
-__device__ __forceinline__ int residual_edge(const float* res, int n, bool first_one, FullSmem& sm)
-{
-    // the first / the last index with a positive residual
-    int at = first_one ? 0x7fffffff : -1;
-    for (int i = threadIdx.x; i < n; i += kT)
-        if (res[i] > 0.0f) {
-            at = i;
-            if (first_one) break;
-        }
-    at = first_one ? sr_wave_min_i32(at) : -sr_wave_min_i32(-at);
-    __syncthreads();
-    if (sr_lane() == 0) sm.redi[sr_wave_id()] = at;
-    __syncthreads();
-    int f = first_one ? 0x7fffffff : -1;
-    for (int w = 0; w < kW; w++) f = first_one ? min(f, sm.redi[w]) : max(f, sm.redi[w]);
-    __syncthreads();
-    return f;
-}
-__device__ __forceinline__ int resample_residual_prepared(const float* res, const SeqSegFunc* funcs, const float* p, int n, double u,
-                                                          FullSmem& sm, float m1, float m2)
-{
-    const bool walker = sr_wave_id() == 0;
-    int dummy;
-    __syncthreads();  // (sm.segst and sm.segbc are free)
-    if (walker) {
-        const float sum = seg_walk<false>(res, n, funcs, 0.0f, 0.0f, &dummy, sm.segst);
-        if (sr_lane() == 0) sm.segbc[0] = sr_f2u(sum);
-    }
-    __syncthreads();
-    const float sum = sr_u2f(sm.segbc[0]);
-    if (!(sum > 0.0f)) return draw_from_row(p, n, u, sm, m1, m2);  // sum <= 0 or NaN
-    const float target = __fmul_rn(__double2float_rn(u), sum);
-    if (target <= 0.0f) return residual_edge(res, n, true, sm);  // a zero target must not stop on a zero term
-    if (walker) {
-        float at;
-        const int found = seg_search_states(res, n, sm.segst, target, &at);
-        if (sr_lane() == 0) sm.segbc[1] = (uint32_t)found;
-    }
-    __syncthreads();
-    const int found = (int)sm.segbc[1];
-    return found >= 0 ? found : residual_edge(res, n, false, sm);  // (rounding: the sum of the search fell short of the target)
-}
-// SampleFromDistribution (Sampler.cs:564-576) over a stored row with its segments' functions: draw_from_row by one wave
-__device__ __forceinline__ int draw_from_prepared(const float* terms, const SeqSegFunc* funcs, int n, double u, FullSmem& sm)
-{
-    const float r = __double2float_rn(u);
-    __syncthreads();
-    if (sr_wave_id() == 0) {
-        int found;
-        const float at = seg_walk<true>(terms, n, funcs, 0.0f, r, &found, nullptr);
-        if (sr_lane() == 0) {
-            sm.segbc[1] = (uint32_t)found;
-            SR_AMB_IF(found >= 0 ? sr_stop_near(at, terms[found], r) : sr_near(at, r));
-        }
-    }
-    __syncthreads();
-    const int found = (int)sm.segbc[1];
-    return found >= 0 ? found : n - 1;
-}
-
 // Every position of a row is filtered with the row's own parameters (SpeculativeDecoder.cs:535): the batch's row
 // descriptors, one copy per position, without their allow-masks
 __global__ __launch_bounds__(256) void k_expand_rows(const SrRow* src, SrRow* dst, int rows, int positions)
@@ -4288,6 +4224,42 @@ __global__ __launch_bounds__(256) void k_expand_rows(const SrRow* src, SrRow* ds
     dst[i] = d;
 }
 
+// The terms of the draw behind a row's accept loop: max(0, fl(fl(p m1) m2) - q) of its first rejected position, or the scaled target
+// row of the bonus position
+struct SpecTerms {
+    const float* p;   // (starts on 16 bytes)
+    const float* q;   // at any address; null: the bonus position
+    float m1, m2;
+    int n;
+    __device__ __forceinline__ float term(float pv, float qv) const
+    {
+        const float sp = __fmul_rn(__fmul_rn(pv, m1), m2), r = q ? __fsub_rn(sp, qv) : sp;
+        return q ? (r > 0.0f ? r : 0.0f) : sp;
+    }
+    __device__ __forceinline__ float at(int i) const { return term(p[i], q ? q[i] : 0.0f); }
+    // four consecutive terms from i0, zeros past the end
+    __device__ __forceinline__ float4 four(int i0) const
+    {
+        float4 o = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (i0 + 4 <= n) {
+            const float4 pv = *(const float4*)(p + i0), qv = q ? sr_load_f4(q + i0) : o;
+            o = make_float4(term(pv.x, qv.x), term(pv.y, qv.y), term(pv.z, qv.z), term(pv.w, qv.w));
+        } else if (i0 < n) {
+            o.x = at(i0);
+            if (i0 + 1 < n) o.y = at(i0 + 1);
+            if (i0 + 2 < n) o.z = at(i0 + 2);
+        }
+        return o;
+    }
+    __device__ __forceinline__ void run(int seg, float (&x)[SR_SEQ_RUN]) const  // a lane's 16 terms of a segment
+    {
+        float4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = four(seg * SR_SEG_TERMS + sr_lane() * SR_SEQ_RUN + 4 * k);
+#pragma unroll
+        for (int k = 0; k < 4; k++) { x[4 * k] = v[k].x; x[4 * k + 1] = v[k].y; x[4 * k + 2] = v[k].z; x[4 * k + 3] = v[k].w; }
+    }
+};
 // The accept loop of a row under the ratio test needs one element of p and of q per position, no pass over a row:
 // one wave walks it ahead of everything else and names the first rejected position, so that the residual row of
 // that position -- which the row's workgroup would otherwise compute twice, from two rows, at the rate of one compute
@@ -4300,8 +4272,6 @@ __global__ __launch_bounds__(SR_WAVE) void k_spec_walk(SrSpecArgs a)
     const bool true_spec = !(rd.p_min > 0.0f && rd.p_min < 1.0f) && (rd.flags & SR_ROWBIT_DRAFT_FROM_LOOKUP) == 0u;
     int reject = -1;
     if (true_spec) {
-        // (every draft accepted, and a bonus token to draw: position L, whose scaled row k_spec_residual writes out)
-        if (a.seg_func && rd.temperature > 0.0f) reject = L;
         const float* pr = a.p_all + (size_t)row * (L + 1) * (size_t)a.p_stride;
         const double* u = a.uniforms + (size_t)row * a.uniforms_per_row;
         for (int i0 = 0; i0 < L; i0 += SR_WAVE) {
@@ -4331,72 +4301,230 @@ __global__ __launch_bounds__(SR_WAVE) void k_spec_walk(SrSpecArgs a)
 }
 
 // The terms the row's workgroup will add, written by the whole device: max(0, fl(fl(p m1) m2) - q) of the first rejected
-// position, or the scaled target row fl(fl(p m1) m2) of the bonus position when every draft was accepted (reject == L).
-// A wave takes whole segments of SR_SEG_TERMS terms and leaves each segment's approximate sum for k_seq_funcs.
+// position.
 __global__ __launch_bounds__(256) void k_spec_residual(SrSpecArgs a)
 {
     const int row = blockIdx.y;
     const int i = a.reject[row];
     if (i < 0) return;
-    const int n = a.vocab, L = a.n_draft, lane = sr_lane();
-    const bool bonus = i == L;
-    const float* pd = a.p_all + ((size_t)row * (L + 1) + i) * (size_t)a.p_stride;
-    const float* qd = bonus ? pd : a.draft_probs + ((size_t)row * L + i) * n;
+    const int n = a.vocab, L = a.n_draft;
+    SpecTerms t;
+    t.p = a.p_all + ((size_t)row * (L + 1) + i) * (size_t)a.p_stride;
+    t.q = a.draft_probs + ((size_t)row * L + i) * n;
     const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
-    const float m1 = sl->mul1, m2 = sl->mul2;
-    float* out = a.resid + (size_t)row * (size_t)a.resid_stride;
-    auto res = [&](float pv, float qv) -> float {
-        const float sp = __fmul_rn(__fmul_rn(pv, m1), m2);
-        if (bonus) return sp;
-        const float r = __fsub_rn(sp, qv);
-        return r > 0.0f ? r : 0.0f;
-    };
-    const bool aligned = ((((uintptr_t)pd) | ((uintptr_t)qd)) & 15u) == 0u;
-    const int nseg = seg_count(n);
-    for (int seg = (int)blockIdx.x * 4 + sr_wave_id(); seg < nseg; seg += (int)gridDim.x * 4) {
-        double acc = 0.0;
-#pragma unroll
-        for (int k = 0; k < SR_SEG_TERMS / (4 * SR_WAVE); k++) {
-            const int x0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
-            if (aligned && x0 + 4 <= n) {
-                const float4 pv = *(const float4*)(pd + x0), qv = *(const float4*)(qd + x0);
-                float4 o;
-                o.x = res(pv.x, qv.x); o.y = res(pv.y, qv.y); o.z = res(pv.z, qv.z); o.w = res(pv.w, qv.w);
-                *(float4*)(out + x0) = o;  // (the rows of a.resid start on 16-byte boundaries)
-                acc += ((double)o.x + (double)o.y) + ((double)o.z + (double)o.w);
-            } else {
-                for (int x = x0; x < min(x0 + 4, n); x++) {
-                    const float o = res(pd[x], qd[x]);
-                    out[x] = o;
-                    acc += (double)o;
-                }
-            }
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-        if (a.seg_part && lane == 0) a.seg_part[(size_t)row * a.seg_stride + seg] = acc;
-    }
+    t.m1 = sl->mul1;
+    t.m2 = sl->mul2;
+    t.n = n;
+    float* const out = a.resid + (size_t)row * (size_t)a.resid_stride;
+    for (int x0 = ((int)blockIdx.x * 256 + (int)threadIdx.x) * 4; x0 < n; x0 += (int)gridDim.x * 1024) *(float4*)(out + x0) = t.four(x0);
+    // (the rows of a.resid start on 16 bytes and are a multiple of 16 bytes long)
 }
 
-// The record of every segment of every row of terms (SeqSegFunc), for the binades that the approximate sums predict:
-// the sums of the segments in front (part, left by the kernel that wrote the terms) and, inside the segment, of the
-// lanes in front.  One wave per segment.
-__global__ __launch_bounds__(256) void k_seq_funcs(const float* terms, int64_t stride, int n, const double* part, SeqSegFunc* func,
-                                                   int seg_stride, const int32_t* active)
+// ---- speculative verification of rows under the ratio test (StepSampled, SpeculativeDecoder.cs:530-559) --------------------
+// The accept loop of such a row needs one element of p and of q per position, and the draw behind it one row of terms: max(0,
+// fl(fl(p m1) m2) - q) of the first rejected position, or the scaled target row fl(fl(p m1) m2) of the bonus position when every
+// draft was accepted.  One launch, a workgroup per eight segments of the row: each finds the position for itself (one wave, a
+// position a lane: less than a meeting would cost), makes the terms of its segments, leaves their sums, and when the row's workgroups are
+// all there, their records; whoever comes last walks them, draws and writes the row's results.  The terms stay in registers; the
+// walk makes those it needs again from p and q.
+// What bounds it: the serial chain again (two trips for the position, the terms, a meeting, records, walk, search).  As four
+// launches with the terms written and read back: 46 us for 16 rows of 262,144 and 8 drafts.
+// The wait is bounded: a workgroup whose wait runs out marks the row and counts itself in, and whoever comes last adds all of the
+// row's terms by its own.
+// reject[row] = kSpecDone, or -1: the row is k_spec_verify's (other accept rules, a bonus token of a greedy row).
+constexpr int kSpecT = 512, kSpecDone = -2;
+constexpr int kSpecWaves = kSpecT / SR_WAVE;
+// the exact running sum (or the search) over all segments from their terms, by one wave; the slow way of the rare cases
+template <bool kSearch>
+__device__ __forceinline__ float spec_sum_alone(const SpecTerms& t, int nseg, float target, int* found, float* states)
 {
-    const int row = blockIdx.y, lane = sr_lane();
-    if (active && active[row] < 0) return;
-    const int seg = (int)blockIdx.x * 4 + sr_wave_id();
-    if (seg >= seg_count(n)) return;
-    const double* pr = part + (size_t)row * seg_stride;
-    double before = 0.0;
-    for (int g = lane; g < seg; g += SR_WAVE) before += pr[g];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
-    const float* t = terms + (size_t)row * (size_t)stride;
+    float s = 0.0f;
+    *found = -1;
+    for (int sg = 0; sg < nseg; sg++) {
+        float x[SR_SEQ_RUN];
+        t.run(sg, x);
+        int at;
+        s = sr_seq_wave<SR_SEQ_RUN, kSearch>(x, s, target, &at);
+        if (kSearch && at >= 0) {
+            *found = sg * SR_SEG_TERMS + at;
+            return s;
+        }
+        if (states && sr_lane() == 0) states[sg] = s;
+    }
+    return s;
+}
+__global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
+{
+    __shared__ float4 turn_all[kSpecWaves][SR_WAVE * 5];
+    __shared__ float states[SR_SEG_MAX];  // every segment's part of the sum, then the running sum behind every segment
+    __shared__ uint32_t bc;
+    __shared__ int said[2];
+    const int row = blockIdx.y, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
+    const SrRow rd = a.rows[row];
+    const int n = a.vocab, L = a.n_draft, nseg = seg_count(n);
+    unsigned long long* const sync = a.sync + (size_t)row * SR_ROW_SYNC_STRIDE;
+    if ((rd.p_min > 0.0f && rd.p_min < 1.0f) || (rd.flags & SR_ROWBIT_DRAFT_FROM_LOOKUP) != 0u) {
+        if (blockIdx.x == 0 && tid == 0) a.reject[row] = -1;
+        return;
+    }
+    const double* const u = a.uniforms + (size_t)row * a.uniforms_per_row;
+    if (wave == 0) {
+        // the first position that is not accepted: kind 0 rejected, 1 none (position L), 2 an id outside the vocabulary, which
+        // ends the row without a correction
+        const float* const pr = a.p_all + (size_t)row * (L + 1) * (size_t)a.p_stride;
+        int pos = L, kind = 1;
+        for (int i0 = 0; i0 < L; i0 += SR_WAVE) {
+            const int i = i0 + lane;
+            bool stop = false, bad = false;
+            if (i < L) {
+                const int tok = a.draft_tokens[(size_t)row * L + i];
+                bad = (uint32_t)tok >= (uint32_t)n;
+                if (!bad) {
+                    const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
+                    const float px = __fmul_rn(__fmul_rn(pr[(size_t)i * (size_t)a.p_stride + tok], sl->mul1), sl->mul2);
+                    const float qx = a.draft_probs[((size_t)row * L + i) * n + tok];
+                    const float acc = qx > 0.0f ? fminf(1.0f, __fdiv_rn(px, qx)) : (px > 0.0f ? 1.0f : 0.0f);
+                    stop = !(u[i] < (double)acc);  // (every position before it was accepted and drew one uniform)
+                }
+            }
+            const unsigned long long ends = __ballot(stop || bad);
+            if (ends != 0ull) {
+                const int l = (int)__ffsll((long long)ends) - 1;
+                pos = i0 + l;
+                kind = ((__ballot(bad) >> l) & 1ull) != 0ull ? 2 : 0;
+                break;
+            }
+        }
+        if (lane == 0) { said[0] = pos; said[1] = kind; }
+    } else if (tid == SR_WAVE) {
+        // (the number of the launch: nothing clears the words between launches)
+        const unsigned long long was = __hip_atomic_fetch_max(sync, (unsigned long long)a.seq << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" : : "v"(was) : "memory");
+    }
+    __syncthreads();
+    const int pos = said[0], kind = said[1];
+    auto results = [&](int correction) __attribute__((always_inline)) {  // (by one wave)
+        int* const out = a.out_tokens + (size_t)row * (L + 1);
+        for (int i = lane; i <= L; i += SR_WAVE) out[i] = i < pos ? a.draft_tokens[(size_t)row * L + i] : i == pos ? correction : -1;
+        if (lane == 0) {
+            a.out_accepted[row] = pos;
+            a.reject[row] = kSpecDone;
+        }
+    };
+    if (kind == 2) {
+        if (blockIdx.x == 0 && wave == 0) results(-1);
+        return;
+    }
+    if (kind == 1 && rd.temperature <= 0.0f) {  // (the bonus token of a greedy row: its argmax)
+        if (blockIdx.x == 0 && tid == 0) a.reject[row] = -1;
+        return;
+    }
+    SpecTerms t;
+    t.p = a.p_all + ((size_t)row * (L + 1) + pos) * (size_t)a.p_stride;
+    t.q = kind == 0 ? a.draft_probs + ((size_t)row * L + pos) * n : nullptr;
+    {
+        const SrFullState* sl = a.state + (size_t)row * (L + 1) + pos;
+        t.m1 = sl->mul1;
+        t.m2 = sl->mul2;
+    }
+    t.n = n;
+    const int seg = (int)blockIdx.x * kSpecWaves + wave;
+    SeqSegFunc* const funcs = a.seg_func + (size_t)row * a.seg_stride;
+    float* const sums = a.seg_part + (size_t)row * a.seg_stride;
     float x[SR_SEQ_RUN];
-    seq_load_run(t, ((uintptr_t)t & 15u) == 0u, seg * SR_SEG_TERMS + lane * SR_SEQ_RUN, n, x);
-    seg_make_record(x, seg, before, func + (size_t)row * seg_stride + seg);
+    float own = 0.0f;
+    if (seg < nseg) {
+        float4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) v[k] = t.four(seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4);
+        float4* const turn = turn_all[wave];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i = (k * SR_WAVE + lane) * 4;
+            own += (v[k].x + v[k].y) + (v[k].z + v[k].w);
+            turn[(i >> 4) * 5 + ((i & 15) >> 2)] = v[k];
+        }
+        own = sr_wave_sum_f32(own);
+        if (lane == 0) sr_store_agent(&sums[seg], own);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float4 w = turn[lane * 5 + k];
+            x[4 * k] = w.x; x[4 * k + 1] = w.y; x[4 * k + 2] = w.z; x[4 * k + 3] = w.w;
+        }
+    }
+    sr_drain_stores();
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint32_t ok = ((uint32_t)was & 0xffffu) + 1u == gridDim.x ? 1u : 0u;
+        for (uint32_t it = 0; ok == 0u && it < a.wait_limit; it++) {
+            ok = ((uint32_t)sr_load_agent(sync) & 0xffffu) == gridDim.x ? 1u : 0u;
+            if (ok == 0u) __builtin_amdgcn_s_sleep(1);
+        }
+        if (ok == 0u) sr_store_agent(sync + 1, (unsigned long long)a.seq);
+        bc = ok;
+    }
+    __syncthreads();
+    if (bc != 0u) {
+        for (int g = tid; g < nseg; g += kSpecT) states[g] = sr_load_agent(&sums[g]);
+        __syncthreads();
+        if (seg < nseg) {
+            float before = 0.0f;
+            for (int g = lane; g < seg; g += SR_WAVE) before += states[g];
+            before = sr_wave_sum_f32(before);
+            seg_make_record<true>(x, seg, (double)before, funcs + seg, own);
+        }
+    }
+    sr_drain_stores();
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        bc = ((uint32_t)(was >> 16) & 0xffffu) + 1u == gridDim.x ? (sr_load_agent(sync + 1) == (unsigned long long)a.seq ? 2u : 1u) : 0u;
+    }
+    __syncthreads();
+    if (bc == 0u || wave != 0) return;
+    const bool alone = bc == 2u;
+    const double ud = u[kind == 0 ? pos + 1 : L];
+    const float r = __double2float_rn(ud);
+    auto load = [&](int sg, float (&xs)[SR_SEQ_RUN]) __attribute__((always_inline)) { t.run(sg, xs); };
+    int found;
+    if (kind == 1) {
+        // SampleFromDistribution (Sampler.cs:564-576) over the bonus position
+        if (alone) spec_sum_alone<true>(t, nseg, r, &found, nullptr);
+        else seg_walk_from<true, true>(load, nseg, funcs, 0.0f, r, &found, nullptr);
+        results(found >= 0 ? found : n - 1);
+        return;
+    }
+    // ResampleResidual (Sampler.cs:587-618)
+    int none;
+    const float sum = alone ? spec_sum_alone<false>(t, nseg, 0.0f, &none, states) : seg_walk_from<false, true>(load, nseg, funcs, 0.0f, 0.0f, &none, states);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (!(sum > 0.0f)) {  // sum <= 0 or NaN: a draw from p
+        t.q = nullptr;
+        spec_sum_alone<true>(t, nseg, r, &found, nullptr);
+        results(found >= 0 ? found : n - 1);
+        return;
+    }
+    const float target = __fmul_rn(r, sum);
+    float at_sum;
+    found = target > 0.0f ? seg_search_states(load, nseg, states, target, &at_sum) : -1;
+    if (found < 0) {
+        // a zero target must not stop on a zero term: the first positive one; and where rounding left the sum of the search
+        // short of the target, the last positive one
+        int edge = target <= 0.0f ? 0x7fffffff : -1;
+        for (int i = lane; i < n; i += SR_WAVE)
+            if (t.at(i) > 0.0f) {
+                edge = i;
+                if (target <= 0.0f) break;
+            }
+        found = target <= 0.0f ? sr_wave_min_i32(edge) : -sr_wave_min_i32(-edge);
+    }
+    results(found);
 }
 
 // ---- speculative verification: the accept loop of StepSampled (SpeculativeDecoder.cs:530-559) ---------
@@ -4407,6 +4535,7 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
     const int row = blockIdx.x;
     const SrRow rd = a.rows[row];
     const int n = a.vocab, L = a.n_draft;
+    if (a.reject && a.reject[row] == kSpecDone) return;
     const float* pr = a.p_all + (size_t)row * (L + 1) * (size_t)a.p_stride;
     const float* lg = a.target_logits + (size_t)row * (L + 1) * n;
     const double* u = a.uniforms + (size_t)row * a.uniforms_per_row;
@@ -4462,10 +4591,7 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
         }
         const float m1 = sl->mul1, m2 = sl->mul2;
         const double uc = u[udraws++];
-        if (true_spec && a.reject && a.reject[row] == i && a.seg_func)  // the residual row and its segments' functions are there
-            correction = resample_residual_prepared(a.resid + (size_t)row * (size_t)a.resid_stride,
-                                                    a.seg_func + (size_t)row * a.seg_stride, pd, n, uc, sm, m1, m2);
-        else if (true_spec && a.reject && a.reject[row] == i)  // the residual row is there already
+        if (true_spec && a.reject && a.reject[row] == i)  // the residual row is there already
             correction = resample_residual_stored(a.resid + (size_t)row * (size_t)a.resid_stride, pd, n, uc, sm, m1, m2);
         else
             correction = true_spec ? resample_residual_row(pd, qd, n, uc, sm, m1, m2) : draw_from_row(pd, n, uc, sm, m1, m2);
@@ -4476,9 +4602,6 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
         const float* pd = pr + (size_t)L * (size_t)a.p_stride;
         const SrFullState* sl = a.state + (size_t)row * (L + 1) + L;
         if (rd.temperature <= 0.0f) correction = row_argmax(pd, n, sm);
-        else if (a.seg_func && a.reject[row] == L)  // the scaled row and its segments' functions are there
-            correction = draw_from_prepared(a.resid + (size_t)row * (size_t)a.resid_stride, a.seg_func + (size_t)row * a.seg_stride, n,
-                                            u[udraws++], sm);
         else correction = draw_from_row(pd, n, u[udraws++], sm, sl->mul1, sl->mul2);
     }
     if (threadIdx.x == 0) {
@@ -4527,6 +4650,26 @@ __global__ __launch_bounds__(kT) void k_mtp_verify(const float* logits, int64_t 
 }
 
 #ifdef SR_TEST_HOOKS
+// The record of every segment of every row of terms (SeqSegFunc), for the binades that the approximate sums predict:
+// the sums of the segments in front (part, left by the kernel that wrote the terms) and, inside the segment, of the
+// lanes in front.  One wave per segment.
+__global__ __launch_bounds__(256) void k_seq_funcs(const float* terms, int64_t stride, int n, const double* part, SeqSegFunc* func,
+                                                   int seg_stride)
+{
+    const int row = blockIdx.y, lane = sr_lane();
+    const int seg = (int)blockIdx.x * 4 + sr_wave_id();
+    if (seg >= seg_count(n)) return;
+    const double* pr = part + (size_t)row * seg_stride;
+    double before = 0.0;
+    for (int g = lane; g < seg; g += SR_WAVE) before += pr[g];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o);
+    const float* t = terms + (size_t)row * (size_t)stride;
+    float x[SR_SEQ_RUN];
+    seq_load_run(t, ((uintptr_t)t & 15u) == 0u, seg * SR_SEG_TERMS + lane * SR_SEQ_RUN, n, x);
+    seg_make_record(x, seg, before, func + (size_t)row * seg_stride + seg);
+}
+
 __global__ __launch_bounds__(kT) void k_selftest_seqsum(const float* x, int n, float s0, float target, float* out_sum,
                                                          int* out_idx)
 {
@@ -4565,7 +4708,9 @@ __global__ __launch_bounds__(kT) void k_selftest_segwalk(const float* x, int n, 
     float s2 = s;
     if (target == target) {
         float at = 0.0f;
-        found = seg_search_states(x, n, sm.segst, target, &at);
+        found = seg_search_states([&](int seg, float (&v)[SR_SEQ_RUN]) {
+            seq_load_run(x, ((uintptr_t)x & 15u) == 0u, seg * SR_SEG_TERMS + sr_lane() * SR_SEQ_RUN, n, v);
+        }, seg_count(n), sm.segst, target, &at);
         s2 = seg_walk<true>(x, n, funcs, 0.0f, target, &found2, nullptr);
     }
     if (sr_lane() == 0) { out_sum[0] = s; out_sum[1] = s2; out_idx[0] = found; out_idx[1] = found2; }
@@ -4684,22 +4829,21 @@ hipError_t sr_launch_expand_rows(const SrRow* src, SrRow* dst, int rows, int pos
     hipLaunchKernelGGL(k_expand_rows, dim3((unsigned)((rows * positions + 255) / 256)), dim3(256), 0, st, src, dst, rows, positions);
     return hipGetLastError();
 }
-hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, hipStream_t st)
+static int seg_count_of(int n) { return (n + SR_SEG_TERMS - 1) / SR_SEG_TERMS; }
+hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, bool any_other, hipStream_t st)
 {
     if (rows <= 0) return hipSuccess;
     SrSpecArgs b = a;
-    if (!(b.resid && b.reject && b.n_draft > 0 && b.draft_probs && rows <= 65535)) {  // (rows are the grid's second dimension)
+    if (!(b.reject && b.n_draft > 0 && b.draft_probs && rows <= 65535)) {  // (rows are the grid's second dimension)
         b.resid = nullptr;
         b.reject = nullptr;
-        b.seg_func = nullptr;
+    } else if (b.seg_func) {
+        hipLaunchKernelGGL(k_spec_rows, dim3((unsigned)((seg_count_of(b.vocab) + kSpecWaves - 1) / kSpecWaves), rows), dim3(kSpecT), 0, st, b);
+        if (!any_other) return hipGetLastError();
     } else {
-        const int nseg = (b.vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
-        if (!(b.seg_func && b.seg_part && nseg <= SR_SEG_MAX && nseg <= b.seg_stride)) b.seg_func = nullptr;
+        const int nseg = seg_count_of(b.vocab);
         hipLaunchKernelGGL(k_spec_walk, dim3(rows), dim3(SR_WAVE), 0, st, b);
         hipLaunchKernelGGL(k_spec_residual, dim3((unsigned)std::min(64, (nseg + 3) / 4), rows), dim3(256), 0, st, b);
-        if (b.seg_func)
-            hipLaunchKernelGGL(k_seq_funcs, dim3((unsigned)((nseg + 3) / 4), rows), dim3(256), 0, st, b.resid, b.resid_stride, b.vocab,
-                               b.seg_part, (SeqSegFunc*)b.seg_func, b.seg_stride, b.reject);
     }
     hipLaunchKernelGGL(k_spec_verify, dim3(rows), dim3(kT), 0, st, b);
     return hipGetLastError();
@@ -4724,8 +4868,7 @@ hipError_t sr_launch_selftest_segsum(const float* x, int n, double skew, float t
 {
     const int nseg = (n + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
     hipLaunchKernelGGL(k_selftest_segpart, dim3((unsigned)((nseg + 3) / 4)), dim3(256), 0, st, x, n, skew, part);
-    hipLaunchKernelGGL(k_seq_funcs, dim3((unsigned)((nseg + 3) / 4), 1), dim3(256), 0, st, x, (int64_t)0, n, part, funcs, nseg,
-                       (const int32_t*)nullptr);
+    hipLaunchKernelGGL(k_seq_funcs, dim3((unsigned)((nseg + 3) / 4), 1), dim3(256), 0, st, x, (int64_t)0, n, part, funcs, nseg);
     hipLaunchKernelGGL(k_selftest_segwalk, dim3(1), dim3(kT), 0, st, x, n, funcs, target, out_sum, out_idx);
     return hipGetLastError();
 }

@@ -97,6 +97,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     if (++ctx->full_seq == 0u) {  // the numbers have gone round: nothing of an earlier launch may look like this one's
         SR_HIP(ctx, hipMemsetAsync(ctx->full_state.p, 0, ctx->full_state.cap, st));
         if (ctx->full_row_sync.p) SR_HIP(ctx, hipMemsetAsync(ctx->full_row_sync.p, 0, ctx->full_row_sync.cap, st));
+        if (ctx->spec_sync.p) SR_HIP(ctx, hipMemsetAsync(ctx->spec_sync.p, 0, ctx->spec_sync.cap, st));
         ctx->full_seq = 1u;
     }
     a.seq = ctx->full_seq;
@@ -530,19 +531,30 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     a.uniforms_per_row = b->upr;
     a.out_accepted = out_accepted_dev;
     a.out_tokens = out_tokens_dev;
-    a.resid_stride = ((int64_t)V + 3) & ~(int64_t)3;
-    SR_HIP(ctx, ctx->spec_resid.reserve((size_t)rows * (size_t)a.resid_stride * sizeof(float), st));
     SR_HIP(ctx, ctx->spec_reject.reserve((size_t)rows * sizeof(int32_t), st));
-    a.resid = ctx->spec_resid.as<float>();
     a.reject = ctx->spec_reject.as<int32_t>();
     a.seg_stride = (V + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
-    if (a.seg_stride <= SR_SEG_MAX) {  // (longer rows are added by their workgroups alone)
-        SR_HIP(ctx, ctx->seg_part.reserve((size_t)rows * (size_t)a.seg_stride * sizeof(double), st));
+    if (a.seg_stride <= SR_SEG_MAX) {
+        SR_HIP(ctx, ctx->seg_part.reserve((size_t)rows * (size_t)a.seg_stride * sizeof(float), st));
         SR_HIP(ctx, ctx->seg_func.reserve((size_t)rows * (size_t)a.seg_stride * sizeof(SeqSegFunc), st));
-        a.seg_part = ctx->seg_part.as<double>();
+        // (cleared when new, and when the launches' numbers have gone round: run_full)
+        SR_HIP(ctx, ctx->spec_sync.reserve((size_t)rows * SR_ROW_SYNC_STRIDE * sizeof(unsigned long long), st, true));
+        a.seg_part = ctx->seg_part.as<float>();
         a.seg_func = (SeqSegFunc*)ctx->seg_func.p;
+        a.sync = ctx->spec_sync.as<unsigned long long>();
+        a.seq = ctx->full_seq;
+        a.wait_limit = ctx->behind_wait_limit;
+    } else {  // (longer rows are added by their workgroups alone)
+        a.resid_stride = ((int64_t)V + 3) & ~(int64_t)3;
+        SR_HIP(ctx, ctx->spec_resid.reserve((size_t)rows * (size_t)a.resid_stride * sizeof(float), st));
+        a.resid = ctx->spec_resid.as<float>();
     }
-    SR_HIP(ctx, sr_launch_spec_verify(a, rows, st));
+    bool any_other = false;
+    for (int r = 0; r < rows; r++) {
+        const SrRow& d = b->h_rows[(size_t)r];
+        any_other = any_other || (d.p_min > 0.0f && d.p_min < 1.0f) || (d.flags & SR_ROW_DRAFT_FROM_LOOKUP) || !(d.temperature > 0.0f);
+    }
+    SR_HIP(ctx, sr_launch_spec_verify(a, rows, any_other, st));
     return SR_OK;
 }
 

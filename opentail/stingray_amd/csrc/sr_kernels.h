@@ -257,15 +257,19 @@ struct SrSpecArgs {
     int32_t uniforms_per_row;
     int32_t* out_accepted;       // [rows]
     int32_t* out_tokens;         // [rows][n_draft + 1]
+    int32_t* reject;             // [rows]: what k_spec_verify needs to know of the launches in front of it
+    // rows of up to SR_SEG_MAX segments (k_spec_rows), else null:
+    SeqSegFunc* seg_func;        // [rows][seg_stride]: the records of the segments of the terms that the row draws from
+    float* seg_part;             // [rows][seg_stride]: about the sum of every segment of them
+    int32_t seg_stride;
+    unsigned long long* sync;    // [row * SR_ROW_SYNC_STRIDE]: as SrFullArgs::row_sync, and behind it the last launch in which a wait ran out
+    uint32_t seq, wait_limit;
+    // ... and of more:
     float* resid;                // [rows][resid_stride]: max(0, p - q) of the row's first rejected position
     int64_t resid_stride;
-    int32_t* reject;             // [rows]: that position, or -1 (none, or a row that does not take the ratio test), or
-                                 // n_draft (every draft accepted and a bonus token to draw: resid holds the scaled row)
-    double* seg_part;            // [rows][seg_stride]: approximate sum of every SR_SEG_TERMS terms of the row of resid
-    SeqSegFunc* seg_func;        // [rows][seg_stride]: the increment functions of those segments; null: not prepared
-    int32_t seg_stride;
 };
-hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, hipStream_t st);
+// any_other: some row is not under the ratio test, or greedy
+hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, bool any_other, hipStream_t st);
 hipError_t sr_launch_expand_rows(const SrRow* src, SrRow* dst, int rows, int positions, hipStream_t st);
 hipError_t sr_launch_mtp_verify(const float* logits, int64_t stride, int n, int rows, const int* draft, float p_min,
                                 int* out_argmax, int* out_accept, float* out_prob, hipStream_t st);

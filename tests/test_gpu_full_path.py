@@ -327,6 +327,36 @@ def test_corrections_drawn_at_both_ends_of_the_residual(ctx):
             _check_spec(ctx, t, q, k, params, uu)
 
 
+@pytest.mark.parametrize("polls", [0, 2, 1 << 15])
+@pytest.mark.parametrize("V", [1023, 8_193, 70_001, 1_050_000])  # one segment; one entry in a block of its own; odd rows; longer than prepared
+def test_verification_by_one_launch_and_by_the_workgroups_that_come_last(ctx, V, polls):
+    """Rows under the ratio test are verified by one launch whose workgroups meet once; where the wait runs out, the last one adds all
+    of the row's terms.  Beside them rows of the other rule, a greedy row, an id outside the vocabulary, and a row whose p
+    and q are the same, with a first uniform of 1 that nothing accepts (the residual is empty: the draw is from p)."""
+    rows, L = (2, 1) if V > 1_000_000 else (6, 3)
+    params = [SamplingParams(), SamplingParams(Temperature=0.8, TopP=0.9), SamplingParams(Temperature=0.9, SpecDraftPMin=0.3),
+              SamplingParams(Temperature=0.0), SamplingParams(), SamplingParams()][:rows]
+    t, q, k, u = _spec_case(rows, L, V, params, V, True)
+    if rows > 2:
+        k[4, 1] = V
+        for i in range(L):
+            q[5, i] = orc.build_filtered_distribution(t[5, i], to_oracle(params[5]))
+        u[5, 0] = 1.0
+    try:
+        ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 0x80000000 | polls))
+        for _ in range(2):
+            acc, out = ctx.spec_verify(_cuda(t), _cuda(q), _cuda(k), params, u)
+            for r in range(rows):
+                if r == 4:  # (the reference throws at the id: what was accepted in front of it stands, and no correction)
+                    assert acc[r] <= 1 and (acc[r] < 1 or list(out[r]) == [k[r, 0], -1] + [-1] * (L - 1)), (acc[r], out[r])
+                    continue
+                wa, wt = orc.spec_verify_row(t[r], q[r], k[r], to_oracle(params[r]), orc.Rng(replay=u[r]))
+                assert acc[r] == wa and list(out[r][: wa + 1]) == list(wt) and np.all(out[r][wa + 1:] == -1), (r, acc[r], wa, out[r], wt)
+            u[:, 1:] = np.random.default_rng(V + polls).random((rows, L))
+    finally:
+        ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
+
+
 def test_verification_after_tokens_were_appended_to_the_batch(ctx):
     # The verifier copies the batch's row descriptors on the device: rows with penalties whose histories grew by
     # sr_batch_append_tokens (in place, no new upload) must be verified with the histories as they are now.
