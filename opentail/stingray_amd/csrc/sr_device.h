@@ -35,6 +35,14 @@ __device__ __forceinline__ float sr_max_f32(float a, float b)
 
 __device__ __forceinline__ float sr_bf16_to_f32(uint16_t h) { return sr_u2f(((uint32_t)h) << 16); }
 
+// ... of three
+__device__ __forceinline__ float sr_max3_f32(float a, float b, float c)
+{
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 // glibc expf (2^(i/32) table, cubic in double, one rounding to float) with the FMA contractions of the
 // x86-64 -mfma build: the managed sampler's MathF.Exp on Linux.  Every operation is spelled with an
 // explicitly rounded intrinsic so the compiler can neither fuse nor reorder.
@@ -85,22 +93,23 @@ __device__ __forceinline__ float sr_expf_tab(float x, const uint64_t* tab)
     e = (xb == 0xff800000u) ? 0.0f : e;
     return e;
 }
-// ... of x <= 0 or -inf, where nothing overflows and nothing is a NaN: a quarter of the instructions less
+// ... of x <= 0 or -inf, where nothing overflows and nothing is a NaN: 16 instructions instead of 30.  The product is rounded
+// once with the shift's addition, not by itself, and what underflows is taken at -104, whose value rounds to zero: for every
+// float from -0 to -130 the result is the one above, bit for bit (compared on a CPU), and from -104 down it is 0.
 __device__ __forceinline__ float sr_expf_neg(float x, const uint64_t* tab)
 {
     const double inv_ln2_n = 0x1.71547652b82fep+0 * 32.0;
     const double shift = 0x1.8p+52;
-    const double xd = (double)x;
-    double kd = __dadd_rn(__dmul_rn(inv_ln2_n, xd), shift);
-    const uint64_t ki = (uint64_t)__double_as_longlong(kd);
+    const double xd = (double)sr_max_f32(x, -104.0f);
+    double kd = __fma_rn(inv_ln2_n, xd, shift);
+    const uint32_t ki = (uint32_t)(uint64_t)__double_as_longlong(kd);
     kd = __dsub_rn(kd, shift);
     const double r = __fma_rn(inv_ln2_n, xd, -kd);
-    uint64_t t = tab[ki & 31u];
-    t += ki << (52 - 5);
+    const uint64_t t = tab[ki & 31u];
+    const uint32_t hi = (uint32_t)(t >> 32) + (ki << (52 - 5 - 32));  // (the low word takes nothing)
     const double zz = __fma_rn(0x1.c6af84b912394p-5 / (32.0 * 32.0 * 32.0), r, 0x1.ebfce50fac4f3p-3 / (32.0 * 32.0));
     const double y = __fma_rn(zz, __dmul_rn(r, r), __fma_rn(0x1.62e42ff0c52d6p-1 / 32.0, r, 1.0));
-    const float e = __double2float_rn(__dmul_rn(y, __longlong_as_double((long long)t)));
-    return x < -0x1.9fe368p6f ? 0.0f : e;
+    return __double2float_rn(__dmul_rn(y, __hiloint2double((int)hi, (int)(uint32_t)t)));
 }
 __device__ __forceinline__ float sr_expf(float x) { return sr_expf_tab(x, sr_exp2f_tab); }
 

@@ -525,9 +525,12 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
     };
     {
         // a segment without a term (masked, or cut) changes no sum whatever its binade
-        float any = x[0];
+        float any = seg_sum;
+        if (seg_sum < 0.0f) {
+            any = x[0];
 #pragma unroll
-        for (int j = 1; j < SR_SEQ_RUN; j++) any = sr_max_f32(any, x[j]);
+            for (int j = 1; j < SR_SEQ_RUN; j++) any = sr_max_f32(any, x[j]);
+        }
         if (__ballot(any > 0.0f) == 0ull) {
             if (lane == 0) put(0, 0u, 0u, 0u, SR_SEG_ZERO);
             return;
@@ -1366,8 +1369,13 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
             for (int k = 0; k < K; k++) {
                 const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * E;
                 raw[k] = sr_load16<ES>(src.rowp + (size_t)i0 * ES);
-                keep[k] = 0xffffffffu;
-                if (src.mrow) keep[k] = src.mrow[i0 >> 5] >> (i0 & 31);
+            }
+            if (src.mrow) {
+#pragma unroll
+                for (int k = 0; k < K; k++) {
+                    const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * E;
+                    keep[k] = src.mrow[i0 >> 5] >> (i0 & 31);
+                }
             }
 #pragma unroll
             for (int k = 0; k < K; k++) {
@@ -1382,11 +1390,18 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
                         xv[(2 * q + 1) % E] = sr_u2f(r[q] & 0xffff0000u);
                     }
                 }
+            }
+            // (each behind one test for the whole row: as selections per element they were a seventh of the pass's instructions
+            // in rows that have neither)
+            if (src.mrow) {
 #pragma unroll
-                for (int q = 0; q < E; q++) {
-                    const float v = ((keep[k] >> q) & 1u) ? xv[q] : SR_NEG_INF;
-                    xv[q] = src.scale ? __fmul_rn(v, src.inv_temp) : v;
-                }
+                for (int k = 0; k < K; k++)
+#pragma unroll
+                    for (int q = 0; q < E; q++) x[k * E + q] = ((keep[k] >> q) & 1u) ? x[k * E + q] : SR_NEG_INF;
+            }
+            if (src.scale) {
+#pragma unroll
+                for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = __fmul_rn(x[j], src.inv_temp);
             }
         } else {
             float4 rw[K * E / 4];
@@ -1509,10 +1524,11 @@ constexpr uint32_t kKeyInf = 0xff800000u;  // +inf as an ordered key; above it: 
 // a segment's largest value as an ordered key; 0xffffffff = it holds a NaN (which propagates: TensorPrimitives.Max)
 __device__ __forceinline__ uint32_t seg_max_key(const float (&x)[SR_SEQ_RUN])
 {
-    float m = x[0];
+    static_assert(SR_SEQ_RUN % 2 == 0, "the first, then two at a time, then the last");
+    float m = sr_max_f32(x[0], x[SR_SEQ_RUN - 1]);
     bool nan = false;
 #pragma unroll
-    for (int j = 1; j < SR_SEQ_RUN; j++) m = sr_max_f32(m, x[j]);
+    for (int j = 1; j + 1 < SR_SEQ_RUN; j += 2) m = sr_max3_f32(m, x[j], x[j + 1]);
 #pragma unroll
     for (int j = 0; j < SR_SEQ_RUN; j += 2) nan = nan || __builtin_isunordered(x[j], x[j + 1]);
     return nan ? 0xffffffffu : sr_okey(m);
