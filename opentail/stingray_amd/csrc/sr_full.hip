@@ -1585,7 +1585,7 @@ __device__ __forceinline__ uint32_t min_p_list_from(const SrRow& rd)
 }
 
 template <int ES, int kW, int kS>
-__global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 4 : 6) void k_full_softmax_seg(SrFullArgs a)
+__global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_seg(SrFullArgs a)
 {
     constexpr int kThreads = kW * SR_WAVE;
     constexpr int E = 16 / ES, K = SR_SEG_TERMS / (SR_WAVE * E);
