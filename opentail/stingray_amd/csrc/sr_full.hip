@@ -4846,7 +4846,7 @@ hipError_t sr_launch_expand_rows(const SrRow* src, SrRow* dst, int rows, int pos
     return hipGetLastError();
 }
 static int seg_count_of(int n) { return (n + SR_SEG_TERMS - 1) / SR_SEG_TERMS; }
-hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, bool any_other, hipStream_t st)
+hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, hipStream_t st)
 {
     if (rows <= 0) return hipSuccess;
     SrSpecArgs b = a;
@@ -4855,7 +4855,7 @@ hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, bool any_other, 
         b.reject = nullptr;
     } else if (b.seg_func) {
         hipLaunchKernelGGL(k_spec_rows, dim3((unsigned)((seg_count_of(b.vocab) + kSpecWaves - 1) / kSpecWaves), rows), dim3(kSpecT), 0, st, b);
-        if (!any_other) return hipGetLastError();
+        if (!b.any_other) return hipGetLastError();
     } else {
         const int nseg = seg_count_of(b.vocab);
         hipLaunchKernelGGL(k_spec_walk, dim3(rows), dim3(SR_WAVE), 0, st, b);

@@ -549,12 +549,11 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
         SR_HIP(ctx, ctx->spec_resid.reserve((size_t)rows * (size_t)a.resid_stride * sizeof(float), st));
         a.resid = ctx->spec_resid.as<float>();
     }
-    bool any_other = false;
     for (int r = 0; r < rows; r++) {
         const SrRow& d = b->h_rows[(size_t)r];
-        any_other = any_other || (d.p_min > 0.0f && d.p_min < 1.0f) || (d.flags & SR_ROW_DRAFT_FROM_LOOKUP) || !(d.temperature > 0.0f);
+        if ((d.p_min > 0.0f && d.p_min < 1.0f) || (d.flags & SR_ROW_DRAFT_FROM_LOOKUP) || !(d.temperature > 0.0f)) a.any_other = 1;
     }
-    SR_HIP(ctx, sr_launch_spec_verify(a, rows, any_other, st));
+    SR_HIP(ctx, sr_launch_spec_verify(a, rows, st));
     return SR_OK;
 }
 

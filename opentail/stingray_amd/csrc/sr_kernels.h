@@ -264,12 +264,12 @@ struct SrSpecArgs {
     int32_t seg_stride;
     unsigned long long* sync;    // [row * SR_ROW_SYNC_STRIDE]: as SrFullArgs::row_sync, and behind it the last launch in which a wait ran out
     uint32_t seq, wait_limit;
+    int32_t any_other;           // some row is not under the ratio test, or greedy: k_spec_verify follows
     // ... and of more:
     float* resid;                // [rows][resid_stride]: max(0, p - q) of the row's first rejected position
     int64_t resid_stride;
 };
-// any_other: some row is not under the ratio test, or greedy
-hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, bool any_other, hipStream_t st);
+hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, hipStream_t st);
 hipError_t sr_launch_expand_rows(const SrRow* src, SrRow* dst, int rows, int positions, hipStream_t st);
 hipError_t sr_launch_mtp_verify(const float* logits, int64_t stride, int n, int rows, const int* draft, float p_min,
                                 int* out_argmax, int* out_accept, float* out_prob, hipStream_t st);
