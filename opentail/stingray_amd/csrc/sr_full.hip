@@ -1584,6 +1584,63 @@ __device__ __forceinline__ uint32_t min_p_list_from(const SrRow& rd)
     return rd.min_p >= 1e-30f ? sr_f2u(__fmul_rn(rd.min_p, 1.0f - 2.0f * SR_AMBIG_REL - 1e-6f)) : 0u;
 }
 
+// A greedy row that rides along (SrFullArgs::n_greedy): the largest of its masked logits, the first by index among equals, NaN left
+// out -- what the selection kernel finds for such a row.  The row's word for it is zero between launches: whoever counts in last
+// takes the result and puts the zero back.
+template <int ES, int kW, int kS>
+__device__ __forceinline__ void seg_greedy(const SrFullArgs& a, const SrRow& rd, int slot, int row, unsigned long long* of_wave)
+{
+    const int lane = sr_lane(), wave = sr_wave_id(), n = a.vocab, nseg = seg_count(n);
+    SegSource<ES> src;
+    src.rowp = (const char*)a.logits + (size_t)row * (size_t)a.row_stride * ES;
+    src.mrow = (rd.mask_row >= 0) ? a.mask + (size_t)rd.mask_row * a.mask_stride : nullptr;
+    src.w = nullptr;
+    src.scale = false;
+    src.inv_temp = 1.0f;
+    const int seg0 = (int)blockIdx.x * (kW * kS) + wave;
+    float t[kS][SR_SEQ_RUN];
+#pragma unroll
+    for (int s = 0; s < kS; s++)
+        if (seg0 + s * kW < nseg) seg_load_logits<ES>(src, seg0 + s * kW, lane, n, t[s]);
+    unsigned long long best = 0ull;  // ordered key << 32 | ~index; 0: nothing above -inf
+#pragma unroll
+    for (int s = 0; s < kS; s++) {
+        const int seg = seg0 + s * kW;
+        if (seg >= nseg) continue;
+        float m = sr_max_f32(t[s][0], t[s][SR_SEQ_RUN - 1]);
+#pragma unroll
+        for (int j = 1; j + 1 < SR_SEQ_RUN; j += 2) m = sr_max3_f32(m, t[s][j], t[s][j + 1]);
+        const uint32_t k = sr_wave_max_u32(m == m ? sr_okey(m) : 0u);
+        if (k <= 0x007fffffu || k < (uint32_t)(best >> 32)) continue;
+        const float mk = sr_okey_inv(k);
+        int at = 0x7fffffff;
+#pragma unroll
+        for (int j = SR_SEQ_RUN - 1; j >= 0; j--)
+            if (t[s][j] == mk) at = min(at, seg_elem<ES>(seg, lane, j));
+        at = sr_wave_min_i32(at);
+        const unsigned long long found = ((unsigned long long)k << 32) | (unsigned long long)(0xffffffffu - (uint32_t)at);
+        best = found > best ? found : best;
+    }
+    if (lane == 0) of_wave[wave] = best;
+    sr_barrier_lds();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 0; w < kW; w++) best = of_wave[w] > best ? of_wave[w] : best;
+        // (each atomic's returned value is waited for before the next is issued: whoever counts in last finds the result complete)
+        unsigned long long* const sync = a.row_sync + (size_t)slot * SR_ROW_SYNC_STRIDE;
+        const unsigned long long s0 = __hip_atomic_fetch_max(sync, (unsigned long long)a.seq << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned long long s1 = __hip_atomic_fetch_max(sync + 2, best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("" : : "v"(s0), "v"(s1) : "memory");
+        const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (((uint32_t)was & 0xffffu) + 1u == gridDim.x) {
+            const unsigned long long r = __hip_atomic_exchange(sync + 2, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // (nothing above -inf: every masked logit is -inf and the first index wins)
+            a.out_tokens[row] = r != 0ull ? (int)(0xffffffffu - (uint32_t)r) : 0;
+            if (a.out_flags) a.out_flags[row] = SR_KFLAG_GREEDY | (r != 0ull ? 0u : SR_KFLAG_DEGENERATE);
+        }
+    }
+}
+
 template <int ES, int kW, int kS>
 __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_seg(SrFullArgs a)
 {
@@ -1593,7 +1650,6 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     const int slot = blockIdx.y, lane = sr_lane(), wave = sr_wave_id();
     const int row = a.row_list[slot];
     const SrRow rd = a.rows[row];
-    if (rd.temperature <= 0.0f) return;  // greedy rows keep their logits
     __shared__ uint64_t tab[32];  // the expf table: a lookup per element from global memory is a long dependent load
     // a wave's segment on its way from the order of the loads to 16 terms a lane: a lane's 16 terms lie together, 16
     // bytes apart from the next lane's, so that neither the stores nor the loads of 16 bytes a lane collide on a bank
@@ -1610,6 +1666,10 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     constexpr int kHitCap = 256;
     __shared__ unsigned long long hits[kHitCap];
     __shared__ uint32_t n_hits;
+    if (rd.temperature <= 0.0f) {  // greedy rows keep their logits where a distribution is asked for
+        if (a.mode == 0) seg_greedy<ES, kW, kS>(a, rd, slot, row, hits);
+        return;
+    }
     const int n = a.vocab, nseg = seg_count(n);
     SrFullState* st = a.state + slot;
     unsigned long long* sync = a.row_sync + (size_t)slot * SR_ROW_SYNC_STRIDE;
@@ -4755,10 +4815,10 @@ hipError_t sr_launch_full_prep(const SrFullArgs& a, int n_rows, hipStream_t st)
         // fp32: 33 -> 26 us, 64 of 151,936: 55 -> 36).  Below, one and two measure the same, and one starts sooner (a row
         // of 151,936, whole step: 56.6 against 58.9 us).  Four for the verifier's large launches, whose waves keep nothing
         // else in registers (144 rows of 262,144: 98 -> 92 us; 36 rows: 119.6 -> 121.6 a call).
-        const long long segs = (long long)a.n_sampled * nseg;
+        const long long segs = (long long)(a.n_sampled + a.n_greedy) * nseg;
         const bool four = a.lazy_scale && a.dtype != 1 && segs > 12288, two = segs > 3072;
         const int per_group = 4 * (four ? 4 : two ? 2 : 1);
-        dim3 fgrid((unsigned)((nseg + per_group - 1) / per_group), n_rows);
+        dim3 fgrid((unsigned)((nseg + per_group - 1) / per_group), n_rows + a.n_greedy);
         if (a.dtype == 1) {
             if (two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2>), fgrid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 1>), fgrid, dim3(256), 0, st, a);

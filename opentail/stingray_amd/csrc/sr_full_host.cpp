@@ -12,7 +12,7 @@ namespace {
 //   mode 0: work rows live in ctx scratch, tokens out.   mode 1/2: work rows ARE the caller's probs rows.
 int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows, bool any_top_p, const void* logits_dev,
              int dtype, int64_t row_stride, int mode, float* probs_dev, int64_t probs_stride, int32_t* out_tokens_dev,
-             uint32_t* out_flags_dev, bool lazy_scale = false, const std::vector<SrRow>* host_rows = nullptr)
+             uint32_t* out_flags_dev, bool lazy_scale = false, const std::vector<SrRow>* host_rows = nullptr, int n_greedy = 0)
 {
     if (n_rows <= 0) return SR_OK;
     hipStream_t st = ctx->stream;
@@ -28,6 +28,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     a.mask = sr_batch_mask_ptr(b);
     a.mask_stride = sr_batch_mask_stride(b);
     a.mode = mode;
+    a.n_greedy = n_greedy;  // (a further n_greedy rows of the list: they need nothing of what follows but a meeting point)
     a.prof = ctx->prof;
     if (mode == 0) {
         const int64_t ws = (vocab + 3) & ~3;
@@ -127,7 +128,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             SR_HIP(ctx, ctx->full_seg_sum.reserve(segs * sizeof(float), st));
             SR_HIP(ctx, ctx->full_seg_cnt.reserve(segs * sizeof(uint32_t), st));
             SR_HIP(ctx, ctx->full_mass.reserve((size_t)n_rows * 256 * sizeof(float), st, true));
-            SR_HIP(ctx, ctx->full_row_sync.reserve((size_t)n_rows * SR_ROW_SYNC_STRIDE * sizeof(unsigned long long), st, true));
+            SR_HIP(ctx, ctx->full_row_sync.reserve((size_t)(n_rows + n_greedy) * SR_ROW_SYNC_STRIDE * sizeof(unsigned long long), st, true));
             a.row_sync = ctx->full_row_sync.as<unsigned long long>();
             a.seg_func = (SeqSegFunc*)ctx->full_seg_func.p;
             a.seg_sum = ctx->full_seg_sum.as<float>();
@@ -212,8 +213,8 @@ int sr_full_rows_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, 
 {
     bool any_top_p = false;
     for (int32_t r : b->h_full_list) any_top_p = any_top_p || row_uses_top_p(b->h_rows[(size_t)r]);
-    return run_full(ctx, b, b->d_full_list.as<int32_t>(), (int)b->h_full_list.size(), any_top_p, logits_dev, dtype,
-                    row_stride, 0, nullptr, 0, out_tokens_dev, out_flags_dev);
+    return run_full(ctx, b, b->d_full_list.as<int32_t>(), (int)b->h_full_list.size() - b->full_greedy, any_top_p, logits_dev, dtype,
+                    row_stride, 0, nullptr, 0, out_tokens_dev, out_flags_dev, false, nullptr, b->full_greedy);
 }
 
 // SampleTopK (Sampler.cs:216-357) for rows whose k + history length exceeds what the selection kernel's row tail

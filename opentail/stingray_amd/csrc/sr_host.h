@@ -331,6 +331,7 @@ struct sr_batch {
     int32_t rows = 0, vocab = 0, upr = 0;
     std::vector<SrRow> h_rows;
     std::vector<SrEdit> h_edits;
+    int32_t full_greedy = 0;           // greedy rows at the end of h_full_list
     std::vector<int32_t> h_sel_list;   // rows on the selection kernel: TOPK and plain GREEDY
     std::vector<int32_t> h_full_list;  // rows on the full-vocabulary path
     std::vector<int32_t> h_sched;     // the selection kernel's programs and chunk items (host copy, read by an async upload)

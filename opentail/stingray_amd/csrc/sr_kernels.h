@@ -153,7 +153,8 @@ static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // SrFullArgs::row_sync, a word per row (rows 256 bytes apart: every workgroup of a row adds to its word and polls it):
 // launch number << 32 | workgroups of k_full_softmax_seg at the second meeting point << 16 | at the first.  The number is
 // put in by an atomic maximum before the first count of a launch, so nothing clears the words.  The word behind it counts the
-// workgroups of k_prepared_row the same way; k_full_row, which leaves the row to them, starts it.
+// workgroups of k_prepared_row the same way; k_full_row, which leaves the row to them, starts it.  The third one holds what the
+// workgroups of a greedy row have found so far (zero between launches).
 #define SR_ROW_SYNC_STRIDE 32
 
 struct SeqSegFunc;
@@ -202,6 +203,7 @@ struct SrFullArgs {
     int32_t prepared;              // the launches behind k_full_row follow: it may leave rows to the whole device
     int32_t finish_most;           // members up to which k_full_row normalises and draws by itself
     uint32_t seq;                  // the launch's number (never 0): see SrFullState::maxkey
+    int32_t n_greedy;              // greedy rows behind the others in row_list, whose token k_full_softmax_seg finds (mode 0)
     int32_t n_sampled;             // rows of the launch with a temperature above 0 (greedy rows leave the passes at once)
     int32_t any_edits;             // some row of the launch has edits for k_full_edits (else it is not launched)
     int32_t edits_in_pass;         // seg_func is set: sampled rows with up to SR_FULL_EDIT_VALUES edits keep no adjusted copy and

@@ -852,6 +852,50 @@ def test_workgroups_that_stop_waiting_leave_a_prepared_row_to_the_last_one(ctx, 
         ctx._check(H.sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
 
 
+@pytest.mark.parametrize("vocab", [4096, 4097, 40_968, 151_937])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_greedy_rows_that_ride_along_with_the_full_path(ctx, vocab, bf16):
+    """Greedy rows beside rows on the full path: ties (the first index), the largest logit in the last place, masks down to one
+    token and to none, rows of -inf, +inf and NaN (left out), -0 and +0; the same batch again, with other masks, and alone."""
+    import torch
+
+    rng = np.random.default_rng(vocab + bf16)
+    rows = 10
+    params = [SamplingParams(Temperature=0.9, TopP=0.9) if r % 5 == 0 else SamplingParams(Temperature=0.0) for r in range(rows)]
+    x = rng.normal(0, 2.0, (rows, vocab)).astype(np.float32)
+    x[1, [vocab // 3, vocab // 2, vocab - 1]] = 30.0
+    x[2, vocab - 1] = 40.0
+    x[3] = NEG_INF
+    x[4] = np.where(rng.random(vocab) < 0.5, np.float32(-0.0), np.float32(0.0))
+    x[6, vocab - 2] = np.inf
+    allowed = rng.random((rows, vocab)) < 0.3
+    allowed[7] = False
+    allowed[8] = False
+    allowed[8, vocab - 1] = True
+    active = np.array([0, 1, 0, 1, 0, 1, 0, 1, 1, 0], dtype=np.uint8)
+    if bf16:
+        bits = synthetic.to_bf16_bits(x)
+        x = synthetic.bf16_bits_to_f32(bits)
+        dev = torch.from_numpy(bits.view(np.int16)).view(torch.bfloat16).cuda()
+    else:
+        dev = _cuda(x)
+    for mask, act in ((pack_allow_mask(allowed), active), (None, None), (pack_allow_mask(~allowed), np.ones(rows, np.uint8))):
+        u = rng.random(rows)
+        got, flags = ctx.sample_batch(dev, params, u, mask, act, return_flags=True)
+        want = oracle_tokens(x, params, u, mask, act)
+        assert np.array_equal(got, want), (got, want)
+        alone = np.array([r for r in range(rows) if r % 5])  # (no row on the full path: the selection kernel)
+        m, a = (None, None) if mask is None else (mask[alone], act[alone])
+        got1, flags1 = ctx.sample_batch(dev[alone], [params[r] for r in alone], u[alone], m, a, return_flags=True)
+        assert np.array_equal(got1, got[alone]) and np.array_equal(flags1, flags[alone]), (got1, got[alone], flags1, flags[alone])
+    y = x.copy()  # NaN: left out by both
+    y[[1, 9], 5] = np.nan
+    nan_dev = _cuda(y) if not bf16 else torch.from_numpy(y).cuda().to(torch.bfloat16)
+    u = rng.random(rows)
+    both, one = ctx.sample_batch(nan_dev, params, u), ctx.sample_batch(nan_dev[[1, 9]], [params[1], params[9]], u[[1, 9]])
+    assert list(one) == [both[1], both[9]]
+
+
 def test_edits_crowded_into_a_few_segments_of_a_long_row(ctx):
     """The pass over long rows applies the edits of a sampled row where it loads the row: a workgroup lists the edits
     that fall into its segments (room for 256) and goes through the row's whole edit list when there are more.  Rows
