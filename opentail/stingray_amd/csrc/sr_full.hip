@@ -2003,9 +2003,10 @@ __device__ __forceinline__ int draw_from_row(const float* p, int n, double u, Fu
 struct NoFill {
     __device__ __forceinline__ void operator()(int, int) const {}
 };
+__device__ __forceinline__ int list_layout(int i) { return (i & ~1023) | ((i & 15) << 6) | ((i >> 4) & 63); }
 template <typename Fill = NoFill>
 __device__ __forceinline__ void finish_from_ordered_list(const SrFullArgs& a, float* p, int n, int m, int row, FullSmem& sm,
-                                                         Fill fill = Fill(), int cap = kSmall)
+                                                         Fill fill = Fill(), int cap = kSmall, bool laid_out = false)
 {
     // (cap: what a list that is in shared memory already may hold -- kSmall, or 2 kSmall where the launch gave the
     // workgroup the room: the list then runs on from sm.sortbuf through the two arrays behind it)
@@ -2019,7 +2020,8 @@ __device__ __forceinline__ void finish_from_ordered_list(const SrFullArgs& a, fl
     // entries of the other chains as zeros.
     // A lane's sixteen consecutive entries would all lie in the same LDS banks as every other lane's: inside each
     // thousand entries the list is laid out anew, entry 16 l + j at place 64 j + l.
-    auto place_of = [](int i) -> int { return (i & ~1023) | ((i & 15) << 6) | ((i >> 4) & 63); };
+    // (laid_out: the caller has put its list there that way)
+    auto place_of = [](int i) -> int { return list_layout(i); };
     auto lay_out = [&]() __attribute__((always_inline)) {
         static_assert(kSmall == 4 * kT, "four entries per thread, or eight");
         unsigned long long t[kPerT];
@@ -2087,7 +2089,7 @@ __device__ __forceinline__ void finish_from_ordered_list(const SrFullArgs& a, fl
         return;
     }
     float sc = 0.0f;
-    if (kResident) lay_out();
+    if (kResident && !laid_out) lay_out();
     const int step = kResident ? cap : kSmall;  // (a resident list is one block)
     for (int first = 0; first < m; first += step) {
         const int cnt = min(step, m - first);
@@ -2814,10 +2816,19 @@ __device__ __forceinline__ void row_deferred(const SrFullArgs& a, SrFullState* s
     }
 }
 
+// kPer: most entries of a thread.  (One function for every length spent a microsecond a step on entries that are not there.)
+// A list of up to kT entries has its indices in list_ids(sm), in the list's order.
+__device__ __forceinline__ uint32_t* list_ids(FullSmem& sm) { return sm.tags + (kSmall - kT); }
+// an entry of e in (0, 1] in whole units of 2^-40
+__device__ __forceinline__ unsigned long long e_units(uint32_t ebits)
+{
+    return ((unsigned long long)((ebits & 0x7fffffu) | 0x800000u) << 17) >> min(127u - (ebits >> 23), 63u);
+}
+template <int kPer>
 __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& rd, SrFullState* st, float* p, int n, int slot, int row,
                                              bool do_scale, float inv, int N, FullSmem& sm, uint32_t* more)
 {
-    constexpr int kPer = SR_LIST_CAP_BIG / kT;  // most entries of a thread
+    constexpr bool kOne = kPer == 1;
     const int tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f, use_min_p = rd.min_p > 0.0f;
     const int nseg = seg_count(n);
@@ -2830,11 +2841,14 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     static_assert(SR_LIST_GROUPS_BIG * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags) &&
                   (SR_LIST_GROUPS_SMALL + SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16) * 4 <=
                       sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags), "the tables fit the three arrays");
+    static_assert((2 * kT + SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16) * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags) - kT * 4,
+                  "... and those of a list with its indices leave them alone");
     // (behind the barrier that follows the gathering)
     // A thread takes 2^sh consecutive entries, as few as the list's length allows (always 16: a list of 1,000 kept one wave
     // busy, 12 us).
     int sh = 0;
-    while ((kT << sh) < N) sh++;
+    if (!kOne)
+        while ((kT << sh) < N) sh++;
     const int per = 1 << sh;
     const int G = min(more ? SR_LIST_GROUPS_BIG : SR_LIST_GROUPS_SMALL, kT << (sh + 1));  // groups: two to an entry, where there is room
     const int i0 = tid << sh;
@@ -2844,43 +2858,60 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     for (int r = 0; r < kPer; r++) ev[r] = r < mine ? grp[list_place(i0 + r)] : 0u;
     auto prob = [&](uint32_t ebits) -> float { return do_scale ? __fmul_rn(sr_u2f(ebits), inv) : sr_u2f(ebits); };
 
-    // Sorted by value: groups of equal width in the bit patterns, counted, placed, and every value ranked inside its group -- a group of one value (the equal logits of a coarse grid) needs no ranks and is
-    // told by its neighbours.  (4,096 groups with their extremes counted along: 12 - 20 us for 14,000 entries, most of it the
-    // longest group of every wave looked through 16 times.)
-    for (int i = tid; i < G; i += kT) cnt[i] = 0u;
-    if (tid == 0) sm.bc[12] = 0u;
-    __syncthreads();
-    const uint32_t span = 0x3f800000u - min(from, 0x3f800000u);
-    int gshift = 0;
-    while ((span >> gshift) >= (uint32_t)G) gshift++;
-    auto group_of = [&](uint32_t v) -> uint32_t { return min((0x3f800000u - v) >> gshift, (uint32_t)(G - 1)); };
-#pragma unroll
-    for (int r = 0; r < kPer; r++)
-        if (r < mine) atomicAdd(&cnt[group_of(ev[r])], 1u);
-    __syncthreads();
-    {
-        // a wave's share of the groups, 64 at a time: the sums inside the wave, then what stands in front of it
-        const int g0 = wave * (G / kW);
-        int in_wave = 0;
-        for (int g = g0; g < g0 + G / kW; g += SR_WAVE) {
-            const int c = (int)cnt[g + lane];
-            const int incl = sr_wave_incl_scan_i32(c);
-            cnt[g + lane] = (uint32_t)(in_wave + incl - c);
-            in_wave += __builtin_amdgcn_readlane(incl, SR_WAVE - 1);
+    if (kOne && N <= kT / 4) {
+        // A short list: every entry against every other, four threads to an entry (lists of 80 to 140: 1.5 us, 6 by groups)
+        const int e = tid >> 2;
+        const uint32_t v = e < N ? grp[list_place(e)] : 0u;
+        int rank = 0;
+#pragma unroll 8
+        for (int j = tid & 3; j < N; j += 4) {
+            const uint32_t o = grp[list_place(j)];
+            rank += (o > v) | ((o == v) & (j < e)) ? 1 : 0;
         }
-        if (lane == 0) sm.redi[wave] = in_wave;
+        rank += (int)sr_dpp_u32<kDppXor1>((uint32_t)rank);
+        rank += (int)sr_dpp_u32<kDppXor2>((uint32_t)rank);
         __syncthreads();
-        int before = 0;
+        if (e < N && (tid & 3) == 0) grp[list_place(rank)] = v;
+    } else {
+        // Sorted by value: groups of equal width in the bit patterns, counted, placed, and every value ranked inside its group -- a group of one value (the equal logits of a coarse grid) needs no ranks and is
+        // told by its neighbours.  (4,096 groups with their extremes counted along: 12 - 20 us for 14,000 entries, most of it the
+        // longest group of every wave looked through 16 times.)
+        for (int i = tid; i < G; i += kT) cnt[i] = 0u;
+        if (tid == 0) sm.bc[12] = 0u;
+        __syncthreads();
+        const uint32_t span = 0x3f800000u - min(from, 0x3f800000u);
+        int gshift = 0;
+        while ((span >> gshift) >= (uint32_t)G) gshift++;
+        auto group_of = [&](uint32_t v) -> uint32_t { return min((0x3f800000u - v) >> gshift, (uint32_t)(G - 1)); };
 #pragma unroll
-        for (int w = 0; w < kW; w++) before += w < wave ? sm.redi[w] : 0;
-        for (int g = g0; g < g0 + G / kW; g += SR_WAVE) cnt[g + lane] += (uint32_t)before;
-    }
-    __syncthreads();
+        for (int r = 0; r < kPer; r++)
+            if (r < mine) atomicAdd(&cnt[group_of(ev[r])], 1u);
+        __syncthreads();
+        {
+            // a wave's share of the groups, 64 at a time: the sums inside the wave, then what stands in front of it
+            const int g0 = wave * (G / kW);
+            int in_wave = 0;
+            for (int g = g0; g < g0 + G / kW; g += SR_WAVE) {
+                const int c = (int)cnt[g + lane];
+                const int incl = sr_wave_incl_scan_i32(c);
+                cnt[g + lane] = (uint32_t)(in_wave + incl - c);
+                in_wave += __builtin_amdgcn_readlane(incl, SR_WAVE - 1);
+            }
+            if (lane == 0) sm.redi[wave] = in_wave;
+            __syncthreads();
+            int before = 0;
 #pragma unroll
-    for (int r = 0; r < kPer; r++)
-        if (r < mine) grp[list_place((int)atomicAdd(&cnt[group_of(ev[r])], 1u))] = ev[r];
-    __syncthreads();  // cnt[g] is now where group g ends
-    {
+            for (int w = 0; w < kW; w++) before += w < wave ? sm.redi[w] : 0;
+            for (int g = g0; g < g0 + G / kW; g += SR_WAVE) cnt[g + lane] += (uint32_t)before;
+        }
+        __syncthreads();
+        uint32_t at[kPer];  // (all places are asked for before the first is used)
+#pragma unroll
+        for (int r = 0; r < kPer; r++) at[r] = r < mine ? atomicAdd(&cnt[group_of(ev[r])], 1u) : 0u;
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if (r < mine) grp[list_place((int)at[r])] = ev[r];
+        __syncthreads();  // cnt[g] is now where group g ends
         constexpr uint32_t kMixed = 0x80000000u;  // (of cnt: the group holds more than one value)
         uint32_t v[kPer];
         uint32_t last = (mine > 0 && i0 > 0) ? grp[list_place(i0 - 1)] : 0u;
@@ -2892,23 +2923,24 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
             last = v[r];
         }
         __syncthreads();
+        uint32_t ce[kPer];
+#pragma unroll
+        for (int r = 0; r < kPer; r++) ce[r] = r < mine ? cnt[group_of(v[r])] : 0u;
         int rank[kPer];
 #pragma unroll
         for (int r = 0; r < kPer; r++) {
             rank[r] = i0 + r;
-            if (r < mine) {
+            if (ce[r] & kMixed) {
                 const int i = i0 + r;
-                const uint32_t g = group_of(v[r]), ce = cnt[g];
-                if (ce & kMixed) {
-                    const int b = g > 0u ? (int)(cnt[g - 1u] & ~kMixed) : 0, e = (int)(ce & ~kMixed);
-                    if (e - b > 128) sm.bc[12] = 1u;
-                    int k = b;
-                    for (int j = b; j < min(e, b + 128); j++) {
-                        const uint32_t o = grp[list_place(j)];
-                        k += (o > v[r] || (o == v[r] && j < i)) ? 1 : 0;
-                    }
-                    rank[r] = k;
+                const uint32_t g = group_of(v[r]);
+                const int b = g > 0u ? (int)(cnt[g - 1u] & ~kMixed) : 0, e = (int)(ce[r] & ~kMixed);
+                if (e - b > 128) sm.bc[12] = 1u;
+                int k = b;
+                for (int j = b; j < min(e, b + 128); j++) {
+                    const uint32_t o = grp[list_place(j)];
+                    k += (o > v[r] || (o == v[r] && j < i)) ? 1 : 0;
                 }
+                rank[r] = k;
             }
         }
         __syncthreads();
@@ -2935,32 +2967,21 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     FPROF(a, slot, 11);
     int found = -1;
     if (use_top_p) {
-        if (ns <= SR_WAVE) {
-            // a handful of survivors: one thread adds them the way the scalar loop does
-            if (tid == 0) {
-                float s = 0.0f;
-                int f = -1;
-                for (int i = 0; i < ns && f < 0; i++) {
-                    s = __fadd_rn(s, prob(grp[list_place(i)]));
-                    if (s >= rd.top_p) f = i;
-                }
-                sm.segbc[1] = (uint32_t)f;
-                sm.segbc[2] = sr_f2u(s);
-            }
-            __syncthreads();
-            found = (int)sm.segbc[1];
-        } else if (ns <= 2 * SR_SEG_TERMS) {
-            // up to two thousand: one wave, without the block-wide steps
+        if (kOne || ns <= 6 * SR_SEG_TERMS) {
+            // by one wave, without the block-wide steps, a thousand in 0.9 us (by the workgroup: 6 us for 3,000 to 5,000)
             if (wave == 0) {
                 float s = 0.0f;
                 int f = -1;
-                for (int b0 = 0; b0 < ns && f < 0; b0 += SR_SEG_TERMS) {
-                    float x[SR_SEQ_RUN];
+                auto fetch = [&](int b0, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
 #pragma unroll
                     for (int j = 0; j < SR_SEQ_RUN; j++) {
                         const int i = b0 + lane * SR_SEQ_RUN + j;
                         x[j] = i < ns ? prob(grp[list_place(i)]) : 0.0f;
                     }
+                };
+                for (int b0 = 0; b0 < ns && f < 0; b0 += SR_SEG_TERMS) {
+                    float x[SR_SEQ_RUN];
+                    fetch(b0, x);
                     int at;
                     s = sr_seq_wave<SR_SEQ_RUN, true>(x, s, rd.top_p, &at);
                     if (at >= 0) f = b0 + at;
@@ -2988,60 +3009,79 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
             }
         }
     }
-    const int cutoff = found >= 0 ? found + 1 : ns;
+    const int cutoff = found >= 0 ? found + 1 : ns, m = cutoff;
     const float ycut = prob(grp[list_place(cutoff - 1)]);
-    // Members: everything above the value at the cut, and of the entries equal to it the first ones by index.
-    int gt = 0, eq = 0;
-#pragma unroll
-    for (int r = 0; r < kPer; r++)
-        if (r < mine) {
-            const float y = prob(ev[r]);
-            gt += y > ycut ? 1 : 0;
-            eq += y == ycut ? 1 : 0;
-        }
-    int tot_eq;
-    const int eq0 = blk_excl_scan(eq, &tot_eq, sm);
-    const int keep_eq = cutoff - blk_sum_i(gt, sm);
+    const bool finish = a.mode == 0 && m <= a.finish_most;
+    if (!finish && !a.prepared) return kListGeneral;
+    // Members: everything above the value at the cut, and of the entries equal to it the first ones by index -- nearly always all of
+    // them: nothing behind the cut has its value.
+    const bool tie = cutoff < ns && prob(grp[list_place(cutoff)]) == ycut;
     uint32_t members = 0u;
     int last_here = -1;
-    {
+    if (tie) {
+        int gt = 0, eq = 0;
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if (r < mine) {
+                const float y = prob(ev[r]);
+                gt += y > ycut ? 1 : 0;
+                eq += y == ycut ? 1 : 0;
+            }
+        int tot_eq;
+        const int eq0 = blk_excl_scan(eq, &tot_eq, sm);
+        const int keep_eq = cutoff - blk_sum_i(gt, sm);
         int k = eq0;
 #pragma unroll
         for (int r = 0; r < kPer; r++)
             if (r < mine) {
                 const float y = prob(ev[r]);
-                const bool tie = y == ycut;
-                if (y > ycut || (tie && k < keep_eq)) members |= 1u << r;
-                if (tie && k == keep_eq - 1) last_here = r;
-                k += tie ? 1 : 0;
+                const bool same = y == ycut;
+                if (y > ycut || (same && k < keep_eq)) members |= 1u << r;
+                if (same && k == keep_eq - 1) last_here = r;
+                k += same ? 1 : 0;
             }
+    } else {
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if (r < mine && prob(ev[r]) >= ycut) members |= 1u << r;
     }
-    const int m = cutoff;
-    const bool finish = a.mode == 0 && m <= a.finish_most;
-    if (!finish && !a.prepared) return kListGeneral;
-    // The members by their places in the list: a bit each, and how many stand in front of every thread's.  The waves then go
-    // through the segments once more and know the index and the rank of every member they meet.
+    if (kOne && finish) {
+        // in the order of the list, which is the order of the indices
+        int tot;
+        const int at = blk_excl_scan((int)(members & 1u), &tot, sm);  // (its barriers: the sorted values have been read)
+        const uint32_t idx = tid < N ? list_ids(sm)[tid] : 0u;
+        const bool laid_out = m > SR_WAVE;
+        if (members & 1u) sm.sortbuf[laid_out ? list_layout(at) : at] = ((unsigned long long)(0xffffffffu - idx) << 32) | (unsigned long long)sr_f2u(prob(ev[0]));
+        __syncthreads();
+        finish_from_ordered_list(a, p, n, m, row, sm, NoFill(), kSmall, laid_out);
+        return kListDone;
+    }
+    // The waves go through the segments once more.  Where the members are to be put in order, or are not told by their value, a bit each
+    // by their places in the list, and how many stand in front of every thread's.
+    const bool by_bits = finish || tie;
     uint16_t* const bits = more ? (uint16_t*)more : (uint16_t*)sm.tags;
     int* const in_front = (int*)(bits + kT);
     static_assert(kT * (2 + 4) <= sizeof(FullSmem::tags), "the members' bits fit");
-    if (tid == 0) sm.bc[9] = 0u;
-    {
+    if (tid == 0) sm.bc[9] = (uint32_t)n;  // (the last index that is a member of the value at the cut; without a tie all are)
+    __syncthreads();  // (the sorted values have been read)
+    if (by_bits) {
         int tot;
-        const int at = blk_excl_scan(__popc(members), &tot, sm);  // (its barriers: the sorted values have been read)
+        const int at = blk_excl_scan(__popc(members), &tot, sm);
         bits[tid] = (uint16_t)members;
         in_front[tid] = at;
         if (last_here >= 0) sm.bc[10] = (uint32_t)(i0 + last_here);
     }
     float* const ssum = (float*)sm.sortbuf;
-    float* const csum = ssum + SR_SEG_MAX;
-    static_assert((SR_SEG_MAX + SR_SEG_MAX / SR_HALF_BLOCK_SEGS * SR_SEQ_CHAINS) * 4 <= sizeof(FullSmem::sortbuf), "the sums fit");
+    // (whole numbers: an atomic addition of floats in shared memory takes a wave some 190 cycles, 9 us for 5,000 members)
+    unsigned long long* const csum = (unsigned long long*)(ssum + SR_SEG_MAX);
+    static_assert(SR_SEG_MAX * 4 + SR_SEG_MAX / SR_HALF_BLOCK_SEGS * SR_SEQ_CHAINS * 8 <= sizeof(FullSmem::sortbuf), "the sums fit");
     if (!finish)
-        for (int i = tid; i < a.chain_stride; i += kT) csum[i] = 0.0f;
+        for (int i = tid; i < a.chain_stride; i += kT) csum[i] = 0ull;
     __syncthreads();
     FPROF(a, slot, 12);
     const uint32_t* gk = a.sort_keys_in + (size_t)slot * (size_t)a.sort_stride;
     const int32_t* gi = a.sort_vals_in + (size_t)slot * (size_t)a.sort_stride;
-    const int last_place = (int)sm.bc[10], nv8 = (n / 8) * 8;
+    const int last_place = tie ? (int)sm.bc[10] : -1, nv8 = (n / 8) * 8;
     for (int s0 = wave; s0 < nseg; s0 += 4 * kW) {
         uint32_t v[4], v2[4];
         int id[4], id2[4], at[4], len[4];
@@ -3065,15 +3105,20 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
                 const uint32_t ebits = i < SR_WAVE ? v[q] : i < 2 * SR_WAVE ? v2[q] : gk[(size_t)sg * SR_SEG_TERMS + i];
                 const int idx = i < SR_WAVE ? id[q] : i < 2 * SR_WAVE ? id2[q] : gi[(size_t)sg * SR_SEG_TERMS + i];
                 if (place == last_place) sm.bc[9] = (uint32_t)idx;
-                const uint32_t b = bits[place >> sh];
                 const int in_run = place & (per - 1);
-                if (!((b >> in_run) & 1u)) continue;
+                uint32_t b = 0u;
+                if (by_bits) {
+                    b = bits[place >> sh];
+                    if (!((b >> in_run) & 1u)) continue;
+                } else if (!(prob(ebits) >= ycut)) {
+                    continue;
+                }
                 if (finish) {
                     const int rank = in_front[place >> sh] + __popc(b & ((1u << in_run) - 1u));
                     sm.sortbuf[rank] = ((unsigned long long)(0xffffffffu - (uint32_t)idx) << 32) | (unsigned long long)sr_f2u(prob(ebits));
                 } else {
                     own += sr_u2f(ebits);
-                    if (idx < nv8) unsafeAtomicAdd(&csum[idx / (SR_HALF_BLOCK_SEGS * SR_SEG_TERMS) * SR_SEQ_CHAINS + (idx & (SR_SEQ_CHAINS - 1))], sr_u2f(ebits));
+                    if (idx < nv8) atomicAdd(&csum[idx / (SR_HALF_BLOCK_SEGS * SR_SEG_TERMS) * SR_SEQ_CHAINS + (idx & (SR_SEQ_CHAINS - 1))], e_units(ebits));
                 }
             }
             if (!finish && sg < nseg) {
@@ -3089,7 +3134,7 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     }
     // left to the whole device: the members' part of every segment and of every half block of the eight accumulators
     for (int i = tid; i < nseg; i += kT) a.seg_sum[(size_t)slot * a.seg_stride + i] = ssum[i];
-    for (int i = tid; i < a.chain_stride; i += kT) a.chain_sum[(size_t)slot * a.chain_stride + i] = csum[i];
+    for (int i = tid; i < a.chain_stride; i += kT) a.chain_sum[(size_t)slot * a.chain_stride + i] = (float)csum[i] * 0x1p-40f;
     row_deferred(a, st, inv, ycut, (int)sm.bc[9], sm);
     return kListDeferred;
 }
@@ -3355,9 +3400,10 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                     } else if (n_list <= list_cap(more != nullptr)) {
                         uint32_t* const grp = list_values(more, sm);
                         const uint32_t* gk = a.sort_keys_in + (size_t)slot * (size_t)a.sort_stride;
+                        const int32_t* gi = a.sort_vals_in + (size_t)slot * (size_t)a.sort_stride;
                         // (four segments' first entries on their way at a time)
                         for (int s0 = sr_wave_id() - 1; s0 < nseg; s0 += 4 * (kW - 1)) {
-                            uint32_t v[4];
+                            uint32_t v[4], id[4] = {0u, 0u, 0u, 0u};
                             int at[4], len[4];
 #pragma unroll
                             for (int q = 0; q < 4; q++) {
@@ -3366,11 +3412,22 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                                 len[q] = sg < nseg ? (sg + 1 < nseg ? off[sg + 1] : n_list) - at[q] : 0;
                                 v[q] = lane < len[q] ? gk[(size_t)sg * SR_SEG_TERMS + lane] : 0u;
                             }
+                            if (n_list <= kT) {
+#pragma unroll
+                                for (int q = 0; q < 4; q++) {
+                                    const int sg = s0 + q * (kW - 1);
+                                    id[q] = lane < len[q] ? (uint32_t)gi[(size_t)sg * SR_SEG_TERMS + lane] : 0u;
+                                }
+                            }
 #pragma unroll
                             for (int q = 0; q < 4; q++) {
                                 const int sg = s0 + q * (kW - 1);
                                 if (lane < len[q]) grp[list_place(at[q] + lane)] = v[q];
-                                for (int i = lane + SR_WAVE; i < len[q]; i += SR_WAVE) grp[list_place(at[q] + i)] = gk[(size_t)sg * SR_SEG_TERMS + i];
+                                if (lane < len[q] && n_list <= kT) list_ids(sm)[at[q] + lane] = id[q];
+                                for (int i = lane + SR_WAVE; i < len[q]; i += SR_WAVE) {
+                                    grp[list_place(at[q] + i)] = gk[(size_t)sg * SR_SEG_TERMS + i];
+                                    if (n_list <= kT) list_ids(sm)[at[q] + i] = (uint32_t)gi[(size_t)sg * SR_SEG_TERMS + i];
+                                }
                             }
                         }
                     }
@@ -3411,7 +3468,9 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                 if (n_list > 0 && n_list <= SR_WAVE)
                     way = cut_from_short_list(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm);
                 else if (n_list > 0 && n_list <= list_cap(more != nullptr))
-                    way = cut_from_list(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm, more);
+                    way = n_list <= kT ? cut_from_list<1>(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm, more)
+                          : n_list <= 4 * kT ? cut_from_list<4>(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm, more)
+                                             : cut_from_list<SR_LIST_CAP_BIG / kT>(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm, more);
                 if (way != kListGeneral) {
                     FPROF(a, slot, 9);
                     __syncthreads();
