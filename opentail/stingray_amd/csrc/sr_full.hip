@@ -405,77 +405,78 @@ __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSeg
         const uint32_t T = (uint32_t)sr_wave_incl_scan_i32(simple ? (int)r.f.x : 0);
         uint32_t eb = sr_state_eb(sb), off = sr_state_n(sb, eb);
         uint32_t pre = off, ebv = eb;  // behind a lane's segment the sum is pre + T in the binade ebv
-        // One form for both kinds of records, no branch per segment: a plain one has sixteen zeros for the terms of its crossing and a
-        // second function that adds nothing.  [lo2, lo2 + size2): the bits of the second function's binade.
-        const uint32_t eb1 = kind == SR_SEG_PLAIN || split ? (uint32_t)r.f.z : 0xffffu, odd1 = r.f.y - r.f.x;
-        const uint32_t inc2 = split ? r.g.x : 0u, odd2 = split ? r.g.y - r.g.x : 0u, eb2 = split ? (uint32_t)r.g.z : eb1;
-        const uint32_t lo2 = eb2 > 1u ? eb2 << 23 : 0u, size2 = eb2 > 1u ? 1u << 23 : 1u << 24;
-        const uint32_t words[16] = {r.x0.x, r.x0.y, r.x0.z, r.x0.w, r.x1.x, r.x1.y, r.x1.z, r.x1.w,
-                                    r.x2.x, r.x2.y, r.x2.z, r.x2.w, r.x3.x, r.x3.y, r.x3.z, r.x3.w};
-        float xs[16];
-#pragma unroll
-        for (int j = 0; j < 16; j++) xs[j] = split ? sr_u2f(words[j]) : 0.0f;
-        auto terms = [&](int t, uint32_t before) __attribute__((always_inline)) -> uint32_t {
-            float x[SR_SEQ_RUN];
-            load(base + t, x);
-            int at;
-            return (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(sr_seq_wave<SR_SEQ_RUN, false>(x, sr_u2f(before), 0.0f, &at)));
-        };
         unsigned long long todo = stops;
-        int pos = 0;     // the segments below were where they were planned
-        int again = -1;  // a segment to be added from its terms, everything in front of which is exact
-        if (sb == 0u) {
+        if (sb == 0u && stops != 0ull) {
             // the first segment that has a term, where its record carries the sum behind it
-            const unsigned long long exacts = __ballot(kind == SR_SEG_EXACT);
-            if (exacts != 0ull && (stops & (0ull - stops)) == (exacts & (0ull - exacts))) {
-                const int t = (int)__ffsll((long long)stops) - 1;
-                const uint32_t Tt = (uint32_t)__builtin_amdgcn_readlane((int)T, t);
-                if (Tt == 0u) {
-                    const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)r.g.w, t);
-                    eb = sr_state_eb(to);
-                    off = sr_state_n(to, eb);
-                    if (lane >= t) { pre = off; ebv = eb; }
-                    todo &= todo - 1ull;
-                }
+            const int t = (int)__ffsll((long long)stops) - 1;
+            const uint32_t k = (uint32_t)__builtin_amdgcn_readlane((int)kind, t), Tt = (uint32_t)__builtin_amdgcn_readlane((int)T, t);
+            if (k == SR_SEG_EXACT && Tt == 0u) {
+                const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)r.g.w, t);
+                eb = sr_state_eb(to);
+                off = sr_state_n(to, eb);
+                if (lane >= t) { pre = off; ebv = eb; }
+                todo &= todo - 1ull;
             }
         }
-        for (;;) {
-            while (todo != 0ull || again >= 0) {
-                const int t = again >= 0 ? again : (int)__ffsll((long long)todo) - 1;
-                const uint32_t Tt = (uint32_t)__builtin_amdgcn_readlane((int)T, t);
-                uint32_t to, before;
-                bool fits = false;
-                if (again >= 0) {
-                    before = t > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)sr_state_bits(pre + T, ebv), t - 1) : sb;
-                    to = 0u;
-                    again = -1;
-                } else {
-                    todo &= todo - 1ull;
-                    const uint32_t n = off + Tt;
-                    if (n >= (1u << 24)) break;  // (a segment in front of this one left its binade unforeseen)
-                    before = sr_state_bits(n, eb);
-                    const uint32_t b1 = before + (r.f.x + (odd1 & (0u - (n & 1u))));
-                    float acc = sr_u2f(b1);
+        const uint32_t eb1 = kind == SR_SEG_PLAIN || split ? (uint32_t)r.f.z : 0xffffu;
+        // One form for both kinds of records, no branch per segment: a plain one has sixteen zeros for the terms of its crossing and a
+        // second function that adds nothing.  [lo2, lo2 + size2): the bits of the second function's binade.
+        uint32_t odd1 = 0u, inc2 = 0u, odd2 = 0u, lo2 = 0u, size2 = 0u;
+        float xs[16] = {};
+        if (todo != 0ull) {
+            odd1 = r.f.y - r.f.x;
+            inc2 = split ? r.g.x : 0u;
+            odd2 = split ? r.g.y - r.g.x : 0u;
+            const uint32_t eb2 = split ? (uint32_t)r.g.z : eb1;
+            lo2 = eb2 > 1u ? eb2 << 23 : 0u;
+            size2 = eb2 > 1u ? 1u << 23 : 1u << 24;
+            const uint32_t words[16] = {r.x0.x, r.x0.y, r.x0.z, r.x0.w, r.x1.x, r.x1.y, r.x1.z, r.x1.w,
+                                        r.x2.x, r.x2.y, r.x2.z, r.x2.w, r.x3.x, r.x3.y, r.x3.z, r.x3.w};
 #pragma unroll
-                    for (int j = 0; j < 16; j++) acc = __fadd_rn(acc, xs[j]);
-                    const uint32_t b2 = sr_f2u(acc), b3 = b2 + (inc2 + (odd2 & (0u - (b2 & 1u))));
-                    // (one comparison each: the record is for the binade the sum is in, the first function ends in it, the second one
-                    // starts and ends in its own)
-                    const unsigned long long ok = __ballot(eb1 == eb) & __ballot(b1 < sr_state_bits(1u << 24, eb)) & __ballot(b2 >= lo2) & __ballot(b3 - lo2 < size2);
-                    fits = ((ok >> t) & 1ull) != 0ull;
-                    to = (uint32_t)__builtin_amdgcn_readlane((int)b3, t);
+            for (int j = 0; j < 16; j++) xs[j] = split ? sr_u2f(words[j]) : 0.0f;
+        }
+        int pos = 0;  // the segments below were where they were planned
+        for (;;) {
+            int fix = -1;  // a segment to be added from its terms
+            uint32_t before = 0u;
+            while (todo != 0ull) {
+                const int t = (int)__ffsll((long long)todo) - 1;
+                todo &= todo - 1ull;
+                const uint32_t Tt = (uint32_t)__builtin_amdgcn_readlane((int)T, t), n = off + Tt;
+                before = sr_state_bits(n, eb);
+                const uint32_t b1 = before + (r.f.x + (odd1 & (0u - (n & 1u))));
+                float acc = sr_u2f(b1);
+#pragma unroll
+                for (int j = 0; j < 16; j++) acc = __fadd_rn(acc, xs[j]);
+                const uint32_t b2 = sr_f2u(acc), b3 = b2 + (inc2 + (odd2 & (0u - (b2 & 1u))));
+                // (one comparison each: the record is for the binade the sum is in, the first function ends in it, the second one
+                // starts and ends in its own)
+                const unsigned long long ok = __ballot(eb1 == eb) & __ballot(b1 < sr_state_bits(1u << 24, eb)) & __ballot(b2 >= lo2) & __ballot(b3 - lo2 < size2);
+                const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)b3, t);
+                if (((ok >> t) & 1ull) == 0ull || n >= (1u << 24)) {
+                    fix = n >= (1u << 24) ? -1 : t;  // (-1: a segment in front of this one left its binade unforeseen)
+                    break;
                 }
-                if (!fits) to = terms(t, before);
                 eb = sr_state_eb(to);
                 off = sr_state_n(to, eb) - Tt;
                 if (lane >= t) { pre = off; ebv = eb; }
             }
-            const unsigned long long bad = __ballot(simple && lane >= pos && (eb1 != ebv || pre + T >= (1u << 24)));
-            if (bad == 0ull) break;
-            // (everything in front of this segment is exact)
-            again = (int)__ffsll((long long)bad) - 1;
-            pos = again + 1;
-            todo = pos < SR_WAVE ? stops & (~0ull << pos) : 0ull;
+            if (fix < 0) {
+                const unsigned long long bad = __ballot(simple && lane >= pos && (eb1 != ebv || pre + T >= (1u << 24)));
+                if (bad == 0ull) break;
+                // (everything in front of this segment is exact)
+                fix = (int)__ffsll((long long)bad) - 1;
+                pos = fix + 1;
+                before = fix > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)sr_state_bits(pre + T, ebv), fix - 1) : sb;
+                todo = pos < SR_WAVE ? stops & (~0ull << pos) : 0ull;
+            }
+            float x[SR_SEQ_RUN];
+            load(base + fix, x);
+            int at;
+            const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)sr_f2u(sr_seq_wave<SR_SEQ_RUN, false>(x, sr_u2f(before), 0.0f, &at)));
+            eb = sr_state_eb(to);
+            off = sr_state_n(to, eb) - (uint32_t)__builtin_amdgcn_readlane((int)T, fix);
+            if (lane >= fix) { pre = off; ebv = eb; }
         }
         const uint32_t ends = sr_state_bits(pre + T, ebv);
         if (!kSearch && states && base + lane < nseg) states[base + lane] = sr_u2f(ends);

@@ -346,8 +346,7 @@ __device__ __forceinline__ float sr_seq_wave(const float (&x)[N], float s, float
                 const int t = (int)__ffsll((long long)todo) - 1;
                 todo &= todo - 1ull;
                 const uint32_t Tt = (uint32_t)__builtin_amdgcn_readlane((int)T, t);
-                if (off + Tt >= (1u << 24)) break;  // (a lane in front of this one left its binade unforeseen)
-                float acc = sr_u2f(sr_state_bits(off + Tt, eb));
+                float acc = sr_u2f(sr_state_bits(off + Tt, eb));  // (of no use where a lane in front left its binade unforeseen: done again)
 #pragma unroll
                 for (int j = 0; j < N; j++) acc = __fadd_rn(acc, x[j]);
                 const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)sr_f2u(acc), t);
