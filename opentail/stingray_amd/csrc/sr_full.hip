@@ -1668,7 +1668,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     __shared__ unsigned long long hits[kHitCap];
     __shared__ uint32_t n_hits;
     if (rd.temperature <= 0.0f) {  // greedy rows keep their logits where a distribution is asked for
-        if (a.mode == 0) seg_greedy<ES, kW, kS>(a, rd, slot, row, hits);
+        if (kS != 4 && a.mode == 0) seg_greedy<ES, kW, kS>(a, rd, slot, row, hits);
         return;
     }
     const int n = a.vocab, nseg = seg_count(n);
@@ -1711,7 +1711,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
 #pragma unroll
         for (int j = 0; j < kIds; j++) {
             const int e = (int)threadIdx.x + j * kThreads;
-            ids[j] = e < rd.edit_cnt ? ed[e].id : -1;
+            ids[j] = kS != 4 && e < rd.edit_cnt ? ed[e].id : -1;
         }
     }
     // (a wave takes kS segments, the workgroup's waves side by side: every one of its loads is out before the first is used)
@@ -1724,6 +1724,8 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
         const int lo = (int)blockIdx.x * (kW * kS) * SR_SEG_TERMS, hi = lo + kW * kS * SR_SEG_TERMS;
 #pragma unroll
         for (int j = 0; j < kIds; j++) {
+            // (beside four segments there is no room to ask for them ahead)
+            if (kS == 4) ids[j] = (int)threadIdx.x + j * kThreads < rd.edit_cnt ? ed[(int)threadIdx.x + j * kThreads].id : -1;
             if (ids[j] >= lo && ids[j] < hi) {
                 const uint32_t pos = atomicAdd(&n_hits, 1u);
                 if (pos < (uint32_t)kHitCap)
