@@ -3852,15 +3852,15 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
 // The members' probabilities y = fl(e inv) are known by the cut (all of them, in a row that nothing cuts).  One launch
 // (k_prepared_row), a workgroup per block of 8,192 entries, which it reads once:
 //   its waves, one per lane accumulator of TensorPrimitives.Sum, make the records of their 1,024 terms of the block;
-//   when the row's workgroups are all there, every one of them walks the eight accumulators (the same work in all of them
-//   costs less than a second meeting), and its waves take a segment each: z = fl(y / sum), written where the distribution is
-//   handed out, and the segment's record for the running sum of the draw;
+//   whoever of the row's workgroups is there last walks the eight accumulators, and the others wait for the factor;
+//   then every wave takes a segment: z = fl(y / sum), written where the distribution is handed out, and the segment's record
+//   for the running sum of the draw;
 //   whoever comes last walks those records to the draw's target.
 // What bounds it: the serial chain (data, records, meeting, walk of the accumulators, records, walk of the draw), about a
 // third of it trips to memory.  32 ragged bf16 rows of 100,003: 23 us, 16 rows of 262,144 fp32: 33; as three launches --
 // each 4 us before its first byte, and the row read twice -- the same steps took 27 and 38.
 // The wait is bounded: a workgroup whose wait runs out marks the row (SrFullState::late_behind), counts itself in as if it had done
-// its block, and whoever comes last does all blocks of the row from the records of the accumulators, which are all there.
+// its block, and whoever comes last does all blocks of the row again.
 struct PreparedRow {
     const float* e;
     float inv, ycut;
@@ -3952,7 +3952,7 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
 {
     __shared__ float4 room[SR_SEQ_CHAINS * SR_WAVE * 5];  // the block chain by chain, then every wave's segment on its way to 16 terms a lane
     __shared__ float lane_sum[SR_SEQ_CHAINS];
-    __shared__ uint32_t bc;
+    __shared__ uint32_t bc[2];
     const int slot = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
     SrFullState* st = a.state + slot;
     if (st->deferred != a.seq) return;
@@ -3997,19 +3997,11 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
     __syncthreads();  // (the workgroup's records are out, and nobody reads the block any more)
     if (tid == 0) {
         const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        uint32_t ok = ((uint32_t)was & 0xffffu) + 1u == gridDim.x ? 1u : 0u;
-        if (!a.lazy_scale) {
-            for (uint32_t it = 0; ok == 0u && it < a.behind_wait_limit; it++) {
-                ok = ((uint32_t)sr_load_agent(sync) & 0xffffu) == gridDim.x ? 1u : 0u;
-                if (ok == 0u) __builtin_amdgcn_s_sleep(1);
-            }
-            if (ok == 0u) sr_store_agent(&st->late_behind, a.seq);
-        }
-        bc = ok;
+        bc[0] = ((uint32_t)was & 0xffffu) + 1u == gridDim.x ? 1u : 0u;
     }
     __syncthreads();
-    bool here = bc != 0u;
-    if (a.lazy_scale && !here) return;  // (the last one has all there is to do)
+    const bool last_in = bc[0] != 0u;
+    if (a.lazy_scale && !last_in) return;  // (the last one has all there is to do)
     // the eight accumulators, a wave each: the sum of the members, and 1 over it
     auto normaliser = [&]() __attribute__((always_inline)) -> float {
         int dummy;
@@ -4036,26 +4028,48 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
         const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
         return (sum > 0.0f && sum != 1.0f) ? __fdiv_rn(1.0f, sum) : 1.0f;
     };
+    // Whoever counts in last walks them, and the others wait for the factor.  (All workgroups of the row walking for themselves, the
+    // same work: 512 of them, at 16 rows of 262,144, fetched 12 MB of records past the caches and took 2.6 - 8 us for it.)
+    unsigned long long* const factor = sync + 2;  // launch number << 32 | the factor's bits
     float inv2 = 1.0f;
-    if (here) {
+    bool here = true;
+    if (last_in) {
         inv2 = normaliser();
-        if (a.lazy_scale) {
-            if (tid == 0) st->mul2 = inv2;
-            return;
+        if (tid == 0) {
+            st->mul2 = inv2;
+            sr_store_agent(factor, ((unsigned long long)a.seq << 32) | (unsigned long long)sr_f2u(inv2));
         }
-        if (seg < nseg) prepared_segment(a, r, slot, row, seg, lane, v, sr_wave_sum_f32(before_seg), inv2, room + wave * SR_WAVE * 5);
+        if (a.lazy_scale) return;
+    } else {
+        if (tid == 0) {
+            uint32_t ok = 0u;
+            unsigned long long v = 0ull;
+            for (uint32_t it = 0; it < a.behind_wait_limit; it++) {
+                v = sr_load_agent(factor);
+                if ((uint32_t)(v >> 32) == a.seq) { ok = 1u; break; }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            if (ok == 0u) sr_store_agent(&st->late_behind, a.seq);
+            bc[0] = ok;
+            bc[1] = (uint32_t)v;
+        }
+        __syncthreads();
+        here = bc[0] != 0u;
+        inv2 = sr_u2f(bc[1]);
     }
+    if (here && seg < nseg) prepared_segment(a, r, slot, row, seg, lane, v, sr_wave_sum_f32(before_seg), inv2, room + wave * SR_WAVE * 5);
     sr_drain_stores();
     __syncthreads();
     if (tid == 0) {
         const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bc = ((uint32_t)(was >> 16) & 0xffffu) + 1u == gridDim.x ? (sr_load_agent(&st->late_behind) == a.seq ? 2u : 1u) : 0u;
+        bc[0] = ((uint32_t)(was >> 16) & 0xffffu) + 1u == gridDim.x ? (sr_load_agent(&st->late_behind) == a.seq ? 2u : 1u) : 0u;
+        if (bc[0] == 2u) bc[1] = (uint32_t)sr_load_agent(factor);
     }
     __syncthreads();
-    if (bc == 0u) return;
-    if (bc == 2u) {
-        // some workgroup stopped waiting: all of the row again, from the accumulators' records
-        inv2 = normaliser();
+    if (bc[0] == 0u) return;
+    if (bc[0] == 2u) {
+        // some workgroup stopped waiting: all of the row again (everyone has counted in: the factor is there)
+        inv2 = sr_u2f(bc[1]);
         for (int b = 0; b < (int)gridDim.x; b++) {
             const int sg = b * SR_SEQ_CHAINS + wave;
             if (sg >= nseg) break;
@@ -4067,7 +4081,6 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
         sr_drain_stores();
         __syncthreads();
     }
-    if (tid == 0) st->mul2 = inv2;
     if (a.mode == 1 || wave != 0) return;
     const float u = st->u;
     int found;

@@ -154,7 +154,8 @@ static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // launch number << 32 | workgroups of k_full_softmax_seg at the second meeting point << 16 | at the first.  The number is
 // put in by an atomic maximum before the first count of a launch, so nothing clears the words.  The word behind it counts the
 // workgroups of k_prepared_row the same way; k_full_row, which leaves the row to them, starts it.  The third one holds what the
-// workgroups of a greedy row have found so far (zero between launches).
+// workgroups of a greedy row have found so far (zero between launches), the fourth one the factor that k_prepared_row's workgroups
+// wait for, with the launch number above it.
 #define SR_ROW_SYNC_STRIDE 32
 
 struct SeqSegFunc;
