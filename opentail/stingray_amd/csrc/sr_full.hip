@@ -385,8 +385,8 @@ __device__ __forceinline__ void seg_load_rec(const SeqSegFunc* funcs, int seg, i
 // follows is done again.  A segment taken by itself costs some 50 instructions of the one wave, 0.1 us, a sum that
 // starts at zero has about a dozen; looking for the end of every run of segments as it went, the walk took 0.45 us for each:
 // 98 segments of a row of 100,003 entries 5.3 us, and a search over as many 7.5.
-// first64: the first 64 records, where the caller has asked for them already.
-template <bool kSearch, bool kAgent = false, typename Load>
+// first64: the first 64 records, where the caller has asked for them already.  kFew: there are no more than those.
+template <bool kSearch, bool kAgent = false, bool kFew = false, typename Load>
 __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSegFunc* funcs, float s0, float target, int* found,
                                                float* states, const SegRec* first64 = nullptr)
 {
@@ -398,7 +398,7 @@ __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSeg
     else seg_load_rec<kAgent>(funcs, lane, nseg, next);
     for (int base = 0; base < nseg; base += SR_WAVE) {
         const SegRec r = next;
-        if (base + SR_WAVE < nseg) seg_load_rec<kAgent>(funcs, base + SR_WAVE + lane, nseg, next);  // (the next 64 segments' come in meanwhile)
+        if (!kFew && base + SR_WAVE < nseg) seg_load_rec<kAgent>(funcs, base + SR_WAVE + lane, nseg, next);  // (the next 64 segments' come in meanwhile)
         const uint32_t kind = r.f.w & 0xffu;
         const bool simple = kind == SR_SEG_PLAIN && r.f.x == r.f.y && r.f.x < (1u << 24), split = kind == SR_SEG_SPLIT;
         const unsigned long long stops = ~__ballot(simple || kind == SR_SEG_ZERO);
@@ -2891,21 +2891,29 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
             if (r < mine) atomicAdd(&cnt[group_of(ev[r])], 1u);
         __syncthreads();
         {
-            // a wave's share of the groups, 64 at a time: the sums inside the wave, then what stands in front of it
-            const int g0 = wave * (G / kW);
+            // a wave's share of the groups, 64 at a time: the sums inside each 64, one behind the other inside the wave, then what stands
+            // in front of it.  (All of them are read before the first is scanned: 16,384 groups took 4.4 us one by one.)
+            constexpr int kRuns = kPer == 1 ? 2 : kPer == 4 ? 8 : SR_LIST_GROUPS_BIG / kT;
+            const int g0 = wave * (G / kW), runs = G / kT;
+            int c[kRuns], incl[kRuns];
+#pragma unroll
+            for (int q = 0; q < kRuns; q++) c[q] = q < runs ? (int)cnt[g0 + q * SR_WAVE + lane] : 0;
             int in_wave = 0;
-            for (int g = g0; g < g0 + G / kW; g += SR_WAVE) {
-                const int c = (int)cnt[g + lane];
-                const int incl = sr_wave_incl_scan_i32(c);
-                cnt[g + lane] = (uint32_t)(in_wave + incl - c);
-                in_wave += __builtin_amdgcn_readlane(incl, SR_WAVE - 1);
+#pragma unroll
+            for (int q = 0; q < kRuns; q++) incl[q] = sr_wave_incl_scan_i32(c[q]);
+#pragma unroll
+            for (int q = 0; q < kRuns; q++) {
+                c[q] = in_wave + incl[q] - c[q];
+                in_wave += __builtin_amdgcn_readlane(incl[q], SR_WAVE - 1);
             }
             if (lane == 0) sm.redi[wave] = in_wave;
             __syncthreads();
             int before = 0;
 #pragma unroll
             for (int w = 0; w < kW; w++) before += w < wave ? sm.redi[w] : 0;
-            for (int g = g0; g < g0 + G / kW; g += SR_WAVE) cnt[g + lane] += (uint32_t)before;
+#pragma unroll
+            for (int q = 0; q < kRuns; q++)
+                if (q < runs) cnt[g0 + q * SR_WAVE + lane] = (uint32_t)(before + c[q]);
         }
         __syncthreads();
         uint32_t at[kPer];  // (all places are asked for before the first is used)
@@ -2926,22 +2934,23 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
             last = v[r];
         }
         __syncthreads();
-        uint32_t ce[kPer];
-#pragma unroll
-        for (int r = 0; r < kPer; r++) ce[r] = r < mine ? cnt[group_of(v[r])] : 0u;
         int rank[kPer];
 #pragma unroll
         for (int r = 0; r < kPer; r++) {
             rank[r] = i0 + r;
-            if (ce[r] & kMixed) {
+            const uint32_t ce = r < mine ? cnt[group_of(v[r])] : 0u;
+            if (ce & kMixed) {
                 const int i = i0 + r;
                 const uint32_t g = group_of(v[r]);
-                const int b = g > 0u ? (int)(cnt[g - 1u] & ~kMixed) : 0, e = (int)(ce[r] & ~kMixed);
+                const int b = g > 0u ? (int)(cnt[g - 1u] & ~kMixed) : 0, e = (int)(ce & ~kMixed);
                 if (e - b > 128) sm.bc[12] = 1u;
                 int k = b;
-                for (int j = b; j < min(e, b + 128); j++) {
-                    const uint32_t o = grp[list_place(j)];
-                    k += (o > v[r] || (o == v[r] && j < i)) ? 1 : 0;
+                for (int j0 = b; j0 < min(e, b + 128); j0 += 4) {  // (four on their way at a time)
+                    uint32_t o[4];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) o[q] = grp[list_place(min(j0 + q, N - 1))];
+#pragma unroll
+                    for (int q = 0; q < 4; q++) k += (j0 + q < e) & ((o[q] > v[r]) | ((o[q] == v[r]) & (j0 + q < i))) ? 1 : 0;
                 }
                 rank[r] = k;
             }
@@ -2968,36 +2977,82 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     __syncthreads();
     if (ns <= 0) return kListGeneral;
     FPROF(a, slot, 11);
+    // The indices of the thread's entries, asked for in front of the cut where there is room to keep them: an entry's place in the
+    // list names its segment and its place there.  (A pass over all segments behind the cut, for the members' indices: 5 - 6 us.)
+    const int32_t* gi = a.sort_vals_in + (size_t)slot * (size_t)a.sort_stride;
+    int idx[kPer];
+    auto fetch_indices = [&]() __attribute__((always_inline)) {
+        if (kOne) {
+            idx[0] = tid < N ? (int)list_ids(sm)[tid] : 0;
+            return;
+        }
+        int sg = 0;
+        for (int half = SR_SEG_MAX / 2; half > 0; half >>= 1)  // the last segment that starts at the first entry or in front of it
+            if (sg + half < nseg && off[sg + half] <= i0) sg += half;
+        int start = off[sg], next = sg + 1 < nseg ? off[sg + 1] : N;
+#pragma unroll
+        for (int r = 0; r < kPer; r++) {
+            idx[r] = 0;
+            if (r < mine) {
+                while (next <= i0 + r) {  // (ends at the last segment, whose entries end the list)
+                    sg++;
+                    start = next;
+                    next = sg + 1 < nseg ? off[sg + 1] : N;
+                }
+                idx[r] = gi[(size_t)sg * SR_SEG_TERMS + (size_t)(i0 + r - start)];
+            }
+        }
+    };
+    if (kPer <= 4) fetch_indices();
     int found = -1;
     if (use_top_p) {
-        if (kOne || ns <= 6 * SR_SEG_TERMS) {
-            // by one wave, without the block-wide steps, a thousand in 0.9 us (by the workgroup: 6 us for 3,000 to 5,000)
-            if (wave == 0) {
-                float s = 0.0f;
-                int f = -1;
-                auto fetch = [&](int b0, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
+        auto fetch = [&](int b0, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
 #pragma unroll
-                    for (int j = 0; j < SR_SEQ_RUN; j++) {
-                        const int i = b0 + lane * SR_SEQ_RUN + j;
-                        x[j] = i < ns ? prob(grp[list_place(i)]) : 0.0f;
-                    }
-                };
-                for (int b0 = 0; b0 < ns && f < 0; b0 += SR_SEG_TERMS) {
-                    float x[SR_SEQ_RUN];
-                    fetch(b0, x);
-                    int at;
-                    s = sr_seq_wave<SR_SEQ_RUN, true>(x, s, rd.top_p, &at);
-                    if (at >= 0) f = b0 + at;
-                }
-                if (lane == 0) { sm.segbc[1] = (uint32_t)f; sm.segbc[2] = sr_f2u(s); }
+            for (int j = 0; j < SR_SEQ_RUN; j++) {
+                const int i = b0 + lane * SR_SEQ_RUN + j;
+                x[j] = i < ns ? prob(grp[list_place(i)]) : 0.0f;
+            }
+        };
+        if (kOne || ns <= SR_SEG_TERMS) {
+            if (wave == 0) {
+                float x[SR_SEQ_RUN];
+                fetch(0, x);
+                int at;
+                const float s = sr_seq_wave<SR_SEQ_RUN, true>(x, 0.0f, rd.top_p, &at);
+                if (lane == 0) { sm.segbc[1] = (uint32_t)at; sm.segbc[2] = sr_f2u(s); }
+            }
+        } else {
+            // a thousand to a wave: their records, as for any long sum, and one wave walks them (one wave by itself: 6.5 us for
+            // 3,500; by the workgroup's tiles as many)
+            SeqSegFunc* const recs = (SeqSegFunc*)(sm.tags + kSmall / 2);  // (the groups are done with)
+            static_assert(SR_LIST_CAP_BIG / SR_SEG_TERMS <= kW && kW * sizeof(SeqSegFunc) <= kSmall * 2 &&
+                          (SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16) * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob), "a wave each; the records fit");
+            const int nrec = seg_count(ns);
+            float x[SR_SEQ_RUN], own = 0.0f;
+            if (wave < nrec) {
+                fetch(wave * SR_SEG_TERMS, x);
+#pragma unroll
+                for (int j = 0; j < SR_SEQ_RUN; j++) own += x[j];
+                own = sr_wave_sum_f32(own);
+                if (lane == 0) sm.redf[wave] = own;
             }
             __syncthreads();
-            found = (int)sm.segbc[1];
-        } else {
-            const float run = seq_sum<true>([&](int i) -> float { return prob(grp[list_place(i)]); }, ns, 0.0f, rd.top_p, &found, sm);
-            if (tid == 0) sm.segbc[2] = sr_f2u(run);
+            if (wave < nrec) {
+                float before = 0.0f;
+#pragma unroll
+                for (int w = 0; w < kW; w++) before += w < wave ? sm.redf[w] : 0.0f;
+                seg_make_record(x, wave, (double)before, recs + wave, own);
+            }
             __syncthreads();
+            if (wave == 0) {
+                int at;
+                const float s = seg_walk_from<true, false, true>([&](int sg, float (&y)[SR_SEQ_RUN]) __attribute__((always_inline)) { fetch(sg * SR_SEG_TERMS, y); },
+                                                    nrec, recs, 0.0f, rd.top_p, &at, nullptr);
+                if (lane == 0) { sm.segbc[1] = (uint32_t)at; sm.segbc[2] = sr_f2u(s); }
+            }
         }
+        __syncthreads();
+        found = (int)sm.segbc[1];
         // the list ended before the sum was there, and the row goes on behind it
         if (found < 0 && from > 1u && min_p_list_from(rd) < from) return kListGeneral;
         // ... or an entry behind the list's end shares the probability at the cut
@@ -3019,6 +3074,7 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     // Members: everything above the value at the cut, and of the entries equal to it the first ones by index -- nearly always all of
     // them: nothing behind the cut has its value.
     const bool tie = cutoff < ns && prob(grp[list_place(cutoff)]) == ycut;
+    if (kPer > 4) fetch_indices();
     uint32_t members = 0u;
     int last_here = -1;
     if (tie) {
@@ -3048,95 +3104,53 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
         for (int r = 0; r < kPer; r++)
             if (r < mine && prob(ev[r]) >= ycut) members |= 1u << r;
     }
-    if (kOne && finish) {
+    if (finish) {
         // in the order of the list, which is the order of the indices
         int tot;
-        const int at = blk_excl_scan((int)(members & 1u), &tot, sm);  // (its barriers: the sorted values have been read)
-        const uint32_t idx = tid < N ? list_ids(sm)[tid] : 0u;
-        const bool laid_out = m > SR_WAVE;
-        if (members & 1u) sm.sortbuf[laid_out ? list_layout(at) : at] = ((unsigned long long)(0xffffffffu - idx) << 32) | (unsigned long long)sr_f2u(prob(ev[0]));
+        int at = blk_excl_scan(__popc(members), &tot, sm);  // (its barriers: the sorted values have been read)
+        const bool laid_out = kOne && m > SR_WAVE;
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if ((members >> r) & 1u) {
+                sm.sortbuf[laid_out ? list_layout(at) : at] = ((unsigned long long)(0xffffffffu - (uint32_t)idx[r]) << 32) | (unsigned long long)sr_f2u(prob(ev[r]));
+                at++;
+            }
         __syncthreads();
-        finish_from_ordered_list(a, p, n, m, row, sm, NoFill(), kSmall, laid_out);
+        finish_from_ordered_list(a, p, n, m, row, sm, NoFill(), m <= kSmall ? kSmall : 2 * kSmall, laid_out);
         return kListDone;
     }
-    // The waves go through the segments once more.  Where the members are to be put in order, or are not told by their value, a bit each
-    // by their places in the list, and how many stand in front of every thread's.
-    const bool by_bits = finish || tie;
-    uint16_t* const bits = more ? (uint16_t*)more : (uint16_t*)sm.tags;
-    int* const in_front = (int*)(bits + kT);
-    static_assert(kT * (2 + 4) <= sizeof(FullSmem::tags), "the members' bits fit");
+    // Left to the whole device: the members' part of every segment and of every half block of the eight accumulators.  (In whole
+    // numbers: an atomic addition of floats in shared memory takes a wave some 190 cycles, 9 us for 5,000 members.)
     if (tid == 0) sm.bc[9] = (uint32_t)n;  // (the last index that is a member of the value at the cut; without a tie all are)
-    __syncthreads();  // (the sorted values have been read)
-    if (by_bits) {
-        int tot;
-        const int at = blk_excl_scan(__popc(members), &tot, sm);
-        bits[tid] = (uint16_t)members;
-        in_front[tid] = at;
-        if (last_here >= 0) sm.bc[10] = (uint32_t)(i0 + last_here);
-    }
-    float* const ssum = (float*)sm.sortbuf;
-    // (whole numbers: an atomic addition of floats in shared memory takes a wave some 190 cycles, 9 us for 5,000 members)
-    unsigned long long* const csum = (unsigned long long*)(ssum + SR_SEG_MAX);
-    static_assert(SR_SEG_MAX * 4 + SR_SEG_MAX / SR_HALF_BLOCK_SEGS * SR_SEQ_CHAINS * 8 <= sizeof(FullSmem::sortbuf), "the sums fit");
-    if (!finish)
-        for (int i = tid; i < a.chain_stride; i += kT) csum[i] = 0ull;
+    __syncthreads();                       // (the sorted values have been read)
+    unsigned long long* const ssum = sm.sortbuf;
+    unsigned long long* const csum = ssum + SR_SEG_MAX;
+    static_assert((SR_SEG_MAX + SR_SEG_MAX / SR_HALF_BLOCK_SEGS * SR_SEQ_CHAINS) * 8 <= sizeof(FullSmem::sortbuf), "the sums fit");
+    for (int i = tid; i < nseg; i += kT) ssum[i] = 0ull;
+    for (int i = tid; i < a.chain_stride; i += kT) csum[i] = 0ull;
     __syncthreads();
     FPROF(a, slot, 12);
-    const uint32_t* gk = a.sort_keys_in + (size_t)slot * (size_t)a.sort_stride;
-    const int32_t* gi = a.sort_vals_in + (size_t)slot * (size_t)a.sort_stride;
-    const int last_place = tie ? (int)sm.bc[10] : -1, nv8 = (n / 8) * 8;
-    for (int s0 = wave; s0 < nseg; s0 += 4 * kW) {
-        uint32_t v[4], v2[4];
-        int id[4], id2[4], at[4], len[4];
+    const int nv8 = (n / 8) * 8;
+    {
+        unsigned long long run = 0ull;  // of the entries of one segment, which follow each other
+        int sg = 0;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {  // (the first 128 entries of four segments on their way at a time)
-            const int sg = s0 + q * kW;
-            const size_t from_seg = (size_t)sg * SR_SEG_TERMS + lane;
-            at[q] = sg < nseg ? off[sg] : 0;
-            len[q] = sg < nseg ? (sg + 1 < nseg ? off[sg + 1] : N) - at[q] : 0;
-            v[q] = lane < len[q] ? gk[from_seg] : 0u;
-            id[q] = lane < len[q] ? gi[from_seg] : 0;
-            v2[q] = lane + SR_WAVE < len[q] ? gk[from_seg + SR_WAVE] : 0u;
-            id2[q] = lane + SR_WAVE < len[q] ? gi[from_seg + SR_WAVE] : 0;
-        }
-#pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int sg = s0 + q * kW;
-            float own = 0.0f;
-            for (int i = lane; i < len[q]; i += SR_WAVE) {
-                const int place = at[q] + i;
-                const uint32_t ebits = i < SR_WAVE ? v[q] : i < 2 * SR_WAVE ? v2[q] : gk[(size_t)sg * SR_SEG_TERMS + i];
-                const int idx = i < SR_WAVE ? id[q] : i < 2 * SR_WAVE ? id2[q] : gi[(size_t)sg * SR_SEG_TERMS + i];
-                if (place == last_place) sm.bc[9] = (uint32_t)idx;
-                const int in_run = place & (per - 1);
-                uint32_t b = 0u;
-                if (by_bits) {
-                    b = bits[place >> sh];
-                    if (!((b >> in_run) & 1u)) continue;
-                } else if (!(prob(ebits) >= ycut)) {
-                    continue;
+        for (int r = 0; r < kPer; r++)
+            if ((members >> r) & 1u) {
+                const unsigned long long units = e_units(ev[r]);
+                if (idx[r] / SR_SEG_TERMS != sg && run != 0ull) {
+                    atomicAdd(&ssum[sg], run);
+                    run = 0ull;
                 }
-                if (finish) {
-                    const int rank = in_front[place >> sh] + __popc(b & ((1u << in_run) - 1u));
-                    sm.sortbuf[rank] = ((unsigned long long)(0xffffffffu - (uint32_t)idx) << 32) | (unsigned long long)sr_f2u(prob(ebits));
-                } else {
-                    own += sr_u2f(ebits);
-                    if (idx < nv8) atomicAdd(&csum[idx / (SR_HALF_BLOCK_SEGS * SR_SEG_TERMS) * SR_SEQ_CHAINS + (idx & (SR_SEQ_CHAINS - 1))], e_units(ebits));
-                }
+                sg = idx[r] / SR_SEG_TERMS;
+                run += units;
+                if (idx[r] < nv8) atomicAdd(&csum[idx[r] / (SR_HALF_BLOCK_SEGS * SR_SEG_TERMS) * SR_SEQ_CHAINS + (idx[r] & (SR_SEQ_CHAINS - 1))], units);
+                if (r == last_here) sm.bc[9] = (uint32_t)idx[r];
             }
-            if (!finish && sg < nseg) {
-                own = sr_wave_sum_f32(own);
-                if (lane == 0) ssum[sg] = own;
-            }
-        }
+        if (run != 0ull) atomicAdd(&ssum[sg], run);
     }
     __syncthreads();
-    if (finish) {
-        finish_from_ordered_list(a, p, n, m, row, sm, NoFill(), m <= kSmall ? kSmall : 2 * kSmall);
-        return kListDone;
-    }
-    // left to the whole device: the members' part of every segment and of every half block of the eight accumulators
-    for (int i = tid; i < nseg; i += kT) a.seg_sum[(size_t)slot * a.seg_stride + i] = ssum[i];
+    for (int i = tid; i < nseg; i += kT) a.seg_sum[(size_t)slot * a.seg_stride + i] = (float)ssum[i] * 0x1p-40f;
     for (int i = tid; i < a.chain_stride; i += kT) a.chain_sum[(size_t)slot * a.chain_stride + i] = (float)csum[i] * 0x1p-40f;
     row_deferred(a, st, inv, ycut, (int)sm.bc[9], sm);
     return kListDeferred;
