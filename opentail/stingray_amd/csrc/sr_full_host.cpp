@@ -50,7 +50,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     const int nseg = (vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
     const bool seg_mode = vocab >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX;
     a.edits_in_pass = seg_mode ? 1 : 0;
-    bool any_table = false, any_copy = false, any_edits = false, any_list = false, prepared = false, any_min_p = false;
+    bool any_table = false, any_copy = false, any_edits = false, any_list = false, prepared = false, any_plain = false, any_min_p = false;
     int n_sampled = 0, n_seen = 0;
     for (const SrRow& r : (host_rows ? *host_rows : b->h_rows)) {
         if (mode == 0 && r.path != SR_PATH_FULL) continue;
@@ -65,21 +65,25 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             // Rows that the row kernel may leave to the whole device: those that nothing cuts and, but for the verifier, whose
             // reader takes e where it is, those that only top-p cuts (a few members or tens of thousands).  What a min-p of some
             // size leaves is mostly little, and nobody knows before the launch: tokens of 64 rows of 151,936 with 300 entries left
-            // take 72 us, 78 where three launches follow that find nothing to do; with 2,000 77 against 128, since up to 8,192
-            // the row's workgroup then finishes by itself; with 8,300 to 16,384 184 against 147, and with more the launches find
-            // nothing again.  Distributions: SR_PREPARED_MIN_SEGS_MIN_P, whatever the min-p.
+            // took 72 us, 78 where more launches followed that found nothing to do; with 2,000 77 against 128, since up to 8,192
+            // the row's workgroup then finishes by itself.  Distributions: SR_PREPARED_MIN_SEGS_MIN_P, whatever the min-p.
             const bool by_min_p = mode != 0 ? r.min_p > 0.0f : r.min_p >= 0.002f;
             prepared = prepared || (lazy_scale ? !sr_row_cut(r) : !by_min_p);
+            any_plain = any_plain || !sr_row_cut(r);
             any_min_p = any_min_p || by_min_p;
         }
     }
-    // (distributions at odd addresses, where the row's workgroup passes over its row an entry at a time: at every length.  1, 16 and
-    // 64 rows cut by top-p, of 4,099: 59, 67, 70 us against 95, 106, 109; of 12,289: 71, 81, 82 against 115, 120, 122; of 24,001:
-    // 83, 91, 97 against 141, 174, 176; that nothing cuts, of 4,099: 41, 45, 50 against 50, 53, 56; only sharp rows of some lengths lose, 16 of 12,289 at top-p
-    // 0.9 and temperature 0.4 59 against 50, of 4,097 49 against 88)
     const bool odd_rows = mode != 0 && !lazy_scale && (probs_stride & 3) != 0;
-    prepared = prepared && (odd_rows || nseg >= (lazy_scale ? SR_PREPARED_MIN_SEGS_VERIFY : SR_PREPARED_MIN_SEGS)) &&
-               (long long)n_rows * nseg <= (lazy_scale ? SR_PREPARED_SEGS_VERIFY : mode != 0 ? SR_PREPARED_SEGS_DISTRIBUTIONS : SR_PREPARED_SEGS);
+    const long long segs = (long long)n_rows * nseg;
+    if (lazy_scale) {
+        prepared = prepared && nseg >= SR_PREPARED_MIN_SEGS_VERIFY && n_rows <= SR_PREPARED_ROWS_VERIFY;
+    } else if (mode != 0) {
+        prepared = prepared && segs <= SR_PREPARED_SEGS_DISTRIBUTIONS;
+    } else {
+        // (any_list: some row is cut)
+        const bool mixed = any_plain && nseg >= SR_PREPARED_MIN_SEGS_MIXED && n_rows <= SR_PREPARED_ROWS_MIXED;
+        prepared = prepared && ((any_plain && !any_list) || mixed || nseg >= SR_PREPARED_MIN_SEGS) && segs <= SR_PREPARED_SEGS;
+    }
     if (mode != 0 && !lazy_scale && any_min_p)
         prepared = prepared || (nseg >= (odd_rows ? SR_PREPARED_MIN_SEGS_MIN_P_ODD : SR_PREPARED_MIN_SEGS_MIN_P) && (long long)n_rows * nseg <= SR_PREPARED_SEGS_MIN_P);
     a.any_copy = any_copy ? 1 : 0;
@@ -142,7 +146,9 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             a.chain_sum = ctx->full_chain_sum.as<float>();
             a.chain_func = (SeqSegFunc*)ctx->full_chain_func.p;
             a.prepared = prepared ? 1 : 0;
-            a.finish_most = prepared ? 1024 : 8192;  // (up to 1,024 members cost the row's workgroup less than the launches behind it)
+            // (up to 1,024 members cost the row's workgroup less than the launch behind it; of short rows more: 256 rows of 12,290, half of
+            // them cut to some thousand members, 98 us, with 1,024 134)
+            a.finish_most = prepared && nseg >= SR_PREPARED_MIN_SEGS ? 1024 : 8192;
             // e = expf(x - max): in the work rows of tokens-only launches and of the verifier (whose reader applies the factors);
             // apart from the caller's rows where the probabilities take shape there
             a.e_rows = a.work;

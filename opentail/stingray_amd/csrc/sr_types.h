@@ -103,17 +103,31 @@ struct SrMaskClear {
 #define SR_SEG_TERMS 1024                  // terms per segment of a sum that the whole device prepares (64 lanes x 16)
 #define SR_SEG_MIN_VOCAB 4096              // shorter rows are not worth the preparation
 #define SR_HALF_BLOCK_SEGS 4               // segments of a half block of the final Normalize's eight accumulators (4,096 entries)
-// Segments of all of a launch's rows up to which it leaves its long rows to the whole device.  The row's own workgroup costs about
-// the same for one row and for 256; the launches behind it cost 25 us and what the rows hold together: tokens of 192
-// rows of 151,936 (28,608 segments) 182 -> 159 us, distributions of 64 rows 132 -> 109 and of 128 rows (19,072) 161 -> 164;
-// the verifier, where the workgroup passes over its row once and not three times: 24 rows of 262,144 (6,144) 108 -> 103, 36
-// rows 118.5 -> 119.6.
-// (And down to how many segments of a row: those launches cost the same for a short row, which its workgroup passes over in less.
-// Tokens, 16 rows of 16,384: 58.1 against 51.8 us, of 32,768 both 58, of 49,152: 58 against 67; the verifier, 20 rows of
-// 65,536: 69 against 65 us, of 131,072: 80 against 79, 2 rows of 262,144: 70 against 84.)
-#define SR_PREPARED_MIN_SEGS 32
-#define SR_PREPARED_MIN_SEGS_VERIFY 128
-// Distributions of rows that min-p cuts, where no other row asks for those launches: worth it for few long rows.  20,
+// Which launches have a second one behind them (k_prepared_row) that spreads their long rows over the whole device.  A row's own
+// workgroup costs about the same for one row and for 256; the launch behind it costs 10 to 20 us and what the rows hold
+// together.  Measured both ways, us with it against without; sharp and flat are rows over N(0, 1.5^2) with a few large entries at
+// top-p 0.9 and temperature 0.6, and at top-p 0.95 and temperature 1.5.
+// Tokens of rows that nothing cuts: at every length.  16 rows of 4,608: 34 against 49, of 16,384: 37 against 48, of 49,152: 43
+// against 64; 64 rows of 151,936: 91 against 122; 192 (28,608 segments): 199 against 197; 256: 266 against 251.  That only
+// top-p cuts, where it finds nothing to do for sharp rows: 16 rows of 24,576 23 against 22 (sharp) and 101 against 200 (flat), of
+// 16,384 23 against 21 and 77 against 72.  Both kinds of rows together, sharp and flat ones: 16 rows of 31,000 44 against 60 and 131
+// against 250, of 20,480 41 against 49 and 103 against 183, of 16,384 40 against 52 and 92 against 73, of 8,192 37 against 57
+// and 62 against 55; 256 rows of 31,000 84 against 76 and 251 against 285.
+// Distributions: at every length.  16 rows of 4,608 37 against 51, cut by top-p 32 against 82; of 16,384 37 against 47, 33 against 37
+// (flat: 77 against 131).  128 rows of 151,936 (19,072 segments) 147 against 158 and 131 against 146, 192 rows 223 against 198 and
+// 199 against 196; 160 rows of 131,072 (20,480) 161 both, 136 against 157.
+// The verifier, where the workgroup passes over its row once and not three times, so that the number of rows decides: of 65,536 3
+// rows 44 against 48, 32 rows 51 against 53, 45 rows 56 against 54; of 131,072 44 against 55, 59 against 68, 72 against 70; of
+// 262,144 50 against 74, 88 against 93, 106 against 98; of 32,768 3 rows 40 against 42, 24 rows 47 against 45.
+#define SR_PREPARED_MIN_SEGS 32        // tokens, rows that are cut
+#define SR_PREPARED_MIN_SEGS_MIXED 20  // ... beside rows that are not
+#define SR_PREPARED_ROWS_MIXED 128
+#define SR_PREPARED_SEGS 32768
+#define SR_PREPARED_SEGS_DISTRIBUTIONS 20480
+#define SR_PREPARED_MIN_SEGS_VERIFY 64
+#define SR_PREPARED_ROWS_VERIFY 32
+// Distributions of rows that min-p cuts, where no other row asks for that launch: worth it for few long rows.  Some ten entries left,
+// 16 rows of 65,536: 36 us against 34, of 131,072 43 against 49, of 262,144 59 against 80.  When three launches did its work, 20,
 // 200, 2,000, 8,000 and 15,000 entries left, 16 rows of 262,144: 71, 98, 106, 120, 143 us against 88, 99, 118, 181, 184 without;
 // of 131,072: 59, 79, 83, 101, 126 against 56, 68, 85, 112, 113; one row: 47, 63, 68, 87, 104 against 51, 60, 78, 102, 103; 64 rows
 // of 151,936: 96, 125, 131, 145, 165 against 78, 90, 109, 145, 145; 16 rows of 32,768: 52, 68, 70, 90, 112 against 33, 48, 61, 62, 63.
@@ -122,9 +136,6 @@ struct SrMaskClear {
 #define SR_PREPARED_MIN_SEGS_MIN_P 128
 #define SR_PREPARED_MIN_SEGS_MIN_P_ODD 96
 #define SR_PREPARED_SEGS_MIN_P 4096
-#define SR_PREPARED_SEGS 32768
-#define SR_PREPARED_SEGS_DISTRIBUTIONS 16384
-#define SR_PREPARED_SEGS_VERIFY 8192
 // candidates of a row that k_full_row sorts, and the groups it sorts them by: with a compute unit to itself, and without
 #define SR_LIST_CAP_BIG 16384
 #define SR_LIST_CAP_SMALL 4096

@@ -925,3 +925,30 @@ def test_edits_crowded_into_a_few_segments_of_a_long_row(ctx):
     exact = synthetic.bf16_bits_to_f32(bits)
     u = rng.random(5)
     assert np.array_equal(ctx.sample_batch(dev, params, u), oracle_tokens(exact, params, u))
+
+
+@pytest.mark.parametrize("V", [4_096, 4_099, 8_192, 12_290, 19 * 1024, 19 * 1024 + 1, 31 * 1024 + 5])
+def test_short_rows_that_the_launch_behind_finishes(ctx, V):
+    """Tokens of short rows take the launch over the whole device where nothing cuts them, from 20 segments on where others beside
+    them are cut, and distributions at every length: sharp and flat rows, nuclei of a handful and of thousands."""
+    rng = np.random.default_rng(V)
+    logits = rng.normal(0, 1.5, (8, V)).astype(np.float32)
+    logits[::2, rng.permutation(V)[:12]] += 9.0
+    plain = [SamplingParams(Temperature=0.5 + 0.15 * r) for r in range(8)]
+    mixed = [SamplingParams(Temperature=1.5 if r % 2 else 0.8, TopP=1.0 if r in (0, 3) else 0.95, MinP=0.05 if r == 6 else 0.0) for r in range(8)]
+    cut = [SamplingParams(Temperature=1.5 if r % 2 else 0.6, TopP=0.9 + 0.01 * r) for r in range(8)]
+    for params in (plain, mixed, cut):
+        u = rng.random(8)
+        _check_rows(ctx, logits, params, u)
+        _check_distribution(ctx, logits, params)
+        tokens, _ = ctx.sample_with_distribution(_cuda(logits), params, u)
+        want = [orc.sample_with_distribution(logits[r], to_oracle(params[r]), orc.Rng(replay=[u[r]]))[0] for r in range(8)]
+        assert list(tokens) == want
+
+
+@pytest.mark.parametrize("V, rows, L", [(63 * 1024, 2, 3), (64 * 1024 - 3, 8, 3), (64 * 1024, 9, 3)])
+def test_verification_where_the_launch_behind_starts(ctx, V, rows, L):
+    """The second sum of a verified row, by its workgroup (fewer than 64 segments, more than 32 rows) and by the launch behind it."""
+    params = [SamplingParams(Temperature=0.7 + 0.05 * r) for r in range(rows)]
+    t, q, k, u = _spec_case(rows, L, V, params, V + rows, True)
+    _check_spec(ctx, t, q, k, params, u)
