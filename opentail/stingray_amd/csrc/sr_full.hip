@@ -3962,6 +3962,10 @@ __device__ __forceinline__ void prepared_segment(const SrFullArgs& a, const Prep
     // (the records of the denominator have been walked: theirs take their place)
     seg_make_record<true>(t, seg, (double)(before * r.inv * inv2), a.seg_func + (size_t)slot * a.seg_stride + seg, own);
 }
+// kPhase 0: all of it.  1 and 2: up to the factor, and from there on, as two launches of which neither waits, for launches of several
+// times the workgroups that the device holds (behind_twice): there the ones that wait keep others out, most of all where a
+// row's workgroups do not all fit behind the rows in front of it.
+template <int kPhase>
 __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
 {
     __shared__ float4 room[SR_SEQ_CHAINS * SR_WAVE * 5];  // the block chain by chain, then every wave's segment on its way to 16 terms a lane
@@ -3986,9 +3990,9 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
     for (int hb = lane; hb < 2 * blk; hb += SR_WAVE) before += cs[hb * SR_SEQ_CHAINS + wave];
     if (2 * blk < hb1) own = cs[2 * blk * SR_SEQ_CHAINS + wave];
     if (2 * blk + 1 < hb1) own += cs[(2 * blk + 1) * SR_SEQ_CHAINS + wave];
-    if (!a.lazy_scale && a.mode != 1 && seg < nseg)
+    if (kPhase != 1 && !a.lazy_scale && a.mode != 1 && seg < nseg)
         for (int g = lane; g < seg; g += SR_WAVE) before_seg += sums[g];
-    if (blk < nblk) {
+    if (kPhase != 2 && blk < nblk) {
         before = sr_wave_sum_f32(before) * r.inv;
         // chain by chain in shared memory: the place of term 16 l + j of chain g is g 1024 + 64 j + (l + 2 j) mod 64, so that
         // the lanes of a wave read a term from 64 consecutive places and a piece's stores fall two to a bank
@@ -4007,15 +4011,18 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
         for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = buf[wave * 1024 + 64 * j + ((lane + 2 * j) & 63)];
         seg_make_record<true>(x, blk, (double)before, chain + blk, own * r.inv);
     }
-    sr_drain_stores();
-    __syncthreads();  // (the workgroup's records are out, and nobody reads the block any more)
-    if (tid == 0) {
-        const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bc[0] = ((uint32_t)was & 0xffffu) + 1u == gridDim.x ? 1u : 0u;
+    bool last_in = false;
+    if (kPhase != 2) {
+        sr_drain_stores();
+        __syncthreads();  // (the workgroup's records are out, and nobody reads the block any more)
+        if (tid == 0) {
+            const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bc[0] = ((uint32_t)was & 0xffffu) + 1u == gridDim.x ? 1u : 0u;
+        }
+        __syncthreads();
+        last_in = bc[0] != 0u;
+        if ((kPhase == 1 || a.lazy_scale) && !last_in) return;  // (the last one has all there is to do)
     }
-    __syncthreads();
-    const bool last_in = bc[0] != 0u;
-    if (a.lazy_scale && !last_in) return;  // (the last one has all there is to do)
     // the eight accumulators, a wave each: the sum of the members, and 1 over it
     auto normaliser = [&]() __attribute__((always_inline)) -> float {
         int dummy;
@@ -4047,13 +4054,15 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
     unsigned long long* const factor = sync + 2;  // launch number << 32 | the factor's bits
     float inv2 = 1.0f;
     bool here = true;
-    if (last_in) {
+    if (kPhase == 2) {
+        inv2 = st->mul2;
+    } else if (last_in) {
         inv2 = normaliser();
         if (tid == 0) {
             st->mul2 = inv2;
             sr_store_agent(factor, ((unsigned long long)a.seq << 32) | (unsigned long long)sr_f2u(inv2));
         }
-        if (a.lazy_scale) return;
+        if (kPhase == 1 || a.lazy_scale) return;
     } else {
         if (tid == 0) {
             uint32_t ok = 0u;
@@ -4970,7 +4979,13 @@ hipError_t sr_launch_full_row(const SrFullArgs& a, int n_rows, hipStream_t st)
     hipLaunchKernelGGL(k_full_row, dim3(n_rows), dim3(kT), more, st, a);
     if (a.prepared) {
         const int nseg = (a.vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
-        hipLaunchKernelGGL(k_prepared_row, dim3((unsigned)((nseg + SR_SEQ_CHAINS - 1) / SR_SEQ_CHAINS), n_rows), dim3(kPrepT), 0, st, a);
+        const dim3 grid((unsigned)((nseg + SR_SEQ_CHAINS - 1) / SR_SEQ_CHAINS), n_rows);
+        if (a.behind_twice) {
+            hipLaunchKernelGGL(k_prepared_row<1>, grid, dim3(kPrepT), 0, st, a);
+            hipLaunchKernelGGL(k_prepared_row<2>, grid, dim3(kPrepT), 0, st, a);
+        } else {
+            hipLaunchKernelGGL(k_prepared_row<0>, grid, dim3(kPrepT), 0, st, a);
+        }
     }
     return hipGetLastError();
 }

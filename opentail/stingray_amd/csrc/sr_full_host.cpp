@@ -146,6 +146,15 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             a.chain_sum = ctx->full_chain_sum.as<float>();
             a.chain_func = (SeqSegFunc*)ctx->full_chain_func.p;
             a.prepared = prepared ? 1 : 0;
+            // Two launches of k_prepared_row in place of one whose workgroups wait, from twice the workgroups on that the device
+            // holds, where these are not whole rows.  One and two launches, us: tokens that nothing cuts, 56 rows of
+            // 200,064 97 and 90, 64 of 151,936 90 and 83, 192 of 151,936 199 and 180, 96 of 100,003 88.5 and 85, 160 of 50,257 82 and 80;
+            // whole rows: 128 of 131,072 130 and 141, 48 of 262,144 122 and 124; fewer workgroups: 48 of 151,936 76.5 and 75.5,
+            // beside rows cut by top-p 68 and 70.5.  Distributions of rows that are all cut, whose launch passes memory at most: 48 of
+            // 262,144 106 and 100, 128 of 131,072 114 and 112, 128 of 65,536 69 both.
+            const int blocks = (half_blocks + 1) / 2, held = 2 * ctx->cu_count;
+            a.behind_twice = prepared && !lazy_scale && (long long)n_rows * blocks >= 2 * held &&
+                             (any_plain ? blocks >= 7 && held % blocks != 0 : mode != 0 && blocks >= 12) ? 1 : 0;
             // (up to 1,024 members cost the row's workgroup less than the launch behind it; of short rows more: 256 rows of 12,290, half of
             // them cut to some thousand members, 98 us, with 1,024 134)
             a.finish_most = prepared && nseg >= SR_PREPARED_MIN_SEGS ? 1024 : 8192;

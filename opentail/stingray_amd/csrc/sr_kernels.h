@@ -202,6 +202,7 @@ struct SrFullArgs {
     float* e_rows;                 // [slot][e_stride] expf(x - max) of the rows; starts on 16 bytes
     int64_t e_stride;
     int32_t prepared;              // the launches behind k_full_row follow: it may leave rows to the whole device
+    int32_t behind_twice;          // k_prepared_row as two launches, the second from the factor on
     int32_t finish_most;           // members up to which k_full_row normalises and draws by itself
     uint32_t seq;                  // the launch's number (never 0): see SrFullState::maxkey
     int32_t n_greedy;              // greedy rows behind the others in row_list, whose token k_full_softmax_seg finds (mode 0)

@@ -952,3 +952,23 @@ def test_verification_where_the_launch_behind_starts(ctx, V, rows, L):
     params = [SamplingParams(Temperature=0.7 + 0.05 * r) for r in range(rows)]
     t, q, k, u = _spec_case(rows, L, V, params, V + rows, True)
     _check_spec(ctx, t, q, k, params, u)
+
+
+@pytest.mark.parametrize("V, rows", [(50_257, 150), (98_305, 82)])
+def test_more_rows_than_the_device_holds_at_a_time(ctx, V, rows):
+    """Launches of more than a thousand workgroups behind the row kernel go as two: up to the rows' factors, and from there on.  Rows
+    that nothing cuts and rows of which top-p leaves thousands, tokens and distributions; and distributions of cut rows alone."""
+    rng = np.random.default_rng(V)
+    logits = np.tile(rng.normal(0, 1.5, (10, V)).astype(np.float32), (rows // 10 + 1, 1))[:rows]
+    logits += rng.normal(0, 0.01, (rows, 1)).astype(np.float32)
+    mixed = [SamplingParams(Temperature=0.6 + 0.005 * r) if r % 4 else SamplingParams(Temperature=1.4, TopP=0.97) for r in range(rows)]
+    cut = [SamplingParams(Temperature=0.7 + 0.005 * r, TopP=0.8 + 0.001 * r) for r in range(rows)]
+    u = rng.random(rows)
+    _check_rows(ctx, logits, mixed, u)
+    for params in (mixed, cut):
+        tokens, probs = ctx.sample_with_distribution(_cuda(logits), params, u)
+        probs = probs.cpu().numpy()
+        for r in list(range(0, rows, 9)) + [rows - 1]:
+            t, d = orc.sample_with_distribution(logits[r], to_oracle(params[r]), orc.Rng(replay=[u[r]]))
+            assert tokens[r] == t, r
+            assert np.array_equal(probs[r].view(np.uint32), d.view(np.uint32)), r
