@@ -1124,6 +1124,11 @@ __device__ __forceinline__ bool row_is_listed(const SrRow& rd, const SrFullArgs&
 {
     return !a.lazy_scale && (a.mode == 0 || a.prepared) && a.seg_func != nullptr && rd.temperature > 0.0f && sr_row_cut(rd) && !(rd.top_k > 0 && rd.top_k < a.vocab);
 }
+// A row of the verifier whose drafts are accepted by the ratio test (SpeculativeDecoder.cs:538-548).
+__device__ __forceinline__ bool spec_by_ratio(const SrRow& rd)
+{
+    return !(rd.p_min > 0.0f && rd.p_min < 1.0f) && (rd.flags & SR_ROWBIT_DRAFT_FROM_LOOKUP) == 0u;
+}
 // the longest list that its workgroup takes
 __device__ __forceinline__ int list_cap(bool big) { return big ? SR_LIST_CAP_BIG : SR_LIST_CAP_SMALL; }
 // A sampled row that nothing cuts.
@@ -1131,6 +1136,20 @@ __device__ __forceinline__ bool row_is_plain(const SrRow& rd, const SrFullArgs& 
 {
     return a.seg_func != nullptr && rd.temperature > 0.0f && !sr_row_cut(rd) && !(rd.top_k > 0 && rd.top_k < a.vocab);
 }
+// Rows of the verifier under the ratio test whose e no launch writes down: k_spec_factor makes it for one row of a handful (SrFullState::e_open).
+__device__ __forceinline__ bool row_e_open(const SrRow& rd, const SrFullArgs& a)
+{
+    return a.factor_later && row_is_plain(rd, a) && spec_by_ratio(rd) && rd.edit_cnt == 0 && rd.mask_row < 0;
+}
+// e of a row: where it stands, or expf(x - max) of its fp32 logits, to the last bit what the pass over the whole device had.
+struct ERow {
+    const float* e;   // (starts on 16 bytes)
+    const float* lg;  // at any address; null: e is there
+    float inv_temp, max;
+    const uint64_t* tab;  // of expf, in shared memory
+    __device__ __forceinline__ float of(float x) const { return sr_expf_neg(__fsub_rn(__fmul_rn(x, inv_temp), max), tab); }
+};
+__device__ __forceinline__ float row_inv_temp(const SrRow& rd) { return rd.temperature != 1.0f ? __fdiv_rn(1.0f, rd.temperature) : 1.0f; }
 // Where e = expf(x - max) of a row lies: in the work row, or, where distributions are handed out and the launches behind k_full_row
 // follow, in scratch memory of its own (one place for all rows of a launch, which the host names).
 __device__ __forceinline__ float* row_e(const SrFullArgs& a, int slot) { return a.e_rows + (size_t)slot * (size_t)a.e_stride; }
@@ -1642,7 +1661,8 @@ __device__ __forceinline__ void seg_greedy(const SrFullArgs& a, const SrRow& rd,
     }
 }
 
-template <int ES, int kW, int kS>
+// kLater: a verifier's launch with factor_later (144 rows of 131,072, which do without, were 2 us slower with the test in it)
+template <int ES, int kW, int kS, bool kLater = false>
 __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_seg(SrFullArgs a)
 {
     constexpr int kThreads = kW * SR_WAVE;
@@ -1683,7 +1703,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     // (four segments a wave: the verifier's launches, which list nothing)
     const bool plain = a.prepared && row_is_plain(rd, a), listed = kS != 4 && row_is_listed(rd, a);
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
-    const bool out_now = !a.prepared && ((uintptr_t)w & 15u) == 0u;
+    const bool out_now = !a.prepared && ((uintptr_t)w & 15u) == 0u, open_e = kLater && row_e_open(rd, a);
     // (a row that min-p cuts as well lists everything down to its threshold: entries on it count for SR_OUT_AMBIGUOUS wherever
     // top-p ends)
     const bool by_mass = listed && use_top_p && !(rd.min_p > 0.0f);
@@ -1815,6 +1835,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
 #pragma unroll
         for (int k2 = 0; k2 < K; k2++) {
             const int i0 = seg * SR_SEG_TERMS + (k2 * SR_WAVE + lane) * E;
+            if (kLater && open_e) continue;
             if (i0 + E <= n) {
 #pragma unroll
                 for (int q = 0; q < E; q += 4) {
@@ -3284,6 +3305,8 @@ __device__ __forceinline__ uint32_t row_alone(const SrFullArgs& a, const SrRow& 
 // ---- stage 3: softmax, top-k, min-p, top-p on the work row --------------------------------------------
 // One workgroup per row, one launch: the row is cut, normalised and drawn from here.  A nucleus that the walk by
 // slabs cannot close has its survivors compacted into the row's sort segment and sorted there by this workgroup.
+// kLater: a verifier's launch with factor_later (what that asks for cost all others 0.7 us here)
+template <bool kLater>
 __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
 {
     __shared__ FullSmem sm;
@@ -3383,8 +3406,47 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                 // the whole device has prepared the sum (k_full_softmax_seg): one wave walks the segments' records while the
                 // others fetch the row's list, if it has one
                 if (sr_wave_id() == 0) {
-                    const float s = seg_walk<false>(e_row, n, a.seg_func + (size_t)slot * a.seg_stride, 0.0f, 0.0f, &dummy, nullptr, &first64);
+                    ERow er;
+                    er.e = e_row;
+                    er.lg = nullptr;
+                    if (kLater && row_e_open(rd, a)) {
+                        er.lg = (const float*)a.logits + (size_t)row * (size_t)a.row_stride;
+                        er.inv_temp = row_inv_temp(rd);
+                        er.max = m;
+                        er.tab = (const uint64_t*)sm.sortbuf;  // (no list is fetched beside this walk)
+                        if (sr_lane() < 32) ((uint64_t*)sm.sortbuf)[sr_lane()] = sr_exp2f_tab[sr_lane()];
+                        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                        __builtin_amdgcn_wave_barrier();
+                        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                    }
+                    const bool aligned = ((uintptr_t)e_row & 15u) == 0u;
+                    const float s = seg_walk_from<false>([&](int seg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
+                        const int i0 = seg * SR_SEG_TERMS + sr_lane() * SR_SEQ_RUN;
+                        if (!kLater || !er.lg) {
+                            seq_load_run(e_row, aligned, i0, n, x);
+                            return;
+                        }
+                        if (seg * SR_SEG_TERMS + SR_SEG_TERMS <= n) {
+#pragma unroll
+                            for (int j = 0; j < SR_SEQ_RUN; j += 4) {
+                                const float4 l = sr_load_f4(er.lg + i0 + j);
+                                x[j] = l.x; x[j + 1] = l.y; x[j + 2] = l.z; x[j + 3] = l.w;
+                            }
+                        } else {
+#pragma unroll
+                            for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = er.lg[min(i0 + j, n - 1)];
+                        }
+#pragma unroll
+                        for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = i0 + j < n ? er.of(x[j]) : 0.0f;
+                    }, seg_count(n), a.seg_func + (size_t)slot * a.seg_stride, 0.0f, 0.0f, &dummy, nullptr, &first64);
                     if (sr_lane() == 0) sm.segbc[0] = sr_f2u(s);
+                } else if (kLater && sr_wave_id() == 1) {
+                    // about the same sum, without the roundings of n additions one behind the other (spec_spread)
+                    const int nseg = seg_count(n);
+                    float about = 0.0f;
+                    for (int g = sr_lane(); g < nseg; g += SR_WAVE) about += a.seg_sum[(size_t)slot * a.seg_stride + g];
+                    about = sr_wave_sum_f32(about);
+                    if (sr_lane() == 0) sm.segbc[3] = sr_f2u(about);
                 } else if (has_list) {
                     // where the segments' entries start: every wave adds up the counts for itself and writes all of them, the
                     // same values (a scan by the workgroup, in front of the walk, was two barriers)
@@ -3460,9 +3522,16 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
             FPROF(a, slot, 2);
             const bool do_scale = sum > 0.0f && sum != 1.0f;
             const float inv = do_scale ? __fdiv_rn(1.0f, sum) : 1.0f;
-            if (plain && a.prepared) {
+            // (the verifier asks for the factors of few of its positions: k_spec_factor)
+            if (plain && (a.prepared || (kLater && spec_by_ratio(rd)))) {
                 row_deferred(a, st, inv, -1.0f, 0, sm);
-                if (tid == 0) st->flags = flags;
+                if (tid == 0) {
+                    if (kLater) {
+                        st->e_open = row_e_open(rd, a) ? a.seq : 0u;
+                        st->mul2 = __fdiv_rn(sum, sr_u2f(sm.segbc[3]));
+                    }
+                    st->flags = flags;
+                }
                 return;
             }
             if (a.lazy_scale && a.mode == 1 && !(rd.top_k > 0 && rd.top_k < n) && !(rd.min_p > 0.0f) && !use_top_p) {
@@ -3875,8 +3944,9 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
 // each 4 us before its first byte, and the row read twice -- the same steps took 27 and 38.
 // The wait is bounded: a workgroup whose wait runs out marks the row (SrFullState::late_behind), counts itself in as if it had done
 // its block, and whoever comes last does all blocks of the row again.
+template <bool kLogits>
 struct PreparedRow {
-    const float* e;
+    ERow row;  // (kLogits: of the verifier, whose e may not be there)
     float inv, ycut;
     int idx_last, n;
     __device__ __forceinline__ float cut(float ev, int i) const  // y, or 0 outside the nucleus
@@ -3885,10 +3955,17 @@ struct PreparedRow {
         return (y > ycut) | ((y == ycut) & (i <= idx_last)) ? y : 0.0f;  // (no branch per entry)
     }
 };
-__device__ __forceinline__ PreparedRow prepared_row(const SrFullArgs& a, const SrFullState* st, int slot)
+template <bool kLogits>
+__device__ __forceinline__ PreparedRow<kLogits> prepared_row(const SrFullArgs& a, const SrFullState* st, int slot, const uint64_t* tab, float inv_temp)
 {
-    PreparedRow r;
-    r.e = row_e(a, slot);
+    PreparedRow<kLogits> r;
+    r.row.e = row_e(a, slot);
+    if (kLogits) {
+        r.row.lg = st->e_open == a.seq ? (const float*)a.logits + (size_t)slot * (size_t)a.row_stride : nullptr;  // (the verifier's slots are its rows)
+        r.row.inv_temp = inv_temp;
+        r.row.max = sr_okey_inv((uint32_t)st->maxkey);
+        r.row.tab = tab;
+    }
     r.inv = st->mul1;
     r.ycut = st->ycut;
     r.idx_last = st->idx_last;
@@ -3899,28 +3976,37 @@ constexpr int kPrepT = 512;
 static_assert(kPrepT / SR_WAVE == SR_SEQ_CHAINS, "a wave per chain, and one per segment");
 constexpr int kPrepBlock = SR_SEQ_CHAINS * SR_SEG_TERMS;
 // y of the wave's segment of block blk, as it is loaded: lane l the pieces l, 64 + l, ... of four entries
-__device__ __forceinline__ void prepared_load(const PreparedRow& r, int blk, int wave, int lane, float4 (&v)[4])
+template <bool kLogits>
+__device__ __forceinline__ void prepared_load(const PreparedRow<kLogits>& r, int blk, int wave, int lane, float4 (&v)[4], float4* ev = nullptr)
 {
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int i0 = blk * kPrepBlock + wave * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
         v[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (i0 + 4 <= r.n) {
-            v[k] = *(const float4*)(r.e + i0);  // (the rows of e start on 16-byte boundaries)
+            // (the rows of e start on 16-byte boundaries; what is loaded from the logits becomes e behind all loads)
+            v[k] = kLogits && r.row.lg ? sr_load_f4(r.row.lg + i0) : *(const float4*)(r.row.e + i0);
         } else if (i0 < r.n) {
-            v[k].x = r.e[i0];
-            if (i0 + 1 < r.n) v[k].y = r.e[i0 + 1];
-            if (i0 + 2 < r.n) v[k].z = r.e[i0 + 2];
+            const float* const from = kLogits && r.row.lg ? r.row.lg : r.row.e;
+            v[k].x = from[i0];
+            if (i0 + 1 < r.n) v[k].y = from[i0 + 1];
+            if (i0 + 2 < r.n) v[k].z = from[i0 + 2];
         }
     }
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int i0 = blk * kPrepBlock + wave * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
+        if (kLogits && r.row.lg) {
+            v[k].x = i0 < r.n ? r.row.of(v[k].x) : 0.0f; v[k].y = i0 + 1 < r.n ? r.row.of(v[k].y) : 0.0f;
+            v[k].z = i0 + 2 < r.n ? r.row.of(v[k].z) : 0.0f; v[k].w = i0 + 3 < r.n ? r.row.of(v[k].w) : 0.0f;
+            ev[k] = v[k];
+        }
         v[k].x = r.cut(v[k].x, i0); v[k].y = r.cut(v[k].y, i0 + 1); v[k].z = r.cut(v[k].z, i0 + 2); v[k].w = r.cut(v[k].w, i0 + 3);
     }
 }
 // z of the wave's segment: to the caller's row where the distribution is handed out, and the segment's record for the draw
-__device__ __forceinline__ void prepared_segment(const SrFullArgs& a, const PreparedRow& r, int slot, int row, int seg, int lane, float4 (&v)[4],
+template <bool kLogits>
+__device__ __forceinline__ void prepared_segment(const SrFullArgs& a, const PreparedRow<kLogits>& r, int slot, int row, int seg, int lane, float4 (&v)[4],
                                                  float before, float inv2, float4* turn)
 {
     const int n = r.n;
@@ -3965,35 +4051,44 @@ __device__ __forceinline__ void prepared_segment(const SrFullArgs& a, const Prep
 // kPhase 0: all of it.  1 and 2: up to the factor, and from there on, as two launches of which neither waits, for launches of several
 // times the workgroups that the device holds (behind_twice): there the ones that wait keep others out, most of all where a
 // row's workgroups do not all fit behind the rows in front of it.
+// 3: as 1, for rows whose shares of the accumulators nobody has added up (k_spec_factor): the workgroups meet over them (bounded; what
+// stands in front of a block's terms only has to be about right, so a wait that runs out takes an eighth of the segments' sums).
+struct PreparedSmem {
+    float4 room[SR_SEQ_CHAINS * SR_WAVE * 5];  // the block chain by chain, then every wave's segment on its way to 16 terms a lane
+    float lane_sum[SR_SEQ_CHAINS];
+    uint32_t bc[2];
+};
 template <int kPhase>
-__global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
+__device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, PreparedSmem& sm, const uint64_t* tab = nullptr, float inv_temp = 1.0f)
 {
-    __shared__ float4 room[SR_SEQ_CHAINS * SR_WAVE * 5];  // the block chain by chain, then every wave's segment on its way to 16 terms a lane
-    __shared__ float lane_sum[SR_SEQ_CHAINS];
-    __shared__ uint32_t bc[2];
-    const int slot = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
+    float4* const room = sm.room;
+    float* const lane_sum = sm.lane_sum;
+    uint32_t* const bc = sm.bc;
+    const int blk = blockIdx.x, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
     SrFullState* st = a.state + slot;
-    if (st->deferred != a.seq) return;
-    const int row = a.row_list[slot];
-    const PreparedRow r = prepared_row(a, st, slot);
+    const int row = kPhase == 3 ? slot : a.row_list[slot];
+    const PreparedRow<kPhase == 3> r = prepared_row<kPhase == 3>(a, st, slot, tab, inv_temp);
     const int n = r.n, nv = n / 8, rem = n - nv * 8, body = nv * 8, nblk = (nv + SR_SEG_TERMS - 1) / SR_SEG_TERMS, nseg = seg_count(n);
     unsigned long long* const sync = a.row_sync + (size_t)slot * SR_ROW_SYNC_STRIDE + 1;
     const float* const sums = a.seg_sum + (size_t)slot * a.seg_stride;
     SeqSegFunc* const chain = a.chain_func + ((size_t)slot * SR_SEQ_CHAINS + wave) * a.chain_blocks;
     const int seg = blk * SR_SEQ_CHAINS + wave;
     float4 v[4];
-    prepared_load(r, blk, wave, lane, v);
+    float4 ev[4];  // (phase 3)
+    prepared_load(r, blk, wave, lane, v, ev);
     // about what stands in front of the block's terms of the wave's chain, and of the wave's segment
     const float* const cs = a.chain_sum + (size_t)slot * a.chain_stride;
     float before = 0.0f, before_seg = 0.0f, own = 0.0f;
     const int hb1 = a.chain_stride / SR_SEQ_CHAINS;
-    for (int hb = lane; hb < 2 * blk; hb += SR_WAVE) before += cs[hb * SR_SEQ_CHAINS + wave];
-    if (2 * blk < hb1) own = cs[2 * blk * SR_SEQ_CHAINS + wave];
-    if (2 * blk + 1 < hb1) own += cs[(2 * blk + 1) * SR_SEQ_CHAINS + wave];
-    if (kPhase != 1 && !a.lazy_scale && a.mode != 1 && seg < nseg)
+    if (kPhase != 3) {
+        for (int hb = lane; hb < 2 * blk; hb += SR_WAVE) before += cs[hb * SR_SEQ_CHAINS + wave];
+        if (2 * blk < hb1) own = cs[2 * blk * SR_SEQ_CHAINS + wave];
+        if (2 * blk + 1 < hb1) own += cs[(2 * blk + 1) * SR_SEQ_CHAINS + wave];
+    }
+    if (kPhase != 1 && kPhase != 3 && !a.lazy_scale && a.mode != 1 && seg < nseg)
         for (int g = lane; g < seg; g += SR_WAVE) before_seg += sums[g];
+    float x[SR_SEQ_RUN];
     if (kPhase != 2 && blk < nblk) {
-        before = sr_wave_sum_f32(before) * r.inv;
         // chain by chain in shared memory: the place of term 16 l + j of chain g is g 1024 + 64 j + (l + 2 j) mod 64, so that
         // the lanes of a wave read a term from 64 consecutive places and a piece's stores fall two to a bank
         float* const buf = (float*)room;
@@ -4006,10 +4101,49 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
             at[0] = in ? v[k].x : 0.0f; at[1024] = in ? v[k].y : 0.0f; at[2048] = in ? v[k].z : 0.0f; at[3072] = in ? v[k].w : 0.0f;
         }
         __syncthreads();
-        float x[SR_SEQ_RUN];
 #pragma unroll
         for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = buf[wave * 1024 + 64 * j + ((lane + 2 * j) & 63)];
-        seg_make_record<true>(x, blk, (double)before, chain + blk, own * r.inv);
+    }
+    if (kPhase == 3) {
+        if (blk < nblk) {
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) own += x[j];
+            own = sr_wave_sum_f32(own);
+            if (lane == 0) sr_store_agent(&a.chain_sum[(size_t)slot * a.chain_stride + (size_t)blk * SR_SEQ_CHAINS + wave], own);
+        }
+        sr_drain_stores();
+        __syncthreads();
+        if (tid == 0) {
+            const unsigned long long was = __hip_atomic_fetch_add(sync, 1ull << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            uint32_t ok = ((uint32_t)(was >> 16) & 0xffffu) + 1u == gridDim.x ? 1u : 0u;
+            for (uint32_t it = 0; ok == 0u && it < a.behind_wait_limit; it++) {
+                ok = ((uint32_t)(sr_load_agent(sync) >> 16) & 0xffffu) == gridDim.x ? 1u : 0u;
+                if (ok == 0u) __builtin_amdgcn_s_sleep(1);
+            }
+            bc[0] = ok;
+        }
+        __syncthreads();
+        if (blk < nblk) {
+            if (bc[0] != 0u) {
+                for (int b = lane; b < blk; b += SR_WAVE) before += sr_load_agent(&cs[b * SR_SEQ_CHAINS + wave]);
+            } else {
+                for (int g = lane; g < blk * SR_SEQ_CHAINS; g += SR_WAVE) before += sums[g] * (r.inv / SR_SEQ_CHAINS);
+            }
+        }
+    }
+    if (kPhase == 3 && r.row.lg) {
+        // (behind the meeting: a barrier waits for what is on its way to memory, and this is only needed by whoever counts in last.
+        // The rows of e are whole pieces long)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i0 = blk * kPrepBlock + wave * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
+            if (i0 < n) sr_store_agent_f4((float4*)(const_cast<float*>(r.row.e) + i0), ev[k].x, ev[k].y, ev[k].z, ev[k].w);
+        }
+    }
+    if (kPhase != 2 && blk < nblk) {
+        const float by = kPhase == 3 ? 1.0f : r.inv;  // (what phase 3 has added up is normalised already)
+        before = sr_wave_sum_f32(before) * by;
+        seg_make_record<true>(x, blk, (double)before, chain + blk, own * by);
     }
     bool last_in = false;
     if (kPhase != 2) {
@@ -4021,7 +4155,7 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
         }
         __syncthreads();
         last_in = bc[0] != 0u;
-        if ((kPhase == 1 || a.lazy_scale) && !last_in) return;  // (the last one has all there is to do)
+        if ((kPhase == 1 || kPhase == 3 || a.lazy_scale) && !last_in) return;  // (the last one has all there is to do)
     }
     // the eight accumulators, a wave each: the sum of the members, and 1 over it
     auto normaliser = [&]() __attribute__((always_inline)) -> float {
@@ -4030,18 +4164,18 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
             // (no condition stands between the loads: with one each they wait for each other; a whole block by offsets from one
             // address)
             const int t0 = b * SR_SEG_TERMS + lane * SR_SEQ_RUN;
-            const float* const e0 = r.e + (size_t)t0 * 8 + wave;
+            const float* const e0 = r.row.e + (size_t)t0 * 8 + wave;
             if ((b + 1) * SR_SEG_TERMS <= nv) {
 #pragma unroll
                 for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = e0[j * 8];
             } else {
 #pragma unroll
-                for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = r.e[min(t0 + j, nv - 1) * 8 + wave];
+                for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = e0[(min(t0 + j, nv - 1) - t0) * 8];
             }
 #pragma unroll
             for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = t0 + j < nv ? r.cut(x[j], (t0 + j) * 8 + wave) : 0.0f;
         }, nblk, chain, 0.0f, 0.0f, &dummy, nullptr);
-        if (rem > 0 && wave >= 8 - rem) s = __fadd_rn(s, r.cut(r.e[n - 8 + wave], n - 8 + wave));  // the overlapped last vector
+        if (rem > 0 && wave >= 8 - rem) s = __fadd_rn(s, r.cut(r.row.e[n - 8 + wave], n - 8 + wave));  // the overlapped last vector
         if (lane == 0) lane_sum[wave] = s;
         __syncthreads();
         const float l0 = lane_sum[0], l1 = lane_sum[1], l2 = lane_sum[2], l3 = lane_sum[3], l4 = lane_sum[4], l5 = lane_sum[5],
@@ -4049,6 +4183,8 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
         const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
         return (sum > 0.0f && sum != 1.0f) ? __fdiv_rn(1.0f, sum) : 1.0f;
     };
+    // (phase 3: the row's workgroups wrote e just now, through to memory; blocks and rows start on lines of their own, so no cache
+    // holds one of these lines from before it was written)
     // Whoever counts in last walks them, and the others wait for the factor.  (All workgroups of the row walking for themselves, the
     // same work: 512 of them, at 16 rows of 262,144, fetched 12 MB of records past the caches and took 2.6 - 8 us for it.)
     unsigned long long* const factor = sync + 2;  // launch number << 32 | the factor's bits
@@ -4060,9 +4196,10 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
         inv2 = normaliser();
         if (tid == 0) {
             st->mul2 = inv2;
+            if (kPhase == 3) st->e_open = 0u;
             sr_store_agent(factor, ((unsigned long long)a.seq << 32) | (unsigned long long)sr_f2u(inv2));
         }
-        if (kPhase == 1 || a.lazy_scale) return;
+        if (kPhase == 1 || kPhase == 3 || a.lazy_scale) return;
     } else {
         if (tid == 0) {
             uint32_t ok = 0u;
@@ -4109,15 +4246,24 @@ __global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
     int found;
     const float at = seg_walk_from<true, true>([&](int sg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
         const int i0 = sg * SR_SEG_TERMS + lane * SR_SEQ_RUN;
-        seq_load_run(r.e, true, i0, n, x);  // (zeros past the end stay zeros)
+        seq_load_run(r.row.e, true, i0, n, x);  // (zeros past the end stay zeros)
 #pragma unroll
         for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = __fmul_rn(r.cut(x[j], i0 + j), inv2);
     }, nseg, a.seg_func + (size_t)slot * a.seg_stride, 0.0f, u, &found, nullptr);
     if (lane == 0) {
-        const bool amb = found >= 0 ? sr_stop_near(at, __fmul_rn(r.cut(r.e[found], found), inv2), u) : sr_near(at, u);
+        const bool amb = found >= 0 ? sr_stop_near(at, __fmul_rn(r.cut(r.row.e[found], found), inv2), u) : sr_near(at, u);
         if (a.out_tokens) a.out_tokens[row] = found >= 0 ? found : n - 1;
         if (a.out_flags) a.out_flags[row] = st->flags | (amb ? SR_KFLAG_AMBIGUOUS : 0u);
     }
+}
+
+template <int kPhase>
+__global__ __launch_bounds__(kPrepT, 4) void k_prepared_row(SrFullArgs a)
+{
+    __shared__ PreparedSmem sm;
+    const int slot = blockIdx.y;
+    if (a.state[slot].deferred != a.seq) return;
+    prepared_block<kPhase>(a, slot, sm);
 }
 
 // ---- SampleTopK (Sampler.cs:216-357) for rows wider than the selection kernel takes -----------------------
@@ -4434,6 +4580,27 @@ struct SpecTerms {
         for (int k = 0; k < 4; k++) { x[4 * k] = v[k].x; x[4 * k + 1] = v[k].y; x[4 * k + 2] = v[k].z; x[4 * k + 3] = v[k].w; }
     }
 };
+// e of token tok at a position of the verifier's batch (both of its places are asked for beside the state that says which holds)
+__device__ __forceinline__ float spec_e(const SrSpecArgs& a, const SrRow& rd, size_t slot, int tok, const uint64_t* tab)
+{
+    const SrFullState* sl = a.state + slot;
+    const uint32_t open = sl->e_open;
+    const float there = a.p_all[slot * (size_t)a.p_stride + tok], x = a.target_logits[slot * (size_t)a.vocab + tok];
+    ERow r;
+    r.inv_temp = row_inv_temp(rd);
+    r.max = sr_okey_inv((uint32_t)sl->maxkey);
+    r.tab = tab;
+    const float made = r.of(x);
+    return open == a.seq ? made : there;
+}
+__device__ __forceinline__ void spec_table(uint64_t* tab)  // by the first wave, which uses it first
+{
+    if (threadIdx.x < 32) tab[threadIdx.x] = sr_exp2f_tab[threadIdx.x];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+__device__ __forceinline__ float spec_accept(float px, float qx) { return qx > 0.0f ? fminf(1.0f, __fdiv_rn(px, qx)) : (px > 0.0f ? 1.0f : 0.0f); }
 // The accept loop of a row under the ratio test needs one element of p and of q per position, no pass over a row:
 // one wave walks it ahead of everything else and names the first rejected position, so that the residual row of
 // that position -- which the row's workgroup would otherwise compute twice, from two rows, at the rate of one compute
@@ -4443,7 +4610,7 @@ __global__ __launch_bounds__(SR_WAVE) void k_spec_walk(SrSpecArgs a)
     const int row = blockIdx.x, lane = sr_lane();
     const SrRow rd = a.rows[row];
     const int n = a.vocab, L = a.n_draft;
-    const bool true_spec = !(rd.p_min > 0.0f && rd.p_min < 1.0f) && (rd.flags & SR_ROWBIT_DRAFT_FROM_LOOKUP) == 0u;
+    const bool true_spec = spec_by_ratio(rd);
     int reject = -1;
     if (true_spec) {
         const float* pr = a.p_all + (size_t)row * (L + 1) * (size_t)a.p_stride;
@@ -4458,7 +4625,7 @@ __global__ __launch_bounds__(SR_WAVE) void k_spec_walk(SrSpecArgs a)
                     const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
                     const float px = __fmul_rn(__fmul_rn(pr[(size_t)i * (size_t)a.p_stride + tok], sl->mul1), sl->mul2);
                     const float qx = a.draft_probs[((size_t)row * L + i) * n + tok];
-                    const float acc = qx > 0.0f ? fminf(1.0f, __fdiv_rn(px, qx)) : (px > 0.0f ? 1.0f : 0.0f);
+                    const float acc = spec_accept(px, qx);
                     stop = !(u[i] < (double)acc);  // (every position before it was accepted and drew one uniform)
                 }
             }
@@ -4494,6 +4661,69 @@ __global__ __launch_bounds__(256) void k_spec_residual(SrSpecArgs a)
     // (the rows of a.resid start on 16 bytes and are a multiple of 16 bytes long)
 }
 
+// The factors 1 / (sum of the probabilities) of the final Normalize (Sampler.cs:91-92), for the positions that need theirs.  A row
+// that nothing cuts has probabilities fl(fl(e m1) m2), m1 = fl(1 / s) with s the sum of e added one behind the other, and m2 hangs on
+// the exact sum of all fl(e m1) in the eight accumulators.  About the sum of e, S, is known from the segments' sums to 50
+// roundings, so m2 is s / S but for those and the n / 8 additions of an accumulator (all terms are positive): spec_spread(n), 0.2 % at
+// 262,144.  Nearly every accept test comes out the same at both ends.  What needs m2 itself: the positions in front of the first
+// certain rejection whose test is open, and the position that the row draws from.  k_full_row leaves all of them at s / S
+// (SrFullState::deferred), a workgroup per block of a row's 8,192 entries finds those positions for itself, a position a lane, and
+// takes them as k_prepared_row takes a row up to the factor.  The positions left at s / S are tested with that.
+// So e of the others is read nowhere but at their draft token, and is not written at all (row_e_open).  What bounds it: the chain again, two trips
+// for the positions 2.4 us, the block from its logits 10 - 12 us (expf of 16 entries a lane is a third), the meeting 4 - 5, records 3, the
+// walk 5.  144 rows of 262,144, us: k_full_softmax_seg 72 -> 59, k_full_row, whose workgroups made the sums of all of them, 48 -> 15, this
+// one 28; the call 143 -> 127.  (e stored in front of the meeting, whose barrier waits for it: this kernel 30.)
+__device__ __forceinline__ double spec_spread(int n) { return ((double)(n / 8) + 200.0) * (1.1 / 16777216.0) + 1e-6; }
+__global__ __launch_bounds__(kPrepT, 4) void k_spec_factor(SrFullArgs a, SrSpecArgs s)
+{
+    __shared__ PreparedSmem sm;
+    __shared__ unsigned long long said;
+    __shared__ uint64_t tab[32];
+    const int row = blockIdx.y, lane = sr_lane();
+    const SrRow rd = s.rows[row];
+    if (!spec_by_ratio(rd)) return;
+    const int n = s.vocab, L = s.n_draft;  // (L < SR_WAVE)
+    if (sr_wave_id() == 0) {
+        spec_table(tab);
+        bool open = false, ends = false, bad = false;
+        if (lane < L) {
+            const int tok = s.draft_tokens[(size_t)row * L + lane];
+            bad = (uint32_t)tok >= (uint32_t)n;
+            if (!bad) {
+                const SrFullState* sl = s.state + (size_t)row * (L + 1) + lane;
+                const bool any = sl->deferred == a.seq;  // m2 is s / S so far
+                const float y = __fmul_rn(spec_e(s, rd, (size_t)row * (L + 1) + lane, tok, tab), sl->mul1);
+                const float qx = s.draft_probs[((size_t)row * L + lane) * n + tok];
+                const double u = s.uniforms[(size_t)row * s.uniforms_per_row + lane];
+                const float acc = spec_accept(__fmul_rn(y, sl->mul2), qx);
+                ends = !(u < (double)acc);
+                if (any && y > 0.0f) {
+                    if (!(qx > 0.0f)) {
+                        open = y < 1e-30f;
+                    } else {
+                        const double ratio = (double)y * (double)sl->mul2 / (double)qx, d = spec_spread(n);
+                        const bool low = u < fmin(1.0, ratio * (1.0 - d)), high = u < fmin(1.0, ratio * (1.0 + d));
+                        open = low != high || y < 1e-30f || !(ratio >= 1e-30);  // (relative bounds end where numbers lose digits)
+                    }
+                }
+            }
+        }
+        const unsigned long long end = __ballot(!open && (ends || bad)), wrong = __ballot(bad), undecided = __ballot(open);
+        const int last = end != 0ull ? (int)__ffsll((long long)end) - 1 : L;
+        unsigned long long pick = undecided & ((1ull << last) - 1ull);
+        if (((wrong >> last) & 1ull) == 0ull) pick |= 1ull << last;  // (an id outside the vocabulary ends the row without a draw)
+        if (lane == 0) said = pick;
+    }
+    __syncthreads();
+    const float inv_temp = row_inv_temp(rd);
+    for (unsigned long long pick = said; pick != 0ull; pick &= pick - 1ull) {
+        const int slot = row * (L + 1) + (int)__ffsll((long long)pick) - 1;
+        if (a.state[slot].deferred != a.seq) continue;
+        prepared_block<3>(a, slot, sm, tab, inv_temp);
+        __syncthreads();
+    }
+}
+
 // ---- speculative verification of rows under the ratio test (StepSampled, SpeculativeDecoder.cs:530-559) --------------------
 // The accept loop of such a row needs one element of p and of q per position, and the draw behind it one row of terms: max(0,
 // fl(fl(p m1) m2) - q) of the first rejected position, or the scaled target row fl(fl(p m1) m2) of the bonus position when every
@@ -4527,25 +4757,27 @@ __device__ __forceinline__ float spec_sum_alone(const SpecTerms& t, int nseg, fl
     }
     return s;
 }
+template <bool kLater>  // k_spec_factor was launched in front
 __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
 {
     __shared__ float4 turn_all[kSpecWaves][SR_WAVE * 5];
     __shared__ float states[SR_SEG_MAX];  // every segment's part of the sum, then the running sum behind every segment
     __shared__ uint32_t bc;
     __shared__ int said[2];
+    __shared__ uint64_t tab[32];
     const int row = blockIdx.y, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
     const SrRow rd = a.rows[row];
     const int n = a.vocab, L = a.n_draft, nseg = seg_count(n);
     unsigned long long* const sync = a.sync + (size_t)row * SR_ROW_SYNC_STRIDE;
-    if ((rd.p_min > 0.0f && rd.p_min < 1.0f) || (rd.flags & SR_ROWBIT_DRAFT_FROM_LOOKUP) != 0u) {
+    if (!spec_by_ratio(rd)) {
         if (blockIdx.x == 0 && tid == 0) a.reject[row] = -1;
         return;
     }
     const double* const u = a.uniforms + (size_t)row * a.uniforms_per_row;
     if (wave == 0) {
+        if (kLater) spec_table(tab);
         // the first position that is not accepted: kind 0 rejected, 1 none (position L), 2 an id outside the vocabulary, which
         // ends the row without a correction
-        const float* const pr = a.p_all + (size_t)row * (L + 1) * (size_t)a.p_stride;
         int pos = L, kind = 1;
         for (int i0 = 0; i0 < L; i0 += SR_WAVE) {
             const int i = i0 + lane;
@@ -4555,9 +4787,10 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
                 bad = (uint32_t)tok >= (uint32_t)n;
                 if (!bad) {
                     const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
-                    const float px = __fmul_rn(__fmul_rn(pr[(size_t)i * (size_t)a.p_stride + tok], sl->mul1), sl->mul2);
+                    const float px = __fmul_rn(__fmul_rn(kLater ? spec_e(a, rd, (size_t)row * (L + 1) + i, tok, tab)
+                                                            : a.p_all[((size_t)row * (L + 1) + i) * (size_t)a.p_stride + tok], sl->mul1), sl->mul2);
                     const float qx = a.draft_probs[((size_t)row * L + i) * n + tok];
-                    const float acc = qx > 0.0f ? fminf(1.0f, __fdiv_rn(px, qx)) : (px > 0.0f ? 1.0f : 0.0f);
+                    const float acc = spec_accept(px, qx);
                     stop = !(u[i] < (double)acc);  // (every position before it was accepted and drew one uniform)
                 }
             }
@@ -4594,7 +4827,7 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
         return;
     }
     SpecTerms t;
-    t.p = a.p_all + ((size_t)row * (L + 1) + pos) * (size_t)a.p_stride;
+    t.p = a.p_all + ((size_t)row * (L + 1) + pos) * (size_t)a.p_stride;  // (k_spec_factor has seen to it that e is there)
     t.q = kind == 0 ? a.draft_probs + ((size_t)row * L + pos) * n : nullptr;
     {
         const SrFullState* sl = a.state + (size_t)row * (L + 1) + pos;
@@ -4715,7 +4948,7 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
     const double* u = a.uniforms + (size_t)row * a.uniforms_per_row;
     int* out = a.out_tokens + (size_t)row * (L + 1);
     // SpeculativeDecoder.cs:192 and :538, :549 (`_trueSpecSampling && !usedPld`)
-    const bool true_spec = !(rd.p_min > 0.0f && rd.p_min < 1.0f) && (rd.flags & SR_ROWBIT_DRAFT_FROM_LOOKUP) == 0u;
+    const bool true_spec = spec_by_ratio(rd);
     for (int i = threadIdx.x; i <= L; i += kT) out[i] = -1;
     __syncthreads();
     int accepted = 0, udraws = 0, correction = -1;
@@ -4750,7 +4983,7 @@ __global__ __launch_bounds__(kT) void k_spec_verify(SrSpecArgs a)
         bool accept;
         if (true_spec) {
             const float qx = staged ? sm.sprob[kStage + i] : qd[tok];
-            const float acc = qx > 0.0f ? fminf(1.0f, __fdiv_rn(px, qx)) : (px > 0.0f ? 1.0f : 0.0f);
+            const float acc = spec_accept(px, qx);
             const double ui = staged ? __longlong_as_double((long long)sm.sortbuf[udraws]) : u[udraws];
             udraws++;
             accept = ui < (double)acc;
@@ -4914,14 +5147,15 @@ hipError_t sr_launch_full_prep(const SrFullArgs& a, int n_rows, hipStream_t st)
         // of 151,936, whole step: 56.6 against 58.9 us).  Four for the verifier's large launches, whose waves keep nothing
         // else in registers (144 rows of 262,144: 98 -> 92 us; 36 rows: 119.6 -> 121.6 a call).
         const long long segs = (long long)(a.n_sampled + a.n_greedy) * nseg;
-        const bool four = a.lazy_scale && a.dtype != 1 && segs > 12288, two = segs > 3072;
+        const bool four = a.factor_later || (a.lazy_scale && a.dtype != 1 && segs > 12288), two = segs > 3072;
         const int per_group = 4 * (four ? 4 : two ? 2 : 1);
         dim3 fgrid((unsigned)((nseg + per_group - 1) / per_group), n_rows + a.n_greedy);
         if (a.dtype == 1) {
             if (two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2>), fgrid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 1>), fgrid, dim3(256), 0, st, a);
         } else {
-            if (four) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 4>), fgrid, dim3(256), 0, st, a);
+            if (a.factor_later) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 4, true>), fgrid, dim3(256), 0, st, a);
+            else if (four) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 4>), fgrid, dim3(256), 0, st, a);
             else if (two) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 2>), fgrid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 1>), fgrid, dim3(256), 0, st, a);
         }
@@ -4971,12 +5205,15 @@ hipError_t sr_launch_full_row(const SrFullArgs& a, int n_rows, hipStream_t st)
         hipError_t e = hipGetDevice(&dev);
         if (e != hipSuccess) return e;
         if (dev < 0 || dev >= 64 || !allowed[dev]) {
-            e = hipFuncSetAttribute((const void*)k_full_row, hipFuncAttributeMaxDynamicSharedMemorySize, (int)more);
-            if (e != hipSuccess) return e;
+            for (const void* k : {(const void*)k_full_row<false>, (const void*)k_full_row<true>}) {
+                e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)more);
+                if (e != hipSuccess) return e;
+            }
             if (dev >= 0 && dev < 64) allowed[dev] = true;
         }
     }
-    hipLaunchKernelGGL(k_full_row, dim3(n_rows), dim3(kT), more, st, a);
+    if (a.factor_later) hipLaunchKernelGGL(k_full_row<true>, dim3(n_rows), dim3(kT), more, st, a);
+    else hipLaunchKernelGGL(k_full_row<false>, dim3(n_rows), dim3(kT), more, st, a);
     if (a.prepared) {
         const int nseg = (a.vocab + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
         const dim3 grid((unsigned)((nseg + SR_SEQ_CHAINS - 1) / SR_SEQ_CHAINS), n_rows);
@@ -5018,7 +5255,15 @@ hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, hipStream_t st)
         b.resid = nullptr;
         b.reject = nullptr;
     } else if (b.seg_func) {
-        hipLaunchKernelGGL(k_spec_rows, dim3((unsigned)((seg_count_of(b.vocab) + kSpecWaves - 1) / kSpecWaves), rows), dim3(kSpecT), 0, st, b);
+        const dim3 grid((unsigned)((seg_count_of(b.vocab) + kSpecWaves - 1) / kSpecWaves), rows);
+        static_assert(kSpecWaves == SR_SEQ_CHAINS && kSpecT == kPrepT, "the same blocks of a row");
+        b.open_factors = nullptr;
+        if (a.open_factors) {
+            hipLaunchKernelGGL(k_spec_factor, grid, dim3(kPrepT), 0, st, *a.open_factors, b);
+            hipLaunchKernelGGL(k_spec_rows<true>, grid, dim3(kSpecT), 0, st, b);
+        } else {
+            hipLaunchKernelGGL(k_spec_rows<false>, grid, dim3(kSpecT), 0, st, b);
+        }
         if (!b.any_other) return hipGetLastError();
     } else {
         const int nseg = seg_count_of(b.vocab);

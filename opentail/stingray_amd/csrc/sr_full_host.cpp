@@ -8,11 +8,15 @@
 
 namespace {
 
+// a row of the verifier whose drafts are accepted by the ratio test
+bool by_ratio(const SrRow& r) { return !(r.p_min > 0.0f && r.p_min < 1.0f) && !(r.flags & SR_ROW_DRAFT_FROM_LOOKUP); }
+
 // Runs the full-vocabulary pipeline for the rows in `list` (device array of n_rows row indices).
 //   mode 0: work rows live in ctx scratch, tokens out.   mode 1/2: work rows ARE the caller's probs rows.
 int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows, bool any_top_p, const void* logits_dev,
              int dtype, int64_t row_stride, int mode, float* probs_dev, int64_t probs_stride, int32_t* out_tokens_dev,
-             uint32_t* out_flags_dev, bool lazy_scale = false, const std::vector<SrRow>* host_rows = nullptr, int n_greedy = 0)
+             uint32_t* out_flags_dev, bool lazy_scale = false, const std::vector<SrRow>* host_rows = nullptr, int n_greedy = 0,
+             SrFullArgs* factor_later = nullptr)
 {
     if (n_rows <= 0) return SR_OK;
     hipStream_t st = ctx->stream;
@@ -77,6 +81,10 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     const long long segs = (long long)n_rows * nseg;
     if (lazy_scale) {
         prepared = prepared && nseg >= SR_PREPARED_MIN_SEGS_VERIFY && n_rows <= SR_PREPARED_ROWS_VERIFY;
+        if (factor_later && any_plain && seg_mode && dtype == SR_DTYPE_F32 && segs >= (n_rows > ctx->cu_count ? SR_FACTOR_LATER_SEGS : SR_FACTOR_LATER_SEGS_FEW)) {
+            a.factor_later = 1;
+            prepared = false;
+        }
     } else if (mode != 0) {
         prepared = prepared && segs <= SR_PREPARED_SEGS_DISTRIBUTIONS;
     } else {
@@ -179,6 +187,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
 
     SR_HIP(ctx, sr_launch_full_prep(a, n_rows, st));
     SR_HIP(ctx, sr_launch_full_row(a, n_rows, st));  // (every row is finished by this one launch)
+    if (factor_later) *factor_later = a;
     return SR_OK;
 }
 
@@ -493,7 +502,7 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
         // only rows under the ratio test read q (SpeculativeDecoder.cs:538-543)
         for (int r = 0; r < b->rows; r++) {
             const SrRow& d = b->h_rows[(size_t)r];
-            if (!(d.p_min > 0.0f && d.p_min < 1.0f) && !(d.flags & SR_ROW_DRAFT_FROM_LOOKUP))
+            if (by_ratio(d))
                 return sr_fail(ctx, SR_ERR_NULL_ARGUMENT, "sr_spec_verify_launch: a row under the ratio test needs the draft distributions");
         }
     }
@@ -515,7 +524,7 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
         SR_HIP(ctx, sr_launch_expand_rows(b->d_rows.as<SrRow>(), b->spec_rows.as<SrRow>(), rows, P, st));
         b->spec_positions = P;
     }
-    const int64_t p_stride = ((int64_t)V + 3) & ~(int64_t)3;  // (rows of e start on 16-byte boundaries)
+    const int64_t p_stride = ((int64_t)V + 63) & ~(int64_t)63;  // (no row of e shares a cache line with another: k_spec_factor)
     SR_HIP(ctx, ctx->spec_probs.reserve((size_t)rows * P * (size_t)p_stride * sizeof(float), st));
     sr_batch tmp;  // a view: expanded rows, the original edits
     tmp.ctx = ctx;
@@ -527,9 +536,11 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     tmp.mask_stride = 0;
     const int32_t* list = nullptr;
     int rc = identity_list(ctx, rows * P, &list);
+    SrFullArgs full{};
+    const bool in_one = n_draft > 0 && n_draft < 64 && draft_probs_dev && rows <= 65535;  // (k_spec_factor: a position a lane)
     if (rc == SR_OK)
         rc = run_full(ctx, &tmp, list, rows * P, any_top_p, target_logits_dev, SR_DTYPE_F32, V, 1, ctx->spec_probs.as<float>(), p_stride,
-                      nullptr, nullptr, true, &b->h_rows);  // (the verifier applies the normalising factors of unfiltered rows itself)
+                      nullptr, nullptr, true, &b->h_rows, 0, in_one ? &full : nullptr);  // (the verifier applies the normalising factors of unfiltered rows itself)
     tmp.d_rows.p = nullptr;  // borrowed
     tmp.d_edits.p = nullptr;
     if (rc != SR_OK) return rc;
@@ -567,8 +578,9 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     }
     for (int r = 0; r < rows; r++) {
         const SrRow& d = b->h_rows[(size_t)r];
-        if ((d.p_min > 0.0f && d.p_min < 1.0f) || (d.flags & SR_ROW_DRAFT_FROM_LOOKUP) || !(d.temperature > 0.0f)) a.any_other = 1;
+        if (!by_ratio(d) || !(d.temperature > 0.0f)) a.any_other = 1;
     }
+    if (full.factor_later) a.open_factors = &full;
     SR_HIP(ctx, sr_launch_spec_verify(a, rows, st));
     return SR_OK;
 }

@@ -147,7 +147,8 @@ struct SrFullState {
     uint32_t list_from;   // the row's list of candidates holds its e from this value on (as bits); 0: it would have been too long
     uint32_t late_behind; // the number of the last launch in which a workgroup of k_prepared_row stopped waiting for the row's others
     float u;              // the uniform of the draw, of a row left to the whole device
-    int32_t pad[3];
+    uint32_t e_open;      // the number of the last launch that did not write the row's e down: its reader takes it from the logits
+    int32_t pad[2];
 };
 static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // SrFullArgs::row_sync, a word per row (rows 256 bytes apart: every workgroup of a row adds to its word and polls it):
@@ -202,6 +203,7 @@ struct SrFullArgs {
     float* e_rows;                 // [slot][e_stride] expf(x - max) of the rows; starts on 16 bytes
     int64_t e_stride;
     int32_t prepared;              // the launches behind k_full_row follow: it may leave rows to the whole device
+    int32_t factor_later;          // lazy_scale: mul2 of rows that nothing cuts is left to k_spec_factor, under the ratio test
     int32_t behind_twice;          // k_prepared_row as two launches, the second from the factor on
     int32_t finish_most;           // members up to which k_full_row normalises and draws by itself
     uint32_t seq;                  // the launch's number (never 0): see SrFullState::maxkey
@@ -268,6 +270,7 @@ struct SrSpecArgs {
     int32_t seg_stride;
     unsigned long long* sync;    // [row * SR_ROW_SYNC_STRIDE]: as SrFullArgs::row_sync, and behind it the last launch in which a wait ran out
     uint32_t seq, wait_limit;
+    const SrFullArgs* open_factors;  // on the host: the launch that left factors open (SrFullArgs::factor_later), or null; n_draft < 64
     int32_t any_other;           // some row is not under the ratio test, or greedy: k_spec_verify follows
     // ... and of more:
     float* resid;                // [rows][resid_stride]: max(0, p - q) of the row's first rejected position

@@ -119,6 +119,11 @@ struct SrMaskClear {
 // The verifier, where the workgroup passes over its row once and not three times, so that the number of rows decides: of 65,536 3
 // rows 44 against 48, 32 rows 51 against 53, 45 rows 56 against 54; of 131,072 44 against 55, 59 against 68, 72 against 70; of
 // 262,144 50 against 74, 88 against 93, 106 against 98; of 32,768 3 rows 40 against 42, 24 rows 47 against 45.
+// From so many segments on, fewer where every row has a compute unit to itself in k_full_row, the verifier's second sums are left to
+// k_spec_factor instead, and e is not written down: calls of 144 rows (16 sequences of 8 drafts) of 262,144 128 us against 143, 80 rows
+// of it 102 against 106, 192 of 151,936 108 against 111, 176 of 131,072 94 against 97, 144 of it (18,432 segments) 88 against 86, 96 of
+// 151,936 92 against 85; 448 rows of 65,536 108 against 118, 576 of 32,768 92 against 99, 288 of 50,257 (14,400) 84 against 92, 224 of
+// it 78 against 70, 384 of 32,768 (12,288) 84 against 77, 2,304 of 16,384 153 against 210, 768 of it 89 against 83.
 #define SR_PREPARED_MIN_SEGS 32        // tokens, rows that are cut
 #define SR_PREPARED_MIN_SEGS_MIXED 20  // ... beside rows that are not
 #define SR_PREPARED_ROWS_MIXED 128
@@ -126,6 +131,8 @@ struct SrMaskClear {
 #define SR_PREPARED_SEGS_DISTRIBUTIONS 20480
 #define SR_PREPARED_MIN_SEGS_VERIFY 64
 #define SR_PREPARED_ROWS_VERIFY 32
+#define SR_FACTOR_LATER_SEGS 14336
+#define SR_FACTOR_LATER_SEGS_FEW 20480
 // Distributions of rows that min-p cuts, where no other row asks for that launch: worth it for few long rows.  Some ten entries left,
 // 16 rows of 65,536: 36 us against 34, of 131,072 43 against 49, of 262,144 59 against 80.  When three launches did its work, 20,
 // 200, 2,000, 8,000 and 15,000 entries left, 16 rows of 262,144: 71, 98, 106, 120, 143 us against 88, 99, 118, 181, 184 without;

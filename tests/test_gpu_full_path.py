@@ -357,6 +357,49 @@ def test_verification_by_one_launch_and_by_the_workgroups_that_come_last(ctx, V,
         ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
 
 
+# a block and a half of a block to a row, odd rows, long ones; 64 drafts: every position's factor is worked out.  Launches of
+# 14,336 segments and more, and of 20,480 where they have fewer rows than compute units; waits that run out in the launch behind, and in the pass itself
+@pytest.mark.parametrize("V, rows, L, polls", [(4_096, 56, 64, 1 << 15), (4_097, 46, 63, 1 << 15), (8_193, 25, 63, 0x80000000), (8_193, 25, 63, 0x80000002),
+                                               (70_001, 36, 5, 1 << 15), (70_001, 36, 5, 0), (300_001, 24, 2, 1 << 15)])
+def test_accept_tests_that_hang_on_the_last_digits(ctx, V, rows, L, polls):
+    """Rows that nothing cuts: the verifier works out the factor of the final Normalize for the positions whose accept test is open
+    without it, and for the one that is drawn from.  Uniforms on the ratio p / q, one step of a double below it, and so far
+    from it that it decides without the factor, or hardly; a draft that q gives nothing, one of no probability at all; beside them
+    rows of the other rule, with a bias, cut by top-p, and greedy ones."""
+    rng = np.random.default_rng(V + L)
+    kinds = [SamplingParams(), SamplingParams(Temperature=0.7), SamplingParams(Temperature=0.9, SpecDraftPMin=0.3), SamplingParams(LogitBias={5: 1.0}),
+             SamplingParams(Temperature=0.8, TopP=0.9), SamplingParams(Temperature=0.0)]
+    params = [kinds[r % 8] if r % 8 < 6 else SamplingParams(Temperature=0.6 + 0.02 * r) for r in range(rows)]
+    base = synthetic.zipf_head_logits(rng, rows * L, V).reshape(rows, L, V)
+    t = np.empty((rows, L + 1, V), dtype=np.float32)
+    t[:, :L] = base + rng.normal(0, 0.1, (rows, 1, V)).astype(np.float32)
+    t[:, L] = synthetic.zipf_head_logits(rng, rows, V)
+    q = np.exp(base - base.max(axis=2, keepdims=True))
+    q /= q.sum(axis=2, keepdims=True)
+    k = rng.integers(0, 20, (rows, L))
+    k = np.take_along_axis(np.argpartition(-base, 20, axis=2), k[:, :, None], axis=2)[:, :, 0].astype(np.int32)
+    u = rng.random((rows, L + 1))
+    t[6, 0, k[6, 0]] = -200.0  # expf leaves nothing of it
+    q[7, L // 2, k[7, L // 2]] = 0.0
+    p = np.empty((rows, L), dtype=np.float32)
+    for r in range(rows):
+        for i in range(L):
+            p[r, i] = orc.build_filtered_distribution(t[r, i], to_oracle(params[r]))[k[r, i]]
+    qk = np.take_along_axis(q, k[:, :, None], axis=2)[:, :, 0]
+    ratio = np.minimum(np.float32(1), p / np.maximum(qk, np.float32(1e-38))).astype(np.float64)
+    near = np.stack([np.nextafter(ratio, 0.0), ratio * (1 - 1e-4), ratio * 0.5, ratio * (1 - 0.004)])
+    u[:, :L] = np.take_along_axis(near, rng.integers(0, 4, (1, rows, L)), axis=0)[0]
+    for r in range(rows):  # where a row's first rejection is: nowhere, on the ratio itself, or for certain
+        if r % 3:
+            at = int(rng.integers(0, L))
+            u[r, at] = ratio[r, at] if r % 3 == 1 else 0.9999999
+    try:
+        ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, polls))
+        _check_spec(ctx, t, q, k, params, u)
+    finally:
+        ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
+
+
 def test_verification_after_tokens_were_appended_to_the_batch(ctx):
     # The verifier copies the batch's row descriptors on the device: rows with penalties whose histories grew by
     # sr_batch_append_tokens (in place, no new upload) must be verified with the histories as they are now.
