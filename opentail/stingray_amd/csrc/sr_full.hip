@@ -4183,8 +4183,10 @@ __device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, Pr
         const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
         return (sum > 0.0f && sum != 1.0f) ? __fdiv_rn(1.0f, sum) : 1.0f;
     };
-    // (phase 3: the row's workgroups wrote e just now, through to memory; blocks and rows start on lines of their own, so no cache
-    // holds one of these lines from before it was written)
+    // (phase 3: the row's workgroups, on other dies too, wrote e just now, through to memory.  No cache holds one of these lines from
+    // before it was written: rows and blocks start on lines of their own, and nothing in the launch loads e of a position that it has
+    // still to write -- spec_e<true>.  Read past the caches by agent-scope loads the blocks that no record fits cost 1.5 us of 127 at 16
+    // rows of 262,144 and 8 drafts, 3 of 109 at 64 of 65,536 and 6: eight waves take 4 bytes of every 32 each)
     // Whoever counts in last walks them, and the others wait for the factor.  (All workgroups of the row walking for themselves, the
     // same work: 512 of them, at 16 rows of 262,144, fetched 12 MB of records past the caches and took 2.6 - 8 us for it.)
     unsigned long long* const factor = sync + 2;  // launch number << 32 | the factor's bits
@@ -4580,12 +4582,19 @@ struct SpecTerms {
         for (int k = 0; k < 4; k++) { x[4 * k] = v[k].x; x[4 * k + 1] = v[k].y; x[4 * k + 2] = v[k].z; x[4 * k + 3] = v[k].w; }
     }
 };
-// e of token tok at a position of the verifier's batch (both of its places are asked for beside the state that says which holds)
+// e of token tok at a position of the verifier's batch (its place in the logits is asked for beside the state that says which holds).
+// kOpenUnread: in the launch that writes e of open positions, where whoever counts in last reads it behind this: what stands there
+// before is not loaded at all, or this die's cache would keep the line as it was.  Behind that launch both places are asked for at
+// once (with the branch there too 0.5 - 0.9 us).
+template <bool kOpenUnread>
 __device__ __forceinline__ float spec_e(const SrSpecArgs& a, const SrRow& rd, size_t slot, int tok, const uint64_t* tab)
 {
     const SrFullState* sl = a.state + slot;
     const uint32_t open = sl->e_open;
-    const float there = a.p_all[slot * (size_t)a.p_stride + tok], x = a.target_logits[slot * (size_t)a.vocab + tok];
+    const float* const at = a.p_all + slot * (size_t)a.p_stride + tok;
+    const float x = a.target_logits[slot * (size_t)a.vocab + tok];
+    float there = 0.0f;
+    if (!kOpenUnread || open != a.seq) there = *at;
     ERow r;
     r.inv_temp = row_inv_temp(rd);
     r.max = sr_okey_inv((uint32_t)sl->maxkey);
@@ -4692,7 +4701,7 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_factor(SrFullArgs a, SrSpecA
             if (!bad) {
                 const SrFullState* sl = s.state + (size_t)row * (L + 1) + lane;
                 const bool any = sl->deferred == a.seq;  // m2 is s / S so far
-                const float y = __fmul_rn(spec_e(s, rd, (size_t)row * (L + 1) + lane, tok, tab), sl->mul1);
+                const float y = __fmul_rn(spec_e<true>(s, rd, (size_t)row * (L + 1) + lane, tok, tab), sl->mul1);
                 const float qx = s.draft_probs[((size_t)row * L + lane) * n + tok];
                 const double u = s.uniforms[(size_t)row * s.uniforms_per_row + lane];
                 const float acc = spec_accept(__fmul_rn(y, sl->mul2), qx);
@@ -4787,7 +4796,7 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
                 bad = (uint32_t)tok >= (uint32_t)n;
                 if (!bad) {
                     const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
-                    const float px = __fmul_rn(__fmul_rn(kLater ? spec_e(a, rd, (size_t)row * (L + 1) + i, tok, tab)
+                    const float px = __fmul_rn(__fmul_rn(kLater ? spec_e<false>(a, rd, (size_t)row * (L + 1) + i, tok, tab)
                                                             : a.p_all[((size_t)row * (L + 1) + i) * (size_t)a.p_stride + tok], sl->mul1), sl->mul2);
                     const float qx = a.draft_probs[((size_t)row * L + i) * n + tok];
                     const float acc = spec_accept(px, qx);

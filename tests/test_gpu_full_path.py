@@ -400,6 +400,32 @@ def test_accept_tests_that_hang_on_the_last_digits(ctx, V, rows, L, polls):
         ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
 
 
+@pytest.mark.parametrize("V, rows, L", [(8_199, 25, 63), (16_391, 14, 63), (70_007, 36, 5)])  # seven entries behind the last whole vector
+def test_drafts_in_the_last_line_of_rows_that_an_earlier_call_has_filled(ctx, V, rows, L):
+    """Accept tests that hang on the last digits, drafts among the last eight ids of their rows (every third anywhere): the launch
+    that works out the factors looks at the drafts' entries of e before it writes e, and adds the end of the row again from
+    what its workgroups have written.  Calls on one context, the last entries large and small in turn, so that what an
+    earlier call has left there would be noticed."""
+    rng = np.random.default_rng(V)
+    params = [SamplingParams(Temperature=0.7 + 0.01 * r) for r in range(rows)]
+    rr, ii = np.arange(rows)[:, None], np.arange(L)[None, :]
+    for turn in range(3):
+        base = rng.normal(0, 1.5, (rows, L, V)).astype(np.float32)
+        base[:, :, -64:] += np.float32(6.0 if turn == 1 else -4.0)
+        k = np.where((rr + ii) % 3 == 0, rng.integers(0, V, (rows, L)), V - 1 - rng.integers(0, 8, (rows, L))).astype(np.int32)
+        base[rr, ii, k] = np.float32(9.0) + rng.normal(0, 1, (rows, L)).astype(np.float32)
+        t = np.concatenate([base + rng.normal(0, 0.1, (rows, 1, V)).astype(np.float32), rng.normal(0, 1.5, (rows, 1, V)).astype(np.float32)], axis=1)
+        q = np.exp(base - base.max(axis=2, keepdims=True))
+        q /= q.sum(axis=2, keepdims=True)
+        u = rng.random((rows, L + 1))
+        for r in range(rows):
+            for i in range(L):
+                p = orc.build_filtered_distribution(t[r, i], to_oracle(params[r]))[k[r, i]]
+                ratio = np.float64(np.minimum(np.float32(1), p / q[r, i, k[r, i]]))
+                u[r, i] = ratio if i == L - 1 - r % 7 and r % 2 else np.nextafter(ratio, 0.0)  # on the ratio: rejected (but at 1)
+        _check_spec(ctx, t, q, k, params, u)
+
+
 def test_verification_after_tokens_were_appended_to_the_batch(ctx):
     # The verifier copies the batch's row descriptors on the device: rows with penalties whose histories grew by
     # sr_batch_append_tokens (in place, no new upload) must be verified with the histories as they are now.
