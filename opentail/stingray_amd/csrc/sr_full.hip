@@ -4056,7 +4056,9 @@ __device__ __forceinline__ void prepared_segment(const SrFullArgs& a, const Prep
 struct PreparedSmem {
     float4 room[SR_SEQ_CHAINS * SR_WAVE * 5];  // the block chain by chain, then every wave's segment on its way to 16 terms a lane
     float lane_sum[SR_SEQ_CHAINS];
-    uint32_t bc[2];
+    // 0: whether the workgroup is the row's last   1: the factor   2: whether the wait for it ended in time (a word of its own: the
+    // waiting thread writes it while others may still have to read the first)
+    uint32_t bc[3];
 };
 template <int kPhase>
 __device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, PreparedSmem& sm, const uint64_t* tab = nullptr, float inv_temp = 1.0f)
@@ -4212,11 +4214,11 @@ __device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, Pr
                 __builtin_amdgcn_s_sleep(1);
             }
             if (ok == 0u) sr_store_agent(&st->late_behind, a.seq);
-            bc[0] = ok;
+            bc[2] = ok;
             bc[1] = (uint32_t)v;
         }
         __syncthreads();
-        here = bc[0] != 0u;
+        here = bc[2] != 0u;
         inv2 = sr_u2f(bc[1]);
     }
     if (here && seg < nseg) prepared_segment(a, r, slot, row, seg, lane, v, sr_wave_sum_f32(before_seg), inv2, room + wave * SR_WAVE * 5);

@@ -921,6 +921,27 @@ def test_workgroups_that_stop_waiting_leave_a_prepared_row_to_the_last_one(ctx, 
         ctx._check(H.sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
 
 
+@pytest.mark.parametrize("polls", [1, 1 << 15])
+@pytest.mark.parametrize("vocab, rows", [(8_193, 240), (16_390, 96), (24_583, 60)])  # two, three and four workgroups a row
+def test_factors_that_are_there_when_the_wait_for_them_begins(ctx, vocab, rows, polls):
+    """Rows of few workgroups, so that the last one's factor is out by the time another starts to wait for it, or nearly: a
+    workgroup that waits is no last one, whatever the outcome.  Tokens and distributions, rows cut by top-p and rows that nothing cuts."""
+    rng = np.random.default_rng(vocab)
+    logits = rng.normal(0, 1.5, (rows, vocab)).astype(np.float32)
+    params = [SamplingParams(Temperature=0.7 + 0.003 * r) if r % 3 else SamplingParams(Temperature=1.3, TopP=0.95) for r in range(rows)]
+    u = rng.random(rows)
+    try:
+        ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 0x80000000 | polls))
+        _check_rows(ctx, logits, params, u)
+        tokens, probs = ctx.sample_with_distribution(_cuda(logits), params, u)
+        probs = probs.cpu().numpy()
+        for r in range(rows):
+            t, d = orc.sample_with_distribution(logits[r], to_oracle(params[r]), orc.Rng(replay=[u[r]]))
+            assert tokens[r] == t and np.array_equal(probs[r].view(np.uint32), d.view(np.uint32)), r
+    finally:
+        ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
+
+
 @pytest.mark.parametrize("vocab", [4096, 4097, 40_968, 151_937])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_greedy_rows_that_ride_along_with_the_full_path(ctx, vocab, bf16):
