@@ -1044,6 +1044,28 @@ def test_verification_where_the_launch_behind_starts(ctx, V, rows, L):
     _check_spec(ctx, t, q, k, params, u)
 
 
+@pytest.mark.parametrize("V, small", [(16_384, 8_192), (24_576, 16_300), (24_583, 16_300)])
+def test_blocks_whose_members_are_all_too_small_to_count(ctx, V, small):
+    """Rows cut by a tiny min-p: one entry of nearly all the mass, 40 between 1e-8 and 1e-6 behind blocks of thousands below
+    9e-13, which in whole units of 2^-40 are nothing.  They are members: in the exact sums of the accumulators that hold no large
+    entry they decide the last digit of every tenth row's factor."""
+    rows, lo = 64, V // 8192 * 8192 - 8192
+    rng = np.random.default_rng(V)
+    logits = np.full((rows, V), NEG_INF, dtype=np.float32)
+    decided = 0
+    for x in logits:
+        x[rng.permutation(lo)[:small]] = np.log(rng.uniform(5e-13, 9e-13, small))
+        at = lo + rng.permutation(8_192)[:40]
+        x[at] = np.log(10.0 ** rng.uniform(-8, -6, 40))
+        x[at[0]] = 0.0
+        e = np.exp(x.astype(np.float64)).astype(np.float32)
+        y = (e * (np.float32(1) / np.cumsum(e, dtype=np.float32)[-1]))[: V // 8 * 8].reshape(-1, 8)
+        sums = [np.add.reduce(np.cumsum(c, axis=0, dtype=np.float32)[-1].reshape(4, 2), axis=1) for c in (y, y[lo // 8:])]
+        decided += len({np.float32(1) / np.float32((s[0] + s[1]) + (s[2] + s[3])) for s in sums}) - 1
+    assert decided > 0  # (rows in which leaving them out changes the factor)
+    _check_distribution(ctx, logits, [SamplingParams(MinP=1e-13)] * (rows - 1) + [SamplingParams()])
+
+
 @pytest.mark.parametrize("V, rows", [(50_257, 150), (98_305, 82)])
 def test_more_rows_than_the_device_holds_at_a_time(ctx, V, rows):
     """Launches of more than a thousand workgroups behind the row kernel go as two: up to the rows' factors, and from there on.  Rows
