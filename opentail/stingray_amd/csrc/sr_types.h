@@ -109,8 +109,11 @@ struct SrMaskClear {
 // top-p 0.9 and temperature 0.6, and at top-p 0.95 and temperature 1.5.
 // Tokens of rows that nothing cuts: at every length.  16 rows of 4,608: 34 against 49, of 16,384: 37 against 48, of 49,152: 43
 // against 64; 64 rows of 151,936: 91 against 122; 192 (28,608 segments): 199 against 197; 256: 266 against 251.  That only
-// top-p cuts, where it finds nothing to do for sharp rows: 16 rows of 24,576 23 against 22 (sharp) and 101 against 200 (flat), of
-// 16,384 23 against 21 and 77 against 72.  Both kinds of rows together, sharp and flat ones: 16 rows of 31,000 44 against 60 and 131
+// top-p cuts, where it finds nothing to do for sharp rows, and where a flat row's nucleus outgrows what its workgroup finishes by
+// itself: 1, 16, 64 and 256 rows of 24,576 21, 23, 24, 36 against 20, 21, 22, 30 (sharp) and 81, 102, 110, 144 against 111, 196,
+// 207, 231 (flat); of 28,672 21, 24, 25, 39 against 19, 21, 23, 34 and 74, 116, 129, 172 against 103, 225, 240, 267; of 20,480, where
+// one flat row or four gain nothing, 21, 22, 24, 34 against 19, 20, 22, 29 and 69, 92, 101, 131 against 65, 151, 188, 211; of 16,384
+// 23 against 21 and 76 against 72.  Both kinds of rows together, sharp and flat ones: 16 rows of 31,000 44 against 60 and 131
 // against 250, of 20,480 41 against 49 and 103 against 183, of 16,384 40 against 52 and 92 against 73, of 8,192 37 against 57
 // and 62 against 55; 256 rows of 31,000 84 against 76 and 251 against 285.
 // Distributions: at every length.  16 rows of 4,608 37 against 51, cut by top-p 32 against 82; of 16,384 37 against 47, 33 against 37
@@ -124,7 +127,7 @@ struct SrMaskClear {
 // of it 102 against 106, 192 of 151,936 108 against 111, 176 of 131,072 94 against 97, 144 of it (18,432 segments) 88 against 86, 96 of
 // 151,936 92 against 85; 448 rows of 65,536 108 against 118, 576 of 32,768 92 against 99, 288 of 50,257 (14,400) 84 against 92, 224 of
 // it 78 against 70, 384 of 32,768 (12,288) 84 against 77, 2,304 of 16,384 153 against 210, 768 of it 89 against 83.
-#define SR_PREPARED_MIN_SEGS 32        // tokens, rows that are cut
+#define SR_PREPARED_MIN_SEGS 24        // tokens, rows that are cut
 #define SR_PREPARED_MIN_SEGS_MIXED 20  // ... beside rows that are not
 #define SR_PREPARED_ROWS_MIXED 128
 #define SR_PREPARED_SEGS 32768
@@ -133,13 +136,15 @@ struct SrMaskClear {
 #define SR_PREPARED_ROWS_VERIFY 32
 #define SR_FACTOR_LATER_SEGS 14336
 #define SR_FACTOR_LATER_SEGS_FEW 20480
-// Distributions of rows that min-p cuts, where no other row asks for that launch: worth it for few long rows.  Some ten entries left,
-// 16 rows of 65,536: 36 us against 34, of 131,072 43 against 49, of 262,144 59 against 80.  When three launches did its work, 20,
-// 200, 2,000, 8,000 and 15,000 entries left, 16 rows of 262,144: 71, 98, 106, 120, 143 us against 88, 99, 118, 181, 184 without;
-// of 131,072: 59, 79, 83, 101, 126 against 56, 68, 85, 112, 113; one row: 47, 63, 68, 87, 104 against 51, 60, 78, 102, 103; 64 rows
-// of 151,936: 96, 125, 131, 145, 165 against 78, 90, 109, 145, 145; 16 rows of 32,768: 52, 68, 70, 90, 112 against 33, 48, 61, 62, 63.
-// At odd addresses, 16 rows of 65,537: 54, 72, 76, 93, 116 against 45, 56, 72, 129, 129; of 100,003: 58, 77, 80, 100, 121 against 51,
-// 62, 80, 163, 163; 64 rows of 100,003: 84, 109, 107, 123, 149 against 62, 76, 91, 176, 174.
+// Distributions of rows that min-p cuts, where no other row asks for that launch: worth it for few long rows.  10, 200, 2,000, 8,000
+// and 15,000 entries left, with it against without: one row of 131,072 36, 44, 50, 73, 102 us against 44, 56, 70, 102, 103; 16 rows
+// 47, 56, 62, 83, 111 against 49, 61, 76, 110, 110; 32 (4,096 segments) 51, 62, 69, 91, 119 against 56, 68, 82, 118, 119; 64 rows 75, 88,
+// 96, 121, 150 against 60, 72, 86, 121, 122; 16 rows of 262,144 59, 69, 77, 96, 124 against 82, 94, 109, 176, 179; 32 of 151,936 (4,768)
+// 64, 76, 84, 103, 134 against 62, 74, 88, 130, 131, 48 of them 71, 85, 90, 109, 140 against 65, 76, 91, 132, 133; 16 rows of 98,304
+// 45, 53, 58, 82, 112 against 43, 54, 68, 95, 95, of 65,536 40, 49, 54, 78, 105 against 35, 47, 60, 76, 76.  At odd addresses, one row
+// of 100,003 37, 46, 51, 75, 102 against 39, 50, 63, 89, 89, 16 rows 45, 55, 59, 83, 111 against 44, 56, 69, 158, 157; 64 rows (6,272)
+// 68, 81, 85, 108, 138 against 54, 66, 80, 168, 170; 16 rows of 65,537 41, 50, 54, 79, 106 against 38, 49, 62, 126, 123, one row 35, 45, 49,
+// 73, 97 against 32, 45, 56, 72, 71.
 #define SR_PREPARED_MIN_SEGS_MIN_P 128
 #define SR_PREPARED_MIN_SEGS_MIN_P_ODD 96
 #define SR_PREPARED_SEGS_MIN_P 4096

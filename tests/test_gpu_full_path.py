@@ -1017,10 +1017,10 @@ def test_edits_crowded_into_a_few_segments_of_a_long_row(ctx):
     assert np.array_equal(ctx.sample_batch(dev, params, u), oracle_tokens(exact, params, u))
 
 
-@pytest.mark.parametrize("V", [4_096, 4_099, 8_192, 12_290, 19 * 1024, 19 * 1024 + 1, 31 * 1024 + 5])
+@pytest.mark.parametrize("V", [4_096, 4_099, 8_192, 12_290, 19 * 1024, 19 * 1024 + 1, 23 * 1024, 23 * 1024 + 1, 31 * 1024 + 5])
 def test_short_rows_that_the_launch_behind_finishes(ctx, V):
     """Tokens of short rows take the launch over the whole device where nothing cuts them, from 20 segments on where others beside
-    them are cut, and distributions at every length: sharp and flat rows, nuclei of a handful and of thousands."""
+    them are cut, from 24 on where all are, and distributions at every length: sharp and flat rows, nuclei of a handful and of thousands."""
     rng = np.random.default_rng(V)
     logits = rng.normal(0, 1.5, (8, V)).astype(np.float32)
     logits[::2, rng.permutation(V)[:12]] += 9.0
