@@ -360,7 +360,7 @@ def test_verification_by_one_launch_and_by_the_workgroups_that_come_last(ctx, V,
 # a block and a half of a block to a row, odd rows, long ones; 64 drafts: every position's factor is worked out.  Launches of
 # 14,336 segments and more, and of 20,480 where they have fewer rows than compute units; waits that run out in the launch behind, and in the pass itself
 @pytest.mark.parametrize("V, rows, L, polls", [(4_096, 56, 64, 1 << 15), (4_097, 46, 63, 1 << 15), (8_193, 25, 63, 0x80000000), (8_193, 25, 63, 0x80000002),
-                                               (70_001, 36, 5, 1 << 15), (70_001, 36, 5, 0), (300_001, 24, 2, 1 << 15)])
+                                               (70_001, 43, 5, 1 << 15), (70_001, 43, 5, 0), (300_001, 24, 2, 1 << 15)])
 def test_accept_tests_that_hang_on_the_last_digits(ctx, V, rows, L, polls):
     """Rows that nothing cuts: the verifier works out the factor of the final Normalize for the positions whose accept test is open
     without it, and for the one that is drawn from.  Uniforms on the ratio p / q, one step of a double below it, and so far
@@ -400,7 +400,7 @@ def test_accept_tests_that_hang_on_the_last_digits(ctx, V, rows, L, polls):
         ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
 
 
-@pytest.mark.parametrize("V, rows, L", [(8_199, 25, 63), (16_391, 14, 63), (70_007, 36, 5)])  # seven entries behind the last whole vector
+@pytest.mark.parametrize("V, rows, L", [(8_199, 25, 63), (16_391, 14, 63), (70_007, 43, 5)])  # seven entries behind the last whole vector
 def test_drafts_in_the_last_line_of_rows_that_an_earlier_call_has_filled(ctx, V, rows, L):
     """Accept tests that hang on the last digits, drafts among the last eight ids of their rows (every third anywhere): the launch
     that works out the factors looks at the drafts' entries of e before it writes e, and adds the end of the row again from
@@ -925,14 +925,15 @@ def test_workgroups_that_stop_waiting_leave_a_prepared_row_to_the_last_one(ctx, 
 @pytest.mark.parametrize("vocab, rows", [(8_193, 240), (16_390, 96), (24_583, 60)])  # two, three and four workgroups a row
 def test_factors_that_are_there_when_the_wait_for_them_begins(ctx, vocab, rows, polls):
     """Rows of few workgroups, so that the last one's factor is out by the time another starts to wait for it, or nearly: a
-    workgroup that waits is no last one, whatever the outcome.  Tokens and distributions, rows cut by top-p and rows that nothing cuts."""
+    workgroup that waits is no last one, whatever the outcome.  Tokens of rows that nothing cuts; distributions, with tokens, of such
+    rows and of rows cut by top-p."""
     rng = np.random.default_rng(vocab)
     logits = rng.normal(0, 1.5, (rows, vocab)).astype(np.float32)
     params = [SamplingParams(Temperature=0.7 + 0.003 * r) if r % 3 else SamplingParams(Temperature=1.3, TopP=0.95) for r in range(rows)]
     u = rng.random(rows)
     try:
         ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 0x80000000 | polls))
-        _check_rows(ctx, logits, params, u)
+        _check_rows(ctx, logits, [SamplingParams(Temperature=0.7 + 0.003 * r) for r in range(rows)], u)
         tokens, probs = ctx.sample_with_distribution(_cuda(logits), params, u)
         probs = probs.cpu().numpy()
         for r in range(rows):
