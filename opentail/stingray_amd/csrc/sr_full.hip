@@ -340,8 +340,8 @@ __device__ __forceinline__ float seq_sum_residual(const float* p, const float* q
 // ---- exact sums prepared by the whole device ---------------------------------------------------------------
 // One workgroup adds a row at the rate at which one compute unit reads and scans it (1 MB in ~45 us).  Where the terms
 // lie in memory before that workgroup starts, the whole device prepares the sum: the row is cut into segments of
-// SR_SEG_TERMS terms, a first kernel leaves an approximate sum of every segment (double precision, any order), and
-// k_seq_funcs turns every segment into its increment function n -> n + a[n & 1] (sr_seqsum.h) for the binade that the
+// SR_SEG_TERMS terms, its workgroups leave an approximate sum of every segment (any order), and seg_make_record turns
+// every segment into its increment function n -> n + a[n & 1] (sr_seqsum.h) for the binade that the
 // approximate prefix predicts for the segment's start.  The workgroup that needs the sum then only walks the
 // functions (seg_walk, one wave): a function is applied when the exact running sum in front of its segment lies in the
 // binade it was made for and stays there; any other segment -- one in which the sum changes binade (a sum that starts

@@ -69,8 +69,9 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             // Rows that the row kernel may leave to the whole device: those that nothing cuts and, but for the verifier, whose
             // reader takes e where it is, those that only top-p cuts (a few members or tens of thousands).  What a min-p of some
             // size leaves is mostly little, and nobody knows before the launch: tokens of 64 rows of 151,936 with 300 entries left
-            // took 72 us, 78 where more launches followed that found nothing to do; with 2,000 77 against 128, since up to 8,192
-            // the row's workgroup then finishes by itself.  Distributions: SR_PREPARED_MIN_SEGS_MIN_P, whatever the min-p.
+            // take 51 us with the launch behind and 47 without, with 2,000 102 and 57, with 8,000 119 and 92, since up to 8,192 the row's
+            // workgroup then finishes by itself; with 9,000 to 16,000 132 - 156 and 180 - 198, and with 30,000, where it finds nothing to
+            // do, 162 and 159.  Distributions: SR_PREPARED_MIN_SEGS_MIN_P, whatever the min-p.
             const bool by_min_p = mode != 0 ? r.min_p > 0.0f : r.min_p >= 0.002f;
             prepared = prepared || (lazy_scale ? !sr_row_cut(r) : !by_min_p);
             any_plain = any_plain || !sr_row_cut(r);

@@ -231,7 +231,7 @@ hipError_t sr_launch_draw_rows(const float* probs, int64_t stride, int n, int ro
 hipError_t sr_launch_residual_rows(const float* p, int64_t ps, const float* q, int64_t qs, int n, int rows,
                                    const double* u, int* out, hipStream_t st);
 
-// One segment of SR_SEG_TERMS terms of a row whose exact sum the whole device prepares (k_seq_funcs, seg_walk in
+// One segment of SR_SEG_TERMS terms of a row whose exact sum the whole device prepares (seg_make_record, seg_walk in
 // sr_full.hip): the increment function n -> n + a[n & 1] of its terms in the binade `eb` (sr_seqsum.h), and for a
 // segment in which the running sum is expected to change binade once, inside the 16 terms of lane `cross`: the function
 // of the terms in front of those 16 (a0, a1, eb), the 16 terms themselves, and the function of the terms behind them
