@@ -1239,7 +1239,6 @@ int sr_sample_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int
         a.n_workers = b->n_workers;
         a.cu_count = ctx->cu_count;
         a.own_rows = b->own_rows ? 1 : 0;
-        a.kept = (b->own_rows && b->n_workers <= ctx->cu_count) ? 1 : 0;
         a.short_lists = b->max_sel <= SR_TK_SHORT_SEL ? 1 : 0;
         a.n_items = b->n_items;
         a.sel_list = b->d_sel_list.as<int32_t>();

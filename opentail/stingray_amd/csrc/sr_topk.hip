@@ -1856,16 +1856,15 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
 // registers, so every thread has up to kVec loads in flight from its first chunk to its last, and the stores, the
 // per-wave bound and the hand-off of a chunk run under the loads of the next one.
 //
-// kKept: every worker streams all chunks (at most kKeptChunks) of the one row it finishes and there is at most one
-// worker per compute unit.  Nothing is handed over then, so nothing is written out: the group results of all chunks
-// stay in the thread's registers (the workgroup has the register file of its compute unit to itself) and the waves'
-// shares of the bound go through LDS.
-// kRoomy: a launch of at most one worker per compute unit whose rows' chunks several workers stream (a batch of few
-// rows): compiled for two waves a SIMD like the register-keeping shape, so that the row tail keeps its registers
-// (with four waves a SIMD it spills a hundred bytes a lane, which the tails of a launch that has the compute units to
-// itself need not pay for).
-template <int EPV, int kVec, int kWindow, bool kKept, bool kShort, bool kRoomy = false>
-__global__ __launch_bounds__(kThreads, (kKept || kRoomy) ? 2 : 4) void k_topk_rows(SrTopkArgs a)
+// kKept: every worker streams all chunks (at most kKeptChunks) of the one row it finishes.  Nothing is handed over then,
+// so nothing is written out: the group results of all chunks stay in the thread's registers and the waves' shares of the
+// bound go through LDS.  Also where two workers share a compute unit: 128 registers hold it (the tail spills 44 bytes a lane;
+// of the shape that writes its results and reads them back 84, and that one pays a bound loop per chunk): 1,024
+// rows of 151,936 fp32 147.5 -> 113.5 us, 512 80.0 -> 59.7, 320 62.1 -> 47.6, 1,024 of bf16 95.7 -> 69.5.
+// kRoomy: a launch of at most one worker per compute unit, compiled for two waves a SIMD, so that the row tail keeps its
+// registers.
+template <int EPV, int kVec, int kWindow, bool kKept, bool kShort, bool kRoomy>
+__global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkArgs a)
 {
     __shared__ TopkSmem sm;
     using VO = VecOps<EPV>;
@@ -1977,16 +1976,31 @@ __global__ __launch_bounds__(kThreads, (kKept || kRoomy) ? 2 : 4) void k_topk_ro
         // two bodies, or a condition around the loads, the compiler keeps the incoming vectors in registers of their
         // own and spills.
         int last_sel = 0;
-        // (kKept) The wave's share of the row's bound, taken from the largest group maximum of every lane and chunk folded
-        // so far (one value per lane and chunk instead of four: a lane with two groups of a chunk at or above the value
-        // counts once, which can only lower the value and keeps it a bound -- a twelfth of the count at the largest
-        // shares -- and a count costs four ballots instead of sixteen): the largest key, to 16 bits, with at least
-        // `need` of those values at or above it; 0 when there is none.  *wmax = the wave's largest kept element.
+        // (kKept) The wave's share of the row's bound, taken from the largest group maxima of every lane folded so far: the
+        // largest key, to 16 bits, with at least `need` of those values at or above it; 0 when there is none.  *wmax = the
+        // wave's largest kept element.  Four values a lane, four ballots a count: of one chunk the four groups', of two
+        // chunks the larger one of every two groups', of more chunks one value each (two of the first of three) -- a lane with two groups at
+        // or above the value counts once, which can only lower the value and keeps it a bound.  (One value a chunk for every number of chunks left a list
+        // of hundreds without a bound in rows of one and two: 256 rows of 20,000 fp32, top-k up to 1,000, 40.6 us, 23.1 now.)
         auto kept_share = [&](int need, uint32_t* wmax_out) SR_INL -> uint32_t {
             float pool[kKeptChunks];
+            if (S == 1) {
+                pool[0] = kept.g1[0].x; pool[1] = kept.g1[0].y; pool[2] = kept.g1[0].z; pool[3] = kept.g1[0].w;
+            } else if (S == 2) {
 #pragma unroll
-            for (int c = 0; c < kKeptChunks; c++)
-                pool[c] = fmaxf(fmaxf(kept.g1[c].x, kept.g1[c].y), fmaxf(kept.g1[c].z, kept.g1[c].w));
+                for (int c = 0; c < 2; c++) {
+                    pool[2 * c] = fmaxf(kept.g1[c].x, kept.g1[c].y);
+                    pool[2 * c + 1] = fmaxf(kept.g1[c].z, kept.g1[c].w);
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < kKeptChunks; c++)
+                    pool[c] = fmaxf(fmaxf(kept.g1[c].x, kept.g1[c].y), fmaxf(kept.g1[c].z, kept.g1[c].w));
+                if (S == 3) {
+                    pool[0] = fmaxf(kept.g1[0].x, kept.g1[0].y);
+                    pool[3] = fmaxf(kept.g1[0].z, kept.g1[0].w);
+                }
+            }
             auto enough = [&](uint32_t cnd) SR_INL -> bool {
                 const float fc = sr_okey_inv(cnd);  // a key in the NaN range compares false: the right answer for it
                 int cge = 0;
@@ -1994,8 +2008,8 @@ __global__ __launch_bounds__(kThreads, (kKept || kRoomy) ? 2 : 4) void k_topk_ro
                 for (int c = 0; c < kKeptChunks; c++) cge += __popcll(__ballot(pool[c] >= fc));
                 return cge >= need;
             };
-            const uint32_t wmax = sr_wave_max_u32(sr_okey(fmaxf(fmaxf(pool[0], pool[1]), fmaxf(pool[2], pool[3]))));
             static_assert(kKeptChunks == 4, "four pool values");
+            const uint32_t wmax = sr_wave_max_u32(sr_okey(fmaxf(fmaxf(pool[0], pool[1]), fmaxf(pool[2], pool[3]))));
             *wmax_out = wmax;
             const uint32_t K = largest_key16(wmax, enough);
             return K;
@@ -2417,17 +2431,16 @@ hipError_t sr_launch_topk(const SrTopkArgs& a, int n_rows, hipStream_t stream)
 {
     if (n_rows <= 0) return hipSuccess;
     dim3 grid((unsigned)a.n_workers), block(kThreads);
-    // workers with a row of their own are few per compute unit: each keeps more of its vectors in flight
-    // ... and where there is at most one of them per compute unit, the results of its chunks stay in its registers
-    const bool kept = a.own_rows && a.kept && a.chunks <= kKeptChunks;
+    // workers with a row of their own keep the results of its chunks in their registers, where these are few enough
+    const bool kept = a.own_rows && a.chunks <= kKeptChunks, roomy = a.n_workers <= a.cu_count;
     // ... and a launch whose rows all ask for few entries carries the steps that pay for such rows only
     auto launch = [&](auto epv, auto vec, auto shrt) {
         constexpr int kE = decltype(epv)::value, kV = decltype(vec)::value;
         constexpr bool kS = decltype(shrt)::value;
-        if (kept) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS>), grid, block, 0, stream, a);
-        else if (a.own_rows) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_OWN, false, kS>), grid, block, 0, stream, a);
-        else if (a.n_workers <= a.cu_count) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW, false, kS, true>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW, false, kS>), grid, block, 0, stream, a);
+        if (kept && roomy) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS, true>), grid, block, 0, stream, a);
+        else if (kept) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS, false>), grid, block, 0, stream, a);
+        else if (roomy && !a.own_rows) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW, false, kS, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_OWN, false, kS, false>), grid, block, 0, stream, a);
     };
     using std::integral_constant;
     if (a.dtype == 1) {

@@ -1,0 +1,61 @@
+"""The ways in which the selection kernel's workers take the rows of a launch, at the sizes where one way ends and the next
+begins, against the CPU oracle.  Token ids are the same."""
+import numpy as np
+import pytest
+
+from opentail.stingray_amd import SamplerContext, SamplingParams, pack_allow_mask, synthetic
+from tests.helpers import oracle_tokens
+
+pytestmark = pytest.mark.gpu
+CHUNK = 512 * 19 * 4  # elements of fp32 logits that a worker's registers hold (bf16: 512 * 10 * 8)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = SamplerContext(0)
+    yield c
+    c.close()
+
+
+def _batch(rng, rows, vocab, longest):
+    logits = synthetic.zipf_head_logits(rng, rows, vocab)
+    logits[rows // 2] = np.round(logits[rows // 2])  # ties, and hundreds of entries at the bound
+    logits[rows // 3, :] = -3.0
+    params, allowed = [], np.ones((rows, vocab), dtype=bool)
+    for r in range(rows):
+        p = SamplingParams(Temperature=0.0 if r % 9 == 4 else float(rng.uniform(0.3, 1.6)), TopK=int(rng.integers(1, min(longest, vocab - 1) + 1)),
+                           TopP=float(rng.choice([1.0, 0.95, 0.6])), MinP=float(rng.choice([0.0, 0.02])))
+        if r % 3 == 1:
+            p.PreviousTokens = rng.integers(0, vocab, 50).tolist() + np.argsort(-logits[r])[:10].tolist()
+            p.RepetitionPenalty, p.FrequencyPenalty = 1.2, 0.1
+        if r % 5 == 2:
+            allowed[r] = rng.random(vocab) < 0.3
+            allowed[r, 0] = True
+        params.append(p)
+    return logits, params, pack_allow_mask(allowed), np.array([r % 5 == 2 for r in range(rows)], dtype=np.uint8)
+
+
+def _check(ctx, rng, rows, vocab, longest, bf16):
+    import torch
+
+    logits, params, mask, active = _batch(rng, rows, vocab, longest)
+    u = rng.random(rows)
+    if bf16:
+        bits = synthetic.to_bf16_bits(logits)
+        logits = synthetic.bf16_bits_to_f32(bits)
+        dev = torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16)
+    else:
+        dev = torch.from_numpy(logits).cuda()
+    got = ctx.sample_batch(dev, params, u, mask, active)
+    want = oracle_tokens(logits, params, u, mask, active)
+    assert np.array_equal(got, want), (rows, vocab, longest, bf16, np.nonzero(got != want)[0][:10])
+
+
+# Two workers to a compute unit that keep their rows' results: one row more than the device has compute units, the rows of a
+# second turn, and chunks that end with a chunk's last vector and one element behind it.
+@pytest.mark.parametrize("rows,vocab,longest,bf16", [
+    (257, 1000, 900, False), (257, CHUNK, 40, False), (257, CHUNK + 1, 1000, False), (300, 2 * CHUNK - 3, 1000, False), (257, 2 * CHUNK + 1, 1000, False),
+    (257, 3 * CHUNK + 1, 1000, False), (520, 9_001, 64, False), (513, 4 * CHUNK - 4, 300, False), (257, 4 * CHUNK + 1, 1000, False),
+    (600, 33_333, 1000, True), (257, 512 * 10 * 8 + 1, 1000, True), (300, 100_003, 200, True), (257, 131_072, 1000, True)])
+def test_more_rows_than_compute_units(ctx, rows, vocab, longest, bf16):
+    _check(ctx, np.random.default_rng(rows * 7 + vocab), rows, vocab, longest, bf16)
