@@ -46,24 +46,57 @@ inline bool has_history_penalty(const sr_row_params& p)
     return p.repetition_penalty != 1.0f || p.presence_penalty != 0.0f || p.frequency_penalty != 0.0f;
 }
 
-// Chunking of a row for the selection kernel: a chunk is a whole number of 64-vector blocks of the row's
-// window of 16-byte vectors and must fit the per-workgroup register window.
-void topk_geometry(int vocab, int dtype, int n_rows, int cu_count, int* chunks, int* chunk_vecs)
+// How the selection kernel takes the rows of a launch: chunks per row (a chunk is a whole number of 64-vector blocks of the
+// row's window of 16-byte vectors and fits the per-workgroup register window), and whether every row has a worker of its own
+// that streams all of its chunks and finishes it, or the chunks are dealt out to whichever worker is free.
+struct TopkGeometry {
+    int chunks, chunk_vecs;
+    bool own_rows;
+};
+TopkGeometry topk_geometry(int vocab, int dtype, int n_rows, int cu_count, int max_sel)
 {
     const int epv = dtype == SR_DTYPE_BF16 ? 8 : 4;
     const int window = (dtype == SR_DTYPE_BF16 ? SR_TK_VEC_BF16 : SR_TK_VEC) * SR_TK_THREADS;  // vectors a workgroup holds
     const int nvt = (vocab + 2 * epv - 2) / epv;                   // vectors of a row that starts mid-vector
-    int s_min = (nvt + window - 1) / window;
-    int s_par = (2 * cu_count + n_rows - 1) / std::max(n_rows, 1);  // aim for two workgroups per CU
-    // the row tail keeps the per-group results of up to 4 chunks in registers; more chunks only when the row needs them
-    int s_cap = std::min(4, std::max(1, vocab / 8192));
-    int s = std::max(s_min, std::min(s_par, s_cap));
+    const int s_min = (nvt + window - 1) / window;
+    TopkGeometry g;
+    // A worker of its own for every row, which keeps the row's results in its registers:
+    // * rows of one chunk, in any number.  1, 8 and 64 rows of 16,384 fp32 13.5, 14.8, 15.8 us (lists of up to 40; dealt out as two
+    //   chunks 15.0, 16.4, 17.6), of 32,768 13.4, 14.8, 16.2 (four chunks 13.8, 15.3, 16.9), of 32,768 bf16 with top-k up to 1,000
+    //   15.8, 16.6, 18.7 (18.0, 19.1, 35.6).
+    // * rows of two to four chunks from where the chunks are more than the compute units (eighths of them: `from`); with lists
+    //   of hundreds, whose bound is closer with a share per chunk, and with bf16, which streams in half the time, from some more on.
+    //   Own and dealt, us: two chunks, 128 rows of 49,152 fp32 19.3 and 19.2 (lists of 40), 23.5 and 21.9 (up to 1,000), 144 rows 19.2
+    //   and 23.5, 23.4 and 23.2; of 60,000 bf16 144 rows 19.0 and 22.2, 21.7 and 20.7, 192 rows 19.2 and 23.0, 22.1 and 22.3; three
+    //   chunks, 96 rows of 100,003 fp32 23.0 and 24.9, 27.7 and 25.4, 128 rows 23.9 and 27.3, 28.3 and 27.4, bf16 112 rows 21.3 and 22.1,
+    //   24.6 and 21.4; four, 80 rows of 151,936 fp32 26.2 and 25.1, 30.3 and 26.8, 96 rows 26.7 and 27.3, 30.5 and 28.3, 112 rows 27.1 and
+    //   28.6, 30.7 and 30.6 (with penalties, 120 rows of 131,072 30.3 and 29.6), bf16 112 rows 24.4 and 23.0, 26.5 and 25.1, 128 rows 24.4 and 26.7, 26.6 and 26.5 (with penalties 34.5 and 31.6).
+    // * longer rows, whose results are written and read back, from about half the compute units on: there nothing is gained by
+    //   spreading a row over workers, since a compute unit streams at little more than its share of the memory bandwidth anyway,
+    //   and tails that run beside the streaming slow it down by more than they gain.
+    static const int from[2][2][3] = {{{8, 9, 10}, {8, 11, 15}}, {{8, 11, 14}, {12, 13, 17}}};
+    if (s_min <= 1)
+        g.own_rows = true;
+    else if (s_min <= 4)
+        g.own_rows = n_rows * s_min * 8 > cu_count * from[epv == 8][max_sel > SR_TK_LONG_SEL][s_min - 2];
+    else
+        g.own_rows = n_rows * 32 >= cu_count * 17;
+    int s = s_min;
+    if (!g.own_rows) {
+        // As many chunks as there are compute units for them.  Of the up to 4 whose results a row tail keeps in registers, chunks of
+        // no fewer elements than leave every thread's four groups some: a list of hundreds over 12,288 elements a chunk finds
+        // several of its entries in most groups, and these are fetched again (64 rows of 49,152 bf16, top-k up to 1,000: four chunks
+        // 31.3 us, two 19.1; 64 rows of 49,152 fp32 21.9 and 20.7).  Short lists do not, and stream faster by more workers (one row of
+        // 49,152 fp32, top-k 40: 13.7 us by four, 14.3 by three, 15.3 by two).
+        const int least = max_sel <= SR_TK_SHORT_SEL ? 8192 : 32768;
+        s = std::max(s_min, std::min(cu_count / std::max(n_rows, 1), std::min(4, vocab / least)));
+    }
     int cv = (nvt + s - 1) / s;
     cv = (cv + 63) & ~63;
     if (cv > window) cv = window;  // window is a multiple of 64
-    s = (nvt + cv - 1) / cv;
-    *chunks = std::max(s, 1);
-    *chunk_vecs = cv;
+    g.chunks = std::max((nvt + cv - 1) / cv, 1);
+    g.chunk_vecs = cv;
+    return g;
 }
 
 // Sends the packed pieces: one kernel reads them from the pinned memory and writes them where they belong.  To be
@@ -133,8 +166,8 @@ int prepare_scan(sr_batch* b, int epv, unsigned long long base_addr, long long s
     b->scan_stride_mod = stride_mod;
     if (b->h_scan.empty()) return SR_OK;
     const int n_sel = (int)b->h_sel_list.size();
-    int chunks = 1, chunk_vecs = 0;
-    topk_geometry(b->vocab, epv == 8 ? SR_DTYPE_BF16 : SR_DTYPE_F32, n_sel, ctx->cu_count, &chunks, &chunk_vecs);
+    const TopkGeometry geom = topk_geometry(b->vocab, epv == 8 ? SR_DTYPE_BF16 : SR_DTYPE_F32, n_sel, ctx->cu_count, b->max_sel);
+    const int chunks = geom.chunks, chunk_vecs = geom.chunk_vecs;
     {
         // The selection kernel's grid: workers with a program each -- chunk items to stream, then at most one row to
         // finish.  One worker per CU is resident from the start and a later one starts when one of them ends.  (A CU
@@ -182,13 +215,7 @@ int prepare_scan(sr_batch* b, int epv, unsigned long long base_addr, long long s
             const int n_first = std::min(per_pool, (total_items + n_pool - 1) / n_pool);
             for (int w = 0; w < n_first; w++) new_worker(p, 0.0);
         }
-        // With rows for more than about half the compute units nothing is gained by spreading a row over workers
-        // (a compute unit streams at little more than its share of the memory bandwidth anyway, and tails that run
-        // beside the streaming slow it down by more than they gain): every worker streams all chunks of one row and
-        // finishes it, waits for nobody and hands nothing over.  (Measured on 256 compute units, 151,936 fp32 logits
-        // a row: the two ways cost the same at 136 rows; at 192 rows 37.8 against 45.9 us, at 128 rows 36.0 against
-        // 33.2 us.)
-        const bool affine = n_sel * 32 >= ctx->cu_count * 17;
+        const bool affine = geom.own_rows;  // (waits for nobody and hands nothing over)
         if (affine) {
             prog_items.assign((size_t)n_sel, {});
             prog_tail.assign((size_t)n_sel, -1);
@@ -1231,7 +1258,8 @@ int sr_sample_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int
         int rc = scan_for_launch(const_cast<sr_batch*>(b), epv, (unsigned long long)(uintptr_t)logits_dev,
                                  (long long)row_stride_elems * (dtype == SR_DTYPE_BF16 ? 2 : 4));
         if (rc != SR_OK) return rc;
-        topk_geometry(b->vocab, dtype, n_sel, ctx->cu_count, &a.chunks, &a.chunk_vecs);
+        a.chunks = b->scan_chunks;  // (as the programs and the scan masks were made)
+        a.chunk_vecs = b->scan_chunk_vecs;
         if (a.chunks > SR_TK_MAX_CHUNKS)
             return sr_fail(ctx, SR_ERR_UNSUPPORTED, "sr_sample_launch: vocabulary too large for the selection kernel");
         a.progs = b->d_sched.as<int4>();

@@ -59,3 +59,13 @@ def _check(ctx, rng, rows, vocab, longest, bf16):
     (600, 33_333, 1000, True), (257, 512 * 10 * 8 + 1, 1000, True), (300, 100_003, 200, True), (257, 131_072, 1000, True)])
 def test_more_rows_than_compute_units(ctx, rows, vocab, longest, bf16):
     _check(ctx, np.random.default_rng(rows * 7 + vocab), rows, vocab, longest, bf16)
+
+
+# Where rows get a worker of their own, and what the others' chunks are: rows of one chunk in any number, and both sides of the lines
+# for two, three and four chunks, short and long lists.
+@pytest.mark.parametrize("rows,vocab,longest,bf16", [
+    (1, CHUNK, 40, False), (5, CHUNK, 1000, False), (1, CHUNK + 1, 40, False), (64, 49_152, 1000, False), (64, 49_152, 1000, True), (24, 24_001, 64, True),
+    (128, 2 * CHUNK - 3, 40, False), (129, 2 * CHUNK - 3, 40, False), (97, 100_003, 40, False), (96, 100_003, 40, False), (118, 100_003, 1000, False),
+    (117, 100_003, 1000, False), (81, 4 * CHUNK - 4, 64, False), (121, 131_072, 1000, False), (113, 131_072, 40, True), (193, 60_000, 1000, True), (192, 60_000, 1000, True)])
+def test_rows_with_and_without_a_worker_of_their_own(ctx, rows, vocab, longest, bf16):
+    _check(ctx, np.random.default_rng(rows * 5 + vocab), rows, vocab, longest, bf16)
