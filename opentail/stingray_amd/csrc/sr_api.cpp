@@ -1267,6 +1267,8 @@ int sr_sample_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int
         a.n_workers = b->n_workers;
         a.cu_count = ctx->cu_count;
         a.own_rows = b->own_rows ? 1 : 0;
+        if (b->own_rows && b->n_workers > 2 * ctx->cu_count)
+            a.start_gap = (uint32_t)std::min((double)b->vocab * (dtype == SR_DTYPE_BF16 ? 2.0 : 4.0) * ctx->cu_count / SR_TK_START_GAP, 1e5);
         a.short_lists = b->max_sel <= SR_TK_SHORT_SEL ? 1 : 0;
         a.n_items = b->n_items;
         a.sel_list = b->d_sel_list.as<int32_t>();

@@ -50,6 +50,7 @@ struct SrTopkArgs {
     int32_t n_workers, n_items;
     int32_t cu_count;        // compute units of the device
     int32_t own_rows;        // every worker's program is one whole row (all its chunks, then its tail)
+    uint32_t start_gap;      // ticks of the 100 MHz clock that every compute unit's second worker starts behind its first (0: none)
     int32_t short_lists;     // no row of the launch asks for more than SR_TK_SHORT_SEL entries
     const int32_t* sel_list; // [n_rows] batch row of every launch slot
     const SrRow* rows;

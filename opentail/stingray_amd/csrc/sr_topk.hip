@@ -1923,6 +1923,13 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
         return __builtin_nontemporal_load((const u32x4*)((const char*)g.cp + off));
     };
 
+    // The second worker of a compute unit starts when the first has nearly streamed its row: from then on one streams while the other
+    // finishes a row, turn after turn, where both would stream at half the rate, and then both finish, with the memory
+    // idle.  The first one streams at the full rate meanwhile.  (For launches of more than two turns' workers: SR_TK_START_GAP.)
+    if (kKept && !kRoomy && a.start_gap != 0u && blockIdx.x - (uint32_t)a.cu_count < (uint32_t)a.cu_count) {
+        const unsigned long long t0 = wall_clock64();
+        for (int it = 0; it < 4096 && wall_clock64() - t0 < (unsigned long long)a.start_gap; it++) __builtin_amdgcn_s_sleep(4);
+    }
     KeptGroups kept;
     KeptHistory kept_hist;
     int trow = 0;

@@ -92,6 +92,12 @@ struct SrMaskClear {
                                            // while every chunk ended with a bound loop for the loads to hide; without those loops it
                                            // costs 1.3 us a launch at 256 rows: what is in flight beyond the window only queues.  1,024
                                            // rows of 151,936 fp32, two workers to a compute unit: 3 vectors 118.7 us, 4 115.6, 5 113.9, 7 113.8)
+// Bytes that the compute units' first rows hold, over this: ticks of the 100 MHz clock in eight tenths of the time in which 6.8 TB/s
+// bring them, after which the second workers start.  None, 0.5, 0.8 and 1.0 of it, us: 1,024 rows of 151,936 fp32 114.2, 109.4, 106.8,
+// 107.2; 768 93.9, 82.0, 80.1, 83.4; 520 66.8, 62.5, 62.3, 65.0; 1,024 of bf16 69.4, 67.2, 66.4, 66.4; 600 of 49,152 fp32 40.0, 39.7, 38.2,
+// 37.3; 1,024 of 16,384 39.7, 39.2, 38.9, 38.8.  Up to two workers to a compute unit it gains nothing: 512 rows 59.7 and 59.0, 384 50.7
+// both, 320 47.6 and 48.0, 512 of bf16 38.8 and 39.5.
+#define SR_TK_START_GAP 85000.0
 #define SR_TK_MASK_WORDS 3                 // 32-bit keep-words per chunk thread: 19 x 4 and 10 x 8 bits both fit 96
 #define SR_TK_GROUPS 4                     // group maxima per thread
 #define SR_TK_SHORT_SEL 64                 // a launch whose rows all ask for at most this many entries: see k_topk_rows

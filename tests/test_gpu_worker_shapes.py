@@ -69,3 +69,19 @@ def test_more_rows_than_compute_units(ctx, rows, vocab, longest, bf16):
     (117, 100_003, 1000, False), (81, 4 * CHUNK - 4, 64, False), (121, 131_072, 1000, False), (113, 131_072, 40, True), (193, 60_000, 1000, True), (192, 60_000, 1000, True)])
 def test_rows_with_and_without_a_worker_of_their_own(ctx, rows, vocab, longest, bf16):
     _check(ctx, np.random.default_rng(rows * 5 + vocab), rows, vocab, longest, bf16)
+
+
+# Launches of more than two turns of workers, whose second ones start late: the same tokens at every step, also with work of other
+# streams on the device.
+@pytest.mark.parametrize("rows,vocab,bf16", [(513, 20_011, False), (1030, 40_000, True)])
+def test_launches_of_several_turns_beside_other_work(ctx, rows, vocab, bf16):
+    import torch
+
+    rng = np.random.default_rng(rows)
+    noise = torch.randn(4096, 4096, device="cuda")
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for _ in range(20):
+            noise = noise * 0.5 + 1.0
+    _check(ctx, rng, rows, vocab, 1000, bf16)
+    side.synchronize()
