@@ -64,21 +64,24 @@ TopkGeometry topk_geometry(int vocab, int dtype, int n_rows, int cu_count, int m
     // * rows of one chunk, in any number.  1, 8 and 64 rows of 16,384 fp32 13.5, 14.8, 15.8 us (lists of up to 40; dealt out as two
     //   chunks 15.0, 16.4, 17.6), of 32,768 13.4, 14.8, 16.2 (four chunks 13.8, 15.3, 16.9), of 32,768 bf16 with top-k up to 1,000
     //   15.8, 16.6, 18.7 (18.0, 19.1, 35.6).
-    // * rows of two to four chunks from where the chunks are more than the compute units (eighths of them: `from`); with lists
-    //   of hundreds, whose bound is closer with a share per chunk, and with bf16, which streams in half the time, from some more on.
+    // * rows of two to eight chunks from where the chunks are more than the compute units, or some more: with more chunks, with
+    //   lists of hundreds, whose bound is closer with a share per chunk, and with bf16, which streams in half the time.
     //   Own and dealt, us: two chunks, 128 rows of 49,152 fp32 19.3 and 19.2 (lists of 40), 23.5 and 21.9 (up to 1,000), 144 rows 19.2
     //   and 23.5, 23.4 and 23.2; of 60,000 bf16 144 rows 19.0 and 22.2, 21.7 and 20.7, 192 rows 19.2 and 23.0, 22.1 and 22.3; three
     //   chunks, 96 rows of 100,003 fp32 23.0 and 24.9, 27.7 and 25.4, 128 rows 23.9 and 27.3, 28.3 and 27.4, bf16 112 rows 21.3 and 22.1,
     //   24.6 and 21.4; four, 80 rows of 151,936 fp32 26.2 and 25.1, 30.3 and 26.8, 96 rows 26.7 and 27.3, 30.5 and 28.3, 112 rows 27.1 and
-    //   28.6, 30.7 and 30.6 (with penalties, 120 rows of 131,072 30.3 and 29.6), bf16 112 rows 24.4 and 23.0, 26.5 and 25.1, 128 rows 24.4 and 26.7, 26.6 and 26.5 (with penalties 34.5 and 31.6).
+    //   28.6, 30.7 and 30.6 (with penalties, 120 rows of 131,072 30.3 and 29.6), bf16 112 rows 24.4 and 23.0, 26.5 and 25.1, 128 rows 24.4
+    //   and 26.7, 26.6 and 26.5 (with penalties 34.5 and 31.6); seven, 80 rows of 262,144 fp32 36.0 and 36.5, 40.6 and 35.4, 100 rows 36.5
+    //   and 42.3, 41.3 and 40.4, 128 rows 37.2 and 49.7, 42.6 and 47.3, bf16 100 rows 32.3 and 33.3, 34.9 and 35.2 (with penalties, 128 rows
+    //   46.3 and 41.4, 160 46.4 and 44.6).
     // * longer rows, whose results are written and read back, from about half the compute units on: there nothing is gained by
     //   spreading a row over workers, since a compute unit streams at little more than its share of the memory bandwidth anyway,
     //   and tails that run beside the streaming slow it down by more than they gain.
-    static const int from[2][2][3] = {{{8, 9, 10}, {8, 11, 15}}, {{8, 11, 14}, {12, 13, 17}}};
+    static const int above[2][2][3] = {{{16, 12, 10}, {16, 15, 15}}, {{16, 14, 13}, {24, 17, 17}}};  // rows, in 32nds of the compute units
     if (s_min <= 1)
         g.own_rows = true;
-    else if (s_min <= 4)
-        g.own_rows = n_rows * s_min * 8 > cu_count * from[epv == 8][max_sel > SR_TK_LONG_SEL][s_min - 2];
+    else if (s_min <= SR_TK_KEPT_CHUNKS)
+        g.own_rows = n_rows * 32 > cu_count * above[epv == 8][max_sel > SR_TK_LONG_SEL][std::min(s_min, 4) - 2];
     else
         g.own_rows = n_rows * 32 >= cu_count * 17;
     int s = s_min;
@@ -1267,7 +1270,7 @@ int sr_sample_launch(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int
         a.n_workers = b->n_workers;
         a.cu_count = ctx->cu_count;
         a.own_rows = b->own_rows ? 1 : 0;
-        if (b->own_rows && b->n_workers > 2 * ctx->cu_count)
+        if (b->own_rows && a.chunks <= SR_TK_KEPT_CHUNKS && b->n_workers > 2 * ctx->cu_count)
             a.start_gap = (uint32_t)std::min((double)b->vocab * (dtype == SR_DTYPE_BF16 ? 2.0 : 4.0) * ctx->cu_count / SR_TK_START_GAP, 1e5);
         a.short_lists = b->max_sel <= SR_TK_SHORT_SEL ? 1 : 0;
         a.n_items = b->n_items;

@@ -470,9 +470,18 @@ __device__ __forceinline__ uint32_t largest_key16(uint32_t kmax, Enough enough)
 // Called by every thread of the tail workgroup of a row once all chunks of the row have been counted in.
 // slot = position of the row in this launch.
 // What a worker that streams all chunks of its own row keeps of them in registers instead of writing it out: per
-// chunk (at most kKeptChunks) the thread's four group maxima, second maxima and packed positions.  The waves' shares
+// chunk (at most kKeptChunks, or pairs of them: kFold) the thread's four group maxima, second maxima and packed positions.  The waves' shares
 // of the row's bound and their largest kept elements lie in sm.hist, two words per (chunk, wave).
 constexpr int kKeptChunks = 4;
+// Rows of five to eight chunks (kFold): chunk c + 4 joins the groups of chunk c, in the registers of the one that keeps its row's
+// results as it streams, in those of a tail that reads them as it reads them.  A position inside such a group is the chunk's
+// own, and kFoldPos more in the second chunk.  Without, a tail of more than four chunks fetched every group at or above the bound
+// again, and every worker wrote its results out: 1, 64, 256 and 590 rows of 262,144 fp32 (top-k up to 1,000) 30.4, 54.2, 89.5, 181
+// -> 18.7, 32.7, 54.6, 111 us; 1, 64 and 256 of 160,000 27.8, 45.8, 69.1 -> 18.0, 27.1, 40.6; of 262,144 bf16 33.1, 48.6, 71.5 ->
+// 18.3, 31.0, 37.8.  (Launches of up to four chunks are compiled without it.)
+constexpr int kFoldChunks = 2 * kKeptChunks;
+static_assert(kFoldChunks == SR_TK_KEPT_CHUNKS, "as the host deals the rows");
+template <int EPV, int kVec> constexpr int kFoldPos = (kVec + SR_TK_GROUPS - 1) / SR_TK_GROUPS * EPV;
 struct KeptGroups {
     float4 g1[kKeptChunks], g2[kKeptChunks];
     uint32_t gp[kKeptChunks];
@@ -510,7 +519,7 @@ __device__ __forceinline__ bool row_history_in_registers(const SrRow& rd)
     return use_edits && (rd.flags & kRowHistExcl) != 0u && rd.path == SR_PATH_TOPK && rd.edit_cnt <= kHistRegs * kThreads;
 }
 
-template <int EPV, int kVec, bool kKept, bool kShort, typename Early, typename Late>
+template <int EPV, int kVec, bool kKept, bool kShort, bool kFold, typename Early, typename Late>
 __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, int row, const SrRow& rd, bool want_bins,
                                                 bool force_exact, float inv_temp, BinMap* map_out,
                                                 float* bound_out, bool* binned, const KeptGroups& kept, Early&& early,
@@ -521,7 +530,7 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
 // kShort: the launch holds no row that asks for more than kShortSel entries; the tail then carries the two steps that
 // pay for such rows only (a closer bound from the waves' pairs, ranking a short list by counting).  They are compiled
 // into launches of their own because their mere presence costs the long tails of other launches 0.6 us.
-template <int EPV, int kVec, bool kKept, bool kShort>
+template <int EPV, int kVec, bool kKept, bool kShort, bool kFold>
 __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int row, const SrRow& rd, bool force_exact,
                                               const KeptGroups& kept, const KeptHistory& kept_hist, TopkSmem& sm)
 {
@@ -566,7 +575,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
     if (tid == 0) sm.bcast[4] = 0u;  // the short list's count of history entries (the barriers of the next call publish it)
     BinMap map0;
     float bound0 = 0.0f;
-    const int n_c = build_candidates<EPV, kVec, kKept, kShort>(
+    const int n_c = build_candidates<EPV, kVec, kKept, kShort, kFold>(
         a, slot, row, rd, want_bins, force_exact, inv_temp, &map0, &bound0, &binned, kept,
         [&]() SR_INL {
             if constexpr (!(kKept)) {
@@ -1357,7 +1366,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
 // force_exact, and any row whose candidates overflow the lists: the row's sel-th largest kept element is found by a
 // radix select over the logits themselves, and the candidates are exactly the sel largest in (value desc, index asc)
 // order.  Slow (several passes over the row), exact for any data, and independent of the chunk results.
-template <int EPV, int kVec, bool kKept, bool kShort, typename Early, typename Late>
+template <int EPV, int kVec, bool kKept, bool kShort, bool kFold, typename Early, typename Late>
 __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, int row, const SrRow& rd, bool want_bins,
                                                 bool force_exact, float inv_temp, BinMap* map_out,
                                                 float* bound_out, bool* binned, const KeptGroups& kept, Early&& early,
@@ -1390,6 +1399,10 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
     auto gm_load = [&](int c) SR_INL -> float4 { return gm[(size_t)c * kThreads]; };
     // the element index of the largest element of group g of chunk c: p = (vector inside the group) * EPV + q
     auto idx_of = [&](int c, int g, uint32_t p) SR_INL -> int {
+        if (kFold && p >= (uint32_t)kFoldPos<EPV, kVec>) {
+            c += kKeptChunks;
+            p -= (uint32_t)kFoldPos<EPV, kVec>;
+        }
         const int fv = c * a.chunk_vecs + (g + (int)(p / EPV) * SR_TK_GROUPS) * kThreads + tid;
         return fv * EPV + (int)(p % EPV) - mis;
     };
@@ -1547,10 +1560,12 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
         if constexpr (kKept) gmr[c] = c < S ? kept.g1[c] : make_float4(SR_NEG_INF, SR_NEG_INF, SR_NEG_INF, SR_NEG_INF);
         else gmr[c] = c < S ? gm_load(c) : make_float4(SR_NEG_INF, SR_NEG_INF, SR_NEG_INF, SR_NEG_INF);
     }
+    float4 gmb[kGmRegs], g2b[kGmRegs];  // (kFold) of the chunks that join
+    uint32_t gpb[kGmRegs];
     static_assert(kGmRegs == kKeptChunks, "kept chunks fill the direct path's registers");
     // with few chunks the second maxima and the positions of the maxima come along in the same batch of loads
     constexpr int kG2Regs = 4;
-    const bool direct = S <= kG2Regs;  // a group whose second largest is below the bound hands over its largest directly
+    const bool direct = kFold || S <= kG2Regs;  // a group whose second largest is below the bound hands over its largest directly
     float4 g2r[kG2Regs];
     uint32_t gpr[kG2Regs];
 #pragma unroll
@@ -1564,6 +1579,16 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
             gpr[c] = in ? a.gpos[((size_t)slot * S + c) * kThreads + tid] : 0u;
         }
     }
+    if constexpr (kFold && !kKept) {
+#pragma unroll
+        for (int c = 0; c < kG2Regs; c++) {
+            const bool in = c + kKeptChunks < S;
+            const size_t go = ((size_t)slot * S + c + kKeptChunks) * kThreads + tid;
+            gmb[c] = in ? a.gmax[go] : make_float4(SR_NEG_INF, SR_NEG_INF, SR_NEG_INF, SR_NEG_INF);
+            g2b[c] = in ? a.gmax2[go] : make_float4(SR_NEG_INF, SR_NEG_INF, SR_NEG_INF, SR_NEG_INF);
+            gpb[c] = in ? a.gpos[go] : 0u;
+        }
+    }
     // (not kKept) the waves' shares of the bound, asked for with the group results: behind the barrier below they
     // would be a round trip to memory of their own
     const int nb = kKept ? kWaves : S * kWaves;  // (a worker that keeps its row's results: one share per wave and row)
@@ -1572,11 +1597,28 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
         if (lane < nb) gb0 = ((const uint2*)a.gbound + (size_t)slot * nb)[lane];
     }
     early();
+    if constexpr (kFold && !kKept) {
+        // (the first of equal values is the earlier chunk's)
+        auto join = [&](float& m1, float& m2, uint32_t& gp, float b1, float b2, uint32_t bp, int g) SR_INL {
+            const bool up = b1 > m1;
+            gp = up ? (gp & ~(0xffu << (8 * g))) | ((((bp >> (8 * g)) & 0xffu) + (uint32_t)kFoldPos<EPV, kVec>) << (8 * g)) : gp;
+            m2 = fmaxf(fminf(m1, b1), fmaxf(m2, b2));
+            m1 = fmaxf(m1, b1);
+        };
+#pragma unroll
+        for (int c = 0; c < kG2Regs; c++) {
+            join(gmr[c].x, g2r[c].x, gpr[c], gmb[c].x, g2b[c].x, gpb[c], 0);
+            join(gmr[c].y, g2r[c].y, gpr[c], gmb[c].y, g2b[c].y, gpb[c], 1);
+            join(gmr[c].z, g2r[c].z, gpr[c], gmb[c].z, g2b[c].z, gpb[c], 2);
+            join(gmr[c].w, g2r[c].w, gpr[c], gmb[c].w, g2b[c].w, gpb[c], 3);
+        }
+    }
     auto each_gm = [&](auto&& f) SR_INL {
 #pragma unroll
         for (int c = 0; c < kGmRegs; c++)
             if (c < S) f(c, gmr[c]);
-        for (int c = kGmRegs; c < S; c++) f(c, gm_load(c));
+        if constexpr (!kFold)
+            for (int c = kGmRegs; c < S; c++) f(c, gm_load(c));
     };
     bool bins = false;
     BinMap map;
@@ -1606,7 +1648,7 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
     // fetches the listed groups, kBatch (group, vector) items per thread at a time -- values and keep-bits
     // of all of them in one batch of loads -- and appends every kept element that pred admits to the candidates
     auto gather = [&](int nq, auto&& pred) SR_INL {
-        const int n_items = nq * kGV;
+        const int n_items = nq * kGV * (kFold ? 2 : 1);
         for (int i0 = 0; i0 < n_items; i0 += kBatch * kThreads) {
             u32x4 v[kBatch];
             uint32_t kw[kBatch];
@@ -1618,9 +1660,10 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
                 v[r] = VO::neg_inf();
                 kw[r] = 0u;
                 if (i0 + r * kThreads < n_items && i < n_items) {  // the first test is uniform: unused slots cost nothing
-                    const uint32_t gid = qlist[i / kGV];
-                    const int m = i - (i / kGV) * kGV;
-                    const int g = (int)(gid & 3u), t = (int)((gid >> 2) & (kThreads - 1)), c = (int)(gid >> 11);
+                    const int part = i / kGV;  // (kFold: two of a group)
+                    const uint32_t gid = qlist[kFold ? part >> 1 : part];
+                    const int m = i - part * kGV;
+                    const int g = (int)(gid & 3u), t = (int)((gid >> 2) & (kThreads - 1)), c = (int)(gid >> 11) + (kFold ? (part & 1) * kKeptChunks : 0);
                     const int f0 = c * a.chunk_vecs;
                     const int nv = min(a.chunk_vecs, nvt - f0);
                     const int j = g + m * SR_TK_GROUPS;
@@ -1856,14 +1899,14 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
 // registers, so every thread has up to kVec loads in flight from its first chunk to its last, and the stores, the
 // per-wave bound and the hand-off of a chunk run under the loads of the next one.
 //
-// kKept: every worker streams all chunks (at most kKeptChunks) of the one row it finishes.  Nothing is handed over then,
+// kKept: every worker streams all chunks (at most kFoldChunks) of the one row it finishes.  Nothing is handed over then,
 // so nothing is written out: the group results of all chunks stay in the thread's registers and the waves' shares of the
 // bound go through LDS.  Also where two workers share a compute unit: 128 registers hold it (the tail spills 44 bytes a lane;
 // of the shape that writes its results and reads them back 84, and that one pays a bound loop per chunk): 1,024
 // rows of 151,936 fp32 147.5 -> 113.5 us, 512 80.0 -> 59.7, 320 62.1 -> 47.6, 1,024 of bf16 95.7 -> 69.5.
 // kRoomy: a launch of at most one worker per compute unit, compiled for two waves a SIMD, so that the row tail keeps its
 // registers.
-template <int EPV, int kVec, int kWindow, bool kKept, bool kShort, bool kRoomy>
+template <int EPV, int kVec, int kWindow, bool kKept, bool kShort, bool kRoomy, bool kFold>
 __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkArgs a)
 {
     __shared__ TopkSmem sm;
@@ -2042,6 +2085,23 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
             int gp1[SR_TK_GROUPS];
 #pragma unroll
             for (int g = 0; g < SR_TK_GROUPS; g++) { gm1[g] = SR_NEG_INF; gm2[g] = SR_NEG_INF; gp1[g] = 0; }
+            constexpr bool kJoin = kFold && kKept;
+            const bool joins = kJoin && cur.c >= kKeptChunks;
+            if constexpr (kJoin) {
+                // the groups of the chunk that this one joins; their positions count from this one's (negative)
+                if (joins) {
+#pragma unroll
+                    for (int c = 0; c < kKeptChunks; c++) {
+                        const bool on = cur.c - kKeptChunks == c;
+                        gm1[0] = on ? kept.g1[c].x : gm1[0]; gm1[1] = on ? kept.g1[c].y : gm1[1];
+                        gm1[2] = on ? kept.g1[c].z : gm1[2]; gm1[3] = on ? kept.g1[c].w : gm1[3];
+                        gm2[0] = on ? kept.g2[c].x : gm2[0]; gm2[1] = on ? kept.g2[c].y : gm2[1];
+                        gm2[2] = on ? kept.g2[c].z : gm2[2]; gm2[3] = on ? kept.g2[c].w : gm2[3];
+#pragma unroll
+                        for (int g = 0; g < SR_TK_GROUPS; g++) gp1[g] = on ? (int)((kept.gp[c] >> (8 * g)) & 0xffu) - kFoldPos<EPV, kVec> : gp1[g];
+                    }
+                }
+            }
 #pragma unroll
             for (int j = 0; j < kVecP; j++) {
                 const int g = j % SR_TK_GROUPS;
@@ -2079,11 +2139,17 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
                 const uint32_t* mw = keep_words(nxt);
                 kw0 = mw[0]; kw1 = mw[1]; kw2 = mw[2];
             }
+            if constexpr (kJoin) {
+                if (joins) {
+#pragma unroll
+                    for (int g = 0; g < SR_TK_GROUPS; g++) gp1[g] += kFoldPos<EPV, kVec>;
+                }
+            }
             const uint32_t gpk = (uint32_t)gp1[0] | ((uint32_t)gp1[1] << 8) | ((uint32_t)gp1[2] << 16) | ((uint32_t)gp1[3] << 24);
             if constexpr (kKept) {
 #pragma unroll
                 for (int c = 0; c < kKeptChunks; c++) {
-                    const bool on = cur.c == c;
+                    const bool on = (kFold ? cur.c & (kKeptChunks - 1) : cur.c) == c;
                     kept.g1[c].x = on ? gm1[0] : kept.g1[c].x; kept.g1[c].y = on ? gm1[1] : kept.g1[c].y;
                     kept.g1[c].z = on ? gm1[2] : kept.g1[c].z; kept.g1[c].w = on ? gm1[3] : kept.g1[c].w;
                     kept.g2[c].x = on ? gm2[0] : kept.g2[c].x; kept.g2[c].y = on ? gm2[1] : kept.g2[c].y;
@@ -2182,7 +2248,7 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
         // the row's results are in this workgroup's registers and LDS; a worker whose program is not of that kind (the
         // host writes none for this kernel) selects its row from the logits alone
         // (the waves' shares of the bound are read behind the barrier that follows the clearing of the tail's lists)
-        handed_over = own_row && S <= kKeptChunks && a.spin_limit != 0u;
+        handed_over = own_row && S <= (kFold ? kFoldChunks : kKeptChunks) && a.spin_limit != 0u;
     } else {
         if (own_row) sr_drain_stores();  // every wave's own stores; the barrier below joins them
         if (tid == 0) {
@@ -2200,7 +2266,7 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
     }
     SR_PROF(ap, 4);
     __builtin_amdgcn_s_setprio(3);  // the tail is the longer dependent chain: its waves go first
-    topk_row_tail<EPV, kVec, kKept, kShort>(ap, tslot, trow, trd, !handed_over, kept, kept_hist, sm);
+    topk_row_tail<EPV, kVec, kKept, kShort, kFold>(ap, tslot, trow, trd, !handed_over, kept, kept_hist, sm);
     SR_PROF(ap, 15);
 }
 
@@ -2439,15 +2505,18 @@ hipError_t sr_launch_topk(const SrTopkArgs& a, int n_rows, hipStream_t stream)
     if (n_rows <= 0) return hipSuccess;
     dim3 grid((unsigned)a.n_workers), block(kThreads);
     // workers with a row of their own keep the results of its chunks in their registers, where these are few enough
-    const bool kept = a.own_rows && a.chunks <= kKeptChunks, roomy = a.n_workers <= a.cu_count;
+    const bool kept = a.own_rows && a.chunks <= kFoldChunks, roomy = a.n_workers <= a.cu_count, fold = a.chunks > kKeptChunks && a.chunks <= kFoldChunks;
     // ... and a launch whose rows all ask for few entries carries the steps that pay for such rows only
     auto launch = [&](auto epv, auto vec, auto shrt) {
         constexpr int kE = decltype(epv)::value, kV = decltype(vec)::value;
         constexpr bool kS = decltype(shrt)::value;
-        if (kept && roomy) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS, true>), grid, block, 0, stream, a);
-        else if (kept) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS, false>), grid, block, 0, stream, a);
-        else if (roomy && !a.own_rows) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW, false, kS, true>), grid, block, 0, stream, a);
-        else hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_OWN, false, kS, false>), grid, block, 0, stream, a);
+        if (kept && roomy && fold) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS, true, true>), grid, block, 0, stream, a);
+        else if (kept && roomy) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS, true, false>), grid, block, 0, stream, a);
+        else if (kept && fold) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS, false, true>), grid, block, 0, stream, a);
+        else if (kept) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_KEPT, true, kS, false, false>), grid, block, 0, stream, a);
+        else if (roomy && fold) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW, false, kS, true, true>), grid, block, 0, stream, a);
+        else if (roomy && !a.own_rows) hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW, false, kS, true, false>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((k_topk_rows<kE, kV, SR_TK_WINDOW_OWN, false, kS, false, false>), grid, block, 0, stream, a);
     };
     using std::integral_constant;
     if (a.dtype == 1) {

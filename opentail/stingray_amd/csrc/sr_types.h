@@ -104,6 +104,7 @@ struct SrMaskClear {
 #define SR_TK_LONG_SEL 256                 // ... and one of which some row asks for more than this many: see topk_geometry
 #define SR_TK_SEL_MAX 2048                 // most entries (candidates + history ids) the row tail sorts
 #define SR_TK_ROW_CAP 8192                 // candidates all chunks of a row may hand to its tail (16 per thread)
+#define SR_TK_KEPT_CHUNKS 8                 // most of a row whose results a worker keeps in registers, in pairs beyond four
 #define SR_TK_MAX_CHUNKS 128               // most workgroups one row is split over
 
 // Full-vocabulary path: nucleus candidates up to this count are sorted inside the row kernel.

@@ -71,6 +71,34 @@ def test_rows_with_and_without_a_worker_of_their_own(ctx, rows, vocab, longest, 
     _check(ctx, np.random.default_rng(rows * 5 + vocab), rows, vocab, longest, bf16)
 
 
+# Rows of five to eight chunks, whose second four join the groups of the first, and of nine: the chunks' edges, with the largest
+# entries in both chunks of a pair and ties across them, dealt out, a worker to a row, and two to a compute unit.
+@pytest.mark.parametrize("rows", [1, 7, 90, 140, 258])
+@pytest.mark.parametrize("vocab,longest,bf16", [(4 * CHUNK + 1, 1000, False), (6 * CHUNK + 5, 64, False), (8 * CHUNK - 3, 1000, False), (8 * CHUNK + 3, 300, False),
+                                                (7 * 512 * 10 * 8 - 1, 1000, True)])
+def test_rows_of_more_than_four_chunks(ctx, rows, vocab, longest, bf16):
+    if rows > 100 and vocab > 7 * CHUNK:
+        vocab = 5 * CHUNK + 7
+    _check(ctx, np.random.default_rng(rows * 3 + vocab), rows, vocab, longest, bf16)
+
+
+def test_ties_across_chunks_that_share_their_groups(ctx):
+    import torch
+
+    rng = np.random.default_rng(5)
+    vocab, rows = 6 * CHUNK, 9
+    for n in (rows, 150):
+        logits = rng.normal(0, 1, (n, vocab)).astype(np.float32)
+        at = 4 * (512 * 4 * 3 + 200) + 1  # an element of a group, and the ones at its place in the chunk that joins it
+        logits[:, at] = logits[:, at + 4 * CHUNK] = 9.0
+        logits[::2, at + CHUNK] = logits[::2, at + 5 * CHUNK] = 9.0
+        logits[1::3, at + 4 * CHUNK] = 9.5
+        params = [SamplingParams(Temperature=0.0 if r % 3 == 0 else 0.7, TopK=[1, 2, 3, 50][r % 4], RepetitionPenalty=1.0) for r in range(n)]
+        u = rng.random(n)
+        got = ctx.sample_batch(torch.from_numpy(logits).cuda(), params, u)
+        assert np.array_equal(got, oracle_tokens(logits, params, u)), n
+
+
 # Launches of more than two turns of workers, whose second ones start late: the same tokens at every step, also with work of other
 # streams on the device.
 @pytest.mark.parametrize("rows,vocab,bf16", [(513, 20_011, False), (1030, 40_000, True)])
