@@ -385,8 +385,9 @@ __device__ __forceinline__ void seg_load_rec(const SeqSegFunc* funcs, int seg, i
 // follows is done again.  A segment taken by itself costs some 50 instructions of the one wave, 0.1 us, a sum that
 // starts at zero has about a dozen; looking for the end of every run of segments as it went, the walk took 0.45 us for each:
 // 98 segments of a row of 100,003 entries 5.3 us, and a search over as many 7.5.
-// first64: the first 64 records, where the caller has asked for them already.  kFew: there are no more than those.
-template <bool kSearch, bool kAgent = false, bool kFew = false, typename Load>
+// first64: the first 64 records, where the caller has asked for them already.  kFew: there are no more than those.  kNear: they lie in
+// shared memory, mostly, and are not asked for ahead (24 registers less).
+template <bool kSearch, bool kAgent = false, bool kFew = false, bool kNear = false, typename Load>
 __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSegFunc* funcs, float s0, float target, int* found,
                                                float* states, const SegRec* first64 = nullptr)
 {
@@ -397,8 +398,9 @@ __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSeg
     if (first64) next = *first64;
     else seg_load_rec<kAgent>(funcs, lane, nseg, next);
     for (int base = 0; base < nseg; base += SR_WAVE) {
+        if (kNear && base > 0) seg_load_rec<kAgent>(funcs, base + lane, nseg, next);
         const SegRec r = next;
-        if (!kFew && base + SR_WAVE < nseg) seg_load_rec<kAgent>(funcs, base + SR_WAVE + lane, nseg, next);  // (the next 64 segments' come in meanwhile)
+        if (!kFew && !kNear && base + SR_WAVE < nseg) seg_load_rec<kAgent>(funcs, base + SR_WAVE + lane, nseg, next);  // (the next 64 segments' come in meanwhile)
         const uint32_t kind = r.f.w & 0xffu;
         const bool simple = kind == SR_SEG_PLAIN && r.f.x == r.f.y && r.f.x < (1u << 24), split = kind == SR_SEG_SPLIT;
         const unsigned long long stops = ~__ballot(simple || kind == SR_SEG_ZERO);
@@ -4738,6 +4740,461 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_factor(SrFullArgs a, SrSpecA
     }
 }
 
+// ---- launches of which every row is open: nothing cuts, biases or penalises it, and the ratio test decides ------------------------
+// An accept test needs p at one token, and p = fl(fl(e m1) m2) is e / S to spec_open_spread(n) whatever the exact sums are: m1 = fl(1 / s), and m2 is s
+// / S but for the roundings of the accumulators.  So the pass over all positions needs neither e to the last bit nor a sum in
+// order, and no position waits for another's: k_spec_units reads the logits once, a wave a unit of 2,048, and leaves every unit's
+// maximum and about its sum of exp(x - maximum), by lane accumulator.  What needs the exact factors -- the positions in front of the
+// first certain rejection whose test is open, and the one that is drawn from, one or two of nine -- k_spec_open works out from
+// the logits: e, the records of its sum, m1; the records of the eight accumulators over fl(e m1), m2.
+// 16 sequences of 8 drafts over 262,144 (144 rows), us: this one 23 (6.6 TB/s; k_full_softmax_seg, with e, two meetings and records, 59),
+// k_full_row none (15), k_spec_open 45 (k_spec_factor 28; its chain: tests 3.4, the block from its logits 8, records 5, walk 7, records 5,
+// walk 4), k_spec_rows 23 both; the call 127 -> 98.  A further position with an open test is another 25.
+// A unit's maximum is exact; a term's exponential is v_exp_f32 of a difference rounded once: 2^-24 of the exponent's size, which is
+// below 28 for all terms that make up more than 2^-22 of the sum.
+// What k_spec_open leaves of a row's tests, behind its meeting point (SrSpecArgs::sync): the positions that it worked out, a bit each; those
+// of them whose draft is accepted; the position that ends the row for certain, and above it whether its id lies outside the vocabulary
+constexpr int kSpecPicked = 4, kSpecAccepted = 5, kSpecLast = 6;
+constexpr int kSpecDone = -2;  // SrSpecArgs::reject of a row whose results are written
+constexpr int kUnitVecs = SR_UNIT_TERMS / (4 * SR_WAVE);
+constexpr float kLog2E = 0x1.715476p+0f;
+__global__ __launch_bounds__(256) void k_spec_units(SrFullArgs a, SrSpecArgs s)
+{
+    const int slot = blockIdx.y, lane = sr_lane(), u = (int)blockIdx.x * 4 + sr_wave_id(), n = s.vocab;
+    if (blockIdx.x == 0 && threadIdx.x < 2) {  // nobody has counted in
+        a.row_sync[(size_t)slot * SR_ROW_SYNC_STRIDE + 1 + threadIdx.x] = 0ull;
+        if (slot % (s.n_draft + 1) == 0 && threadIdx.x == 0) s.sync[(size_t)(slot / (s.n_draft + 1)) * SR_ROW_SYNC_STRIDE + kSpecAccepted] = 0ull;
+    }
+    if (u >= s.n_units) return;
+    const SrRow rd = s.rows[slot / (s.n_draft + 1)];
+    const float inv_temp = row_inv_temp(rd);
+    const float* const x = s.target_logits + (size_t)slot * (size_t)n;
+    float v[kUnitVecs][4];
+    const int base = u * SR_UNIT_TERMS + lane * 4;
+    if ((u + 1) * SR_UNIT_TERMS <= n) {
+#pragma unroll
+        for (int k = 0; k < kUnitVecs; k++) {
+            const float4 t = sr_load_f4(x + base + k * 4 * SR_WAVE);
+            v[k][0] = t.x; v[k][1] = t.y; v[k][2] = t.z; v[k][3] = t.w;
+        }
+        if (rd.temperature != 1.0f) {
+#pragma unroll
+            for (int k = 0; k < kUnitVecs; k++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[k][q] = __fmul_rn(v[k][q], inv_temp);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < kUnitVecs; k++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int i = base + k * 4 * SR_WAVE + q;
+                v[k][q] = i < n ? __fmul_rn(x[i], inv_temp) : SR_NEG_INF;
+            }
+    }
+    float m = v[0][0];
+#pragma unroll
+    for (int k = 0; k < kUnitVecs; k++) m = sr_max3_f32(sr_max3_f32(m, v[k][0], v[k][1]), v[k][2], v[k][3]);
+    m = sr_okey_inv(sr_wave_max_u32(m == m ? sr_okey(m) : 0x007fffffu));  // (a NaN beside numbers is left out here; its exponential is one)
+    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < kUnitVecs; k++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) acc[q] += __builtin_amdgcn_exp2f((v[k][q] - m) * kLog2E);
+    // lane l holds the terms of the accumulators 4 (l & 1) ... 4 (l & 1) + 3
+    float c[SR_SEQ_CHAINS];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        c[q] = (lane & 1) ? 0.0f : acc[q];
+        c[4 + q] = (lane & 1) ? acc[q] : 0.0f;
+    }
+    float chain = wave_sum_8(c);  // (of accumulator lane & 7)
+    float sum = sr_wave_sum_f32((acc[0] + acc[1]) + (acc[2] + acc[3]));
+    if (!(sum > 0.0f)) {  // (the same in every lane) nothing above -inf, +inf, or a NaN
+        bool nan = false;
+#pragma unroll
+        for (int k = 0; k < kUnitVecs; k++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) nan = nan || v[k][q] != v[k][q];
+        if (__ballot(nan) != 0ull) m = sr_u2f(0x7fc00000u);
+        sum = chain = 0.0f;
+    }
+    const size_t at = (size_t)slot * s.n_units + u;
+    if (lane < SR_SEQ_CHAINS) s.unit_chains[at * SR_SEQ_CHAINS + lane] = chain;
+    if (lane == 0) s.units[at] = make_float2(m, sum);
+}
+
+// A row's units, kUnits a lane: its maximum, and about its sum relative to it.  One wave.
+constexpr int kUnitsMost = SR_SEG_MAX * SR_SEG_TERMS / SR_UNIT_TERMS / SR_WAVE, kUnitsFew = 2;
+struct SpecRow {
+    float max, sum;
+    int kind;  // 0: numbers   1: a NaN, or nothing above -inf: the row is uniform   2: +inf
+};
+template <int kUnits>
+__device__ __forceinline__ SpecRow spec_row(const SrSpecArgs& s, size_t slot, float2 (&w)[kUnits])
+{
+    const int lane = sr_lane();
+    SpecRow r;
+    float m = SR_NEG_INF;
+    bool nan = false;
+#pragma unroll
+    for (int k = 0; k < kUnits; k++) {
+        // (no lane's load behind a condition: they would wait for each other)
+        w[k] = make_float2(SR_NEG_INF, 0.0f);
+        if (k * SR_WAVE < s.n_units) w[k] = s.units[slot * s.n_units + min(k * SR_WAVE + lane, s.n_units - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < kUnits; k++)
+        if (k * SR_WAVE + lane >= s.n_units) w[k] = make_float2(SR_NEG_INF, 0.0f);
+#pragma unroll
+    for (int k = 0; k < kUnits; k++) {
+        nan = nan || w[k].x != w[k].x;
+        m = fmaxf(m, w[k].x);
+    }
+    r.max = sr_okey_inv(sr_wave_max_u32(sr_okey(m)));
+    r.kind = __ballot(nan) != 0ull || r.max == SR_NEG_INF ? 1 : r.max == -SR_NEG_INF ? 2 : 0;
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kUnits; k++)
+        if (k * SR_WAVE < s.n_units) sum += w[k].x > SR_NEG_INF ? w[k].y * __builtin_amdgcn_exp2f((w[k].x - r.max) * kLog2E) : 0.0f;
+    r.sum = sr_wave_sum_f32(sum);
+    return r;
+}
+// How far p is from e / S, as a part of it: n / 8 additions of an accumulator and a handful of roundings, and S itself (above).
+__device__ __forceinline__ double spec_open_spread(int n) { return ((double)(n / 8) + 200.0) * (1.1 / 16777216.0) + 3e-5; }
+
+// A workgroup per block of a row's 8,192 entries.  Each finds the positions whose factors are asked for by itself (a position a wave,
+// from the units), and takes them one by one: e of its block from the logits; the records of its eight segments (what stands in front is
+// known from the units: no meeting); counts in, and whoever is there last walks the row's records to s, while the others write e
+// and wait for m1 (bounded); then fl(e m1) by accumulator, the records, counts in, and whoever is there last walks those to m2.
+// A workgroup whose wait runs out marks the position (SrFullState::late_behind) and counts itself in; the last one then adds the
+// accumulators without records.  The words behind a position's meeting point (row_sync): 1 workgroups at the first count, 2 at
+// the second, 3 m1 with the launch's number above it.
+// one position of a row: e from the logits
+struct SpecOpenRow {
+    const float* lg;
+    const uint64_t* tab;  // of expf, in shared memory
+    float inv_temp, max, uniform;
+    int kind, n, lane;
+    __device__ __forceinline__ float e(float x) const
+    {
+        const float d = __fsub_rn(__fmul_rn(x, inv_temp), max);
+        const float v = d == d ? sr_expf_neg(d, tab) : d;  // (beside +inf, +inf is no number and everything else 0)
+        return kind == 1 ? uniform : v;
+    }
+    // (for the walks' rare segments: a few at a time, beside which the walk keeps its registers)
+    template <int kN> __device__ __forceinline__ void all(float (&x)[kN]) const
+    {
+#pragma unroll
+        for (int j = 0; j < kN; j++) {
+            x[j] = e(x[j]);
+            if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // a lane's 16 entries of e of a segment
+    __device__ __forceinline__ void run(int sg, float (&x)[SR_SEQ_RUN]) const
+    {
+        const int i0 = sg * SR_SEG_TERMS + lane * SR_SEQ_RUN;
+        if ((sg + 1) * SR_SEG_TERMS <= n) {
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j += 4) {
+                const float4 l = sr_load_f4(lg + i0 + j);
+                x[j] = l.x; x[j + 1] = l.y; x[j + 2] = l.z; x[j + 3] = l.w;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = lg[min(i0 + j, n - 1)];
+        }
+        all(x);
+#pragma unroll
+        for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = i0 + j < n ? x[j] : 0.0f;
+    }
+    // ... and of accumulator g of a block: fl(e m1)
+    __device__ __forceinline__ void accumulator(int b, int g, float m1, float (&x)[SR_SEQ_RUN]) const
+    {
+        const int t0 = b * SR_SEG_TERMS + lane * SR_SEQ_RUN, nv = n / 8;
+#pragma unroll
+        for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = lg[(size_t)min(t0 + j, nv - 1) * 8 + g];
+        all(x);
+#pragma unroll
+        for (int j = 0; j < SR_SEQ_RUN; j++) x[j] = t0 + j < nv ? __fmul_rn(x[j], m1) : 0.0f;
+    }
+};
+__device__ __forceinline__ float spec_m(float sum) { return sum > 0.0f && sum != 1.0f ? __fdiv_rn(1.0f, sum) : 1.0f; }
+// All records of a row that others of the launch have made, into shared memory, by the workgroup, where they fit: the waves' trips to
+// memory overlap, where the walk of one wave makes them one behind the other.
+template <int kThreads>
+__device__ __forceinline__ bool stage_records(const SeqSegFunc* recs, int nrec, float4* room, int room_bytes)
+{
+    const bool fits = nrec * (int)sizeof(SeqSegFunc) <= room_bytes;
+    if (fits) {
+        const unsigned long long* const from = (const unsigned long long*)recs;
+        unsigned long long* const to = (unsigned long long*)room;
+        constexpr int kWords = sizeof(SeqSegFunc) / 8, kAhead = 6;
+        for (int i0 = threadIdx.x; i0 < nrec * kWords; i0 += kThreads * kAhead) {
+            unsigned long long v[kAhead];
+#pragma unroll
+            for (int k = 0; k < kAhead; k++) v[k] = i0 + k * kThreads < nrec * kWords ? sr_load_agent(from + i0 + k * kThreads) : 0ull;
+#pragma unroll
+            for (int k = 0; k < kAhead; k++)
+                if (i0 + k * kThreads < nrec * kWords) to[i0 + k * kThreads] = v[k];
+        }
+    }
+    __syncthreads();
+    return fits;
+}
+
+template <int kUnits>  // a lane (eight cost 30 registers that most vocabularies do not need)
+__global__ __launch_bounds__(kPrepT, 4) void k_spec_open(SrFullArgs a, SrSpecArgs s)
+{
+    __shared__ PreparedSmem sm;
+    __shared__ uint64_t tab[32];
+    __shared__ int test[SR_WAVE];       // of every position   1: its test is open   2: it ends the row   4: an id outside the vocabulary
+    __shared__ float seg_own[SR_SEQ_CHAINS];
+    const int row = blockIdx.y, blk = blockIdx.x, tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
+    const SrRow rd = s.rows[row];
+    const int n = s.vocab, L = s.n_draft, nseg = seg_count(n);  // (L < SR_WAVE)
+    const int nv = n / 8, rem = n - nv * 8, body = nv * 8, nblk = (nv + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
+    SpecOpenRow t;
+    t.tab = tab;
+    t.inv_temp = row_inv_temp(rd);
+    t.n = n;
+    t.uniform = __fdiv_rn(1.0f, (float)n);
+    if (tid < 32) tab[tid] = sr_exp2f_tab[tid];
+    __syncthreads();
+    float2 w[kUnits];
+    for (int i = wave; i < L; i += SR_SEQ_CHAINS) {
+        const size_t slot = (size_t)row * (L + 1) + i;
+        const int tok = s.draft_tokens[(size_t)row * L + i];
+        const bool bad = (uint32_t)tok >= (uint32_t)n;
+        const float x = bad ? 0.0f : s.target_logits[slot * (size_t)n + tok], qx = bad ? 0.0f : s.draft_probs[((size_t)row * L + i) * n + tok];
+        const double u = s.uniforms[(size_t)row * s.uniforms_per_row + i];
+        const SpecRow r = spec_row(s, slot, w);
+        bool open = r.kind != 0, ends = bad;
+        if (!bad && r.kind == 0) {
+            const float e = sr_expf_neg(__fsub_rn(__fmul_rn(x, t.inv_temp), r.max), tab);
+            const double y = (double)e / (double)r.sum;
+            if (!(e > 0.0f)) {
+                ends = !(u < 0.0);  // (p is 0, whatever the factors are, and so is the ratio)
+            } else if (!(qx > 0.0f)) {
+                open = y < 1e-29;
+                ends = !(u < 1.0);
+            } else {
+                const double ratio = y / (double)qx, d = spec_open_spread(n);
+                const bool low = u < fmin(1.0, ratio * (1.0 - d)), high = u < fmin(1.0, ratio * (1.0 + d));
+                open = low != high || y < 1e-29 || !(ratio >= 1e-30);  // (relative bounds end where numbers lose digits)
+                ends = !low;
+            }
+        }
+        if (lane == 0) test[i] = (open && !bad ? 1 : 0) | (ends ? 2 : 0) | (bad ? 4 : 0);
+    }
+    __syncthreads();
+    unsigned long long pick;
+    int last;
+    {
+        const int f = lane < L ? test[lane] : 0;
+        const unsigned long long end = __ballot((f & 3) == 2), wrong = __ballot((f & 4) != 0), undecided = __ballot((f & 1) != 0);
+        last = end != 0ull ? (int)__ffsll((long long)end) - 1 : L;
+        pick = undecided & ((1ull << last) - 1ull);
+        if (((wrong >> last) & 1ull) == 0ull) pick |= 1ull << last;  // (an id outside the vocabulary ends the row without a draw)
+    }
+    unsigned long long* const said = s.sync + (size_t)row * SR_ROW_SYNC_STRIDE;
+    if (blk == 0 && tid == 0) {
+        said[kSpecPicked] = pick;
+        said[kSpecLast] = (unsigned long long)last | (last < L && (test[last] & 4) != 0 ? 1ull << 32 : 0ull);
+    }
+    for (; pick != 0ull; pick &= pick - 1ull) {
+        // (what the lane's number gives is worked out here: kept over the whole loop, its dozens of offsets cost that many registers)
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        t.lane = ln;
+        const int pos = (int)__ffsll((long long)pick) - 1;
+        const size_t slot = (size_t)row * (L + 1) + (size_t)pos;
+        SrFullState* const st = a.state + slot;
+        unsigned long long* const sync = a.row_sync + slot * SR_ROW_SYNC_STRIDE;
+        SeqSegFunc* const recs = a.seg_func + slot * a.seg_stride;
+        SeqSegFunc* const chain = a.chain_func + (slot * SR_SEQ_CHAINS + wave) * a.chain_blocks;
+        float* const e_row = const_cast<float*>(s.p_all) + slot * (size_t)s.p_stride;
+        const int seg = blk * SR_SEQ_CHAINS + wave;
+        t.lg = s.target_logits + slot * (size_t)n;
+        // (all loads of a whole segment without a condition)
+        float v[4][4];
+        if ((seg + 1) * SR_SEG_TERMS <= n) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float4 x = sr_load_f4(t.lg + seg * SR_SEG_TERMS + (k * SR_WAVE + ln) * 4);
+                v[k][0] = x.x; v[k][1] = x.y; v[k][2] = x.z; v[k][3] = x.w;
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[k][q] = t.lg[min(seg * SR_SEG_TERMS + (k * SR_WAVE + ln) * 4 + q, n - 1)];
+        }
+        // about what stands in front of the block, of all terms and of the wave's accumulator
+        constexpr int kBlockUnits = kPrepBlock / SR_UNIT_TERMS;
+        float uc[kUnits] = {};
+#pragma unroll
+        for (int k = 0; k < kUnits; k++)
+            if (k * SR_WAVE < blk * kBlockUnits) uc[k] = s.unit_chains[(slot * s.n_units + min(k * SR_WAVE + ln, s.n_units - 1)) * SR_SEQ_CHAINS + wave];
+        const SpecRow r = spec_row(s, slot, w);
+        t.max = r.max;
+        t.kind = __builtin_amdgcn_readfirstlane(r.kind);
+        float before = 0.0f, before_chain = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kUnits; k++)
+            if (k * SR_WAVE < blk * kBlockUnits) {
+                const float scale = k * SR_WAVE + ln < blk * kBlockUnits && w[k].x > SR_NEG_INF ? __builtin_amdgcn_exp2f((w[k].x - r.max) * kLog2E) : 0.0f;
+                before += w[k].y * scale;
+                before_chain += uc[k] * scale;
+            }
+        before = sr_wave_sum_f32(before);
+        before_chain = sr_wave_sum_f32(before_chain);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[k][q] = t.e(v[k][q]);
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[k][q] = seg * SR_SEG_TERMS + (k * SR_WAVE + ln) * 4 + q < n ? v[k][q] : 0.0f;
+        }
+        auto write_e = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + ln) * 4;
+                if (i0 < n) sr_store_agent_f4((float4*)(e_row + i0), v[k][0], v[k][1], v[k][2], v[k][3]);  // (the rows of e are whole pieces long)
+            }
+        };
+        auto count_in = [&](int word) __attribute__((always_inline)) -> bool {  // whether this workgroup is the last one
+            sr_drain_stores();
+            __syncthreads();
+            if (tid == 0) sm.bc[0] = (uint32_t)__hip_atomic_fetch_add(sync + word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u == gridDim.x ? 1u : 0u;
+            __syncthreads();
+            return sm.bc[0] != 0u;
+        };
+        float m1 = 1.0f, x[SR_SEQ_RUN], own = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) own += (v[k][0] + v[k][1]) + (v[k][2] + v[k][3]);
+        own = sr_wave_sum_f32(own);
+        bool here = true;
+        if (t.kind == 0) {
+            // into the order of the sum, 16 terms a ln
+            float4* const turn = sm.room + wave * SR_WAVE * 5;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int i = (k * SR_WAVE + ln) * 4;
+                turn[(i >> 4) * 5 + ((i & 15) >> 2)] = make_float4(v[k][0], v[k][1], v[k][2], v[k][3]);
+            }
+            if (ln == 0) seg_own[wave] = own;
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float4 q = turn[ln * 5 + k];
+                x[4 * k] = q.x; x[4 * k + 1] = q.y; x[4 * k + 2] = q.z; x[4 * k + 3] = q.w;
+            }
+#pragma unroll
+            for (int g = 0; g < SR_SEQ_CHAINS; g++) before += g < wave ? seg_own[g] : 0.0f;
+            if (seg < nseg) seg_make_record<true>(x, seg, (double)before, recs + seg, own);
+            if (count_in(1)) {
+                const bool staged = stage_records<kPrepT>(recs, nseg, sm.room, (int)sizeof(sm.room));
+                if (wave == 0) {
+                    int dummy;
+                    auto load = [&](int sg, float (&y)[SR_SEQ_RUN]) __attribute__((always_inline)) { t.run(sg, y); };
+                    // (one piece of code for both places)
+                    const float f = spec_m(seg_walk_from<false, true, false, true>(load, nseg, staged ? (const SeqSegFunc*)sm.room : recs, 0.0f, 0.0f, &dummy, nullptr));
+                    if (ln == 0) {
+                        sr_store_agent(sync + 3, ((unsigned long long)a.seq << 32) | (unsigned long long)sr_f2u(f));
+                        sm.bc[1] = sr_f2u(f);
+                        sm.bc[2] = 1u;
+                    }
+                }
+                write_e();
+            } else {
+                write_e();
+                if (tid == 0) {
+                    uint32_t ok = 0u;
+                    unsigned long long word = 0ull;
+                    for (uint32_t it = 0; it < a.behind_wait_limit; it++) {
+                        word = sr_load_agent(sync + 3);
+                        if ((uint32_t)(word >> 32) == a.seq) { ok = 1u; break; }
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    if (ok == 0u) sr_store_agent(&st->late_behind, a.seq);
+                    sm.bc[2] = ok;
+                    sm.bc[1] = (uint32_t)word;
+                }
+            }
+            __syncthreads();
+            here = sm.bc[2] != 0u;
+            m1 = sr_u2f(sm.bc[1]);
+        } else {
+            write_e();
+        }
+        if (t.kind != 2 && here && blk < nblk) {
+            // chain by chain in shared memory, as in prepared_block
+            float* const buf = (float*)sm.room;
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int t4 = wave * (SR_SEG_TERMS / 4) + k * SR_WAVE + ln;
+                const int vec = t4 >> 1, j = vec & 15, l = vec >> 4;
+                const bool in = blk * kPrepBlock + 4 * t4 < body;
+                float* at = buf + (4 * (t4 & 1)) * 1024 + 64 * j + ((l + 2 * j) & 63);
+#pragma unroll
+                for (int q = 0; q < 4; q++) at[1024 * q] = in ? __fmul_rn(v[k][q], m1) : 0.0f;
+            }
+            __syncthreads();
+            own = 0.0f;
+#pragma unroll
+            for (int j = 0; j < SR_SEQ_RUN; j++) {
+                x[j] = buf[wave * 1024 + 64 * j + ((ln + 2 * j) & 63)];
+                own += x[j];
+            }
+            own = sr_wave_sum_f32(own);
+            const float front = t.kind == 0 ? before_chain * m1 : (float)(blk * SR_SEG_TERMS) * t.uniform;
+            seg_make_record<true>(x, blk, (double)front, chain + blk, own);
+        }
+        if (count_in(2)) {
+            // (everyone's e, records and marks are out; m1 is there)
+            if (tid == 0) {
+                sm.bc[2] = sr_load_agent(&st->late_behind) == a.seq ? 1u : 0u;
+                if (t.kind == 0) sm.bc[1] = (uint32_t)sr_load_agent(sync + 3);
+            }
+            __syncthreads();
+            if (t.kind == 0) m1 = sr_u2f(sm.bc[1]);
+            float m2 = 1.0f;
+            if (t.kind != 2) {
+                int dummy;
+                float sum = 0.0f;
+                if (sm.bc[2] == 0u) {
+                    sum = seg_walk_from<false, true, false, true>([&](int b, float (&y)[SR_SEQ_RUN]) __attribute__((always_inline)) { t.accumulator(b, wave, m1, y); },
+                                                     nblk, chain, 0.0f, 0.0f, &dummy, nullptr);
+                } else {
+                    for (int b = 0; b < nblk; b++) {  // (some workgroup stopped waiting and made no records)
+                        t.accumulator(b, wave, m1, x);
+                        sum = sr_seq_wave<SR_SEQ_RUN, false>(x, sum, 0.0f, &dummy);
+                    }
+                }
+                if (rem > 0 && wave >= 8 - rem) sum = __fadd_rn(sum, __fmul_rn(t.e(t.lg[n - 8 + wave]), m1));  // the overlapped last vector
+                if (ln == 0) sm.lane_sum[wave] = sum;
+                __syncthreads();
+                const float* const l = sm.lane_sum;
+                m2 = spec_m(__fadd_rn(__fadd_rn(__fadd_rn(l[0], l[1]), __fadd_rn(l[2], l[3])), __fadd_rn(__fadd_rn(l[4], l[5]), __fadd_rn(l[6], l[7]))));
+            }
+            if (tid == 0) {
+                st->mul1 = m1;
+                st->mul2 = m2;
+                if (pos != last) {  // (an open test: with the factors it is exact)
+                    const int tok = s.draft_tokens[(size_t)row * L + pos];
+                    const float px = __fmul_rn(__fmul_rn(t.e(t.lg[tok]), m1), m2);
+                    if (s.uniforms[(size_t)row * s.uniforms_per_row + pos] < (double)spec_accept(px, s.draft_probs[((size_t)row * L + pos) * n + tok]))
+                        __hip_atomic_fetch_or(said + kSpecAccepted, 1ull << pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+        }
+        __syncthreads();
+    }
+}
+
 // ---- speculative verification of rows under the ratio test (StepSampled, SpeculativeDecoder.cs:530-559) --------------------
 // The accept loop of such a row needs one element of p and of q per position, and the draw behind it one row of terms: max(0,
 // fl(fl(p m1) m2) - q) of the first rejected position, or the scaled target row fl(fl(p m1) m2) of the bonus position when every
@@ -4750,7 +5207,7 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_factor(SrFullArgs a, SrSpecA
 // The wait is bounded: a workgroup whose wait runs out marks the row and counts itself in, and whoever comes last adds all of the
 // row's terms by its own.
 // reject[row] = kSpecDone, or -1: the row is k_spec_verify's (other accept rules, a bonus token of a greedy row).
-constexpr int kSpecT = 512, kSpecDone = -2;
+constexpr int kSpecT = 512;
 constexpr int kSpecWaves = kSpecT / SR_WAVE;
 // the exact running sum (or the search) over all segments from their terms, by one wave; the slow way of the rare cases
 template <bool kSearch>
@@ -4771,7 +5228,8 @@ __device__ __forceinline__ float spec_sum_alone(const SpecTerms& t, int nseg, fl
     }
     return s;
 }
-template <bool kLater>  // k_spec_factor was launched in front
+// kFrom 1: k_spec_factor was launched in front   2: k_spec_open, which has found the position
+template <int kFrom>
 __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
 {
     __shared__ float4 turn_all[kSpecWaves][SR_WAVE * 5];
@@ -4788,8 +5246,17 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
         return;
     }
     const double* const u = a.uniforms + (size_t)row * a.uniforms_per_row;
-    if (wave == 0) {
-        if (kLater) spec_table(tab);
+    if (kFrom == 2) {
+        if (tid == 0) {
+            const unsigned long long picked = sync[kSpecPicked] & ~sync[kSpecAccepted], last = sync[kSpecLast];
+            said[0] = picked != 0ull ? (int)__ffsll((long long)picked) - 1 : (int)(uint32_t)last;
+            said[1] = picked == 0ull ? 2 : said[0] < L ? 0 : 1;
+        } else if (tid == SR_WAVE) {
+            const unsigned long long was = __hip_atomic_fetch_max(sync, (unsigned long long)a.seq << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("" : : "v"(was) : "memory");
+        }
+    } else if (wave == 0) {
+        if (kFrom == 1) spec_table(tab);
         // the first position that is not accepted: kind 0 rejected, 1 none (position L), 2 an id outside the vocabulary, which
         // ends the row without a correction
         int pos = L, kind = 1;
@@ -4801,7 +5268,7 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
                 bad = (uint32_t)tok >= (uint32_t)n;
                 if (!bad) {
                     const SrFullState* sl = a.state + (size_t)row * (L + 1) + i;
-                    const float px = __fmul_rn(__fmul_rn(kLater ? spec_e<false>(a, rd, (size_t)row * (L + 1) + i, tok, tab)
+                    const float px = __fmul_rn(__fmul_rn(kFrom == 1 ? spec_e<false>(a, rd, (size_t)row * (L + 1) + i, tok, tab)
                                                             : a.p_all[((size_t)row * (L + 1) + i) * (size_t)a.p_stride + tok], sl->mul1), sl->mul2);
                     const float qx = a.draft_probs[((size_t)row * L + i) * n + tok];
                     const float acc = spec_accept(px, qx);
@@ -4906,22 +5373,27 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
         bc = ((uint32_t)(was >> 16) & 0xffffu) + 1u == gridDim.x ? (sr_load_agent(sync + 1) == (unsigned long long)a.seq ? 2u : 1u) : 0u;
     }
     __syncthreads();
-    if (bc == 0u || wave != 0) return;
+    if (bc == 0u) return;
     const bool alone = bc == 2u;
+    const bool staged = stage_records<kSpecT>(funcs, nseg, &turn_all[0][0], (int)sizeof(turn_all));
+    if (wave != 0) return;
     const double ud = u[kind == 0 ? pos + 1 : L];
     const float r = __double2float_rn(ud);
     auto load = [&](int sg, float (&xs)[SR_SEQ_RUN]) __attribute__((always_inline)) { t.run(sg, xs); };
+    const SeqSegFunc* const near = (const SeqSegFunc*)&turn_all[0][0];
     int found;
     if (kind == 1) {
         // SampleFromDistribution (Sampler.cs:564-576) over the bonus position
         if (alone) spec_sum_alone<true>(t, nseg, r, &found, nullptr);
+        else if (staged) seg_walk_from<true>(load, nseg, near, 0.0f, r, &found, nullptr);
         else seg_walk_from<true, true>(load, nseg, funcs, 0.0f, r, &found, nullptr);
         results(found >= 0 ? found : n - 1);
         return;
     }
     // ResampleResidual (Sampler.cs:587-618)
     int none;
-    const float sum = alone ? spec_sum_alone<false>(t, nseg, 0.0f, &none, states) : seg_walk_from<false, true>(load, nseg, funcs, 0.0f, 0.0f, &none, states);
+    const float sum = alone ? spec_sum_alone<false>(t, nseg, 0.0f, &none, states) : staged ? seg_walk_from<false>(load, nseg, near, 0.0f, 0.0f, &none, states)
+                            : seg_walk_from<false, true>(load, nseg, funcs, 0.0f, 0.0f, &none, states);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -5272,11 +5744,16 @@ hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, hipStream_t st)
         const dim3 grid((unsigned)((seg_count_of(b.vocab) + kSpecWaves - 1) / kSpecWaves), rows);
         static_assert(kSpecWaves == SR_SEQ_CHAINS && kSpecT == kPrepT, "the same blocks of a row");
         b.open_factors = nullptr;
-        if (a.open_factors) {
+        if (a.all_open) {
+            hipLaunchKernelGGL(k_spec_units, dim3((unsigned)((b.n_units + 3) / 4), rows * (b.n_draft + 1)), dim3(256), 0, st, *a.open_factors, b);
+            if (b.n_units <= kUnitsFew * SR_WAVE) hipLaunchKernelGGL(k_spec_open<kUnitsFew>, grid, dim3(kPrepT), 0, st, *a.open_factors, b);
+            else hipLaunchKernelGGL(k_spec_open<kUnitsMost>, grid, dim3(kPrepT), 0, st, *a.open_factors, b);
+            hipLaunchKernelGGL(k_spec_rows<2>, grid, dim3(kSpecT), 0, st, b);
+        } else if (a.open_factors) {
             hipLaunchKernelGGL(k_spec_factor, grid, dim3(kPrepT), 0, st, *a.open_factors, b);
-            hipLaunchKernelGGL(k_spec_rows<true>, grid, dim3(kSpecT), 0, st, b);
+            hipLaunchKernelGGL(k_spec_rows<1>, grid, dim3(kSpecT), 0, st, b);
         } else {
-            hipLaunchKernelGGL(k_spec_rows<false>, grid, dim3(kSpecT), 0, st, b);
+            hipLaunchKernelGGL(k_spec_rows<0>, grid, dim3(kSpecT), 0, st, b);
         }
         if (!b.any_other) return hipGetLastError();
     } else {

@@ -11,6 +11,18 @@ namespace {
 // a row of the verifier whose drafts are accepted by the ratio test
 bool by_ratio(const SrRow& r) { return !(r.p_min > 0.0f && r.p_min < 1.0f) && !(r.flags & SR_ROW_DRAFT_FROM_LOOKUP); }
 
+// the number of the next launch (full_state is there)
+hipError_t next_launch(sr_ctx* ctx)
+{
+    if (++ctx->full_seq != 0u) return hipSuccess;
+    // the numbers have gone round: nothing of an earlier launch may look like this one's
+    hipError_t e = hipMemsetAsync(ctx->full_state.p, 0, ctx->full_state.cap, ctx->stream);
+    if (e == hipSuccess && ctx->full_row_sync.p) e = hipMemsetAsync(ctx->full_row_sync.p, 0, ctx->full_row_sync.cap, ctx->stream);
+    if (e == hipSuccess && ctx->spec_sync.p) e = hipMemsetAsync(ctx->spec_sync.p, 0, ctx->spec_sync.cap, ctx->stream);
+    ctx->full_seq = 1u;
+    return e;
+}
+
 // Runs the full-vocabulary pipeline for the rows in `list` (device array of n_rows row indices).
 //   mode 0: work rows live in ctx scratch, tokens out.   mode 1/2: work rows ARE the caller's probs rows.
 int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows, bool any_top_p, const void* logits_dev,
@@ -108,12 +120,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     // otherwise left by each launch the way the next one expects them)
     SR_HIP(ctx, ctx->full_state.reserve((size_t)n_rows * sizeof(SrFullState), st, true));
     a.state = ctx->full_state.as<SrFullState>();
-    if (++ctx->full_seq == 0u) {  // the numbers have gone round: nothing of an earlier launch may look like this one's
-        SR_HIP(ctx, hipMemsetAsync(ctx->full_state.p, 0, ctx->full_state.cap, st));
-        if (ctx->full_row_sync.p) SR_HIP(ctx, hipMemsetAsync(ctx->full_row_sync.p, 0, ctx->full_row_sync.cap, st));
-        if (ctx->spec_sync.p) SR_HIP(ctx, hipMemsetAsync(ctx->spec_sync.p, 0, ctx->spec_sync.cap, st));
-        ctx->full_seq = 1u;
-    }
+    SR_HIP(ctx, next_launch(ctx));
     a.seq = ctx->full_seq;
     a.row_wait_limit = ctx->row_wait_limit;
     a.behind_wait_limit = ctx->behind_wait_limit;
@@ -536,10 +543,34 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     tmp.d_edits.p = b->d_edits.p;
     tmp.mask_stride = 0;
     const int32_t* list = nullptr;
-    int rc = identity_list(ctx, rows * P, &list);
     SrFullArgs full{};
     const bool in_one = n_draft > 0 && n_draft < 64 && draft_probs_dev && rows <= 65535;  // (k_spec_factor: a position a lane)
-    if (rc == SR_OK)
+    // rows that nothing touches, all of them: k_spec_units and k_spec_open (the lines: SR_OPEN_*)
+    const int nseg = (V + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
+    bool all_open = in_one && V >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX && (int64_t)rows * P <= 65535 &&
+                    (nseg < SR_OPEN_SHORT_SEGS || rows * P > ctx->cu_count || (nseg >= SR_OPEN_MIN_SEGS && (int64_t)rows * P * nseg >= SR_OPEN_SEGS));
+    for (int r = 0; r < rows && all_open; r++) {
+        const SrRow& d = b->h_rows[(size_t)r];
+        all_open = d.temperature > 0.0f && by_ratio(d) && !sr_row_cut(d) && !(d.top_k > 0 && d.top_k < V) && d.edit_cnt <= 0 && d.mask_row < 0;
+    }
+    int rc = all_open ? SR_OK : identity_list(ctx, rows * P, &list);
+    if (all_open) {
+        const size_t slots = (size_t)rows * (size_t)P;
+        const int half_blocks = (nseg + SR_HALF_BLOCK_SEGS - 1) / SR_HALF_BLOCK_SEGS;
+        full.seg_stride = nseg;
+        full.chain_blocks = (half_blocks + 1) / 2;
+        SR_HIP(ctx, ctx->full_state.reserve(slots * sizeof(SrFullState), st, true));
+        SR_HIP(ctx, ctx->full_row_sync.reserve(slots * SR_ROW_SYNC_STRIDE * sizeof(unsigned long long), st, true));
+        SR_HIP(ctx, ctx->full_seg_func.reserve(slots * (size_t)nseg * sizeof(SeqSegFunc), st));
+        SR_HIP(ctx, ctx->full_chain_func.reserve(slots * 8 * (size_t)full.chain_blocks * sizeof(SeqSegFunc), st));
+        SR_HIP(ctx, next_launch(ctx));
+        full.state = ctx->full_state.as<SrFullState>();
+        full.row_sync = ctx->full_row_sync.as<unsigned long long>();
+        full.seg_func = (SeqSegFunc*)ctx->full_seg_func.p;
+        full.chain_func = (SeqSegFunc*)ctx->full_chain_func.p;
+        full.seq = ctx->full_seq;
+        full.behind_wait_limit = ctx->behind_wait_limit;
+    } else if (rc == SR_OK)
         rc = run_full(ctx, &tmp, list, rows * P, any_top_p, target_logits_dev, SR_DTYPE_F32, V, 1, ctx->spec_probs.as<float>(), p_stride,
                       nullptr, nullptr, true, &b->h_rows, 0, in_one ? &full : nullptr);  // (the verifier applies the normalising factors of unfiltered rows itself)
     tmp.d_rows.p = nullptr;  // borrowed
@@ -581,7 +612,16 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
         const SrRow& d = b->h_rows[(size_t)r];
         if (!by_ratio(d) || !(d.temperature > 0.0f)) a.any_other = 1;
     }
-    if (full.factor_later) a.open_factors = &full;
+    if (full.factor_later || all_open) a.open_factors = &full;
+    if (all_open) {
+        a.all_open = 1;
+        a.n_units = (V + SR_UNIT_TERMS - 1) / SR_UNIT_TERMS;
+        const size_t units = (size_t)rows * (size_t)P * (size_t)a.n_units;
+        SR_HIP(ctx, ctx->spec_units.reserve(units * sizeof(float2), st));
+        SR_HIP(ctx, ctx->spec_unit_chains.reserve(units * 8 * sizeof(float), st));
+        a.units = (float2*)ctx->spec_units.p;
+        a.unit_chains = ctx->spec_unit_chains.as<float>();
+    }
     SR_HIP(ctx, sr_launch_spec_verify(a, rows, st));
     return SR_OK;
 }

@@ -270,6 +270,11 @@ struct SrSpecArgs {
     int32_t seg_stride;
     unsigned long long* sync;    // [row * SR_ROW_SYNC_STRIDE]: as SrFullArgs::row_sync, and behind it the last launch in which a wait ran out
     uint32_t seq, wait_limit;
+    // launches of which every row is one that nothing touches, under the ratio test (k_spec_units, k_spec_open):
+    float2* units;               // [rows][n_draft + 1][n_units]: every unit's largest scaled logit (NaN: it holds one) and about its sum of exp(x - that)
+    float* unit_chains;          // ... [8]: every lane accumulator's part of the sum
+    int32_t n_units;
+    int32_t all_open;            // the launch is one of these: units are set, open_factors holds what k_spec_open needs
     const SrFullArgs* open_factors;  // on the host: the launch that left factors open (SrFullArgs::factor_later), or null; n_draft < 64
     int32_t any_other;           // some row is not under the ratio test, or greedy: k_spec_verify follows
     // ... and of more:

@@ -1085,3 +1085,46 @@ def test_more_rows_than_the_device_holds_at_a_time(ctx, V, rows):
             t, d = orc.sample_with_distribution(logits[r], to_oracle(params[r]), orc.Rng(replay=[u[r]]))
             assert tokens[r] == t, r
             assert np.array_equal(probs[r].view(np.uint32), d.view(np.uint32)), r
+
+
+# Launches of rows that nothing touches (one and a half blocks, a block and one entry, many rows, long ones, more units than two a lane),
+# with waits that end at once, and of every second poll
+@pytest.mark.parametrize("V, rows, L, polls", [(4_096, 5, 63, 1 << 15), (8_193, 7, 20, 0), (12_290, 9, 3, 1 << 15), (8_199, 3, 5, 0x80000002), (20_003, 66, 3, 1 << 15),
+                                               (70_001, 7, 5, 1 << 15), (70_001, 7, 5, 0), (262_145, 2, 2, 1 << 15), (300_001, 2, 2, 0)])
+def test_rows_that_nothing_touches_are_verified_without_sums_of_the_other_positions(ctx, V, rows, L, polls):
+    """Accept tests that come out the same whatever the sums are, and ones that hang on the last digits (uniforms on the ratio p / q,
+    and one step of a double below it), several to a row; a draft that q gives nothing, one of no probability; ids outside the
+    vocabulary; rows with a NaN, with nothing above -inf and with +inf; everything accepted, so that the bonus position is drawn."""
+    rng = np.random.default_rng(V + L + rows)
+    params = [SamplingParams(Temperature=1.0 if r % 2 else 0.6 + 0.03 * (r % 9)) for r in range(rows)]
+    base = synthetic.zipf_head_logits(rng, rows * L, V).reshape(rows, L, V)
+    t = np.concatenate([base + rng.normal(0, 0.2, (rows, 1, V)).astype(np.float32), synthetic.zipf_head_logits(rng, rows, V).reshape(rows, 1, V)], axis=1)
+    q = np.exp(base - base.max(axis=2, keepdims=True))
+    q /= q.sum(axis=2, keepdims=True)
+    k = rng.integers(0, 20, (rows, L))
+    k = np.take_along_axis(np.argpartition(-base, 20, axis=2), k[:, :, None], axis=2)[:, :, 0].astype(np.int32)
+    t[0, 0, k[0, 0]] = -200.0  # expf leaves nothing of it
+    q[1, L // 2, k[1, L // 2]] = 0.0
+    if rows > 2:
+        t[2, L - 1, 5] = np.nan
+        t[min(3, rows - 1), L, :] = -np.inf
+        t[rows - 1, 0, 77] = np.inf
+    u = rng.random((rows, L + 1))
+    for r in range(rows):
+        for i in range(L):
+            p = orc.build_filtered_distribution(t[r, i], to_oracle(params[r]))[k[r, i]]
+            qx = q[r, i, k[r, i]]
+            if not (qx > 0) or not (p > 0):
+                continue
+            ratio = np.float64(np.minimum(np.float32(1), p / qx))
+            u[r, i] = [np.nextafter(ratio, 0.0), ratio * 0.5, ratio * (1 - 1e-5), ratio * 0.9][(r + i) % 4]
+        if r % 3 == 1:
+            u[r, int(rng.integers(0, L))] = 0.9999999
+        if r % 5 == 4:
+            k[r, L - 1] = V + 3
+    try:
+        ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, polls))
+        for _ in range(2):
+            _check_spec(ctx, t, q, k, params, u)
+    finally:
+        ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
