@@ -2,7 +2,7 @@
 // the reference's llm_argmax_rows (CudaTextKernels.cs:465-479).  Lowest index wins on equal values; a NaN
 // element wins outright (first NaN), as TensorPrimitives.IndexOfMax documents.
 //
-// One launch, grid = rows x chunks.  A workgroup streams its chunk with 16-byte non-temporal loads (eight in
+// One launch, grid = rows x chunks.  A workgroup streams its chunk with 16-byte loads (up to eight in
 // flight per thread), reduces it to a packed (key << 32 | ~index) and, when the row has more than one chunk,
 // folds that into the row's slot with a 64-bit atomic max and counts itself in; the workgroup that counts in
 // last writes the row's result and puts slot and counter back to zero, so the scratch of one launch is ready
@@ -22,7 +22,7 @@ static __device__ __align__(256) unsigned long long scratch[SR_ARGMAX_STATIC_ROW
 
 namespace {
 constexpr int kThreads = 256;
-constexpr int kUnroll = 8;
+constexpr int kUnroll = 4;
 
 typedef uint32_t __attribute__((ext_vector_type(4))) u32x4;
 
@@ -41,34 +41,64 @@ template <int ES> __device__ __forceinline__ float load_elem(const char* p, int6
     return sr_bf16_to_f32(((const uint16_t*)p)[i]);
 }
 
-// A thread's best element so far: key (NaN above everything) and index.  A thread meets its elements in ascending
-// index order, so "strictly larger" keeps the first of equal keys.
-struct Best {
-    uint32_t key, idx;
-};
-__device__ __forceinline__ void fold(Best& b, float v, uint32_t i)
+// An element's order as a signed whole number, the same way back: the bits of a negative number turned round.  +0 is just above -0
+// (sr_okey makes them the same), a positive NaN above +inf, a negative one below -inf.
+__device__ __forceinline__ uint32_t turned(uint32_t x) { return x ^ ((uint32_t)((int)x >> 31) & 0x7fffffffu); }
+typedef short __attribute__((ext_vector_type(2))) i16x2;
+__device__ __forceinline__ i16x2 as_i16x2(uint32_t x) { return __builtin_bit_cast(i16x2, x); }
+__device__ __forceinline__ i16x2 turned2(uint32_t x)  // two bf16 elements at once
 {
-    const uint32_t k = (v != v) ? 0xffffffffu : sr_okey(v);
-    const bool up = k > b.key;
-    b.idx = up ? i : b.idx;
-    b.key = up ? k : b.key;
+    return as_i16x2(x ^ (__builtin_bit_cast(uint32_t, as_i16x2(x) >> (short)15) & 0x7fff7fffu));
 }
-
-template <int ES> __device__ __forceinline__ void fold_vec(Best& best, const u32x4 t, uint32_t first)
-{
+// What a tile of a thread's vectors holds: its largest and its smallest element in that order.
+template <int ES> struct Span;
+template <> struct Span<4> {
+    int hi, lo;
+    __device__ __forceinline__ void start(const u32x4& t) { hi = lo = (int)turned(t[0]); }
+    __device__ __forceinline__ void fold(const u32x4& t)
+    {
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
-        if (ES == 4) {
-            fold(best, sr_u2f(t[w]), first + w);
-        } else {
-            fold(best, sr_u2f(t[w] << 16), first + 2 * w);
-            fold(best, sr_u2f(t[w] & 0xffff0000u), first + 2 * w + 1);
+        for (int w = 0; w < 4; w++) {
+            const int k = (int)turned(t[w]);
+            hi = max(hi, k);
+            lo = min(lo, k);
         }
     }
+    __device__ __forceinline__ int largest() const { return hi; }
+    __device__ __forceinline__ bool nan() const { return hi > 0x7f800000 || lo < (int)0x807fffffu; }
+};
+template <> struct Span<2> {
+    i16x2 hi, lo;
+    __device__ __forceinline__ void start(const u32x4& t) { hi = lo = turned2(t[0]); }
+    __device__ __forceinline__ void fold(const u32x4& t)
+    {
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const i16x2 k = turned2(t[w]);
+            hi = __builtin_elementwise_max(hi, k);
+            lo = __builtin_elementwise_min(lo, k);
+        }
+    }
+    __device__ __forceinline__ int largest() const { return max((int)hi[0], (int)hi[1]); }
+    __device__ __forceinline__ bool nan() const { return largest() > 0x7f80 || min((int)lo[0], (int)lo[1]) < (int)(short)0x807f; }
+};
+// element e of a vector as the bits of an fp32 number
+template <int ES> __device__ __forceinline__ uint32_t bits_of(const u32x4& t, int e)
+{
+    if (ES == 4) return t[e];
+    return (e & 1) ? t[e >> 1] & 0xffff0000u : t[e >> 1] << 16;
 }
+__device__ __forceinline__ bool is_nan_bits(uint32_t x) { return (x & 0x7fffffffu) > 0x7f800000u; }
 
-// kVec: the rows start on 16-byte boundaries and chunk_len is a multiple of the elements of a vector
-template <int ES, bool kVec> __global__ __launch_bounds__(kThreads) void k_argmax_rows(SrArgmaxArgs a)
+// kAligned: the rows start on 16-byte boundaries.  What bounds it: memory, where there is enough of it; a launch over little waits for
+// its first vectors and for its chunks to come together.  Two tiles of four vectors a thread in turn, the loads of one under the
+// folding of the other, two and a half (bf16, in pairs) and four instructions an element; an element's index is looked for only
+// where a wave's tile holds more than its tiles before.  Against eight or nine instructions an element, key and index carried along, a
+// tile of eight at a time, and element by element in rows at odd addresses, whole calls in us: 128 rows of 151,936 bf16 24.4 -> 21.6, 256
+// 32.0 -> 28.0, 1 16.3 -> 14.5, 512 45.6 -> 39.5; 64 rows of 100,003 bf16 30 -> 18, 300 of 100,003 fp32 84 -> 34, 1,024 of 20,011 bf16 45 -> 26.
+// (Tiles of eight 27 at 128 rows, of six 26.7, of two and three as of four; three to six workgroups to a compute unit 24.6 - 25.4 where
+// two took 24.8.  With four instructions an element in the search for the index, in place of two, 24.8.)
+template <int ES, bool kAligned> __global__ __launch_bounds__(kThreads) void k_argmax_rows(SrArgmaxArgs a)
 {
     __shared__ unsigned long long s_best[kThreads / SR_WAVE];
     constexpr int EPV = 16 / ES;
@@ -77,40 +107,83 @@ template <int ES, bool kVec> __global__ __launch_bounds__(kThreads) void k_argma
     const int lo = c * a.chunk_len, hi = min(a.vocab, lo + a.chunk_len);
     const char* rowp = (const char*)a.logits + (size_t)row * (size_t)a.row_stride * ES;
     const int tid = (int)threadIdx.x;
-    Best tb;
-    tb.key = 0u;  // (no element has the key 0: an empty chunk leaves it)
-    tb.idx = 0u;
-    int scalar_from = lo;
-    if (kVec) {
-        const u32x4* vp = (const u32x4*)rowp;
-        const int v_lo = lo / EPV, v_hi = hi / EPV;  // whole vectors; only the row's last chunk can leave elements over
-        // Sets of kUnroll vectors per thread, all of a set's loads issued before the first is folded.  The chunk's last
-        // set is loaded whole too -- a vector past the chunk's end is the chunk's last one again and is not folded --
-        // rather than vector by vector, each of which would be a trip to memory of its own.
+    unsigned long long best = 0ull;  // of the wave: key << 32 | ~index (NaN above everything); 0: no element yet
+    const int v_lo = lo / EPV, v_hi = hi / EPV;  // whole vectors; only the row's last chunk can leave elements over
+    if (v_lo < v_hi) {
+        // (a vector past the chunk's end is the chunk's last one again)
         const int last = v_hi - 1;
-        for (int base = v_lo; base < v_hi; base += kUnroll * kThreads) {
-            const int i = base + tid;
-            u32x4 t[kUnroll];
-            if (base + kUnroll * kThreads <= v_hi) {
+        auto load = [&](int base, u32x4 (&t)[kUnroll]) __attribute__((always_inline)) {
 #pragma unroll
-                for (int j = 0; j < kUnroll; j++) t[j] = __builtin_nontemporal_load(vp + i + j * kThreads);
-#pragma unroll
-                for (int j = 0; j < kUnroll; j++) fold_vec<ES>(tb, t[j], (uint32_t)(i + j * kThreads) * EPV);
-            } else {
-#pragma unroll
-                for (int j = 0; j < kUnroll; j++) t[j] = __builtin_nontemporal_load(vp + min(i + j * kThreads, last));
-#pragma unroll
-                for (int j = 0; j < kUnroll; j++)
-                    if (i + j * kThreads < v_hi) fold_vec<ES>(tb, t[j], (uint32_t)(i + j * kThreads) * EPV);
+            for (int j = 0; j < kUnroll; j++) {
+                const char* const at = rowp + (size_t)min(base + tid + j * kThreads, last) * 16;
+                if (kAligned) {
+                    t[j] = __builtin_nontemporal_load((const u32x4*)at);
+                } else {
+                    const uint4 v = sr_load16<ES>(at);
+                    t[j] = u32x4{v.x, v.y, v.z, v.w};
+                }
             }
+        };
+        auto fold = [&](int base, const u32x4 (&t)[kUnroll]) __attribute__((always_inline)) {
+            Span<ES> s;
+            s.start(t[0]);
+#pragma unroll
+            for (int j = 0; j < kUnroll; j++) s.fold(t[j]);
+            const bool nan = __ballot(s.nan()) != 0ull;
+            const uint32_t k = sr_wave_max_u32((uint32_t)s.largest() ^ 0x80000000u) ^ 0x80000000u;
+            // the largest element's bits, and its key
+            const uint32_t bits = ES == 4 ? turned(k) : (k ^ ((uint32_t)((int)k >> 31) & 0x7fffu)) << 16;
+            const uint32_t key = nan ? 0xffffffffu : sr_okey(sr_u2f(bits));
+            if (key <= (uint32_t)(best >> 32)) return;  // (of equal ones the first stays: its index is lower)
+            // (from the last to the first: a comparison and a selection each)
+            int code = -1;
+            if (nan || (bits << 1) == 0u) {  // (a zero is as large with either sign)
+#pragma unroll
+                for (int j = kUnroll - 1; j >= 0; j--)
+#pragma unroll
+                    for (int e = EPV - 1; e >= 0; e--) {
+                        const uint32_t x = bits_of<ES>(t[j], e);
+                        code = (nan ? is_nan_bits(x) : (x << 1) == 0u) ? j * EPV + e : code;
+                    }
+            } else {
+                const uint32_t half = bits >> 16;
+#pragma unroll
+                for (int j = kUnroll - 1; j >= 0; j--)
+#pragma unroll
+                    for (int e = EPV - 1; e >= 0; e--) {
+                        const bool is = ES == 4 ? t[j][e] == bits : ((e & 1) ? t[j][e >> 1] >> 16 : t[j][e >> 1] & 0xffffu) == half;
+                        code = is ? j * EPV + e : code;
+                    }
+            }
+            uint32_t at = code < 0 ? 0xffffffffu : (uint32_t)min(base + tid + (code / EPV) * kThreads, last) * EPV + (uint32_t)(code % EPV);
+            at = ~sr_wave_max_u32(~at);
+            best = ((unsigned long long)key << 32) | (unsigned long long)(0xffffffffu - at);
+        };
+        constexpr int kStep = kUnroll * kThreads;
+        u32x4 t0[kUnroll], t1[kUnroll];
+        load(v_lo, t0);
+        for (int base = v_lo; base < v_hi; base += 2 * kStep) {
+            if (base + kStep < v_hi) load(base + kStep, t1);
+            fold(base, t0);
+            if (base + 2 * kStep < v_hi) load(base + 2 * kStep, t0);
+            if (base + kStep < v_hi) fold(base + kStep, t1);
         }
-        scalar_from = max(lo, v_hi * EPV);
     }
-    for (int i = scalar_from + tid; i < hi; i += kThreads) fold(tb, load_elem<ES>(rowp, i), (uint32_t)i);
+    {
+        // the elements behind the row's last whole vector
+        const int i = max(lo, v_hi * EPV) + tid;
+        unsigned long long own = 0ull;
+        if (i < hi) {
+            const float v = load_elem<ES>(rowp, i);
+            own = ((unsigned long long)(v != v ? 0xffffffffu : sr_okey(v)) << 32) | (unsigned long long)(0xffffffffu - (uint32_t)i);
+        }
+        if (max(lo, v_hi * EPV) < hi) {  // (fewer than a vector's: one each)
+            own = sr_wave_max_u64(own);
+            best = own > best ? own : best;
+        }
+    }
 
     // (key << 32 | ~index): the largest key wins, among equal keys the lowest index
-    unsigned long long best = tb.key ? ((unsigned long long)tb.key << 32) | (unsigned long long)(0xffffffffu - tb.idx) : 0ull;
-    best = sr_wave_max_u64(best);
     if (sr_lane() == 0) s_best[sr_wave_id()] = best;
     __syncthreads();
     if (tid != 0) return;
@@ -128,7 +201,9 @@ template <int ES, bool kVec> __global__ __launch_bounds__(kThreads) void k_argma
         __hip_atomic_store(&a.done[row], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     const int idx = best ? (int)(0xffffffffu - (uint32_t)(best & 0xffffffffull)) : 0;  // empty row -> 0
-    const float val = a.vocab > 0 ? load_elem<ES>(rowp, idx) : 0.0f;  // the original bits, not a decode
+    // the original bits: the key's, the same way back; a NaN's and a zero's are fetched (a trip to memory of its own)
+    const uint32_t key = (uint32_t)(best >> 32);
+    const float val = best == 0ull ? 0.0f : key == 0xffffffffu || key == 0x80000000u ? load_elem<ES>(rowp, idx) : sr_okey_inv(key);
     if (a.host) {
         // The host goes on when it sees its word, in front of this kernel's end: what the device arrays get is written through
         // to memory, not left in this die's L2 for the kernel's end to write back, and waited for, before the word goes out.
@@ -160,7 +235,7 @@ void sr_argmax_plan(SrArgmaxArgs& a, int cu_count)
 {
     const int es = a.dtype == 1 ? 2 : 4, epv = 16 / es;
     a.vec = ((uintptr_t)a.logits % 16 == 0 && ((size_t)a.row_stride * es) % 16 == 0) ? 1 : 0;
-    // enough workgroups for two per compute unit (64 KB of loads in flight on each: what the memory's latency takes at
+    // enough workgroups for two per compute unit (64 KB of loads in flight on each, two tiles a thread: what the memory's latency takes at
     // the machine's rate; eight per compute unit, with their dispatch and their atomics, were 5 us slower on 256 rows of
     // 151,936), none with less than one unrolled pass of work
     const int per_pass = kThreads * kUnroll * epv;
