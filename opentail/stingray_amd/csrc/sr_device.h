@@ -151,6 +151,12 @@ template <int kAlign> __device__ __forceinline__ uint4 sr_load16(const void* p)
     const SrPacked16<kAlign> v = *(const SrPacked16<kAlign>*)p;
     return make_uint4(v.x, v.y, v.z, v.w);
 }
+template <int kAlign> struct __attribute__((packed, aligned(kAlign))) SrPacked8 { uint32_t x, y; };
+template <int kAlign> __device__ __forceinline__ uint2 sr_load8(const void* p)
+{
+    const SrPacked8<kAlign> v = *(const SrPacked8<kAlign>*)p;
+    return make_uint2(v.x, v.y);
+}
 __device__ __forceinline__ float4 sr_load_f4(const float* p)
 {
     const uint4 v = sr_load16<4>(p);

@@ -1371,19 +1371,26 @@ __device__ __forceinline__ SegSource<ES> seg_source(const SrRow& rd, const SrFul
     }
     return src;
 }
-// The wave's segment as it is loaded: 16-byte vectors, lane l the vectors l, 64 + l, ... of the segment, so that every
-// load instruction of the wave covers consecutive memory.  x[k E + q] is element (k 64 + l) E + q of the segment
-// (E elements per vector: 4 for fp32 logits, 8 for bf16); -inf past the row's end.
-template <int ES>
+// The wave's segment as it is loaded: vectors of E elements, lane l the vectors l, 64 + l, ... of the segment, so that every
+// load instruction of the wave covers consecutive memory.  x[E k + q] is element (k 64 + l) E + q of the segment; -inf past the
+// row's end.  fp32: 4.  bf16: 8, or 4 in launches that write e through to memory as they go (out_now), where with eight a store
+// instruction leaves every second 16 bytes of its lines to the next one: 64 penalised rows of 151,936 48.3 -> 41.8 us, of 65,537 34.3 -> 30.7, 24 of
+// 262,144 42.9 -> 38.6; launches whose e goes to the caches lose 0.5 - 2 % by the narrower loads (32 ragged rows of 100,003 51.9 -> 52.3).
+template <int ES, int E> __device__ __forceinline__ uint4 seg_load_vec(const char* p)  // the vector's bits
+{
+    if (ES * E == 16) return sr_load16<ES>(p);
+    const uint2 v = sr_load8<ES>(p);
+    return make_uint4(v.x, v.y, 0u, 0u);
+}
+template <int E>
 __device__ __forceinline__ int seg_elem(int seg, int lane, int slot_kq)
 {
-    constexpr int E = 16 / ES;
     return seg * SR_SEG_TERMS + ((slot_kq / E) * SR_WAVE + lane) * E + (slot_kq % E);
 }
-template <int ES>
+template <int ES, int E>
 __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int seg, int lane, int n, float (&x)[SR_SEQ_RUN])
 {
-    constexpr int E = 16 / ES, K = SR_SEG_TERMS / (SR_WAVE * E);
+    constexpr int K = SR_SEG_TERMS / (SR_WAVE * E);
     static_assert(K * E == SR_SEQ_RUN, "sixteen elements per lane");
     if ((seg + 1) * SR_SEG_TERMS <= n) {
         // a whole segment (all but a row's last): every load is issued before anything is done with one of them
@@ -1393,7 +1400,7 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
 #pragma unroll
             for (int k = 0; k < K; k++) {
                 const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * E;
-                raw[k] = sr_load16<ES>(src.rowp + (size_t)i0 * ES);
+                raw[k] = seg_load_vec<ES, E>(src.rowp + (size_t)i0 * ES);
             }
             if (src.mrow) {
 #pragma unroll
@@ -1410,9 +1417,9 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
                 } else {
                     const uint32_t r[4] = {raw[k].x, raw[k].y, raw[k].z, raw[k].w};
 #pragma unroll
-                    for (int q = 0; q < 4; q++) {
-                        xv[(2 * q) % E] = sr_u2f(r[q] << 16);
-                        xv[(2 * q + 1) % E] = sr_u2f(r[q] & 0xffff0000u);
+                    for (int q = 0; q < E / 2; q++) {
+                        xv[2 * q] = sr_u2f(r[q] << 16);
+                        xv[2 * q + 1] = sr_u2f(r[q] & 0xffff0000u);
                     }
                 }
             }
@@ -1468,15 +1475,15 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
         uint32_t keep = (1u << E) - 1u;
         if (src.mrow) keep = src.mrow[i0 >> 5] >> (i0 & 31);
         if (whole) {
-            const uint4 v = sr_load16<ES>(src.rowp + (size_t)i0 * ES);
+            const uint4 v = seg_load_vec<ES, E>(src.rowp + (size_t)i0 * ES);
             if (ES == 4) {
                 xv[0] = sr_u2f(v.x); xv[1] = sr_u2f(v.y); xv[2] = sr_u2f(v.z); xv[3] = sr_u2f(v.w);
             } else {
                 const uint32_t r[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    xv[(2 * q) % E] = sr_u2f(r[q] << 16);
-                    xv[(2 * q + 1) % E] = sr_u2f(r[q] & 0xffff0000u);
+                for (int q = 0; q < E / 2; q++) {
+                    xv[2 * q] = sr_u2f(r[q] << 16);
+                    xv[2 * q + 1] = sr_u2f(r[q] & 0xffff0000u);
                 }
             }
         } else {
@@ -1496,11 +1503,10 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
 // logit, then the temperature (Sampler.cs:51-58, :367-419).  entry(i, id, e) names the i-th candidate of `count`: an id and
 // its place in the row's edit list; 64 candidates at a time, a lane each, then the owners of the hits take them one
 // by one.
-template <int ES, typename Entry>
+template <int ES, int E, typename Entry>
 __device__ __forceinline__ void seg_apply_edits(const SrFullArgs& a, const SrRow& rd, const SegSource<ES>& src, int seg, int lane,
                                                 int count, Entry entry, float (&x)[SR_SEQ_RUN])
 {
-    constexpr int E = 16 / ES;
     const SrEdit* ed = a.edits + rd.edit_off;
     const bool pen = (rd.flags & SR_ROWFLAG_HAS_PENALTY) != 0u;
     const int lo = seg * SR_SEG_TERMS;
@@ -1612,7 +1618,7 @@ __device__ __forceinline__ uint32_t min_p_list_from(const SrRow& rd)
 // A greedy row that rides along (SrFullArgs::n_greedy): the largest of its masked logits, the first by index among equals, NaN left
 // out -- what the selection kernel finds for such a row.  The row's word for it is zero between launches: whoever counts in last
 // takes the result and puts the zero back.
-template <int ES, int kW, int kS>
+template <int ES, int kW, int kS, int E>
 __device__ __forceinline__ void seg_greedy(const SrFullArgs& a, const SrRow& rd, int slot, int row, unsigned long long* of_wave)
 {
     const int lane = sr_lane(), wave = sr_wave_id(), n = a.vocab, nseg = seg_count(n);
@@ -1626,7 +1632,7 @@ __device__ __forceinline__ void seg_greedy(const SrFullArgs& a, const SrRow& rd,
     float t[kS][SR_SEQ_RUN];
 #pragma unroll
     for (int s = 0; s < kS; s++)
-        if (seg0 + s * kW < nseg) seg_load_logits<ES>(src, seg0 + s * kW, lane, n, t[s]);
+        if (seg0 + s * kW < nseg) seg_load_logits<ES, E>(src, seg0 + s * kW, lane, n, t[s]);
     unsigned long long best = 0ull;  // ordered key << 32 | ~index; 0: nothing above -inf
 #pragma unroll
     for (int s = 0; s < kS; s++) {
@@ -1641,7 +1647,7 @@ __device__ __forceinline__ void seg_greedy(const SrFullArgs& a, const SrRow& rd,
         int at = 0x7fffffff;
 #pragma unroll
         for (int j = SR_SEQ_RUN - 1; j >= 0; j--)
-            if (t[s][j] == mk) at = min(at, seg_elem<ES>(seg, lane, j));
+            if (t[s][j] == mk) at = min(at, seg_elem<E>(seg, lane, j));
         at = sr_wave_min_i32(at);
         const unsigned long long found = ((unsigned long long)k << 32) | (unsigned long long)(0xffffffffu - (uint32_t)at);
         best = found > best ? found : best;
@@ -1667,11 +1673,11 @@ __device__ __forceinline__ void seg_greedy(const SrFullArgs& a, const SrRow& rd,
 }
 
 // kLater: a verifier's launch with factor_later (144 rows of 131,072, which do without, were 2 us slower with the test in it)
-template <int ES, int kW, int kS, bool kLater = false>
+template <int ES, int kW, int kS, bool kLater = false, int E = 16 / ES>
 __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_seg(SrFullArgs a)
 {
     constexpr int kThreads = kW * SR_WAVE;
-    constexpr int E = 16 / ES, K = SR_SEG_TERMS / (SR_WAVE * E);
+    constexpr int K = SR_SEG_TERMS / (SR_WAVE * E);
     static_assert(kW == SR_HALF_BLOCK_SEGS, "a workgroup's segments are whole half blocks");
     const int slot = blockIdx.y, lane = sr_lane(), wave = sr_wave_id();
     const int row = a.row_list[slot];
@@ -1693,7 +1699,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     __shared__ unsigned long long hits[kHitCap];
     __shared__ uint32_t n_hits;
     if (rd.temperature <= 0.0f) {  // greedy rows keep their logits where a distribution is asked for
-        if (kS != 4 && a.mode == 0) seg_greedy<ES, kW, kS>(a, rd, slot, row, hits);
+        if (kS != 4 && a.mode == 0) seg_greedy<ES, kW, kS, E>(a, rd, slot, row, hits);
         return;
     }
     const int n = a.vocab, nseg = seg_count(n);
@@ -1744,7 +1750,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     float t[kS][SR_SEQ_RUN];
 #pragma unroll
     for (int s = 0; s < kS; s++)
-        if (seg0 + s * kW < nseg) seg_load_logits<ES>(src, seg0 + s * kW, lane, n, t[s]);
+        if (seg0 + s * kW < nseg) seg_load_logits<ES, E>(src, seg0 + s * kW, lane, n, t[s]);
     if (edits) {
         const int lo = (int)blockIdx.x * (kW * kS) * SR_SEG_TERMS, hi = lo + kW * kS * SR_SEG_TERMS;
 #pragma unroll
@@ -1762,7 +1768,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
 #pragma unroll
         for (int s = 0; s < kS; s++)
             if (seg0 + s * kW < nseg)
-                seg_apply_edits<ES>(a, rd, src, seg0 + s * kW, lane, from_hits ? (int)n_hits : rd.edit_cnt, [&](int i, int& id, int& e) {
+                seg_apply_edits<ES, E>(a, rd, src, seg0 + s * kW, lane, from_hits ? (int)n_hits : rd.edit_cnt, [&](int i, int& id, int& e) {
                     if (from_hits) {
                         const unsigned long long h = hits[i];
                         id = (int)(h >> 32);
@@ -1835,7 +1841,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
             for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = sr_expf_neg(__fsub_rn(t[s][j], m), tab);
         } else {
 #pragma unroll
-            for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = seg_elem<ES>(seg, lane, j) < n ? sr_expf_neg(__fsub_rn(t[s][j], m), tab) : 0.0f;
+            for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = seg_elem<E>(seg, lane, j) < n ? sr_expf_neg(__fsub_rn(t[s][j], m), tab) : 0.0f;
         }
 #pragma unroll
         for (int k2 = 0; k2 < K; k2++) {
@@ -5637,7 +5643,9 @@ hipError_t sr_launch_full_prep(const SrFullArgs& a, int n_rows, hipStream_t st)
         const int per_group = 4 * (four ? 4 : two ? 2 : 1);
         dim3 fgrid((unsigned)((nseg + per_group - 1) / per_group), n_rows + a.n_greedy);
         if (a.dtype == 1) {
-            if (two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2>), fgrid, dim3(256), 0, st, a);
+            if (!a.prepared && two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2, false, 4>), fgrid, dim3(256), 0, st, a);
+            else if (!a.prepared) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 1, false, 4>), fgrid, dim3(256), 0, st, a);
+            else if (two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2>), fgrid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 1>), fgrid, dim3(256), 0, st, a);
         } else {
             if (a.factor_later) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 4, true>), fgrid, dim3(256), 0, st, a);

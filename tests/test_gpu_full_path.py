@@ -1128,3 +1128,26 @@ def test_rows_that_nothing_touches_are_verified_without_sums_of_the_other_positi
             _check_spec(ctx, t, q, k, params, u)
     finally:
         ctx._check(hooks_lib().sr_debug_set_row_wait_limit(ctx.h, 1 << 15))
+
+
+# bf16 rows whose e goes out while the pass goes on, in vectors of four: the end of a segment and of a row inside one, rows at odd
+# addresses, bias and penalties on ids of every place of a vector, one and two segments a wave
+@pytest.mark.parametrize("V, rows", [(4_096, 3), (4_099, 3), (8_197, 5), (20_002, 4), (49_151, 64), (100_003, 33)])
+def test_bf16_rows_cut_by_min_p_with_edits_at_every_place(ctx, V, rows):
+    import torch
+
+    rng = np.random.default_rng(V)
+    logits = synthetic.zipf_head_logits(rng, rows, V)
+    bits = synthetic.to_bf16_bits(logits)
+    logits = synthetic.bf16_bits_to_f32(bits)
+    params = []
+    for r in range(rows):
+        top = np.argsort(-logits[r])[:24]
+        params.append(SamplingParams(Temperature=0.6 + 0.02 * (r % 20), MinP=float(rng.choice([0.002, 0.05, 0.3])), TopP=float(rng.choice([1.0, 0.9])),
+                                     FrequencyPenalty=0.4, PresencePenalty=0.2, RepetitionPenalty=1.1,
+                                     PreviousTokens=np.concatenate([top[::2], rng.integers(0, V, 300), np.arange(V - 9, V)]).tolist(),
+                                     LogitBias={int(top[1]): 1.5, int(V - 1): 6.0, int(V // 2): 5.0} if r % 3 == 0 else None))
+    u = rng.random(rows)
+    dev = torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16)
+    got = ctx.sample_batch(dev, params, u)
+    assert np.array_equal(got, oracle_tokens(logits, params, u)), (V, rows)
