@@ -1672,8 +1672,9 @@ __device__ __forceinline__ void seg_greedy(const SrFullArgs& a, const SrRow& rd,
     }
 }
 
+// kLists: the launch may have rows that list their candidates, and greedy ones (not the verifier's).
 // kLater: a verifier's launch with factor_later (144 rows of 131,072, which do without, were 2 us slower with the test in it)
-template <int ES, int kW, int kS, bool kLater = false, int E = 16 / ES>
+template <int ES, int kW, int kS, bool kLater = false, int E = 16 / ES, bool kLists = kS != 4>
 __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_seg(SrFullArgs a)
 {
     constexpr int kThreads = kW * SR_WAVE;
@@ -1699,7 +1700,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     __shared__ unsigned long long hits[kHitCap];
     __shared__ uint32_t n_hits;
     if (rd.temperature <= 0.0f) {  // greedy rows keep their logits where a distribution is asked for
-        if (kS != 4 && a.mode == 0) seg_greedy<ES, kW, kS, E>(a, rd, slot, row, hits);
+        if (kLists && a.mode == 0) seg_greedy<ES, kW, kS, E>(a, rd, slot, row, hits);
         return;
     }
     const int n = a.vocab, nseg = seg_count(n);
@@ -1711,8 +1712,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     if (threadIdx.x < 32) tab[threadIdx.x] = sr_exp2f_tab[threadIdx.x];
     const SegSource<ES> src = seg_source<ES>(rd, a, slot, row);
     float* const w = row_e(a, slot);
-    // (four segments a wave: the verifier's launches, which list nothing)
-    const bool plain = a.prepared && row_is_plain(rd, a), listed = kS != 4 && row_is_listed(rd, a);
+    const bool plain = a.prepared && row_is_plain(rd, a), listed = kLists && row_is_listed(rd, a);
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
     const bool out_now = !a.prepared && ((uintptr_t)w & 15u) == 0u, open_e = kLater && row_e_open(rd, a);
     // (a row that min-p cuts as well lists everything down to its threshold: entries on it count for SR_OUT_AMBIGUOUS wherever
@@ -5640,15 +5640,24 @@ hipError_t sr_launch_full_prep(const SrFullArgs& a, int n_rows, hipStream_t st)
         // else in registers (144 rows of 262,144: 98 -> 92 us; 36 rows: 119.6 -> 121.6 a call).
         const long long segs = (long long)(a.n_sampled + a.n_greedy) * nseg;
         const bool four = a.factor_later || (a.lazy_scale && a.dtype != 1 && segs > 12288), two = segs > 3072;
-        const int per_group = 4 * (four ? 4 : two ? 2 : 1);
+        // ... and four where two make a little more workgroups than the device holds at six to a compute unit, and four fit at
+        // five: two and four, us, 64 rows of 262,144 fp32 67 and 58 (bf16 68 and 55; cut by nothing or by top-p 110 and 100), 64 of 200,003
+        // 57.5 and 54, 96 of 151,936 59 and 55.5, 128 64 and 62; that fit already, 64 of 151,936 42 and 50, 80 45 and 53; in several turns either
+        // way, 256 of 100,003 83 and 91; shorter rows, 128 of 100,003 54 both, 200 of 65,537 55 and 56.5.
+        const long long sampled = a.n_sampled + a.n_greedy;
+        const bool big = !a.lazy_scale && nseg >= 128 && sampled * ((nseg + 7) / 8) > 6 * a.cu_count && sampled * ((nseg + 15) / 16) <= 5 * a.cu_count;
+        const int per_group = 4 * (four || big ? 4 : two ? 2 : 1);
         dim3 fgrid((unsigned)((nseg + per_group - 1) / per_group), n_rows + a.n_greedy);
         if (a.dtype == 1) {
-            if (!a.prepared && two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2, false, 4>), fgrid, dim3(256), 0, st, a);
+            if (big && !a.prepared) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 4, false, 4, true>), fgrid, dim3(256), 0, st, a);
+            else if (big) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 4, false, 8, true>), fgrid, dim3(256), 0, st, a);
+            else if (!a.prepared && two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2, false, 4>), fgrid, dim3(256), 0, st, a);
             else if (!a.prepared) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 1, false, 4>), fgrid, dim3(256), 0, st, a);
             else if (two) hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 2>), fgrid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_full_softmax_seg<2, 4, 1>), fgrid, dim3(256), 0, st, a);
         } else {
             if (a.factor_later) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 4, true>), fgrid, dim3(256), 0, st, a);
+            else if (big) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 4, false, 4, true>), fgrid, dim3(256), 0, st, a);
             else if (four) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 4>), fgrid, dim3(256), 0, st, a);
             else if (two) hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 2>), fgrid, dim3(256), 0, st, a);
             else hipLaunchKernelGGL((k_full_softmax_seg<4, 4, 1>), fgrid, dim3(256), 0, st, a);

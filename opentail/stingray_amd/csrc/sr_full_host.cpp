@@ -44,6 +44,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
     a.mask = sr_batch_mask_ptr(b);
     a.mask_stride = sr_batch_mask_stride(b);
     a.mode = mode;
+    a.cu_count = ctx->cu_count;
     a.n_greedy = n_greedy;  // (a further n_greedy rows of the list: they need nothing of what follows but a meeting point)
     a.prof = ctx->prof;
     if (mode == 0) {

@@ -208,6 +208,7 @@ struct SrFullArgs {
     int32_t finish_most;           // members up to which k_full_row normalises and draws by itself
     uint32_t seq;                  // the launch's number (never 0): see SrFullState::maxkey
     int32_t n_greedy;              // greedy rows behind the others in row_list, whose token k_full_softmax_seg finds (mode 0)
+    int32_t cu_count;              // compute units of the device
     int32_t n_sampled;             // rows of the launch with a temperature above 0 (greedy rows leave the passes at once)
     int32_t any_edits;             // some row of the launch has edits for k_full_edits (else it is not launched)
     int32_t edits_in_pass;         // seg_func is set: sampled rows with up to SR_FULL_EDIT_VALUES edits keep no adjusted copy and

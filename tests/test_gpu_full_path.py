@@ -1151,3 +1151,39 @@ def test_bf16_rows_cut_by_min_p_with_edits_at_every_place(ctx, V, rows):
     dev = torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16)
     got = ctx.sample_batch(dev, params, u)
     assert np.array_equal(got, oracle_tokens(logits, params, u)), (V, rows)
+
+
+# Launches of a few more workgroups than the device holds with two segments a wave, which take four: penalties and bias, masks, greedy rows
+# that ride along, rows cut by top-p, by min-p and not at all
+@pytest.mark.parametrize("V, rows, bf16", [(131_073, 100, False), (200_003, 64, True), (262_144, 52, False)])
+def test_rows_of_launches_with_four_segments_a_wave(ctx, V, rows, bf16):
+    import torch
+
+    rng = np.random.default_rng(V)
+    logits = synthetic.zipf_head_logits(rng, rows, V)
+    if bf16:
+        bits = synthetic.to_bf16_bits(logits)
+        logits = synthetic.bf16_bits_to_f32(bits)
+        dev = torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16)
+    else:
+        dev = torch.from_numpy(logits).cuda()
+    kinds = [SamplingParams(), SamplingParams(Temperature=0.8, TopP=0.9), SamplingParams(Temperature=0.7, MinP=0.02, TopP=0.95), SamplingParams(Temperature=0.0),
+             SamplingParams(Temperature=1.2, TopP=0.97), SamplingParams(Temperature=0.9, MinP=0.001)]
+    for only in (range(6), [2], [1, 4]):
+        params = []
+        for r in range(rows):
+            p = kinds[list(only)[r % len(list(only))]]
+            p = SamplingParams(Temperature=p.Temperature, TopP=p.TopP, MinP=p.MinP)
+            if r % 4 == 2 and p.Temperature > 0:
+                p.PreviousTokens = rng.integers(0, V, 200).tolist() + np.argsort(-logits[r])[:5].tolist()
+                p.FrequencyPenalty, p.PresencePenalty = 0.5, 0.3
+            params.append(p)
+        allowed = np.ones((rows, V), dtype=bool)
+        active = np.zeros(rows, dtype=np.uint8)
+        for r in range(1, rows, 9):
+            allowed[r] = rng.random(V) < 0.2
+            active[r] = 1
+        mask = pack_allow_mask(allowed)
+        u = rng.random(rows)
+        got = ctx.sample_batch(dev, params, u, mask, active)
+        assert np.array_equal(got, oracle_tokens(logits, params, u, mask, active)), (V, rows, list(only))
