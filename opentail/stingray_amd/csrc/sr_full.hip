@@ -6,6 +6,8 @@
 // one pass of a 1024-thread workgroup over that row.  All running sums that the reference evaluates
 // left to right go through the exact evaluator in sr_seqsum.h, so probabilities, cut-offs and draws
 // carry the reference's bits.
+#include <algorithm>
+
 #include "sr_device.h"
 #include "sr_kernels.h"
 #include "sr_seqsum.h"
@@ -5640,12 +5642,16 @@ hipError_t sr_launch_full_prep(const SrFullArgs& a, int n_rows, hipStream_t st)
         // else in registers (144 rows of 262,144: 98 -> 92 us; 36 rows: 119.6 -> 121.6 a call).
         const long long segs = (long long)(a.n_sampled + a.n_greedy) * nseg;
         const bool four = a.factor_later || (a.lazy_scale && a.dtype != 1 && segs > 12288), two = segs > 3072;
-        // ... and four where two make a little more workgroups than the device holds at six to a compute unit, and four fit at
-        // five: two and four, us, 64 rows of 262,144 fp32 67 and 58 (bf16 68 and 55; cut by nothing or by top-p 110 and 100), 64 of 200,003
-        // 57.5 and 54, 96 of 151,936 59 and 55.5, 128 64 and 62; that fit already, 64 of 151,936 42 and 50, 80 45 and 53; in several turns either
-        // way, 256 of 100,003 83 and 91; shorter rows, 128 of 100,003 54 both, 200 of 65,537 55 and 56.5.
-        const long long sampled = a.n_sampled + a.n_greedy;
-        const bool big = !a.lazy_scale && nseg >= 128 && sampled * ((nseg + 7) / 8) > 6 * a.cu_count && sampled * ((nseg + 15) / 16) <= 5 * a.cu_count;
+        // ... and four where they take fewer turns of workgroups (five to a compute unit; with two segments a wave six), and where
+        // these are the last, or the rows so long that what their last workgroup has too many is little.  Two and four, us: one turn for
+        // two, 64 rows of 262,144 fp32 67 and 58 (bf16 68 and 55; cut by nothing or by top-p 110 and 100), 64 of 200,003 57.5 and 54, 96
+        // of 151,936 59 and 55.5, 128 64 and 62; more turns, 128 of 262,144 114 and 103 (bf16 114 and 94), 256 214 and 196 (212 and 173),
+        // 160 of 200,003 104 and 100.5 (100 and 90), 256 166 both (160 and 145).  As many turns, 64 of 151,936 42 and 50, 160 74 and 85, 96
+        // of 262,144 85 and 88 (83 and 78).  Shorter rows, 192 of 151,936 91 and 94, 256 121 and 118, 256 of 131,073 99 and 105,
+        // 256 of 100,003 83 and 91, 128 54 both, 200 of 65,537 55 and 56.5.
+        const long long sampled = a.n_sampled + a.n_greedy, at_two = 6 * std::max(a.cu_count, 1), at_four = 5 * std::max(a.cu_count, 1);
+        const long long turns_two = (sampled * ((nseg + 7) / 8) + at_two - 1) / at_two, turns_four = (sampled * ((nseg + 15) / 16) + at_four - 1) / at_four;
+        const bool big = !a.lazy_scale && turns_four < turns_two && (nseg >= 192 || (nseg >= 128 && turns_four == 1));
         const int per_group = 4 * (four || big ? 4 : two ? 2 : 1);
         dim3 fgrid((unsigned)((nseg + per_group - 1) / per_group), n_rows + a.n_greedy);
         if (a.dtype == 1) {

@@ -1153,9 +1153,9 @@ def test_bf16_rows_cut_by_min_p_with_edits_at_every_place(ctx, V, rows):
     assert np.array_equal(got, oracle_tokens(logits, params, u)), (V, rows)
 
 
-# Launches of a few more workgroups than the device holds with two segments a wave, which take four: penalties and bias, masks, greedy rows
+# Launches that four segments a wave bring into fewer turns of workgroups, the last one or not: penalties and bias, masks, greedy rows
 # that ride along, rows cut by top-p, by min-p and not at all
-@pytest.mark.parametrize("V, rows, bf16", [(131_073, 100, False), (200_003, 64, True), (262_144, 52, False)])
+@pytest.mark.parametrize("V, rows, bf16", [(131_073, 100, False), (200_003, 64, True), (262_144, 52, False), (200_003, 128, False), (262_144, 110, True)])
 def test_rows_of_launches_with_four_segments_a_wave(ctx, V, rows, bf16):
     import torch
 
