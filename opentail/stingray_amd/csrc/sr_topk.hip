@@ -1725,7 +1725,11 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
         // 64 words about 50).  With one pair per lane it is found with ballots, to 16 bits, rounded down (worth its
         // eight or nine pairs of ballots only where the shares are that small).
         uint32_t k_close = 0u;
-        const int share = (sel + nb - 1) / nb;  // (the waves' share was this or more)
+        // (the waves' share was this or more; where lists are short, and others stream the row, at least two, so that there are twice as many words as waves: the
+        // 40th largest of 64 maxima has some 63 elements above it, of 64 pairs 42, and with a history of 64 the list is
+        // ranked by counting.  1, 4, 16, 32 rows of 262,144 fp32, top-k 40: 16.3, 17.3, 19.2, 21.2 -> 14.3, 15.5, 17.6, 19.4 us;
+        // rows of up to four chunks the same or 0.2 us less)
+        const int share = !kKept && kShort && nb <= SR_WAVE ? max((sel + nb - 1) / nb, 2) : (sel + nb - 1) / nb;
         const uint32_t km_lane = km;
         km = sr_wave_max_u32(km);
         if (kShort && nb <= SR_WAVE && share <= 2) {
@@ -2169,7 +2173,7 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
             // group maxima of all its chunks.)
             last_sel = cur.sel;
             if constexpr (!kKept) {
-                const int need = max((cur.sel + S * kWaves - 1) / (S * kWaves), 1);
+                const int need = max((cur.sel + S * kWaves - 1) / (S * kWaves), kShort && S * kWaves <= SR_WAVE ? 2 : 1);
                 // the wave's largest kept element: the row tail drops what lies hopelessly far below the row's
                 const float pa = fmaxf(gm1[0], gm1[1]), pb = fminf(gm1[0], gm1[1]), pc = fmaxf(gm1[2], gm1[3]), pd = fminf(gm1[2], gm1[3]);
                 const uint32_t k1 = sr_okey(fmaxf(pa, pc));  // the lane's largest group maximum

@@ -113,3 +113,31 @@ def test_launches_of_several_turns_beside_other_work(ctx, rows, vocab, bf16):
             noise = noise * 0.5 + 1.0
     _check(ctx, rng, rows, vocab, 1000, bf16)
     side.synchronize()
+
+
+# Short lists over many waves: each gives its two largest, of which the bound comes also where one a wave would do (lists of up to as
+# many entries as waves); waves with one entry and with none among them
+@pytest.mark.parametrize("vocab,bf16", [(4 * CHUNK - 1, False), (5 * CHUNK, False), (8 * CHUNK - 3, False), (8 * CHUNK + 1, False), (327_000, True)])
+def test_short_lists_of_rows_that_many_waves_stream(ctx, vocab, bf16):
+    import torch
+
+    rng = np.random.default_rng(vocab)
+    rows = 12
+    logits = rng.normal(0, 1.5, (rows, vocab)).astype(np.float32)
+    allowed = np.ones((rows, vocab), dtype=bool)
+    allowed[1] = False
+    allowed[1, rng.integers(0, vocab, 9)] = True           # most waves have nothing, the others one
+    allowed[2, : vocab // 2] = False                       # half the waves have nothing
+    logits[3, : 3000] += 20.0                              # a few waves have everything
+    logits[4] = np.round(logits[4] * 2) / 2                # ties at the bound
+    bits = synthetic.to_bf16_bits(logits)
+    if bf16:
+        logits = synthetic.bf16_bits_to_f32(bits)
+    dev = torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16) if bf16 else torch.from_numpy(logits).cuda()
+    active = np.isin(np.arange(rows), (1, 2)).astype(np.uint8)
+    for k in (1, 2, 31, 32, 33, 40, 63, 64):
+        params = [SamplingParams(Temperature=0.8, TopK=k, TopP=0.95, RepetitionPenalty=1.1 if r % 2 else 1.0,
+                                 PreviousTokens=rng.integers(0, vocab, 60).tolist() if r % 2 else []) for r in range(rows)]
+        mask, u = pack_allow_mask(allowed), rng.random(rows)
+        got = ctx.sample_batch(dev, params, u, mask, active)
+        assert np.array_equal(got, oracle_tokens(logits, params, u, mask, active)), (vocab, bf16, k)
