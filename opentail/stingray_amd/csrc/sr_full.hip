@@ -4764,13 +4764,16 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_factor(SrFullArgs a, SrSpecA
 // of them whose draft is accepted; the position that ends the row for certain, and above it whether its id lies outside the vocabulary
 constexpr int kSpecPicked = 4, kSpecAccepted = 5, kSpecLast = 6;
 constexpr int kSpecDone = -2;  // SrSpecArgs::reject of a row whose results are written
+// The words behind a position's meeting point (SrFullArgs::row_sync) that count its workgroups in, k_spec_units clears them.  (Not
+// those of k_prepared_row and of the greedy rows: other launches of the context find these as they left them.)
+constexpr int kOpenFirst = 4, kOpenSecond = 5;
 constexpr int kUnitVecs = SR_UNIT_TERMS / (4 * SR_WAVE);
 constexpr float kLog2E = 0x1.715476p+0f;
 __global__ __launch_bounds__(256) void k_spec_units(SrFullArgs a, SrSpecArgs s)
 {
     const int slot = blockIdx.y, lane = sr_lane(), u = (int)blockIdx.x * 4 + sr_wave_id(), n = s.vocab;
     if (blockIdx.x == 0 && threadIdx.x < 2) {  // nobody has counted in
-        a.row_sync[(size_t)slot * SR_ROW_SYNC_STRIDE + 1 + threadIdx.x] = 0ull;
+        a.row_sync[(size_t)slot * SR_ROW_SYNC_STRIDE + kOpenFirst + threadIdx.x] = 0ull;
         if (slot % (s.n_draft + 1) == 0 && threadIdx.x == 0) s.sync[(size_t)(slot / (s.n_draft + 1)) * SR_ROW_SYNC_STRIDE + kSpecAccepted] = 0ull;
     }
     if (u >= s.n_units) return;
@@ -4876,8 +4879,7 @@ __device__ __forceinline__ double spec_open_spread(int n) { return ((double)(n /
 // known from the units: no meeting); counts in, and whoever is there last walks the row's records to s, while the others write e
 // and wait for m1 (bounded); then fl(e m1) by accumulator, the records, counts in, and whoever is there last walks those to m2.
 // A workgroup whose wait runs out marks the position (SrFullState::late_behind) and counts itself in; the last one then adds the
-// accumulators without records.  The words behind a position's meeting point (row_sync): 1 workgroups at the first count, 2 at
-// the second, 3 m1 with the launch's number above it.
+// accumulators without records.
 // one position of a row: e from the logits
 struct SpecOpenRow {
     const float* lg;
@@ -5102,7 +5104,7 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_open(SrFullArgs a, SrSpecArg
 #pragma unroll
             for (int g = 0; g < SR_SEQ_CHAINS; g++) before += g < wave ? seg_own[g] : 0.0f;
             if (seg < nseg) seg_make_record<true>(x, seg, (double)before, recs + seg, own);
-            if (count_in(1)) {
+            if (count_in(kOpenFirst)) {
                 const bool staged = stage_records<kPrepT>(recs, nseg, sm.room, (int)sizeof(sm.room));
                 if (wave == 0) {
                     int dummy;
@@ -5161,7 +5163,7 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_open(SrFullArgs a, SrSpecArg
             const float front = t.kind == 0 ? before_chain * m1 : (float)(blk * SR_SEG_TERMS) * t.uniform;
             seg_make_record<true>(x, blk, (double)front, chain + blk, own);
         }
-        if (count_in(2)) {
+        if (count_in(kOpenSecond)) {
             // (everyone's e, records and marks are out; m1 is there)
             if (tid == 0) {
                 sm.bc[2] = sr_load_agent(&st->late_behind) == a.seq ? 1u : 0u;

@@ -156,7 +156,8 @@ static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // put in by an atomic maximum before the first count of a launch, so nothing clears the words.  The word behind it counts the
 // workgroups of k_prepared_row the same way; k_full_row, which leaves the row to them, starts it.  The third one holds what the
 // workgroups of a greedy row have found so far (zero between launches), the fourth one the factor that k_prepared_row's workgroups
-// wait for, with the launch number above it.
+// wait for, with the launch number above it; k_spec_open's wait for theirs there too, and the fifth and the sixth one count them in at
+// their two meeting points (k_spec_units clears both).
 #define SR_ROW_SYNC_STRIDE 32
 
 struct SeqSegFunc;

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 from oracle import binding as orc
-from opentail.stingray_amd import Sampler, SamplerContext, SamplingParams, pack_allow_mask, synthetic
+from opentail.stingray_amd import SR_OUT_DEGENERATE, Sampler, SamplerContext, SamplingParams, pack_allow_mask, synthetic
 from tests.helpers import DotnetRandom, ReplayRandom, hooks_lib, oracle_tokens, to_oracle
 
 pytestmark = pytest.mark.gpu
@@ -1187,3 +1187,36 @@ def test_rows_of_launches_with_four_segments_a_wave(ctx, V, rows, bf16):
         u = rng.random(rows)
         got = ctx.sample_batch(dev, params, u, mask, active)
         assert np.array_equal(got, oracle_tokens(logits, params, u, mask, active)), (V, rows, list(only))
+
+
+# Rows that hold nothing above -inf, greedy, beside a row on the full path, in every place that a verification of the same context has
+# worked out a position in (all of them: every accept test hangs on its last digits)
+@pytest.mark.parametrize("V, rows, L", [(4_096, 3, 20), (8_193, 9, 6), (70_001, 7, 5)])
+def test_greedy_rows_of_nothing_behind_a_verification(ctx, V, rows, L):
+    rng = np.random.default_rng(V)
+    params = [SamplingParams(Temperature=1.0 if r % 2 else 0.8) for r in range(rows)]
+    t = synthetic.zipf_head_logits(rng, rows * (L + 1), V).reshape(rows, L + 1, V)
+    q = np.full((rows, L, V), 1e-6, dtype=np.float32)
+    k = np.argmax(t[:, :L], axis=2).astype(np.int32)
+    u = rng.random((rows, L + 1))
+    for r in range(rows):
+        for i in range(L):
+            p = orc.build_filtered_distribution(t[r, i], to_oracle(params[r]))[k[r, i]]
+            q[r, i, k[r, i]] = p * np.float32(1.25)
+            u[r, i] = np.nextafter(np.float64(np.float32(p / q[r, i, k[r, i]])), 0.0)
+    n = 1 + rows * (L + 1)
+    x = rng.normal(0, 2.0, (n, V)).astype(np.float32)
+    x[1::4] = NEG_INF
+    x[2::4] = np.nan
+    allowed = np.ones((n, V), dtype=bool)
+    allowed[3::4] = False
+    active = np.array([r % 4 == 3 for r in range(n)], dtype=np.uint8)
+    step = [SamplingParams(Temperature=0.9, TopP=0.9)] + [SamplingParams(Temperature=0.0)] * (n - 1)
+    for _ in range(2):
+        _check_spec(ctx, t, q, k, params, u)
+        tokens, flags = ctx.sample_batch(_cuda(x), step, rng.random(n), pack_allow_mask(allowed), active, return_flags=True)
+        for r in range(1, n):
+            if r % 4:
+                assert tokens[r] == 0 and flags[r] & SR_OUT_DEGENERATE, (r, tokens[r], flags[r])
+            else:
+                assert tokens[r] == np.argmax(x[r]) and not flags[r] & SR_OUT_DEGENERATE, (r, tokens[r], flags[r])
