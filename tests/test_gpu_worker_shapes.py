@@ -99,20 +99,41 @@ def test_ties_across_chunks_that_share_their_groups(ctx):
         assert np.array_equal(got, oracle_tokens(logits, params, u)), n
 
 
-# Launches of more than two turns of workers, whose second ones start late: the same tokens at every step, also with work of other
-# streams on the device.
+# Launches of more than two turns of workers, whose second ones start late: the same tokens at every step, alone and between passes of two
+# other streams over 64 MB each, which are queued with the steps and last longer than these do
 @pytest.mark.parametrize("rows,vocab,bf16", [(513, 20_011, False), (1030, 40_000, True)])
 def test_launches_of_several_turns_beside_other_work(ctx, rows, vocab, bf16):
     import torch
 
     rng = np.random.default_rng(rows)
-    noise = torch.randn(4096, 4096, device="cuda")
-    side = torch.cuda.Stream()
-    with torch.cuda.stream(side):
-        for _ in range(20):
-            noise = noise * 0.5 + 1.0
-    _check(ctx, rng, rows, vocab, 1000, bf16)
-    side.synchronize()
+    logits, params, mask, active = _batch(rng, rows, vocab, 1000)
+    u = rng.random(rows)
+    dev = torch.from_numpy(logits).cuda()
+    if bf16:
+        bits = synthetic.to_bf16_bits(logits)
+        logits = synthetic.bf16_bits_to_f32(bits)
+        dev = torch.from_numpy(bits.view(np.int16)).cuda().view(torch.bfloat16)
+    want = oracle_tokens(logits, params, u, mask, active)
+    steps = 8
+    tokens = torch.full((2 * steps, rows), -7, dtype=torch.int32, device="cuda")
+    noise = [torch.randn(4096, 4096, device="cuda") for _ in range(2)]
+    sides = [torch.cuda.Stream() for _ in noise]
+    batch = ctx.new_batch().upload(params, vocab, u, mask, active)
+    for t in range(steps):
+        ctx.sample_launch(batch, dev, tokens[t])
+    for side in sides:
+        side.wait_stream(torch.cuda.current_stream())
+    for t in range(steps, 2 * steps):
+        for x, side in zip(noise, sides):
+            with torch.cuda.stream(side):
+                for _ in range(10):
+                    x.mul_(0.5).add_(1.0)
+        ctx.sample_launch(batch, dev, tokens[t])
+    ctx.synchronize()
+    torch.cuda.synchronize()
+    batch.close()
+    for t, got in enumerate(tokens.cpu().numpy()):
+        assert np.array_equal(got, want), (t, np.nonzero(got != want)[0][:10])
 
 
 # Short lists over many waves: each gives its two largest, of which the bound comes also where one a wave would do (lists of up to as
