@@ -1220,3 +1220,32 @@ def test_greedy_rows_of_nothing_behind_a_verification(ctx, V, rows, L):
                 assert tokens[r] == 0 and flags[r] & SR_OUT_DEGENERATE, (r, tokens[r], flags[r])
             else:
                 assert tokens[r] == np.argmax(x[r]) and not flags[r] & SR_OUT_DEGENERATE, (r, tokens[r], flags[r])
+
+
+# A context's states, meeting points and records are shared by verifications (of rows that nothing touches, and of others), steps of the
+# full path with greedy rows in its pass, and distributions: every one of them behind every other one
+@pytest.mark.parametrize("V", [9_001, 70_001])
+def test_calls_of_every_kind_behind_each_other(V):
+    rng = np.random.default_rng(V)
+    rows, L = 4, 4
+    plain = [SamplingParams(Temperature=0.7 + 0.1 * r) for r in range(rows)]
+    mixed = [SamplingParams(Temperature=0.9, TopP=0.9 if r % 2 else 1.0) for r in range(rows)]
+    chain = [SamplingParams(Temperature=0.0 if r % 3 == 0 else 1.1, TopP=0.95 if r % 2 else 1.0, MinP=0.02 if r % 5 == 1 else 0.0) for r in range(3 * rows)]
+    logits = synthetic.zipf_head_logits(rng, 3 * rows, V)
+    logits[6] = NEG_INF  # (greedy)
+    open_case, other_case, u = _spec_case(rows, L, V, plain, V + 1, False), _spec_case(rows, L, V, mixed, V + 2, True), rng.random(3 * rows)
+
+    sampled = [r for r in range(3 * rows) if r % 3]
+
+    def step(c):
+        assert _check_rows(c, logits, chain, u)[6] & SR_OUT_DEGENERATE
+
+    calls = [lambda c: _check_spec(c, *open_case[:3], plain, open_case[3]), lambda c: _check_spec(c, *other_case[:3], mixed, other_case[3]),
+             step,
+             lambda c: _check_distribution(c, logits[sampled], [chain[r] for r in sampled])]
+    c = SamplerContext(0)
+    try:
+        for i in (0, 1, 2, 3, 0, 2, 1, 3, 1, 0, 3, 2, 0, 0):
+            calls[i](c)
+    finally:
+        c.close()
