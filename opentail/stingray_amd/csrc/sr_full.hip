@@ -5385,7 +5385,10 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
     __syncthreads();
     if (bc == 0u) return;
     const bool alone = bc == 2u;
-    const bool staged = stage_records<kSpecT>(funcs, nseg, &turn_all[0][0], (int)sizeof(turn_all));
+    // (Not where neither launch stood in front, which takes smaller launches and rows that are cut: 16 x 8 of 50,257 under min-p 54.5
+    // us with it and 53.8 without, of 20,011 that nothing touches 48.7 and 48.3, 64 x 4 of 32,768 under top-p 108.3 and 107.8, 1 x 2 of
+    // 151,936 44.9 and 45.1.  16 x 8 of 262,144, one sequence under top-p, which has k_spec_factor in front: 231.3 and 231.7.)
+    const bool staged = kFrom != 0 && stage_records<kSpecT>(funcs, nseg, &turn_all[0][0], (int)sizeof(turn_all));
     if (wave != 0) return;
     const double ud = u[kind == 0 ? pos + 1 : L];
     const float r = __double2float_rn(ud);
