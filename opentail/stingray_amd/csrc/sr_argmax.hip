@@ -94,10 +94,11 @@ __device__ __forceinline__ bool is_nan_bits(uint32_t x) { return (x & 0x7fffffff
 // its first vectors and for its chunks to come together.  Two tiles of four vectors a thread in turn, the loads of one under the
 // folding of the other, two and a half (bf16, in pairs) and four instructions an element; an element's index is looked for only
 // where a wave's tile holds more than its tiles before.  Against eight or nine instructions an element, key and index carried along, a
-// tile of eight at a time, and element by element in rows at odd addresses, whole calls in us: 128 rows of 151,936 bf16 24.4 -> 21.6, 256
-// 32.0 -> 28.0, 1 16.3 -> 14.5, 512 45.6 -> 39.5; 64 rows of 100,003 bf16 30 -> 18, 300 of 100,003 fp32 84 -> 34, 1,024 of 20,011 bf16 45 -> 26.
-// (Tiles of eight 27 at 128 rows, of six 26.7, of two and three as of four; three to six workgroups to a compute unit 24.6 - 25.4 where
-// two took 24.8.  With four instructions an element in the search for the index, in place of two, 24.8.)
+// tile of eight at a time, and element by element in rows at odd addresses, whole calls with host results one behind the other, four buffers
+// in turn, both kernels on one card, us: 128 rows of 151,936 bf16 23.2 -> 19.6, 256 30.6 -> 25.8, 1 15.6 -> 13.6, 512 44.1 -> 35.6; 64 rows
+// of 100,003 bf16 35.3 -> 17.4, 300 of 100,003 fp32 113 -> 35.8, 1,024 of 20,011 bf16 42.7 -> 21.1.
+// (In a run of its own, 128 rows: tiles of eight 27, of six 26.7, of two and three as of four; three to six workgroups to a compute unit
+// 24.6 - 25.4 where two took 24.8.  With four instructions an element in the search for the index, in place of two, 24.8.)
 template <int ES, bool kAligned> __global__ __launch_bounds__(kThreads) void k_argmax_rows(SrArgmaxArgs a)
 {
     __shared__ unsigned long long s_best[kThreads / SR_WAVE];
