@@ -96,7 +96,11 @@ struct SrMaskClear {
 // bring them, after which the second workers start.  None, 0.5, 0.8 and 1.0 of it, us: 1,024 rows of 151,936 fp32 114.2, 109.4, 106.8,
 // 107.2; 768 93.9, 82.0, 80.1, 83.4; 520 66.8, 62.5, 62.3, 65.0; 1,024 of bf16 69.4, 67.2, 66.4, 66.4; 600 of 49,152 fp32 40.0, 39.7, 38.2,
 // 37.3; 1,024 of 16,384 39.7, 39.2, 38.9, 38.8.  Up to two workers to a compute unit it gains nothing: 512 rows 59.7 and 59.0, 384 50.7
-// both, 320 47.6 and 48.0, 512 of bf16 38.8 and 39.5.
+// both, 320 47.6 and 48.0, 512 of bf16 38.8 and 39.5.  That workgroups cu_count ... 2 cu_count - 1 are the compute units' second ones holds
+// only where the launch has the device to itself.  Beside another stream that is never idle the wait is lost time, none and 0.8, us a step and in
+// brackets until both streams are through: four passes over 64 MB a step, 1,024 rows 183 and 182 (183 and 182), 768 143 and 153 (157 and
+// 153), 520 122 and 132 (137 both); a 4,096^3 bf16 product a step, 198 and 202, 176 and 179, 155 and 161.  Beside three small kernels a step
+// it gains what it gains alone (114 and 106, 94 and 81, 67 and 64).
 #define SR_TK_START_GAP 85000.0
 #define SR_TK_MASK_WORDS 3                 // 32-bit keep-words per chunk thread: 19 x 4 and 10 x 8 bits both fit 96
 #define SR_TK_GROUPS 4                     // group maxima per thread
