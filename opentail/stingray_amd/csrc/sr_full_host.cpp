@@ -546,7 +546,10 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     const int32_t* list = nullptr;
     SrFullArgs full{};
     const bool in_one = n_draft > 0 && n_draft < 64 && draft_probs_dev && rows <= 65535;  // (k_spec_factor: a position a lane)
-    // rows that nothing touches, all of them: k_spec_units and k_spec_open (the lines: SR_OPEN_*)
+    // Rows that nothing touches, all of them: k_spec_units and k_spec_open (the lines: SR_OPEN_*).  Not the untouched rows of a mixed call:
+    // it lasts as long as the cut row's positions, which one workgroup each finishes.  16 x 8 of 262,144, none, one and all sequences
+    // under top-p, us: 114, 229, 270; with one, k_full_softmax_seg 59, k_full_row 110, k_spec_factor 38, k_spec_rows 22, where the other
+    // way's 23 + 69 + 23 would stand beside a pass and a k_full_row for the cut row's nine positions.
     const int nseg = (V + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
     bool all_open = in_one && V >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX && (int64_t)rows * P <= 65535 &&
                     (nseg < SR_OPEN_SHORT_SEGS || rows * P > ctx->cu_count || (nseg >= SR_OPEN_MIN_SEGS && (int64_t)rows * P * nseg >= SR_OPEN_SEGS));
