@@ -1230,15 +1230,18 @@ def test_calls_of_every_kind_behind_each_other(V):
     rows, L = 4, 4
     plain = [SamplingParams(Temperature=0.7 + 0.1 * r) for r in range(rows)]
     mixed = [SamplingParams(Temperature=0.9, TopP=0.9 if r % 2 else 1.0) for r in range(rows)]
-    chain = [SamplingParams(Temperature=0.0 if r % 3 == 0 else 1.1, TopP=0.95 if r % 2 else 1.0, MinP=0.02 if r % 5 == 1 else 0.0) for r in range(3 * rows)]
-    logits = synthetic.zipf_head_logits(rng, 3 * rows, V)
-    logits[6] = NEG_INF  # (greedy)
-    open_case, other_case, u = _spec_case(rows, L, V, plain, V + 1, False), _spec_case(rows, L, V, mixed, V + 2, True), rng.random(3 * rows)
+    n = rows * (L + 1) + 1
+    chain = [SamplingParams(Temperature=0.0 if r % 4 else 1.1, TopP=0.95 if r % 8 else 1.0, MinP=0.02 if r % 16 == 4 else 0.0) for r in range(n)]
+    logits = synthetic.zipf_head_logits(rng, n, V)
+    nothing = [r for r in range(2, n) if r % 4]  # (greedy, in the places of the last sequences' positions, of which each has been drawn from in one)
+    logits[nothing] = NEG_INF
+    open_case, other_case, u = _spec_case(rows, L, V, plain, V + 1, False), _spec_case(rows, L, V, mixed, V + 2, True), rng.random(n)
 
-    sampled = [r for r in range(3 * rows) if r % 3]
+    sampled = [r for r in range(n) if r % 4 == 0]
 
     def step(c):
-        assert _check_rows(c, logits, chain, u)[6] & SR_OUT_DEGENERATE
+        flags = _check_rows(c, logits, chain, u)
+        assert all(flags[r] & SR_OUT_DEGENERATE for r in nothing)
 
     calls = [lambda c: _check_spec(c, *open_case[:3], plain, open_case[3]), lambda c: _check_spec(c, *other_case[:3], mixed, other_case[3]),
              step,
