@@ -404,7 +404,7 @@ void sr_destroy(sr_ctx* ctx)
                          &ctx->work, &ctx->edit_tab, &ctx->host_logits, &ctx->stage_probs, &ctx->out_tokens,
                          &ctx->full_state, &ctx->sort_k0, &ctx->sort_v0,
                          &ctx->sort_v1, &ctx->ident, &ctx->redo_list, &ctx->spec_probs, &ctx->spec_resid, &ctx->spec_reject,
-                         &ctx->spec_units, &ctx->spec_unit_chains, &ctx->seg_part, &ctx->seg_func, &ctx->full_row_sync, &ctx->spec_sync, &ctx->full_seg_func, &ctx->full_seg_sum, &ctx->full_seg_cnt, &ctx->full_mass, &ctx->full_chain_sum, &ctx->full_chain_func};
+                         &ctx->spec_units, &ctx->spec_unit_chains, &ctx->seg_part, &ctx->seg_func, &ctx->full_row_sync, &ctx->full_meet, &ctx->spec_sync, &ctx->full_seg_func, &ctx->full_seg_sum, &ctx->full_seg_cnt, &ctx->full_mass, &ctx->full_chain_sum, &ctx->full_chain_func};
     for (DeviceBuf* b : bufs) b->release();
     ctx->uni_ring.release(ctx->pinned);
     ctx->pinned.release();

@@ -1542,12 +1542,18 @@ __device__ __forceinline__ void seg_apply_edits(const SrFullArgs& a, const SrRow
 }
 
 // Everything is one launch (k_full_softmax_seg): a wave keeps its segments in registers, so the logits are read once.  The
-// workgroups of a row meet twice: each folds its largest logit into the row's and counts itself in; when the count is
-// full it computes e = expf(x - max), leaves its segments' sums (and, for rows that top-p cuts, its share of the row's
-// mass by size of e), meets again, and makes the segments' records from the sums in front of them.  Workgroups start in
+// workgroups of a row meet twice: each leaves its largest logit, and when it has everyone's computes e = expf(x - max), leaves its
+// segments' sums (and, for rows that top-p cuts, its share of the row's mass by size of e), and when it has everyone's makes
+// the segments' records from the sums in front of them.  Workgroups start in
 // the order of their numbers, a row's side by side, so those that a waiting workgroup waits for are running or next to
-// start; the waits are bounded all the same: a workgroup whose wait runs out marks the row (SrFullState::late), counts itself
-// in everywhere and leaves, and the row's own workgroup does the whole row by itself from the logits (row_alone).
+// start; the waits are bounded all the same: a workgroup whose wait runs out marks the row (SrFullState::late), leaves its words
+// for the others and ends, and the row's own workgroup does the whole row by itself from the logits (row_alone).
+// What is left at a meeting carries the launch's number (SrFullArgs::meet), so that the poll that finds it has it: a maximum and a count of
+// the row by atomics, polled and then read, were four trips to memory one behind the other, and the atomics of a row queue.  41 meetings in a row on
+// their own, us each, atomics and words: 19 workgroups x 64 rows 5.6 and 2.4, 13 x 32 2.7 and 1.3, 32 x 16 3.8 and 2.3; the second,
+// whose sums were written through, waited for, counted and read, 4.1 and 2.6, 2.2 and 1.5, 2.8 and 2.0.  Of calls, where the slowest
+// workgroup is waited for either way: 16 rows of 262,144 fp32 with distributions 65.0 -> 63.4, 32 ragged bf16 rows of 100,003 52.0 -> 50.8, 64
+// penalised rows of 151,936 41.15 -> 40.7.
 //
 // What bounds it: the vector units (the double-precision expf is 30 instructions an element).  The first pass used to
 // take a fast exponential of every element, for approximate sums relative to the segment's own maximum, to save the second
@@ -1707,8 +1713,9 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     }
     const int n = a.vocab, nseg = seg_count(n);
     SrFullState* st = a.state + slot;
-    unsigned long long* sync = a.row_sync + (size_t)slot * SR_ROW_SYNC_STRIDE;
     const unsigned long long stamp = (unsigned long long)a.seq << 32;
+    unsigned long long* const met_max = a.meet + (size_t)slot * a.meet_stride;  // a word per workgroup
+    unsigned long long* const met_sum = met_max + a.meet_sums;                  // ... and per segment
     SeqSegFunc* recs = a.seg_func + (size_t)slot * a.seg_stride;
     float* sums = a.seg_sum + (size_t)slot * a.seg_stride;
     if (threadIdx.x < 32) tab[threadIdx.x] = sr_exp2f_tab[threadIdx.x];
@@ -1787,41 +1794,46 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
         if (seg0 + s * kW < nseg) k = max(k, seg_max_key(t[s]));
     k = sr_wave_max_u32(k);
     if (lane == 0) wkey[wave] = k;
-    // The meeting point: `ready` goes in (behind everything the workgroup has written through or added), and the workgroup
-    // waits until the row's workgroups are all in.  part = 0, 1: the first, the second meeting.
-    auto met = [&](int part) -> bool {
-        if (threadIdx.x == 0) {
-            __hip_atomic_fetch_add(sync, 1ull << (16 * part), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            uint32_t ok = 0u;
-            for (uint32_t it = 0; it < a.row_wait_limit; it++) {
-                const unsigned long long v = sr_load_agent(sync);
-                if ((uint32_t)(v >> 32) == a.seq && ((uint32_t)(v >> (16 * part)) & 0xffffu) == gridDim.x) { ok = 1u; break; }
-                __builtin_amdgcn_s_sleep(2);
-            }
-            if (ok == 0u) {
-                // the wait ran out: the row is left to its own workgroup, and nobody waits for this one
-                sr_store_agent(&st->late, a.seq);
-                if (part == 0) __hip_atomic_fetch_add(sync, 1ull << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else if (part == 0) {
-                bc[1] = full_maxkey_of(a, sr_load_agent(&st->maxkey));
-            }
-            bc[0] = ok;
-        }
-        __syncthreads();
-        return bc[0] != 0u;
-    };
     sr_barrier_lds();
-    if (threadIdx.x == 0) {
+    // The first meeting: a word of every workgroup, its largest logit below the launch's number, which all of the row's
+    // workgroups read until it is this launch's.
+    if (wave == 0) {
         k = wkey[0];
 #pragma unroll
         for (int j = 1; j < kW; j++) k = max(k, wkey[j]);
-        // (each atomic's returned value is waited for before the next is issued: whoever finds the count full finds the
-        // maximum complete)
-        const unsigned long long s0 = __hip_atomic_fetch_max(sync, stamp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long s1 = __hip_atomic_fetch_max(&st->maxkey, full_maxkey(a, k), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        asm volatile("" : : "v"(s0), "v"(s1) : "memory");
+        if (lane == 0) sr_store_agent(met_max + blockIdx.x, stamp | (unsigned long long)k);
+        bool here = true;
+        for (int g0 = 0; g0 < (int)gridDim.x; g0 += SR_WAVE) {
+            if (g0 + lane >= (int)gridDim.x) break;
+            unsigned long long v = 0ull;
+            bool in = false;
+            for (uint32_t it = 0; it < a.row_wait_limit; it++) {
+                v = sr_load_agent(met_max + g0 + lane);
+                if ((uint32_t)(v >> 32) == a.seq) { in = true; break; }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            here = here && in;
+            k = max(k, (uint32_t)v);
+        }
+        here = __ballot(!here) == 0ull;
+        k = sr_wave_max_u32(k);
+        if (lane == 0) {
+            bc[0] = here ? 1u : 0u;
+            bc[1] = k;
+            // the wait ran out: the row is left to its own workgroup
+            if (!here) sr_store_agent(&st->late, a.seq);
+            else if (blockIdx.x == 0) st->maxkey = full_maxkey(a, k);
+        }
     }
-    if (!met(0)) return;
+    __syncthreads();
+    if (bc[0] == 0u) {
+        // (nobody waits for this one)
+        if (lane == 0)
+#pragma unroll
+            for (int s = 0; s < kS; s++)
+                if (seg0 + s * kW < nseg) sr_store_agent(met_sum + seg0 + s * kW, stamp);
+        return;
+    }
     const uint32_t mk = bc[1];
     // A NaN, or nothing above -inf: the row's workgroup makes it uniform.  A maximum of +inf, beside which e is no number where it
     // stands: the row's workgroup takes the row alone, so that every x - max below is at most 0, or -inf.
@@ -1914,7 +1926,6 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
             const float mine = wave_sum_8(c);
             if (lane < SR_SEQ_CHAINS) unsafeAtomicAdd(&chains[s][lane], mine);
         }
-        if (lane == 0) sr_store_agent(&sums[seg], own[s]);
     }
     sr_barrier_lds();
     if (by_mass) {
@@ -1930,9 +1941,35 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
         if (hb < a.chain_stride / SR_SEQ_CHAINS)
             a.chain_sum[(size_t)slot * a.chain_stride + (size_t)hb * SR_SEQ_CHAINS + (threadIdx.x & (SR_SEQ_CHAINS - 1))] = (&chains[0][0])[threadIdx.x];
     }
-    sr_drain_stores();
+    if (by_mass || by_count) {  // (added to before the workgroup's segments count as in)
+        sr_drain_stores();
+        __syncthreads();
+    }
+    // The second one: a word of every segment, its sum.
+    if (lane == 0) {
+#pragma unroll
+        for (int s = 0; s < kS; s++)
+            if (seg0 + s * kW < nseg) {
+                sr_store_agent(met_sum + seg0 + s * kW, stamp | (unsigned long long)sr_f2u(own[s]));
+                sums[seg0 + s * kW] = own[s];  // (for the launches behind)
+            }
+    }
+    for (int g = threadIdx.x; g < nseg; g += kThreads) {
+        unsigned long long v = 0ull;
+        bool in = false;
+        for (uint32_t it = 0; it < a.row_wait_limit; it++) {
+            v = sr_load_agent(met_sum + g);
+            if ((uint32_t)(v >> 32) == a.seq) { in = true; break; }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        if (!in) bc[0] = 0u;
+        share[g] = sr_u2f((uint32_t)v);
+    }
     __syncthreads();
-    if (!met(1)) return;
+    if (bc[0] == 0u) {
+        if (threadIdx.x == 0) sr_store_agent(&st->late, a.seq);
+        return;
+    }
     // (the row's mass by size, four buckets a lane, or the length of its list, on its way beside the segments' sums)
     float row_mass[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     const float* const mass_at = a.mass + (size_t)slot * kMassBuckets;
@@ -1942,7 +1979,6 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     } else if (by_count) {
         row_mass[0] = sr_load_agent(mass_at);
     }
-    for (int g = threadIdx.x; g < nseg; g += kThreads) share[g] = sr_load_agent(&sums[g]);
     // what the list of a row that is cut holds: everything that can survive its min-p, or enough of the largest for top-p
     uint32_t from = 0xffffffffu;
     bool too_long = false;
@@ -1963,7 +1999,6 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
         too_long = least > (float)list_cap(a.big_slabs != 0);
         if (blockIdx.x == 0 && threadIdx.x == 0) st->list_from = too_long ? 0u : from;
     }
-    sr_barrier_lds();
 #pragma unroll
     for (int s = 0; s < kS; s++) {
         const int seg = seg0 + s * kW;

@@ -18,6 +18,7 @@ hipError_t next_launch(sr_ctx* ctx)
     // the numbers have gone round: nothing of an earlier launch may look like this one's
     hipError_t e = hipMemsetAsync(ctx->full_state.p, 0, ctx->full_state.cap, ctx->stream);
     if (e == hipSuccess && ctx->full_row_sync.p) e = hipMemsetAsync(ctx->full_row_sync.p, 0, ctx->full_row_sync.cap, ctx->stream);
+    if (e == hipSuccess && ctx->full_meet.p) e = hipMemsetAsync(ctx->full_meet.p, 0, ctx->full_meet.cap, ctx->stream);
     if (e == hipSuccess && ctx->spec_sync.p) e = hipMemsetAsync(ctx->spec_sync.p, 0, ctx->spec_sync.cap, ctx->stream);
     ctx->full_seq = 1u;
     return e;
@@ -151,6 +152,10 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             SR_HIP(ctx, ctx->full_mass.reserve((size_t)n_rows * 256 * sizeof(float), st, true));
             SR_HIP(ctx, ctx->full_row_sync.reserve((size_t)(n_rows + n_greedy) * SR_ROW_SYNC_STRIDE * sizeof(unsigned long long), st, true));
             a.row_sync = ctx->full_row_sync.as<unsigned long long>();
+            a.meet_sums = (half_blocks + 15) & ~15;
+            a.meet_stride = (a.meet_sums + nseg + 15) & ~15;
+            SR_HIP(ctx, ctx->full_meet.reserve((size_t)n_rows * (size_t)a.meet_stride * sizeof(unsigned long long), st, true));
+            a.meet = ctx->full_meet.as<unsigned long long>();
             a.seg_func = (SeqSegFunc*)ctx->full_seg_func.p;
             a.seg_sum = ctx->full_seg_sum.as<float>();
             a.seg_cnt = ctx->full_seg_cnt.as<uint32_t>();

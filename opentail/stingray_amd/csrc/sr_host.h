@@ -301,7 +301,7 @@ struct sr_ctx {
     DeviceBuf spec_resid, spec_reject;  // ... the residual row of every row's first rejected position, that position
     DeviceBuf spec_units, spec_unit_chains;  // SrSpecArgs::units, ::unit_chains
     DeviceBuf seg_part, seg_func;       // approximate sums and increment functions of the segments of prepared rows
-    DeviceBuf full_row_sync, spec_sync;  // the rows' meeting points (SrFullArgs::row_sync, SrSpecArgs::sync)
+    DeviceBuf full_row_sync, full_meet, spec_sync;  // the rows' meeting points (SrFullArgs::row_sync, ::meet, SrSpecArgs::sync)
     DeviceBuf full_seg_func, full_seg_sum, full_seg_cnt, full_mass, full_chain_sum, full_chain_func;  // ... of the full-vocabulary path's denominators
     sr_batch* tmp_batch = nullptr;
     PinnedPool pinned;

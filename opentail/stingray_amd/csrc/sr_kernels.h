@@ -134,8 +134,8 @@ hipError_t sr_launch_selftest_expf(const float* x, float* y, int64_t n, hipStrea
 // ---- full-vocabulary path (sr_full.hip) ---------------------------------------------------------------
 struct SrFullState {
     // launch number << 32 | ordered key of the row's largest adjusted logit (0xffffffff = the row holds a NaN; 0 = none
-    // yet), raised with 64-bit atomic maxima: what an earlier launch left is below anything of the present one, so the
-    // word needs no clearing between launches
+    // yet); short and very long rows raise it with 64-bit atomic maxima: what an earlier launch left is below anything of the
+    // present one, so the word needs no clearing between launches
     unsigned long long maxkey;
     uint32_t flags;
     int32_t n_survivors;  // entries with probability > 0 when top-p starts
@@ -152,7 +152,7 @@ struct SrFullState {
 };
 static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // SrFullArgs::row_sync, a word per row (rows 256 bytes apart: every workgroup of a row adds to its word and polls it):
-// launch number << 32 | workgroups of k_full_softmax_seg at the second meeting point << 16 | at the first.  The number is
+// launch number << 32 | workgroups of a greedy row that have counted in.  The number is
 // put in by an atomic maximum before the first count of a launch, so nothing clears the words.  The word behind it counts the
 // workgroups of k_prepared_row the same way; k_full_row, which leaves the row to them, starts it.  The third one holds what the
 // workgroups of a greedy row have found so far (zero between launches), the fourth one the factor that k_prepared_row's workgroups
@@ -215,6 +215,10 @@ struct SrFullArgs {
     int32_t edits_in_pass;         // seg_func is set: sampled rows with up to SR_FULL_EDIT_VALUES edits keep no adjusted copy and
                                    // need no table either (k_full_softmax_seg applies their edits where it loads the row)
     unsigned long long* row_sync;  // [slot * SR_ROW_SYNC_STRIDE]
+    // [slot * meet_stride] what k_full_softmax_seg's workgroups leave for each other, the launch's number << 32 above every word (so nothing
+    // clears them between launches): a workgroup's largest logit as an ordered key, and from meet_sums on a segment's sum of e
+    unsigned long long* meet;
+    int32_t meet_stride, meet_sums;
     uint32_t row_wait_limit;       // polls of a row's count before a workgroup of k_full_softmax_seg stops waiting for it
     uint32_t behind_wait_limit;    // ... of k_prepared_row
     int32_t big_slabs;             // k_full_row gets 68 KB of shared memory more: lists of 16,384 candidates, slabs of 8,192 entries
