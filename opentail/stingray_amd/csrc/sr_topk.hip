@@ -498,6 +498,22 @@ struct KeptHistory {
     SrEdit hee[kHistRegs];
     float hx[kHistRegs];
 };
+// A worker that knows the row it will finish from the start, and has the registers, fetches the row's descriptor and its history before
+// it streams: in front of the tail they are four trips to memory one behind the other (in a launch that also asks whether the
+// largest entry decides: below).
+template <bool kKept, bool kRoomy> constexpr bool kHistBefore = kKept || kRoomy;
+// The largest entry decides.  What a row's token is follows from its largest entry alone where that entry's probability reaches
+// top-p (the running sum stops at the first entry), or where nothing is cut and it covers the draw.  Whether it does is known
+// as soon as the groups at or above the bound are: the k best all lie in them, so the exponentials of the groups' largest entries, with the
+// second largest standing in for what may lie below it, add up to at least the row's sum.  Such a row is done there; fetching groups, ordering
+// the list, the exact sums and the searches are for the others.  Nothing is decided that the exact arithmetic could see otherwise: the margins cover
+// its roundings, a draw or cut near a boundary (SR_OUT_AMBIGUOUS) is left to it, and so is a largest entry that is not the only one.
+// In launches of short lists, of dealt rows, and of more rows than compute units, us a launch before and now, rows whose largest entry stands
+// out and flat ones (N(0, 1.5^2)): 1 row of 49,152 fp32, top-k 40, 12.9 -> 10.8 and 14.0 -> 14.5, with a history of 64 13.2 -> 11.4 and 14.5 -> 14.9; 24 of
+// 100,003 bf16, top-k up to 1,000, 19.0 -> 12.0 and 24.6 -> 24.8; 512 of 151,936 fp32 61.2 -> 52.9 and 67.0 -> 66.5, 1,024 109 -> 96.9 and 117.6
+// -> 113.4 (3 to 4 of each from SR_RARE).  A launch of a worker to every compute unit ends with its flattest rows, which the question only keeps waiting.
+template <bool kKept, bool kShort, bool kRoomy> constexpr bool kDecides = kHistBefore<kKept, kRoomy> && (kShort || !kKept || !kRoomy);
+constexpr int kDecided = -3;  // what build_candidates returns for such a row
 // The masked logit of one token id of a row.
 __device__ __forceinline__ float row_logit(const SrTopkArgs& a, int row, const SrRow& rd, int id)
 {
@@ -525,18 +541,18 @@ __device__ __forceinline__ bool row_history_in_registers(const SrRow& rd)
     return use_edits && (rd.flags & kRowHistExcl) != 0u && rd.path == SR_PATH_TOPK && rd.edit_cnt <= kHistRegs * kThreads;
 }
 
-template <int EPV, int kVec, bool kKept, bool kShort, bool kFold, typename Early, typename Late>
+template <int EPV, int kVec, bool kKept, bool kShort, bool kFold, bool kDecide, typename Early, typename Late, typename Ask, typename HistMass, typename Decide>
 __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, int row, const SrRow& rd, bool want_bins,
                                                 bool force_exact, float inv_temp, BinMap* map_out,
                                                 float* bound_out, bool* binned, const KeptGroups& kept, Early&& early,
-                                                Late&& late, TopkSmem& sm);
+                                                Late&& late, Ask&& worth_asking, HistMass&& hist_mass, Decide&& decide, TopkSmem& sm);
 
 // force_exact: the chunk results of the row are not used, the candidates come from the logits themselves (what a row
 // whose candidates overflow the lists falls back to, and a row whose chunks were not handed over in time).
 // kShort: the launch holds no row that asks for more than kShortSel entries; the tail then carries the two steps that
 // pay for such rows only (a closer bound from the waves' pairs, ranking a short list by counting).  They are compiled
 // into launches of their own because their mere presence costs the long tails of other launches 0.6 us.
-template <int EPV, int kVec, bool kKept, bool kShort, bool kFold>
+template <int EPV, int kVec, bool kKept, bool kShort, bool kRoomy, bool kFold>
 __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int row, const SrRow& rd, bool force_exact,
                                               const KeptGroups& kept, const KeptHistory& kept_hist, TopkSmem& sm)
 {
@@ -565,11 +581,13 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
     // The history ids and their logits are fetched behind the candidate builder's own loads, so that neither
     // waits for the other.
     const bool hist_regs = row_history_in_registers(rd);
+    constexpr bool kHistEarly = kHistBefore<kKept, kRoomy>;
+    constexpr bool kDecide = kDecides<kKept, kShort, kRoomy>;
     SrEdit hee[kHistRegs];
     float hx[kHistRegs];
 #pragma unroll
     for (int r = 0; r < kHistRegs; r++) {
-        if constexpr (kKept) { hee[r] = kept_hist.hee[r]; hx[r] = kept_hist.hx[r]; }
+        if constexpr (kHistEarly) { hee[r] = kept_hist.hee[r]; hx[r] = kept_hist.hx[r]; }
         else { hee[r] = SrEdit{}; hx[r] = SR_NEG_INF; }
     }
     const float inv_temp = rd.temperature == 1.0f ? 1.0f : __fdiv_rn(1.0f, rd.temperature);
@@ -581,10 +599,34 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
     if (tid == 0) sm.bcast[4] = 0u;  // the short list's count of history entries (the barriers of the next call publish it)
     BinMap map0;
     float bound0 = 0.0f;
-    const int n_c = build_candidates<EPV, kVec, kKept, kShort, kFold>(
+    // the history entries' keys, raw and adjusted (0: none)
+    uint32_t hadj[kHistRegs], hraw[kHistRegs];
+    auto adjust_history = [&]() SR_INL {
+#pragma unroll
+        for (int r = 0; r < kHistRegs; r++) {
+            hadj[r] = hraw[r] = 0u;
+            const int e = r * kThreads + tid;
+            if (e < ne) {
+                const SrEdit ee = hee[r];
+                const float x = hx[r];
+                // -inf never enters the reference's selection (Sampler.cs:240-249)
+                if (x == x && sr_f2u(x) != 0xff800000u) {
+                    float v = x;
+                    // Sampler.cs:261-287: pen = pow(rep, occWindow) once; presence/frequency over the whole history
+                    if (ee.occ_all > 0) {
+                        if (rd.rep != 1.0f && ee.occ_win > 0) v = v > 0.0f ? __fdiv_rn(v, ee.pen) : __fmul_rn(v, ee.pen);
+                        v = __fsub_rn(v, __fadd_rn(rd.presence, __fmul_rn(rd.frequency, (float)ee.occ_all)));
+                    }
+                    hraw[r] = sr_okey(x);
+                    hadj[r] = sr_okey(v);
+                }
+            }
+        }
+    };
+    const int n_c = build_candidates<EPV, kVec, kKept, kShort, kFold, kDecide>(
         a, slot, row, rd, want_bins, force_exact, inv_temp, &map0, &bound0, &binned, kept,
         [&]() SR_INL {
-            if constexpr (!(kKept)) {
+            if constexpr (!kHistEarly) {
 #pragma unroll
                 for (int r = 0; r < kHistRegs; r++) {
                     const int e = r * kThreads + tid;
@@ -593,7 +635,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
             }
         },
         [&]() SR_INL {
-            if constexpr (!(kKept)) {
+            if constexpr (!kHistEarly) {
 #pragma unroll
                 for (int r = 0; r < kHistRegs; r++) {
                     const int e = r * kThreads + tid;
@@ -601,7 +643,46 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
                 }
             }
         },
+        // whether the largest entry may decide, when the others have this much at least (in its units)
+        [&](float rest) SR_INL -> bool {
+            const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
+            const float needs = use_top_p ? fmaxf(rd.top_p, 0.505f) : 0.505f;
+            return rest * needs < 1.0f - needs && !(rd.min_p > 0.0f && rest > rd.min_p);
+        },
+        // the thread's history entries at or above the bound: about what they add to the row's sum, in units of the entry x_top,
+        // and the largest of them, (adjusted key << 32 | ~id); scale = log2(e) / T
+        [&](float bound, float x_top, float scale, unsigned long long* best) SR_INL -> float {
+            float mass = 0.0f;
+            adjust_history();  // (fetched before the row was streamed)
+            const uint32_t bound_key = sr_okey(bound);
+#pragma unroll
+            for (int r = 0; r < kHistRegs; r++) {
+                if (r * kThreads >= ne) continue;  // uniform
+                if (hraw[r] != 0u && hadj[r] >= bound_key) {
+                    mass += __builtin_amdgcn_exp2f(__fmul_rn(__fsub_rn(sr_okey_inv(hadj[r]), x_top), scale));
+                    const unsigned long long cmp = ((unsigned long long)hadj[r] << 32) | (unsigned long long)(0xffffffffu - (uint32_t)hee[r].id);
+                    *best = cmp > *best ? cmp : *best;
+                }
+            }
+            return mass;
+        },
+        // Whether the row's largest entry is the answer: `mass` is at least the sum of the exponentials of everything that can be
+        // among the k best, in units of the entry x_top, `top` the largest entry's own.  See "the largest entry decides".
+        [&](float mass, float top) SR_INL -> bool {
+            // (the k best are added in fp32, 2,048 roundings at most: 1.3e-4; the exponentials here are good to 1e-5)
+            const float least = top / mass * (1.0f - 4e-4f), rest = mass / top * (1.0f + 4e-4f) - 1.0f;  // p_0 >= least, all others' e <= rest
+            const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
+            bool yes = top > 0.0f && mass < 1e30f && least > 0.505f && u_row > 2e-6f && u_row < 1.0f - 4e-6f;
+            if (rd.min_p > 0.0f) yes = yes && rd.min_p < 0.99f && rest < rd.min_p * 0.999f;  // (nothing else survives, nor is near it)
+            if (use_top_p) yes = yes && rd.top_p > 1e-5f && least > rd.top_p;                // (the running sum stops at the first entry)
+            else if (!(rd.min_p > 0.0f)) yes = yes && u_row < least;                         // (all k stay, the draw stops at the first)
+            return yes;
+        },
         sm);
+    if (kDecide && n_c == kDecided) {
+        if (tid == 0 && a.out_flags) a.out_flags[row] = out_flag;  // (its token is written)
+        return;
+    }
     if (SR_RARE(sel > kSelMax || n_c < 0 || n_c > kRowCap)) { give_up(SR_KFLAG_UNSUPPORTED, -1); return; }
 
     SR_PROF(a, 11);
@@ -818,27 +899,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
     } else {
         // ---- no penalties, or penalties that only lower: candidates outside the history + the history ids --
         if (ne > kHistRegs * kThreads) { give_up(SR_KFLAG_UNSUPPORTED, -1); return; }
-        uint32_t hadj[kHistRegs], hraw[kHistRegs];
-#pragma unroll
-        for (int r = 0; r < kHistRegs; r++) {
-            hadj[r] = hraw[r] = 0u;
-            const int e = r * kThreads + tid;
-            if (e < ne) {
-                const SrEdit ee = hee[r];
-                const float x = hx[r];
-                // -inf never enters the reference's selection (Sampler.cs:240-249)
-                if (x == x && sr_f2u(x) != 0xff800000u) {
-                    float v = x;
-                    // Sampler.cs:261-287: pen = pow(rep, occWindow) once; presence/frequency over the whole history
-                    if (ee.occ_all > 0) {
-                        if (rd.rep != 1.0f && ee.occ_win > 0) v = v > 0.0f ? __fdiv_rn(v, ee.pen) : __fmul_rn(v, ee.pen);
-                        v = __fsub_rn(v, __fadd_rn(rd.presence, __fmul_rn(rd.frequency, (float)ee.occ_all)));
-                    }
-                    hraw[r] = sr_okey(x);
-                    hadj[r] = sr_okey(v);
-                }
-            }
-        }
+        adjust_history();
         SR_PROF(a, 5);
         // How far an entry lies below the bins' origin, in 1/56 of a log-unit: -1 = absent or dropped, else
         // 0..1023.  Never increasing with the key, so "bin <= b" is a prefix of the descending order.
@@ -1372,11 +1433,11 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
 // force_exact, and any row whose candidates overflow the lists: the row's sel-th largest kept element is found by a
 // radix select over the logits themselves, and the candidates are exactly the sel largest in (value desc, index asc)
 // order.  Slow (several passes over the row), exact for any data, and independent of the chunk results.
-template <int EPV, int kVec, bool kKept, bool kShort, bool kFold, typename Early, typename Late>
+template <int EPV, int kVec, bool kKept, bool kShort, bool kFold, bool kDecide, typename Early, typename Late, typename Ask, typename HistMass, typename Decide>
 __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, int row, const SrRow& rd, bool want_bins,
                                                 bool force_exact, float inv_temp, BinMap* map_out,
                                                 float* bound_out, bool* binned, const KeptGroups& kept, Early&& early,
-                                                Late&& late, TopkSmem& sm)
+                                                Late&& late, Ask&& worth_asking, HistMass&& hist_mass, Decide&& decide, TopkSmem& sm)
 {
     *binned = false;
     *map_out = BinMap{};
@@ -1707,6 +1768,7 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
     // The chunk workgroups' waves each left a value with their share of sel group maxima at or above it: the
     // smallest of them has at least sel group maxima of the row at or above it.
     float tval = -3.402823466e38f;
+    uint32_t row_max;  // the row's largest kept element
     {
         uint32_t k = 0xffffffffu, km = 0u;
         if constexpr (kKept) {
@@ -1738,6 +1800,7 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
         const int share = !kKept && kShort && nb <= SR_WAVE ? max((sel + nb - 1) / nb, 2) : (sel + nb - 1) / nb;
         const uint32_t km_lane = km;
         km = sr_wave_max_u32(km);
+        row_max = km;
         if (kShort && nb <= SR_WAVE && share <= 2) {
             const bool in = lane < nb;
             k_close = largest_key16(km, [&](uint32_t cnd) SR_INL -> bool {
@@ -1774,12 +1837,11 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
     }
     late();
     SR_PROF(a, 1);
-    uint32_t mq1 = 0u, base_a = 0u;
+    uint32_t mq1 = 0u, mq2 = 0u, base_a = 0u;
     if (direct) {
         // The thread's 16 groups as two bit masks -- largest element at or above the bound with the second largest
         // below it (handed over directly), second largest at or above it (listed, fetched below) --, one
         // reservation per wave and list, then every lane places its own.
-        uint32_t mq2 = 0u;
 #pragma unroll
         for (int c = 0; c < kG2Regs; c++) {
             if (c < S) {
@@ -1827,25 +1889,91 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
     __syncthreads();
     const int n_q = (int)sm.bcast[13];
     SR_PROF(a, 2);
-    // The largest element of every group with one element at or above the bound, picked out of the thread's registers
-    // by the bit number and handed over as it is.  Selects written as mask arithmetic: as conditionals the compiler
-    // may turn them into branches.
+    // An entry out of the thread's registers by its group's bit number.  Selects written as mask arithmetic: as conditionals
+    // the compiler may turn them into branches.
+    auto sel2 = [](uint32_t x0, uint32_t x1, int bit) SR_INL -> uint32_t {
+        const uint32_t m = 0u - (uint32_t)(bit & 1);
+        return (x0 & ~m) | (x1 & m);
+    };
+    auto pick4 = [&](const float4& v, int g) SR_INL -> uint32_t {
+        return sel2(sel2(sr_f2u(v.x), sr_f2u(v.y), g), sel2(sr_f2u(v.z), sr_f2u(v.w), g), g >> 1);
+    };
+    auto pick16 = [&](const float4 (&v)[4], int bit) SR_INL -> float {
+        const int c = bit >> 2, g = bit & 3;
+        return sr_u2f(sel2(sel2(pick4(v[0], g), pick4(v[1], g), c), sel2(pick4(v[2], g), pick4(v[3], g), c), c >> 1));
+    };
+    if constexpr (kDecide) {
+        // (a step of its own, which rows that do not take it do not pay for)
+        constexpr int kGroup = kFoldPos<EPV, kVec> * (kFold ? 2 : 1);  // most elements of a group
+        const float scale = __fmul_rn(inv_temp, 1.44269504f), x_top = sr_okey_inv(row_max);
+        // an entry's exponential in units of the largest one's
+        auto weight = [&](float x) SR_INL -> float { return __builtin_amdgcn_exp2f(__fmul_rn(__fsub_rn(x, x_top), scale)); };
+        // (sel entries at the bound say for most flat rows that there is nothing to ask)
+        if (direct && want_bins && row_max > kKeyNegInf && worth_asking((float)(sel - 1) * weight(tval))) {
+            // (all of a chunk's groups at once, and one exponential for the lane's second ones: walking the set bits, as the lists are made, took
+            // 2.5 us where hundreds are at the bound)
+            float mass = 0.0f, second = SR_NEG_INF;
+#pragma unroll
+            for (int c = 0; c < kG2Regs; c++) {
+                const uint32_t at = ((mq1 | mq2) >> (4 * c)) & 15u;
+                if (__ballot(at != 0u) == 0ull) continue;
+                const float m1[4] = {gmr[c].x, gmr[c].y, gmr[c].z, gmr[c].w};
+#pragma unroll
+                for (int g = 0; g < 4; g++) mass += ((at >> g) & 1u) != 0u ? weight(m1[g]) : 0.0f;
+                second = fmaxf(fmaxf(second, fmaxf(g2r[c].x, g2r[c].y)), fmaxf(g2r[c].z, g2r[c].w));
+            }
+            mass += mq2 != 0u ? (float)(__popc(mq2) * (kGroup - 1)) * weight(second) : 0.0f;
+            unsigned long long best = 0ull;
+            if (rd.edit_cnt > 0) {
+                mass += hist_mass(tval, x_top, scale, &best);
+                best = sr_wave_max_u64(best);
+            }
+            mass = sr_wave_sum_f32(mass);
+            if (lane == 0) {
+                sm.hist[64 + (tid >> 6)] = sr_f2u(mass);
+                sm.hist[80 + 2 * (tid >> 6)] = (uint32_t)best;
+                sm.hist[81 + 2 * (tid >> 6)] = (uint32_t)(best >> 32);
+            }
+            __syncthreads();
+            mass = 0.0f;
+            best = 0ull;
+#pragma unroll
+            for (int w = 0; w < kWaves; w++) mass += sr_u2f(sm.hist[64 + w]);
+            if (rd.edit_cnt > 0) {
+#pragma unroll
+                for (int w = 0; w < kWaves; w++) {
+                    const unsigned long long b = ((unsigned long long)sm.hist[81 + 2 * w] << 32) | (unsigned long long)sm.hist[80 + 2 * w];
+                    best = b > best ? b : best;
+                }
+            }
+            const uint32_t hist_top = (uint32_t)(best >> 32);
+            if (decide(mass, hist_top > row_max ? weight(sr_okey_inv(hist_top)) : 1.0f)) {
+                if (hist_top > row_max) {
+                    if (tid == 0) a.out_tokens[row] = (int)(0xffffffffu - (uint32_t)best);
+                } else {
+                    // (the only entry of its value: one group of one thread)
+#pragma unroll
+                    for (int c = 0; c < kG2Regs; c++) {
+                        const float m1[4] = {gmr[c].x, gmr[c].y, gmr[c].z, gmr[c].w};
+#pragma unroll
+                        for (int g = 0; g < 4; g++)
+                            if (c < S && sr_okey(m1[g]) == row_max) a.out_tokens[row] = idx_of(c, g, (gpr[c] >> (8 * g)) & 0xffu);
+                    }
+                }
+                return kDecided;
+            }
+        }
+    }
+    // The largest element of every group with one element at or above the bound, handed over as it is.
     auto hand_over_direct = [&]() SR_INL {
-        auto sel = [](uint32_t x0, uint32_t x1, int bit) SR_INL -> uint32_t {
-            const uint32_t m = 0u - (uint32_t)(bit & 1);
-            return (x0 & ~m) | (x1 & m);
-        };
-        auto pick4 = [&](const float4& v, int g) SR_INL -> uint32_t {
-            return sel(sel(sr_f2u(v.x), sr_f2u(v.y), g), sel(sr_f2u(v.z), sr_f2u(v.w), g), g >> 1);
-        };
         uint32_t m = mq1, pos = base_a;
         while (__ballot(m != 0u) != 0ull) {
             const bool on = m != 0u;
             const int bit = on ? __ffs((int)m) - 1 : 0;
             m &= m - 1u;
             const int c = bit >> 2, g = bit & 3;
-            const float x = sr_u2f(sel(sel(pick4(gmr[0], g), pick4(gmr[1], g), c), sel(pick4(gmr[2], g), pick4(gmr[3], g), c), c >> 1));
-            const uint32_t gp = sel(sel(gpr[0], gpr[1], c), sel(gpr[2], gpr[3], c), c >> 1);
+            const float x = sr_u2f(sel2(sel2(pick4(gmr[0], g), pick4(gmr[1], g), c), sel2(pick4(gmr[2], g), pick4(gmr[3], g), c), c >> 1));
+            const uint32_t gp = sel2(sel2(gpr[0], gpr[1], c), sel2(gpr[2], gpr[3], c), c >> 1);
             if (on) place(pos++, x, idx_of(c, g, (gp >> (8 * g)) & 0xffu));
         }
     };
@@ -1994,9 +2122,14 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
             kept.g2[c] = kept.g1[c];
             kept.gp[c] = 0u;
         }
-        // the row to finish is known from the start: its descriptor, and the history ids with their logits, are
-        // fetched now and wait in registers while the row streams
-        if (prog.z >= 0) {
+    }
+    // The row to finish is known from the start: its descriptor, and the history ids with their logits, are fetched while the first
+    // vectors come in, and wait in registers while the row streams.  (In front of the first vectors, four trips to memory that the stream
+    // waits for, 256 rows of 151,936 bf16 took 27.4 us, 26.4 so, of fp32 with a history of 64 38.8 and 38.6.  Dealt rows with short lists, whose workers
+    // stream a chunk or two, lose by it: 64 rows of 49,152 13.5 and 14.3.)
+    auto fetch_row = [&]() SR_INL {
+        if constexpr (kHistBefore<kKept, kRoomy>) {
+            if (prog.z < 0) return;
             typedef const int __attribute__((address_space(4))) const_i32;
             trow = ((const_i32*)(uintptr_t)a.sel_list)[prog.z];
             trd = load_row_uniform(a.rows + trow);
@@ -2009,7 +2142,9 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
                 kept_hist.hx[r] = in ? row_logit(a, trow, trd, kept_hist.hee[r].id) : SR_NEG_INF;
             }
         }
-    }
+    };
+    constexpr bool kFetchFirst = kShort && !kKept;
+    if (kFetchFirst || n_items <= 0) fetch_row();
     if (n_items > 0) {
         const i32x4 info = q[0];  // (chunk | launch slot of the row, batch row, scan-mask row, sel)
         Geom cur = geom(info);
@@ -2030,6 +2165,7 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
         u32x4 t[kWin];
 #pragma unroll
         for (int j = 0; j < kWin; j++) t[j] = load_vec(cur, j);
+        if (!kFetchFirst) fetch_row();
 
         // One chunk per turn.  Behind the worker's last chunk the registers are refilled from that chunk's first
         // vector, to no effect (one line, already in cache), so that the loop body is the same for every chunk: with
@@ -2241,8 +2377,12 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
     // ---- the row tail
     const int tslot = prog.z;
     if constexpr (!kKept) {
-        trow = a.sel_list[tslot];
-        trd = a.rows[trow];
+        // (the descriptor is read once more where the history was fetched by it: kept in scalar registers over the streaming it
+        // costs the tail hundreds of moves out of vector registers)
+        const SrRow* rows = a.rows;
+        asm volatile("" : "+s"(rows));
+        if constexpr (!kHistBefore<kKept, kRoomy>) trow = a.sel_list[tslot];
+        trd = rows[trow];
     }
 #ifdef SR_PROFILE
     SrTopkArgs ap = a;
@@ -2276,7 +2416,7 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
     }
     SR_PROF(ap, 4);
     __builtin_amdgcn_s_setprio(3);  // the tail is the longer dependent chain: its waves go first
-    topk_row_tail<EPV, kVec, kKept, kShort, kFold>(ap, tslot, trow, trd, !handed_over, kept, kept_hist, sm);
+    topk_row_tail<EPV, kVec, kKept, kShort, kRoomy, kFold>(ap, tslot, trow, trd, !handed_over, kept, kept_hist, sm);
     SR_PROF(ap, 15);
 }
 

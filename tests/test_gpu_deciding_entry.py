@@ -1,0 +1,87 @@
+"""Rows whose largest entry decides the token: around the lines where it just does and just does not, in every shape of the
+launch that asks.  Tokens are the oracle's, and tokens and flags those of the way that never asks (forced from the host: a poll limit
+of zero for the kernels' bounded waits)."""
+
+import numpy as np
+import pytest
+from opentail.stingray_amd import SamplerContext, SamplingParams, synthetic
+from tests.helpers import hooks_lib, oracle_tokens
+
+pytestmark = pytest.mark.gpu
+CHUNK = 512 * 19 * 4  # elements of a worker's chunk of fp32 logits
+
+
+@pytest.fixture()
+def ctx():
+    c = SamplerContext(0)
+    yield c
+    c.close()
+
+
+def _rows(rng, rows, vocab, top_k, bf16):
+    """Rows with one entry well above the rest: `gap` nats above all others that count together.  top-p, min-p and the uniform lie on both
+    sides of what that entry covers, some within a few roundings of it."""
+    logits = rng.normal(0, 1, (rows, vocab)).astype(np.float32)
+    params, u = [], rng.random(rows)
+    for r in range(rows):
+        k = int(rng.integers(2, top_k + 1)) if top_k else 0
+        t = float(np.float32(rng.uniform(0.4, 1.3)))
+        x = np.sort(logits[r].astype(np.float64))[::-1][: k - 1 if k else None] / t
+        rest = x[0] + np.log(np.exp(x - x[0]).sum())
+        gap = rng.uniform(-1.0, 7.0)
+        at = int(rng.choice([0, vocab - 1, int(rng.integers(vocab))]))
+        raised = 0.0
+        p = SamplingParams(Temperature=t, TopK=k)
+        if r % 3 == 1:  # the entry is in the history, and what the penalty takes away was added
+            p.PresencePenalty, p.FrequencyPenalty = 0.25, 0.125
+            p.PreviousTokens = rng.integers(0, vocab, 40).tolist() + ([at] * 3 if r % 2 else [])
+            raised = 0.25 + 0.125 * p.PreviousTokens.count(at) if at in p.PreviousTokens else 0.0
+        logits[r, at] = np.float32((rest + gap) * t + raised)
+        covers = 1.0 / (1.0 + np.exp(-gap))
+        near = covers * (1.0 + float(rng.choice([-1e-2, -1e-3, -2e-4, -1e-6, 0.0, 1e-6, 1e-3])))
+        kind = r % 4
+        if kind == 0:
+            p.TopP = float(np.float32(min(near, 0.9999)))
+        elif kind == 1:
+            p.MinP = float(np.float32(np.exp(x[0] - rest - gap) * rng.choice([0.5, 1.0, 1.001, 2.0, 50.0])))
+            p.TopP = float(rng.choice([1.0, 0.9]))
+        elif kind == 2:
+            u[r] = min(near, 0.9999999)
+        if r % 7 == 3:
+            u[r] = rng.choice([0.0, 1e-7, 1e-6, 0.9999995, 0.99999997])
+        if r % 11 == 5:
+            logits[r, (at + vocab // 2) % vocab] = logits[r, at]  # not the only one
+        params.append(p)
+    if bf16:
+        logits = synthetic.bf16_bits_to_f32(synthetic.to_bf16_bits(logits))
+    return logits, params, u
+
+
+def _check(ctx, rng, rows, vocab, top_k, bf16, rounds):
+    import torch
+
+    h = hooks_lib()
+    for _ in range(rounds):
+        logits, params, u = _rows(rng, rows, vocab, top_k, bf16)
+        dev = torch.from_numpy(logits).cuda()
+        if bf16:
+            dev = dev.to(torch.bfloat16)
+        got, flags = ctx.sample_batch(dev, params, u, return_flags=True)
+        want = oracle_tokens(logits, params, u)
+        assert np.array_equal(got, want), np.nonzero(got != want)[0][:10]
+        h.sr_debug_set_spin_limit(ctx.h, 0)
+        h.sr_debug_set_row_wait_limit(ctx.h, 0)
+        other, other_flags = ctx.sample_batch(dev, params, u, return_flags=True)
+        h.sr_debug_set_spin_limit(ctx.h, 1 << 22)
+        h.sr_debug_set_row_wait_limit(ctx.h, 1 << 15)
+        assert np.array_equal(got, other)
+        assert np.array_equal(flags, other_flags), np.nonzero(flags != other_flags)[0][:10]
+
+
+# Dealt rows of one and of several chunks, short and long lists; chunks that join in pairs; a row to a worker; two workers to a
+# compute unit; more of them than that.
+@pytest.mark.parametrize("rows,vocab,top_k,bf16", [
+    (1, 49_152, 40, False), (9, 4 * CHUNK - 1, 64, False), (24, 100_003, 300, True), (7, 6 * CHUNK + 3, 500, False), (5, 5 * CHUNK, 64, False),
+    (20, 12_345, 50, False), (270, 9_001, 900, False), (300, 20_011, 60, True), (530, 16_384, 200, False), (260, 4 * CHUNK + 9, 100, False)])
+def test_rows_that_their_largest_entry_decides(ctx, rows, vocab, top_k, bf16):
+    _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, top_k, bf16, 12 if rows < 10 else 3 if rows < 100 else 1)
