@@ -1554,6 +1554,12 @@ __device__ __forceinline__ void seg_apply_edits(const SrFullArgs& a, const SrRow
 // whose sums were written through, waited for, counted and read, 4.1 and 2.6, 2.2 and 1.5, 2.8 and 2.0.  Of calls, where the slowest
 // workgroup is waited for either way: 16 rows of 262,144 fp32 with distributions 65.0 -> 63.4, 32 ragged bf16 rows of 100,003 52.0 -> 50.8, 64
 // penalised rows of 151,936 41.15 -> 40.7.
+// Where tokens are all that is asked for, the first meeting also has about the sum of the row's exponentials, relative to its largest: fast
+// ones of the logits in the registers, a dozen cycles each.  With it a row whose largest entry decides (row_decided) is done there -- no e, no
+// records, no list, nothing for the launches behind --, and any other row that is not cut by its mass needs no second meeting.  us a call,
+// before -> now, rows whose largest entry stands out and flat ones (N(0, 1.5^2)): 64 rows of 151,936 under min-p 37.6 -> 14.7 and 49.4 -> 48.5, 16
+// of them 28.2 -> 10.8 and 40.1 -> 36.0; 32 bf16 rows of 100,003 under top-p 30.2 -> 13.1 and 680 -> 684, that nothing cuts 50.4 -> 13.1 and 47.5 ->
+// 47.2; one row of 151,936 38.3 -> 13.3 and 39.5 -> 37.8, 64 83.7 -> 50.9 (one of them open) and 82.1 -> 80.4.
 //
 // What bounds it: the vector units (the double-precision expf is 30 instructions an element).  The first pass used to
 // take a fast exponential of every element, for approximate sums relative to the segment's own maximum, to save the second
@@ -1621,6 +1627,28 @@ __device__ __forceinline__ uint32_t mass_list_from(const float (&v)[4], float sh
 __device__ __forceinline__ uint32_t min_p_list_from(const SrRow& rd)
 {
     return rd.min_p >= 1e-30f ? sr_f2u(__fmul_rn(rd.min_p, 1.0f - 2.0f * SR_AMBIG_REL - 1e-6f)) : 0u;
+}
+
+constexpr float kLog2E = 0x1.715476p+0f;
+// Whether a row's largest entry, e = 1, is its token: its nucleus is that entry alone, or, in a row that nothing cuts, the draw lands
+// on it.  all: about the sum of the row's e, front: of what stands in front of the workgroup that holds the largest, own: of what that one holds
+// (fast exponentials: 2e-5 at most).  The exact sums go one by one in fp32 and end near these: an addition is off by 2^-24 of the sum at most, and by the
+// smaller of its two operands at most, so n of them by n 2^-24 of the sum and by the mass beside the largest entry, whichever is less; the eight
+// accumulators of the final Normalize by n / 8 + 200 roundings.  What lies nearer to a line than that is not decided here, nor is anything that
+// could count as ambiguous: draws at either end, cuts beside the threshold, a largest entry that is not the only one (it covers more than half).
+__device__ __forceinline__ bool row_decided(const SrRow& rd, int n, float all, float front, float own, float u)
+{
+    const float by_n = (float)n * 6.3e-8f, beside = fmaxf(all - 1.0f, 0.0f) + 4e-5f * all;
+    const float least = (1.0f - 1e-5f) / (all * (1.0f + 4e-5f) + fminf(all * by_n, beside));  // its probability is at least this
+    const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f, use_min_p = rd.min_p > 0.0f;
+    bool yes = all < 1e30f && least > 0.505f && u > 2e-6f && u < 1.0f - 4e-6f;
+    if (use_min_p) yes = yes && rd.min_p < 0.99f && beside < 0.999f * rd.min_p;  // (nothing else survives)
+    if (use_top_p) yes = yes && rd.top_p > 1e-5f && least > rd.top_p;            // (the running sum stops at the first)
+    if (!use_top_p && !use_min_p) {
+        const float inv = 1.0f / all, off = fminf(by_n, beside * inv) * 1.05f + ((float)(n / 8) + 200.0f) * 6.6e-8f + 8e-5f;
+        yes = yes && u > (front + fmaxf(own - 1.0f, 0.0f)) * inv + off && u < (front + 1.0f) * inv - off;
+    }
+    return yes;
 }
 
 // A greedy row that rides along (SrFullArgs::n_greedy): the largest of its masked logits, the first by index among equals, NaN left
@@ -1701,7 +1729,9 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     __shared__ float mass_rest;              // ... of its last bucket
     __shared__ float chains[kS][SR_SEQ_CHAINS];
     __shared__ uint32_t wkey[kW];
-    __shared__ uint32_t bc[2];            // 0: the row's count came in   1: the row's maximum
+    __shared__ float wsum[kW];
+    // 0: the row's words came in, and 2: its largest entry decides   1: the row's maximum   2: about the sum of e in front of the workgroup
+    __shared__ uint32_t bc[3];
     // the row's edits that fall into this workgroup's segments (id << 32 | place in the row's edit list), and how many
     // there are (more than the list holds: the waves go through the row's whole edit list instead)
     constexpr int kHitCap = 256;
@@ -1714,7 +1744,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     const int n = a.vocab, nseg = seg_count(n);
     SrFullState* st = a.state + slot;
     const unsigned long long stamp = (unsigned long long)a.seq << 32;
-    unsigned long long* const met_max = a.meet + (size_t)slot * a.meet_stride;  // a word per workgroup
+    unsigned long long* const met_max = a.meet + (size_t)slot * a.meet_stride;  // two words per workgroup
     unsigned long long* const met_sum = met_max + a.meet_sums;                  // ... and per segment
     SeqSegFunc* recs = a.seg_func + (size_t)slot * a.seg_stride;
     float* sums = a.seg_sum + (size_t)slot * a.seg_stride;
@@ -1729,6 +1759,8 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     const bool by_mass = listed && use_top_p && !(rd.min_p > 0.0f);
     const bool by_count = listed && !by_mass && a.mode != 0;
     const uint32_t min_p_from = max(min_p_list_from(rd), 1u);
+    // a row whose token is all that is asked for: its largest entry may decide
+    const bool asks = kLists && a.mode == 0 && !(rd.top_k > 0 && rd.top_k < n);
     // (the row's sum is at least 1: n entries below this make up less than half of what top-p leaves out)
     const float mass_min = (1.0f - rd.top_p) * 0.5f / (float)n;
     if (by_mass || by_count) {
@@ -1788,38 +1820,115 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
                     }
                 }, t[s]);
     }
+    double u_row = 0.0;  // (behind the logits: it may come over the bus)
+    if (asks && wave == 0) u_row = a.uniforms[(size_t)row * a.uniforms_per_row];
     uint32_t k = 0u;
 #pragma unroll
     for (int s = 0; s < kS; s++)
         if (seg0 + s * kW < nseg) k = max(k, seg_max_key(t[s]));
     k = sr_wave_max_u32(k);
     if (lane == 0) wkey[wave] = k;
-    sr_barrier_lds();
-    // The first meeting: a word of every workgroup, its largest logit below the launch's number, which all of the row's
-    // workgroups read until it is this launch's.
-    if (wave == 0) {
-        k = wkey[0];
+    if (asks) {
+        // about the sum of the wave's exponentials, relative to the wave's largest
+        float sum = 0.0f;
+        if (k > 0x007fffffu && k < kKeyInf) {
+            const float mw = sr_okey_inv(k);
 #pragma unroll
-        for (int j = 1; j < kW; j++) k = max(k, wkey[j]);
-        if (lane == 0) sr_store_agent(met_max + blockIdx.x, stamp | (unsigned long long)k);
+            for (int s = 0; s < kS; s++)
+                if (seg0 + s * kW < nseg)
+#pragma unroll
+                    for (int j = 0; j < SR_SEQ_RUN; j++) {
+                        sum += __builtin_amdgcn_exp2f((t[s][j] - mw) * kLog2E);
+                        if (j % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (a few at a time: the registers are the segments')
+                    }
+            sum = sr_wave_sum_f32(sum);
+        }
+        if (lane == 0) wsum[wave] = sum;
+    }
+    sr_barrier_lds();
+    // The first meeting: every workgroup's largest logit, and where the row asks about the sum of its exponentials relative to that, each
+    // in a word below the launch's number, which all of the row's workgroups read until it is this launch's.
+    auto about = [](uint32_t key, float sum, float m) __attribute__((always_inline)) -> float {
+        return key > 0x007fffffu ? sum * __builtin_amdgcn_exp2f((sr_okey_inv(key) - m) * kLog2E) : 0.0f;
+    };
+    uint32_t k_group = wkey[0];
+#pragma unroll
+    for (int j = 1; j < kW; j++) k_group = max(k_group, wkey[j]);
+    if (wave == 0) {
+        float sum = 0.0f;
+        if (asks) {
+            const float m = sr_okey_inv(k_group);
+#pragma unroll
+            for (int j = 0; j < kW; j++) sum += about(wkey[j], wsum[j], m);
+        }
+        if (lane == 0) {
+            sr_store_agent(met_max + 2 * blockIdx.x, stamp | (unsigned long long)k_group);
+            if (asks) sr_store_agent(met_max + 2 * blockIdx.x + 1, stamp | (unsigned long long)sr_f2u(sum));
+        }
+    }
+    // where the workgroup's largest logit is, should it be the row's token: found while the words are under way
+    int top_at = -1;
+    if (asks && k == k_group) {
+        const float mg = sr_okey_inv(k);
+#pragma unroll
+        for (int s = 0; s < kS; s++)
+            if (seg0 + s * kW < nseg)
+#pragma unroll
+                for (int j = 0; j < SR_SEQ_RUN; j++) top_at = t[s][j] == mg ? s * SR_SEQ_RUN + j : top_at;
+    }
+    if (wave == 0) {
+        constexpr int kWords = SR_SEG_MAX / (kW * kS) / SR_WAVE > 0 ? SR_SEG_MAX / (kW * kS) / SR_WAVE : 1;  // a lane, of each kind
+        k = k_group;
         bool here = true;
-        for (int g0 = 0; g0 < (int)gridDim.x; g0 += SR_WAVE) {
-            if (g0 + lane >= (int)gridDim.x) break;
-            unsigned long long v = 0ull;
+        uint32_t key[kWords];
+        float part[kWords];
+#pragma unroll
+        for (int w = 0; w < kWords; w++) {
+            const int g = w * SR_WAVE + lane;
+            key[w] = 0u;
+            part[w] = 0.0f;
+            if (g >= (int)gridDim.x) continue;
             bool in = false;
             for (uint32_t it = 0; it < a.row_wait_limit; it++) {
-                v = sr_load_agent(met_max + g0 + lane);
-                if ((uint32_t)(v >> 32) == a.seq) { in = true; break; }
+                const unsigned long long v = sr_load_agent(met_max + 2 * g), e = asks ? sr_load_agent(met_max + 2 * g + 1) : v;
+                key[w] = (uint32_t)v;
+                part[w] = sr_u2f((uint32_t)e);
+                if ((uint32_t)(v >> 32) == a.seq && (uint32_t)(e >> 32) == a.seq) { in = true; break; }
                 __builtin_amdgcn_s_sleep(1);
             }
             here = here && in;
-            k = max(k, (uint32_t)v);
+            k = max(k, key[w]);
         }
         here = __ballot(!here) == 0ull;
         k = sr_wave_max_u32(k);
+        bool decided = false;
+        float before = 0.0f;
+        if (asks && here && k > 0x007fffffu && k < kKeyInf) {
+            const float m = sr_okey_inv(k);
+            float all = 0.0f;
+            int first = (int)gridDim.x;  // the workgroup that holds the largest entry
+#pragma unroll
+            for (int w = kWords - 1; w >= 0; w--) {
+                part[w] = about(key[w], part[w], m);
+                const unsigned long long top = __ballot(key[w] == k);
+                if (top != 0ull) first = w * SR_WAVE + (int)__ffsll((long long)top) - 1;
+            }
+            float front = 0.0f, own = 0.0f;
+#pragma unroll
+            for (int w = 0; w < kWords; w++) {
+                const int g = w * SR_WAVE + lane;
+                all += part[w];
+                before += g < (int)blockIdx.x ? part[w] : 0.0f;
+                front += g < first ? part[w] : 0.0f;
+                own += g == first ? part[w] : 0.0f;
+            }
+            before = sr_wave_sum_f32(before);
+            decided = row_decided(rd, n, sr_wave_sum_f32(all), sr_wave_sum_f32(front), sr_wave_sum_f32(own), __double2float_rn(u_row));
+        }
         if (lane == 0) {
-            bc[0] = here ? 1u : 0u;
+            bc[0] = here ? (decided ? 2u : 1u) : 0u;
             bc[1] = k;
+            bc[2] = sr_f2u(before);
             // the wait ran out: the row is left to its own workgroup
             if (!here) sr_store_agent(&st->late, a.seq);
             else if (blockIdx.x == 0) st->maxkey = full_maxkey(a, k);
@@ -1839,6 +1948,16 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     // stands: the row's workgroup takes the row alone, so that every x - max below is at most 0, or -inf.
     if (mk >= kKeyInf || mk <= 0x007fffffu) return;
     const float m = sr_okey_inv(mk);
+    if (asks && bc[0] == 2u) {
+        if (wkey[wave] == mk) {
+            if (top_at >= 0) a.out_tokens[row] = seg_elem<E>(seg0 + top_at / SR_SEQ_RUN * kW, lane, top_at % SR_SEQ_RUN);  // (the only one of its value)
+            if (lane == 0) {
+                if (a.out_flags) a.out_flags[row] = SR_KFLAG_FULL;
+                st->decided = a.seq;
+            }
+        }
+        return;
+    }
 
     // e of the wave's segments: written to the row, counted by size, and turned into the order of the sum
     float own[kS];
@@ -1945,8 +2064,15 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
         sr_drain_stores();
         __syncthreads();
     }
-    // The second one: a word of every segment, its sum.
-    if (lane == 0) {
+    // The second one: a word of every segment, its sum -- but where the first has told all there is to ask.
+    const bool meets = !asks || by_mass;
+    if (!meets) {
+        if (lane == 0) {
+#pragma unroll
+            for (int s = 0; s < kS; s++)
+                if (seg0 + s * kW < nseg) share[s * kW + wave] = sums[seg0 + s * kW] = own[s];
+        }
+    } else if (lane == 0) {
 #pragma unroll
         for (int s = 0; s < kS; s++)
             if (seg0 + s * kW < nseg) {
@@ -1954,7 +2080,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
                 sums[seg0 + s * kW] = own[s];  // (for the launches behind)
             }
     }
-    for (int g = threadIdx.x; g < nseg; g += kThreads) {
+    for (int g = meets ? (int)threadIdx.x : nseg; g < nseg; g += kThreads) {
         unsigned long long v = 0ull;
         bool in = false;
         for (uint32_t it = 0; it < a.row_wait_limit; it++) {
@@ -2004,8 +2130,9 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
         const int seg = seg0 + s * kW;
         if (seg >= nseg) continue;
         float before = 0.0f;
-        for (int g = lane; g < seg; g += SR_WAVE) before += share[g];
+        for (int g = lane; g < (meets ? seg : s * kW + wave); g += SR_WAVE) before += share[g];
         before = sr_wave_sum_f32(before);
+        if (!meets) before += sr_u2f(bc[2]);
         seg_make_record(t[s], seg, (double)before, recs + seg, own[s]);
         if (too_long) {
             if (a.mode != 0) {  // (what is left of the row's last four, k_full_row copies)
@@ -3364,8 +3491,9 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     SrFullState* st = a.state + slot;
     // What does not hang on the row's descriptor is asked for beside it: the row's state, the first records of its sum (by the
     // wave that will walk them) and how many entries its segments have listed (by the others).
-    const uint32_t st_late = st->late, st_list_from = st->list_from;
+    const uint32_t st_late = st->late, st_list_from = st->list_from, st_decided = st->decided;
     const unsigned long long st_maxkey = st->maxkey;
+    if (st_decided == a.seq && st_late != a.seq) return;
     SegRec first64 = {};
     constexpr int kCntAhead = 4;
     int cnt_ahead[kCntAhead] = {};
@@ -4803,7 +4931,6 @@ constexpr int kSpecDone = -2;  // SrSpecArgs::reject of a row whose results are 
 // those of k_prepared_row and of the greedy rows: other launches of the context find these as they left them.)
 constexpr int kOpenFirst = 4, kOpenSecond = 5;
 constexpr int kUnitVecs = SR_UNIT_TERMS / (4 * SR_WAVE);
-constexpr float kLog2E = 0x1.715476p+0f;
 __global__ __launch_bounds__(256) void k_spec_units(SrFullArgs a, SrSpecArgs s)
 {
     const int slot = blockIdx.y, lane = sr_lane(), u = (int)blockIdx.x * 4 + sr_wave_id(), n = s.vocab;

@@ -152,7 +152,7 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             SR_HIP(ctx, ctx->full_mass.reserve((size_t)n_rows * 256 * sizeof(float), st, true));
             SR_HIP(ctx, ctx->full_row_sync.reserve((size_t)(n_rows + n_greedy) * SR_ROW_SYNC_STRIDE * sizeof(unsigned long long), st, true));
             a.row_sync = ctx->full_row_sync.as<unsigned long long>();
-            a.meet_sums = (half_blocks + 15) & ~15;
+            a.meet_sums = (2 * half_blocks + 15) & ~15;
             a.meet_stride = (a.meet_sums + nseg + 15) & ~15;
             SR_HIP(ctx, ctx->full_meet.reserve((size_t)n_rows * (size_t)a.meet_stride * sizeof(unsigned long long), st, true));
             a.meet = ctx->full_meet.as<unsigned long long>();

@@ -148,7 +148,8 @@ struct SrFullState {
     uint32_t late_behind; // the number of the last launch in which a workgroup of k_prepared_row stopped waiting for the row's others
     float u;              // the uniform of the draw, of a row left to the whole device
     uint32_t e_open;      // the number of the last launch that did not write the row's e down: its reader takes it from the logits
-    int32_t pad[2];
+    uint32_t decided;     // the number of the last launch in which k_full_softmax_seg found the row's token
+    int32_t pad;
 };
 static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // SrFullArgs::row_sync, a word per row (rows 256 bytes apart: every workgroup of a row adds to its word and polls it):
@@ -216,7 +217,8 @@ struct SrFullArgs {
                                    // need no table either (k_full_softmax_seg applies their edits where it loads the row)
     unsigned long long* row_sync;  // [slot * SR_ROW_SYNC_STRIDE]
     // [slot * meet_stride] what k_full_softmax_seg's workgroups leave for each other, the launch's number << 32 above every word (so nothing
-    // clears them between launches): a workgroup's largest logit as an ordered key, and from meet_sums on a segment's sum of e
+    // clears them between launches): a workgroup's largest logit as an ordered key and about the sum of its exponentials relative to that, and from
+    // meet_sums on a segment's sum of e
     unsigned long long* meet;
     int32_t meet_stride, meet_sums;
     uint32_t row_wait_limit;       // polls of a row's count before a workgroup of k_full_softmax_seg stops waiting for it

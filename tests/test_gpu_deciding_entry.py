@@ -85,3 +85,10 @@ def _check(ctx, rng, rows, vocab, top_k, bf16, rounds):
     (20, 12_345, 50, False), (270, 9_001, 900, False), (300, 20_011, 60, True), (530, 16_384, 200, False), (260, 4 * CHUNK + 9, 100, False)])
 def test_rows_that_their_largest_entry_decides(ctx, rows, vocab, top_k, bf16):
     _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, top_k, bf16, 12 if rows < 10 else 3 if rows < 100 else 1)
+
+
+# The full-vocabulary path: one, two and four segments a wave, rows that end inside a segment, rows of odd addresses, several turns of workgroups.
+@pytest.mark.parametrize("rows,vocab,bf16", [(1, 4_096, False), (3, 5_001, False), (30, 100_003, True), (33, 100_003, False), (6, 262_144, False),
+                                             (66, 200_064, False), (40, 50_257, True), (280, 16_385, False)])
+def test_rows_of_the_whole_vocabulary_that_their_largest_entry_decides(ctx, rows, vocab, bf16):
+    _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, 0, bf16, 8 if rows < 10 else 2 if rows < 50 else 1)
