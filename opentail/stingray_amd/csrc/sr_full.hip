@@ -457,7 +457,7 @@ __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSeg
                 // starts and ends in its own)
                 const unsigned long long ok = __ballot(eb1 == eb) & __ballot(b1 < sr_state_bits(1u << 24, eb)) & __ballot(b2 >= lo2) & __ballot(b3 - lo2 < size2);
                 const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)b3, t);
-                if (((ok >> t) & 1ull) == 0ull || n >= (1u << 24)) {
+                if (SR_RARE(((ok >> t) & 1ull) == 0ull || n >= (1u << 24))) {
                     fix = n >= (1u << 24) ? -1 : t;  // (-1: a segment in front of this one left its binade unforeseen)
                     break;
                 }
@@ -467,7 +467,7 @@ __device__ __forceinline__ float seg_walk_from(Load load, int nseg, const SeqSeg
             }
             if (fix < 0) {
                 const unsigned long long bad = __ballot(simple && lane >= pos && (eb1 != ebv || pre + T >= (1u << 24)));
-                if (bad == 0ull) break;
+                if (SR_USUAL(bad == 0ull)) break;
                 // (everything in front of this segment is exact)
                 fix = (int)__ffsll((long long)bad) - 1;
                 pos = fix + 1;
@@ -551,7 +551,7 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
         int eb_lo, eb_hi;
         sr_split(lo * 0.9999f, &nn, &eb_lo);
         sr_split(hi * 1.0001f, &nn, &eb_hi);
-        if (eb_lo == eb_hi) {  // (wave-uniform: both are the same in every lane)
+        if (SR_USUAL(eb_lo == eb_hi)) {  // (wave-uniform: both are the same in every lane)
             const SrInc sc = sr_scan_inc<false>(sr_run_inc(x, eb_lo));
             if (lane == SR_WAVE - 1) {
                 put(0, sc.a0, sc.a1, (uint32_t)eb_lo, SR_SEG_PLAIN);
@@ -576,7 +576,7 @@ __device__ __forceinline__ void seg_make_record(const float (&x)[SR_SEQ_RUN], in
     f.a0 = f.a1 = f.b0 = f.b1 = SR_SEQ_SAT;
     f.eb = eb_first; f.eb2 = eb_last; f.kind = SR_SEG_PLAIN; f.end_bits = 0u;
     int cross = -1;
-    if (first) {
+    if (SR_RARE(first)) {
         // the row's first segment (that has a term) starts from +0 exactly: its end, once and for all
         int dummy;
         const float end = sr_seq_wave<SR_SEQ_RUN, false>(x, 0.0f, 0.0f, &dummy);
@@ -1394,7 +1394,7 @@ __device__ __forceinline__ void seg_load_logits(const SegSource<ES>& src, int se
 {
     constexpr int K = SR_SEG_TERMS / (SR_WAVE * E);
     static_assert(K * E == SR_SEQ_RUN, "sixteen elements per lane");
-    if ((seg + 1) * SR_SEG_TERMS <= n) {
+    if (SR_USUAL((seg + 1) * SR_SEG_TERMS <= n)) {
         // a whole segment (all but a row's last): every load is issued before anything is done with one of them
         if (src.rowp) {
             uint4 raw[K];
@@ -1737,7 +1737,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     constexpr int kHitCap = 256;
     __shared__ unsigned long long hits[kHitCap];
     __shared__ uint32_t n_hits;
-    if (rd.temperature <= 0.0f) {  // greedy rows keep their logits where a distribution is asked for
+    if (SR_RARE(rd.temperature <= 0.0f)) {  // greedy rows keep their logits where a distribution is asked for
         if (kLists && a.mode == 0) seg_greedy<ES, kW, kS, E>(a, rd, slot, row, hits);
         return;
     }
@@ -1935,7 +1935,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
         }
     }
     __syncthreads();
-    if (bc[0] == 0u) {
+    if (SR_RARE(bc[0] == 0u)) {
         // (nobody waits for this one)
         if (lane == 0)
 #pragma unroll
@@ -1946,7 +1946,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
     const uint32_t mk = bc[1];
     // A NaN, or nothing above -inf: the row's workgroup makes it uniform.  A maximum of +inf, beside which e is no number where it
     // stands: the row's workgroup takes the row alone, so that every x - max below is at most 0, or -inf.
-    if (mk >= kKeyInf || mk <= 0x007fffffu) return;
+    if (SR_RARE(mk >= kKeyInf || mk <= 0x007fffffu)) return;
     const float m = sr_okey_inv(mk);
     if (asks && bc[0] == 2u) {
         if (wkey[wave] == mk) {
@@ -1969,7 +1969,7 @@ __global__ __launch_bounds__(kW * SR_WAVE, kS == 4 ? 5 : 6) void k_full_softmax_
         if (seg >= nseg) continue;
         float e[SR_SEQ_RUN];
         // (a whole segment without a test per element: the 16 chains of a lane then run interleaved)
-        if ((seg + 1) * SR_SEG_TERMS <= n) {
+        if (SR_USUAL((seg + 1) * SR_SEG_TERMS <= n)) {
 #pragma unroll
             for (int j = 0; j < SR_SEQ_RUN; j++) e[j] = sr_expf_neg(__fsub_rn(t[s][j], m), tab);
         } else {
@@ -3547,7 +3547,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
         // (a list that would have been too long was not made)
         const bool has_list = walked && row_is_listed(rd, a) && st_list_from != 0u, plain = walked && row_is_plain(rd, a);
         float* const e_row = walked ? row_e(a, slot) : p;
-        const uint32_t mk = alone ? row_alone(a, rd, p, n, row, sm) : full_maxkey_of(a, st_maxkey);
+        const uint32_t mk = SR_RARE(alone) ? row_alone(a, rd, p, n, row, sm) : full_maxkey_of(a, st_maxkey);
         const bool any_nan = mk == 0xffffffffu;
         const float m = mk == 0u ? SR_NEG_INF : sr_okey_inv(mk);
         FPROF(a, slot, 1);
@@ -3557,14 +3557,14 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
         int ns_listed = -1;  // >= 0: the block-wide count, and sm.sortbuf[0, ns_listed) holds the survivors
         bool row_unwritten = false;  // the row still holds expf(x - max): it will be finished from the list
         bool no_slabs = false;       // the nucleus is known to be too large for the walk by slabs
-        if (any_nan || sr_f2u(m) == 0xff800000u) {
+        if (SR_RARE(any_nan || sr_f2u(m) == 0xff800000u)) {
             const float uni = n > 0 ? __fdiv_rn(1.0f, (float)n) : 0.0f;
             row_pass<true>(p, n, [&](float, int) -> float { return uni; });
             flags |= SR_KFLAG_DEGENERATE;
             if (tid == kT - 1) sm.u = u_row;
             __syncthreads();
         } else {
-            if (row_edits_on_the_fly(rd, a) && !a.seg_func) {
+            if (SR_RARE(row_edits_on_the_fly(rd, a) && !a.seg_func)) {
                 // the ids that the row's edits touch were left out of the expf pass: their e, from the adjusted values
                 // that k_full_edits kept
                 const float* vals = (const float*)(a.edit_tab + (size_t)slot * (size_t)a.edit_tab_stride + (n + 31) / 32);
@@ -3578,7 +3578,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
             int dummy;
             float sum;
             int n_list = 0;
-            if (walked) {
+            if (SR_USUAL(walked)) {
                 // the whole device has prepared the sum (k_full_softmax_seg): one wave walks the segments' records while the
                 // others fetch the row's list, if it has one
                 if (sr_wave_id() == 0) {
@@ -3733,7 +3733,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                     way = n_list <= kT ? cut_from_list<1>(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm, more)
                           : n_list <= 4 * kT ? cut_from_list<4>(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm, more)
                                              : cut_from_list<SR_LIST_CAP_BIG / kT>(a, rd, st, p, n, slot, row, do_scale, inv, n_list, sm, more);
-                if (way != kListGeneral) {
+                if (SR_USUAL(way != kListGeneral)) {
                     FPROF(a, slot, 9);
                     __syncthreads();
                     if (tid == 0) {
@@ -4407,7 +4407,7 @@ __device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, Pr
     }
     __syncthreads();
     if (bc[0] == 0u) return;
-    if (bc[0] == 2u) {
+    if (SR_RARE(bc[0] == 2u)) {
         // some workgroup stopped waiting: all of the row again (everyone has counted in: the factor is there)
         inv2 = sr_u2f(bc[1]);
         for (int b = 0; b < (int)gridDim.x; b++) {

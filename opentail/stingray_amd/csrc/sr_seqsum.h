@@ -107,7 +107,7 @@ __device__ __forceinline__ SrInc sr_scan_inc(SrInc v)
 {
     // Nearly always every lane's increment is the same for both parities (they differ only behind an add that fell
     // exactly half way between two values): the functions are then plain numbers and their composition is a sum.
-    if (__ballot(v.a0 != v.a1) == 0ull) {
+    if (SR_USUAL(__ballot(v.a0 != v.a1) == 0ull)) {
         uint32_t t = v.a0;
         t = sr_sat_add(t, sr_dpp_u32<0x111>(t));
         t = sr_sat_add(t, sr_dpp_u32<0x112>(t));
