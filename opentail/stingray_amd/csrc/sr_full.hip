@@ -3023,6 +3023,283 @@ __device__ __forceinline__ unsigned long long e_units(uint32_t ebits)
 {
     return ((unsigned long long)((ebits & 0x7fffffu) | 0x800000u) << 17) >> min(127u - (ebits >> 23), 63u);
 }
+// Where the running sum over a long list's probabilities, the largest first, reaches `target`, without the list in order.
+// Inside a binade an addition of a term moves the sum by a whole number of its last places, the same number wherever the sum stands -- but for a
+// term that falls exactly half way between two --, so the terms of a stretch may come in any order.  The entries are counted by value
+// into groups of equal width in the bit patterns; what stands in front of a group is then known to about half a group's width, and
+// with it the binade, in which its terms' increments are added up in whole numbers.  In order are only those that need it: the first 32 (the
+// sum doubles from term to term), groups in which the sum may change binade, groups that hold a term half way, and the one in which
+// it gets to the target.  A walk of one thread's length over those, the stretches between them as one integer each, gives every state exactly;
+// it checks that each stretch lies in the binade it was added up for, and what does not fit goes by the sorted list.
+// Sorting such a list in shared memory is bound by what one compute unit's banks take: 14,000 entries 33 us and 10 for the sums in order, 7,800
+// 20 and 8, 3,000 9 and 6; this 13, 11 and 9 for all of it.  us a call, rows of 151,936 fp32 at temperature 0.6 and top-p 0.95 under masks that leave 0.4, 0.2, 0.1
+// of them: one row 92 -> 75, 72 -> 65, 60 -> 58; 64 rows 152 -> 134, 131 -> 123, 117 -> 115.  Two rows to a compute unit, lists of 2,000: 72.6 -> 73.5.
+struct ListCut {
+    int ns;        // entries that min-p leaves
+    int cutoff;    // of which the first so many are members
+    uint32_t ebits;  // e of the last member
+    float run;     // the sum behind it, or of all entries
+    bool found;    // the sum got to the target
+};
+constexpr int kInOrder = 1024;  // most entries that are put in order
+template <int kPer>
+__device__ __forceinline__ bool cut_unsorted(const uint32_t (&ev)[kPer], uint32_t valid, uint32_t from, bool do_scale, float inv, float target, uint32_t* base,
+                                             int G, ListCut* cut, FullSmem& sm)
+{
+    const int tid = threadIdx.x, lane = sr_lane(), wave = sr_wave_id();
+    uint32_t* const cnt = base;          // entries of a group, then of all groups in front
+    uint32_t* const info = base + G;     // a group's binade, and why its entries are in order
+    uint32_t* const inc = base + 2 * G;  // a group's increments, then those of all groups in front
+    uint32_t* const list = base + 3 * G; // the entries that are put in order: as they come, sorted, the stretch in front of each, the state behind each
+    uint32_t* const sorted = list + kInOrder;
+    uint32_t* const gap = sorted + kInOrder;
+    uint32_t* const state = gap + kInOrder;
+    constexpr uint32_t kOrdered = 0x100u, kHalfWay = 0x200u;
+    constexpr int kMost = 4;  // groups of a thread
+    auto prob = [&](uint32_t ebits) -> float { return do_scale ? __fmul_rn(sr_u2f(ebits), inv) : sr_u2f(ebits); };
+    const uint32_t span = 0x3f800000u - min(from, 0x3f800000u);
+    int gshift = 0;
+    while ((span >> gshift) >= (uint32_t)G) gshift++;
+    auto group_of = [&](uint32_t v) -> uint32_t { return min((0x3f800000u - v) >> gshift, (uint32_t)(G - 1)); };
+    const int per = G / kT, g0 = tid * per;
+    for (int i = tid; i < G; i += kT) { cnt[i] = 0u; inc[i] = 0u; }
+    // 11: a group found by all   12: it does not fit   13: entries in order   14: some group holds a term half way
+    if (tid >= 11 && tid <= 14) sm.bc[tid] = tid == 11 ? 0xffffffffu : 0u;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+        if ((valid >> r) & 1u) atomicAdd(&cnt[group_of(ev[r])], 1u);
+    __syncthreads();
+    {
+        int c[kMost], cs = 0;
+        float m[kMost], ms = 0.0f;
+#pragma unroll
+        for (int q = 0; q < kMost; q++) {
+            c[q] = q < per ? (int)cnt[g0 + q] : 0;
+            const uint32_t middle = 0x3f800000u - ((uint32_t)(g0 + q) << gshift) - ((1u << gshift) >> 1);
+            m[q] = c[q] > 0 ? (float)c[q] * prob(middle) : 0.0f;
+            cs += c[q];
+            ms += m[q];
+        }
+        const int ci = sr_wave_incl_scan_i32(cs);
+        const float mi = sr_wave_incl_sum_f32(ms);
+        if (lane == SR_WAVE - 1) { sm.redi[wave] = ci; sm.redf[wave] = mi; }
+        __syncthreads();
+        int cb = ci - cs, all = 0;
+        float mb = mi - ms;
+#pragma unroll
+        for (int w = 0; w < kW; w++) {
+            if (w < wave) { cb += sm.redi[w]; mb += sm.redf[w]; }
+            all += sm.redi[w];
+        }
+        cut->ns = all;
+        // (half of a group's width, and what n additions may be off)
+        const float off = sr_u2f((uint32_t)(127 - 23 + gshift) << 23) * 0.55f + 3e-4f;
+#pragma unroll
+        for (int q = 0; q < kMost; q++)
+            if (q < per) {
+                const uint32_t e0 = sr_f2u(mb * (1.0f - off)) >> 23, e1 = sr_f2u((mb + m[q]) * (1.0f + off)) >> 23;
+                info[g0 + q] = (sr_f2u(mb) >> 23) | (cb < 32 || e0 != e1 ? kOrdered : 0u);
+                cnt[g0 + q] = (uint32_t)cb;
+                cb += c[q];
+                mb += m[q];
+            }
+        if (all == 0) return false;
+    }
+    __syncthreads();
+    auto in_order = [&](uint32_t v) {
+        const uint32_t pos = atomicAdd(&sm.bc[13], 1u);
+        if (pos < (uint32_t)kInOrder) list[pos] = v;
+    };
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+        if ((valid >> r) & 1u) {
+            const uint32_t g = group_of(ev[r]), in = info[g];
+            if (in & kOrdered) {
+                in_order(ev[r]);
+            } else {
+                const uint32_t b = (in & 0xffu) << 23;
+                const float y = prob(ev[r]);
+                const uint32_t even = sr_f2u(__fadd_rn(sr_u2f(b), y)) - b, odd = sr_f2u(__fadd_rn(sr_u2f(b + 1u), y)) - (b + 1u);
+                atomicAdd(&inc[g], even);
+                if (even != odd) {
+                    atomicOr(&info[g], kHalfWay);
+                    sm.bc[14] = 1u;
+                }
+            }
+        }
+    __syncthreads();
+    if (sm.bc[14] != 0u) {
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if (((valid >> r) & 1u) && (info[group_of(ev[r])] & (kOrdered | kHalfWay)) == kHalfWay) in_order(ev[r]);
+        __syncthreads();
+    }
+    const int n = (int)sm.bc[13];
+    if (SR_RARE(n > kInOrder - 8)) return false;
+    auto put_in_order = [&](int len) {  // list -> sorted, the largest first: every entry against every other, four threads to an entry where they are few
+        const int sh = len <= kT / 4 ? 2 : len <= kT / 2 ? 1 : 0, e = tid >> sh;
+        const uint32_t v = e < len ? list[e] : 0u;
+        int rank = 0;
+        for (int j = tid & ((1 << sh) - 1); j < len; j += 1 << sh) {
+            const uint32_t o = list[j];
+            rank += (o > v) | ((o == v) & (j < e)) ? 1 : 0;
+        }
+        if (sh > 0) rank += (int)sr_dpp_u32<kDppXor1>((uint32_t)rank);
+        if (sh > 1) rank += (int)sr_dpp_u32<kDppXor2>((uint32_t)rank);
+        if (e < len && (tid & ((1 << sh) - 1)) == 0) sorted[rank] = v;
+    };
+    uint32_t all_inc = 0u;
+    {
+        uint32_t d[kMost], ds = 0u;
+#pragma unroll
+        for (int q = 0; q < kMost; q++) {
+            d[q] = q < per && (info[g0 + q] & (kOrdered | kHalfWay)) == 0u ? inc[g0 + q] : 0u;
+            ds += d[q];
+        }
+        const uint32_t di = (uint32_t)sr_wave_incl_scan_i32((int)ds);
+        if (lane == SR_WAVE - 1) sm.redu[wave] = di;
+        put_in_order(n);
+        __syncthreads();
+        uint32_t db = di - ds;
+#pragma unroll
+        for (int w = 0; w < kW; w++) {
+            if (w < wave) db += sm.redu[w];
+            all_inc += sm.redu[w];
+        }
+#pragma unroll
+        for (int q = 0; q < kMost; q++)
+            if (q < per) { inc[g0 + q] = db; db += d[q]; }
+    }
+    __syncthreads();
+    // The stretch in front of every entry in order, and behind the last one, in increments; beside it the entry's probability.  (Zeros up to a
+    // multiple of eight, for the walk.)
+    float* const ys = (float*)list;
+    auto stretch = [&](int i) -> uint32_t {  // i = 1 ... n
+        const uint32_t g = i < n ? group_of(sorted[i]) : (uint32_t)G;
+        return (g < (uint32_t)G ? inc[g] : all_inc) - inc[group_of(sorted[i - 1])];
+    };
+    for (int i = tid; i < ((n + 7) & ~7); i += kT) {
+        gap[i] = i > 0 && i < n ? stretch(i) : 0u;
+        ys[i] = i < n ? prob(sorted[i]) : 0.0f;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        // (one wave, every lane the same; what bounds it is its instructions, two an entry beside the loads and stores)
+        uint32_t b = 0u;
+        for (int i0 = 0; i0 < n; i0 += 8) {
+            const float4 y0 = *(const float4*)(ys + i0), y1 = *(const float4*)(ys + i0 + 4);
+            const uint4 d0 = *(const uint4*)(gap + i0), d1 = *(const uint4*)(gap + i0 + 4);
+            uint4 t0, t1;
+            t0.x = b = sr_f2u(__fadd_rn(sr_u2f(b + d0.x), y0.x));
+            t0.y = b = sr_f2u(__fadd_rn(sr_u2f(b + d0.y), y0.y));
+            t0.z = b = sr_f2u(__fadd_rn(sr_u2f(b + d0.z), y0.z));
+            t0.w = b = sr_f2u(__fadd_rn(sr_u2f(b + d0.w), y0.w));
+            t1.x = b = sr_f2u(__fadd_rn(sr_u2f(b + d1.x), y1.x));
+            t1.y = b = sr_f2u(__fadd_rn(sr_u2f(b + d1.y), y1.y));
+            t1.z = b = sr_f2u(__fadd_rn(sr_u2f(b + d1.z), y1.z));
+            t1.w = b = sr_f2u(__fadd_rn(sr_u2f(b + d1.w), y1.w));
+            if (lane == 0) {
+                *(uint4*)(state + i0) = t0;
+                *(uint4*)(state + i0 + 4) = t1;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        int at = -1, kind = 0;
+        bool misfit = false;
+        uint32_t last = 0u;  // (of lane n mod 64) the sum behind everything
+        for (int i0 = 0; i0 <= n && at < 0; i0 += SR_WAVE) {
+            const int i = i0 + lane;
+            uint32_t before = 0u, d = 0u;
+            if (i > 0 && i <= n) {
+                before = state[i - 1];
+                d = i < n ? gap[i] : stretch(n);
+                if (d != 0u) {
+                    // the stretch's groups were added up for one binade, and the sum is in it from end to end
+                    const uint32_t eb = info[group_of(sorted[i - 1]) + 1u] & 0xffu, eb1 = info[(i < n ? group_of(sorted[i]) : (uint32_t)G) - 1u] & 0xffu;
+                    misfit = misfit || d >= (1u << 24) || eb1 != eb || (before >> 23) != eb || ((before + d) >> 23) != eb;
+                }
+            }
+            const bool in_gap = d != 0u && sr_u2f(before + d) >= target, on_it = i < n && sr_u2f(state[min(i, n - 1)]) >= target;
+            if (i == n) last = before + d;
+            const unsigned long long hit = __ballot(in_gap || on_it);
+            if (hit != 0ull) {
+                const int l = (int)__ffsll((long long)hit) - 1;
+                at = i0 + l;
+                kind = ((__ballot(in_gap) >> l) & 1ull) != 0ull ? 2 : 1;
+            }
+        }
+        if (__ballot(misfit) != 0ull && lane == 0) sm.bc[12] = 1u;
+        if (kind == 0 && lane == (n & (SR_WAVE - 1))) sm.segbc[2] = last;
+        if (kind == 1) {
+            const uint32_t g = group_of(sorted[at]);
+            int before = 0;  // entries of the same group in front
+            for (int j0 = 0; j0 < at; j0 += SR_WAVE) before += __popcll(__ballot(j0 + lane < at && group_of(sorted[min(j0 + lane, n - 1)]) == g));
+            if (lane == 0) sm.segbc[2] = cnt[g] + (uint32_t)before + 1u;
+        }
+        if (lane == 0) {
+            sm.segbc[0] = (uint32_t)kind;
+            sm.segbc[1] = (uint32_t)at;
+        }
+    }
+    __syncthreads();
+    if (SR_RARE(sm.bc[12] != 0u)) return false;
+    const int kind = (int)sm.segbc[0], at = (int)sm.segbc[1];
+    cut->found = kind != 0;
+    if (kind == 0) {
+        cut->run = sr_u2f(sm.segbc[2]);
+        cut->cutoff = cut->ns;
+        cut->ebits = 0u;
+        return true;
+    }
+    if (kind == 1) {
+        cut->run = sr_u2f(state[at]);
+        cut->cutoff = (int)sm.segbc[2];
+        cut->ebits = sorted[at];
+        return true;
+    }
+    // inside a stretch: the group in which the sum gets there, and its entries in order
+    const uint32_t gp = group_of(sorted[at - 1]), g_end = at < n ? group_of(sorted[at]) : (uint32_t)G, front = state[at - 1];
+    uint32_t first = 0xffffffffu;
+#pragma unroll
+    for (int q = kMost - 1; q >= 0; q--) {
+        const uint32_t g = (uint32_t)(g0 + q);
+        if (q < per && g > gp && g < g_end) {
+            const uint32_t to = front + ((g + 1u < (uint32_t)G ? inc[g + 1u] : all_inc) - inc[gp]);
+            if (sr_u2f(to) >= target) first = g;
+        }
+    }
+    first = sr_wave_min_u32(first);  // (an atomic of every group behind the cut: 8 us)
+    if (lane == 0 && first != 0xffffffffu) atomicMin(&sm.bc[11], first);
+    if (tid == 0) sm.bc[13] = 0u;
+    __syncthreads();
+    const uint32_t gc = sm.bc[11];
+    if (SR_RARE(gc >= (uint32_t)G)) return false;
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+        if (((valid >> r) & 1u) && group_of(ev[r]) == gc) in_order(ev[r]);
+    __syncthreads();
+    const int m = (int)sm.bc[13];
+    const uint32_t s0 = front + (inc[gc] - inc[gp]);
+    if (SR_RARE(m > kInOrder)) return false;
+    put_in_order(m);
+    __syncthreads();
+    uint32_t b = s0, e = 0u;
+    int k = 0;
+    for (; k < m; k++) {  // (every thread the same: a few dozen)
+        e = sorted[k];
+        b = sr_f2u(__fadd_rn(sr_u2f(b), prob(e)));
+        if (sr_u2f(b) >= target) break;
+    }
+    if (SR_RARE(k >= m)) return false;
+    cut->run = sr_u2f(b);
+    cut->cutoff = (int)cnt[gc] + k + 1;
+    cut->ebits = e;
+    return true;
+}
+
 template <int kPer>
 __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& rd, SrFullState* st, float* p, int n, int slot, int row,
                                              bool do_scale, float inv, int N, FullSmem& sm, uint32_t* more)
@@ -3057,7 +3334,25 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     for (int r = 0; r < kPer; r++) ev[r] = r < mine ? grp[list_place(i0 + r)] : 0u;
     auto prob = [&](uint32_t ebits) -> float { return do_scale ? __fmul_rn(sr_u2f(ebits), inv) : sr_u2f(ebits); };
 
-    if (kOne && N <= kT / 4) {
+    bool in_place = false;  // the cut is known from the list as it stands
+    ListCut cut = {};
+    if (!kOne && use_top_p) {
+        uint32_t valid = 0u;
+#pragma unroll
+        for (int r = 0; r < kPer; r++)
+            if (r < mine) {
+                const float y = prob(ev[r]);
+                if (use_min_p) SR_AMB_IF(sr_near(y, thr));  // an entry on the threshold
+                valid |= !use_min_p || y >= thr ? 1u << r : 0u;
+            }
+        static_assert((3 * 4096 + 4 * kInOrder) * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags) &&
+                      (SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16 + 3 * 2048 + 4 * kInOrder) * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags),
+                      "the tables fit");
+        in_place = cut_unsorted<kPer>(ev, valid, from, do_scale, inv, rd.top_p, cnt, more ? 4096 : 2048, &cut, sm);
+        if (!in_place) __syncthreads();
+    }
+    if (!kOne && in_place) {
+    } else if (kOne && N <= kT / 4) {
         // A short list: every entry against every other, four threads to an entry (lists of 80 to 140: 1.5 us, 6 by groups)
         const int e = tid >> 2;
         const uint32_t v = e < N ? grp[list_place(e)] : 0u;
@@ -3158,8 +3453,8 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
             if (r < mine) grp[list_place(rank[r])] = v[r];
     }
     // the survivors of min-p (the largest ones)
-    int ns = N;
-    if (use_min_p) {
+    int ns = in_place ? cut.ns : N;
+    if (use_min_p && !in_place) {
         int c = 0;
 #pragma unroll
         for (int r = 0; r < kPer; r++)
@@ -3201,7 +3496,11 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
     };
     if (kPer <= 4) fetch_indices();
     int found = -1;
-    if (use_top_p) {
+    if (!kOne && in_place) {
+        found = cut.found ? cut.cutoff - 1 : -1;
+        if (found < 0 && from > 1u && min_p_list_from(rd) < from) return kListGeneral;
+        if (found >= 0 && from > 1u && prob(from - 1u) >= prob(cut.ebits)) return kListGeneral;
+    } else if (use_top_p) {
         auto fetch = [&](int b0, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < SR_SEQ_RUN; j++) {
@@ -3264,12 +3563,41 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
         }
     }
     const int cutoff = found >= 0 ? found + 1 : ns, m = cutoff;
-    const float ycut = prob(grp[list_place(cutoff - 1)]);
+    float ycut;
+    bool tie;
+    if (!kOne && in_place) {
+        // the value at the cut (where nothing was cut, the smallest that is left), and whether an entry behind the cut has it
+        if (found >= 0) {
+            ycut = prob(cut.ebits);
+        } else {
+            uint32_t least = 0xffffffffu;
+#pragma unroll
+            for (int r = 0; r < kPer; r++)
+                if (r < mine) {
+                    const float y = prob(ev[r]);
+                    if (!use_min_p || y >= thr) least = min(least, sr_f2u(y));
+                }
+            least = sr_wave_min_u32(least);
+            if (lane == 0) sm.redu[wave] = least;
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < kW; w++) least = min(least, sm.redu[w]);
+            ycut = sr_u2f(least);
+        }
+        int c = 0;
+#pragma unroll
+        for (int r = 0; r < kPer; r++) c += r < mine && prob(ev[r]) >= ycut ? 1 : 0;
+        tie = blk_sum_i(c, sm) > cutoff;
+        if (tid == 0) SR_AMB_IF(found >= 0 ? sr_stop_near(cut.run, ycut, rd.top_p) || tie : sr_near(cut.run, rd.top_p));
+    } else {
+        ycut = prob(grp[list_place(cutoff - 1)]);
+        tie = false;
+    }
     const bool finish = a.mode == 0 && m <= a.finish_most;
     if (!finish && !a.prepared) return kListGeneral;
     // Members: everything above the value at the cut, and of the entries equal to it the first ones by index -- nearly always all of
     // them: nothing behind the cut has its value.
-    const bool tie = cutoff < ns && prob(grp[list_place(cutoff)]) == ycut;
+    if (!in_place) tie = cutoff < ns && prob(grp[list_place(cutoff)]) == ycut;
     if (kPer > 4) fetch_indices();
     uint32_t members = 0u;
     int last_here = -1;

@@ -177,9 +177,12 @@ int run_full(sr_ctx* ctx, const sr_batch* b, const int32_t* list_dev, int n_rows
             const int blocks = (half_blocks + 1) / 2, held = 2 * ctx->cu_count;
             a.behind_twice = prepared && !lazy_scale && (long long)n_rows * blocks >= 2 * held &&
                              (any_plain ? blocks >= 7 && held % blocks != 0 : mode != 0 && blocks >= 12) ? 1 : 0;
-            // (up to 1,024 members cost the row's workgroup less than the launch behind it; of short rows more: 256 rows of 12,290, half of
-            // them cut to some thousand members, 98 us, with 1,024 134)
-            a.finish_most = prepared && nseg >= SR_PREPARED_MIN_SEGS ? 1024 : 8192;
+            // Up to 8,192 members cost the row's workgroup less than the launch behind it (us a call, top-p 0.95 at temperature 0.6 under masks that leave
+            // 0.4, 0.2, 0.1, 0.03 of the row, 1,024 and 8,192: 64 rows of 151,936 134 and 134, 123 and 89, 115 and 74, 90 and 67; 200 of 65,536 142 and 99, 133
+            // and 83, 133 and 77; one row 75 both, 65 and 63, 58 and 49), but where a row that nothing cuts takes that launch anyway: then it waits
+            // for them (every third row of 32 of 100,003 87 and 104, 76 and 87, 71 and 75).  Of short rows more, whatever stands beside them:
+            // 256 rows of 12,290, half of them cut to some thousand members, 98 us, with 1,024 134.
+            a.finish_most = prepared && any_plain && nseg >= SR_PREPARED_MIN_SEGS ? 1024 : 8192;
             // e = expf(x - max): in the work rows of tokens-only launches and of the verifier (whose reader applies the factors);
             // apart from the caller's rows where the probabilities take shape there
             a.e_rows = a.work;
