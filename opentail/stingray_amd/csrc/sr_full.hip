@@ -3300,6 +3300,133 @@ __device__ __forceinline__ bool cut_unsorted(const uint32_t (&ev)[kPer], uint32_
     return true;
 }
 
+// Final Normalize and draw (Sampler.cs:91-92, :553-576) of a sampled row whose members are thousands of its list's entries: members holds
+// those of the thread, idx their indices; the threads' entries follow each other in the order of the indices.
+// The eight accumulators' terms are put side by side, each accumulator's in the order of the indices, so that a wave passes over a thousand terms
+// of its own; over all members with the others' as zeros (finish_from_ordered_list) it is eight times as many rounds.  Putting them there takes 3.7 us, so lists of up
+// to 4,096 go that way: 3,000 members 9.6 us to the sum and 10.2 that way, 7,800 13.4 and 17.7.
+template <int kPer, typename Prob>
+__device__ __forceinline__ void finish_members(const SrFullArgs& a, int n, int row, const uint32_t (&ev)[kPer], const int (&idx)[kPer], uint32_t members, Prob prob,
+                                               uint32_t* more, FullSmem& sm)
+{
+    const int lane = sr_lane(), wave = sr_wave_id(), tid = threadIdx.x, nv8 = (n / 8) * 8;
+    unsigned long long* const list = sm.sortbuf;  // index << 32 | bits of the probability, at list_layout
+    uint32_t* const terms = more ? more : (uint32_t*)sm.sprob;  // the accumulators' terms, at list_place
+    static_assert((2 * kSmall + 8 * 16) * 17 / 16 <= SR_LIST_CAP_BIG + SR_LIST_CAP_BIG / 16 && (kSmall + 8 * 16) * 17 / 16 <= 2 * kSmall,
+                  "the terms of 8,192 members fit behind 68 KB, of 4,096 in the two arrays behind the list");
+    auto chain_of = [&](int i) -> int { return i < nv8 ? i & 7 : i - (n - 8); };
+    // members of every accumulator, two counts to a word (8,192 at most), in front of the thread's
+    uint32_t cc[4] = {0u, 0u, 0u, 0u}, in[4];
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+        if ((members >> r) & 1u) {
+            const int c = chain_of(idx[r]);
+#pragma unroll
+            for (int k = 0; k < 4; k++) cc[k] += (c >> 1) == k ? 1u << (16 * (c & 1)) : 0u;
+        }
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        in[k] = (uint32_t)sr_wave_incl_scan_i32((int)cc[k]);
+        if (lane == SR_WAVE - 1) sm.hist[4 * wave + k] = in[k];
+        in[k] -= cc[k];
+    }
+    __syncthreads();  // (and nobody reads what lies in the lists' places any more)
+    uint32_t tot[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int w = 0; w < kW; w++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t v = sm.hist[4 * w + k];
+            tot[k] += v;
+            in[k] += w < wave ? v : 0u;
+        }
+    int at = 0, m = 0, base = 0, own_base = 0, own_cnt = 0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        at += (int)(in[k] & 0xffffu) + (int)(in[k] >> 16);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int cnt = (int)((tot[k] >> (16 * h)) & 0xffffu);
+            if (lane == 0) sm.hist[128 + 8 * wave + 2 * k + h] = (uint32_t)base;  // (a copy of the wave's own)
+            if (wave == 2 * k + h) { own_base = base; own_cnt = cnt; }
+            base += (cnt + 15) & ~15;
+            m += cnt;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+        if ((members >> r) & 1u) {
+            const int c = chain_of(idx[r]);
+            uint32_t p = 0u;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                p = (c >> 1) == k ? in[k] : p;
+                in[k] += (c >> 1) == k ? 1u << (16 * (c & 1)) : 0u;
+            }
+            p = (p >> (16 * (c & 1))) & 0xffffu;
+            const uint32_t y = sr_f2u(prob(ev[r]));
+            terms[list_place((int)(sm.hist[128 + 8 * wave + c] + p))] = y;
+            list[list_layout(at)] = ((unsigned long long)(uint32_t)idx[r] << 32) | (unsigned long long)y;
+            at++;
+        }
+    __syncthreads();
+    if (wave < SR_SEQ_CHAINS) {
+        float sc = 0.0f;
+        for (int b0 = 0; b0 < own_cnt; b0 += 16 * SR_WAVE) {
+            float x[16];
+#pragma unroll
+            for (int j = 0; j < 16; j++) {
+                const int i = b0 + 16 * lane + j;
+                x[j] = i < own_cnt ? sr_u2f(terms[list_place(own_base + i)]) : 0.0f;
+            }
+            int dummy;
+            sc = sr_seq_wave<16, false>(x, sc, 0.0f, &dummy);
+        }
+        if (lane == 0) sm.lane_sum[wave] = sc;
+    }
+    __syncthreads();
+    const float l0 = sm.lane_sum[0], l1 = sm.lane_sum[1], l2 = sm.lane_sum[2], l3 = sm.lane_sum[3],
+                l4 = sm.lane_sum[4], l5 = sm.lane_sum[5], l6 = sm.lane_sum[6], l7 = sm.lane_sum[7];
+    const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
+    const bool scale = sum > 0.0f && sum != 1.0f;
+    const float inv = scale ? __fdiv_rn(1.0f, sum) : 1.0f, u = __double2float_rn(sm.u);
+    if (!(u > 0.0f)) {  // the running sum starts at p[0] >= 0: index 0 reaches a target of zero whatever it holds
+        if (tid == 0 && a.out_tokens) a.out_tokens[row] = 0;
+        return;
+    }
+    if (wave != 0) return;
+    // (a thousand at a time to where the draw lands: on average half of them.  Records by a wave each and a walk over them: 6.6 us whatever
+    // u is, this 2.6 to 4.7)
+    float acc = 0.0f;
+    int f = -1;
+    for (int b0 = 0; b0 < m && f < 0; b0 += 16 * SR_WAVE) {
+        float x[16];
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const int i = b0 + 16 * lane + j;
+            const float y = i < m ? sr_u2f((uint32_t)list[list_layout(i)]) : 0.0f;
+            x[j] = scale ? __fmul_rn(y, inv) : y;
+        }
+        acc = sr_seq_wave<16, true>(x, acc, u, &f);
+        if (f >= 0) f += b0;
+    }
+    if (lane == 0) {
+        int token = n - 1;  // (the draw ran off the end of the list: the last index, by the rounding fallback)
+        if (f >= 0) {
+            const unsigned long long v = list[list_layout(f)];
+            token = (int)(v >> 32);
+            const float y = sr_u2f((uint32_t)v);
+            SR_AMB_IF(sr_stop_near(acc, scale ? __fmul_rn(y, inv) : y, u));
+        } else {
+            SR_AMB_IF(sr_near(acc, u));
+        }
+        if (a.out_tokens) a.out_tokens[row] = token;
+    }
+}
+
 template <int kPer>
 __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& rd, SrFullState* st, float* p, int n, int slot, int row,
                                              bool do_scale, float inv, int N, FullSmem& sm, uint32_t* more)
@@ -3340,11 +3467,12 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
         uint32_t valid = 0u;
 #pragma unroll
         for (int r = 0; r < kPer; r++)
-            if (r < mine) {
+            if (r < mine && use_min_p) {
                 const float y = prob(ev[r]);
-                if (use_min_p) SR_AMB_IF(sr_near(y, thr));  // an entry on the threshold
-                valid |= !use_min_p || y >= thr ? 1u << r : 0u;
+                SR_AMB_IF(sr_near(y, thr));  // an entry on the threshold
+                valid |= y >= thr ? 1u << r : 0u;
             }
+        if (!use_min_p) valid = (1u << mine) - 1u;
         static_assert((3 * 4096 + 4 * kInOrder) * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags) &&
                       (SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16 + 3 * 2048 + 4 * kInOrder) * 4 <= sizeof(FullSmem::sortbuf) + sizeof(FullSmem::sprob) + sizeof(FullSmem::tags),
                       "the tables fit");
@@ -3627,6 +3755,10 @@ __device__ __forceinline__ int cut_from_list(const SrFullArgs& a, const SrRow& r
 #pragma unroll
         for (int r = 0; r < kPer; r++)
             if (r < mine && prob(ev[r]) >= ycut) members |= 1u << r;
+    }
+    if (kPer > 4 && finish && m > SR_SEG_TERMS) {
+        finish_members<kPer>(a, n, row, ev, idx, members, prob, more, sm);
+        return kListDone;
     }
     if (finish) {
         // in the order of the list, which is the order of the indices
