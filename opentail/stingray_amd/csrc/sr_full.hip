@@ -5380,12 +5380,14 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_factor(SrFullArgs a, SrSpecA
 // the logits: e, the records of its sum, m1; the records of the eight accumulators over fl(e m1), m2.
 // 16 sequences of 8 drafts over 262,144 (144 rows), us: this one 23 (6.6 TB/s; k_full_softmax_seg, with e, two meetings and records, 59),
 // k_full_row none (15), k_spec_open 45 (k_spec_factor 28; its chain: tests 3.4, the block from its logits 8, records 5, walk 7, records 5,
-// walk 4), k_spec_rows 23 both; the call 127 -> 98.  A further position with an open test is another 25.
+// walk 4), k_spec_rows 23 both; the call 127 -> 98.  A further position with an open test is another 25.  A bonus row whose largest entry
+// decides (row_decided: the units bound its draw) needs none of it: calls without a rejection 45, 1 x 8 of 262,144 50 -> 17, 16 x 4 of 128,256 62 -> 25.
 // A unit's maximum is exact; a term's exponential is v_exp_f32 of a difference rounded once: 2^-24 of the exponent's size, which is
 // below 28 for all terms that make up more than 2^-22 of the sum.
 // What k_spec_open leaves of a row's tests, behind its meeting point (SrSpecArgs::sync): the positions that it worked out, a bit each; those
 // of them whose draft is accepted; the position that ends the row for certain, and above it whether its id lies outside the vocabulary
 constexpr int kSpecPicked = 4, kSpecAccepted = 5, kSpecLast = 6;
+constexpr unsigned long long kSpecWritten = 1ull << 33;  // ... or that the row's results are written
 constexpr int kSpecDone = -2;  // SrSpecArgs::reject of a row whose results are written
 // The words behind a position's meeting point (SrFullArgs::row_sync) that count its workgroups in, k_spec_units clears them.  (Not
 // those of k_prepared_row and of the greedy rows: other launches of the context find these as they left them.)
@@ -5635,6 +5637,8 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_open(SrFullArgs a, SrSpecArg
         said[kSpecPicked] = pick;
         said[kSpecLast] = (unsigned long long)last | (last < L && (test[last] & 4) != 0 ? 1ull << 32 : 0ull);
     }
+    const bool only_bonus = pick == 1ull << L;  // every draft is accepted for certain
+    const float u_bonus = only_bonus ? __double2float_rn(s.uniforms[(size_t)row * s.uniforms_per_row + L]) : 0.0f;
     for (; pick != 0ull; pick &= pick - 1ull) {
         // (what the lane's number gives is worked out here: kept over the whole loop, its dozens of offsets cost that many registers)
         int ln = lane;
@@ -5680,6 +5684,45 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_open(SrFullArgs a, SrSpecArg
                 before += w[k].y * scale;
                 before_chain += uc[k] * scale;
             }
+        if (only_bonus && t.kind == 0) {
+            // whether the bonus row's largest entry is its token: the same answer in every workgroup
+            int first = s.n_units;  // the unit that holds it
+#pragma unroll
+            for (int k = kUnits - 1; k >= 0; k--) {
+                const unsigned long long top = __ballot(w[k].x == r.max);
+                if (top != 0ull) first = k * SR_WAVE + (int)__ffsll((long long)top) - 1;
+            }
+            float front = 0.0f, own_unit = 0.0f;
+#pragma unroll
+            for (int k = 0; k < kUnits; k++) {
+                const float part = w[k].x > SR_NEG_INF ? w[k].y * __builtin_amdgcn_exp2f((w[k].x - r.max) * kLog2E) : 0.0f;
+                front += k * SR_WAVE + ln < first ? part : 0.0f;
+                own_unit += k * SR_WAVE + ln == first ? part : 0.0f;
+            }
+            if (row_decided(rd, n, r.sum, sr_wave_sum_f32(front), sr_wave_sum_f32(own_unit), u_bonus)) {
+                if (blk == 0 && tid == 0) said[kSpecLast] = (unsigned long long)L | kSpecWritten;
+                int at = -1;  // (the only entry of its value: one lane of one workgroup)
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int i = seg * SR_SEG_TERMS + (k * SR_WAVE + ln) * 4 + q;
+                        at = i < n && __fmul_rn(v[k][q], t.inv_temp) == r.max ? i : at;
+                    }
+                const unsigned long long has = __ballot(at >= 0);
+                if (has != 0ull) {
+                    const int token = __builtin_amdgcn_readlane(at, (int)__ffsll((long long)has) - 1);
+                    int* const out = s.out_tokens + (size_t)row * (L + 1);
+                    if (ln < L) out[ln] = s.draft_tokens[(size_t)row * L + ln];
+                    if (ln == L) out[ln] = token;
+                    if (ln == 0) {
+                        s.out_accepted[row] = L;
+                        s.reject[row] = kSpecDone;
+                    }
+                }
+                break;
+            }
+        }
         before = sr_wave_sum_f32(before);
         before_chain = sr_wave_sum_f32(before_chain);
 #pragma unroll
@@ -5882,7 +5925,7 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
         if (tid == 0) {
             const unsigned long long picked = sync[kSpecPicked] & ~sync[kSpecAccepted], last = sync[kSpecLast];
             said[0] = picked != 0ull ? (int)__ffsll((long long)picked) - 1 : (int)(uint32_t)last;
-            said[1] = picked == 0ull ? 2 : said[0] < L ? 0 : 1;
+            said[1] = (last & kSpecWritten) != 0ull ? 3 : picked == 0ull ? 2 : said[0] < L ? 0 : 1;
         } else if (tid == SR_WAVE) {
             const unsigned long long was = __hip_atomic_fetch_max(sync, (unsigned long long)a.seq << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             asm volatile("" : : "v"(was) : "memory");
@@ -5931,6 +5974,7 @@ __global__ __launch_bounds__(kSpecT, 4) void k_spec_rows(SrSpecArgs a)
             a.reject[row] = kSpecDone;
         }
     };
+    if (kFrom == 2 && kind == 3) return;
     if (kind == 2) {
         if (blockIdx.x == 0 && wave == 0) results(-1);
         return;

@@ -92,3 +92,46 @@ def test_rows_that_their_largest_entry_decides(ctx, rows, vocab, top_k, bf16):
                                              (66, 200_064, False), (40, 50_257, True), (280, 16_385, False)])
 def test_rows_of_the_whole_vocabulary_that_their_largest_entry_decides(ctx, rows, vocab, bf16):
     _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, 0, bf16, 8 if rows < 10 else 2 if rows < 50 else 1)
+
+
+# A verification whose drafts are all accepted: the bonus row's largest entry is its token, or is not.  A row and a half of blocks, one entry in a
+# unit of its own, a block's last entry; short rows, many positions.
+@pytest.mark.parametrize("rows,drafts,vocab", [(16, 2, 50_001), (9, 8, 65_537), (3, 4, 262_144), (40, 7, 8_193), (300, 1, 4_096)])
+def test_bonus_rows_that_their_largest_entry_decides(ctx, rows, drafts, vocab):
+    import torch
+    from oracle import binding as orc
+    from tests.helpers import to_oracle
+
+    rng = np.random.default_rng(rows + vocab)
+    for _ in range(3 if rows < 100 else 1):
+        t = rng.normal(0, 1, (rows, drafts + 1, vocab)).astype(np.float32)
+        u = rng.uniform(0.05, 0.5, (rows, drafts + 1))
+        temps = [float(np.float32(rng.choice([1.0, rng.uniform(0.5, 1.3)]))) for _ in range(rows)]
+        k = rng.integers(0, vocab, (rows, drafts))
+        q = np.full((rows, drafts, vocab), 1e-9, dtype=np.float32)
+        for r in range(rows):
+            for i in range(drafts):
+                t[r, i, k[r, i]] = 30.0  # accepted for certain
+                q[r, i, k[r, i]] = 0.9
+            x = t[r, drafts].astype(np.float64) / temps[r]
+            rest = x.max() + np.log(np.exp(x - x.max()).sum())
+            gap = rng.uniform(-1.0, 7.0)
+            at = int(rng.choice([0, vocab - 1, 8_191 % vocab, 2_048 % vocab, int(rng.integers(vocab))]))
+            t[r, drafts, at] = np.float32((rest + gap) * temps[r])
+            # the sum in front of the entry and behind it, of all
+            x = t[r, drafts].astype(np.float64) / temps[r]
+            p = np.exp(x - x.max())
+            line = p[: at + int(rng.integers(2))].sum() / p.sum()
+            u[r, drafts] = np.clip(line + rng.choice([-0.3, -3e-2, -1e-3, -1e-5, 0.0, 1e-5, 1e-3, 3e-2, 0.3]), 0.0, 0.99999999)
+            if r % 9 == 4:
+                u[r, drafts] = rng.choice([0.0, 1e-7, 0.9999999])
+            if r % 9 == 5:
+                t[r, drafts, (at + vocab // 2) % vocab] = t[r, drafts, at]  # not the only one
+            if r % 9 == 7:
+                u[r, rng.integers(drafts)] = 0.9999999  # and a row that rejects
+        params = [SamplingParams(Temperature=T) for T in temps]
+        dev = [torch.from_numpy(v).cuda() for v in (t, q, k.astype(np.int32))]
+        acc, tok = ctx.spec_verify(dev[0], dev[1], dev[2], params, u)
+        for r in range(rows):
+            wa, wt = orc.spec_verify_row(t[r], q[r], k[r], to_oracle(params[r]), orc.Rng(replay=u[r]))
+            assert acc[r] == wa and np.array_equal(tok[r][: len(wt)], wt), (r, acc[r], wa, tok[r], wt)
