@@ -5633,13 +5633,17 @@ __global__ __launch_bounds__(kPrepT, 4) void k_spec_open(SrFullArgs a, SrSpecArg
         if (((wrong >> last) & 1ull) == 0ull) pick |= 1ull << last;  // (an id outside the vocabulary ends the row without a draw)
     }
     unsigned long long* const said = s.sync + (size_t)row * SR_ROW_SYNC_STRIDE;
-    if (blk == 0 && tid == 0) {
+    if (blk == 0 && blockIdx.z == 0 && tid == 0) {
         said[kSpecPicked] = pick;
         said[kSpecLast] = (unsigned long long)last | (last < L && (test[last] & 4) != 0 ? 1ull << 32 : 0ull);
     }
     const bool only_bonus = pick == 1ull << L;  // every draft is accepted for certain
     const float u_bonus = only_bonus ? __double2float_rn(s.uniforms[(size_t)row * s.uniforms_per_row + L]) : 0.0f;
-    for (; pick != 0ull; pick &= pick - 1ull) {
+    // (the grid's third dimension: positions side by side)
+    auto next = [&](int by) __attribute__((always_inline)) {
+        for (int i = 0; i < by; i++) pick &= pick - 1ull;
+    };
+    for (next((int)blockIdx.z); pick != 0ull; next((int)gridDim.z)) {
         // (what the lane's number gives is worked out here: kept over the whole loop, its dozens of offsets cost that many registers)
         int ln = lane;
         asm volatile("" : "+v"(ln));
@@ -6439,9 +6443,10 @@ hipError_t sr_launch_spec_verify(const SrSpecArgs& a, int rows, hipStream_t st)
         static_assert(kSpecWaves == SR_SEQ_CHAINS && kSpecT == kPrepT, "the same blocks of a row");
         b.open_factors = nullptr;
         if (a.all_open) {
+            const dim3 open_grid(grid.x, grid.y, (unsigned)b.open_side);
             hipLaunchKernelGGL(k_spec_units, dim3((unsigned)((b.n_units + 3) / 4), rows * (b.n_draft + 1)), dim3(256), 0, st, *a.open_factors, b);
-            if (b.n_units <= kUnitsFew * SR_WAVE) hipLaunchKernelGGL(k_spec_open<kUnitsFew>, grid, dim3(kPrepT), 0, st, *a.open_factors, b);
-            else hipLaunchKernelGGL(k_spec_open<kUnitsMost>, grid, dim3(kPrepT), 0, st, *a.open_factors, b);
+            if (b.n_units <= kUnitsFew * SR_WAVE) hipLaunchKernelGGL(k_spec_open<kUnitsFew>, open_grid, dim3(kPrepT), 0, st, *a.open_factors, b);
+            else hipLaunchKernelGGL(k_spec_open<kUnitsMost>, open_grid, dim3(kPrepT), 0, st, *a.open_factors, b);
             hipLaunchKernelGGL(k_spec_rows<2>, grid, dim3(kSpecT), 0, st, b);
         } else if (a.open_factors) {
             hipLaunchKernelGGL(k_spec_factor, grid, dim3(kPrepT), 0, st, *a.open_factors, b);

@@ -554,13 +554,12 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     const int32_t* list = nullptr;
     SrFullArgs full{};
     const bool in_one = n_draft > 0 && n_draft < 64 && draft_probs_dev && rows <= 65535;  // (k_spec_factor: a position a lane)
-    // Rows that nothing touches, all of them: k_spec_units and k_spec_open (the lines: SR_OPEN_*).  Not the untouched rows of a mixed call:
+    // Rows that nothing touches, all of them: k_spec_units and k_spec_open (both sides measured: sr_types.h).  Not the untouched rows of a mixed call:
     // it lasts as long as the cut row's positions, which one workgroup each finishes.  16 x 8 of 262,144, none, one and all sequences
     // under top-p, us: 114, 229, 270; with one, k_full_softmax_seg 59, k_full_row 110, k_spec_factor 38, k_spec_rows 22, where the other
     // way's 23 + 69 + 23 would stand beside a pass and a k_full_row for the cut row's nine positions.
     const int nseg = (V + SR_SEG_TERMS - 1) / SR_SEG_TERMS;
-    bool all_open = in_one && V >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX && (int64_t)rows * P <= 65535 &&
-                    (nseg < SR_OPEN_SHORT_SEGS || rows * P > ctx->cu_count || (nseg >= SR_OPEN_MIN_SEGS && (int64_t)rows * P * nseg >= SR_OPEN_SEGS));
+    bool all_open = in_one && V >= SR_SEG_MIN_VOCAB && nseg <= SR_SEG_MAX && (int64_t)rows * P <= 65535;
     for (int r = 0; r < rows && all_open; r++) {
         const SrRow& d = b->h_rows[(size_t)r];
         all_open = d.temperature > 0.0f && by_ratio(d) && !sr_row_cut(d) && !(d.top_k > 0 && d.top_k < V) && d.edit_cnt <= 0 && d.mask_row < 0;
@@ -627,6 +626,11 @@ int sr_spec_verify_launch(sr_ctx* ctx, const sr_batch* b, const float* target_lo
     if (full.factor_later || all_open) a.open_factors = &full;
     if (all_open) {
         a.all_open = 1;
+        // as many positions side by side as the device holds workgroups beside the first ones': 16 x 8 of 20,011 and of 40,000 with two open in
+        // a row 70 us -> 49 and 68 -> 47.  (Not more: 16 x 8 of 262,144, whose first ones fill it, 105 -> 92 where a row has two, but 44.6 -> 47.3
+        // where none has.)
+        const long long held = 2 * ctx->cu_count / std::max(1LL, (long long)rows * full.chain_blocks);
+        a.open_side = (int)std::max(1LL, std::min({held, (long long)P, 4LL}));
         a.n_units = (V + SR_UNIT_TERMS - 1) / SR_UNIT_TERMS;
         const size_t units = (size_t)rows * (size_t)P * (size_t)a.n_units;
         SR_HIP(ctx, ctx->spec_units.reserve(units * sizeof(float2), st));

@@ -282,6 +282,7 @@ struct SrSpecArgs {
     float2* units;               // [rows][n_draft + 1][n_units]: every unit's largest scaled logit (NaN: it holds one) and about its sum of exp(x - that)
     float* unit_chains;          // ... [8]: every lane accumulator's part of the sum
     int32_t n_units;
+    int32_t open_side;           // positions of a row that k_spec_open takes side by side
     int32_t all_open;            // the launch is one of these: units are set, open_factors holds what k_spec_open needs
     const SrFullArgs* open_factors;  // on the host: the launch that left factors open (SrFullArgs::factor_later), or null; n_draft < 64
     int32_t any_other;           // some row is not under the ratio test, or greedy: k_spec_verify follows

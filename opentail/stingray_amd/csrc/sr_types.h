@@ -141,17 +141,13 @@ struct SrMaskClear {
 // of it 102 against 106, 192 of 151,936 108 against 111, 176 of 131,072 94 against 97, 144 of it (18,432 segments) 88 against 86, 96 of
 // 151,936 92 against 85; 448 rows of 65,536 108 against 118, 576 of 32,768 92 against 99, 288 of 50,257 (14,400) 84 against 92, 224 of
 // it 78 against 70, 384 of 32,768 (12,288) 84 against 77, 2,304 of 16,384 153 against 210, 768 of it 89 against 83.
-// The verifier's launches of rows that nothing touches, as two launches that leave all sums in order to the positions that need them
-// (k_spec_units, k_spec_open) against the pass, the row kernel and what follows them.  Sequences x drafts, us with them against
-// without: 16 x 8 of 262,144 98 against 127, 1 x 8 51 against 64, 1 x 2 50 against 51; 16 x 8 of 151,936 84 against 104, 4 x 4 50 against
-// 61, 1 x 8 (1,341 segments) 50 against 53, 1 x 2 (447) 50 against 47; of 65,537 16 x 8 57 against 64, 4 x 4 (1,300) 48 against 49, 1 x
-// 8 (585) 45 both.  Rows of 16 to 47 segments from where they are more than the compute units: 64 x 4 of 16,384 53 against 61, of 32,768
-// 55 against 73; 16 x 8 of 20,011 52 against 49, of 28,000 51 against 53, of 40,000 56 both; 1 x 2 of 16,384 40 against 37.  Shorter rows, whose
-// accumulators the row kernel adds up by itself, at every number: 1 x 2 of 4,096 34 against 45, 16 x 8 40 against 50, 64 x 4 42 against
-// 72; 2 x 3 of 14,001 44 against 55.
-#define SR_OPEN_SHORT_SEGS 16
-#define SR_OPEN_MIN_SEGS 48
-#define SR_OPEN_SEGS 1280
+// The verifier's launches of rows that nothing touches go by two launches that leave all sums in order to the positions that need them
+// (k_spec_units, k_spec_open), not by the pass, the row kernel and what follows them, at every length: where every draft is accepted and the
+// bonus rows' largest entries decide, nothing needs them.  Sequences x drafts, us with them against without, such calls and calls with flat
+// bonus rows (N(0, 1.5^2)): 1 x 2 of 16,384 15 against 37 and 41 against 36, 16 x 8 16 against 44 and 46 against 43; 1 x 4 of 32,768 15 against 42 and 43
+// against 40; 16 x 8 of 20,011 19 against 48 and 49 against 47, of 28,000 18 against 52 and 49 against 50, of 40,000 20 against 55 and 51 against
+// 52; 1 x 2 of 49,152 15 against 44 and 41 against 42, of 100,003 18 against 45 and 47 against 44, of 151,936 17 against 46 and 47 against 45, of
+// 262,144 17 against 50 and 51 against 50; 16 x 8 of 262,144 45 against 127 and 98 against 127.
 #define SR_PREPARED_MIN_SEGS 24        // tokens, rows that are cut
 #define SR_PREPARED_MIN_SEGS_MIXED 20  // ... beside rows that are not
 #define SR_PREPARED_ROWS_MIXED 128

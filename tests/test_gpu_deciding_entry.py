@@ -96,7 +96,7 @@ def test_rows_of_the_whole_vocabulary_that_their_largest_entry_decides(ctx, rows
 
 # A verification whose drafts are all accepted: the bonus row's largest entry is its token, or is not.  A row and a half of blocks, one entry in a
 # unit of its own, a block's last entry; short rows, many positions.
-@pytest.mark.parametrize("rows,drafts,vocab", [(16, 2, 50_001), (9, 8, 65_537), (3, 4, 262_144), (40, 7, 8_193), (300, 1, 4_096)])
+@pytest.mark.parametrize("rows,drafts,vocab", [(16, 2, 50_001), (9, 8, 65_537), (3, 4, 262_144), (40, 7, 8_193), (300, 1, 4_096), (2, 3, 16_385), (16, 8, 20_011)])
 def test_bonus_rows_that_their_largest_entry_decides(ctx, rows, drafts, vocab):
     import torch
     from oracle import binding as orc
