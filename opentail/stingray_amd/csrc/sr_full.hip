@@ -2203,6 +2203,52 @@ struct NoFill {
     __device__ __forceinline__ void operator()(int, int) const {}
 };
 __device__ __forceinline__ int list_layout(int i) { return (i & ~1023) | ((i & 15) << 6) | ((i >> 4) & 63); }
+// ... of at most 64 members, at sm.sortbuf as they come: one thread per chain adds its own, and one thread draws.  What the final Normalize
+// multiplies by, 1 where it leaves the values alone.
+__device__ __forceinline__ float finish_short_list(const SrFullArgs& a, int n, int m, int row, FullSmem& sm)
+{
+    const int nv8 = (n / 8) * 8;
+    const int tid = threadIdx.x;
+    if (tid < SR_SEQ_CHAINS) {
+        float s = 0.0f;
+        for (int i = 0; i < m; i++) {
+            const unsigned long long v = sm.sortbuf[i];
+            const int e = (int)(0xffffffffu - (uint32_t)(v >> 32));
+            const int chain = e < nv8 ? (e & 7) : e - (n - 8);
+            if (chain == tid) s = __fadd_rn(s, sr_u2f((uint32_t)v));
+        }
+        sm.lane_sum[tid] = s;
+    }
+    __syncthreads();
+    const float l0 = sm.lane_sum[0], l1 = sm.lane_sum[1], l2 = sm.lane_sum[2], l3 = sm.lane_sum[3],
+                l4 = sm.lane_sum[4], l5 = sm.lane_sum[5], l6 = sm.lane_sum[6], l7 = sm.lane_sum[7];
+    const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
+    const bool scale = sum > 0.0f && sum != 1.0f;
+    const float inv = scale ? __fdiv_rn(1.0f, sum) : 1.0f;
+    if (a.mode != 1 && tid == 0) {
+        const float r = __double2float_rn(sm.u);
+        int token = n - 1;
+        if (!(r > 0.0f)) {
+            token = 0;  // the running sum starts at p[0] >= 0: index 0 reaches a target of zero whatever it holds
+        } else {
+            float acc = 0.0f;
+            bool hit = false;
+            for (int i = 0; i < m && !hit; i++) {
+                const unsigned long long v = sm.sortbuf[i];
+                const float x = sr_u2f((uint32_t)v), xs = scale ? __fmul_rn(x, inv) : x;
+                acc = __fadd_rn(acc, xs);
+                if (acc >= r) {
+                    token = (int)(0xffffffffu - (uint32_t)(v >> 32));
+                    hit = true;
+                    SR_AMB_IF(sr_stop_near(acc, xs, r));
+                }
+            }
+            if (!hit) SR_AMB_IF(sr_near(acc, r));
+        }
+        if (a.out_tokens) a.out_tokens[row] = token;
+    }
+    return inv;
+}
 template <typename Fill = NoFill>
 __device__ __forceinline__ void finish_from_ordered_list(const SrFullArgs& a, float* p, int n, int m, int row, FullSmem& sm,
                                                          Fill fill = Fill(), int cap = kSmall, bool laid_out = false)
@@ -2244,47 +2290,8 @@ __device__ __forceinline__ void finish_from_ordered_list(const SrFullArgs& a, fl
         }
     };
     if (kResident && m <= SR_WAVE) {
-        // A short list: one thread per chain adds its members as they come, and one thread draws.
-        const int tid = threadIdx.x;
-        if (tid < SR_SEQ_CHAINS) {
-            float s = 0.0f;
-            for (int i = 0; i < m; i++) {
-                const unsigned long long v = sm.sortbuf[i];
-                const int e = (int)(0xffffffffu - (uint32_t)(v >> 32));
-                const int chain = e < nv8 ? (e & 7) : e - (n - 8);
-                if (chain == tid) s = __fadd_rn(s, sr_u2f((uint32_t)v));
-            }
-            sm.lane_sum[tid] = s;
-        }
-        __syncthreads();
-        const float l0 = sm.lane_sum[0], l1 = sm.lane_sum[1], l2 = sm.lane_sum[2], l3 = sm.lane_sum[3],
-                    l4 = sm.lane_sum[4], l5 = sm.lane_sum[5], l6 = sm.lane_sum[6], l7 = sm.lane_sum[7];
-        const float sum = __fadd_rn(__fadd_rn(__fadd_rn(l0, l1), __fadd_rn(l2, l3)), __fadd_rn(__fadd_rn(l4, l5), __fadd_rn(l6, l7)));
-        const bool scale = sum > 0.0f && sum != 1.0f;
-        const float inv = scale ? __fdiv_rn(1.0f, sum) : 1.0f;
-        if (a.mode != 0 && scale) row_pass<true>(p, n, [&](float x, int) -> float { return __fmul_rn(x, inv); });
-        if (a.mode != 1 && tid == 0) {
-            const float r = __double2float_rn(sm.u);
-            int token = n - 1;
-            if (!(r > 0.0f)) {
-                token = 0;  // the running sum starts at p[0] >= 0: index 0 reaches a target of zero whatever it holds
-            } else {
-                float acc = 0.0f;
-                bool hit = false;
-                for (int i = 0; i < m && !hit; i++) {
-                    const unsigned long long v = sm.sortbuf[i];
-                    const float x = sr_u2f((uint32_t)v), xs = scale ? __fmul_rn(x, inv) : x;
-                    acc = __fadd_rn(acc, xs);
-                    if (acc >= r) {
-                        token = (int)(0xffffffffu - (uint32_t)(v >> 32));
-                        hit = true;
-                        SR_AMB_IF(sr_stop_near(acc, xs, r));
-                    }
-                }
-                if (!hit) SR_AMB_IF(sr_near(acc, r));
-            }
-            if (a.out_tokens) a.out_tokens[row] = token;
-        }
+        const float inv = finish_short_list(a, n, m, row, sm);
+        if (a.mode != 0 && inv != 1.0f) row_pass<true>(p, n, [&](float x, int) -> float { return __fmul_rn(x, inv); });
         return;
     }
     float sc = 0.0f;
@@ -2995,7 +3002,7 @@ __device__ __forceinline__ void sort_survivors_in_place(uint32_t* keys, int32_t*
 // (One workgroup used to count the row's e into a histogram, read the row once per 8,192 entries of its nucleus to list
 // them, and once more to list the members: 113 us a launch of 16 constrained rows of 151,936, of which the listing reads
 // -- 600 KB each at what one compute unit takes in -- were two thirds.)
-enum ListWay : int { kListDone = 0, kListDeferred = 1, kListGeneral = 2 };
+enum ListWay : int { kListDone = 0, kListDeferred = 1, kListGeneral = 2, kListClosed = 3 };
 __device__ __forceinline__ int list_place(int i) { return i + (i >> 4); }  // (runs of 16 start in different banks)
 
 __device__ __forceinline__ uint32_t* list_values(uint32_t* more, FullSmem& sm) { return more ? more : (uint32_t*)sm.sortbuf; }
@@ -3819,15 +3826,7 @@ __device__ __forceinline__ int cut_from_short_list(const SrFullArgs& a, const Sr
 {
     const int tid = threadIdx.x, lane = sr_lane();
     const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f, use_min_p = rd.min_p > 0.0f;
-    const int nseg = seg_count(n);
     const uint32_t from = st->list_from;
-    float* const ssum = (float*)sm.sortbuf + 2 * SR_WAVE;  // (behind the members of the list)
-    float* const csum = ssum + SR_SEG_MAX;
-    if (a.mode != 0) {
-        for (int i = tid; i < nseg; i += kT) ssum[i] = 0.0f;
-        for (int i = tid; i < a.chain_stride; i += kT) csum[i] = 0.0f;
-        __syncthreads();
-    }
     if (sr_wave_id() == 0) {
         const float mp = do_scale ? __fmul_rn(1.0f, inv) : 1.0f;  // the largest probability: the largest e is expf(0) = 1
         const float thr = use_min_p ? __fmul_rn(rd.min_p, mp) : 0.0f;
@@ -3875,10 +3874,6 @@ __device__ __forceinline__ int cut_from_short_list(const SrFullArgs& a, const Sr
         if (member) {
             sm.sortbuf[__popcll(ms & ((1ull << lane) - 1ull))] = ((unsigned long long)(0xffffffffu - (uint32_t)idx) << 32) | (unsigned long long)sr_f2u(y);
             if (rank == cutoff - 1) { sm.bc[9] = (uint32_t)idx; sm.bc[10] = sr_f2u(y); }
-            if (a.mode != 0) {
-                unsafeAtomicAdd(&ssum[idx / SR_SEG_TERMS], e);
-                if (idx < (n / 8) * 8) unsafeAtomicAdd(&csum[idx / (SR_HALF_BLOCK_SEGS * SR_SEG_TERMS) * SR_SEQ_CHAINS + (idx & (SR_SEQ_CHAINS - 1))], e);
-            }
         }
         if (lane == 0) sm.segbc[1] = (uint32_t)(found == -2 ? 0 : cutoff);
     }
@@ -3889,10 +3884,16 @@ __device__ __forceinline__ int cut_from_short_list(const SrFullArgs& a, const Sr
         finish_from_ordered_list(a, p, n, m, row, sm);
         return kListDone;
     }
-    for (int i = tid; i < nseg; i += kT) a.seg_sum[(size_t)slot * a.seg_stride + i] = ssum[i];
-    for (int i = tid; i < a.chain_stride; i += kT) a.chain_sum[(size_t)slot * a.chain_stride + i] = csum[i];
+    // The members' sum and the draw are at hand: k_prepared_row has the row to write, nothing to meet for.  (With what it leaves out for
+    // rows that their largest entry decides, distributions with tokens, us before and now: 16 rows of 262,144, every third uncut, 67 -> 54, 64 of
+    // 151,936 87 -> 74, 16 bf16 rows of 100,003 49 -> 40, one row of 151,936 39 -> 31.)
+    const float inv2 = finish_short_list(a, n, m, row, sm);
     row_deferred(a, st, inv, sr_u2f(sm.bc[10]), (int)sm.bc[9], sm);
-    return kListDeferred;
+    if (tid == 0) {
+        st->mul2 = inv2;
+        st->drawn = a.seq;
+    }
+    return kListClosed;
 }
 
 // A row whose workgroups did not meet (SrFullState::late): everything by this workgroup alone, from the logits -- the adjusted
@@ -4006,6 +4007,9 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
         const bool walked = a.seg_func != nullptr && !alone;
         // (a list that would have been too long was not made)
         const bool has_list = walked && row_is_listed(rd, a) && st_list_from != 0u, plain = walked && row_is_plain(rd, a);
+        // A row whose distribution is asked for as well, nothing cuts, and its largest entry decides: k_prepared_row makes neither the
+        // records of the draw nor the walk over them (SrFullState::drawn).  It costs nothing here: a wave beside the one that walks.
+        const bool asks_draw = !kLater && plain && a.prepared && a.mode == 2;
         float* const e_row = walked ? row_e(a, slot) : p;
         const uint32_t mk = SR_RARE(alone) ? row_alone(a, rd, p, n, row, sm) : full_maxkey_of(a, st_maxkey);
         const bool any_nan = mk == 0xffffffffu;
@@ -4083,6 +4087,25 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                     for (int g = sr_lane(); g < nseg; g += SR_WAVE) about += a.seg_sum[(size_t)slot * a.seg_stride + g];
                     about = sr_wave_sum_f32(about);
                     if (sr_lane() == 0) sm.segbc[3] = sr_f2u(about);
+                } else if (asks_draw) {
+                    // (where e = 1 stands: the row is not decided unless all others' e add up to less than that)
+                    if (sr_wave_id() == 1) {
+                        const double u = a.uniforms[(size_t)row * a.uniforms_per_row];
+                        const int nseg = seg_count(n), lane = sr_lane();
+                        float all = 0.0f, front = 0.0f, own = 0.0f;
+                        int top = -1;
+                        for (int g0 = 0; g0 < nseg; g0 += SR_WAVE) {
+                            const float part = g0 + lane < nseg ? a.seg_sum[(size_t)slot * a.seg_stride + g0 + lane] : 0.0f;
+                            const unsigned long long has = __ballot(part >= 1.0f);
+                            const int l = has != 0ull ? (int)__ffsll((long long)has) - 1 : SR_WAVE;
+                            all += part;
+                            front += top < 0 && lane < l ? part : 0.0f;
+                            own += top < 0 && lane == l ? part : 0.0f;
+                            if (has != 0ull) top = g0 + l;
+                        }
+                        const bool yes = row_decided(rd, n, sr_wave_sum_f32(all), sr_wave_sum_f32(front), sr_wave_sum_f32(own), __double2float_rn(u));
+                        if (lane == 0) sm.segbc[3] = top >= 0 && yes ? 1u : 0u;
+                    }
                 } else if (has_list) {
                     // where the segments' entries start: every wave adds up the counts for itself and writes all of them, the
                     // same values (a scan by the workgroup, in front of the walk, was two barriers)
@@ -4162,6 +4185,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
             if (plain && (a.prepared || (kLater && spec_by_ratio(rd)))) {
                 row_deferred(a, st, inv, -1.0f, 0, sm);
                 if (tid == 0) {
+                    if (asks_draw) st->drawn = sm.segbc[3] != 0u ? a.seq : 0u;
                     if (kLater) {
                         st->e_open = row_e_open(rd, a) ? a.seq : 0u;
                         st->mul2 = __fdiv_rn(sum, sr_u2f(sm.segbc[3]));
@@ -4199,7 +4223,7 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
                     if (tid == 0) {
                         const uint32_t f = flags | (sm.bc[SR_AMB_WORD] ? SR_KFLAG_AMBIGUOUS : 0u);
                         st->flags = f;
-                        if (way == kListDone && a.out_flags) a.out_flags[row] = f;
+                        if ((way == kListDone || (way == kListClosed && a.mode == 2)) && a.out_flags) a.out_flags[row] = f;
                     }
                     return;
                 }
@@ -4643,10 +4667,22 @@ __device__ __forceinline__ void prepared_load(const PreparedRow<kLogits>& r, int
 // z of the wave's segment: to the caller's row where the distribution is handed out, and the segment's record for the draw
 template <bool kLogits>
 __device__ __forceinline__ void prepared_segment(const SrFullArgs& a, const PreparedRow<kLogits>& r, int slot, int row, int seg, int lane, float4 (&v)[4],
-                                                 float before, float inv2, float4* turn)
+                                                 float before, float inv2, float4* turn, bool drawn)
 {
     const int n = r.n;
     float* const p = a.work + (size_t)(a.work_by_row ? row : slot) * a.work_stride;
+    if (drawn && r.ycut < 0.0f) {
+        // the uncut row's token is its largest entry, e = 1, the only one whose fl(e m1) is m1
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
+            const int at = v[k].x == r.inv ? i0 : v[k].y == r.inv ? i0 + 1 : v[k].z == r.inv ? i0 + 2 : v[k].w == r.inv ? i0 + 3 : -1;
+            if (at >= 0) {
+                if (a.out_tokens) a.out_tokens[row] = at;
+                if (a.out_flags) a.out_flags[row] = a.state[slot].flags;
+            }
+        }
+    }
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         const int i0 = seg * SR_SEG_TERMS + (k * SR_WAVE + lane) * 4;
@@ -4661,7 +4697,7 @@ __device__ __forceinline__ void prepared_segment(const SrFullArgs& a, const Prep
             }
         }
     }
-    if (a.mode == 1) return;
+    if (a.mode == 1 || drawn) return;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -4713,7 +4749,13 @@ __device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, Pr
     const int seg = blk * SR_SEQ_CHAINS + wave;
     float4 v[4];
     float4 ev[4];  // (phase 3)
+    const bool drawn = kPhase != 3 && st->drawn == a.seq, closed = drawn && !(r.ycut < 0.0f);
+    if (closed && kPhase == 1) return;
     prepared_load(r, blk, wave, lane, v, ev);
+    if (closed) {
+        if (seg < nseg) prepared_segment(a, r, slot, row, seg, lane, v, 0.0f, st->mul2, room, true);
+        return;
+    }
     // about what stands in front of the block's terms of the wave's chain, and of the wave's segment
     const float* const cs = a.chain_sum + (size_t)slot * a.chain_stride;
     float before = 0.0f, before_seg = 0.0f, own = 0.0f;
@@ -4723,7 +4765,7 @@ __device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, Pr
         if (2 * blk < hb1) own = cs[2 * blk * SR_SEQ_CHAINS + wave];
         if (2 * blk + 1 < hb1) own += cs[(2 * blk + 1) * SR_SEQ_CHAINS + wave];
     }
-    if (kPhase != 1 && kPhase != 3 && !a.lazy_scale && a.mode != 1 && seg < nseg)
+    if (kPhase != 1 && kPhase != 3 && !a.lazy_scale && a.mode != 1 && !drawn && seg < nseg)
         for (int g = lane; g < seg; g += SR_WAVE) before_seg += sums[g];
     float x[SR_SEQ_RUN];
     if (kPhase != 2 && blk < nblk) {
@@ -4857,7 +4899,7 @@ __device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, Pr
         here = bc[2] != 0u;
         inv2 = sr_u2f(bc[1]);
     }
-    if (here && seg < nseg) prepared_segment(a, r, slot, row, seg, lane, v, sr_wave_sum_f32(before_seg), inv2, room + wave * SR_WAVE * 5);
+    if (here && seg < nseg) prepared_segment(a, r, slot, row, seg, lane, v, sr_wave_sum_f32(before_seg), inv2, room + wave * SR_WAVE * 5, drawn);
     sr_drain_stores();
     __syncthreads();
     if (tid == 0) {
@@ -4876,12 +4918,12 @@ __device__ __forceinline__ void prepared_block(const SrFullArgs& a, int slot, Pr
             prepared_load(r, b, wave, lane, v);
             float front = 0.0f;
             for (int g = lane; g < sg; g += SR_WAVE) front += sums[g];
-            prepared_segment(a, r, slot, row, sg, lane, v, sr_wave_sum_f32(front), inv2, room + wave * SR_WAVE * 5);
+            prepared_segment(a, r, slot, row, sg, lane, v, sr_wave_sum_f32(front), inv2, room + wave * SR_WAVE * 5, drawn);
         }
         sr_drain_stores();
         __syncthreads();
     }
-    if (a.mode == 1 || wave != 0) return;
+    if (a.mode == 1 || drawn || wave != 0) return;
     const float u = st->u;
     int found;
     const float at = seg_walk_from<true, true>([&](int sg, float (&x)[SR_SEQ_RUN]) __attribute__((always_inline)) {

@@ -149,7 +149,8 @@ struct SrFullState {
     float u;              // the uniform of the draw, of a row left to the whole device
     uint32_t e_open;      // the number of the last launch that did not write the row's e down: its reader takes it from the logits
     uint32_t decided;     // the number of the last launch in which k_full_softmax_seg found the row's token
-    int32_t pad;
+    uint32_t drawn;       // ... in which k_full_row left the row to the whole device without its draw: of an uncut row that its largest entry
+                          // decides (ycut < 0), or of one whose second factor is known as well (mul2)
 };
 static_assert(sizeof(SrFullState) == 64, "the 8-byte word, aligned, in front");
 // SrFullArgs::row_sync, a word per row (rows 256 bytes apart: every workgroup of a row adds to its word and polls it):

@@ -94,6 +94,29 @@ def test_rows_of_the_whole_vocabulary_that_their_largest_entry_decides(ctx, rows
     _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, 0, bf16, 8 if rows < 10 else 2 if rows < 50 else 1)
 
 
+
+# ... and where the distribution is handed out beside the token, that is written whole, by two launches (many rows) and by one: rows that nothing
+# cuts, nuclei and min-p cuts of a few entries.
+@pytest.mark.parametrize("rows,vocab,bf16", [(3, 20_001, False), (12, 100_003, True), (20, 65_536, False), (90, 65_537, False)])
+def test_distributions_of_rows_that_their_largest_entry_decides(ctx, rows, vocab, bf16):
+    import torch
+    from oracle import binding as orc
+    from tests.helpers import to_oracle
+
+    rng = np.random.default_rng(rows * vocab)
+    for _ in range(2):
+        logits, params, u = _rows(rng, rows, vocab, 0, bf16)
+        dev = torch.from_numpy(logits).cuda()
+        if bf16:
+            dev = dev.to(torch.bfloat16)
+        toks, probs = ctx.sample_with_distribution(dev, params, u)
+        alone = ctx.build_distribution(dev, params).cpu().numpy()
+        probs = probs.cpu().numpy()
+        assert np.array_equal(toks, oracle_tokens(logits, params, u)), np.nonzero(toks != oracle_tokens(logits, params, u))[0][:10]
+        for r in range(rows):
+            want = orc.build_filtered_distribution(logits[r], to_oracle(params[r]))
+            assert np.array_equal(probs[r], want) and np.array_equal(alone[r], want), r
+
 # A verification whose drafts are all accepted: the bonus row's largest entry is its token, or is not.  A row and a half of blocks, one entry in a
 # unit of its own, a block's last entry; short rows, many positions.
 @pytest.mark.parametrize("rows,drafts,vocab", [(16, 2, 50_001), (9, 8, 65_537), (3, 4, 262_144), (40, 7, 8_193), (300, 1, 4_096), (2, 3, 16_385), (16, 8, 20_011)])
