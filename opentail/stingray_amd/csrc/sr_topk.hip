@@ -643,9 +643,9 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
             const float needs = use_top_p ? fmaxf(rd.top_p, 0.505f) : 0.505f;
             return rest * needs < 1.0f - needs && !(rd.min_p > 0.0f && rest > rd.min_p);
         },
-        // the thread's history entries at or above the bound: about what they add to the row's sum, in units of the entry x_top,
-        // and the largest of them, (adjusted key << 32 | ~id); scale = log2(e) / T
-        [&](float bound, float x_top, float scale, unsigned long long* best) SR_INL -> float {
+        // the thread's history entries at or above the bound: about what they add to the row's sum, each by its weight, and the
+        // largest of them, (adjusted key << 32 | ~id)
+        [&](float bound, auto&& weight, unsigned long long* best) SR_INL -> float {
             float mass = 0.0f;
             adjust_history();  // (fetched before the row was streamed)
             const uint32_t bound_key = sr_okey(bound);
@@ -653,7 +653,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
             for (int r = 0; r < kHistRegs; r++) {
                 if (r * kThreads >= ne) continue;  // uniform
                 if (hraw[r] != 0u && hadj[r] >= bound_key) {
-                    mass += __builtin_amdgcn_exp2f(__fmul_rn(__fsub_rn(sr_okey_inv(hadj[r]), x_top), scale));
+                    mass += weight(sr_okey_inv(hadj[r]));
                     const unsigned long long cmp = ((unsigned long long)hadj[r] << 32) | (unsigned long long)(0xffffffffu - (uint32_t)hee[r].id);
                     *best = cmp > *best ? cmp : *best;
                 }
@@ -661,9 +661,10 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
             return mass;
         },
         // Whether the row's largest entry is the answer: `mass` is at least the sum of the exponentials of everything that can be
-        // among the k best, in units of the entry x_top, `top` the largest entry's own.  See "the largest entry decides".
+        // among the k best, in units of the largest kept one, `top` the largest entry's own.  See "the largest entry decides".
         [&](float mass, float top) SR_INL -> bool {
-            // (the k best are added in fp32, 2,048 roundings at most: 1.3e-4; the exponentials here are good to 1e-5)
+            // (the k best are added in fp32, 2,048 roundings at most: 1.3e-4; the exponentials here are good to 1e-5 at any
+            // temperature: their exponents are differences of the values that the exact way takes them of)
             const float least = top / mass * (1.0f - 4e-4f), rest = mass / top * (1.0f + 4e-4f) - 1.0f;  // p_0 >= least, all others' e <= rest
             const bool use_top_p = rd.top_p < 1.0f && rd.top_p > 0.0f;
             bool yes = top > 0.0f && mass < 1e30f && least > 0.505f && u_row > 2e-6f && u_row < 1.0f - 4e-6f;
@@ -1899,9 +1900,11 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
     if constexpr (kDecide) {
         // (a step of its own, which rows that do not take it do not pay for)
         constexpr int kGroup = kFoldPos<EPV, kVec> * (kFold ? 2 : 1);  // most elements of a group
-        const float scale = __fmul_rn(inv_temp, 1.44269504f), x_top = sr_okey_inv(row_max);
-        // an entry's exponential in units of the largest one's
-        auto weight = [&](float x) SR_INL -> float { return __builtin_amdgcn_exp2f(__fmul_rn(__fsub_rn(x, x_top), scale)); };
+        // An entry's exponential in units of the largest one's.  Scaled and rounded first, then subtracted, as the exact way does: the roundings of
+        // x / T grow with it, and at |x| / T of thousands two entries' exponents lie further apart, or less far, by more than any margin
+        // here; they may be one value.  (A scaled maximum that is not finite gives no number, and nothing is decided.)
+        const float y_top = __fmul_rn(sr_okey_inv(row_max), inv_temp);
+        auto weight = [&](float x) SR_INL -> float { return __builtin_amdgcn_exp2f(__fmul_rn(__fsub_rn(__fmul_rn(x, inv_temp), y_top), 1.44269504f)); };
         // (sel entries at the bound say for most flat rows that there is nothing to ask)
         if (direct && want_bins && row_max > kKeyNegInf && worth_asking((float)(sel - 1) * weight(tval))) {
             // (all of a chunk's groups at once, and one exponential for the lane's second ones: walking the set bits, as the lists are made, took
@@ -1919,7 +1922,7 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
             mass += mq2 != 0u ? (float)(__popc(mq2) * (kGroup - 1)) * weight(second) : 0.0f;
             unsigned long long best = 0ull;
             if (rd.edit_cnt > 0) {
-                mass += hist_mass(tval, x_top, scale, &best);
+                mass += hist_mass(tval, weight, &best);
                 best = sr_wave_max_u64(best);
             }
             mass = sr_wave_sum_f32(mass);

@@ -57,12 +57,12 @@ def _rows(rng, rows, vocab, top_k, bf16):
     return logits, params, u
 
 
-def _check(ctx, rng, rows, vocab, top_k, bf16, rounds):
+def _check(ctx, rng, rows, vocab, top_k, bf16, rounds, make=_rows):
     import torch
 
     h = hooks_lib()
     for _ in range(rounds):
-        logits, params, u = _rows(rng, rows, vocab, top_k, bf16)
+        logits, params, u = make(rng, rows, vocab, top_k, bf16)
         dev = torch.from_numpy(logits).cuda()
         if bf16:
             dev = dev.to(torch.bfloat16)
@@ -85,6 +85,79 @@ def _check(ctx, rng, rows, vocab, top_k, bf16, rounds):
     (20, 12_345, 50, False), (270, 9_001, 900, False), (300, 20_011, 60, True), (530, 16_384, 200, False), (260, 4 * CHUNK + 9, 100, False)])
 def test_rows_that_their_largest_entry_decides(ctx, rows, vocab, top_k, bf16):
     _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, top_k, bf16, 12 if rows < 10 else 3 if rows < 100 else 1)
+
+
+def _scaled(x, t):
+    """fl(x / T) as the sampler takes it: times a rounded 1 / T."""
+    return np.asarray(x, dtype=np.float32) * (np.float32(1.0) / np.float32(t))
+
+
+def _cold_rows(rng, rows, vocab, top_k, bf16, most=8e6):
+    """Two entries a few of their last places apart, far above the rest, at temperatures at which the roundings of x / T are as large as what
+    lies between them: what the larger one covers by the values as they stand and by the scaled, rounded ones differs, and the uniform or top-p
+    lies in between, or near it.  |x| / T up to about `most`."""
+    logits = rng.normal(-5, 1, (rows, vocab)).astype(np.float32)
+    params, u = [], rng.random(rows)
+    for r in range(rows):
+        size = float(rng.choice([0.7, 20.0, 28.0, 300.0, 1e4])) * rng.uniform(0.7, 1.3)
+        t = np.float32(max(10.0 ** rng.uniform(-5.2, -2), size / most))
+        if r % 5 == 2:
+            size = -size
+            logits[r] = np.float32(4 * size - 1.0) + logits[r]
+        at, other = (int(i) for i in rng.choice(vocab, 2, replace=False))
+        p = SamplingParams(Temperature=float(t), TopK=int(rng.integers(2, top_k + 1)))
+        x0 = np.float32(size)
+        if bf16:
+            x0 = synthetic.bf16_bits_to_f32(synthetic.to_bf16_bits(np.array([x0])))[0]
+        if r % 3 == 1:  # one of them, or both, through the history
+            p.PresencePenalty, p.FrequencyPenalty = 0.25, 0.125
+            p.PreviousTokens = rng.integers(0, vocab, 30).tolist() + [at] * 3 + ([other] if r % 2 else [])
+        gap = float(rng.choice([0.3, 1.0, 2.0, 4.0])) * float(t)  # ... of each other, or the next value below if that is more
+        x1 = np.float32(float(x0) - gap)
+        if bf16:
+            x1 = synthetic.bf16_bits_to_f32(synthetic.to_bf16_bits(np.array([x1])))[0]
+        if x1 == x0:
+            x1 = np.nextafter(x0, np.float32(-np.inf)) if not bf16 else x0
+        logits[r, at], logits[r, other] = x0, x1
+        # what they have behind the penalties, and what the larger one covers, by differences as they stand and by scaled values
+        adj = {}
+        for i in (at, other):
+            v, c = logits[r, i], (p.PreviousTokens or []).count(i)
+            adj[i] = v - (np.float32(0.25) + np.float32(0.125) * np.float32(c)) if c else v
+        hi, lo = max(adj.values()), min(adj.values())
+        with np.errstate(over="ignore", invalid="ignore"):
+            stands = 1.0 / (1.0 + np.exp(-(float(hi) - float(lo)) / float(t)))
+            scaled = 1.0 / (1.0 + np.exp(-float(_scaled(hi, t) - _scaled(lo, t))))
+        line = float(rng.choice([stands, scaled, 0.5 * (stands + scaled)])) * (1.0 + float(rng.choice([-1e-2, -6e-4, -1e-5, 0.0, 1e-5])))
+        line = min(max(line, 0.0), 0.9999999)
+        if r % 2:
+            p.TopP = float(np.float32(min(max(line, 1e-3), 0.9999)))
+            u[r] = rng.choice([0.3, 0.8, 0.999])
+        else:
+            u[r] = line
+        if r % 4 == 3:
+            p.MinP = float(np.float32(rng.choice([0.02, 0.4, 0.9])))
+        params.append(p)
+    if bf16:
+        logits = synthetic.bf16_bits_to_f32(synthetic.to_bf16_bits(logits))
+    return logits, params, u
+
+
+@pytest.mark.parametrize("rows,vocab,top_k,bf16", [
+    (1, 49_152, 40, False), (20, 12_345, 50, False), (24, 100_003, 300, False), (24, 30_001, 300, True), (7, 6 * CHUNK + 3, 500, False), (300, 20_011, 60, False),
+    (530, 16_384, 200, False), (530, 9_001, 50, True)])
+def test_rows_at_temperatures_at_which_scaled_values_round_apart(ctx, rows, vocab, top_k, bf16):
+    _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, top_k, bf16, 24 if rows == 1 else 6 if rows < 100 else 1, _cold_rows)
+
+
+def test_a_row_at_a_thousandth_whose_draw_lies_between_the_two(ctx):
+    import torch
+
+    logits = np.full((1, 49_152), -5.0, dtype=np.float32)
+    logits[0, 100], logits[0, 200] = 28.457004547, 28.456491470
+    params, u = [SamplingParams(Temperature=1e-3, TopK=40)], np.array([0.6252147])
+    assert oracle_tokens(logits, params, u)[0] == 200
+    assert ctx.sample_batch(torch.from_numpy(logits).cuda(), params, u)[0] == 200
 
 
 # The full-vocabulary path: one, two and four segments a wave, rows that end inside a segment, rows of odd addresses, several turns of workgroups.
