@@ -1811,7 +1811,10 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
         // them, so they need not become candidates.  Rows whose penalties may raise a logit keep the plain bound.
         const bool lowering_only = (rd.flags & kRowHasPenalty) == 0u || rd.edit_cnt <= 0 || (rd.flags & kRowHistExcl) != 0u;
         if (rd.path == SR_PATH_TOPK && lowering_only && km > kKeyNegInf && rd.temperature > 0.0f) {
-            const float tdead = __fsub_rn(sr_okey_inv(km), __fmul_rn(19.0f, rd.temperature));
+            // (An entry's and the maximum's scaled values are rounded, and so is this difference: three last places of |km| / T, which from
+            // |km| / T of 1e7 on is more than what lies between 19 and the 16.7 that count.  Eight are allowed for.)
+            const float top = sr_okey_inv(km);
+            const float tdead = __fsub_rn(top, __fadd_rn(__fmul_rn(19.0f, rd.temperature), __fmul_rn(fabsf(top), 0x1p-21f)));
             tval = fmaxf(tval, tdead);
         }
         bins = want_bins && direct && km > kKeyNegInf;

@@ -92,10 +92,10 @@ def _scaled(x, t):
     return np.asarray(x, dtype=np.float32) * (np.float32(1.0) / np.float32(t))
 
 
-def _cold_rows(rng, rows, vocab, top_k, bf16, most=8e6):
+def _cold_rows(rng, rows, vocab, top_k, bf16, most):
     """Two entries a few of their last places apart, far above the rest, at temperatures at which the roundings of x / T are as large as what
     lies between them: what the larger one covers by the values as they stand and by the scaled, rounded ones differs, and the uniform or top-p
-    lies in between, or near it.  |x| / T up to about `most`."""
+    lies in between, or near it.  |x| / T up to about `most`; beyond 1e9 some rows' scaled maximum is no finite number."""
     logits = rng.normal(-5, 1, (rows, vocab)).astype(np.float32)
     params, u = [], rng.random(rows)
     for r in range(rows):
@@ -137,17 +137,22 @@ def _cold_rows(rng, rows, vocab, top_k, bf16, most=8e6):
             u[r] = line
         if r % 4 == 3:
             p.MinP = float(np.float32(rng.choice([0.02, 0.4, 0.9])))
+        if most > 1e9 and r % 13 == 6:
+            p.Temperature = float(np.float32(rng.choice([1e-35, 1e-38])))
         params.append(p)
     if bf16:
         logits = synthetic.bf16_bits_to_f32(synthetic.to_bf16_bits(logits))
     return logits, params, u
 
 
+# (from |x| / T of some 1e7 on, entries tens of T below the largest may have its scaled value)
+@pytest.mark.parametrize("most", [8e6, 4e9])
 @pytest.mark.parametrize("rows,vocab,top_k,bf16", [
     (1, 49_152, 40, False), (20, 12_345, 50, False), (24, 100_003, 300, False), (24, 30_001, 300, True), (7, 6 * CHUNK + 3, 500, False), (300, 20_011, 60, False),
-    (530, 16_384, 200, False), (530, 9_001, 50, True)])
-def test_rows_at_temperatures_at_which_scaled_values_round_apart(ctx, rows, vocab, top_k, bf16):
-    _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, top_k, bf16, 24 if rows == 1 else 6 if rows < 100 else 1, _cold_rows)
+    (200, 40_000, 900, False), (530, 16_384, 200, False), (530, 9_001, 50, True)])
+def test_rows_at_temperatures_at_which_scaled_values_round_apart(ctx, rows, vocab, top_k, bf16, most):
+    _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, top_k, bf16, 24 if rows == 1 else 6 if rows < 100 else 1,
+           lambda *how: _cold_rows(*how, most))
 
 
 def test_a_row_at_a_thousandth_whose_draw_lies_between_the_two(ctx):
