@@ -50,6 +50,12 @@ SR_API int sr_debug_set_spin_limit(sr_ctx* ctx, uint32_t polls);
  * set it holds for that launch alone. */
 SR_API int sr_debug_set_row_wait_limit(sr_ctx* ctx, uint32_t polls);
 
+/* A step of a batch whose rows all take the full-vocabulary path and are sampled, tokens and flags to the device; then every row is marked as
+ * one of whose workgroups stopped waiting at the row's first meeting, `none` is put into the results, and the launch behind the meetings runs once
+ * more.  A row that its largest entry decided was written before that launch and keeps `none`; every other row gets its token again. */
+SR_API int sr_selftest_late_rows(sr_ctx* ctx, const sr_batch* batch, const void* logits_dev, int dtype, int64_t row_stride, int32_t none,
+                                 int32_t* out_tokens_dev, uint32_t* out_flags_dev);
+
 /* Profiling builds (-DSR_PROFILE) only, SR_ERR_UNSUPPORTED otherwise: phase timestamps (wall_clock64, 100 MHz) of
  * the selection kernel go to prof_dev[unit][16], one unit per chunk item and per row; NULL switches them off. */
 SR_API int sr_debug_set_profile(sr_ctx* ctx, unsigned long long* prof_dev);

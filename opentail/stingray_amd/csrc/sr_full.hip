@@ -3954,7 +3954,9 @@ __global__ __launch_bounds__(kT) void k_full_row(SrFullArgs a)
     // wave that will walk them) and how many entries its segments have listed (by the others).
     const uint32_t st_late = st->late, st_list_from = st->list_from, st_decided = st->decided;
     const unsigned long long st_maxkey = st->maxkey;
-    if (st_decided == a.seq && st_late != a.seq) return;
+    // (Whatever `late` says: only a workgroup that had all of the row's words decides, and one that decides has written the token.  Written once
+    // more, it could come after the caller has it and has begun the next call: into that one's results, from logits given away.)
+    if (st_decided == a.seq) return;
     SegRec first64 = {};
     constexpr int kCntAhead = 4;
     int cnt_ahead[kCntAhead] = {};

@@ -685,6 +685,36 @@ int sr_selftest_segsum(sr_ctx* ctx, const float* x_dev, int32_t n, double skew, 
                                           out_sum_dev, out_idx_dev, ctx->stream));
     return SR_OK;
 }
+// Test hook: the full-vocabulary rows of a batch, and then their last launch once more as if a workgroup of every row had stopped waiting at
+// the row's first meeting, with `none` in the results
+int sr_selftest_late_rows(sr_ctx* ctx, const sr_batch* b, const void* logits_dev, int dtype, int64_t row_stride, int32_t none, int32_t* out_tokens_dev,
+                          uint32_t* out_flags_dev)
+{
+    if (!ctx || !b) return SR_ERR_NULL_ARGUMENT;
+    const int n = (int)b->h_full_list.size();
+    if (n != b->rows || b->full_greedy > 0 || !out_tokens_dev || !out_flags_dev)
+        return sr_fail(ctx, SR_ERR_INVALID_ARGUMENT, "sr_selftest_late_rows: not a batch of sampled full-vocabulary rows");
+    if (int rc = check_batch_call(ctx, b, logits_dev, dtype, row_stride, "sr_selftest_late_rows")) return rc;
+    SR_HIP(ctx, hipSetDevice(ctx->device));
+    bool any_top_p = false;
+    for (const SrRow& r : b->h_rows) any_top_p = any_top_p || row_uses_top_p(r);
+    SrFullArgs a{};
+    if (int rc = run_full(ctx, b, b->d_full_list.as<int32_t>(), n, any_top_p, logits_dev, dtype, row_stride, 0, nullptr, 0, out_tokens_dev, out_flags_dev,
+                          false, nullptr, 0, &a))
+        return rc;
+    std::vector<SrFullState> state((size_t)n);
+    const std::vector<int32_t> nothing((size_t)n, none);
+    SR_HIP(ctx, hipMemcpyAsync(state.data(), a.state, (size_t)n * sizeof(SrFullState), hipMemcpyDeviceToHost, ctx->stream));
+    SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    for (SrFullState& s : state) { s.late = a.seq; s.deferred = 0u; }
+    SR_HIP(ctx, hipMemcpyAsync(a.state, state.data(), (size_t)n * sizeof(SrFullState), hipMemcpyHostToDevice, ctx->stream));
+    SR_HIP(ctx, hipMemcpyAsync(out_tokens_dev, nothing.data(), (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+    SR_HIP(ctx, hipMemcpyAsync(out_flags_dev, nothing.data(), (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream));
+    SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    SR_HIP(ctx, sr_launch_full_row(a, n, ctx->stream));
+    SR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return SR_OK;
+}
 #endif  // SR_TEST_HOOKS
 
 }  // extern "C"

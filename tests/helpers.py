@@ -49,6 +49,7 @@ def hooks_lib():
         H.sr_debug_append_moves.argtypes = [vp]
         H.sr_debug_set_spin_limit.argtypes = [vp, C.c_uint32]
         H.sr_debug_set_row_wait_limit.argtypes = [vp, C.c_uint32]
+        H.sr_selftest_late_rows.argtypes = [vp, vp, vp, C.c_int, C.c_int64, C.c_int32, vp, vp]
         _hooks = H
     return _hooks
 

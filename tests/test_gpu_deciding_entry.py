@@ -172,6 +172,35 @@ def test_rows_of_the_whole_vocabulary_that_their_largest_entry_decides(ctx, rows
     _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, 0, bf16, 8 if rows < 10 else 2 if rows < 50 else 1)
 
 
+# A row whose largest entry decides is written by the pass, once: not again by the launch behind it, although some workgroup of the row has
+# stopped waiting.  A row that nothing decided gets its token there.
+@pytest.mark.parametrize("rows,vocab,bf16", [(1, 49_152, False), (40, 100_003, True), (30, 151_936, False)])
+def test_a_decided_row_that_a_workgroup_has_marked_late_is_not_written_again(ctx, rows, vocab, bf16):
+    import torch
+
+    h, none = hooks_lib(), -77
+    rng = np.random.default_rng(rows)
+    seen = set()
+    for _ in range(24 if rows == 1 else 2):
+        logits, params, u = _rows(rng, rows, vocab, 0, bf16)
+        dev = torch.from_numpy(logits).cuda()
+        if bf16:
+            dev = dev.to(torch.bfloat16)
+        batch = ctx.new_batch().upload(params, vocab, u)
+        tok, flags = (torch.zeros(rows, dtype=torch.int32, device="cuda") for _ in range(2))
+        torch.cuda.synchronize()
+        ctx._check(h.sr_selftest_late_rows(ctx.h, batch.h, dev.data_ptr(), int(bf16), vocab, none, tok.data_ptr(), flags.data_ptr()))
+        got, want, left = tok.cpu().numpy(), oracle_tokens(logits, params, u), flags.cpu().numpy() == none
+        assert np.array_equal(got == none, left)
+        assert np.array_equal(got[~left], want[~left])
+        seen |= set(left.tolist())
+        for polls in (1, 2, 3, 6):  # (few enough that some workgroups leave and others decide; results in pinned memory, call after call)
+            h.sr_debug_set_row_wait_limit(ctx.h, polls)
+            assert np.array_equal(ctx.sample_batch(dev, params, u), want), polls
+        h.sr_debug_set_row_wait_limit(ctx.h, 1 << 15)
+        batch.close()
+    assert seen == {False, True}
+
 
 # ... and where the distribution is handed out beside the token, that is written whole, by two launches (many rows) and by one: rows that nothing
 # cuts, nuclei and min-p cuts of a few entries.
