@@ -7,6 +7,7 @@
 // left to right go through the exact evaluator in sr_seqsum.h, so probabilities, cut-offs and draws
 // carry the reference's bits.
 #include <algorithm>
+#include <cstddef>
 
 #include "sr_device.h"
 #include "sr_kernels.h"
@@ -43,10 +44,11 @@ struct FullSmem {
     float segst[SR_SEG_MAX];  // running sum behind every segment of a prepared row (seg_walk)
     uint32_t segbc[4];
     double u;  // the row's uniform (k_full_row)
-    unsigned long long sortbuf[kSmall];
+    alignas(16) unsigned long long sortbuf[kSmall];  // (cut_unsorted's tables lie here and are read by vectors of 16 bytes)
     float sprob[kSmall];
     uint32_t tags[kSmall];
 };
+static_assert(offsetof(FullSmem, sortbuf) % 16 == 0 && alignof(FullSmem) % 16 == 0, "whole vectors");
 
 // SR_OUT_AMBIGUOUS of the row at work: any thread that sees a cut or the draw land on its boundary (sr_near /
 // sr_stop_near) stores here; the row's flags are written behind a barrier that follows.
@@ -3049,6 +3051,7 @@ struct ListCut {
     bool found;    // the sum got to the target
 };
 constexpr int kInOrder = 1024;  // most entries that are put in order
+static_assert(kInOrder % 4 == 0 && (SR_LIST_CAP_SMALL + SR_LIST_CAP_SMALL / 16) % 4 == 0, "the tables follow each other on whole vectors");
 template <int kPer>
 __device__ __forceinline__ bool cut_unsorted(const uint32_t (&ev)[kPer], uint32_t valid, uint32_t from, bool do_scale, float inv, float target, uint32_t* base,
                                              int G, ListCut* cut, FullSmem& sm)
