@@ -224,8 +224,9 @@ def test_distributions_of_rows_that_their_largest_entry_decides(ctx, rows, vocab
             want = orc.build_filtered_distribution(logits[r], to_oracle(params[r]))
             assert np.array_equal(probs[r], want) and np.array_equal(alone[r], want), r
 
-# A verification whose drafts are all accepted: the bonus row's largest entry is its token, or is not.  A row and a half of blocks, one entry in a
-# unit of its own, a block's last entry; short rows, many positions.
+# Verifications: sequences whose drafts are all accepted for certain, where the bonus row's largest entry is its token or is not, beside some that
+# reject a draft and some with up to three tests too close to tell from about the sums.  A row and a half of blocks, one entry in a unit of its own, a
+# block's last entry; short rows, many positions (of which several are worked out side by side).
 @pytest.mark.parametrize("rows,drafts,vocab", [(16, 2, 50_001), (9, 8, 65_537), (3, 4, 262_144), (40, 7, 8_193), (300, 1, 4_096), (2, 3, 16_385), (16, 8, 20_011)])
 def test_bonus_rows_that_their_largest_entry_decides(ctx, rows, drafts, vocab):
     import torch
@@ -233,7 +234,8 @@ def test_bonus_rows_that_their_largest_entry_decides(ctx, rows, drafts, vocab):
     from tests.helpers import to_oracle
 
     rng = np.random.default_rng(rows + vocab)
-    for _ in range(3 if rows < 100 else 1):
+    rejected = close = 0
+    for turn in range(3 if rows < 100 else 1):
         t = rng.normal(0, 1, (rows, drafts + 1, vocab)).astype(np.float32)
         u = rng.uniform(0.05, 0.5, (rows, drafts + 1))
         temps = [float(np.float32(rng.choice([1.0, rng.uniform(0.5, 1.3)]))) for _ in range(rows)]
@@ -257,11 +259,21 @@ def test_bonus_rows_that_their_largest_entry_decides(ctx, rows, drafts, vocab):
                 u[r, drafts] = rng.choice([0.0, 1e-7, 0.9999999])
             if r % 9 == 5:
                 t[r, drafts, (at + vocab // 2) % vocab] = t[r, drafts, at]  # not the only one
-            if r % 9 == 7:
-                u[r, rng.integers(drafts)] = 0.9999999  # and a row that rejects
+            kind = (r + turn) % 4
+            if kind in (1, 2):  # a rejected draft, or up to three whose test is close: p about half of q, u above p / q or at it
+                for i in rng.choice(drafts, 1 if kind == 1 else min(3, drafts), replace=False):
+                    x = t[r, i].astype(np.float64) / temps[r]
+                    x[k[r, i]] = -np.inf
+                    t[r, i, k[r, i]] = np.float32((x.max() + np.log(np.exp(x - x.max()).sum()) + rng.uniform(-0.5, 0.2)) * temps[r])
+                    x = t[r, i].astype(np.float64) / temps[r]
+                    p = np.exp(x - x.max())
+                    u[r, i] = 0.95 if kind == 1 else p[k[r, i]] / p.sum() / 0.9 * (1.0 + rng.choice([-2e-7, -1e-8, 0.0, 1e-8, 2e-7]))
+                close += kind == 2
         params = [SamplingParams(Temperature=T) for T in temps]
         dev = [torch.from_numpy(v).cuda() for v in (t, q, k.astype(np.int32))]
         acc, tok = ctx.spec_verify(dev[0], dev[1], dev[2], params, u)
         for r in range(rows):
             wa, wt = orc.spec_verify_row(t[r], q[r], k[r], to_oracle(params[r]), orc.Rng(replay=u[r]))
             assert acc[r] == wa and np.array_equal(tok[r][: len(wt)], wt), (r, acc[r], wa, tok[r], wt)
+            rejected += wa < drafts
+    assert rejected > 0 and close > 0
