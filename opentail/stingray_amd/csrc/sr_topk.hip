@@ -487,11 +487,28 @@ struct KeptGroups {
     uint32_t gp[kKeptChunks];
 };
 // ... and what it fetches of its row's history before it starts to stream: the thread's history ids with their
-// counts, and their (masked) logits
+// counts, and their (masked) logits; a worker that keeps its row's groups (kKept) only their ids and keys, see fetch_row
 struct KeptHistory {
     SrEdit hee[kHistRegs];
     float hx[kHistRegs];
+    uint32_t hraw[kHistRegs], hadj[kHistRegs];
 };
+// A history entry's keys, raw and adjusted (0: none), from its (masked) logit
+__device__ __forceinline__ void adjust_entry(const SrRow& rd, const SrEdit& ee, float x, uint32_t* raw, uint32_t* adj)
+{
+    *raw = *adj = 0u;
+    // -inf never enters the reference's selection (Sampler.cs:240-249)
+    if (x == x && sr_f2u(x) != 0xff800000u) {
+        float v = x;
+        // Sampler.cs:261-287: pen = pow(rep, occWindow) once; presence/frequency over the whole history
+        if (ee.occ_all > 0) {
+            if (rd.rep != 1.0f && ee.occ_win > 0) v = v > 0.0f ? __fdiv_rn(v, ee.pen) : __fmul_rn(v, ee.pen);
+            v = __fsub_rn(v, __fadd_rn(rd.presence, __fmul_rn(rd.frequency, (float)ee.occ_all)));
+        }
+        *raw = sr_okey(x);
+        *adj = sr_okey(v);
+    }
+}
 // A worker that knows the row it will finish from the start, and has the registers, fetches the row's descriptor and its history before
 // it streams: in front of the tail they are four trips to memory one behind the other (in a launch that also asks whether the
 // largest entry decides: below).
@@ -599,24 +616,13 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
 #pragma unroll
         for (int r = 0; r < kHistRegs; r++) {
             hadj[r] = hraw[r] = 0u;
-            const int e = r * kThreads + tid;
-            if (e < ne) {
-                const SrEdit ee = hee[r];
-                const float x = hx[r];
-                // -inf never enters the reference's selection (Sampler.cs:240-249)
-                if (x == x && sr_f2u(x) != 0xff800000u) {
-                    float v = x;
-                    // Sampler.cs:261-287: pen = pow(rep, occWindow) once; presence/frequency over the whole history
-                    if (ee.occ_all > 0) {
-                        if (rd.rep != 1.0f && ee.occ_win > 0) v = v > 0.0f ? __fdiv_rn(v, ee.pen) : __fmul_rn(v, ee.pen);
-                        v = __fsub_rn(v, __fadd_rn(rd.presence, __fmul_rn(rd.frequency, (float)ee.occ_all)));
-                    }
-                    hraw[r] = sr_okey(x);
-                    hadj[r] = sr_okey(v);
-                }
-            }
+            if (r * kThreads + tid < ne) adjust_entry(rd, hee[r], hx[r], &hraw[r], &hadj[r]);
         }
     };
+    if constexpr (kKept) {
+#pragma unroll
+        for (int r = 0; r < kHistRegs; r++) { hraw[r] = kept_hist.hraw[r]; hadj[r] = kept_hist.hadj[r]; }
+    }
     const int n_c = build_candidates<EPV, kVec, kKept, kShort, kFold, kDecide>(
         a, slot, row, rd, want_bins, force_exact, inv_temp, &map0, &bound0, &binned, kept,
         [&]() SR_INL {
@@ -647,7 +653,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
         // largest of them, (adjusted key << 32 | ~id)
         [&](float bound, auto&& weight, unsigned long long* best) SR_INL -> float {
             float mass = 0.0f;
-            adjust_history();  // (fetched before the row was streamed)
+            if constexpr (!kKept) adjust_history();  // (fetched before the row was streamed)
             const uint32_t bound_key = sr_okey(bound);
 #pragma unroll
             for (int r = 0; r < kHistRegs; r++) {
@@ -894,7 +900,7 @@ __device__ __forceinline__ void topk_row_tail(const SrTopkArgs& a, int slot, int
     } else {
         // ---- no penalties, or penalties that only lower: candidates outside the history + the history ids --
         if (ne > kHistRegs * kThreads) { give_up(SR_KFLAG_UNSUPPORTED, -1); return; }
-        adjust_history();
+        if constexpr (!kKept) adjust_history();
         SR_PROF(a, 5);
         // How far an entry lies below the bins' origin, in 1/56 of a log-unit: -1 = absent or dropped, else
         // 0..1023.  Never increasing with the key, so "bin <= b" is a prefix of the descending order.
@@ -2140,6 +2146,16 @@ __global__ __launch_bounds__(kThreads, kRoomy ? 2 : 4) void k_topk_rows(SrTopkAr
                 const bool in = hist_regs && e < trd.edit_cnt;
                 kept_hist.hee[r] = in ? a.edits[trd.edit_off + e] : SrEdit{};
                 kept_hist.hx[r] = in ? row_logit(a, trow, trd, kept_hist.hee[r].id) : SR_NEG_INF;
+            }
+            // A worker that keeps its row's groups has no registers to spare: an entry's id and keys wait in three of them, its logit and
+            // counts would in seven.  (So until the tail, and worked out in two places of it, 29 to 53 registers were spilled where two workers share a
+            // compute unit, and fp32 rows of five to eight chunks lost what asking whether the largest entry decides gained elsewhere.  us a
+            // launch, without the question, with it and the tail adjusting, with it and this: 700 rows of 200,000 95.2, 100.2, 92.4, 546 of 261,080
+            // with short lists 115.7, 121.5, 114.3, without a history 109.6, 114.2, 106.2, 300 of it 74.4, 76.7, 71.0; 512 of 151,936 63.1, 62.5,
+            // 61.4.  The others, which stream a chunk or two, would wait here for the logits: 1 row of 49,152 11.0 and 11.1.)
+            if constexpr (kKept) {
+#pragma unroll
+                for (int r = 0; r < kHistRegs; r++) adjust_entry(trd, kept_hist.hee[r], kept_hist.hx[r], &kept_hist.hraw[r], &kept_hist.hadj[r]);
             }
         }
     };
