@@ -4,7 +4,7 @@ of zero for the kernels' bounded waits)."""
 
 import numpy as np
 import pytest
-from opentail.stingray_amd import SamplerContext, SamplingParams, synthetic
+from opentail.stingray_amd import SamplerContext, SamplingParams, pack_allow_mask, synthetic
 from tests.helpers import hooks_lib, oracle_tokens
 
 pytestmark = pytest.mark.gpu
@@ -62,16 +62,16 @@ def _check(ctx, rng, rows, vocab, top_k, bf16, rounds, make=_rows):
 
     h = hooks_lib()
     for _ in range(rounds):
-        logits, params, u = make(rng, rows, vocab, top_k, bf16)
+        logits, params, u, *masks = make(rng, rows, vocab, top_k, bf16)
         dev = torch.from_numpy(logits).cuda()
         if bf16:
             dev = dev.to(torch.bfloat16)
-        got, flags = ctx.sample_batch(dev, params, u, return_flags=True)
-        want = oracle_tokens(logits, params, u)
+        got, flags = ctx.sample_batch(dev, params, u, *masks, return_flags=True)
+        want = oracle_tokens(logits, params, u, *masks)
         assert np.array_equal(got, want), np.nonzero(got != want)[0][:10]
         h.sr_debug_set_spin_limit(ctx.h, 0)
         h.sr_debug_set_row_wait_limit(ctx.h, 0)
-        other, other_flags = ctx.sample_batch(dev, params, u, return_flags=True)
+        other, other_flags = ctx.sample_batch(dev, params, u, *masks, return_flags=True)
         h.sr_debug_set_spin_limit(ctx.h, 1 << 22)
         h.sr_debug_set_row_wait_limit(ctx.h, 1 << 15)
         assert np.array_equal(got, other)
@@ -170,6 +170,43 @@ def test_a_row_at_a_thousandth_whose_draw_lies_between_the_two(ctx):
                                              (66, 200_064, False), (40, 50_257, True), (280, 16_385, False)])
 def test_rows_of_the_whole_vocabulary_that_their_largest_entry_decides(ctx, rows, vocab, bf16):
     _check(ctx, np.random.default_rng(rows + vocab), rows, vocab, 0, bf16, 8 if rows < 10 else 2 if rows < 50 else 1)
+
+
+def _odd_rows(rng, rows, vocab, top_k, bf16):
+    """Every second entry is masked away, far above all others; the largest of the rest carries a bias where no top-k is asked for.  Some
+    rows hold a NaN, a +inf, one or two finite entries, or values a thousand times as large at as many times the temperature."""
+    half, params, u = _rows(rng, rows, vocab // 2, top_k, False)
+    logits = np.full((rows, vocab), 60.0, dtype=np.float32)
+    allowed = np.zeros((rows, vocab), dtype=bool)
+    allowed[:, 1:2 * (vocab // 2):2] = True
+    for r in range(rows):
+        at, p = int(np.argmax(half[r])), params[r]
+        if p.PreviousTokens:
+            p.PreviousTokens = [2 * t + 1 for t in p.PreviousTokens]
+        if not top_k and r % 2:
+            half[r, at] -= np.float32(2.0)
+            p.LogitBias = {2 * at + 1: 2.0, 2 * int(rng.integers(vocab // 2)): -1.0}
+        odd = r % 9
+        if odd == 1:
+            half[r, rng.integers(vocab // 2)] = np.nan
+        elif odd == 2:
+            half[r, rng.integers(vocab // 2)] = np.inf
+        elif odd in (3, 4):
+            keep = rng.choice(vocab // 2, odd - 2, replace=False)
+            half[r] = np.where(np.isin(np.arange(vocab // 2), keep), half[r], -np.inf)
+        elif odd in (5, 6) and not p.PreviousTokens and not p.LogitBias:
+            half[r] *= np.float32(1000.0)
+            p.Temperature *= 1000.0
+        logits[r, 1:2 * (vocab // 2):2] = half[r]
+    if bf16:
+        logits = synthetic.bf16_bits_to_f32(synthetic.to_bf16_bits(logits))
+    return logits, params, u, pack_allow_mask(allowed), np.ones(rows, dtype=np.uint8)
+
+
+@pytest.mark.parametrize("rows,vocab,top_k,bf16", [(9, 40_000, 50, False), (20, 100_003, 300, True), (540, 16_385, 60, False), (9, 50_001, 0, False),
+                                                   (40, 100_003, 0, True), (70, 151_936, 0, False)])
+def test_masked_and_biased_rows_and_odd_values_of_which_the_largest_may_decide(ctx, rows, vocab, top_k, bf16):
+    _check(ctx, np.random.default_rng(rows + vocab + top_k), rows, vocab, top_k, bf16, 8 if rows < 10 else 2 if rows < 50 else 1, _odd_rows)
 
 
 # A row whose largest entry decides is written by the pass, once: not again by the launch behind it, although some workgroup of the row has
