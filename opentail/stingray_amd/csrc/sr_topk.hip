@@ -519,10 +519,11 @@ template <bool kKept, bool kRoomy> constexpr bool kHistBefore = kKept || kRoomy;
 // second largest standing in for what may lie below it, add up to at least the row's sum.  Such a row is done there; fetching groups, ordering
 // the list, the exact sums and the searches are for the others.  Nothing is decided that the exact arithmetic could see otherwise: the margins cover
 // its roundings, a draw or cut near a boundary (SR_OUT_AMBIGUOUS) is left to it, and so is a largest entry that is not the only one.
-// In launches of short lists, of dealt rows, and of more rows than compute units, us a launch before and now, rows whose largest entry stands
-// out and flat ones (N(0, 1.5^2)): 1 row of 49,152 fp32, top-k 40, 12.9 -> 10.8 and 14.0 -> 14.5, with a history of 64 13.2 -> 11.4 and 14.5 -> 14.9; 24 of
-// 100,003 bf16, top-k up to 1,000, 19.0 -> 12.0 and 24.6 -> 24.8; 512 of 151,936 fp32 61.2 -> 52.9 and 67.0 -> 66.5, 1,024 109 -> 96.9 and 117.6
-// -> 113.4 (3 to 4 of each from SR_RARE).  A launch of a worker to every compute unit ends with its flattest rows, which the question only keeps waiting.
+// In launches of short lists, of dealt rows, and of more rows than compute units, us a launch without it and with (and with SR_RARE and a history
+// adjusted where it is fetched), rows of the benchmark's generator, whose largest entry mostly decides, and flat ones (N(0, 1.5^2)): 1 row of 49,152 fp32,
+// top-k 40, 12.9 -> 10.8 and 14.2 -> 14.9, with a history of 64 13.4 -> 11.6 and 13.9 -> 14.3; 24 of 100,003 bf16, top-k up to 1,000, 17.8 -> 15.9 and
+// 23.9 -> 24.6; 512 of 151,936 fp32 60.5 -> 57.1 and 66.4 -> 65.2, 1,024 107.4 -> 99.1 and 115.5 -> 110.9; 700 of 200,000 with histories 95.3 -> 93.5 and
+// 96.7 -> 94.7.  A launch of a worker to every compute unit ends with its flattest rows, which the question only keeps waiting.
 template <bool kKept, bool kShort, bool kRoomy> constexpr bool kDecides = kHistBefore<kKept, kRoomy> && (kShort || !kKept || !kRoomy);
 constexpr int kDecided = -3;  // what build_candidates returns for such a row
 // The masked logit of one token id of a row.
@@ -1902,10 +1903,6 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
     auto pick4 = [&](const float4& v, int g) SR_INL -> uint32_t {
         return sel2(sel2(sr_f2u(v.x), sr_f2u(v.y), g), sel2(sr_f2u(v.z), sr_f2u(v.w), g), g >> 1);
     };
-    auto pick16 = [&](const float4 (&v)[4], int bit) SR_INL -> float {
-        const int c = bit >> 2, g = bit & 3;
-        return sr_u2f(sel2(sel2(pick4(v[0], g), pick4(v[1], g), c), sel2(pick4(v[2], g), pick4(v[3], g), c), c >> 1));
-    };
     if constexpr (kDecide) {
         // (a step of its own, which rows that do not take it do not pay for)
         constexpr int kGroup = kFoldPos<EPV, kVec> * (kFold ? 2 : 1);  // most elements of a group
@@ -2045,8 +2042,8 @@ __device__ __forceinline__ int build_candidates(const SrTopkArgs& a, int slot, i
 //
 // kKept: every worker streams all chunks (at most kFoldChunks) of the one row it finishes.  Nothing is handed over then,
 // so nothing is written out: the group results of all chunks stay in the thread's registers and the waves' shares of the
-// bound go through LDS.  Also where two workers share a compute unit: 128 registers hold it (the tail spills 44 bytes a lane;
-// of the shape that writes its results and reads them back 84, and that one pays a bound loop per chunk): 1,024
+// bound go through LDS.  Also where two workers share a compute unit: 128 registers hold it (the tail spills 76 bytes a lane,
+// that of the shape that writes its results and reads them back 20 to 36, and that one pays a bound loop per chunk): 1,024
 // rows of 151,936 fp32 147.5 -> 113.5 us, 512 80.0 -> 59.7, 320 62.1 -> 47.6, 1,024 of bf16 95.7 -> 69.5.
 // kRoomy: a launch of at most one worker per compute unit, compiled for two waves a SIMD, so that the row tail keeps its
 // registers.

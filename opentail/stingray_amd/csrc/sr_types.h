@@ -143,11 +143,19 @@ struct SrMaskClear {
 // it 78 against 70, 384 of 32,768 (12,288) 84 against 77, 2,304 of 16,384 153 against 210, 768 of it 89 against 83.
 // The verifier's launches of rows that nothing touches go by two launches that leave all sums in order to the positions that need them
 // (k_spec_units, k_spec_open), not by the pass, the row kernel and what follows them, at every length: where every draft is accepted and the
-// bonus rows' largest entries decide, nothing needs them.  Sequences x drafts, us with them against without, such calls and calls with flat
-// bonus rows (N(0, 1.5^2)): 1 x 2 of 16,384 15 against 37 and 41 against 36, 16 x 8 16 against 44 and 46 against 43; 1 x 4 of 32,768 15 against 42 and 43
-// against 40; 16 x 8 of 20,011 19 against 48 and 49 against 47, of 28,000 18 against 52 and 49 against 50, of 40,000 20 against 55 and 51 against
-// 52; 1 x 2 of 49,152 15 against 44 and 41 against 42, of 100,003 18 against 45 and 47 against 44, of 151,936 17 against 46 and 47 against 45, of
-// 262,144 17 against 50 and 51 against 50; 16 x 8 of 262,144 45 against 127 and 98 against 127.
+// bonus rows' largest entries decide, nothing needs them.  Where any sequence of the call rejects a draft, has a test too close to tell, or a flat bonus
+// row (N(0, 1.5^2)), some position does need them, and short or few rows pay for it: the host cannot know, and what such calls lose, up to 13 %, is a
+// quarter of what the others gain at most.  Sequences x drafts, us with them against without: everything decided; flat bonus rows; every sequence with a
+// rejection; every sequence with a close test:
+//    1 x 2 of  16,384   14 against 38   39.8 against 35.1   41.4 against 36.5   41.8 against 36.2
+//   16 x 8 of  16,384   16 against 44   46.7 against 43.4   48.6 against 43.9   49.6 against 44.2
+//    1 x 4 of  32,768   15 against 40   43.8 against 39.7   45.9 against 40.9   46.6 against 41.0
+//   16 x 8 of  20,011   21 against 49   50.4 against 47.0   52.0 against 47.7   54.5 against 48.7
+//   16 x 8 of  40,000   22 against 54   54.0 against 51.1   54.5 against 51.6   56.4 against 51.9
+//    1 x 2 of  49,152   15 against 44   43.2 against 42.6   42.5 against 42.2   44.4 against 42.8
+//    1 x 2 of 100,003   18 against 47   46.6 against 42.6   48.5 against 44.5   48.9 against 43.8
+//    1 x 4 of 151,936   17 against 48   48.1 against 46.2   48.1 against 49.1   49.9 against 48.1
+//   16 x 8 of 262,144   45 against 127   98 against 127  (the pass and k_spec_factor)
 #define SR_PREPARED_MIN_SEGS 24        // tokens, rows that are cut
 #define SR_PREPARED_MIN_SEGS_MIXED 20  // ... beside rows that are not
 #define SR_PREPARED_ROWS_MIXED 128
