@@ -43,10 +43,10 @@ struct FullSmem {
     float ckpt[kCkpt];  // running sum behind every tile of a row's exact sum (SeqMarks)
     float segst[SR_SEG_MAX];  // running sum behind every segment of a prepared row (seg_walk)
     uint32_t segbc[4];
-    double u;  // the row's uniform (k_full_row)
     alignas(16) unsigned long long sortbuf[kSmall];  // (cut_unsorted's tables lie here and are read by vectors of 16 bytes)
     float sprob[kSmall];
     uint32_t tags[kSmall];
+    double u;  // the row's uniform (k_full_row)
 };
 static_assert(offsetof(FullSmem, sortbuf) % 16 == 0 && alignof(FullSmem) % 16 == 0, "whole vectors");
 
